@@ -194,6 +194,20 @@ def check(rc: int) -> None:
     raise RuntimeError(f"hira error {rc}: {msg}")
 
 
+def stream_of(index: int) -> int:
+    """Handle of torch's current HIP stream on device number `index`."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or \
+            (lambda i: torch.cuda.current_stream(i).cuda_stream)
+    return _raw_stream(index)
+
+
+_raw_stream = None
+
+
 def current_stream(device) -> int:
     """Handle of torch's current HIP stream on `device`, for the `stream` argument of the
     library's calls.  The raw getter costs a fraction of a microsecond where

@@ -15,6 +15,7 @@ keeps and reuses: clone it to hold on to a result across calls (searcher/cuda.py
 from __future__ import annotations
 
 import ctypes as C
+from threading import get_ident
 from typing import Optional, Tuple
 
 import torch
@@ -36,7 +37,30 @@ def _on(t: torch.Tensor, device) -> bool:
     return t.device.index == device.index
 
 
+class _Call:
+    """What a call on one tree with one number of heads needs and does not change from call to
+    call: the C structs (only this thread fills them in), the head map, a scale of one per head,
+    the workspace's size.  Made on first use and kept by the searcher: a call that comes with ready
+    tensors (the storage type, on the index's device, contiguous) then allocates and copies nothing
+    and its host side is a handful of attribute reads around one library call (21 -> 8 us for
+    ``search``, 25 -> 11 us for ``search_attention``, which the kernels of small indexes are shorter
+    than)."""
+
+    __slots__ = ("tree", "query", "out", "queue", "dev", "keep", "ones", "ws_bytes", "ws_rows",
+                 "tree_ref", "query_ref", "out_ref", "queue_ref", "launch_ref")
+
+    def __init__(self, tree, launch, query, dev, keep, ones):
+        self.tree, self.query, self.dev, self.keep, self.ones = tree, query, dev, keep, ones
+        self.out = _lib.HiraSearchOut()
+        self.queue = _lib.HiraQueue()
+        self.ws_bytes, self.ws_rows = 0, -1  # the workspace, and the queue rows it was sized for
+        self.tree_ref, self.query_ref = C.byref(tree), C.byref(query)
+        self.out_ref, self.queue_ref, self.launch_ref = C.byref(self.out), C.byref(self.queue), C.byref(launch)
+
+
 class HIPSearcher(BaseSearcher):
+    _MAX_CALLS = 256  # kept call descriptions: a model's layers, several threads, a few growths
+
     def __init__(self, block_c=None, output_fill_value: float = DEFAULT_OUTPUT_FILL_VALUE,
                  *, index_space: str = "slot", block_threads: int = 0, nodes_per_wave: int = 0,
                  kernel: int = 0, separate_merge: bool = False):
@@ -52,6 +76,7 @@ class HIPSearcher(BaseSearcher):
         self._map_cache = {}
         self._workspace: Optional[torch.Tensor] = None
         self._decode_plans: dict = {}
+        self._calls: dict = {}
         self._sel = None
 
     # -------------------------------------------------------------- input coercion
@@ -150,6 +175,49 @@ class HIPSearcher(BaseSearcher):
                             heads.data_ptr(), gmax, group)
         return qs, (q, tau, sc, off, heads)
 
+    def _call(self, query, threshold, indexer, q_head_to_kv, scaling) -> Tuple[_Call, int, tuple]:
+        """(call description with its query filled in, H_q, tensors to keep alive until the launch)."""
+        tree = indexer.tree_struct()
+        dim = indexer.dim
+        if q_head_to_kv is None and isinstance(query, torch.Tensor) and \
+                query.dtype is indexer.dtype and query.is_contiguous():
+            shape = query.shape
+            nd = len(shape)
+            if shape[-1] == dim and (nd == 2 or (nd == 4 and shape[2] == 1)):
+                h_q = query.numel() // dim
+                key = (get_ident(), id(tree), h_q)
+                c = self._calls.get(key)
+                if c is None:
+                    off, heads, gmax, group = self._head_map(h_q, indexer, None)
+                    # (through the host: the copy is complete for every stream when it returns)
+                    ones = torch.ones((h_q,)).to(indexer.keys_buf.device)
+                    qs = _lib.HiraQuery(h_q, None, None, None, off.data_ptr(), heads.data_ptr(), gmax, group)
+                    if len(self._calls) >= self._MAX_CALLS:
+                        self._calls.clear()
+                    c = self._calls[key] = _Call(tree, self.launch, qs, indexer.keys_buf.get_device(),
+                                                 (off, heads), ones)
+                if query.get_device() == c.dev:
+                    dev, qs = c.dev, c.query
+                    if isinstance(threshold, torch.Tensor) and threshold.dtype is torch.float32 and \
+                            threshold.numel() == h_q and threshold.get_device() == dev and \
+                            threshold.is_contiguous():
+                        tau = threshold
+                    else:
+                        tau = self._coerce_threshold(threshold, h_q, indexer.device)
+                    if scaling is None:
+                        sc = c.ones
+                    elif isinstance(scaling, torch.Tensor) and scaling.dtype is torch.float32 and \
+                            scaling.numel() == h_q and scaling.get_device() == dev and \
+                            scaling.is_contiguous():
+                        sc = scaling
+                    else:
+                        sc = self._coerce_scaling(scaling, h_q, indexer.device)
+                    qs.q, qs.tau, qs.scaling = query.data_ptr(), tau.data_ptr(), sc.data_ptr()
+                    return c, h_q, (query, tau, sc)
+        qs, keep = self._query_struct(query, threshold, indexer, q_head_to_kv, scaling)
+        return (_Call(tree, self.launch, qs, indexer.keys_buf.get_device(), keep, None),
+                qs.num_q_heads, keep)
+
     def _get_workspace(self, nbytes: int, device) -> torch.Tensor:
         if self._workspace is None or self._workspace.numel() < nbytes or \
                 not _on(self._workspace, device):
@@ -168,20 +236,24 @@ class HIPSearcher(BaseSearcher):
             self._tmp_out.fill_(self.output_fill_value)
         return self._tmp_out
 
-    def _run(self, indexer, qs, out: _lib.HiraSearchOut, queue: Optional[_lib.HiraQueue]):
+    def _run(self, indexer, c: _Call, attn: bool, queue_rows: int = 0):
         lib = _lib.lib()
-        tree = indexer.tree_struct()
-        ws_ptr, ws_bytes, ws = None, 0, None
-        if out.attn_out:
-            ws_bytes = lib.hira_search_workspace_bytes(
-                C.byref(tree), C.byref(qs), C.byref(queue) if queue else None,
-                C.byref(self.launch))
-            ws = self._get_workspace(ws_bytes, indexer.device)
+        ws_ptr, ws_bytes = None, 0
+        queue_ref = c.queue_ref if queue_rows else None
+        if attn:
+            if queue_rows > c.ws_rows:  # (more rows in the queue may mean more partials)
+                c.ws_rows = queue_rows
+                c.ws_bytes = lib.hira_search_workspace_bytes(c.tree_ref, c.query_ref, queue_ref,
+                                                             c.launch_ref)
+            ws_bytes = c.ws_bytes
+            ws = self._workspace
+            if ws is None or ws.get_device() != c.dev or ws.numel() < ws_bytes:
+                ws = self._get_workspace(ws_bytes, indexer.device)
             ws_ptr = ws.data_ptr()
-        stream = _lib.current_stream(indexer.device)
-        rc = lib.hira_search(C.byref(tree), C.byref(qs), C.byref(queue) if queue else None,
-                             C.byref(out), C.byref(self.launch), ws_ptr, ws_bytes, stream)
-        _lib.check(rc)
+        rc = lib.hira_search(c.tree_ref, c.query_ref, queue_ref, c.out_ref, c.launch_ref, ws_ptr,
+                             ws_bytes, _lib.stream_of(c.dev))
+        if rc:
+            _lib.check(rc)
 
     # -------------------------------------------------------------- public API
     def search(self, query, threshold, indexer, q_head_to_kv: Optional[torch.Tensor] = None,
@@ -190,19 +262,20 @@ class HIPSearcher(BaseSearcher):
         if indexer.keys_buf is None:
             raise ValueError("Indexer is not built: missing children tensor.")
         space = index_space or self.index_space
-        qs, keep = self._query_struct(query, threshold, indexer, q_head_to_kv, scaling)
-        n = indexer.size[0] if space == "slot" else indexer.num_keys
+        c, h_q, keep = self._call(query, threshold, indexer, q_head_to_kv, scaling)
+        slots = space == "slot"
+        n = indexer.size[0] if slots else indexer.num_keys
         # in slot space the search fills what it does not select itself: one launch per call
-        fused_fill = space == "slot"
-        dense = self._prepare_output_buffer(qs.num_q_heads, n, indexer.device, fill=not fused_fill)
-        out = _lib.HiraSearchOut()
-        out.dense = dense.data_ptr()
-        out.dense_stride = dense.stride(0)
-        out.dense_by_position = 1 if space == "position" else 0
-        out.dense_fill = 1 if fused_fill else 0
+        dense = self._tmp_out
+        if not slots or dense is None or dense.shape != (h_q, n) or dense.get_device() != c.dev:
+            dense = self._prepare_output_buffer(h_q, n, indexer.device, fill=not slots)
+        out = c.out
+        out.dense, out.dense_stride = dense.data_ptr(), n
+        out.dense_by_position, out.dense_fill = (0, 1) if slots else (1, 0)
         out.dense_fill_value = self.output_fill_value
+        out.sel_index = out.sel_score = out.sel_count = out.attn_out = None
         out.stats = None if stats is None else stats.data_ptr()
-        self._run(indexer, qs, out, None)
+        self._run(indexer, c, False)
         del keep
         return dense
 
@@ -211,20 +284,22 @@ class HIPSearcher(BaseSearcher):
         """Compact result: (index (H_q, cap) int32, score (H_q, cap) fp32 raw q.k,
         count (H_q,) int32); entries of a head are unordered."""
         space = index_space or self.index_space
-        qs, keep = self._query_struct(query, threshold, indexer, q_head_to_kv, scaling)
+        c, h_q, keep = self._call(query, threshold, indexer, q_head_to_kv, scaling)
         cap = int(capacity or indexer.size[0])
-        h_q, dev = qs.num_q_heads, indexer.device
+        dev = indexer.device
         if self._sel is None or self._sel[0].shape != (h_q, cap) or not _on(self._sel[0], dev):
             self._sel = (torch.empty((h_q, cap), dtype=torch.int32, device=dev),
                          torch.empty((h_q, cap), dtype=torch.float32, device=dev),
                          torch.zeros((h_q,), dtype=torch.int32, device=dev))
         idx, score, count = self._sel
         count.zero_()
-        out = _lib.HiraSearchOut()
+        out = c.out
+        out.dense = out.attn_out = out.stats = None
+        out.dense_fill = 0
         out.dense_by_position = 1 if space == "position" else 0
         out.sel_index, out.sel_score, out.sel_count = idx.data_ptr(), score.data_ptr(), count.data_ptr()
         out.sel_cap = cap
-        self._run(indexer, qs, out, None)
+        self._run(indexer, c, False)
         del keep
         return idx, score, count
 
@@ -266,24 +341,34 @@ class HIPSearcher(BaseSearcher):
         given, every queued key (T, m, D) / value (T, m, Dv).  Returns (H_q, Dv) fp32."""
         if indexer.values_buf is None:
             raise ValueError("the index was built without values: nothing to attend to")
-        qs, keep = self._query_struct(query, threshold, indexer, q_head_to_kv, scaling)
-        h_q, dev = qs.num_q_heads, indexer.device
+        c, h_q, keep = self._call(query, threshold, indexer, q_head_to_kv, scaling)
         if out is None:
-            out = torch.empty((h_q, indexer.vdim), dtype=torch.float32, device=dev)
-        so = _lib.HiraSearchOut()
+            out = torch.empty((h_q, indexer.vdim), dtype=torch.float32, device=indexer.keys_buf.device)
+        so = c.out
+        so.dense = so.sel_index = so.sel_score = so.sel_count = None
+        so.dense_by_position = so.dense_fill = 0
         so.attn_out = out.data_ptr()
         so.stats = None if stats is None else stats.data_ptr()
-        queue = None
+        rows = 0
         if queue_keys is not None and queue_keys.shape[-2] > 0:
-            qk = queue_keys.reshape(indexer.num_trees, -1, indexer.dim)
-            qv = queue_values.reshape(indexer.num_trees, -1, indexer.vdim)
-            qk = qk.to(device=dev, dtype=indexer.dtype).contiguous()
-            qv = qv.to(device=dev, dtype=indexer.dtype).contiguous()
-            queue = _lib.HiraQueue(qk.data_ptr(), qv.data_ptr(), qk.shape[1], qk.shape[1])
+            qk = self._queue_rows(queue_keys, indexer, c.dev, indexer.dim)
+            qv = self._queue_rows(queue_values, indexer, c.dev, indexer.vdim)
+            rows = qk.numel() // (indexer.num_trees * indexer.dim)
+            qu = c.queue
+            qu.keys, qu.values, qu.len, qu.cap = qk.data_ptr(), qv.data_ptr(), rows, rows
             keep = keep + (qk, qv)
-        self._run(indexer, qs, so, queue)
+        self._run(indexer, c, True, rows)
         del keep
         return out
+
+    @staticmethod
+    def _queue_rows(x: torch.Tensor, indexer, dev: int, width: int) -> torch.Tensor:
+        """Queued rows of all trees, contiguous, in the index's storage type and on its device."""
+        if x.dtype is indexer.dtype and x.get_device() == dev and x.is_contiguous() and \
+                x.numel() % (indexer.num_trees * width) == 0:
+            return x
+        x = x.reshape(indexer.num_trees, -1, width)
+        return x.to(device=indexer.device, dtype=indexer.dtype).contiguous()
 
     def decode_plan(self, indexer, num_q_heads: int, scaling: float) -> "DecodePlan":
         """The plan for (this index, head count, one softmax scale for all heads), made on
@@ -317,6 +402,7 @@ class DecodePlan:
         self.searcher = searcher
         self.lib = _lib.lib()
         dev = indexer.device
+        self._dev = indexer.keys_buf.get_device()
         self.scaling = searcher._coerce_scaling(scaling, num_q_heads, dev)
         off, heads, gmax, group = searcher._head_map(num_q_heads, indexer, q_head_to_kv)
         self._keep = (off, heads, stats)
@@ -326,28 +412,30 @@ class DecodePlan:
         self.out.stats = None if stats is None else stats.data_ptr()
         self.launch = searcher.launch
         self.tree = indexer.tree_struct()
-        self.queue = _lib.HiraQueue(1, 1, 1, 1)  # sizes only: room for a queue's partials
+        self.queue = _lib.HiraQueue()
         self.tau_buf: Optional[torch.Tensor] = None  # (H_q,) thresholds written by run_sampled
+        self._ws_rows = 1  # queue rows the workspace is sized for
         self.ws_bytes = self._workspace_need()
         self.ws = torch.zeros(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
         self._refs = (C.byref(self.tree), C.byref(self.query), C.byref(self.out),
-                      C.byref(self.launch))
+                      C.byref(self.launch), C.byref(self.queue))
 
     def _workspace_need(self) -> int:
         fake_q = _lib.HiraQuery(self.query.num_q_heads, 1, 1, 1, 1, 1, self.query.max_group,
                                 self.query.group_size)  # sizes only
+        rows = _lib.HiraQueue(1, 1, self._ws_rows, self._ws_rows)
         return self.lib.hira_search_workspace_bytes(
-            C.byref(self.tree), C.byref(fake_q), C.byref(self.queue), C.byref(self.launch))
+            C.byref(self.tree), C.byref(fake_q), C.byref(rows), C.byref(self.launch))
 
     def _follow_index(self) -> None:
-        if self.indexer.tree_struct() is not self.tree:  # the index grew since the plan was made
-            self.tree = self.indexer.tree_struct()
-            need = self._workspace_need()
-            if need > self.ws.numel():
-                self.ws = torch.zeros(need, dtype=torch.uint8, device=self.indexer.device)
-            self.ws_bytes = need
-            self._refs = (C.byref(self.tree), C.byref(self.query), C.byref(self.out),
-                          C.byref(self.launch))
+        """The index grew since the plan was made, or a queue holds more rows than before."""
+        self.tree = self.indexer.tree_struct()
+        need = self._workspace_need()
+        if need > self.ws.numel():
+            self.ws = torch.zeros(need, dtype=torch.uint8, device=self.indexer.device)
+        self.ws_bytes = need
+        self._refs = (C.byref(self.tree), C.byref(self.query), C.byref(self.out),
+                      C.byref(self.launch), C.byref(self.queue))
 
     def run(self, query: torch.Tensor, threshold: torch.Tensor, out: torch.Tensor,
             stream: Optional[int] = None, queue_keys: Optional[torch.Tensor] = None,
@@ -356,13 +444,14 @@ class DecodePlan:
         leading dimensions amounting to T trees: keys not in the index yet, attended by every
         head of their tree; the first `queue_len` rows of every tree are in use (all `cap`
         when not given)."""
-        self._follow_index()
-        self.query.q = query.data_ptr()
-        self.query.tau = threshold.data_ptr()
+        if self.indexer.tree_struct() is not self.tree:
+            self._follow_index()
+        q = self.query
+        q.q = query.data_ptr()
+        q.tau = threshold.data_ptr()
         self.out.attn_out = out.data_ptr()
         if stream is None:
-            stream = _lib.current_stream(self.indexer.device)
-        t, q, o, l = self._refs
+            stream = _lib.stream_of(self._dev)
         qu = None
         if queue_keys is not None and queue_keys.shape[-2] > 0 and queue_len != 0:
             cap = int(queue_keys.shape[-2])
@@ -370,8 +459,13 @@ class DecodePlan:
             if not 0 < m <= cap or queue_values.shape[-2] != cap:
                 raise ValueError(f"queue: {m} rows in use of {cap} "
                                  f"(values hold {queue_values.shape[-2]})")
-            self.queue = _lib.HiraQueue(queue_keys.data_ptr(), queue_values.data_ptr(), m, cap)
-            qu = C.byref(self.queue)
+            qs = self.queue
+            qs.keys, qs.values, qs.len, qs.cap = queue_keys.data_ptr(), queue_values.data_ptr(), m, cap
+            if m > self._ws_rows:
+                self._ws_rows = m
+                self._follow_index()
+            qu = self._refs[4]
+        t, q, o, l, _ = self._refs
         rc = self.lib.hira_search(t, q, qu, o, l, self.ws.data_ptr(), self.ws_bytes, stream)
         if rc:
             _lib.check(rc)
@@ -396,8 +490,9 @@ class DecodePlan:
             raise ValueError(f"samples {tuple(samples.shape)} {samples.dtype}: expected contiguous "
                              f"({self.tree.num_trees}, S, {self.tree.dim}) {self.indexer.dtype}")
         if stream is None:
-            stream = _lib.current_stream(self.indexer.device)
-        self._follow_index()
+            stream = _lib.stream_of(self._dev)
+        if self.indexer.tree_struct() is not self.tree:
+            self._follow_index()
         self.query.q = query.data_ptr()
         rule = 0 if method == "sample_max" else 1
         if append is not None:
