@@ -17,7 +17,7 @@ HIRA_MAX_LEVELS = 8
 HIRA_STATS_COLS = HIRA_MAX_LEVELS + 3  # counters per tree a search can fill in
 HIRA_F32, HIRA_BF16 = 0, 1
 HIRA_ROW_MAJOR, HIRA_TILE16, HIRA_TILE16_Q8 = 0, 1, 2
-HIRA_ABI_VERSION = 7
+HIRA_ABI_VERSION = 8
 
 _vp = C.c_void_p
 
@@ -88,6 +88,19 @@ class HiraLaunch(C.Structure):
     ]
 
 
+class HiraArray(C.Structure):
+    _fields_ = [("dst", _vp), ("src", _vp), ("dst_stride", C.c_int64), ("src_stride", C.c_int64),
+                ("copy_bytes", C.c_int64), ("fill_from", C.c_int64), ("fill", C.c_uint32),
+                ("reserved_", C.c_int32)]
+
+
+def out_dtype_of(query: HiraQuery) -> C.c_int32:
+    """The struct's `out_dtype` (HIRA_F32 or HIRA_BF16: the type hira_search writes attn_out in).
+    It lies between `num_q_heads` and `q`, in what was padding before; ``_fields_`` leaves it out so
+    that structs filled in by position keep their meaning."""
+    return C.c_int32.from_buffer(query, 4)
+
+
 # every symbol include/hira_hip.h declares: (restype, argtypes)
 SYMBOLS = {
     "hira_abi_version": (C.c_int, []),
@@ -134,6 +147,17 @@ SYMBOLS = {
         [C.POINTER(HiraTree), _vp, _vp, C.c_int32, _vp, _vp, C.c_int32, C.POINTER(HiraQuery),
          C.c_int32, C.c_int32, _vp, _vp],
     ),
+    "hira_enqueue": (
+        C.c_int,
+        [_vp, _vp, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_int32, _vp,
+         _vp, _vp],
+    ),
+    "hira_replace_rows": (
+        C.c_int,
+        [_vp, C.c_int32, C.c_int32, C.c_int32, C.c_int32, _vp, C.c_int32, C.c_int32,
+         C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.c_int32, _vp],
+    ),
+    "hira_fill_arrays": (C.c_int, [C.POINTER(HiraArray), C.c_int32, C.c_int32, _vp]),
     "hira_threshold": (
         C.c_int,
         [_vp, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.POINTER(HiraQuery), C.c_int32,

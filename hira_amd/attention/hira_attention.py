@@ -115,35 +115,41 @@ def hira_attention_forward(module, query, key, value, attention_mask=None, dropo
         hira_threshold = index_thresholds(indexer, query, hira_topk or max(1, indexer.num_keys // 100))
     # one plan per (index, head count, scale): a decode step is then a single library call
     plan = searcher.decode_plan(indexer, b * h_q, scaling)
-    q2 = query.reshape(b * h_q, d)
-    if q2.dtype != indexer.dtype or q2.device != indexer.device:
-        q2 = q2.to(device=indexer.device, dtype=indexer.dtype)
-    q2 = q2.contiguous()
-    out = torch.empty((b * h_q, indexer.vdim), dtype=torch.float32, device=indexer.device)
+    dev = indexer.keys_buf.device
+    q2 = query
+    if q2.dtype is not indexer.dtype or q2.device != dev:
+        q2 = q2.to(device=dev, dtype=indexer.dtype)
+    if not q2.is_contiguous():
+        q2 = q2.contiguous()
+    # (the search writes its output in the query's own type where that is one of its two)
+    direct = query.dtype is torch.bfloat16 or query.dtype is torch.float32
+    out = torch.empty((b, 1, h_q, indexer.vdim), dtype=query.dtype if direct else torch.float32, device=dev)
     # the queue: the cache layer's own buffers as they are when they already hold the index's
     # storage type (rows in use, rows per head), else a converted copy of the rows in use
     qk = qv = None
-    qlen = int(cache.queued_keys.shape[-2]) if cache.queued_keys is not None else 0
+    qlen = getattr(cache, "queue_rows", None)
+    if qlen is None:
+        qlen = int(cache.queued_keys.shape[-2]) if cache.queued_keys is not None else 0
     if qlen > 0:
         store = getattr(cache, "queue_store", None)
-        if store is not None and store[0].dtype == indexer.dtype and store[0].device == indexer.device \
+        if store is not None and store[0].dtype is indexer.dtype and store[0].device == dev \
                 and store[0].is_contiguous() and store[1].is_contiguous():
             qk, qv = store
         else:
-            qk = cache.queued_keys.to(device=indexer.device, dtype=indexer.dtype).reshape(
+            qk = cache.queued_keys.to(device=dev, dtype=indexer.dtype).reshape(
                 indexer.num_trees, qlen, d).contiguous()
-            qv = cache.queued_values.to(device=indexer.device, dtype=indexer.dtype).reshape(
+            qv = cache.queued_values.to(device=dev, dtype=indexer.dtype).reshape(
                 indexer.num_trees, qlen, -1).contiguous()
     if sampled:
         plan.run_sampled(q2, cache.samples, cache.threshold_method, cache.threshold_topk, out,
                          queue_keys=qk, queue_values=qv, queue_len=qlen)
     else:
-        th = torch.as_tensor(hira_threshold, dtype=torch.float32, device=indexer.device)
+        th = torch.as_tensor(hira_threshold, dtype=torch.float32, device=dev)
         if th.ndim == 0:
             th = th.expand(b * h_q)
         th = th.reshape(b * h_q).contiguous()
         plan.run(q2, th, out, queue_keys=qk, queue_values=qv, queue_len=qlen)
-    return out.reshape(b, 1, h_q, -1).to(query.dtype), None
+    return (out if direct else out.to(query.dtype)), None
 
 
 def register_hira_attention(name: str = "hira") -> str:

@@ -12,12 +12,14 @@ releases are provided: ``get_max_cache_shape`` (reference, cache/hira_cache.py:1
 """
 from __future__ import annotations
 
+import ctypes as C
 from dataclasses import dataclass
 from typing import Any
 
 import torch
 from transformers.cache_utils import Cache, CacheLayerMixin
 
+from hira_amd import _lib
 from hira_amd.cache.hira_config import DeviceMode, HiraConfig
 from hira_amd.indexer import HIPIndexer
 from hira_amd.searcher import HIPSearcher
@@ -44,6 +46,16 @@ class CacheOutput:
     # storage type and on its device, the first queued_keys.shape[-2] rows of every head in
     # use.  The attention function hands them to the library as they are.
     queue_store: tuple | None = None
+
+    def __getattr__(self, name):
+        # an output that a layer made knows how many rows of queue_store were in use; the two views
+        # are taken when somebody looks at them (the attention function does not)
+        rows = self.__dict__.get("queue_rows")
+        if rows is not None and name in ("queued_keys", "queued_values"):
+            view = self.queue_store[name == "queued_values"].narrow(2, 0, rows)
+            self.__dict__[name] = view
+            return view
+        raise AttributeError(name)
 
 
 class HiraCacheLayer(CacheLayerMixin):
@@ -88,6 +100,10 @@ class HiraCacheLayer(CacheLayerMixin):
         dev = getattr(self.indexer, "device", None) or self.device
         self._queue_k = torch.empty((self.batch, self.H_kv, rows, self.dim), dtype=dt, device=dev)
         self._queue_v = torch.empty((self.batch, self.H_kv, rows, self.vdim), dtype=dt, device=dev)
+        self._queue_type = _lib.HIRA_F32 if dt == torch.float32 else _lib.HIRA_BF16
+        esize = self._queue_k.element_size()
+        if dt not in (torch.float32, torch.bfloat16) or self.dim * esize % 16 or self.vdim * esize % 16:
+            self._queue_type = None
 
     @property
     def queued_keys(self):
@@ -104,6 +120,18 @@ class HiraCacheLayer(CacheLayerMixin):
             self._alloc_queue(max(2 * old_k.shape[-2], n + m))
             self._queue_k[:, :, :n] = old_k[:, :, :n]
             self._queue_v[:, :, :n] = old_v[:, :, :n]
+        k, v = self._queue_k, self._queue_v
+        if self._queue_type is not None and k.is_cuda and \
+                key_states.dtype is k.dtype and value_states.dtype is v.dtype and \
+                key_states.get_device() == value_states.get_device() == k.get_device() and \
+                key_states.is_contiguous() and value_states.is_contiguous():
+            # one launch for both
+            _lib.check(_lib.lib().hira_enqueue(
+                k.data_ptr(), v.data_ptr(), self._queue_type, self.batch * self.H_kv, k.shape[2],
+                self.queued_len, m, self.dim, self.vdim, key_states.data_ptr(),
+                value_states.data_ptr(), _lib.stream_of(k.get_device())))
+            self.queued_len += m
+            return
         if key_states.ndim != 4:
             key_states = key_states.reshape(self.batch, self.H_kv, m, self.dim)
             value_states = value_states.reshape(self.batch, self.H_kv, m, self.vdim)
@@ -143,7 +171,15 @@ class HiraCacheLayer(CacheLayerMixin):
             self._alloc_queue(max(1, min(int(self.update_every), 4096)))
             self.indexed_len = key_states.shape[-2]
             self._take_samples(key_states)
+            self._sample_facts()
             return self._output(key_states, value_states), None
+        if self.queued_len == 0 and key_states.shape[-2] >= self.update_every:
+            # what would leave the queue at once does not pass through it
+            if key_states.ndim != 4:
+                key_states = key_states.reshape(self.batch, self.H_kv, -1, self.dim)
+                value_states = value_states.reshape(self.batch, self.H_kv, -1, self.vdim)
+            self._fold(key_states, value_states)
+            return self._output(), None
         self._enqueue(key_states, value_states)
         if self.queued_len >= self.update_every:
             self.update_index()
@@ -174,44 +210,71 @@ class HiraCacheLayer(CacheLayerMixin):
             return
         k4 = new_keys if new_keys.ndim == 4 else new_keys[None]
         m = k4.shape[-2]
-        rows = k4.reshape(-1, m, self.dim).to(self.samples.dtype)
         room = self._sample_target - self.samples.shape[1]
         if room > 0:  # a short prompt: the sample holds every key so far
             take = min(room, m)
-            self.samples = torch.cat([self.samples, rows[:, :take]], dim=1).contiguous()
-            rows, seen, m = rows[:, take:], seen + take, m - take
-            if m == 0:
+            rows = k4.narrow(2, 0, take).reshape(-1, take, self.dim).to(self.samples.dtype)
+            self.samples = torch.cat([self.samples, rows], dim=1).contiguous()
+            self._sample_facts()
+            if take == m:
                 return
+            k4, seen, m = k4.narrow(2, take, m - take), seen + take, m - take
         s = self.samples.shape[1]
-        idx = seen + torch.arange(m)
-        join = torch.rand(m, generator=self._sample_gen) < s / (idx + 1).double()
-        if bool(join.any()):
-            who = join.nonzero().squeeze(1)
-            slots = torch.randint(0, s, (who.numel(),), generator=self._sample_gen)
-            # a slot drawn twice keeps its last arrival (an indexed assignment with repeated
-            # targets has no defined order)
-            last = {int(sl): int(wh) for sl, wh in zip(slots.tolist(), who.tolist())}
-            slots = torch.tensor(list(last.keys()), dtype=torch.long)
-            who = torch.tensor(list(last.values()), dtype=torch.long)
-            self.samples[:, slots.to(self.samples.device)] = rows[:, who.to(rows.device)]
+        draws = torch.rand(m, generator=self._sample_gen).tolist()
+        who = [i for i, u in enumerate(draws) if u < s / (seen + i + 1)]
+        if not who:
+            return
+        slots = torch.randint(0, s, (len(who),), generator=self._sample_gen).tolist()
+        # a slot drawn twice keeps its last arrival
+        last = dict(zip(slots, who))
+        smp = self.samples
+        src = k4
+        if smp.is_cuda:
+            # one launch, the lists travel with its arguments.  (The rows of a head must lie one
+            # behind the other and the heads evenly spaced, as the queue's and a model's do.)
+            if src.dtype is not smp.dtype or src.get_device() != smp.get_device():
+                src = src.to(device=smp.device, dtype=smp.dtype)
+            if src.stride(3) != 1 or (m > 1 and src.stride(2) != self.dim) or \
+                    src.stride(1) % self.dim or (src.shape[0] > 1 and
+                                                 src.stride(0) != src.stride(1) * src.shape[1]):
+                src = src.contiguous()
+            if src.shape[1] == 1 and src.shape[0] == 1:
+                stride = m
+            else:
+                stride = (src.stride(1) if src.shape[1] > 1 else src.stride(0)) // self.dim
+            n = len(last)
+            arr = C.c_int32 * n
+            _lib.check(_lib.lib().hira_replace_rows(
+                smp.data_ptr(), _lib.HIRA_F32 if smp.dtype is torch.float32 else _lib.HIRA_BF16,
+                self.dim, smp.shape[0], s, src.data_ptr(), m, stride, arr(*last.keys()),
+                arr(*last.values()), n, _lib.stream_of(smp.get_device())))
+            return
+        rows = src.reshape(-1, m, self.dim).to(smp.dtype)
+        smp[:, torch.tensor(list(last.keys()))] = rows[:, torch.tensor(list(last.values()))].to(smp.device)
+
+    def _sample_facts(self):
+        """The rule as every output of the layer carries it."""
+        kw = self.threshold_kwargs
+        have = self.samples is not None
+        self._rule = (kw.get("method") if have else None,
+                      max(1, min(int(kw.get("topk", 1)), self.samples.shape[1] if have else 1)))
 
     def _output(self, prefill_keys=None, prefill_values=None):
-        kw = self.threshold_kwargs
-        return CacheOutput(
-            queued_keys=self.queued_keys,
-            queued_values=self.queued_values,
-            prefill_keys=prefill_keys,
-            prefill_values=prefill_values,
-            indexer=self.indexer,
-            searcher=self.searcher,
-            samples=self.samples,
-            threshold_method=kw.get("method") if self.samples is not None else None,
-            threshold_topk=max(1, min(int(kw.get("topk", 1)),
-                                      self.samples.shape[1] if self.samples is not None else 1)),
-            queue_store=(self._queue_k, self._queue_v),
-        )
+        # (filled in directly: the views of the queue are taken when looked at)
+        out = CacheOutput.__new__(CacheOutput)
+        out.__dict__.update(
+            prefill_keys=prefill_keys, prefill_values=prefill_values, indexer=self.indexer,
+            searcher=self.searcher, samples=self.samples, threshold_method=self._rule[0],
+            threshold_topk=self._rule[1], queue_store=(self._queue_k, self._queue_v),
+            queue_rows=self.queued_len)
+        return out
 
     def update_index(self):
+        self._fold(self.queued_keys, self.queued_values)
+        self.queued_len = 0
+
+    def _fold(self, keys, values):
+        """New keys and values (B, H_kv, m, ...) into the index, and their share of the sample."""
         # no read-back of the level sizes: the host carries their bounds (HIPIndexer.update,
         # sync=False), so folding the queue into the index does not wait for the GPU; a
         # one-level index has no node counts to bound with and keeps the synchronous form
@@ -220,13 +283,11 @@ class HiraCacheLayer(CacheLayerMixin):
 
             self._update_takes_sync = "sync" in inspect.signature(self.indexer.update).parameters
         if self._update_takes_sync:
-            self.indexer.update(self.queued_keys, self.queued_values,
-                                sync=getattr(self.indexer, "num_levels", 1) < 2)
+            self.indexer.update(keys, values, sync=getattr(self.indexer, "num_levels", 1) < 2)
         else:  # an indexer with the reference's two-argument update
-            self.indexer.update(self.queued_keys, self.queued_values)
-        self._refresh_samples(self.queued_keys, self.indexed_len)
-        self.indexed_len += self.queued_len
-        self.queued_len = 0
+            self.indexer.update(keys, values)
+        self._refresh_samples(keys, self.indexed_len)
+        self.indexed_len += keys.shape[-2]
 
     def get_mask_sizes(self, cache_position):
         kv_offset = 0

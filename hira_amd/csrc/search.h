@@ -57,11 +57,18 @@ struct SearchParams {
     float* part_acc;  // (H_q, P, Dv)
     int32_t num_parts;  // P = gridDim.x
     int32_t gmax_state; // MFMA kernel: heads per pass its LDS state rows are sized for
-    float* attn_out;    // (H_q, Dv): written by the kernel itself when `done` is set
+    void* attn_out;     // (H_q, Dv): written by the kernel itself when `done` is set
+    int32_t out_bf16;   // its type: bf16, else fp32
     int32_t* done;      // (T, passes) arrival counters, zero between launches; NULL: no fold
     int32_t fold_dvl;   // vector-ALU kernel's fold: threads per partial (four columns each)
     unsigned long long* stats;
 };
+
+// element i of the attention output, in the type the caller asked for
+__device__ __forceinline__ void store_out(void* out, int bf16, size_t i, float v) {
+    if (bf16) reinterpret_cast<uint16_t*>(out)[i] = f32_to_bf16_bits(v);  // uniform
+    else reinterpret_cast<float*>(out)[i] = v;
+}
 
 struct SearchPlan {
     int kernel;       // 1 = vector-ALU, 2 = MFMA

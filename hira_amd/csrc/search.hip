@@ -9,12 +9,13 @@ namespace hira {
 __global__ __launch_bounds__(256) void merge_kernel(const float* __restrict__ part_m,
                                                     const float* __restrict__ part_l,
                                                     const float* __restrict__ part_acc, int P,
-                                                    int Dv, int dvl, float* __restrict__ out) {
+                                                    int Dv, int dvl, void* __restrict__ out,
+                                                    int out_bf16) {
     __shared__ float red[4];
     extern __shared__ float smem[];  // (NG, Dv + 1)
     const int head = blockIdx.x;
     fold_partials(part_m + (size_t)head * P, part_l + (size_t)head * P,
-                  part_acc + (size_t)head * P * Dv, P, Dv, dvl, out + (size_t)head * Dv, smem, red);
+                  part_acc + (size_t)head * P * Dv, P, Dv, dvl, out, out_bf16, (size_t)head * Dv, smem, red);
 }
 
 // ---- host side ------------------------------------------------------------------------
@@ -343,6 +344,9 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
         p.part_m = w + (size_t)query->num_q_heads * P * tree->vdim;
         p.part_l = p.part_m + (size_t)query->num_q_heads * P;
         p.attn_out = out->attn_out;
+        HIRA_CHECK_ARG(query->out_dtype == HIRA_F32 || query->out_dtype == HIRA_BF16,
+                       "out_dtype %d", query->out_dtype);
+        p.out_bf16 = query->out_dtype == HIRA_BF16 ? 1 : 0;
         // the search kernel folds the partials itself (the last workgroup of a tree to arrive
         // does it) unless the caller asks for the second launch
         p.fold_dvl = round_pow2((tree->vdim + 3) / 4);
@@ -377,7 +381,7 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
         const int ng = 256 / dvl;
         const size_t smem = (size_t)ng * (tree->vdim + 1) * sizeof(float);
         hipLaunchKernelGGL(merge_kernel, dim3(query->num_q_heads), dim3(256), smem, s, p.part_m,
-                           p.part_l, p.part_acc, P, tree->vdim, dvl, out->attn_out);
+                           p.part_l, p.part_acc, P, tree->vdim, dvl, p.attn_out, p.out_bf16);
         HIRA_CHECK_LAUNCH("merge kernel");
     }
     return HIRA_OK;

@@ -1414,7 +1414,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             const float Lg = s_red[2 * g + 1];
             float sum = 0.0f;
             for (int r = 0; r < n_grp; ++r) sum += red[(size_t)r * G * D + t];
-            p.attn_out[(size_t)(hoff + g) * D + (t % D)] = Lg > 0.0f ? sum / Lg : 0.0f;
+            store_out(p.attn_out, p.out_bf16, (size_t)(hoff + g) * D + (t % D), Lg > 0.0f ? sum / Lg : 0.0f);
         }
         tline.stamp(kTlFoldDone);
         return;
@@ -1462,7 +1462,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             }
         }
         const float inv = Lg > 0.0f ? 1.0f / Lg : 0.0f;
-        p.attn_out[(size_t)head * D + e] = (s0 + s1) * inv;
+        store_out(p.attn_out, p.out_bf16, (size_t)head * D + e, (s0 + s1) * inv);
     }
     tline.stamp(kTlFoldDone);
 }

@@ -22,14 +22,14 @@ namespace hira {
 
 constexpr int kUnroll = 8;  // row loads in flight per lane while scanning a block
 
-// out[:] = sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p over the P partials of one head, by
+// out[o0 ..] = sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p over the P partials of one head, by
 // all threads of the workgroup (a multiple of 64, at least dvl).  Thread t owns four columns of
 // the output (t % dvl) for the partials p = t / dvl (mod ng).  rows: (ng, Dv + 1) floats of
 // LDS, red: one float per wave.  The partials are read with device-scope loads: they may have
 // been written by workgroups behind another L2.
 __device__ __forceinline__ void fold_partials(const float* pm, const float* pl, const float* pa,
-                                              int P, int Dv, int dvl, float* out, float* rows,
-                                              float* red) {
+                                              int P, int Dv, int dvl, void* out, int out_bf16,
+                                              size_t o0, float* rows, float* red) {
     auto ld = [](const float* q) {
         return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
@@ -42,7 +42,7 @@ __device__ __forceinline__ void fold_partials(const float* pm, const float* pl, 
     float M = red[0];
     for (int w = 1; w < nw; ++w) M = fmaxf(M, red[w]);
     if (M == -INFINITY) {  // nothing selected for this head (uniform)
-        for (int e = t; e < Dv; e += nt) out[e] = 0.0f;
+        for (int e = t; e < Dv; e += nt) store_out(out, out_bf16, o0 + e, 0.0f);
         return;
     }
     const int ng = nt / dvl;
@@ -72,7 +72,7 @@ __device__ __forceinline__ void fold_partials(const float* pm, const float* pl, 
     for (int e = t; e < Dv; e += nt) {
         float sum = 0.0f;
         for (int g = 0; g < ng; ++g) sum += rows[(size_t)g * (Dv + 1) + e];
-        out[e] = sum / ltot;
+        store_out(out, out_bf16, o0 + e, sum / ltot);
     }
 }
 
@@ -629,7 +629,7 @@ __global__ __launch_bounds__(256) void search_kernel(const SearchParams p) {
         const int head = by_group ? hoff + g : p.tree_q_heads[hoff + g];
         fold_partials(p.part_m + (size_t)head * p.num_parts, p.part_l + (size_t)head * p.num_parts,
                       p.part_acc + (size_t)head * p.num_parts * Dv, p.num_parts, Dv, p.fold_dvl,
-                      p.attn_out + (size_t)head * Dv, smem, s_fold_red);
+                      p.attn_out, p.out_bf16, (size_t)head * Dv, smem, s_fold_red);
         __syncthreads();
     }
 }

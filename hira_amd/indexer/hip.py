@@ -53,6 +53,23 @@ def from_tiled(x: torch.Tensor) -> torch.Tensor:
     return v.contiguous().reshape(t, r, d)
 
 
+_MINUS_INF = 0xFF800000  # the bits of an fp32 -inf
+
+
+def _fill_arrays(specs, trees: int) -> None:
+    """One launch over several (T, rows, ...) arrays: (dst, src or None, rows to copy from src, first
+    row to fill, fill word).  What growing an index, or clearing its padding, takes."""
+    arr = (_lib.HiraArray * len(specs))()
+    for a, (dst, src, rows, fill_from, word) in zip(arr, specs):
+        row = dst.element_size() * (dst.shape[2] if dst.ndim == 3 else 1)
+        a.dst, a.dst_stride = dst.data_ptr(), dst.shape[1] * row
+        if src is not None:
+            a.src, a.src_stride = src.data_ptr(), src.shape[1] * row
+        a.copy_bytes, a.fill_from, a.fill = rows * row, fill_from * row, word
+    _lib.check(_lib.lib().hira_fill_arrays(arr, len(specs), trees,
+                                           _lib.stream_of(specs[0][0].get_device())))
+
+
 def level_sizes(n: int, bf: int, num_levels: int) -> List[int]:
     """Slots per level of the padded tree: K_1 = ceil(n/bf), K_l = ceil(K_{l-1}/bf); the
     root keeps K_root nodes and each lower level has bf slots per node of the level above
@@ -260,8 +277,21 @@ class HIPIndexer(BaseIndexer):
         return self._level(self.counts, 2)
 
     # ------------------------------------------------------------------ device state
+    def _arrays(self):
+        """(attribute, level or None, fill word) of every array a tree's slots own."""
+        out = [("keys_buf", None, 0), ("perm", None, 0xFFFFFFFF)]
+        if self.values_buf is not None:
+            out.append(("values_buf", None, 0))
+        if self.q8:
+            out += [("keys8", None, 0), ("keps", None, 0)]
+        for l in range(1, self.num_levels):
+            out += [("centers", l, 0), ("radii", l, _MINUS_INF), ("counts", l, 0)]
+        return out
+
     def _allocate(self, batch: int, heads: int, n: int, dim: int, vdim: int,
-                  dtype: torch.dtype) -> None:
+                  dtype: torch.dtype, *, used: bool = False) -> None:
+        """Fresh level arrays for n keys a tree.  used: every slot in use (size) is about to be
+        written by a build, so only the padding behind them is cleared."""
         if dtype not in _DTYPES:
             raise ValueError(f"unsupported key dtype {dtype}: use float32 or bfloat16")
         esize = 4 if dtype == torch.float32 else 2
@@ -281,21 +311,34 @@ class HIPIndexer(BaseIndexer):
         if self.tiled:
             self.cap = [-(-c // 16) * 16 for c in self.cap]
         dev, t = self.device, self.num_trees
-        self.keys_buf = torch.zeros((t, self.cap[0], dim), dtype=dtype, device=dev)
-        self.values_buf = (
-            torch.zeros((t, self.cap[0], vdim), dtype=dtype, device=dev) if vdim else None)
-        self.perm = torch.full((t, self.cap[0]), -1, dtype=torch.int32, device=dev)
+
+        def new(l, width, dt):
+            return torch.empty((t, self.cap[l]) + ((width,) if width else ()), dtype=dt, device=dev)
+
+        self.keys_buf = new(0, dim, dtype)
+        self.values_buf = new(0, vdim, dtype) if vdim else None
+        self.perm = new(0, 0, torch.int32)
         self.keys8 = self.kscale = self.keps = None
         if self.q8:
-            self.keys8 = torch.zeros((t, self.cap[0], dim), dtype=torch.int8, device=dev)
+            self.keys8 = new(0, dim, torch.int8)
             self.kscale = torch.ones((t, dim), dtype=torch.float32, device=dev)
-            self.keps = torch.zeros((t, self.cap[1]), dtype=torch.float32, device=dev)
+            self.keps = new(1, 0, torch.float32)
         self.centers, self.radii, self.counts = [None], [None], [None]
         for l in range(1, nl):
-            self.centers.append(torch.zeros((t, self.cap[l], dim), dtype=dtype, device=dev))
-            self.radii.append(
-                torch.full((t, self.cap[l]), float("-inf"), dtype=torch.float32, device=dev))
-            self.counts.append(torch.zeros((t, self.cap[l]), dtype=torch.int32, device=dev))
+            self.centers.append(new(l, dim, dtype))
+            self.radii.append(new(l, 0, torch.float32))
+            self.counts.append(new(l, 0, torch.int32))
+        specs = []
+        for name, l, word in self._arrays():
+            a = getattr(self, name) if l is None else getattr(self, name)[l]
+            # (a tiled matrix: a row is spread over its tile, so from the tile's first row on)
+            size = self.size[1 if name == "keps" else (l or 0)] if used else 0
+            if self.tiled and name in ("keys_buf", "keys8", "centers"):
+                size = size // 16 * 16
+            if size < a.shape[1]:
+                specs.append((a, None, 0, size, word))
+        if specs:
+            _fill_arrays(specs, t)
         self._tree_struct = None
         self._state = None
 
@@ -326,6 +369,12 @@ class HIPIndexer(BaseIndexer):
                 t.counts[l] = self.counts[l].data_ptr()
             self._tree_struct = t
         return self._tree_struct
+
+    def _sizes_changed(self) -> None:
+        """self.size moved and nothing else: a new struct that differs in the sizes."""
+        if self._tree_struct is not None:
+            t = self._tree_struct = _lib.HiraTree.from_buffer_copy(self._tree_struct)
+            t.size[: self.num_levels] = self.size
 
     # ------------------------------------------------------------------ layouts
     @classmethod
@@ -515,7 +564,7 @@ class HIPIndexer(BaseIndexer):
         b, h, n, d = keys.shape
         dtype = self.storage_dtype(keys.dtype)
         vdim = 0 if values is None else int(values.shape[-1])
-        self._allocate(b, h, n, d, vdim, dtype)
+        self._allocate(b, h, n, d, vdim, dtype, used=True)
         kin = keys.to(device=self.device, dtype=dtype).reshape(b * h, n, d).contiguous()
         vin = None
         if values is not None:
@@ -569,12 +618,12 @@ class HIPIndexer(BaseIndexer):
     def _grow(self, need: List[int]) -> None:
         """Re-allocate the level arrays with at least `need` slots (doubling), keeping the
         contents.  A tile of 16 rows is contiguous, so a tiled matrix grows by rows too."""
+        if all(n <= c for n, c in zip(need, self.cap)):
+            return
         caps = []
         for l, (c, n) in enumerate(zip(self.cap, need)):
             c2 = c if n <= c else max(n, 2 * c)
             caps.append(-(-c2 // 16) * 16 if self.tiled else c2)
-        if caps == self.cap:
-            return
         if self._unsynced_room > 0:
             # a launch captured by begin_unsynced holds the current pointers
             raise RuntimeError(
@@ -582,23 +631,18 @@ class HIPIndexer(BaseIndexer):
                 "(a captured decode step holds its pointers): call sync_sizes() first, or "
                 "reserve() more room before begin_unsynced()")
 
-        def grown(old, cap, fill):
-            new = torch.full((old.shape[0], cap) + tuple(old.shape[2:]), fill, dtype=old.dtype,
-                             device=old.device)
-            new[:, : old.shape[1]] = old
-            return new
-
-        self.keys_buf = grown(self.keys_buf, caps[0], 0)
-        if self.values_buf is not None:
-            self.values_buf = grown(self.values_buf, caps[0], 0)
-        self.perm = grown(self.perm, caps[0], -1)
-        if self.q8:
-            self.keys8 = grown(self.keys8, caps[0], 0)
-            self.keps = grown(self.keps, caps[1], 0)
-        for l in range(1, self.num_levels):
-            self.centers[l] = grown(self.centers[l], caps[l], 0)
-            self.radii[l] = grown(self.radii[l], caps[l], float("-inf"))
-            self.counts[l] = grown(self.counts[l], caps[l], 0)
+        specs = []
+        for name, l, word in self._arrays():
+            old = getattr(self, name) if l is None else getattr(self, name)[l]
+            rows = caps[1 if name == "keps" else (l or 0)]
+            new = torch.empty((old.shape[0], rows) + tuple(old.shape[2:]), dtype=old.dtype,
+                              device=old.device)
+            specs.append((new, old, old.shape[1], old.shape[1], word))
+            if l is None:
+                setattr(self, name, new)
+            else:
+                getattr(self, name)[l] = new
+        _fill_arrays(specs, self.num_trees)  # (`specs` keeps the old arrays until the launch is queued)
         self.cap = caps
         self._tree_struct = None
 
@@ -720,6 +764,12 @@ class HIPIndexer(BaseIndexer):
             self.quantize(first, count)
         return self
 
+    def _rows(self, x: torch.Tensor, t: int, m: int, width: int) -> torch.Tensor:
+        """(T, m, width) rows, contiguous, in the storage type and on the index's device."""
+        if x.dtype is self.dtype and x.get_device() == self.keys_buf.get_device() and x.is_contiguous():
+            return x
+        return x.to(device=self.device, dtype=self.dtype).reshape(t, m, width).contiguous()
+
     def reserve(self, appends: int) -> "HIPIndexer":
         """Room for `appends` more keys per tree, so that updates up to that many do not
         re-allocate: device pointers (and with them captured graphs and plans) stay valid."""
@@ -744,7 +794,7 @@ class HIPIndexer(BaseIndexer):
         self._exact_size = list(self.size)
         self.size = [need[1] * self.branching_factor] + list(need[1:])
         self._unsynced_room = int(appends)
-        self._tree_struct = None
+        self._sizes_changed()
 
     def note_unsynced(self, m: int) -> None:
         """`m` keys per tree were appended by a launch outside ``update`` (a graph replay)."""
@@ -773,18 +823,18 @@ class HIPIndexer(BaseIndexer):
         return self
 
     def _adopt_state(self, st: torch.Tensor) -> None:
-        if int(st[:, _lib.HIRA_MAX_LEVELS + 1].max()) != 0:
+        most = st.numpy().max(axis=0).tolist()
+        if most[_lib.HIRA_MAX_LEVELS + 1] != 0:
             raise RuntimeError("index update ran out of capacity")
         if self.num_levels == 1:
-            self.size = [self.num_keys]
+            size = [self.num_keys]
         else:
-            size = [0] * self.num_levels
-            for l in range(1, self.num_levels):
-                size[l] = int(st[:, l].max())
+            size = most[: self.num_levels]
             size[0] = size[1] * self.branching_factor
-            self.size = size
         self._pending, self._exact_size = 0, None
-        self._tree_struct = None
+        if size != self.size:
+            self.size = size
+            self._sizes_changed()
 
     def update(self, new_keys: torch.Tensor, new_values: Optional[torch.Tensor] = None, *,
                sync: bool = True):
@@ -834,17 +884,14 @@ class HIPIndexer(BaseIndexer):
         t = self.num_trees
         if self._state is None:
             self._init_state()
-        kin = new_keys.to(device=self.device, dtype=self.dtype).reshape(t, m, self.dim).contiguous()
-        vin = None
-        if new_values is not None:
-            vin = new_values.to(device=self.device, dtype=self.dtype).reshape(
-                t, m, self.vdim).contiguous()
+        kin = self._rows(new_keys, t, m, self.dim)
+        vin = None if new_values is None else self._rows(new_values, t, m, self.vdim)
         tree = self.tree_struct()
-        stream = _lib.current_stream(self.device)
         rc = _lib.lib().hira_update(C.byref(tree), kin.data_ptr(),
                                     None if vin is None else vin.data_ptr(), m,
-                                    self._state.data_ptr(), stream)
-        _lib.check(rc)
+                                    self._state.data_ptr(), _lib.stream_of(self.keys_buf.get_device()))
+        if rc:
+            _lib.check(rc)
         self.num_keys += m
         if sync:
             self._adopt_state(self._state.cpu())
@@ -859,7 +906,7 @@ class HIPIndexer(BaseIndexer):
         bound = [max(a, b) for a, b in zip(bound, self.size)]  # (bounds never shrink)
         if bound != self.size:
             self.size = bound
-            self._tree_struct = None
+            self._sizes_changed()
         return self
 
     _warmed: set = set()

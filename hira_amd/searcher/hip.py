@@ -392,7 +392,8 @@ class HIPSearcher(BaseSearcher):
 
 class DecodePlan:
     """One fused search + attention call per ``run``: ``query`` (H_q, D) in the tree dtype,
-    ``threshold`` (H_q,) fp32 and ``out`` (H_q, Dv) fp32 must be contiguous device tensors."""
+    ``threshold`` (H_q,) fp32 and ``out`` (H_q, Dv) fp32 (or bf16: the fp32 sums are then rounded
+    where they are written) must be contiguous device tensors."""
 
     def __init__(self, searcher: HIPSearcher, indexer, num_q_heads: int, scaling, q_head_to_kv,
                  stats):
@@ -408,6 +409,7 @@ class DecodePlan:
         self._keep = (off, heads, stats)
         self.query = _lib.HiraQuery(num_q_heads, None, None, self.scaling.data_ptr(),
                                     off.data_ptr(), heads.data_ptr(), gmax, group)
+        self._out_type = _lib.out_dtype_of(self.query)
         self.out = _lib.HiraSearchOut()
         self.out.stats = None if stats is None else stats.data_ptr()
         self.launch = searcher.launch
@@ -450,6 +452,7 @@ class DecodePlan:
         q.q = query.data_ptr()
         q.tau = threshold.data_ptr()
         self.out.attn_out = out.data_ptr()
+        self._out_type.value = _lib.HIRA_BF16 if out.dtype is torch.bfloat16 else _lib.HIRA_F32
         if stream is None:
             stream = _lib.stream_of(self._dev)
         qu = None

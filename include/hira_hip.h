@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define HIRA_ABI_VERSION 7
+#define HIRA_ABI_VERSION 8
 #define HIRA_MAX_LEVELS 8
 #define HIRA_STATS_COLS (HIRA_MAX_LEVELS + 3) /* counters per tree a search can fill in */
 
@@ -93,6 +93,9 @@ typedef struct HiraTree {
  * including maps that are not monotone (tests/test_cpp_kernels.py:529-565). */
 typedef struct HiraQuery {
     int32_t num_q_heads;         /* H_q (all sequences) */
+    int32_t out_dtype;           /* type hira_search writes attn_out in: HIRA_F32 (0, what callers
+                                    that know no such field leave here) or HIRA_BF16 (rounded
+                                    once, from the fp32 sums) */
     const void* q;               /* (H_q, D), tree dtype */
     const float* tau;            /* (H_q) threshold on the raw score q.k */
     const float* scaling;        /* (H_q) factor applied to returned scores / softmax logits */
@@ -136,7 +139,8 @@ typedef struct HiraSearchOut {
     int32_t* sel_count;
     int32_t sel_cap;
     float dense_fill_value;
-    /* (3) attention over the selected keys (+ the queue): out (H_q, Dv) fp32.
+    /* (3) attention over the selected keys (+ the queue): out (H_q, Dv), fp32 (or bf16 where
+     *     HiraQuery.out_dtype says so: the pointer then leads to 2-byte numbers).
      *     Heads with an empty selection get zeros. */
     float* attn_out;
     /* optional counters, zeroed by the caller: (T, HIRA_STATS_COLS) uint64:
@@ -342,6 +346,45 @@ int hira_update_threshold(const HiraTree* tree, const void* new_keys, const void
 int hira_sparse_attention(const HiraTree* tree, const HiraQuery* query, const int32_t* sel_index,
                           const float* sel_score, const int32_t* sel_count, int32_t sel_cap,
                           float* attn_out, void* stream);
+
+/*
+ * The m new keys and values of every tree (contiguous (T, m, D) / (T, m, Dv)) into rows
+ * [at, at + m) of a queue (T, cap, D) / (T, cap, Dv), one launch: the append to the decode queue
+ * that the reference makes by concatenating tensors (cache/hira_cache.py:121-140).
+ * vdim = 0: no values.  Rows are a multiple of 16 bytes.
+ */
+int hira_enqueue(void* queue_keys, void* queue_values, int32_t dtype, int32_t num_trees, int32_t cap,
+                 int32_t at, int32_t m, int32_t dim, int32_t vdim, const void* new_keys,
+                 const void* new_values, void* stream);
+
+/*
+ * rows[t][slot_host[i]] = from[t][from_host[i]] for every tree t and i < n: members of a key
+ * sample replaced by newer keys (the sample behind cache/hira_config.py:20-22 of the reference).
+ * rows (T, rows_per_tree, D), from (T, from_stride, D) of which the first from_rows are in use;
+ * the two index lists are HOST arrays, read before the call returns; no slot twice.
+ */
+int hira_replace_rows(void* rows, int32_t dtype, int32_t dim, int32_t num_trees, int32_t rows_per_tree,
+                      const void* from, int32_t from_rows, int32_t from_stride, const int32_t* slot_host,
+                      const int32_t* from_host, int32_t n, void* stream);
+
+/*
+ * Up to 32 arrays of num_trees stretches each, in one launch: in every tree bytes
+ * [0, copy_bytes) come from src (strides in bytes), bytes [fill_from, dst_stride) become the
+ * 32-bit word `fill`; bytes between the two are left alone.  What growing the level arrays of an
+ * index is made of, and clearing the padding of freshly allocated ones.  All numbers are
+ * multiples of 4.
+ */
+typedef struct HiraArray {
+    void* dst;
+    const void* src;      /* NULL where copy_bytes is 0 */
+    int64_t dst_stride;   /* bytes per tree */
+    int64_t src_stride;
+    int64_t copy_bytes;
+    int64_t fill_from;    /* >= copy_bytes; dst_stride (or more): nothing is filled */
+    uint32_t fill;
+    int32_t reserved_;
+} HiraArray;
+int hira_fill_arrays(const HiraArray* arrays_host, int32_t n, int32_t num_trees, void* stream);
 
 #ifdef __cplusplus
 }

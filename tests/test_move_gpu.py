@@ -1,0 +1,88 @@
+"""hira_enqueue, hira_replace_rows and hira_fill_arrays against the same moves in torch, and the
+bf16 attention output against the rounded fp32 one."""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("trees,cap,at,m,d,dv", [(1, 1, 0, 1, 8, 8), (3, 7, 2, 5, 80, 24), (128, 16, 15, 1, 128, 128),
+                                                 (2, 300, 0, 300, 256, 8)])
+def test_enqueue(dtype, trees, cap, at, m, d, dv, gpu_device):
+    from hira_amd import _lib
+
+    qk, qv = torch.randn(trees, cap, d, device="cuda").to(dtype), torch.randn(trees, cap, dv, device="cuda").to(dtype)
+    k, v = torch.randn(trees, m, d, device="cuda").to(dtype), torch.randn(trees, m, dv, device="cuda").to(dtype)
+    wk, wv = qk.clone(), qv.clone()
+    wk[:, at:at + m], wv[:, at:at + m] = k, v
+    code = _lib.HIRA_F32 if dtype == torch.float32 else _lib.HIRA_BF16
+    _lib.check(_lib.lib().hira_enqueue(qk.data_ptr(), qv.data_ptr(), code, trees, cap, at, m, d, dv, k.data_ptr(),
+                                       v.data_ptr(), _lib.current_stream(qk.device)))
+    assert torch.equal(qk, wk) and torch.equal(qv, wv)
+    with pytest.raises(ValueError):
+        _lib.check(_lib.lib().hira_enqueue(qk.data_ptr(), qv.data_ptr(), code, trees, cap, cap, m, d, dv, k.data_ptr(),
+                                           v.data_ptr(), _lib.current_stream(qk.device)))
+
+
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 300])
+def test_replace_rows(n, gpu_device):
+    from hira_amd import _lib
+
+    trees, rows, d, m, stride = 3, 400, 72, 310, 320
+    a = torch.randn(trees, rows, d, device="cuda").to(torch.bfloat16)
+    src = torch.randn(trees, stride, d, device="cuda").to(torch.bfloat16)
+    slot, frm = torch.randperm(rows)[:n], torch.randint(0, m, (n,))
+    want = a.clone()
+    want[:, slot.cuda()] = src[:, frm.cuda()]
+    arr = C.c_int32 * n
+    args = (a.data_ptr(), _lib.HIRA_BF16, d, trees, rows, src.data_ptr(), m, stride, arr(*slot.tolist()),
+            arr(*frm.tolist()))
+    _lib.check(_lib.lib().hira_replace_rows(*args, n, _lib.current_stream(a.device)))
+    assert torch.equal(a, want)
+    bad = args[:-2] + (arr(*([rows] * n)), args[-1])
+    with pytest.raises(ValueError):
+        _lib.check(_lib.lib().hira_replace_rows(*bad, n, _lib.current_stream(a.device)))
+
+
+@pytest.mark.parametrize("trees", [1, 5])
+def test_fill_arrays(trees, gpu_device):
+    from hira_amd.indexer.hip import _fill_arrays
+
+    specs, wants = [], []
+    # (rows, width, rows of the source, rows copied, first row filled): whole stretches and ragged ones,
+    # 16-byte rows and single words, a gap that stays as it is
+    for rows, width, have, copied, first in [(5000, 64, 4000, 4000, 4000), (7, 0, 3, 3, 3), (40000, 0, 0, 0, 11),
+                                             (33, 8, 40, 20, 25), (1, 4, 0, 0, 0), (9000, 0, 9000, 9000, 9000)]:
+        shape = (trees, rows) + ((width,) if width else ())
+        dst = torch.randn(shape, device="cuda")
+        src = torch.randn((trees, have) + shape[2:], device="cuda") if have else None
+        want = dst.clone()
+        if copied:
+            want[:, :copied] = src[:, :copied]
+        want[:, first:] = float("-inf")
+        specs.append((dst, src, copied, first, 0xFF800000))
+        wants.append(want)
+    _fill_arrays(specs, trees)
+    for (dst, *_), want in zip(specs, wants):
+        assert torch.equal(dst, want)
+
+
+@pytest.mark.parametrize("dtype,d,bf,group", [(torch.bfloat16, 128, 32, 4), (torch.bfloat16, 64, 10, 4),
+                                              (torch.float32, 80, 10, 1), (torch.bfloat16, 128, 32, 8)])
+def test_output_in_bf16_is_the_rounded_fp32_output(dtype, d, bf, group, gpu_device):
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    keys, vals = (torch.randn(1, 2, 3000, d, device="cuda").to(dtype) for _ in range(2))
+    idx = HIPIndexer(3, 1, bf).build(keys, vals)
+    q = torch.randn(2 * group, d, device="cuda").to(dtype)
+    tau = torch.full((2 * group,), 2.0, device="cuda") * d ** 0.5
+    plan = HIPSearcher().plan_attention(idx, 2 * group, scaling=torch.full((2 * group,), d ** -0.5))
+    a = torch.empty(2 * group, d, device="cuda")
+    b = torch.empty(2 * group, d, device="cuda", dtype=torch.bfloat16)
+    plan.run(q, tau, a)
+    plan.run(q, tau, b)
+    assert bool((a != 0).any()) and torch.equal(b, a.to(torch.bfloat16))
