@@ -19,6 +19,7 @@ struct SearchParams {
     int32_t size[HIRA_MAX_LEVELS];
     int32_t cap[HIRA_MAX_LEVELS];
     int32_t num_levels, bf, dim, vdim;
+    uint32_t bf_magic;  // ceil(2^32 / bf): n / bf = the high word of n * bf_magic (bf > 1, n < 2^26)
     int32_t layout;  // of the centers: HIRA_ROW_MAJOR or HIRA_TILE16
     int32_t key_layout;  // of the keys
     const int8_t* keys8;  // HIRA_TILE16_Q8: the 8-bit shadow, its steps and error bounds
@@ -36,7 +37,7 @@ struct SearchParams {
     const void* queue_values;
     int32_t queue_len, queue_cap;
     // work split
-    int32_t nodes_per_wave;  // level-1 nodes (or pseudo blocks) per wave; MFMA kernel: tiles per workgroup
+    int32_t nodes_per_wave;  // vector-ALU kernel: level-1 nodes (or pseudo blocks) a workgroup walks, per wave of it; MFMA kernel: tiles per workgroup
     int32_t tree_blocks;     // workgroups that walk the tree; the rest scan the queue
     int32_t key_policy;      // MFMA kernel: which cache policy the scan's loads use (0: default,
                              // 1: key tiles non-temporal, 2: value rows too), by the launch's size
@@ -60,7 +61,6 @@ struct SearchParams {
     void* attn_out;     // (H_q, Dv): written by the kernel itself when `done` is set
     int32_t out_bf16;   // its type: bf16, else fp32
     int32_t* done;      // (T, passes) arrival counters, zero between launches; NULL: no fold
-    int32_t fold_dvl;   // vector-ALU kernel's fold: threads per partial (four columns each)
     unsigned long long* stats;
 };
 
@@ -78,7 +78,6 @@ struct SearchPlan {
     int nodes_per_wave;
     int num_nodes, num_queue_blocks;
     int tree_blocks, queue_blocks, head_chunks;
-    int gate_steps;   // vector-ALU kernel: steps of gates a wave batches (1 or 4)
     size_t smem;
 };
 

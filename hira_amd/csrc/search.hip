@@ -88,7 +88,6 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
             HIRA_CHECK_ARG(t->cap[l] % 16 == 0, "tiled layout: cap[%d]=%d not a multiple of 16",
                            l, t->cap[l]);
     }
-    plan->gate_steps = 1;
     plan->num_queue_blocks = 0;
     if (queue && queue->keys && queue->len > 0) {
         HIRA_CHECK_ARG(queue->len <= queue->cap, "queue len %d > cap %d", queue->len,
@@ -165,48 +164,40 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
     }
     plan->gmax = q->max_group <= 1 ? 1 : (q->max_group <= 4 ? 4 : 8);
     plan->head_chunks = (q->max_group + plan->gmax - 1) / plan->gmax;
-    int threads = launch && launch->block_threads ? launch->block_threads : 256;
-    HIRA_CHECK_ARG(threads == 64 || threads == 128 || threads == 256,
-                   "block_threads %d must be 64, 128 or 256", threads);
+    const size_t state = (size_t)plan->gmax * (lpr * epl + 2) * sizeof(float);  // of a wave, in LDS
+    // eight waves a workgroup (as long as their states fit the LDS that needs no asking)
+    int threads = launch && launch->block_threads
+                      ? launch->block_threads
+                      : (kVecThreads / 64 * state <= 48 * 1024 ? kVecThreads : 256);
+    HIRA_CHECK_ARG(threads == 64 || threads == 128 || threads == 256 || threads == kVecThreads,
+                   "block_threads %d must be 64, 128, 256 or %d", threads, kVecThreads);
     plan->threads = threads;
-    const int rpw = 64 / lpr;
-    // nodes that hold very few keys (a step of gates leads to at most 8 rows): a wave batches
-    // two or four steps of gates and scans the batch's keys as one block -- as long as that
-    // leaves the chip's 256 compute units eight waves each (below that the longer chain of a
-    // wave costs more than its trips save)
-    if (t->num_levels >= 2 && t->bf * rpw <= 8) {
-        const long long steps = (long long)t->num_trees * plan->head_chunks *
-                                ((t->size[1] + rpw - 1) / rpw);
-        plan->gate_steps = steps >= 4 * 2048 ? 4 : (steps >= 2 * 2048 ? 2 : 1);
-        if (launch && launch->nodes_per_wave)
-            plan->gate_steps = launch->nodes_per_wave > rpw ? 4 : 1;
-    }
-    int npw = launch && launch->nodes_per_wave ? launch->nodes_per_wave : rpw * plan->gate_steps;
-    HIRA_CHECK_ARG(npw >= 1, "nodes_per_wave %d", npw);
+    const int waves = threads / 64;
     plan->num_nodes = t->num_levels >= 2 ? t->size[1]
                                          : (t->size[0] + kPseudoBlock - 1) / kPseudoBlock;
-    // large trees under attention: a wave takes more steps of nodes, towards 64 partials a head to
-    // fold, as long as the launch keeps two workgroups per compute unit (8 trees x 65536 fp32
-    // keys, fan-out 32, 4 heads a tree: 256 partials 127 us, 128: 103, 64: 94, 32: 158; one such
-    // tree alone: 256 partials 47 us, 128: 55, 64: 82)
-    if (attn && !(launch && launch->nodes_per_wave) && plan->gate_steps == 1) {
-        const int wpb = threads / 64;
-        auto parts = [&](int n) { return (plan->num_nodes + wpb * n - 1) / (wpb * n); };
-        while (parts(npw) > 64 &&
-               (int64_t)t->num_trees * plan->head_chunks * parts(2 * npw) >= 2 * compute_units())
-            npw *= 2;
+    int npw = launch ? launch->nodes_per_wave : 0;
+    HIRA_CHECK_ARG(npw >= 0, "nodes_per_wave %d", npw);
+    if (npw == 0) {
+        // nodes per workgroup: under attention one workgroup per compute unit (every one leaves a
+        // partial per head to fold), otherwise two; no fewer than 128 rows, what its waves scan in
+        // one block each
+        const int rows = t->num_levels >= 2 ? t->bf : kPseudoBlock;
+        const int64_t all = (int64_t)plan->num_nodes * t->num_trees * plan->head_chunks;
+        const int64_t wgs = (attn ? 1 : 2) * compute_units();
+        int64_t per = (all + wgs - 1) / wgs;
+        const int64_t least = (128 + rows - 1) / rows;
+        if (per < least) per = least;
+        npw = (int)((per + waves - 1) / waves);
     }
     plan->nodes_per_wave = npw;
-    const int per_block = (threads / 64) * npw;
+    const int per_block = waves * npw;
     plan->tree_blocks = (plan->num_nodes + per_block - 1) / per_block;
     plan->queue_blocks = (plan->num_queue_blocks + per_block - 1) / per_block;
-    plan->smem = (size_t)(threads / 64) * plan->gmax * (lpr * epl + 2) * sizeof(float);
-    {   // the fold of the last workgroup reuses the same LDS: (ng, vdim + 1) floats
-        const int dvl = round_pow2((t->vdim + 3) / 4);
-        if (dvl > 0 && dvl <= threads) {
-            const size_t fold = (size_t)(threads / dvl) * (t->vdim + 1) * sizeof(float);
-            if (fold > plan->smem) plan->smem = fold;
-        }
+    plan->smem = (size_t)(threads / 64) * state;
+    {   // the fold of the last workgroup reuses the same LDS
+        const size_t heads_parts = (size_t)plan->gmax * (plan->tree_blocks + plan->queue_blocks);
+        const size_t fold = 2 * heads_parts * sizeof(float) + (size_t)threads * 4 * sizeof(float);
+        if (heads_parts <= kVecFoldMax && fold > plan->smem) plan->smem = fold;
     }
     return HIRA_OK;
 }
@@ -281,6 +272,7 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
     }
     p.num_levels = tree->num_levels;
     p.bf = tree->bf;
+    p.bf_magic = tree->bf > 1 ? (uint32_t)((((uint64_t)1 << 32) + tree->bf - 1) / tree->bf) : 0;
     p.dim = tree->dim;
     p.vdim = tree->vdim;
     p.layout = center_layout_of(tree->layout);
@@ -349,12 +341,9 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
         p.out_bf16 = query->out_dtype == HIRA_BF16 ? 1 : 0;
         // the search kernel folds the partials itself (the last workgroup of a tree to arrive
         // does it) unless the caller asks for the second launch
-        p.fold_dvl = round_pow2((tree->vdim + 3) / 4);
-        // (vector-ALU kernel: its last workgroup folds the heads of its pass one after the
-        // other, which only pays for a single head with few partials; the second launch has
-        // a workgroup per head)
-        const bool can_fold = plan.kernel == 2 ||
-                              (p.fold_dvl <= plan.threads && plan.gmax == 1 && P <= 64);
+        const bool can_fold = plan.kernel == 2 || (plan.gmax * P <= kVecFoldMax &&
+                                                   (size_t)query->num_q_heads * P * tree->vdim * sizeof(float) <
+                                                       ((size_t)1 << 31));
         if (can_fold && !(launch && launch->separate_merge))
             p.done = reinterpret_cast<int32_t*>(workspace);
     }

@@ -1,16 +1,25 @@
-// Halfspace range search over the fixed-fan-out ball tree, fused with sparse attention.
+// Halfspace range search over the fixed-fan-out ball tree, fused with sparse attention, on the
+// vector units: any row width, fan-out, depth and type (the matrix-core kernel next door takes
+// the bf16 shapes it is made for).
 //
-// One launch covers every tree and every query head.  A wavefront owns a run of
-// consecutive level-1 nodes ("leaf parents").  For each of them it re-derives the gates of
-// the node's ancestors (levels L-1 .. 2: one row each, shared by whole subtrees and served
-// by the caches), then the node's own gate, and then scans the node's child block of keys.
-// No global frontier is exchanged between workgroups, so the walk needs no grid-wide
-// synchronisation and a pruned subtree costs its waves one or two row reads.
+// One launch covers every tree and every query head.  A workgroup owns a run of consecutive
+// level-1 nodes ("leaf parents") of one tree and takes them up to kBatch at a time, in three steps:
+//   gates   all rows the batch needs -- its nodes and, once each, their ancestors at every level --
+//           are asked for together and dealt out over the workgroup's lane groups; each leaves a
+//           word in LDS saying for which heads it passes;
+//   list    a node survives for the heads that it and all its ancestors pass for: one wave puts the
+//           survivors side by side in LDS;
+//   scan    the survivors' key slots, end to end, are dealt out over the waves in blocks of up to 64
+//           rows; the values of a block's selected rows are asked for together.
+// So a launch is a chain of four trips to memory (arguments, gates, keys, values) plus the hand-off
+// of the partials, whatever the fan-out, and a pruned node costs nothing behind its gate.  No
+// global frontier is exchanged between workgroups.  (Before, every wave walked nodes of its own:
+// each gate repeated the ancestors' rows, and short nodes left most lanes without a row.)
 //
 // Lane layout: a row of D elements is 16-byte chunks; LPR lanes hold one row (lane % LPR =
-// chunk), so a wave reads 64/LPR rows per 128-bit load instruction, fully coalesced.  The
-// G query heads that share the tree (GQA group) are scored against every chunk that is
-// loaded: one HBM read of a centroid or key row serves the whole group.
+// chunk), so a wave reads RPW = 64/LPR rows per 128-bit load instruction, fully coalesced.  The
+// query heads that share the tree (GQA group) are scored against every chunk that is loaded: one
+// HBM read of a centroid or key row serves the whole group.
 //
 // Semantics (reference: kernels/cpp/torch_ext_v3.cpp:172-242, with the conservative
 // non-unit-query bound of searcher/cpu.py:61-63): keep a node when q.c + ||q||*r >= tau,
@@ -20,8 +29,84 @@
 
 namespace hira {
 
-constexpr int kUnroll = 8;  // row loads in flight per lane while scanning a block
+constexpr int kVecThreads = 512;  // workgroup size, at most
+constexpr int kBatch = 64;        // level-1 nodes a workgroup gates together
+// rows of a block that a wave scans at once: eight loads a lane (with eight heads a pass as many as
+// the registers have room for: four, two of bf16), at most 64 rows
+constexpr int vec_rows(int rpw, int gmax, int epl) {
+    const int r = (gmax <= 4 ? 8 : 16 / epl) * rpw;
+    return r < 64 ? r : 64;
+}
 
+// ---- sums over the LPR lanes of a row, many at once ------------------------------------------
+// Every lane comes with NV partial sums (value u * GMAX + g: row u of the lane group's block, head
+// g).  Summing each over the lanes by itself takes log2(LPR) steps a value; here a step over a lane
+// bit also halves the values a lane goes on with (lanes with the bit clear keep the first half,
+// the others the second), until a lane holds the sums of its own max(NV / LPR, 1) values: 77
+// instructions for 32 values over 32 lanes instead of 192 and as many LDS permutes.
+constexpr int vec_kept(int nv, int lpr) { return nv >= lpr ? nv / lpr : 1; }
+// first value whose sum lane `j` of a lane group ends up with
+constexpr int vec_value_of(int j, int nv, int lpr) {
+    int v = 0, n = nv;
+    for (int bit = lpr / 2; bit >= 1 && n > 1; bit /= 2) {
+        n /= 2;
+        if (j & bit) v += n;
+    }
+    return v;
+}
+// lanes of a group that hold a value nobody below them holds too (fewer values than lanes)
+constexpr bool vec_is_owner(int j, int nv, int lpr) {
+    for (int i = 0; i < j; ++i)
+        if (vec_value_of(i, nv, lpr) == vec_value_of(j, nv, lpr)) return false;
+    return true;
+}
+// lanes of the wave that hold a value of row u of their group's block
+template <int GMAX, int NV, int LPR>
+struct VecLanes {
+    uint64_t row[NV / GMAX], any;
+    constexpr VecLanes() : row{}, any(0) {
+        for (int j = 0; j < LPR; ++j) {
+            if (!vec_is_owner(j, NV, LPR)) continue;
+            for (int v = vec_value_of(j, NV, LPR), n = 0; n < vec_kept(NV, LPR); ++v, ++n)
+                for (int r = 0; r < 64 / LPR; ++r) row[v / GMAX] |= 1ull << (r * LPR + j);
+        }
+        for (int u = 0; u < NV / GMAX; ++u) any |= row[u];
+    }
+};
+
+template <int N, int BIT>
+__device__ __forceinline__ void reduce_step(float* v, int lane) {
+    // partner: a lane that differs in BIT (and maybe in lower bits)
+    constexpr int CTRL = BIT == 8 ? 0x140 : BIT == 4 ? 0x141 : BIT == 2 ? 0x1B : 0xB1;
+    if constexpr (N > 1) {
+        constexpr int H = N / 2;
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            if constexpr (BIT >= 16) {
+                const auto r = BIT == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + H]), false, false)
+                                         : __builtin_amdgcn_permlane16_swap(__float_as_uint(v[i]), __float_as_uint(v[i + H]), false, false);
+                v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+            } else {
+                const bool up = (lane & BIT) != 0;
+                const float keep = up ? v[i + H] : v[i], send = up ? v[i] : v[i + H];
+                v[i] = keep + dpp_move<CTRL>(send);
+            }
+        }
+    } else if constexpr (BIT >= 16) {
+        const auto r = BIT == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[0]), false, false)
+                                 : __builtin_amdgcn_permlane16_swap(__float_as_uint(v[0]), __float_as_uint(v[0]), false, false);
+        v[0] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        v[0] += dpp_move<CTRL>(v[0]);
+    }
+}
+template <int N, int BIT>
+__device__ __forceinline__ void reduce_scatter(float* v, int lane) {
+    reduce_step<N, BIT>(v, lane);
+    if constexpr (BIT > 1) reduce_scatter<(N > 1 ? N / 2 : 1), BIT / 2>(v, lane);
+}
+
+// The fold as the work of one workgroup per head (a launch of its own):
 // out[o0 ..] = sum_p 2^(m_p - M) acc_p / sum_p 2^(m_p - M) l_p over the P partials of one head, by
 // all threads of the workgroup (a multiple of 64, at least dvl).  Thread t owns four columns of
 // the output (t % dvl) for the partials p = t / dvl (mod ng).  rows: (ng, Dv + 1) floats of
@@ -50,14 +135,26 @@ __device__ __forceinline__ void fold_partials(const float* pm, const float* pl, 
     float a[4] = {0.f, 0.f, 0.f, 0.f};
     float lsum = 0.0f;
     const bool lane_ok = li * 4 < Dv;
-    for (int i = gi; i < P; i += ng) {
-        const float mp = ld(pm + i);
-        if (mp == -INFINITY) continue;
-        const float w = exp2f(mp - M);
-        lsum += w * ld(pl + i);
-        if (lane_ok) {
+    // (four partials in flight; nothing is asked for only after something else has arrived.  A
+    // partial without a selected key may hold anything: it is masked, not multiplied)
+    constexpr int U = 4;
+    for (int i0 = gi; i0 < P; i0 += U * ng) {
+        float m[U], l[U], v[U][4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) a[c] += w * ld(pa + (size_t)i * Dv + li * 4 + c);
+        for (int u = 0; u < U; ++u) {
+            const int i = min(i0 + u * ng, P - 1);
+            m[u] = ld(pm + i);
+            l[u] = ld(pl + i);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[u][c] = lane_ok ? ld(pa + (size_t)i * Dv + li * 4 + c) : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (i0 + u * ng >= P || m[u] == -INFINITY) continue;
+            const float w = exp2f(m[u] - M);
+            lsum += w * l[u];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) a[c] += w * v[u][c];
         }
     }
     float* row = rows + (size_t)gi * (Dv + 1);
@@ -76,14 +173,130 @@ __device__ __forceinline__ void fold_partials(const float* pm, const float* pl, 
     }
 }
 
-// NGX: steps of gates (RPW nodes each) a wave batches: 4 where a node holds few keys, else 1.
-template <typename T, int LPR, int GMAX, int NGX>
-__global__ __launch_bounds__(256) void search_kernel(const SearchParams p) {
+// The fold by the last workgroup of a tree and pass to arrive: its G heads side by side, in two
+// trips to memory.  A wave per head takes the partials' maxima and sums and lists those that hold
+// anything with their weights; then a thread owns four output columns of a head and every
+// n_grp-th listed partial, eight 16-byte loads in flight; the groups' sums meet in LDS.  (One head
+// after the other, as the fold above would do it, took 7 us more at 4 heads x 64 partials than a
+// second launch with a workgroup per head; side by side it takes less than that launch.)
+//   lds: 2 G P floats, then blockDim.x * 4
+constexpr int kVecFoldMax = 4096;  // G * P at most
+__device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int G, float* lds) {
+    __shared__ float s_l[8];
+    __shared__ int s_n[8];
+    auto ld = [](const float* q) {
+        return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = blockDim.x >> 6;
+    const int P = p.num_parts, Dv = p.vdim;
+    int* list = reinterpret_cast<int*>(lds);   // (G, P)
+    float* wts = lds + (size_t)G * P;          // (G, P)
+    float* red = lds + 2 * (size_t)G * P;      // (n_grp, G * Dv)
+    for (int g = wave; g < G; g += nw) {  // uniform in the wave
+        const int head = p.group_size > 0 ? hoff + g : p.tree_q_heads[hoff + g];
+        const float* pm = p.part_m + (size_t)head * P;
+        const float* pl = p.part_l + (size_t)head * P;
+        float mx = -INFINITY;
+        for (int i = lane; i < P; i += 64) mx = fmaxf(mx, ld(pm + i));
+        const float m0 = lane < P ? ld(pm + lane) : -INFINITY, l0 = lane < P ? ld(pl + lane) : 0.0f;
+        mx = wave_max(mx);
+        float ls = 0.0f;
+        int n = 0;
+        for (int i0 = 0; i0 < P; i0 += 64) {  // uniform
+            const int i = i0 + lane;
+            const float m = i0 == 0 ? m0 : (i < P ? ld(pm + i) : -INFINITY);
+            const float l = i0 == 0 ? l0 : (i < P ? ld(pl + i) : 0.0f);
+            const float w = m > -INFINITY ? exp2f(m - mx) : 0.0f;
+            ls += w * l;
+            const bool nz = w > 0.0f && l > 0.0f;
+            const unsigned long long bal = __ballot(nz);
+            if (nz) {
+                const int k = n + __popcll(bal & ((1ull << lane) - 1ull));
+                list[g * P + k] = i;
+                wts[g * P + k] = w;
+            }
+            n += __popcll(bal);
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) ls += __shfl_xor(ls, off, 64);
+        if (lane == 0) {
+            s_l[g] = ls;
+            s_n[g] = n;
+        }
+    }
+    __syncthreads();
+    const int quads = Dv / 4, items = G * quads;
+    const int n_grp = max((int)blockDim.x / items, 1);
+    for (int i0 = 0; i0 < items; i0 += blockDim.x) {  // uniform; once unless G * Dv > 4 threads
+        const int item = n_grp > 1 ? t % items : i0 + t, grp = n_grp > 1 ? t / items : 0;
+        if (item < items && grp < n_grp) {
+            const int g = item / quads, qd = item % quads;
+            const int head = p.group_size > 0 ? hoff + g : p.tree_q_heads[hoff + g];
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(p.part_acc), 0, 0x7fffffff, 0x00020000);
+            const unsigned col0 = ((unsigned)head * (unsigned)P * (unsigned)Dv + 4u * (unsigned)qd) * 4u;
+            const int n = s_n[g];
+            float sx = 0.0f, sy = 0.0f, sz = 0.0f, sw = 0.0f;
+            for (int k0 = grp; k0 < n; k0 += 8 * n_grp) {
+                u32x4 v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)  // (16: the device-scope bit)
+                    v[u] = __builtin_amdgcn_raw_buffer_load_b128(
+                        rsrc, col0 + (unsigned)list[g * P + min(k0 + u * n_grp, n - 1)] * (unsigned)(Dv * 4), 0, 16);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const float w = k0 + u * n_grp < n ? wts[g * P + k0 + u * n_grp] : 0.0f;
+                    sx += w * __uint_as_float(v[u].x);
+                    sy += w * __uint_as_float(v[u].y);
+                    sz += w * __uint_as_float(v[u].z);
+                    sw += w * __uint_as_float(v[u].w);
+                }
+            }
+            if (n_grp > 1) {
+                float4* r = reinterpret_cast<float4*>(red + (size_t)grp * items * 4 + item * 4);
+                *r = make_float4(sx, sy, sz, sw);
+            } else {
+                const float L = s_l[g];
+                const float o[4] = {sx, sy, sz, sw};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    store_out(p.attn_out, p.out_bf16, (size_t)head * Dv + qd * 4 + c, L > 0.0f ? o[c] / L : 0.0f);
+            }
+        }
+    }
+    if (n_grp == 1) return;
+    __syncthreads();
+    for (int e = t; e < items * 4; e += blockDim.x) {
+        const int g = e / Dv;
+        const int head = p.group_size > 0 ? hoff + g : p.tree_q_heads[hoff + g];
+        float sum = 0.0f;
+        for (int r = 0; r < n_grp; ++r) sum += red[(size_t)r * items * 4 + e];
+        const float L = s_l[g];
+        store_out(p.attn_out, p.out_bf16, (size_t)head * Dv + (e - g * Dv), L > 0.0f ? sum / L : 0.0f);
+    }
+}
+
+template <typename T, int LPR, int GMAX>
+__global__ __launch_bounds__(kVecThreads) __attribute__((amdgpu_waves_per_eu(GMAX == 1 ? 3 : 2)))
+void search_kernel(const SearchParams p) {
     constexpr int EPL = Elem<T>::kPerChunk;
     constexpr int RPW = kWave / LPR;  // rows per wave-wide load
     constexpr int DVP = LPR * EPL;    // widest row a lane group can hold
+    constexpr int KU = vec_rows(RPW, GMAX, EPL) / RPW;  // row loads in flight per lane
+    constexpr int ROWS = KU * RPW;
+    constexpr int NV = KU * GMAX;                  // scores a lane group makes of a block
+    constexpr int KEPT = vec_kept(NV, LPR);
+    constexpr VecLanes<GMAX, NV, LPR> LANES{};
+    constexpr int WAVES = kVecThreads / 64;
 
     extern __shared__ float smem[];
+    // logits, then weights, of a block's rows (-inf / 0: not selected): the wave's lanes share the
+    // work on them, and no lane keeps its rows' scores while the values are on their way
+    __shared__ __attribute__((aligned(16))) float s_tab[WAVES][ROWS * GMAX];
+    __shared__ uint32_t s_pass[HIRA_MAX_LEVELS][kBatch + 1];  // heads a row passes for | 1 << 31: not empty
+    __shared__ uint32_t s_list[kBatch];  // survivors: node - first | child count << 8 | heads << 16
+    __shared__ int s_count;
 
     touch_kernel_arguments();
     const int lane = lane_id();
@@ -106,484 +319,370 @@ __global__ __launch_bounds__(256) void search_kernel(const SearchParams p) {
     const int G = min(GMAX, (by_group ? (tree + 1) * p.group_size : p.tree_q_off[tree + 1]) - hoff);
     if (G <= 0) return;  // uniform for the workgroup
     const unsigned gmask = (1u << G) - 1u;
-
-    // ---- queries of the group: this lane's chunk of each, plus tau, scaling, ||q|| ----
-    int qh[GMAX];
-    float qf[GMAX][EPL];
-    float tau[GMAX], sc[GMAX], qn[GMAX];
-#pragma unroll
-    for (int g = 0; g < GMAX; ++g) {
-        qh[g] = (g < G) ? (by_group ? hoff + g : p.tree_q_heads[hoff + g]) : 0;
-        uint4 raw = make_uint4(0, 0, 0, 0);
-        if (g < G && chunk_ok) raw = load_chunk<T>(p.q, (size_t)qh[g] * D, ch);
-        unpack<T>(raw, qf[g]);
-        tau[g] = (g < G) ? p.tau[qh[g]] : INFINITY;
-        sc[g] = (g < G) ? p.scaling[qh[g]] : 0.0f;
-        float ss = 0.0f;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) ss += qf[g][e] * qf[g][e];
-        qn[g] = sqrtf(group_sum<LPR>(ss));
-    }
-
-    // ---- attention state of this lane group -------------------------------------------
-    float acc[GMAX][EPL];
-    float mrun[GMAX], lrun[GMAX];
-#pragma unroll
-    for (int g = 0; g < GMAX; ++g) {
-        mrun[g] = -INFINITY;
-        lrun[g] = 0.0f;
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
-    }
-
-    unsigned long long st_nodes[HIRA_MAX_LEVELS];
-    unsigned long long st_sel_any = 0, st_sel_pairs = 0;
-#pragma unroll
-    for (int l = 0; l < HIRA_MAX_LEVELS; ++l) st_nodes[l] = 0;
+    auto head_of = [&](int g) { return by_group ? hoff + g : p.tree_q_heads[hoff + g]; };
 
     const bool is_queue = (int)blockIdx.x >= p.tree_blocks;
     const int blk = is_queue ? (int)blockIdx.x - p.tree_blocks : (int)blockIdx.x;
     const int n_nodes = is_queue ? p.num_queue_blocks : p.num_nodes;
     const bool real_nodes = !is_queue && L >= 2;
-    const int node_first = (blk * nwaves + wave) * p.nodes_per_wave;
-    const int node_last = min(node_first + p.nodes_per_wave, n_nodes);
+    const int node_first = blk * nwaves * p.nodes_per_wave;
+    const int node_last = min(node_first + nwaves * p.nodes_per_wave, n_nodes);
+
+    // ---- queries of the group: this lane's chunk of each (asked for here, first used at the gates) ----
+    uint4 qraw[GMAX];
+    float tau[GMAX];
+#pragma unroll
+    for (int g = 0; g < GMAX; ++g) {
+        qraw[g] = make_uint4(0, 0, 0, 0);
+        tau[g] = INFINITY;
+        if (g < G) {
+            const int h = head_of(g);
+            if (chunk_ok) qraw[g] = load_chunk<T>(p.q, (size_t)h * D, ch);
+            tau[g] = p.tau[h];
+        }
+    }
+    // threshold, scale and head of the values whose sums this lane ends up with
+    int vfirst = 0;  // vec_value_of(ch)
+    {
+        int n = NV;
+#pragma unroll
+        for (int bit = LPR / 2; bit >= 1; bit /= 2)
+            if (n > 1) {
+                n /= 2;
+                if (ch & bit) vfirst += n;
+            }
+    }
+    const int my_u = vfirst / GMAX, my_g = vfirst % GMAX;  // row of the block, first head
+    float my_tau[KEPT], my_sc[KEPT];
+    int my_h[KEPT];
+#pragma unroll
+    for (int i = 0; i < KEPT; ++i) {
+        const int g = my_g + i % GMAX;
+        my_h[i] = g < G ? head_of(g) : 0;
+        my_tau[i] = g < G ? p.tau[my_h[i]] : INFINITY;
+        my_sc[i] = g < G ? p.scaling[my_h[i]] : 0.0f;
+    }
 
     const void* kbase = is_queue ? p.queue_keys : p.keys;
     const void* vbase = is_queue ? p.queue_values : p.values;
     const size_t krow0 = (size_t)tree * (is_queue ? p.queue_cap : p.cap[0]);
     const int n_rows = is_queue ? p.queue_len : p.size[0];
     const int block_rows = real_nodes ? p.bf : kPseudoBlock;
+    const float inv_rows = 1.0f / (float)block_rows;
     const int klayout = is_queue ? HIRA_ROW_MAJOR : p.key_layout;
+    auto over_bf = [&](unsigned n) { return p.bf == 1 ? n : __umulhi(n, p.bf_magic); };  // n / bf
 
-    // The dense output's stretch under this wave's nodes starts out as the fill value; the
-    // scores of selected keys follow from the same wave, behind these stores.
-    if (p.dense_fill && !is_queue && node_first < node_last) {
-        const int r0 = node_first * block_rows, r1 = min(node_last * block_rows, n_rows);
+    // counters, straight to memory (registers are worth more here than the few calls that count)
+    auto count = [&](int i, unsigned n) {
+        atomicAdd(p.stats + (size_t)tree * HIRA_STATS_COLS + i, (unsigned long long)n);
+    };
+
+    // ---- attention state: each lane group's sums under the wave's maximum; lane l keeps maximum
+    // and denominator of head l % GMAX (the denominator in parts) ----------------------------
+    float acc[GMAX][EPL];
+    float m_run = -INFINITY, l_run = 0.0f;
 #pragma unroll
-        for (int g = 0; g < GMAX; ++g)
-            if (g < G)
-                for (int i = r0 + lane; i < r1; i += kWave)
-                    p.dense[(int64_t)qh[g] * p.dense_stride + i] = p.dense_fill_value;
-    }
+    for (int g = 0; g < GMAX; ++g)
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
+    float qf[GMAX][EPL];
 
-    if constexpr (NGX == 1) {
-        for (int n0 = node_first; n0 < node_last; n0 += RPW) {
-            // -------- gates: lane group rg owns node n0 + rg -----------------------------
-            const int node = n0 + rg;
-            const bool node_ok = node < node_last;
-            unsigned alive = node_ok ? gmask : 0u;
-            int cnt = 0;
-            if (real_nodes) {
-                // the node's own row, radius and child count, and its ancestors at levels L-1 .. 2:
-                // independent loads, issued together (the node's are wasted when an ancestor
-                // prunes it, which costs bandwidth the gates have to spare, not a trip to memory)
-                uint4 raw1 = make_uint4(0, 0, 0, 0);
-                float rad1 = 0.0f;
-                int cnt1 = 0;
-                if (node_ok) {
-                    const size_t r = (size_t)tree * p.cap[1] + node;
-                    if (chunk_ok)
-                        raw1 = load_row_chunk<T>(p.centers[1], p.layout, D, (size_t)tree * p.cap[1],
-                                                 node, ch);
-                    rad1 = p.radii[1][r];
-                    cnt1 = p.counts[1][r];
+    for (int n0 = node_first; n0 < node_last; n0 += kBatch) {  // uniform in the workgroup
+        const int nb = min(kBatch, node_last - n0);
+        if (n0 > node_first) __syncthreads();  // (the list of the batch before is done with)
+        int cnt = 0;  // child count of node n0 + thread
+        if ((int)threadIdx.x < nb)
+            cnt = real_nodes ? p.counts[1][(size_t)tree * p.cap[1] + n0 + threadIdx.x]
+                             : min(kPseudoBlock, n_rows - (n0 + (int)threadIdx.x) * kPseudoBlock);
+        // ---- gates: rows of levels 1 and 2 over all waves, every level above on a wave of its own ----
+        if (real_nodes) {
+            constexpr int KA = 4;  // level-1 rows a lane group has in flight
+            const int r0 = wave * RPW + rg, rstep = nwaves * RPW;
+            auto ask = [&](int l, int first, int rows, int r, uint4& raw, float& rad) {
+                raw = make_uint4(0, 0, 0, 0);
+                rad = -INFINITY;
+                if (r < rows) {
+                    const size_t t0 = (size_t)tree * p.cap[l];
+                    if (chunk_ok) raw = load_row_chunk<T>(p.centers[l], p.layout, D, t0, first + r, ch);
+                    rad = p.radii[l][t0 + first + r];
                 }
-                uint4 araw[HIRA_MAX_LEVELS - 2];
-                float arad[HIRA_MAX_LEVELS - 2];
-                int aid[HIRA_MAX_LEVELS - 2];
-                {
-                    int id = node;
-    #pragma unroll
-                    for (int l = 2; l < HIRA_MAX_LEVELS; ++l) {
-                        id /= p.bf;
-                        aid[l - 2] = id;
-                        araw[l - 2] = make_uint4(0, 0, 0, 0);
-                        arad[l - 2] = 0.0f;
-                        if (l < L && node_ok) {
-                            const size_t r = (size_t)tree * p.cap[l] + id;
-                            if (chunk_ok)
-                                araw[l - 2] = load_row_chunk<T>(p.centers[l], p.layout, D,
-                                                                (size_t)tree * p.cap[l], id, ch);
-                            arad[l - 2] = p.radii[l][r];
+            };
+            uint4 raw1[KA], raw2;
+            float rad1[KA], rad2;
+#pragma unroll
+            for (int k = 0; k < KA; ++k) ask(1, n0, nb, r0 + k * rstep, raw1[k], rad1[k]);
+            const int first2 = (int)over_bf((unsigned)n0);
+            const int rows2 = L > 2 ? (int)over_bf((unsigned)(n0 + nb - 1)) - first2 + 1 : 0;
+            ask(2, first2, rows2, r0, raw2, rad2);
+            float qn[GMAX];
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) {
+                unpack<T>(qraw[g], qf[g]);
+                float ss = 0.0f;
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) ss += qf[g][e] * qf[g][e];
+                qn[g] = sqrtf(group_sum<LPR>(ss));
+            }
+            auto judge = [&](int l, int rows, int r, const uint4& raw, float rad) {
+                float kf[EPL];
+                unpack<T>(raw, kf);
+                unsigned pass = 0;
+#pragma unroll
+                for (int g = 0; g < GMAX; ++g) {
+                    float d = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
+                    d = group_sum<LPR>(d);
+                    if (d + qn[g] * rad >= tau[g]) pass |= 1u << g;
+                }
+                if (ch == 0 && r < rows) s_pass[l][r] = pass | (rad > -INFINITY ? 0x80000000u : 0u);
+            };
+            if (wave * RPW < rows2) judge(2, rows2, r0, raw2, rad2);  // (conditions: uniform in the wave)
+#pragma unroll
+            for (int k = 0; k < KA; ++k)
+                if (wave * RPW + k * rstep < nb) judge(1, nb, r0 + k * rstep, raw1[k], rad1[k]);
+#pragma unroll 1
+            for (int r = r0 + rstep; r - rg < rows2; r += rstep) {  // (fan-outs of one or two)
+                ask(2, first2, rows2, r, raw2, rad2);
+                judge(2, rows2, r, raw2, rad2);
+            }
+#pragma unroll 1
+            for (int r = r0 + KA * rstep; r - rg < nb; r += rstep) {  // (small workgroups)
+                ask(1, n0, nb, r, raw2, rad2);
+                judge(1, nb, r, raw2, rad2);
+            }
+            int fl = first2, ll = first2 + rows2 - 1;  // first and last row of level l - 1
+#pragma unroll 1
+            for (int l = 3; l < L; ++l) {
+                fl = (int)over_bf((unsigned)fl);
+                ll = (int)over_bf((unsigned)ll);
+                if ((l - 2) % nwaves != wave) continue;
+                const int rows = ll - fl + 1;
+#pragma unroll 1
+                for (int r = rg; r - rg < rows; r += RPW) {
+                    ask(l, fl, rows, r, raw2, rad2);
+                    judge(l, rows, r, raw2, rad2);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) unpack<T>(qraw[g], qf[g]);
+        }
+        // The dense output's stretch under the batch starts out as the fill value; the scores of
+        // selected keys follow behind the barriers.
+        if (p.dense_fill && !is_queue) {
+            const int f0 = n0 * block_rows, f1 = min((n0 + nb) * block_rows, n_rows);
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g)
+                if (g < G) {
+                    float* row = p.dense + (int64_t)head_of(g) * p.dense_stride;
+                    for (int i = f0 + (int)threadIdx.x; i < f1; i += blockDim.x) row[i] = p.dense_fill_value;
+                }
+        }
+        __syncthreads();
+        // ---- list ---------------------------------------------------------------------------
+        if (wave == 0) {
+            unsigned alive = lane < nb ? gmask : 0u;
+            if (real_nodes && lane < nb) {
+                alive &= s_pass[1][lane];
+                int at = lane, below = n0;  // place of my ancestor in the batch, first row of the level below
+#pragma unroll 1
+                for (int l = 2; l < L; ++l) {
+                    const int fl = (int)over_bf((unsigned)below);
+                    // (places inside the batch are small: the float quotient is exact)
+                    at = (int)(((float)(below - fl * p.bf + at) + 0.5f) * inv_rows);
+                    alive &= s_pass[l][at];
+                    below = fl;
+                }
+                if (p.stats) {
+                    // a node counts where a head is alive above it, by its first level-1 descendant
+                    unsigned a = gmask;
+                    for (int l = L - 1; l >= 1; --l) {
+                        unsigned id = (unsigned)(n0 + lane), fl = (unsigned)n0;
+                        bool lead = true;
+                        for (int i = 1; i < l; ++i) {
+                            const unsigned up = over_bf(id);
+                            lead = lead && up * (unsigned)p.bf == id;
+                            id = up;
+                            fl = over_bf(fl);
                         }
+                        const uint32_t w = s_pass[l][id - fl];
+                        if (a && (w >> 31) && lead) count(l, 1);
+                        a &= w;
                     }
                 }
-                // top-down so that `alive` before level l says whether level l is evaluated
-    #pragma unroll
-                for (int l = HIRA_MAX_LEVELS - 1; l >= 2; --l) {
-                    if (l < L) {
-                        if (p.stats && alive && ch == 0 && arad[l - 2] > -INFINITY) {
-                            // count the node once: by its first level-1 descendant
-                            int span = 1;
-                            for (int t = 1; t < l; ++t) span *= p.bf;
-                            if (node % span == 0) st_nodes[l]++;
-                        }
-                        float kf[EPL];
-                        unpack<T>(araw[l - 2], kf);
-                        unsigned pass = 0;
-    #pragma unroll
-                        for (int g = 0; g < GMAX; ++g) {
-                            float d = 0.0f;
-    #pragma unroll
-                            for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
-                            d = group_sum<LPR>(d);
-                            if (d + qn[g] * arad[l - 2] >= tau[g]) pass |= 1u << g;
-                        }
-                        alive &= pass;
-                    }
-                }
-                // the level-1 node itself, only if some head is still alive above it
-                if (alive) {
-                    const float rad = rad1;
-                    cnt = cnt1;
-                    if (p.stats && ch == 0 && rad > -INFINITY) st_nodes[1]++;
-                    float kf[EPL];
-                    unpack<T>(raw1, kf);
-                    unsigned pass = 0;
-    #pragma unroll
-                    for (int g = 0; g < GMAX; ++g) {
-                        float d = 0.0f;
-    #pragma unroll
-                        for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
-                        d = group_sum<LPR>(d);
-                        if (d + qn[g] * rad >= tau[g]) pass |= 1u << g;
-                    }
-                    alive &= pass;
-                }
-            } else if (node_ok) {
-                cnt = min(kPseudoBlock, n_rows - node * kPseudoBlock);
             }
             if (cnt <= 0) alive = 0u;
-
-            // -------- scan the child blocks of the nodes that survived, one at a time -----
-    #pragma unroll 1
-            for (int b = 0; b < RPW; ++b) {
-                const unsigned am = __shfl(alive, b * LPR, 64);  // wave-uniform
-                if (am == 0u) continue;
-                const int bcnt = __shfl(cnt, b * LPR, 64);
-                const int first = (n0 + b) * block_rows;  // first key slot of the block
-                if (p.stats && lane == 0) st_nodes[0] += (unsigned long long)bcnt;
-
-    #pragma unroll 1
-                for (int i0 = 0; i0 < bcnt; i0 += RPW * kUnroll) {
-                    uint4 raw[kUnroll];
-    #pragma unroll
-                    for (int u = 0; u < kUnroll; ++u) {
-                        const int row = i0 + u * RPW + rg;
-                        raw[u] = make_uint4(0, 0, 0, 0);
-                        if (row < bcnt && chunk_ok)
-                            raw[u] = load_row_chunk<T>(kbase, klayout, D, krow0, first + row, ch);
-                    }
-    #pragma unroll
-                    for (int u = 0; u < kUnroll; ++u) {
-                        const int row = i0 + u * RPW + rg;
-                        float kf[EPL];
-                        unpack<T>(raw[u], kf);
-                        float s[GMAX];
-                        unsigned sel = 0;
-    #pragma unroll
-                        for (int g = 0; g < GMAX; ++g) {
-                            float d = 0.0f;
-    #pragma unroll
-                            for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
-                            s[g] = group_sum<LPR>(d);
-                            if (((am >> g) & 1u) && row < bcnt && (is_queue || s[g] >= tau[g]))
-                                sel |= 1u << g;
-                        }
-                        if (__ballot(sel != 0u) == 0ull) continue;  // wave-uniform
-
-                        const int slot = first + row;
-                        const bool owner = (ch == 0) && sel != 0u;
-                        if (p.stats && owner) {
-                            st_sel_any++;
-                            st_sel_pairs += (unsigned long long)__popc(sel);
-                        }
-                        if (!is_queue && (p.dense != nullptr || p.sel_count != nullptr)) {
-                            int idx = slot;
-                            if (owner && p.dense_by_position) idx = p.perm[krow0 + slot];
-    #pragma unroll
-                            for (int g = 0; g < GMAX; ++g) {
-                                const bool mine = owner && ((sel >> g) & 1u);
-                                if (p.dense != nullptr && mine)
-                                    p.dense[(int64_t)qh[g] * p.dense_stride + idx] = s[g] * sc[g];
-                                if (p.sel_count != nullptr) {
-                                    const unsigned long long bal = __ballot(mine);
-                                    if (bal != 0ull) {
-                                        int base = 0;
-                                        if (lane == 0)
-                                            base = atomicAdd(&p.sel_count[qh[g]], __popcll(bal));
-                                        base = __shfl(base, 0, 64);
-                                        const int pos =
-                                            base + __popcll(bal & ((1ull << lane) - 1ull));
-                                        if (mine && pos < p.sel_cap) {
-                                            p.sel_index[(int64_t)qh[g] * p.sel_cap + pos] = idx;
-                                            p.sel_score[(int64_t)qh[g] * p.sel_cap + pos] = s[g];
-                                        }
-                                    }
-                                }
-                            }
-                        }
-                        if (want_attn && sel != 0u) {
-                            uint4 vraw = make_uint4(0, 0, 0, 0);
-                            if (vchunk_ok) vraw = load_chunk<T>(vbase, (krow0 + slot) * Dv, ch);
-                            float vf[EPL];
-                            unpack<T>(vraw, vf);
-    #pragma unroll
-                            for (int g = 0; g < GMAX; ++g) {
-                                if ((sel >> g) & 1u) {
-                                    const float z = s[g] * sc[g] * kLog2e;
-                                    if (z > mrun[g]) {
-                                        const float f = exp2f(mrun[g] - z);
-                                        lrun[g] = lrun[g] * f + 1.0f;
-    #pragma unroll
-                                        for (int e = 0; e < EPL; ++e)
-                                            acc[g][e] = acc[g][e] * f + vf[e];
-                                        mrun[g] = z;
-                                    } else {
-                                        const float w = exp2f(z - mrun[g]);
-                                        lrun[g] += w;
-    #pragma unroll
-                                        for (int e = 0; e < EPL; ++e) acc[g][e] += w * vf[e];
-                                    }
-                                }
-                            }
-                        }
-                    }
-                }
-            }
+            if (p.stats && alive) count(0, (unsigned)cnt);
+            const unsigned long long bal = __ballot(alive != 0u);
+            if (alive) s_list[__popcll(bal & ((1ull << lane) - 1ull))] = (uint32_t)lane | ((uint32_t)cnt << 8) | (alive << 16);
+            if (lane == 0) s_count = __popcll(bal);
         }
-    } else {
-        // A wave takes its nodes NGX * RPW at a time.  All their gates first -- the loads of the NGX
-        // steps do not depend on each other, so they are in flight together -- then the key slots of
-        // the batch, which are consecutive, as ONE block: a row knows from LDS whether its node
-        // survived (and for which heads) and whether it holds a key.  With a fan-out of 4 a wave so
-        // pays two trips to memory for 32 keys instead of one per node.
-        __shared__ uint32_t s_node[4][NGX * RPW];  // heads a node survives for | child count << 16
-        constexpr int KU = kUnroll;
-        const float inv_rows = 1.0f / (float)block_rows;
-        for (int nb0 = node_first; nb0 < node_last; nb0 += NGX * RPW) {
-    #pragma unroll
-            for (int g = 0; g < NGX; ++g) {
-                // -------- gates: lane group rg owns node nb0 + g * RPW + rg -------------------
-                const int node = nb0 + g * RPW + rg;
-                const bool node_ok = node < node_last;
-                unsigned alive = node_ok ? gmask : 0u;
-                int cnt = 0;
-                if (real_nodes) {
-                    // the node's own row, radius and child count, and its ancestors at levels L-1 .. 2:
-                    // independent loads, issued together (the node's are wasted when an ancestor
-                    // prunes it, which costs bandwidth the gates have to spare, not a trip to memory)
-                    uint4 raw1 = make_uint4(0, 0, 0, 0);
-                    float rad1 = 0.0f;
-                    int cnt1 = 0;
-                    if (node_ok) {
-                        const size_t r = (size_t)tree * p.cap[1] + node;
-                        if (chunk_ok)
-                            raw1 = load_row_chunk<T>(p.centers[1], p.layout, D, (size_t)tree * p.cap[1],
-                                                     node, ch);
-                        rad1 = p.radii[1][r];
-                        cnt1 = p.counts[1][r];
-                    }
-                    uint4 araw[HIRA_MAX_LEVELS - 2];
-                    float arad[HIRA_MAX_LEVELS - 2];
-                    int aid[HIRA_MAX_LEVELS - 2];
-                    {
-                        int id = node;
-        #pragma unroll
-                        for (int l = 2; l < HIRA_MAX_LEVELS; ++l) {
-                            id /= p.bf;
-                            aid[l - 2] = id;
-                            araw[l - 2] = make_uint4(0, 0, 0, 0);
-                            arad[l - 2] = 0.0f;
-                            if (l < L && node_ok) {
-                                const size_t r = (size_t)tree * p.cap[l] + id;
-                                if (chunk_ok)
-                                    araw[l - 2] = load_row_chunk<T>(p.centers[l], p.layout, D,
-                                                                    (size_t)tree * p.cap[l], id, ch);
-                                arad[l - 2] = p.radii[l][r];
-                            }
-                        }
-                    }
-                    // top-down so that `alive` before level l says whether level l is evaluated
-        #pragma unroll
-                    for (int l = HIRA_MAX_LEVELS - 1; l >= 2; --l) {
-                        if (l < L) {
-                            if (p.stats && alive && ch == 0 && arad[l - 2] > -INFINITY) {
-                                // count the node once: by its first level-1 descendant
-                                int span = 1;
-                                for (int t = 1; t < l; ++t) span *= p.bf;
-                                if (node % span == 0) st_nodes[l]++;
-                            }
-                            float kf[EPL];
-                            unpack<T>(araw[l - 2], kf);
-                            unsigned pass = 0;
-        #pragma unroll
-                            for (int g = 0; g < GMAX; ++g) {
-                                float d = 0.0f;
-        #pragma unroll
-                                for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
-                                d = group_sum<LPR>(d);
-                                if (d + qn[g] * arad[l - 2] >= tau[g]) pass |= 1u << g;
-                            }
-                            alive &= pass;
-                        }
-                    }
-                    // the level-1 node itself, only if some head is still alive above it
-                    if (alive) {
-                        const float rad = rad1;
-                        cnt = cnt1;
-                        if (p.stats && ch == 0 && rad > -INFINITY) st_nodes[1]++;
-                        float kf[EPL];
-                        unpack<T>(raw1, kf);
-                        unsigned pass = 0;
-        #pragma unroll
-                        for (int g = 0; g < GMAX; ++g) {
-                            float d = 0.0f;
-        #pragma unroll
-                            for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
-                            d = group_sum<LPR>(d);
-                            if (d + qn[g] * rad >= tau[g]) pass |= 1u << g;
-                        }
-                        alive &= pass;
-                    }
-                } else if (node_ok) {
-                    cnt = min(kPseudoBlock, n_rows - node * kPseudoBlock);
-                }
-                if (cnt <= 0) alive = 0u;
-                if (p.stats && ch == 0 && alive) st_nodes[0] += (unsigned long long)cnt;
-                if (ch == 0) s_node[wave][g * RPW + rg] = (uint32_t)alive | ((uint32_t)cnt << 16);
-            }
-            __builtin_amdgcn_wave_barrier();  // the rows below read what other lanes just wrote
-            const int batch_nodes = min(NGX * RPW, node_last - nb0);
-            const int nrows = batch_nodes * block_rows;
-            const int first = nb0 * block_rows;  // first key slot of the batch
-            {
-    #pragma unroll 1
-                for (int i0 = 0; i0 < nrows; i0 += RPW * KU) {
-                    uint4 raw[KU];
-                    unsigned am_u[KU];
-                    bool any = false;
-    #pragma unroll
-                    for (int u = 0; u < KU; ++u) {
-                        const int row = i0 + u * RPW + rg;
-                        // (rows of a batch stay far below 2^22: the float quotient is exact enough)
-                        const int k = min((int)(((float)row + 0.5f) * inv_rows), NGX * RPW - 1);
-                        const uint32_t info = row < nrows ? s_node[wave][k] : 0u;
-                        const bool holds = row - k * block_rows < (int)(info >> 16);
-                        am_u[u] = holds ? (info & 0xFFFFu) : 0u;
-                        any = any || am_u[u] != 0u;
-                        raw[u] = make_uint4(0, 0, 0, 0);
-                        if (am_u[u] != 0u && chunk_ok)
-                            raw[u] = load_row_chunk<T>(kbase, klayout, D, krow0, first + row, ch);
-                    }
-                    if (__ballot(any) == 0ull) continue;  // wave-uniform: nothing alive in these rows
-    #pragma unroll
-                    for (int u = 0; u < KU; ++u) {
-                        const int row = i0 + u * RPW + rg;
-                        const unsigned am = am_u[u];
-                        float kf[EPL];
-                        unpack<T>(raw[u], kf);
-                        float s[GMAX];
-                        unsigned sel = 0;
-    #pragma unroll
-                        for (int g = 0; g < GMAX; ++g) {
-                            float d = 0.0f;
-    #pragma unroll
-                            for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
-                            s[g] = group_sum<LPR>(d);
-                            if (((am >> g) & 1u) && (is_queue || s[g] >= tau[g]))
-                                sel |= 1u << g;
-                        }
-                        if (__ballot(sel != 0u) == 0ull) continue;  // wave-uniform
-
-                        const int slot = first + row;
-                        const bool owner = (ch == 0) && sel != 0u;
-                        if (p.stats && owner) {
-                            st_sel_any++;
-                            st_sel_pairs += (unsigned long long)__popc(sel);
-                        }
-                        if (!is_queue && (p.dense != nullptr || p.sel_count != nullptr)) {
-                            int idx = slot;
-                            if (owner && p.dense_by_position) idx = p.perm[krow0 + slot];
-    #pragma unroll
-                            for (int g = 0; g < GMAX; ++g) {
-                                const bool mine = owner && ((sel >> g) & 1u);
-                                if (p.dense != nullptr && mine)
-                                    p.dense[(int64_t)qh[g] * p.dense_stride + idx] = s[g] * sc[g];
-                                if (p.sel_count != nullptr) {
-                                    const unsigned long long bal = __ballot(mine);
-                                    if (bal != 0ull) {
-                                        int base = 0;
-                                        if (lane == 0)
-                                            base = atomicAdd(&p.sel_count[qh[g]], __popcll(bal));
-                                        base = __shfl(base, 0, 64);
-                                        const int pos =
-                                            base + __popcll(bal & ((1ull << lane) - 1ull));
-                                        if (mine && pos < p.sel_cap) {
-                                            p.sel_index[(int64_t)qh[g] * p.sel_cap + pos] = idx;
-                                            p.sel_score[(int64_t)qh[g] * p.sel_cap + pos] = s[g];
-                                        }
-                                    }
-                                }
-                            }
-                        }
-                        if (want_attn && sel != 0u) {
-                            uint4 vraw = make_uint4(0, 0, 0, 0);
-                            if (vchunk_ok) vraw = load_chunk<T>(vbase, (krow0 + slot) * Dv, ch);
-                            float vf[EPL];
-                            unpack<T>(vraw, vf);
-    #pragma unroll
-                            for (int g = 0; g < GMAX; ++g) {
-                                if ((sel >> g) & 1u) {
-                                    const float z = s[g] * sc[g] * kLog2e;
-                                    if (z > mrun[g]) {
-                                        const float f = exp2f(mrun[g] - z);
-                                        lrun[g] = lrun[g] * f + 1.0f;
-    #pragma unroll
-                                        for (int e = 0; e < EPL; ++e)
-                                            acc[g][e] = acc[g][e] * f + vf[e];
-                                        mrun[g] = z;
-                                    } else {
-                                        const float w = exp2f(z - mrun[g]);
-                                        lrun[g] += w;
-    #pragma unroll
-                                        for (int e = 0; e < EPL; ++e) acc[g][e] += w * vf[e];
-                                    }
-                                }
-                            }
-                        }
-                    }
-                }
-            }
-        }
-    }
-
-    if (p.stats) {
-        unsigned long long* st = p.stats + (size_t)tree * HIRA_STATS_COLS;
+        __syncthreads();
+        // ---- scan ---------------------------------------------------------------------------
+        const int nrows = s_count * block_rows;
+        float* tab = s_tab[wave];
+        // row `row` of the survivors' rows: its key slot, the heads it may be selected for (0: none)
+        auto row_info = [&](int row, int& slot) -> unsigned {
+            // (rows of a batch stay far below 2^22: the float quotient is exact enough)
+            const int k = min((int)(((float)row + 0.5f) * inv_rows), kBatch - 1);
+            const uint32_t info = row < nrows ? s_list[k] : 0u;
+            const int j = row - k * block_rows;
+            slot = (n0 + (int)(info & 0xFFu)) * block_rows + j;
+            return j < (int)((info >> 8) & 0xFFu) ? info >> 16 : 0u;
+        };
+#pragma unroll 1
+        for (int i0 = wave * ROWS; i0 < nrows; i0 += nwaves * ROWS) {
+            uint4 raw[KU];
+            int slot[KU];
 #pragma unroll
-        for (int l = 0; l < HIRA_MAX_LEVELS; ++l)
-            if (st_nodes[l]) atomicAdd(&st[l], st_nodes[l]);
-        if (st_sel_any) atomicAdd(&st[HIRA_MAX_LEVELS], st_sel_any);
-        if (st_sel_pairs) atomicAdd(&st[HIRA_MAX_LEVELS + 1], st_sel_pairs);
+            for (int u = 0; u < KU; ++u) {
+                const unsigned am = row_info(i0 + u * RPW + rg, slot[u]);
+                raw[u] = make_uint4(0, 0, 0, 0);
+                if (am != 0u && chunk_ok) raw[u] = load_row_chunk<T>(kbase, klayout, D, krow0, slot[u], ch);
+            }
+            float s[NV];
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                float kf[EPL];
+                unpack<T>(raw[u], kf);
+#pragma unroll
+                for (int g = 0; g < GMAX; ++g) {
+                    float d = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
+                    s[u * GMAX + g] = d;
+                }
+            }
+            reduce_scatter<NV, LPR / 2>(s, lane);
+            // this lane's sums: row my_u of its group's block, heads my_g ...
+            int my_slot;
+            const unsigned my_am = row_info(i0 + my_u * RPW + rg, my_slot);
+            unsigned sel = 0;  // bit i: value i
+#pragma unroll
+            for (int i = 0; i < KEPT; ++i)
+                if (((my_am >> (my_g + i)) & 1u) && (is_queue || s[i] >= my_tau[i])) sel |= 1u << i;
+            const bool owner = LANES.any == ~0ull || ((LANES.any >> lane) & 1ull);
+            const uint64_t B = __ballot(owner && sel != 0u);  // lanes that hold a selected score
+            if (B == 0ull) continue;  // uniform in the wave
+            if (p.stats) {
+                // a key is selected where any of its heads is: every row once
+#pragma unroll
+                for (int u = 0; u < KU; ++u) {
+                    const uint64_t lanes = B & LANES.row[u];
+                    for (int r = 0; r < RPW; ++r) {
+                        const uint64_t group = LPR == 64 ? ~0ull : ((1ull << (LPR & 63)) - 1ull) << (r * LPR);
+                        if (lane == 0 && (lanes & group)) count(HIRA_MAX_LEVELS, 1);
+                    }
+                }
+                if (owner && sel) count(HIRA_MAX_LEVELS + 1, (unsigned)__popc(sel));
+            }
+            if (!is_queue && (p.dense != nullptr || p.sel_count != nullptr)) {
+                int idx = my_slot;
+                if (owner && sel && p.dense_by_position) idx = p.perm[krow0 + my_slot];
+                if (p.dense != nullptr && owner) {
+#pragma unroll
+                    for (int i = 0; i < KEPT; ++i)
+                        if ((sel >> i) & 1u) p.dense[(int64_t)my_h[i] * p.dense_stride + idx] = s[i] * my_sc[i];
+                }
+                if (p.sel_count != nullptr) {
+#pragma unroll
+                    for (int i = 0; i < KEPT; ++i) {
+                        const uint64_t Bi = __ballot(owner && ((sel >> i) & 1u));
+#pragma unroll
+                        for (int g = 0; g < GMAX; ++g) {
+                            // (a head's entries of the wave go side by side: one atomic)
+                            const bool mine = owner && ((sel >> i) & 1u) && my_g + i == g;
+                            const uint64_t bal = __ballot(mine);
+                            if (Bi == 0ull || bal == 0ull) continue;  // uniform
+                            int base = 0;
+                            if (mine && (bal & ((1ull << lane) - 1ull)) == 0ull)
+                                base = atomicAdd(&p.sel_count[my_h[i]], __popcll(bal));
+                            base = __shfl(base, __ffsll((long long)bal) - 1, 64);
+                            const int pos = base + __popcll(bal & ((1ull << lane) - 1ull));
+                            if (mine && pos < p.sel_cap) {
+                                p.sel_index[(int64_t)my_h[i] * p.sel_cap + pos] = idx;
+                                p.sel_score[(int64_t)my_h[i] * p.sel_cap + pos] = s[i];
+                            }
+                        }
+                    }
+                }
+            }
+            if (!want_attn) continue;  // uniform
+            // ---- the values of the rows that some head selected -------------------------------
+            uint4 vraw[KU];
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                vraw[u] = make_uint4(0, 0, 0, 0);
+                const uint64_t lanes = B & LANES.row[u];
+                const uint64_t group = LPR == 64 ? ~0ull : ((1ull << (LPR & 63)) - 1ull) << (rg * LPR);
+                if ((lanes & group) != 0ull && vchunk_ok) vraw[u] = load_chunk<T>(vbase, (krow0 + slot[u]) * Dv, ch);
+            }
+            if (owner) {
+#pragma unroll
+                for (int i = 0; i < KEPT; ++i)
+                    tab[(my_u * RPW + rg) * GMAX + my_g + i] = (sel >> i) & 1u ? s[i] * my_sc[i] * kLog2e : -INFINITY;
+            }
+            // weights while the values are on their way: lane l takes the table's entries
+            // l, l + 64, ..., all of head l % GMAX
+            constexpr int NE = (ROWS * GMAX + 63) / 64;
+            __builtin_amdgcn_wave_barrier();
+            float z[NE], mx = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < NE; ++i) {
+                const bool mine = ROWS * GMAX >= 64 || lane < ROWS * GMAX;
+                z[i] = mine ? tab[i * 64 + lane] : -INFINITY;
+                mx = fmaxf(mx, z[i]);
+            }
+            mx = fmaxf(cross_group_max<GMAX>(mx), m_run);
+            const float f = m_run == -INFINITY ? 0.0f : exp2f(m_run - mx);
+            l_run *= f;
+            m_run = mx;
+#pragma unroll
+            for (int i = 0; i < NE; ++i) {
+                const float w = z[i] > -INFINITY ? exp2f(z[i] - mx) : 0.0f;
+                l_run += w;
+                if (ROWS * GMAX >= 64 || lane < ROWS * GMAX) tab[i * 64 + lane] = w;
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) {
+                const float fg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), g));
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) acc[g][e] *= fg;
+            }
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                if ((B & LANES.row[u]) == 0ull) continue;  // uniform in the wave
+                float vf[EPL];
+                unpack<T>(vraw[u], vf);
+#pragma unroll
+                for (int g = 0; g < GMAX; ++g) {
+                    const float w = tab[(u * RPW + rg) * GMAX + g];
+#pragma unroll
+                    for (int e = 0; e < EPL; ++e) acc[g][e] += w * vf[e];
+                }
+            }
+        }
     }
 
     if (!want_attn) return;  // uniform
 
-    // ---- merge the lane groups of the wave, then the waves of the workgroup -----------
+    // ---- merge the lane groups of the wave, then the waves of the workgroup (a wave, or a
+    // workgroup, without a selected key for a head only says so) -------------------------------
     float* wsm = smem + (size_t)wave * GMAX * (DVP + 2);
+    l_run = cross_group_sum<GMAX>(l_run);
+    if (lane < GMAX) {
+        wsm[lane * (DVP + 2) + DVP] = m_run;
+        wsm[lane * (DVP + 2) + DVP + 1] = l_run;
+    }
 #pragma unroll
     for (int g = 0; g < GMAX; ++g) {
-        const float mall = cross_group_max<LPR>(mrun[g]);
-        const float f = (mrun[g] == -INFINITY) ? 0.0f : exp2f(mrun[g] - mall);
-        const float lsum = cross_group_sum<LPR>(lrun[g] * f);
+        if (__int_as_float(__builtin_amdgcn_readlane(__float_as_int(m_run), g)) == -INFINITY) continue;  // uniform
 #pragma unroll
         for (int e = 0; e < EPL; ++e) {
-            const float a = cross_group_sum<LPR>(acc[g][e] * f);
+            const float a = cross_group_sum<LPR>(acc[g][e]);
             if (rg == 0) wsm[g * (DVP + 2) + ch * EPL + e] = a;
-        }
-        if (lane == 0) {
-            wsm[g * (DVP + 2) + DVP] = mall;
-            wsm[g * (DVP + 2) + DVP + 1] = lsum;
         }
     }
     __syncthreads();
@@ -596,15 +695,16 @@ __global__ __launch_bounds__(256) void search_kernel(const SearchParams p) {
         for (int w = 0; w < nwaves; ++w) {
             const float* ws = smem + ((size_t)w * GMAX + g) * (DVP + 2);
             const float mw = ws[DVP];
-            const float f = (mw == -INFINITY) ? 0.0f : exp2f(mw - mall);
+            if (mw == -INFINITY) continue;
+            const float f = exp2f(mw - mall);
             a += ws[e] * f;
             lsum += ws[DVP + 1] * f;
         }
-        const int head = by_group ? hoff + g : p.tree_q_heads[hoff + g];
-        const size_t slot = (size_t)head * p.num_parts + blockIdx.x;
+        const size_t slot = (size_t)head_of(g) * p.num_parts + blockIdx.x;
         // device-scope stores: written through, so that the workgroup that folds the partials
         // (maybe behind another L2) reads them without cache-wide flushes
-        __hip_atomic_store(&p.part_acc[slot * Dv + e], a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (mall > -INFINITY)
+            __hip_atomic_store(&p.part_acc[slot * Dv + e], a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (e == 0) {
             __hip_atomic_store(&p.part_m[slot], mall, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&p.part_l[slot], lsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -614,7 +714,6 @@ __global__ __launch_bounds__(256) void search_kernel(const SearchParams p) {
 
     // ---- the last workgroup of this tree (and head pass) to arrive folds its partials ----
     __shared__ int s_last;
-    __shared__ float s_fold_red[4];
     hand_off_release();
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -625,37 +724,24 @@ __global__ __launch_bounds__(256) void search_kernel(const SearchParams p) {
     }
     __syncthreads();
     if (!s_last) return;
-    for (int g = 0; g < G; ++g) {  // uniform
-        const int head = by_group ? hoff + g : p.tree_q_heads[hoff + g];
-        fold_partials(p.part_m + (size_t)head * p.num_parts, p.part_l + (size_t)head * p.num_parts,
-                      p.part_acc + (size_t)head * p.num_parts * Dv, p.num_parts, Dv, p.fold_dvl,
-                      p.attn_out, p.out_bf16, (size_t)head * Dv, smem, s_fold_red);
-        __syncthreads();
-    }
-}
-
-template <typename T, int LPR, int NGX>
-inline void launch_search_ngx(const SearchPlan& plan, const SearchParams& p, dim3 grid,
-                              hipStream_t s) {
-    const size_t smem = p.part_acc ? plan.smem : 0;
-    switch (plan.gmax) {
-        case 1:
-            hipLaunchKernelGGL((search_kernel<T, LPR, 1, NGX>), grid, dim3(plan.threads), smem, s, p);
-            break;
-        case 4:
-            hipLaunchKernelGGL((search_kernel<T, LPR, 4, NGX>), grid, dim3(plan.threads), smem, s, p);
-            break;
-        default:
-            hipLaunchKernelGGL((search_kernel<T, LPR, 8, NGX>), grid, dim3(plan.threads), smem, s, p);
-            break;
-    }
+    fold_heads(p, hoff, G, smem);
 }
 
 template <typename T, int LPR>
 inline void launch_search(const SearchPlan& plan, const SearchParams& p, dim3 grid,
                           hipStream_t s) {
-    if (plan.gate_steps > 1) launch_search_ngx<T, LPR, 4>(plan, p, grid, s);
-    else launch_search_ngx<T, LPR, 1>(plan, p, grid, s);
+    const size_t smem = p.part_acc ? plan.smem : 0;
+    switch (plan.gmax) {
+        case 1:
+            hipLaunchKernelGGL((search_kernel<T, LPR, 1>), grid, dim3(plan.threads), smem, s, p);
+            break;
+        case 4:
+            hipLaunchKernelGGL((search_kernel<T, LPR, 4>), grid, dim3(plan.threads), smem, s, p);
+            break;
+        default:
+            hipLaunchKernelGGL((search_kernel<T, LPR, 8>), grid, dim3(plan.threads), smem, s, p);
+            break;
+    }
 }
 
 template <typename T>

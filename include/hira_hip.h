@@ -152,7 +152,7 @@ typedef struct HiraSearchOut {
 } HiraSearchOut;
 
 typedef struct HiraLaunch {
-    int32_t block_threads;  /* vector-ALU kernel: 64, 128 or 256; MFMA kernel: a multiple of 64
+    int32_t block_threads;  /* vector-ALU kernel: 64, 128, 256 or 512; MFMA kernel: a multiple of 64
                                up to 512; 0 = default */
     int32_t nodes_per_wave; /* vector-ALU kernel: level-1 nodes one wavefront walks; MFMA kernel:
                                tiles of 16 level-1 nodes one workgroup walks (at most 16);
