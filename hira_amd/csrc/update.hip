@@ -47,8 +47,8 @@ struct UpdateParams {
     const void* new_keys;    // (T, m, D)
     const void* new_values;  // (T, m, Dv) or NULL
     int32_t m;
-    int32_t chunk;  // windows: keys whose rows are in LDS at a time
     int32_t* state;
+    int32_t stage_values;  // windows: the values' rows have room in LDS too
 };
 
 // a bound must survive the fp32 rounding of the sums that produced it
@@ -62,13 +62,15 @@ constexpr int kCountsInFlight = 16;  // reads of child counts a lane has in flig
 template <typename T>
 __device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int first, int used,
                                  const float* x, float* red_f, int* red_i, int* not_full,
-                                 int* count_of = nullptr) {
+                                 int* count_of = nullptr, float* dist2_of = nullptr,
+                                 float* radius_of = nullptr) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int D = p.dim;
     const size_t base = (size_t)tree * p.cap[l];
     const int32_t* cnt = p.counts[l] + base;
     float best = INFINITY;
     int arg = -1, argc = 0;  // the best node so far and its child count
+    float argr = 0.0f;       // (its radius, asked for with the centre)
     int low = used;  // lowest index of a node that is not full, among those I have seen
     for (int nb = (first & ~63) + wave * 64; nb < used; nb += kCountsInFlight * 4 * 64) {
         // the reads of the child counts in flight together (a wave's nodes still come in
@@ -91,6 +93,7 @@ __device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int fir
                 const int node_c = __shfl(c4[u], src, 64);
                 bal &= bal - 1ull;
                 float ss = 0.0f;
+                const float rad = radius_of != nullptr ? p.radii[l][base + node] : 0.0f;
                 for (int j = lane; j < D; j += 64) {
                     const float df = x[j] - load_elem<T>(p.centers[l], base * D + elem_index(p.layout, D, (size_t)node, j));
                     ss += df * df;
@@ -101,6 +104,7 @@ __device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int fir
                     best = ss;
                     arg = node;
                     argc = node_c;
+                    argr = rad;
                 }
             }
         }
@@ -136,6 +140,13 @@ __device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int fir
         if (lane == 0) red_i[wave] = argc;
         __syncthreads();
         *count_of = red_i[aw_of];
+        __syncthreads();
+    }
+    if (dist2_of != nullptr) *dist2_of = b;
+    if (radius_of != nullptr) {  // uniform
+        if (lane == 0) red_f[wave] = argr;
+        __syncthreads();
+        *radius_of = red_f[aw_of];
         __syncthreads();
     }
     return a;
@@ -355,8 +366,8 @@ __global__ __launch_bounds__(kTauThreads) void k_update_threshold(
 // compiler keeps the loop's values in registers instead of asking for them again every key).
 template <typename T>
 __device__ __attribute__((noinline)) void update_one_key_called(const UpdateParams& p, const int tree, const int i,
-                                                              float* sm, float* red_f, int* red_i, float* s_dist,
-                                                              float* s_rad) {
+                                                             float* sm, float* red_f, int* red_i, float* s_dist,
+                                                             float* s_rad) {
     update_one_key<T>(p, tree, i, sm, red_f, red_i, s_dist, s_rad);
 }
 
@@ -365,29 +376,40 @@ __device__ __attribute__((noinline)) void update_one_key_called(const UpdatePara
 // the centres of the nodes with room, the ancestors' centres and radii): 4-5 us a key, one key
 // after the other.  But the nodes with room are few -- the tail nodes opened by earlier appends,
 // what a rebuilt subtree left free -- and between two keys of a window only the window itself
-// changes them.  So a workgroup that has a window to place reads them ONCE into LDS (ids, child
+// changes them.  So a workgroup that has a window to place lists them ONCE in LDS (ids, child
 // counts, centres, radii, and for every ancestor on their paths its radius and the distance
-// between consecutive centres, which never changes) and then places key after key from LDS:
-// distances to every candidate, the nearest (ties: the lowest id, as the general way), next slot,
-// radii along the path; memory only sees stores.  A key that finds no candidate goes the general
-// way (it opens a node), after which the candidates are read again.  A tree with more nodes
-// with room than the list holds goes the general way altogether.  Same placement, slots and
-// radii as key by key (the replaced kernels: kernels/triton_update_kernels.py:85-123 nearest
-// centre for a whole window at once, :126-235 slots, :238-326 radii).
+// between consecutive centres, which never changes) and takes the window 64 keys at a time:
+//   distances  of all 64 keys to all candidates, by all waves, into a table in LDS;
+//   choice     wave 0, a candidate a lane, key after key: the smallest distance among the lanes
+//              whose node has room (ties: the lowest id, as the general way) -- one row of the
+//              table, a minimum over the wave, a count: some 100 cycles a key, which is all that has
+//              to happen one key after the other;
+//   rows       of the 64 keys to their slots, 16 bytes a thread.
+// Radii wait until the list is given up: R = max over the keys of what each asks for, and that
+// grows with the distance, so the largest distance a candidate saw gives the radius that key by
+// key would have reached, to the last bit, and so up the levels.  A key that finds no candidate
+// opens a node the general way (all candidates are full then: the new node becomes the list).  A
+// tree with more nodes with room than the list holds goes the general way altogether.  Same
+// placement, slots and radii as key by key (the replaced kernels:
+// kernels/triton_update_kernels.py:85-123 nearest centre for a whole window at once, :126-235 slots,
+// :238-326 radii).
 constexpr int kCandMax = 48;
+constexpr int kWinKeys = 64;  // keys of a window taken together
+constexpr int kWinCols = 4;   // columns of a row a lane holds, at most (rows of up to 256)
+constexpr size_t kWinLds = 128 * 1024;  // dynamic LDS of a workgroup, at most (256 fp32 columns: 126 KiB)
 
 struct WindowLds {
     int n;                                  // candidates listed (may exceed kCandMax: then unusable)
-    int low;                                // lowest level-1 node from `first` on that is not full
+    int low_empty;                          // lowest level-1 slot from `first` on that is no node yet
     int id[kCandMax];                       // level-1 node
     int cnt[kCandMax];                      // its child count (bf: full by now)
-    float rad[kCandMax];                    // its radius
-    float dist[kCandMax];                   // squared distance of the current key
+    int cnt0[kCandMax];                     // its child count as memory has it
+    float rad[kCandMax];                    // its radius, as memory has it
+    float far[kCandMax];                    // largest squared distance of a key it took
     int anc_id[HIRA_MAX_LEVELS][kCandMax];      // [l][c]: c's ancestor at level l
     int anc_rep[HIRA_MAX_LEVELS][kCandMax];     // [l][c]: the first candidate with the same ancestor at level l
     float anc_rad[HIRA_MAX_LEVELS][kCandMax];   // [l][rep]: that ancestor's radius
     float anc_step[HIRA_MAX_LEVELS][kCandMax];  // [l][c]: distance between c's ancestors at levels l-1 and l
-    int best;
 };
 
 // level-l ancestor of level-1 node `node1` (l >= 1)
@@ -405,16 +427,15 @@ __device__ bool window_candidates(const UpdateParams& p, const int tree, WindowL
     int32_t* st = p.state + (size_t)tree * (HIRA_MAX_LEVELS + 2);
     const int used = st[1], first = min(max(st[0], 0), used);
     const size_t b1 = (size_t)tree * p.cap[1];
-    __syncthreads();  // (everybody has read the state; earlier users of the list are done)
     if (t == 0) {
         w.n = 0;
-        w.low = used;
+        w.low_empty = used;
     }
     __syncthreads();
     for (int nb = first & ~63; nb < used; nb += kUpdThreads) {  // uniform
         const int n = nb + t;
         const int c = (n >= first && n < used) ? p.counts[1][b1 + n] : bf;
-        if (c < bf) atomicMin(&w.low, n);
+        if (c <= 0) atomicMin(&w.low_empty, n);
         // a node in use with a free slot; count 0 marks a pad slot, which is not a node yet
         const bool room = c > 0 && c < bf;
         const unsigned long long bal = __ballot(room);
@@ -423,12 +444,12 @@ __device__ bool window_candidates(const UpdateParams& p, const int tree, WindowL
         at = __shfl(at, 0, 64) + __popcll(bal & ((1ull << lane) - 1ull));
         if (room && at < kCandMax) {
             w.id[at] = n;
-            w.cnt[at] = c;
+            w.cnt[at] = w.cnt0[at] = c;
+            w.far[at] = -1.0f;
         }
     }
     __syncthreads();
     const int nc = w.n;
-    if (t == 0) st[0] = max(w.low, first);
     if (nc > kCandMax) return false;
     // (the order in which the waves listed their nodes does not matter: ties between candidates
     // are decided by the node's id)
@@ -472,169 +493,443 @@ __device__ bool window_candidates(const UpdateParams& p, const int tree, WindowL
     return true;
 }
 
-// sum over the wave, the same value in every lane (data-path moves inside rows of 16 lanes, then
-// the four rows' sums: no trip through LDS, a tenth of the latency of six shuffles)
-__device__ __forceinline__ float wave_sum_dpp(float v) {
-    auto mv = [](float x, int ctrl_sel) {
-        const int xi = __float_as_int(x);
-        int r;
-        if (ctrl_sel == 0) r = __builtin_amdgcn_update_dpp(0, xi, 0xB1, 0xF, 0xF, false);        // lanes 1 0 3 2
-        else if (ctrl_sel == 1) r = __builtin_amdgcn_update_dpp(0, xi, 0x4E, 0xF, 0xF, false);   // lanes 2 3 0 1
-        else if (ctrl_sel == 2) r = __builtin_amdgcn_update_dpp(0, xi, 0x141, 0xF, 0xF, false);  // halves of 8 mirrored
-        else r = __builtin_amdgcn_update_dpp(0, xi, 0x140, 0xF, 0xF, false);                     // the row mirrored
-        return __int_as_float(r);
-    };
-    v += mv(v, 0);
-    v += mv(v, 1);
-    v += mv(v, 2);
-    v += mv(v, 3);
-    const int vi = __float_as_int(v);
-    // (added up in the order of the butterfly of shuffles that the general way uses: the two
-    // kernels must agree on a distance to the last bit)
-    return (__int_as_float(__builtin_amdgcn_readlane(vi, 0)) + __int_as_float(__builtin_amdgcn_readlane(vi, 16))) +
-           (__int_as_float(__builtin_amdgcn_readlane(vi, 32)) + __int_as_float(__builtin_amdgcn_readlane(vi, 48)));
+// the value that lane ^ BIT holds, by moves that need no trip through LDS (16, 32: the sum with it)
+template <int BIT>
+__device__ __forceinline__ float win_partner(float v) {
+    if constexpr (BIT == 1) return dpp_move<0xB1>(v);                   // quad [1,0,3,2]
+    else if constexpr (BIT == 2) return dpp_move<0x4E>(v);              // quad [2,3,0,1]
+    else if constexpr (BIT == 4) return dpp_move<0x1B>(dpp_move<0x141>(v));  // halves of 8 mirrored, quads mirrored
+    else return dpp_move<0x128>(v);                                     // 8: row rotated by 8
+}
+template <int BIT>
+__device__ __forceinline__ float win_sum_across(float v) {
+    const auto r = BIT == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false)
+                             : __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Squared distances of keys [k0, k1) of the chunk (rows in LDS) to all candidates:
+// table[k * kCandMax + c].  A wave takes eight keys at a time, its lanes a column (of every 64)
+// each, and goes through the candidates: the eight sums over the lanes halve in number with every
+// one of the first three steps (lanes with the bit set go on with the other half).  The additions are those of a butterfly of lane ^ 1, ^ 2,
+// ..., ^ 32, in that order: the general way's, to the last bit.
+template <typename T>
+__device__ __forceinline__ void window_distances(const int D, const WindowLds& w, const float* cen, const T* rows,
+                                 const int k0, const int k1, float* table) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nc = w.n;
+    if (nc == 0) return;
+    const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
+    const int mine = (b0 ? 4 : 0) + (b1 ? 2 : 0) + (b2 ? 1 : 0);  // the key (of eight) I end up with
+    for (int k = k0 + wave * 8; k < k1; k += kUpdThreads / 64 * 8) {  // uniform in the wave
+        float x[8][kWinCols];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const size_t src = (size_t)min(k + u, k1 - 1) * D;
+#pragma unroll
+            for (int i = 0; i < kWinCols; ++i)
+                if (i * 64 < D) {  // (uniform)
+                    const float xi = load_elem<T>(rows, src + min(i * 64 + lane, D - 1));
+                    x[u][i] = i * 64 + lane < D ? xi : 0.0f;
+                }
+        }
+        for (int c = 0; c < nc; ++c) {  // uniform
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kWinCols; ++i)
+                if (i * 64 < D) {  // uniform
+                    const float ci = cen[(size_t)c * D + min(i * 64 + lane, D - 1)];
+                    const float cj = i * 64 + lane < D ? ci : 0.0f;
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        const float df = x[u][i] - cj;
+                        v[u] += df * df;
+                    }
+                }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = (b0 ? v[u + 4] : v[u]) + win_partner<1>(b0 ? v[u] : v[u + 4]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) v[u] = (b1 ? v[u + 2] : v[u]) + win_partner<2>(b1 ? v[u] : v[u + 2]);
+            float s = (b2 ? v[1] : v[0]) + win_partner<4>(b2 ? v[0] : v[1]);
+            s += win_partner<8>(s);
+            s = win_sum_across<16>(s);
+            s = win_sum_across<32>(s);
+            if (lane < 8 && k + mine < k1) table[(k + mine) * kCandMax + c] = s;
+        }
+    }
+}
+
+__device__ __forceinline__ float win_min(float v) {  // over the wave, the same in every lane
+    v = fminf(v, win_partner<1>(v));
+    v = fminf(v, win_partner<2>(v));
+    v = fminf(v, dpp_move<0x141>(v));  // (any lane of the other four will do)
+    v = fminf(v, win_partner<8>(v));
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fminf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fminf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// The list is given up: child counts and radii of the candidates that took keys, and their
+// ancestors' radii, go to memory.  By wave 0, a candidate a lane.
+__device__ void window_flush(const UpdateParams& p, const int tree, WindowLds& w) {
+    const int c = threadIdx.x, L = p.num_levels;
+    if (c >= 64) return;
+    const bool took = c < w.n && w.cnt[c] != w.cnt0[c];
+    float r = 0.0f;
+    if (took) {
+        const size_t at = (size_t)tree * p.cap[1] + w.id[c];
+        p.counts[1][at] = w.cnt[c];
+        r = fmaxf(w.rad[c], pad_up(sqrtf(w.far[c])));
+        if (r != w.rad[c]) p.radii[1][at] = r;
+    }
+    for (int l = 2; l < L; ++l) {
+        int rep = 0;
+        float have = 0.0f;
+        if (took) {
+            rep = w.anc_rep[l][c];
+            have = w.anc_rad[l][rep];
+        }
+        __builtin_amdgcn_wave_barrier();
+        // (radii are -inf or not negative: their bits order as signed integers)
+        if (took) atomicMax(reinterpret_cast<int*>(&w.anc_rad[l][rep]), __float_as_int(pad_up(w.anc_step[l][c] + r)));
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        if (took) {
+            r = w.anc_rad[l][rep];
+            if (r != have) p.radii[l][(size_t)tree * p.cap[l] + w.anc_id[l][c]] = r;  // (the same from all of them)
+        }
+    }
+}
+
+// Key i of the tree's window opens a level-1 node centred on itself, no node having room: what
+// update_one_key does in that case, in the trips to memory that it cannot do without (the child
+// counts of the level above, the centres and radii of the nodes there with room, the path above the
+// chosen one), the key and the level sizes (s_used) being in LDS.  Returns the node (-1: dropped for
+// lack of capacity); x (LDS) then holds the key in fp32, s_dist[l] the distance between the node's
+// ancestors at levels l - 1 and l, s_rad[l] the radius of the latter.
+template <typename T>
+__device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, const int i,
+                                                 const int position, int* s_used, const T* key, float* x,
+                                                 float* red_f, int* red_i, float* s_dist, float* s_rad) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int D = p.dim, Dv = p.vdim, L = p.num_levels, bf = p.bf;
+    int32_t* st = p.state + (size_t)tree * (HIRA_MAX_LEVELS + 2);
+    const size_t base0 = (size_t)tree * p.cap[0];
+    for (int j = t; j < D; j += kUpdThreads) x[j] = load_elem<T>(key, j);
+    __syncthreads();
+    int top = 1;  // levels 1 .. top get a new node
+    int parent = -1, pcount = 0;
+    float pdist = 0.0f, prad = 0.0f;
+    for (; top < L - 1; ++top) {  // uniform
+        parent = nearest_with_room<T>(p, tree, top + 1, 0, s_used[top + 1], x, red_f, red_i, nullptr, &pcount, &pdist,
+                                      &prad);
+        if (parent >= 0) break;
+    }
+    const long long idx = parent >= 0 ? (long long)parent * bf + pcount : s_used[top];
+    bool fits = true;  // every new node below is the first child of the new node above
+    long long id = idx;
+    for (int l = top; l >= 1; --l) {
+        if (id >= p.cap[l]) fits = false;
+        id *= bf;
+    }
+    if (id >= p.cap[0]) fits = false;
+    __syncthreads();  // (everybody has read the sizes)
+    if (!fits) {
+        if (t == 0) st[HIRA_MAX_LEVELS + 1] = 1;
+        __syncthreads();
+        return -1;  // uniform
+    }
+    // the path above the new nodes: radii, and the distances between centres (a wave per level)
+    for (int l = top + 1 + wave; l < L; l += kUpdThreads / 64) {  // uniform in the wave
+        float d = sqrtf(pdist), rad_now = prad;
+        if (l > top + 1) {
+            const size_t node = ancestor_of((size_t)parent, l - top, bf);
+            rad_now = p.radii[l][(size_t)tree * p.cap[l] + node];
+            const size_t child = ancestor_of((size_t)parent, l - top - 1, bf);
+            const size_t bl = (size_t)tree * p.cap[l], bc = (size_t)tree * p.cap[l - 1];
+            float ss = 0.0f;
+            for (int j = lane; j < D; j += 64) {
+                const float a = load_elem<T>(p.centers[l - 1], bc * D + elem_index(p.layout, D, child, j));
+                const float b = load_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, node, j));
+                ss += (a - b) * (a - b);
+            }
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+            d = sqrtf(ss);
+        }
+        if (lane == 0) {
+            s_dist[l] = d;
+            s_rad[l] = rad_now;
+        }
+    }
+    // the new nodes, the key, its value
+    id = idx;
+    for (int l = top; l >= 1; --l) {
+        const size_t bl = (size_t)tree * p.cap[l];
+        for (int j = t; j < D; j += kUpdThreads)
+            store_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, (size_t)id, j), x[j]);
+        if (t == 0) {
+            p.radii[l][bl + id] = 0.0f;
+            p.counts[l][bl + id] = 1;
+            if (id + 1 > s_used[l]) s_used[l] = st[l] = (int)(id + 1);
+            s_dist[l] = s_rad[l] = 0.0f;
+        }
+        id *= bf;
+    }
+    const size_t slot = (size_t)id;
+    const int node1 = (int)(id / bf);
+    for (int j = t; j < D; j += kUpdThreads)
+        store_elem<T>(p.keys, base0 * D + elem_index(p.key_layout, D, slot, j), x[j]);
+    if (p.new_values && p.values)
+        for (int j = t; j < Dv; j += kUpdThreads)
+            store_elem<T>(p.values, (base0 + slot) * Dv + j, load_elem<T>(p.new_values, ((size_t)tree * p.m + i) * Dv + j));
+    float worst = 0.0f;
+    if (p.keys8 != nullptr) {
+        for (int j = t; j < D; j += kUpdThreads) {
+            const float u = x[j] / p.kscale[(size_t)tree * D + j];
+            const float r = fminf(fmaxf(rintf(u), -127.0f), 127.0f);
+            worst = fmaxf(worst, fabsf(u - r));
+            p.keys8[base0 * D + shadow_index(D, slot, j)] = (int8_t)(int)r;
+        }
+        worst = wave_max(worst);
+        if (lane == 0) red_f[wave] = worst;
+    }
+    __syncthreads();
+    if (t == 0) {
+        if (p.keys8 != nullptr)  // (the node holds no other key: its bound starts here)
+            p.keps[(size_t)tree * p.cap[1] + node1] = fmaxf(fmaxf(red_f[0], red_f[1]), fmaxf(red_f[2], red_f[3]));
+        p.perm[base0 + slot] = position;
+        st[HIRA_MAX_LEVELS] = position + 1;
+        if (parent >= 0) p.counts[top + 1][(size_t)tree * p.cap[top + 1] + parent] = pcount + 1;
+        float r_child = 0.0f;
+        for (int l = top + 1; l < L; ++l) {
+            const float rn = fmaxf(s_rad[l], pad_up(s_dist[l] + r_child));
+            if (rn != s_rad[l]) p.radii[l][(size_t)tree * p.cap[l] + ancestor_of((size_t)parent, l - top, bf)] = rn;
+            s_rad[l] = r_child = rn;
+        }
+    }
+    __syncthreads();
+    return node1;
 }
 
 template <typename T>
 __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParams p) {
-    extern __shared__ float sm[];  // 2 D floats of the general way, kCandMax centres, a chunk of rows
+    // 2 D floats of the general way, kCandMax centres, the table of distances, a chunk of key rows
+    extern __shared__ __attribute__((aligned(16))) float sm[];
     __shared__ float red_f[4];
     __shared__ int red_i[4];
     __shared__ float s_dist[HIRA_MAX_LEVELS], s_rad[HIRA_MAX_LEVELS];
     __shared__ WindowLds w;
-    __shared__ int s_slot[16], s_node[16];  // where the chunk's keys went (slot < 0: not placed yet)
-    __shared__ int s_done;                   // keys of the chunk dealt with so far
+    __shared__ int s_slot[kWinKeys];  // where the chunk's keys went (-1: placed the general way, or dropped)
+    __shared__ int s_done;            // keys of the chunk dealt with so far
+    __shared__ int s_used[HIRA_MAX_LEVELS];  // slots in use per level
+    constexpr int EPL = Elem<T>::kPerChunk;
     const int tree = blockIdx.x;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int D = p.dim, Dv = p.vdim, L = p.num_levels, bf = p.bf;
     float* cen = sm + 2 * (size_t)D;
+    float* table = cen + (size_t)kCandMax * D;
+    T* rows = reinterpret_cast<T*>(table + (size_t)kCandMax * kWinKeys);  // (kWinKeys, D): the chunk's keys
+    uint4* vals = p.stage_values ? reinterpret_cast<uint4*>(rows + (size_t)kWinKeys * D) : nullptr;  // its values
     int32_t* st = p.state + (size_t)tree * (HIRA_MAX_LEVELS + 2);
     const size_t base0 = (size_t)tree * p.cap[0], b1 = (size_t)tree * p.cap[1];
-    bool usable = L >= 2 && window_candidates<T>(p, tree, w, cen);  // false: the tree's keys go
-                                                                    // the general way, all of them
-    // The window's rows come into LDS a chunk of keys at a time.  Wave 0 then places key after key
-    // from the list, on its own: no barrier, nothing asked of memory (it carries the number of keys
-    // inserted so far; device memory only sees stores) -- until the chunk ends or a key finds no
-    // candidate.  Then the workgroup copies the placed keys' rows to their slots, sends the key
-    // without a candidate the general way, and wave 0 carries on.
     const bool with_values = p.new_values != nullptr && p.values != nullptr;
-    const int chunk = p.chunk;
-    float* xs = cen + (size_t)kCandMax * D;  // (chunk, D) keys
-    float* vs = xs + (size_t)chunk * D;      // (chunk, Dv) values
-    for (int i0 = 0; i0 < p.m; i0 += chunk) {  // uniform
-        const int nk = min(chunk, p.m - i0);
-        const size_t r0 = (size_t)tree * p.m + i0;
-        __syncthreads();  // (the chunk before is done with its rows)
-        for (int e = t; e < nk * D; e += kUpdThreads) xs[e] = load_elem<T>(p.new_keys, r0 * D + e);
-        if (with_values)
-            for (int e = t; e < nk * Dv; e += kUpdThreads) vs[e] = load_elem<T>(p.new_values, r0 * Dv + e);
-        if (t == 0) s_done = 0;
-        __syncthreads();
-        int k = 0;
-        while (k < nk) {  // uniform
-            if (!usable) {
-                for (; k < nk; ++k) update_one_key_called<T>(p, tree, i0 + k, sm, red_f, red_i, s_dist, s_rad);
-                break;
+    const int kc = D / EPL;
+    auto stage = [&](int i0) {  // the rows of the chunk that starts at key i0 into LDS
+        const int nk = min(kWinKeys, p.m - i0);
+        const uint4* src = reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(p.new_keys) +
+                                                          ((size_t)tree * p.m + i0) * D);
+        const uint4* vsrc = vals == nullptr ? nullptr
+                                            : reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(p.new_values) +
+                                                                             ((size_t)tree * p.m + i0) * Dv);
+        constexpr int SU = 8;
+        const int nc = nk * kc, nv = vals == nullptr ? 0 : nk * (Dv / EPL);
+        for (int e0 = t; e0 < nc + nv; e0 += SU * kUpdThreads) {
+            uint4 raw[SU];
+#pragma unroll
+            for (int u = 0; u < SU; ++u) {
+                const int e = min(e0 + u * kUpdThreads, nc + nv - 1);
+                raw[u] = e < nc ? src[e] : vsrc[e - nc];
             }
+#pragma unroll
+            for (int u = 0; u < SU; ++u) {
+                const int e = e0 + u * kUpdThreads;
+                if (e < nc) reinterpret_cast<uint4*>(rows)[e] = raw[u];
+                else if (e < nc + nv) vals[e - nc] = raw[u];
+            }
+        }
+    };
+    int position = st[HIRA_MAX_LEVELS];  // of the next key (every thread carries it along)
+    stage(0);
+    if (t >= 1 && t < L) s_used[t] = st[t];
+    if (!window_candidates<T>(p, tree, w, cen)) {  // uniform: the tree's keys go the general way, all of them
+        for (int i = 0; i < p.m; ++i) update_one_key_called<T>(p, tree, i, sm, red_f, red_i, s_dist, s_rad);
+        return;
+    }
+    for (int i0 = 0; i0 < p.m; i0 += kWinKeys) {  // uniform
+        const int nk = min(kWinKeys, p.m - i0);
+        const int position0 = position;
+        if (i0 > 0) {
+            stage(i0);  // (behind the barrier that ends the chunk before: nobody needs its rows any more)
+            __syncthreads();
+        }
+        window_distances<T>(D, w, cen, rows, 0, nk, table);
+        for (int k = 0; k < nk;) {  // uniform
+            __syncthreads();
             if (wave == 0) {
-                int position = st[HIRA_MAX_LEVELS];
+                const int n = w.n;
+                int cnt = lane < n ? w.cnt[lane] : bf;
+                const int id = lane < n ? w.id[lane] : 0x7fffffff;
+                const int cl = min(lane, kCandMax - 1);
+                float far = lane < n ? w.far[lane] : -1.0f;
+                float next = table[k * kCandMax + cl];
                 int kk = k;
                 for (; kk < nk; ++kk) {
-                    const float* x = xs + (size_t)kk * D;
-                    const int nc = w.n;
-                    float best = INFINITY;
-                    int b = -1, best_id = 0x7fffffff;
-                    for (int c = 0; c < nc; ++c) {  // uniform
-                        if (w.cnt[c] >= bf) continue;
-                        float ss = 0.0f;
-                        for (int j = lane; j < D; j += 64) {
-                            const float df = x[j] - cen[(size_t)c * D + j];
-                            ss += df * df;
-                        }
-                        ss = wave_sum_dpp(ss);
-                        const int id = w.id[c];
-                        if (ss < best || (ss == best && id < best_id)) {  // ties: the lowest node
-                            best = ss;
-                            b = c;
-                            best_id = id;
-                        }
-                    }
-                    if (b < 0) break;  // no node has room: the workgroup sends this key the general way
-                    const int node1 = best_id, count1 = w.cnt[b];
-                    const int slot = node1 * bf + count1;
-                    if (lane == 0) {
-                        s_slot[kk] = slot;
-                        s_node[kk] = node1;
-                        w.cnt[b] = count1 + 1;
-                        p.counts[1][b1 + node1] = count1 + 1;
-                        // radii along the key's path: the leaf parent covers the key, every
-                        // ancestor its child
-                        float r_child = fmaxf(w.rad[b], pad_up(sqrtf(best)));
-                        if (r_child != w.rad[b]) {
-                            w.rad[b] = r_child;
-                            p.radii[1][b1 + node1] = r_child;
-                        }
-                        for (int l = 2; l < L; ++l) {
-                            const int rep = w.anc_rep[l][b];
-                            const float have = w.anc_rad[l][rep];
-                            const float rn = fmaxf(have, pad_up(w.anc_step[l][b] + r_child));
-                            if (rn != have) {
-                                w.anc_rad[l][rep] = rn;
-                                p.radii[l][(size_t)tree * p.cap[l] + w.anc_id[l][b]] = rn;
+                    // a single node with room takes the keys that follow until it is full: a key a lane
+                    const unsigned long long room = __ballot(cnt < bf);
+                    if (room != 0ull && (room & (room - 1ull)) == 0ull) {
+                        const int c = __ffsll((long long)room) - 1;
+                        const int have = __builtin_amdgcn_readlane(cnt, c), node = __builtin_amdgcn_readlane(id, c);
+                        const int take = min(bf - have, nk - kk);
+                        const float d = lane < take ? table[(kk + lane) * kCandMax + c] : 0.0f;
+                        if (__ballot(!(d < INFINITY)) == 0ull) {
+                            if (lane < take) s_slot[kk + lane] = node * bf + have + lane;
+                            const float most = -win_min(-d);
+                            if (lane == c) {
+                                cnt += take;
+                                far = fmaxf(far, most);
                             }
-                            r_child = rn;
+                            kk += take - 1;
+                            next = table[min(kk + 1, nk - 1) * kCandMax + cl];
+                            continue;
                         }
-                        p.perm[base0 + slot] = position;
                     }
-                    ++position;
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");  // (lane 0's list updates
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");  //  before the next key reads)
+                    const float d = cnt < bf ? next : INFINITY;
+                    next = table[min(kk + 1, nk - 1) * kCandMax + cl];
+                    const float best = win_min(d);
+                    if (best == INFINITY) break;  // no node has room
+                    unsigned long long who = __ballot(d == best);
+                    if (who & (who - 1ull)) {  // ties: the lowest node
+                        int low = d == best ? id : 0x7fffffff;
+#pragma unroll
+                        for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
+                        who = __ballot(d == best && id == low);
+                    }
+                    if (lane == __ffsll((long long)who) - 1) {
+                        s_slot[kk] = id * bf + cnt;
+                        ++cnt;
+                        far = fmaxf(far, d);
+                    }
+                }
+                if (lane < n) {
+                    w.cnt[lane] = cnt;
+                    w.far[lane] = far;
                 }
                 if (lane == 0) {
-                    st[HIRA_MAX_LEVELS] = position;
                     s_done = kk;
+                    if (kk < nk) s_slot[kk] = -1;
                 }
             }
             __syncthreads();
             const int kd = s_done;
-            // ---- the rows of the keys placed from the list: keys k .. kd - 1 ---------------------
-            for (int q = k; q < kd; ++q) {  // uniform
-                const size_t slot = (size_t)s_slot[q];
-                const float* x = xs + (size_t)q * D;
-                for (int j = t; j < D; j += kUpdThreads)
-                    store_elem<T>(p.keys, base0 * D + elem_index(p.key_layout, D, slot, j), x[j]);
-                if (p.keys8 != nullptr) {
-                    // the key's 8-bit shadow with the tree's steps; a component beyond +-127 steps
-                    // clips, and the node's error bound then covers it
-                    float worst = 0.0f;
-                    for (int j = t; j < D; j += kUpdThreads) {
-                        const float u = x[j] / p.kscale[(size_t)tree * D + j];
-                        const float r = fminf(fmaxf(rintf(u), -127.0f), 127.0f);
-                        worst = fmaxf(worst, fabsf(u - r));
-                        p.keys8[base0 * D + shadow_index(D, slot, j)] = (int8_t)(int)r;
-                    }
-                    worst = wave_max(worst);
-                    if (lane == 0) red_f[wave] = worst;
-                    __syncthreads();
-                    if (t == 0) {
-                        float* e = p.keps + b1 + s_node[q];
-                        *e = fmaxf(*e, fmaxf(fmaxf(red_f[0], red_f[1]), fmaxf(red_f[2], red_f[3])));
-                    }
-                    __syncthreads();
-                }
-                if (with_values)
-                    for (int j = t; j < Dv; j += kUpdThreads)
-                        store_elem<T>(p.values, (base0 + slot) * Dv + j, vs[(size_t)q * Dv + j]);
-            }
+            position += kd - k;
             k = kd;
             if (k < nk) {
-                // key k found no node with room: it opens one, the general way (which reads device
-                // memory that the keys before it wrote: the barrier above was a full one); then
-                // the list is read again
-                update_one_key_called<T>(p, tree, i0 + k, sm, red_f, red_i, s_dist, s_rad);
-                usable = window_candidates<T>(p, tree, w, cen);
+                // key k found no node with room: it opens one.  All listed nodes are full, so the
+                // new one is the whole list from here on.
+                window_flush(p, tree, w);
+                const int node = open_node<T>(p, tree, i0 + k, position, s_used, rows + (size_t)k * D, sm, red_f, red_i, s_dist, s_rad);
+                if (node >= 0) ++position;
+                if (t == 0) {
+                    w.n = node >= 0 ? 1 : 0;
+                    w.id[0] = node;
+                    w.cnt[0] = w.cnt0[0] = 1;
+                    w.rad[0] = s_rad[1];
+                    w.far[0] = -1.0f;
+                    for (int l = 2; l < L; ++l) {
+                        w.anc_id[l][0] = (int)ancestor_of((size_t)max(node, 0), l, bf);
+                        w.anc_rep[l][0] = 0;
+                        w.anc_step[l][0] = s_dist[l];
+                        w.anc_rad[l][0] = s_rad[l];
+                    }
+                }
+                for (int j = t; j < D; j += kUpdThreads) cen[j] = sm[j];  // (its centre is the key)
+                __syncthreads();
                 ++k;
+                window_distances<T>(D, w, cen, rows, k, nk, table);
             }
+        }
+        // ---- the rows of the keys placed from the list, 16 bytes a thread -----------------------
+        const bool v_chunks = with_values && Dv % EPL == 0;
+        const int vc = v_chunks ? Dv / EPL : 0, per = kc + vc;
+        constexpr int RU = 4;  // chunks a thread has in flight
+        const float inv_per = 1.0f / (float)per;  // (at most 64 x 128 chunks: the float quotient is exact)
+        for (int e0 = t; e0 < nk * per; e0 += RU * kUpdThreads) {
+            uint4 raw[RU];
+            T* dst[RU];
+#pragma unroll
+            for (int u = 0; u < RU; ++u) {
+                const int e = min(e0 + u * kUpdThreads, nk * per - 1);
+                const int q = (int)(((float)e + 0.5f) * inv_per), c = e - q * per, slot = s_slot[q];
+                const size_t r = (size_t)tree * p.m + i0 + q;
+                const bool key = c < kc;
+                if (key) raw[u] = reinterpret_cast<const uint4*>(rows)[q * kc + c];
+                else if (vals != nullptr) raw[u] = vals[q * vc + c - kc];
+                else raw[u] = load_chunk<T>(p.new_values, r * Dv, c - kc);
+                dst[u] = slot < 0 || e0 + u * kUpdThreads >= nk * per
+                             ? nullptr
+                             : (key ? reinterpret_cast<T*>(p.keys) + base0 * D + elem_index(p.key_layout, D, (size_t)slot, c * EPL)
+                                    : reinterpret_cast<T*>(p.values) + (base0 + slot) * Dv + (c - kc) * EPL);
+            }
+#pragma unroll
+            for (int u = 0; u < RU; ++u)
+                if (dst[u] != nullptr) *reinterpret_cast<uint4*>(dst[u]) = raw[u];
+        }
+        if (with_values && !v_chunks)  // (value rows that are not made of chunks)
+            for (int e = t; e < nk * Dv; e += kUpdThreads) {
+                const int q = e / Dv, j = e - q * Dv;
+                if (s_slot[q] >= 0)
+                    store_elem<T>(p.values, (base0 + s_slot[q]) * Dv + j,
+                                  load_elem<T>(p.new_values, ((size_t)tree * p.m + i0 + q) * Dv + j));
+            }
+        // (positions: the chunk's keys in order, without those that were dropped -- which can only
+        // be keys that found no room, so every key before the first dropped one has its plain place)
+        if (wave == 0 && lane < nk) {
+            const int slot = s_slot[lane];
+            if (slot >= 0) p.perm[base0 + slot] = position0 + lane;
+        }
+        if (p.keys8 != nullptr) {
+            // the keys' 8-bit shadow with the tree's steps; a component beyond +-127 steps clips,
+            // and the node's error bound then covers it.  A wave per key.
+            for (int q = wave; q < nk; q += kUpdThreads / 64) {  // uniform in the wave
+                const int slot = s_slot[q];
+                if (slot < 0) continue;
+                float worst = 0.0f;
+                for (int j = lane; j < D; j += 64) {
+                    const float u = load_elem<T>(rows, (size_t)q * D + j) / p.kscale[(size_t)tree * D + j];
+                    const float k8 = fminf(fmaxf(rintf(u), -127.0f), 127.0f);
+                    worst = fmaxf(worst, fabsf(u - k8));
+                    p.keys8[base0 * D + shadow_index(D, (size_t)slot, j)] = (int8_t)(int)k8;
+                }
+                worst = wave_max(worst);
+                if (lane == 0) atomicMax(reinterpret_cast<int*>(p.keps + b1 + slot / bf), __float_as_int(worst));
+            }
+        }
+        if (i0 + kWinKeys < p.m) __syncthreads();
+    }
+    window_flush(p, tree, w);
+    if (wave == 0) {
+        // the bound of the next search for room: the lowest listed node that still has some, or
+        // the lowest slot that was no node when the list was made
+        int low = lane < w.n && w.cnt[lane] < bf ? w.id[lane] : 0x7fffffff;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
+        if (lane == 0) {
+            st[0] = min(low, min(w.low_empty, s_used[1]));
+            st[HIRA_MAX_LEVELS] = position;
         }
     }
 }
@@ -691,15 +986,35 @@ static int update_arguments(const HiraTree* tree, const void* new_keys, const vo
     p.m = m;
     p.state = state;
     *smem = 2 * (size_t)tree->dim * sizeof(float);
-    // windows of a few keys and more: the nodes with room are read into LDS once (where they fit:
-    // 48 centres of up to 256 columns beside the rest)
-    const size_t cand_bytes = *smem + (size_t)kCandMax * tree->dim * sizeof(float);
-    const size_t row_bytes = (size_t)(tree->dim + tree->vdim) * sizeof(float);
-    int chunk = cand_bytes + row_bytes <= 60 * 1024 ? (int)((60 * 1024 - cand_bytes) / row_bytes) : 0;
-    chunk = chunk > 16 ? 16 : chunk;
-    *window = m >= 4 && tree->num_levels >= 2 && chunk >= 1;
-    *smem_w = cand_bytes + (size_t)chunk * row_bytes;
-    p.chunk = chunk;
+    // windows of a few keys and more: the nodes with room are listed in LDS (where they fit: 48 centres
+    // of up to 256 columns beside the table of distances and a chunk of rows)
+    *smem_w = *smem + (size_t)kCandMax * (tree->dim + kWinKeys) * sizeof(float) +
+              (size_t)kWinKeys * tree->dim * (tree->dtype == HIRA_F32 ? 4 : 2);
+    *window = m >= 4 && tree->num_levels >= 2 && tree->dim <= 64 * kWinCols && *smem_w <= kWinLds;
+    const size_t vrow = (size_t)tree->vdim * (tree->dtype == HIRA_F32 ? 4 : 2);
+    if (new_values != nullptr && vrow % 16 == 0 && *smem_w + kWinKeys * vrow <= kWinLds) {
+        p.stage_values = 1;
+        *smem_w += kWinKeys * vrow;
+    }
+    return HIRA_OK;
+}
+
+// The window kernel's LDS, its own lists beside the dynamic part, can exceed what a launch gets
+// without asking: asked for once per kernel and device.
+template <typename T>
+static int launch_update_window(const UpdateParams& p, int trees, size_t smem, hipStream_t s) {
+    constexpr int kMaxDevices = 64;
+    static int asked[kMaxDevices];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+        return fail(HIRA_ELAUNCH, "update: no current device");
+    if (__atomic_load_n(&asked[dev], __ATOMIC_RELAXED) == 0) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_update_window<T>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWinLds) != hipSuccess)
+            return fail(HIRA_ELAUNCH, "update: %zu bytes of LDS refused", kWinLds);
+        __atomic_store_n(&asked[dev], 1, __ATOMIC_RELAXED);
+    }
+    hipLaunchKernelGGL(k_update_window<T>, dim3(trees), dim3(kUpdThreads), smem, s, p);
     return HIRA_OK;
 }
 
@@ -714,10 +1029,9 @@ extern "C" int hira_update(const HiraTree* tree, const void* new_keys, const voi
     if (m == 0) return HIRA_OK;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (window) {
-        if (tree->dtype == HIRA_F32)
-            hipLaunchKernelGGL(k_update_window<float>, dim3(tree->num_trees), dim3(kUpdThreads), smem_w, s, p);
-        else
-            hipLaunchKernelGGL(k_update_window<bf16_t>, dim3(tree->num_trees), dim3(kUpdThreads), smem_w, s, p);
+        const int rc = tree->dtype == HIRA_F32 ? launch_update_window<float>(p, tree->num_trees, smem_w, s)
+                                               : launch_update_window<bf16_t>(p, tree->num_trees, smem_w, s);
+        if (rc != HIRA_OK) return rc;
     } else if (tree->dtype == HIRA_F32) {
         hipLaunchKernelGGL(k_update<float>, dim3(tree->num_trees), dim3(kUpdThreads), smem, s, p);
     } else {
