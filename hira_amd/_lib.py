@@ -138,6 +138,7 @@ SYMBOLS = {
     ),
     "hira_quantize": (C.c_int, [C.POINTER(HiraTree), C.c_int32, C.c_int32, C.c_int32, _vp]),
     "hira_update": (C.c_int, [C.POINTER(HiraTree), _vp, _vp, C.c_int32, _vp, _vp]),
+    "hira_update_state": (C.c_int, [C.POINTER(HiraTree), C.c_int32, _vp, _vp]),
     "hira_sparse_attention": (
         C.c_int,
         [C.POINTER(HiraTree), C.POINTER(HiraQuery), _vp, _vp, _vp, C.c_int32, _vp, _vp],

@@ -199,7 +199,20 @@ class HiraCacheLayer(CacheLayerMixin):
         k4 = key_states if key_states.ndim == 4 else key_states[None]
         # (in the index's storage dtype: the threshold kernel reads samples and queries alike)
         store = getattr(self.indexer, "dtype", None) or k4.dtype
+        if k4.is_cuda and k4.dtype is store and k4.is_contiguous() and self._queue_type is not None:
+            # the positions travel with the launches: nothing waits for the build
+            self.samples = torch.empty((k4.shape[0] * k4.shape[1], s, self.dim), dtype=store, device=k4.device)
+            self._replace_rows(self.samples, k4, n, n, range(s), pick.tolist())
+            return
         self.samples = k4[:, :, pick.to(k4.device)].reshape(-1, s, self.dim).to(store).contiguous()
+
+    def _replace_rows(self, dst, src, rows: int, stride: int, slots, which):
+        """dst[t][slots[i]] = src[t][which[i]] for every tree t; src holds `rows` rows a tree, `stride`
+        rows apart."""
+        arr = C.c_int32 * len(which)
+        _lib.check(_lib.lib().hira_replace_rows(
+            dst.data_ptr(), self._queue_type, self.dim, dst.shape[0], dst.shape[1], src.data_ptr(), rows,
+            stride, arr(*slots), arr(*which), len(which), _lib.stream_of(dst.get_device())))
 
     def _refresh_samples(self, new_keys, seen: int):
         """Keep the sample uniform over all indexed keys as the index grows (reservoir
@@ -229,7 +242,7 @@ class HiraCacheLayer(CacheLayerMixin):
         last = dict(zip(slots, who))
         smp = self.samples
         src = k4
-        if smp.is_cuda:
+        if smp.is_cuda and self._queue_type is not None:
             # one launch, the lists travel with its arguments.  (The rows of a head must lie one
             # behind the other and the heads evenly spaced, as the queue's and a model's do.)
             if src.dtype is not smp.dtype or src.get_device() != smp.get_device():
@@ -242,12 +255,7 @@ class HiraCacheLayer(CacheLayerMixin):
                 stride = m
             else:
                 stride = (src.stride(1) if src.shape[1] > 1 else src.stride(0)) // self.dim
-            n = len(last)
-            arr = C.c_int32 * n
-            _lib.check(_lib.lib().hira_replace_rows(
-                smp.data_ptr(), _lib.HIRA_F32 if smp.dtype is torch.float32 else _lib.HIRA_BF16,
-                self.dim, smp.shape[0], s, src.data_ptr(), m, stride, arr(*last.keys()),
-                arr(*last.values()), n, _lib.stream_of(smp.get_device())))
+            self._replace_rows(smp, src, m, stride, last.keys(), last.values())
             return
         rows = src.reshape(-1, m, self.dim).to(smp.dtype)
         smp[:, torch.tensor(list(last.keys()))] = rows[:, torch.tensor(list(last.values()))].to(smp.device)

@@ -24,14 +24,17 @@ __global__ __launch_bounds__(kMoveThreads) void k_enqueue(uint4* qk, uint4* qv, 
     else qv[dst * vc + (c - kc)] = v[(size_t)row * vc + (c - kc)];
 }
 
-constexpr int kPairs = 128;  // replaced rows per launch (they travel with the kernel's arguments)
+// (replaced rows travel with the kernel's arguments: a few for a token, many for a whole sample)
+template <int N>
 struct RowPairs {
-    int32_t slot[kPairs], from[kPairs];
+    int32_t slot[N], from[N];
 };
+constexpr int kFewPairs = 32, kManyPairs = 448;
 
+template <int N>
 __global__ __launch_bounds__(kMoveThreads) void k_replace_rows(uint4* rows, int chunks,
                                                                int rows_per_tree, const uint4* from,
-                                                               int from_stride, const RowPairs pairs,
+                                                               int from_stride, const RowPairs<N> pairs,
                                                                int n, int total) {
     const int i = blockIdx.x * kMoveThreads + threadIdx.x;
     if (i >= total) return;
@@ -122,6 +125,20 @@ extern "C" int hira_enqueue(void* queue_keys, void* queue_values, int32_t dtype,
     return HIRA_OK;
 }
 
+template <int N>
+static void replace_some(void* rows, int chunks, int num_trees, int rows_per_tree, const void* from,
+                         int from_stride, const int32_t* slot_host, const int32_t* from_host, int c,
+                         void* stream) {
+    RowPairs<N> pairs;
+    memset(&pairs, 0, sizeof(pairs));
+    memcpy(pairs.slot, slot_host, c * sizeof(int32_t));
+    memcpy(pairs.from, from_host, c * sizeof(int32_t));
+    const int total = num_trees * c * chunks;
+    hipLaunchKernelGGL((k_replace_rows<N>), dim3((total + kMoveThreads - 1) / kMoveThreads), dim3(kMoveThreads), 0,
+                       reinterpret_cast<hipStream_t>(stream), static_cast<uint4*>(rows), chunks, rows_per_tree,
+                       static_cast<const uint4*>(from), from_stride, pairs, c, total);
+}
+
 /* see include/hira_hip.h */
 extern "C" int hira_replace_rows(void* rows, int32_t dtype, int32_t dim, int32_t num_trees,
                                  int32_t rows_per_tree, const void* from, int32_t from_rows,
@@ -136,18 +153,16 @@ extern "C" int hira_replace_rows(void* rows, int32_t dtype, int32_t dim, int32_t
         HIRA_CHECK_ARG(slot_host[i] >= 0 && slot_host[i] < rows_per_tree && from_host[i] >= 0 &&
                            from_host[i] < from_rows,
                        "hira_replace_rows: row %d from %d", slot_host[i], from_host[i]);
-    HIRA_CHECK_ARG((int64_t)num_trees * kPairs * chunks < (int64_t)1 << 31, "hira_replace_rows: too many trees");
-    for (int i0 = 0; i0 < n; i0 += kPairs) {
-        RowPairs pairs;
-        const int c = n - i0 < kPairs ? n - i0 : kPairs;
-        memset(&pairs, 0, sizeof(pairs));
-        memcpy(pairs.slot, slot_host + i0, c * sizeof(int32_t));
-        memcpy(pairs.from, from_host + i0, c * sizeof(int32_t));
-        const int total = num_trees * c * chunks;
-        hipLaunchKernelGGL(k_replace_rows, dim3((total + kMoveThreads - 1) / kMoveThreads),
-                           dim3(kMoveThreads), 0, reinterpret_cast<hipStream_t>(stream),
-                           static_cast<uint4*>(rows), chunks, rows_per_tree,
-                           static_cast<const uint4*>(from), from_stride, pairs, c, total);
+    HIRA_CHECK_ARG((int64_t)num_trees * kManyPairs * chunks < (int64_t)1 << 31, "hira_replace_rows: too many trees");
+    for (int i0 = 0; i0 < n;) {
+        const int left = n - i0;
+        if (left <= kFewPairs)
+            replace_some<kFewPairs>(rows, chunks, num_trees, rows_per_tree, from, from_stride, slot_host + i0,
+                                    from_host + i0, left, stream);
+        else
+            replace_some<kManyPairs>(rows, chunks, num_trees, rows_per_tree, from, from_stride, slot_host + i0,
+                                     from_host + i0, left < kManyPairs ? left : kManyPairs, stream);
+        i0 += left <= kFewPairs ? left : kManyPairs;
     }
     HIRA_CHECK_LAUNCH("hira_replace_rows");
     return HIRA_OK;

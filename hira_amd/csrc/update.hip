@@ -1018,6 +1018,32 @@ static int launch_update_window(const UpdateParams& p, int trees, size_t smem, h
     return HIRA_OK;
 }
 
+namespace hira {
+struct StateRow {
+    int32_t v[HIRA_MAX_LEVELS + 2];
+};
+__global__ void k_update_state(int32_t* state, const StateRow row, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) state[i] = row.v[i % (HIRA_MAX_LEVELS + 2)];
+}
+}  // namespace hira
+
+/* see include/hira_hip.h */
+extern "C" int hira_update_state(const HiraTree* tree, int32_t num_keys, int32_t* state, void* stream) {
+    HIRA_CHECK_ARG(tree && state && tree->num_trees >= 1 && tree->num_levels >= 1 &&
+                       tree->num_levels <= HIRA_MAX_LEVELS,
+                   "hira_update_state: tree / state");
+    StateRow row;
+    memset(&row, 0, sizeof(row));
+    for (int l = tree->num_levels == 1 ? 0 : 1; l < tree->num_levels; ++l) row.v[l] = tree->size[l];
+    row.v[HIRA_MAX_LEVELS] = num_keys;
+    const int n = tree->num_trees * (HIRA_MAX_LEVELS + 2);
+    hipLaunchKernelGGL(k_update_state, dim3((n + 255) / 256), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                       state, row, n);
+    HIRA_CHECK_LAUNCH("hira_update_state");
+    return HIRA_OK;
+}
+
 /* see include/hira_hip.h */
 extern "C" int hira_update(const HiraTree* tree, const void* new_keys, const void* new_values,
                            int32_t m, int32_t* state, void* stream) {

@@ -805,13 +805,13 @@ class HIPIndexer(BaseIndexer):
         self.num_keys += m
 
     def _init_state(self) -> None:
-        st = torch.zeros((self.num_trees, _lib.HIRA_MAX_LEVELS + 2), dtype=torch.int32)
-        for l in range(self.num_levels):
-            st[:, l] = self.size[l]
-        if self.num_levels >= 2:
-            st[:, 0] = 0  # "every level-1 node below this index is full": nothing known yet
-        st[:, _lib.HIRA_MAX_LEVELS] = self.num_keys
-        self._state = st.to(self.device)
+        # (entry 0 of trees with two or more levels: "every level-1 node below this index is full";
+        # nothing known yet)
+        self._state = torch.empty((self.num_trees, _lib.HIRA_MAX_LEVELS + 2), dtype=torch.int32,
+                                  device=self.device)
+        tree = self.tree_struct()
+        _lib.check(_lib.lib().hira_update_state(C.byref(tree), self.num_keys, self._state.data_ptr(),
+                                                _lib.stream_of(self._state.get_device())))
 
     def sync_sizes(self) -> "HIPIndexer":
         """Read the level sizes back after updates with ``sync=False`` (one small copy that

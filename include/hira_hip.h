@@ -287,6 +287,10 @@ int hira_nearest(const void* x, int32_t dtype, int32_t num_trees, int32_t n,
 int hira_update(const HiraTree* tree, const void* new_keys, const void* new_values, int32_t m,
                 int32_t* state, void* stream);
 
+/* The initial state of every tree, as described above, from tree->size and the number of keys
+ * inserted so far: on the stream, without a copy from the host that would wait for it. */
+int hira_update_state(const HiraTree* tree, int32_t num_keys, int32_t* state, void* stream);
+
 /*
  * (Re)compute the 8-bit shadow of a HIRA_TILE16_Q8 index from its bf16 keys, for the key slots
  * [slot_first, slot_first + slot_count) of every tree (whole level-1 nodes: both multiples of

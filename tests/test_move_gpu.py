@@ -27,11 +27,11 @@ def test_enqueue(dtype, trees, cap, at, m, d, dv, gpu_device):
                                            v.data_ptr(), _lib.current_stream(qk.device)))
 
 
-@pytest.mark.parametrize("n", [1, 127, 128, 129, 300])
+@pytest.mark.parametrize("n", [1, 32, 33, 130, 300, 448, 449, 900])
 def test_replace_rows(n, gpu_device):
     from hira_amd import _lib
 
-    trees, rows, d, m, stride = 3, 400, 72, 310, 320
+    trees, rows, d, m, stride = 3, 1000, 72, 310, 320
     a = torch.randn(trees, rows, d, device="cuda").to(torch.bfloat16)
     src = torch.randn(trees, stride, d, device="cuda").to(torch.bfloat16)
     slot, frm = torch.randperm(rows)[:n], torch.randint(0, m, (n,))
