@@ -7,20 +7,40 @@
 
 namespace hira {
 
-// Counting fused into an assignment launch (all NULL: the launch only assigns).
-//   counts  (T, K)    zero when the launch starts; counts[a] += 1 for every item assigned to a
-//   pos     (T, n_c)  the value the item's increment returned: its place inside the bucket
-//   done    (T)       zero when the launch starts: tickets of the tree's workgroups
-//   offsets (T, K+1)  written by the workgroup that draws a tree's last ticket: the exclusive
-//                     prefix sums of counts (offsets[K] = number of items assigned)
-//   zero    (T)       a counter the launch clears (the list of the round after it), or NULL
+// Bucketing fused into an assignment launch (counts NULL: the launch only assigns).
+//   counts  (T, K)       zero when the round starts; counts[a] += 1 for every item assigned to a.  The
+//                        value the item's increment returned is its place in the bucket:
+//   members (T, K, kBucketCap)  the first kBucketCap items of every bucket, in order of arrival
+//   more    (T, n_c)     (centroid, item) of the items behind those, more_count (T) of them.  Such
+//                        buckets are rare (a few seeds of a Lloyd round); what works on them looks for
+//                        their items here.
+// With the places fixed there is no prefix sum over the counts, no tail of a launch that waits for
+// it and no launch that sorts the items into buckets (4.3 + 5 us a round at 8 x 32768 items).
+//   zero    (T)          a counter the launch clears (the list of the round after it), or NULL
+constexpr int kBucketCap = 256;
 struct AssignCounting {
     int32_t* counts;
-    int32_t* pos;
-    int32_t* done;
-    int32_t* offsets;
+    int32_t* members;
+    int2* more;
+    int32_t* more_count;
     int32_t* zero;
 };
+
+// item `it` of tree t was assigned to centroid k >= 0
+__device__ __forceinline__ void count_item(const AssignCounting& ac, int t, int K, int n_c, int k, int it) {
+    const size_t b = (size_t)t * K + k;
+    const int pos = atomicAdd(&ac.counts[b], 1);
+    if (pos < kBucketCap) {
+        ac.members[b * kBucketCap + pos] = it;
+    } else {  // (one atomic for the lanes of the wave that are here)
+        const unsigned long long here = __ballot(1);
+        const int lane = threadIdx.x & 63, leader = __ffsll((long long)here) - 1;
+        int base = 0;
+        if (lane == leader) base = atomicAdd(&ac.more_count[t], __popcll(here));
+        base = __shfl(base, leader, 64);
+        ac.more[(size_t)t * n_c + base + __popcll(here & ((1ull << lane) - 1ull))] = make_int2(k, it);
+    }
+}
 
 // The centroids that still take items, put side by side (packing rounds from the second on: most
 // blocks are full by then, and a round multiplies every unplaced item with every centroid it is
@@ -75,52 +95,41 @@ __device__ __forceinline__ int32_t load_agent(const int32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// End of an assignment workgroup (256 threads, all of them, also of a workgroup without items):
-// a ticket per workgroup; the tree's last one turns the counts into offsets.
-__device__ __forceinline__ void finish_counts(const AssignCounting& ac, int t, int K, int nblocks) {
-    __shared__ int32_t s_last;
-    // (no fence at device scope: it would write the whole L2 back, once per workgroup.  The
-    // increments are device-scope atomics; a thread that has waited for what they return knows
-    // them done, and the last workgroup reads the counts where they were made.)
-    hand_off_release();
-    __syncthreads();  // the workgroup's increments have all returned
-    if (threadIdx.x == 0) s_last = atomicAdd(&ac.done[t], 1) == nblocks - 1 ? 1 : 0;
-    __syncthreads();
-    if (!s_last) return;
-    const int32_t* cnt = ac.counts + (size_t)t * K;
-    int32_t* off = ac.offsets + (size_t)t * (K + 1);
-    const int total = block_exclusive_scan(
-        K, [&](int k) { return load_agent(cnt + k); }, [&](int k, int v) { off[k] = v; });
-    if (threadIdx.x == 0) off[K] = total;
-}
-
 // ---- centroids as operands of v_mfma_f32_16x16x32_bf16 --------------------------------------
-// A tile holds 16 centroids of D = 32 * KS columns, each split into two bf16 numbers, c = hi + lo:
-// 2 * KS * 64 chunks of 16 bytes, chunk (half, s, kb, i) at half*KS*64 + s*64 + kb*16 + i = columns
-// [s*32 + kb*8, +8) of centroid i of the tile.  cn2 (T, Kt*16): ||hi + lo||^2, +inf for a centroid
-// that takes no items.  A tree has Kt tiles (whole stages of the assignment kernel).
+// A tile holds 16 centroids of up to 32 * KS columns (zeros behind the last one), each split into two
+// bf16 numbers, c = hi + lo: 2 * KS * 64 chunks of 16 bytes, chunk (half, s, kb, i) at half*KS*64 + s*64 +
+// kb*16 + i = columns [s*32 + kb*8, +8) of centroid i of the tile.  A tree has Kt tiles (whole stages
+// of the assignment kernels).  Beside them, per centroid (T, Kt*16):
+//   n2   ||hi + lo||^2, +inf for a centroid that takes no items
+//   lo   a bound of ||c - hi||: what a score made of `hi` alone can be off by, per unit of ||x||
+struct CentroidTiles {
+    uint4* tiles;
+    float* n2;
+    float* lo;
+};
+
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
     return (uint32_t)f32_to_bf16_bits(a) | ((uint32_t)f32_to_bf16_bits(b) << 16);
 }
 
 // Centroid k of tree t, D fp32 numbers at c (LDS or memory), into its tile; called by the 64
 // lanes of one wave.
-__device__ __forceinline__ void emit_centroid(const float* c, int D, int Kt, int t, int k,
-                                              bool usable, uint4* tiles, float* cn2) {
+__device__ __forceinline__ void emit_centroid(const float* c, int D, int KS, int Kt, int t, int k,
+                                              bool usable, const CentroidTiles& ct) {
     const int j = threadIdx.x & 63;
-    const int KS = D >> 5;
-    float ss = 0.0f;
-    if (j < D / 8) {
+    float ss = 0.0f, ls = 0.0f;
+    if (j < KS * 4) {
         const int s = j >> 2, kb = j & 3, i = k & 15;
-        uint4* out = tiles + ((size_t)t * Kt + (k >> 4)) * (size_t)(2 * KS * 64);
+        uint4* out = ct.tiles + ((size_t)t * Kt + (k >> 4)) * (size_t)(2 * KS * 64);
         float hi[8], lo[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float v = c[j * 8 + e];
+            const float v = j * 8 + e < D ? c[j * 8 + e] : 0.0f;
             hi[e] = bf16_bits_to_f32(f32_to_bf16_bits(v));
             lo[e] = bf16_bits_to_f32(f32_to_bf16_bits(v - hi[e]));
             const float w = hi[e] + lo[e];
             ss += w * w;
+            ls += (v - hi[e]) * (v - hi[e]);
         }
         out[s * 64 + kb * 16 + i] = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]),
                                                pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
@@ -129,20 +138,51 @@ __device__ __forceinline__ void emit_centroid(const float* c, int D, int Kt, int
                        pack_bf16(lo[6], lo[7]));
     }
 #pragma unroll
-    for (int off = 1; off < 32; off <<= 1) ss += __shfl_xor(ss, off, 64);
-    if (j == 0) cn2[(size_t)t * Kt * 16 + k] = usable ? ss : INFINITY;
+    for (int off = 1; off < 32; off <<= 1) {
+        ss += __shfl_xor(ss, off, 64);
+        ls += __shfl_xor(ls, off, 64);
+    }
+    if (j == 0) {
+        ct.n2[(size_t)t * Kt * 16 + k] = usable ? ss : INFINITY;
+        // (1e-5 of ||c|| per 32 columns: what the roundings of two sums of products can be worth)
+        ct.lo[(size_t)t * Kt * 16 + k] = sqrtf(ls) * 1.0001f + (float)KS * 1e-5f * sqrtf(ss);
+    }
 }
 
+// What an assignment launch works on.
+struct AssignJob {
+    const void* x;          // (T, n_c, D) items
+    int n_c;
+    size_t x_tree_stride;
+    int dtype, D, num_trees;
+    CentroidTiles ct;       // centroids as operand tiles (all, or the open ones)
+    const float* cent;      // (T, K, D) fp32
+    int K;
+    const int32_t* list;    // NULL: all items, else the items list[0 .. *list_count) of each tree
+    const int32_t* list_count;
+    int32_t* assign;        // (T, n_c)
+    float* dist;            // (T, n_c), or NULL: nobody asks for the distances
+    AssignCounting counting;
+    AssignOpen open;
+    int after_approx;       // the approximate pass has been over it: only what it left is left
+    int32_t* unsure;        // (T, n_c) / (T): items the approximate pass leaves to an exact one
+    int32_t* unsure_count;
+};
+
+// (all trees together) more items than this on a list, and the approximate pass takes it
+constexpr int kApproxListItems = 256 * 256;
+
 // assign_mfma.hip
+int assign_ks(int dtype, int D);        // KS of the operand tiles for rows of D columns, 0: none
+bool assign_exact_on_mfma(int dtype, int D);
+bool assign_approx_pays(int dtype, int D, int K);
 int assign_tiles(int K);
 int launch_cent_prep(int dim, const float* cent, int K, int num_trees, const int32_t* fill, int bf,
                      void* tiles, float* cn2, hipStream_t s);
-int launch_assign_mfma(int dim, const void* x, int n_c, size_t x_tree_stride, const void* tiles,
-                       const float* cn2, int K, int num_trees, const int32_t* list,
-                       const int32_t* list_count, size_t list_stride, int32_t* assign, float* dist,
-                       const AssignCounting& counting, const AssignOpen& open, hipStream_t s);
-int launch_open_centroids(int dim, const void* tiles, const float* cn2, const int32_t* fill, int bf,
-                          int K, int num_trees, int32_t* open_ids, int32_t* open_count,
-                          void* open_tiles, float* open_cn2, hipStream_t s);
+int launch_assign_mfma(const AssignJob& job, hipStream_t s);
+int launch_assign_approx(const AssignJob& job, hipStream_t s);
+int launch_open_centroids(int KS, const CentroidTiles& ct, const int32_t* fill, int bf, int K,
+                          int num_trees, int32_t* open_ids, int32_t* open_count,
+                          const CentroidTiles& open, hipStream_t s);
 
 }  // namespace hira

@@ -9,21 +9,20 @@
 // both halves are multiplied, so the distances are as good as fp32 ones for choosing the
 // nearest centroid.
 //
-// k_cent_prep   centroids (T, K, D) fp32 -> tiles of 16 centroids, hi and lo halves, in the
-//               operand layout (chunk (s, kb, i) of 16 bytes at s*64 + kb*16 + i), plus
-//               ||hi + lo||^2; a centroid that is full (fill[k] >= bf) or past K gets +inf.
-//               (hira_nearest; the build's kernels write the tile of a centroid where they make
-//               the centroid, assign.h.)
-// k_assign_mfma a workgroup of 4 waves owns 256 items (64 a wave: 4 operand tiles kept in
-//               registers) and walks all centroid tiles; four tiles at a time are staged once
-//               per workgroup in LDS (double buffered, one barrier a stage).  Lane (n, kb) of a wave sees
-//               the products of its centroid column n with rows 4*kb + j, keeps the best
-//               (value, index) per row, and the 16 columns are merged at the end
-//               (lowest index on ties).  For the build it also counts the items of every
-//               centroid and, in a tree's last workgroup, turns the counts into offsets
-//               (AssignCounting); over a short list of items it spreads them 64 a workgroup; and
-//               it can walk the centroids with room only, put side by side by k_open_scan /
-//               k_open_gather (AssignOpen).
+// k_cent_prep   centroids (T, K, D) fp32 -> operand tiles (assign.h), for hira_nearest; the build's
+//               kernels write the tile of a centroid where they make the centroid.
+// k_assign_mfma every product with both halves: a workgroup of 4 waves owns 256 items (64 a wave: 4
+//               operand tiles kept in registers) and walks all centroid tiles; four tiles at a
+//               time are staged once per workgroup in LDS (double buffered, one barrier a stage).
+//               Lane (n, kb) of a wave sees the products of its centroid column n with rows 4*kb + j,
+//               keeps the best (value, index) per row, and the 16 columns are merged at the end
+//               (lowest index on ties).  Over a list of items it can spread them 64 a workgroup,
+//               and it can walk the centroids with room only, put side by side by k_open_gather
+//               (AssignOpen).
+// k_assign_approx  the same choice for a fraction of the products and of the comparisons: all
+//               centroids by their `hi` halves alone, then the few that could still be the nearest by
+//               the arithmetic of the exact kernel (k_assign_mfma's for its shapes, k_assign_simple's
+//               for any other type and width up to 256 columns).
 #include "assign.h"
 
 namespace hira {
@@ -33,10 +32,16 @@ typedef __attribute__((ext_vector_type(4))) float af32x4_t;
 
 constexpr int kAssignRI = 4;       // operand tiles of 16 items per wave
 constexpr int kAssignThreads = 256;
+__device__ __forceinline__ bool approx_takes(int n_items, int num_trees) {
+    return (long long)n_items * num_trees > kApproxListItems;
+}
 constexpr int kAssignStage = 4;    // centroid tiles staged together: the time they keep the
                                    // matrix cores busy covers the latency of fetching the next
                                    // four (two for D = 256, whose tiles are twice as large)
 constexpr int assign_stage(int KS) { return KS <= 4 ? kAssignStage : kAssignStage / 2; }
+// centroids from which on the approximate pass is worth its second launch
+constexpr int kApproxMinMfma = 256;
+constexpr int kApproxMinSimple = 48;
 
 template <int KS>
 __global__ __launch_bounds__(64) void k_cent_prep(const float* cent, int K, const int32_t* fill,
@@ -73,12 +78,10 @@ __global__ __launch_bounds__(64) void k_cent_prep(const float* cent, int K, cons
     }
 }
 
-// The items of one workgroup: RI operand tiles of 16 items a wave.
-template <int KS, int RI>
-__device__ __forceinline__ void assign_items(
-    const void* x, int n_c, size_t x_tree_stride, const uint4* tiles, const float* cn2, int Kt,
-    const int32_t* list, int n_items, size_t list_stride, int32_t* assign, float* dist, int K,
-    const AssignCounting& ac, const AssignOpen& open) {
+// ---- every product with both halves, many items: 256 a workgroup --------------------------------
+template <int KS>
+__global__ __launch_bounds__(kAssignThreads, 2) void k_assign_mfma(const AssignJob job, const int Kt) {
+    constexpr int RI = kAssignRI;
     constexpr int D = 32 * KS;
     constexpr int TILE_CHUNKS = 2 * KS * 64;                 // hi and lo halves of 16 centroids
     constexpr int TPS = assign_stage(KS);
@@ -92,8 +95,9 @@ __device__ __forceinline__ void assign_items(
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, kb = lane >> 4;  // operand row / centroid column, column block
-    const int t = blockIdx.y;
+    const int t = blockIdx.y, n_c = job.n_c, K = job.K;
     const int first = (blockIdx.x * (kAssignThreads / 64) + wave) * (RI * 16);
+    if (job.counting.zero != nullptr && blockIdx.x == 0 && threadIdx.x == 0) job.counting.zero[t] = 0;
 
     // ---- my items: operand tiles in registers, ||x||^2 of row lane % 16 ------------------
     int item[RI];
@@ -102,16 +106,15 @@ __device__ __forceinline__ void assign_items(
 #pragma unroll
     for (int ri = 0; ri < RI; ++ri) {
         const int pos = first + ri * 16 + n;
-        item[ri] = -1;
-        if (pos < n_items) item[ri] = list ? list[(size_t)t * list_stride + pos] : pos;
+        item[ri] = pos < n_c ? pos : -1;
         float ss = 0.0f;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             a[ri][s] = make_uint4(0, 0, 0, 0);
             if (item[ri] >= 0)
                 a[ri][s] = *reinterpret_cast<const uint4*>(
-                    reinterpret_cast<const uint16_t*>(x) +
-                    ((size_t)t * x_tree_stride + item[ri]) * D + s * 32 + kb * 8);
+                    reinterpret_cast<const uint16_t*>(job.x) +
+                    ((size_t)t * job.x_tree_stride + item[ri]) * D + s * 32 + kb * 8);
             float f[8];
             unpack<bf16_t>(a[ri][s], f);
 #pragma unroll
@@ -133,11 +136,9 @@ __device__ __forceinline__ void assign_items(
 
     // ---- all centroid tiles, staged through LDS TPS at a time (the last stage may hold fewer;
     // the arrays are padded to whole stages, their norms with +inf) ---------------------------
-    const int Ks_all = (Kt + TPS - 1) / TPS;  // stages a tree's arrays hold
-    // (centroids with room side by side: only the stages that hold any)
-    const int Ks = open.count ? min(((open.count[t] + 15) / 16 + TPS - 1) / TPS, Ks_all) : Ks_all;
-    const uint4* tt = tiles + (size_t)t * Ks_all * STAGE_CHUNKS;
-    const float* n2t = cn2 + (size_t)t * Ks_all * (TPS * 16);
+    const int Ks = (Kt + TPS - 1) / TPS;
+    const uint4* tt = job.ct.tiles + (size_t)t * Ks * STAGE_CHUNKS;
+    const float* n2t = job.ct.n2 + (size_t)t * Ks * (TPS * 16);
     uint4 stage[CPT];
     float stage_n2 = 0.0f;
 #pragma unroll
@@ -200,7 +201,7 @@ __device__ __forceinline__ void assign_items(
     // ---- merge the 16 centroid columns of a row group; the wave's 64 results pass through LDS
     // (free behind the loop's last barrier) so that every lane ends up with one item: one store
     // instruction, and one counting instruction, for the whole wave -----------------------------
-    static_assert(RI == 1 || RI == 4, "a result per lane, or per lane of the first 16");
+    static_assert(RI == 4, "a result per lane");
     int* s_g = reinterpret_cast<int*>(s_dyn) + wave * 128;
     float* s_b = reinterpret_cast<float*>(s_g + 64);
 #pragma unroll
@@ -226,8 +227,7 @@ __device__ __forceinline__ void assign_items(
     __builtin_amdgcn_wave_barrier();
     {
         // lane (kb, n) takes row n of operand tile kb: its item and ||x||^2 are its own
-        int g = s_g[lane];  // (meaningless in the lanes that hold no result: kb >= RI)
-        const float b = s_b[lane];
+        const int g = s_g[lane];
         int it = item[0];
         float xx = x2[0];
 #pragma unroll
@@ -236,80 +236,673 @@ __device__ __forceinline__ void assign_items(
                 it = item[ri];
                 xx = x2[ri];
             }
-        if (kb < RI && it >= 0) {
-            if (open.ids != nullptr && g >= 0) g = open.ids[(size_t)t * K + g];  // column -> centroid
-            assign[(size_t)t * n_c + it] = g;
-            dist[(size_t)t * n_c + it] = fmaxf(b + xx, 0.0f);
-            if (ac.counts != nullptr && g >= 0)
-                ac.pos[(size_t)t * n_c + it] = atomicAdd(&ac.counts[(size_t)t * K + g], 1);
+        if (it >= 0) {
+            job.assign[(size_t)t * n_c + it] = g;
+            if (job.dist != nullptr) job.dist[(size_t)t * n_c + it] = fmaxf(s_b[lane] + xx, 0.0f);
+            if (job.counting.counts != nullptr && g >= 0) count_item(job.counting, t, K, n_c, g, it);
         }
     }
 }
 
-// Few items (the later rounds of the packing walk ever shorter lists) are spread over four times
-// as many workgroups, a single operand tile a wave: a workgroup's time is what its walk over all
-// centroid tiles takes, and that walk is four times shorter.  The lists' lengths are known on
-// the device only, so a launch over a list has workgroups for the narrow shape, and each tree
-// picks its shape by the length of its list.
-constexpr int kAssignNarrowItems = 256 * 256;  // (all trees together; measured: beyond this many the
-                                               // wide shape is faster, its tiles read from LDS once for 64 items)
+// ---- every product with both halves, few items: 64 a workgroup, its waves share out the centroids ----
+// Lists (the packing's, or what the approximate pass leaves) and small levels leave most of the chip
+// idle if a wave walks all centroids for items of its own: here the 8 waves of a workgroup hold the
+// same items and walk every eighth tile, straight from memory to registers (nobody shares a tile
+// inside the workgroup), the next one on its way while one is used.  Centroids are the rows of a
+// product, so a lane's results are four centroids of one item per item tile, and what is left at the
+// end is a minimum over four lanes and eight waves.
+// (1024 centroids, 8 x ~1000 items: 52 us with a walk of all tiles per wave, now 13.)
+constexpr int kSplitThreads = 512;
+constexpr int kSplitBlocks = 128;        // workgroups of a tree, at most: they go through a list in strides
 
-template <int KS, bool LISTED>
-__global__ __launch_bounds__(kAssignThreads, 2) void k_assign_mfma(
-    const void* x, int n_c, size_t x_tree_stride, const uint4* tiles, const float* cn2, int Kt,
-    const int32_t* list, const int32_t* list_count, size_t list_stride, int32_t* assign,
-    float* dist, int K, AssignCounting ac, AssignOpen open) {
-    const int t = blockIdx.y;
-    const int n_items = LISTED ? list_count[t] : n_c;
-    const bool narrow = LISTED && (long long)n_items * gridDim.y <= kAssignNarrowItems;
-    const int per_block = (kAssignThreads / 64) * 16 * (narrow ? 1 : kAssignRI);
-    // (a launch that counts: the tree's first workgroup draws a ticket also when there is no item)
-    const int nblocks = max((n_items + per_block - 1) / per_block, 1);
-    if ((int)blockIdx.x >= nblocks) return;  // uniform
-    if (ac.zero != nullptr && blockIdx.x == 0 && threadIdx.x == 0) ac.zero[t] = 0;
-    if ((int)blockIdx.x * per_block < n_items) {
-        if (LISTED && narrow)
-            assign_items<KS, 1>(x, n_c, x_tree_stride, tiles, cn2, Kt, list, n_items, list_stride,
-                                assign, dist, K, ac, open);
-        else
-            assign_items<KS, kAssignRI>(x, n_c, x_tree_stride, tiles, cn2, Kt, list, n_items,
-                                        list_stride, assign, dist, K, ac, open);
+constexpr int split_ri(int KS) { return KS <= 4 ? 4 : 2; }
+
+template <int KS>
+__device__ __forceinline__ void split_items(const AssignJob& job, int Kt, const int32_t* list, int n_items, int block) {
+    constexpr int D = 32 * KS, RI = split_ri(KS), ITEMS = RI * 16, WAVES = kSplitThreads / 64;
+    constexpr int TILE_CHUNKS = 2 * KS * 64;
+    __shared__ float s_b[WAVES][ITEMS];
+    __shared__ int s_g[WAVES][ITEMS];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 15, kb = lane >> 4;
+    const int t = blockIdx.x, n_c = job.n_c, K = job.K;
+
+    // ---- the first tile of the wave, and the items ---------------------------------------------
+    const uint4* tt = job.ct.tiles + (size_t)t * Kt * TILE_CHUNKS + lane;
+    const float* n2t = job.ct.n2 + (size_t)t * Kt * 16 + 4 * kb;
+    const int tiles = job.open.count ? min((job.open.count[t] + 15) / 16, Kt) : (K + 15) / 16;
+    uint4 c[2][2 * KS];
+    float4 c2[2];
+    auto fetch = [&](int tile, uint4 (&to)[2 * KS], float4& n2) {
+        const uint4* src = tt + (size_t)tile * TILE_CHUNKS;
+#pragma unroll
+        for (int s = 0; s < 2 * KS; ++s) to[s] = src[s * 64];
+        n2 = *reinterpret_cast<const float4*>(n2t + tile * 16);
+    };
+    fetch(min(wave, Kt - 1), c[0], c2[0]);
+    int item[RI];
+    uint4 x[RI][KS];
+    float x2[RI];
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+        const int pos = block * ITEMS + ri * 16 + n;
+        item[ri] = -1;
+        if (pos < n_items) item[ri] = list ? list[(size_t)t * n_c + pos] : pos;
     }
-    if (ac.counts != nullptr) finish_counts(ac, t, K, nblocks);
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri)
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            x[ri][s] = *reinterpret_cast<const uint4*>(
+                reinterpret_cast<const uint16_t*>(job.x) +
+                ((size_t)t * job.x_tree_stride + max(item[ri], 0)) * D + s * 32 + kb * 8);
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            float f[8];
+            unpack<bf16_t>(x[ri][s], f);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
+        }
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        x2[ri] = ss;
+    }
+    float best[RI];
+    int arg[RI];
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+        best[ri] = INFINITY;
+        arg[ri] = -1;
+    }
+    auto use = [&](int tile, const uint4 (&ct)[2 * KS], const float4& n2) {
+        af32x4_t acc[RI];
+#pragma unroll
+        for (int ri = 0; ri < RI; ++ri) acc[ri] = af32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+#pragma unroll
+                for (int ri = 0; ri < RI; ++ri)
+                    acc[ri] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(abf16x8_t, ct[half * KS + s]),
+                                                                      __builtin_bit_cast(abf16x8_t, x[ri][s]), acc[ri], 0, 0, 0);
+        const float nn[4] = {n2.x, n2.y, n2.z, n2.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j)  // (increasing: ties keep the lower one)
+#pragma unroll
+            for (int ri = 0; ri < RI; ++ri) {
+                const float v = nn[j] - 2.0f * acc[ri][j];
+                if (v < best[ri]) {
+                    best[ri] = v;
+                    arg[ri] = tile * 16 + 4 * kb + j;
+                }
+            }
+    };
+    int tile = wave;
+    for (; tile + WAVES < tiles; tile += 2 * WAVES) {  // uniform in the wave; no barrier inside
+        fetch(tile + WAVES, c[1], c2[1]);
+        use(tile, c[0], c2[0]);
+        fetch(min(tile + 2 * WAVES, Kt - 1), c[0], c2[0]);
+        use(tile + WAVES, c[1], c2[1]);
+    }
+    if (tile < tiles) use(tile, c[0], c2[0]);
+
+    // ---- one of the four lanes, then of the eight waves, of an item ------------------------------
+    auto better = [](float b, int g, float ob, int og) { return og >= 0 && (g < 0 || ob < b || (ob == b && og < g)); };
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            const float ob = __shfl_xor(best[ri], off, 64);
+            const int og = __shfl_xor(arg[ri], off, 64);
+            if (better(best[ri], arg[ri], ob, og)) {
+                best[ri] = ob;
+                arg[ri] = og;
+            }
+        }
+        if (kb == 0) {
+            s_b[wave][ri * 16 + n] = best[ri];
+            s_g[wave][ri * 16 + n] = arg[ri];
+        }
+    }
+    __syncthreads();
+    if (wave != 0 || lane >= ITEMS) return;
+    // lane (kb, n) takes item n of tile kb
+    float b = s_b[0][lane];
+    int g = s_g[0][lane];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w)
+        if (better(b, g, s_b[w][lane], s_g[w][lane])) {
+            b = s_b[w][lane];
+            g = s_g[w][lane];
+        }
+    int it = item[0];
+    float xx = x2[0];
+#pragma unroll
+    for (int ri = 1; ri < RI; ++ri)
+        if (kb == ri) {
+            it = item[ri];
+            xx = x2[ri];
+        }
+    if (it < 0) return;
+    if (job.open.ids != nullptr && g >= 0) g = job.open.ids[(size_t)t * K + g];  // column -> centroid
+    job.assign[(size_t)t * n_c + it] = g;
+    if (job.dist != nullptr) job.dist[(size_t)t * n_c + it] = fmaxf(b + xx, 0.0f);
+    if (job.counting.counts != nullptr && g >= 0) count_item(job.counting, t, K, n_c, g, it);
+}
+
+template <int KS>
+__global__ __launch_bounds__(kSplitThreads, 2) void k_assign_split(const AssignJob job, const int Kt) {
+    const int t = blockIdx.x;
+    const int32_t* list = job.list;
+    int n_items = list ? job.list_count[t] : job.n_c;
+    if (job.after_approx && (list == nullptr || approx_takes(n_items, gridDim.x))) {
+        list = job.unsure;
+        n_items = job.unsure_count[t];
+    }
+    if (job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t] = 0;
+    for (int b = blockIdx.y; b * split_ri(KS) * 16 < n_items; b += gridDim.y) {  // uniform
+        if (b != (int)blockIdx.y) __syncthreads();  // (the results of the stride before are out of LDS)
+        split_items<KS>(job, Kt, list, n_items, b);
+    }
+}
+
+// ---- the approximate pass -------------------------------------------------------------------
+// score_k = x.c_k - ||c_k||^2 / 2; the nearest centroid has the largest.  With x = xh + xl (bf16 and
+// rest; xl = 0 for bf16 items) and c = hi + rest:
+//   |x.c - xh.hi| <= ||x|| lo_k + ||xl|| ||c_k||      (lo_k: assign.h, rounding of the sums included)
+// so the products with `hi` alone, started from  -||c_k||^2 / 2 + X lo_k + Xl ||c_k||  (X, Xl: the
+// largest norms among the workgroup's items), are never below the exact score, and above it by at most
+// twice that allowance.  A lane keeps its best and second best of them per item, for even and for
+// odd tiles, the centroid's number in the low bits of the value (one instruction, against a comparison and two selections that
+// a separate index takes; what the bits shift the value by counts as error).  Per item the best lower
+// bound decides who is still in the running: of the four lanes that share the item, and their two
+// bests each, those that reach it.  One candidate: that is the nearest.  Several: each is scored by the exact kernel's own
+// arithmetic, and the smallest distance wins, the lowest centroid on ties -- the exact kernel's
+// result bit for bit.  Where a SECOND best is in the running too, a third could be as well, which
+// nobody noted: such items (1-2 % on normal keys) go on a list that the exact kernel takes.
+// Operands: centroids are the rows (A), items the columns (B): a lane's four results of a product are
+// four centroids of ONE item, so best and second are one pair per item tile instead of four, and the
+// start values are a 16-byte read from LDS.
+// What bounds it is the matrix cores: 8 x 131072 items x 4096 centroids take 1690-1740 us with the
+// exact kernel and 890 us with this one, 1010 us where the distances are asked for (1.2 PFLOP/s, what
+// a large matrix product reaches on this card); 8 x 32768 x 1024: 165 -> 84 / 114 us.
+constexpr float kNoScore = -1e37f;  // start value of a centroid that takes no items
+constexpr int kMaxTagBits = 14;     // centroid numbers inside a lane: Kt * 4 of them
+
+// 16 bytes of every lane straight from memory to LDS: lane i's to dst + i (dst: the wave's)
+__device__ __forceinline__ void load_to_lds(const uint4* src, uint4* dst) {
+    __builtin_amdgcn_global_load_lds(reinterpret_cast<const __attribute__((address_space(1))) void*>(
+                                         reinterpret_cast<uintptr_t>(src)),
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+// (ahead of the barrier behind which the others read them)
+__device__ __forceinline__ void arrived_in_lds() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+template <typename T>
+__device__ __forceinline__ void approx_row(const AssignJob& job, size_t row, int c0, bool have,
+                                           uint4& packed, float& x2, float& l2) {
+    // columns [c0, c0 + 8) of a row: bf16 operand chunk, sums of squares of the row and of what bf16 drops
+    constexpr int EPL = Elem<T>::kPerChunk;
+    float f[8];
+#pragma unroll
+    for (int h = 0; h < 8 / EPL; ++h) {
+        uint4 raw = make_uint4(0, 0, 0, 0);
+        if (have && c0 + h * EPL < job.D) raw = load_chunk<T>(job.x, row * job.D, c0 / EPL + h);
+        float g[EPL];
+        unpack<T>(raw, g);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) f[h * EPL + e] = g[e];
+        if (EPL == 8) packed = raw;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x2 += f[e] * f[e];
+    if (EPL == 4) {
+        packed = make_uint4(pack_bf16(f[0], f[1]), pack_bf16(f[2], f[3]), pack_bf16(f[4], f[5]), pack_bf16(f[6], f[7]));
+        float h[8];
+        unpack<bf16_t>(packed, h);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) l2 += (f[e] - h[e]) * (f[e] - h[e]);
+    }
+}
+
+// a float as an unsigned number of the same order
+__device__ __forceinline__ uint32_t ordered_bits(float v) {
+    const uint32_t u = __float_as_uint(v);
+    return u ^ ((u >> 31) ? 0xffffffffu : 0x80000000u);
+}
+__device__ __forceinline__ float from_ordered(uint32_t u) {
+    return __uint_as_float(u ^ ((u >> 31) ? 0x80000000u : 0xffffffffu));
+}
+
+// sum over each aligned group of `lpr` lanes, in the order of group_sum<lpr>
+__device__ __forceinline__ float group_sum_of(float v, int lpr) {
+    if (lpr >= 2) v += dpp_move<0xB1>(v);
+    if (lpr >= 4) v += dpp_move<0x4E>(v);
+    if (lpr >= 8) v += dpp_move<0x141>(v);
+    if (lpr >= 16) v += dpp_move<0x140>(v);
+    if (lpr >= 32) v += __shfl_xor(v, 16, 64);
+    if (lpr >= 64) v += __shfl_xor(v, 32, 64);
+    return v;
+}
+
+constexpr int kApproxPairs = 512;  // (item, candidate) pairs of a wave: 64 items, at most eight each
+
+template <typename T, int KS, int RI, bool LISTED, bool EXACT_MFMA>
+__device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int tag_bits, int n_items, int block) {
+    constexpr int HALF = KS * 64;                       // chunks of the hi half of 16 centroids
+    constexpr int TILE_CHUNKS = 2 * HALF;
+    constexpr int TPS = assign_stage(KS);
+    constexpr int STAGE = TPS * HALF;
+    constexpr int CPT = STAGE / kAssignThreads;
+    constexpr int ITEMS = RI * 16;                      // of a wave
+    constexpr bool SPLIT = sizeof(T) == 4;              // items lose something in bf16
+    static_assert(STAGE % kAssignThreads == 0, "stage does not split over the workgroup");
+    extern __shared__ uint4 s_dyn[];
+    uint4* s_c = s_dyn;                                             // (2, STAGE)
+    float* s_start = reinterpret_cast<float*>(s_dyn + 2 * STAGE);   // (2, TPS * 16)
+    float* s_x = s_start + 2 * TPS * 16;                            // (2, waves): largest norms
+
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const int n = lane & 15, kb = lane >> 4;
+    const int t = blockIdx.x, n_c = job.n_c, K = job.K;
+    const int first = (block * (kAssignThreads / 64) + wave) * ITEMS;
+
+    // ---- my items ----------------------------------------------------------------------------
+    int item[RI];
+    uint4 b[RI][KS];
+    float x2[RI];
+    float X = 0.0f, Xl = 0.0f;
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+        const int pos = first + ri * 16 + n;
+        item[ri] = -1;
+        if (pos < n_items) item[ri] = LISTED ? job.list[(size_t)t * n_c + pos] : pos;
+    }
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+        float ss = 0.0f, ls = 0.0f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            approx_row<T>(job, (size_t)t * job.x_tree_stride + max(item[ri], 0), s * 32 + kb * 8, item[ri] >= 0, b[ri][s], ss, ls);
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        x2[ri] = ss;
+        X = fmaxf(X, ss);
+        if (SPLIT) {
+            ls += __shfl_xor(ls, 16, 64);
+            ls += __shfl_xor(ls, 32, 64);
+            Xl = fmaxf(Xl, ls);
+        }
+    }
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) {
+        X = fmaxf(X, __shfl_xor(X, off, 64));
+        if (SPLIT) Xl = fmaxf(Xl, __shfl_xor(Xl, off, 64));
+    }
+    if (lane == 0) {
+        s_x[wave] = X;
+        s_x[4 + wave] = Xl;
+    }
+    __syncthreads();
+    X = fmaxf(fmaxf(s_x[0], s_x[1]), fmaxf(s_x[2], s_x[3]));
+    X = sqrtf(X) * 1.0001f;
+    if (SPLIT) {
+        Xl = fmaxf(fmaxf(s_x[4], s_x[5]), fmaxf(s_x[6], s_x[7]));
+        Xl = sqrtf(Xl) * 1.0001f;
+    }
+
+    float best[2][RI], second[2][RI];  // of the even tiles, of the odd ones
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) best[0][ri] = second[0][ri] = best[1][ri] = second[1][ri] = -INFINITY;
+    const uint32_t keep = ~((1u << tag_bits) - 1u);
+
+    // ---- all centroid tiles --------------------------------------------------------------------
+    const int Ks_all = (Kt + TPS - 1) / TPS;
+    const int Ks = job.open.count ? min(((job.open.count[t] + 15) / 16 + TPS - 1) / TPS, Ks_all) : Ks_all;
+    const uint4* tt = job.ct.tiles + (size_t)t * Ks_all * TPS * TILE_CHUNKS;
+    const float* n2t = job.ct.n2 + (size_t)t * Ks_all * (TPS * 16);
+    const float* lot = job.ct.lo + (size_t)t * Ks_all * (TPS * 16);
+    const int q = threadIdx.x & (TPS * 16 - 1);
+    auto put_start = [&](int buf, float n2, float lo) {
+        // (1e-5 of the squared norm: what the rounding of the norm can be worth)
+        float v = fmaf(X, lo, -0.5f * n2 + 1e-5f * n2);
+        if (SPLIT) v = fmaf(Xl, sqrtf(n2), v);
+        s_start[buf * TPS * 16 + q] = n2 < INFINITY ? v : kNoScore;  // (every wave the same: no branch)
+    };
+    // (of a tile only the hi half is fetched)
+    uint32_t from[CPT];
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+        const int ci = c * kAssignThreads + (int)threadIdx.x;
+        from[c] = (uint32_t)(ci / HALF * TILE_CHUNKS + ci % HALF);
+    }
+    auto fetch = [&](int st, int buf) {
+        const uint4* src = tt + (size_t)st * (TPS * TILE_CHUNKS);
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) load_to_lds(src + from[c], s_c + buf * STAGE + c * kAssignThreads + wave_u * 64);
+    };
+    if (Ks > 0) {
+        fetch(0, 0);
+        put_start(0, n2t[q], lot[q]);
+    }
+    arrived_in_lds();
+    __syncthreads();
+    // The results of a tile are looked at while the next tile's products are made: a product keeps the
+    // matrix cores busy for the time of four vector instructions, three of which deal with a result.
+    // The order is the one written here (left to itself the compiler makes all products of a stage
+    // first and looks at all results behind them: 1.3 ms instead of 0.9 at 8 x 131072 x 4096).
+    af32x4_t acc[2][RI];
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) acc[1][ri] = af32x4_t{-3e38f, -3e38f, -3e38f, -3e38f};
+    uint32_t keep_v;  // (in a vector register: with `tag` in a scalar one the bits are one instruction)
+    asm volatile("v_mov_b32 %0, %1" : "=v"(keep_v) : "s"(keep));
+    auto look = [&](int of, uint32_t tag, int o) {
+        const int j = o / RI, ri = o % RI;
+        const float v = __uint_as_float((__float_as_uint(acc[of][ri][j]) & keep_v) | (tag + j));
+        second[of][ri] = __builtin_amdgcn_fmed3f(best[of][ri], second[of][ri], v);
+        asm("v_max_f32 %0, %0, %1" : "+v"(best[of][ri]) : "v"(v));  // (fmaxf is two: it quiets v first)
+    };
+    constexpr int PRODUCTS = KS * RI, RESULTS = 4 * RI;
+    for (int st = 0; st < Ks; ++st) {
+        const int buf = st & 1;
+        const uint4* cbuf = s_c + buf * STAGE + lane;
+        const float* sbuf = s_start + buf * TPS * 16 + 4 * kb;
+        const int nst = min(st + 1, Ks - 1);
+        fetch(nst, buf ^ 1);
+        const float next_n2 = n2t[nst * (TPS * 16) + q], next_lo = lot[nst * (TPS * 16) + q];
+        abf16x8_t a[2][KS];
+        af32x4_t start[2];
+#pragma unroll
+        for (int s = 0; s < KS; ++s) a[0][s] = __builtin_bit_cast(abf16x8_t, cbuf[s * 64]);
+        start[0] = *reinterpret_cast<const af32x4_t*>(sbuf);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ti = 0; ti < TPS; ++ti) {
+            const int me = ti & 1;
+            const uint32_t tag = (uint32_t)max(st * TPS + ti - 1, 0) * 4u;  // of the tile before
+#pragma unroll
+            for (int p = 0; p < PRODUCTS; ++p) {
+                const int s = p / RI, ri = p % RI;
+                acc[me][ri] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    a[me][s], __builtin_bit_cast(abf16x8_t, b[ri][s]), s == 0 ? start[me] : acc[me][ri], 0, 0, 0);
+#pragma unroll
+                for (int o = p * RESULTS / PRODUCTS; o < (p + 1) * RESULTS / PRODUCTS; ++o) look(me ^ 1, tag, o);
+                if (p == 1 && ti + 1 < TPS) {  // the next tile's operands
+#pragma unroll
+                    for (int s2 = 0; s2 < KS; ++s2)
+                        a[me ^ 1][s2] = __builtin_bit_cast(abf16x8_t, cbuf[(ti + 1) * HALF + s2 * 64]);
+                    start[me ^ 1] = *reinterpret_cast<const af32x4_t*>(sbuf + (ti + 1) * 16);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        put_start(buf ^ 1, next_n2, next_lo);
+        arrived_in_lds();
+        __syncthreads();
+    }
+    if (Ks > 0) {
+        static_assert(TPS % 2 == 0, "the last tile's results are in acc[1]");
+#pragma unroll
+        for (int o = 0; o < RESULTS; ++o) look(1, (uint32_t)(Ks * TPS - 1) * 4u, o);
+    }
+
+    // ---- who is still in the running (LDS is free behind the loop's last barrier) -------------------
+    const bool want_dist = job.dist != nullptr;  // uniform: then every item's distance is needed
+    constexpr int WAVE_BYTES = 64 * 8 + kApproxPairs * 8;
+    char* mine = reinterpret_cast<char*>(s_dyn) + wave * WAVE_BYTES;
+    unsigned long long* s_key = reinterpret_cast<unsigned long long*>(mine);  // (64) best (distance, column)
+    int* s_item = reinterpret_cast<int*>(mine + 64 * 8);                      // pairs: item of the wave
+    int* s_col = s_item + kApproxPairs;                                       //        column
+    const float shift = ldexpf(1.0f, tag_bits - 23);
+    s_key[lane] = ~0ull;
+    int npairs = 0;      // uniform in the wave
+    bool unsure[RI];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+        int col[2];
+        bool any[2];
+        float floor_of = -INFINITY;  // the exact score of the best is at least this
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t tag = __float_as_uint(best[e][ri]) & ~keep;
+            col[e] = (int)(tag >> 2) * 16 + 4 * kb + (int)(tag & 3u);
+            any[e] = best[e][ri] > 0.5f * kNoScore && item[ri] >= 0;
+            if (any[e]) {
+                const float n2 = n2t[col[e]], lo = lot[col[e]];
+                float off = 2.0f * (X * lo + 1e-5f * n2);
+                if (SPLIT) off += 2.0f * Xl * sqrtf(n2);
+                if (!EXACT_MFMA) off += 1e-5f * X * X;  // (rounding of sums of squared differences)
+                floor_of = fmaxf(floor_of, best[e][ri] - off - fabsf(best[e][ri]) * shift);
+            }
+        }
+        floor_of = fmaxf(floor_of, __shfl_xor(floor_of, 16, 64));
+        floor_of = fmaxf(floor_of, __shfl_xor(floor_of, 32, 64));
+        bool in[2];
+        int un = 0, cands = 0;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            in[e] = any[e] && best[e][ri] + fabsf(best[e][ri]) * shift >= floor_of;
+            // (a value next to zero does not hold its tag)
+            un |= any[e] && (!(second[e][ri] + fabsf(second[e][ri]) * shift < floor_of) || fabsf(best[e][ri]) < 1e-30f);
+            cands += in[e];
+        }
+        un |= __shfl_xor(un, 16, 64);
+        un |= __shfl_xor(un, 32, 64);
+        cands += __shfl_xor(cands, 16, 64);
+        cands += __shfl_xor(cands, 32, 64);
+        un |= cands == 0;  // (rows with numbers that are none: as the exact kernel has it)
+        unsure[ri] = un;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const bool score = in[e] && !un && (want_dist || cands > 1);
+            const unsigned long long bal = __ballot(score);
+            if (score) {
+                const int at = npairs + __popcll(bal & ((1ull << lane) - 1ull));
+                s_item[at] = ri * 16 + n;
+                s_col[at] = col[e];
+            }
+            npairs += __popcll(bal);
+            if (in[e] && !un && !score) s_key[ri * 16 + n] = (unsigned long long)(uint32_t)col[e];  // (the only one)
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+
+    // ---- the candidates' exact distances ---------------------------------------------------------
+    if constexpr (EXACT_MFMA) {
+        // sixteen pairs at a time: row i of the A operand is the pair's centroid, column i of B its
+        // item, the result on the diagonal; the products in the exact kernel's order
+        for (int p0 = 0; p0 < npairs; p0 += 16) {  // uniform in the wave
+            const int pi = min(p0 + n, npairs - 1);
+            const int it_local = s_item[pi], col = s_col[pi];
+            int it = 0;
+#pragma unroll
+            for (int ri = 0; ri < RI; ++ri) {
+                const int o = __shfl(item[ri], it_local & 15, 64);
+                if ((it_local >> 4) == ri) it = o;
+            }
+            const uint4* ct = tt + (size_t)(col >> 4) * TILE_CHUNKS + kb * 16 + (col & 15);
+            const uint4* xt = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(job.x) +
+                                                             ((size_t)t * job.x_tree_stride + it) * (32 * KS) + kb * 8);
+            uint4 ch[KS], cl[KS], xr[KS];
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                ch[s] = ct[s * 64];
+                cl[s] = ct[HALF + s * 64];
+                xr[s] = xt[s * 4];
+            }
+            const float n2 = n2t[col];
+            af32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(abf16x8_t, ch[s]), __builtin_bit_cast(abf16x8_t, xr[s]), acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(abf16x8_t, cl[s]), __builtin_bit_cast(abf16x8_t, xr[s]), acc, 0, 0, 0);
+            }
+            // the diagonal: row n = 4 * kb + j of column n
+            if (kb == (n >> 2) && p0 + n < npairs) {
+                const int j = n & 3;
+                const float d = j == 0 ? acc[0] : j == 1 ? acc[1] : j == 2 ? acc[2] : acc[3];
+                const float v = n2 - 2.0f * d;
+                atomicMin(&s_key[it_local], ((unsigned long long)ordered_bits(v) << 32) | (uint32_t)col);
+            }
+        }
+    } else {
+        // LPR lanes a pair, as the vector-ALU kernel holds an item and a centroid
+        constexpr int EPL = Elem<T>::kPerChunk;
+        int lpr = 2;
+        while (lpr * EPL < job.D) lpr <<= 1;
+        const int rpw = 64 / lpr, rg = lane / lpr, ch = lane % lpr;
+        const bool chunk_ok = ch * EPL < job.D;
+        for (int p0 = 0; p0 < npairs; p0 += rpw) {  // uniform in the wave
+            const int pi = min(p0 + rg, npairs - 1);
+            const int it_local = s_item[pi], col = s_col[pi];
+            int it = 0;
+#pragma unroll
+            for (int ri = 0; ri < RI; ++ri) {
+                const int o = __shfl(item[ri], it_local & 15, 64);
+                if ((it_local >> 4) == ri) it = o;
+            }
+            const int k = job.open.ids != nullptr ? job.open.ids[(size_t)t * K + col] : col;
+            uint4 raw = make_uint4(0, 0, 0, 0);
+            float c[EPL];
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) c[e] = 0.0f;
+            if (chunk_ok) {
+                raw = load_chunk<T>(job.x, ((size_t)t * job.x_tree_stride + it) * job.D, ch);
+                const float* cp = job.cent + ((size_t)t * K + k) * job.D + ch * EPL;
+#pragma unroll
+                for (int e = 0; e < EPL; e += 4) {
+                    const float4 v = *reinterpret_cast<const float4*>(cp + e);
+                    c[e] = v.x, c[e + 1] = v.y, c[e + 2] = v.z, c[e + 3] = v.w;
+                }
+            }
+            float x[EPL];
+            unpack<T>(raw, x);
+            float ss = 0.0f;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+                const float df = x[e] - c[e];
+                ss += df * df;
+            }
+            ss = group_sum_of(ss, lpr);
+            if (ch == 0 && p0 + rg < npairs)
+                atomicMin(&s_key[it_local], ((unsigned long long)ordered_bits(ss) << 32) | (uint32_t)col);
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // ---- lane (kb, n) takes item n of tile kb ----------------------------------------------------
+    int it = -1;
+    float xx = 0.0f;
+    bool un = false;
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri)
+        if (kb == ri) {
+            it = item[ri];
+            xx = x2[ri];
+            un = unsure[ri];
+        }
+    const bool listed_later = it >= 0 && un;
+    if (__ballot(listed_later) != 0ull) {
+        const unsigned long long bal = __ballot(listed_later);
+        int base = 0;
+        if (lane == __ffsll((long long)bal) - 1) base = atomicAdd(&job.unsure_count[t], __popcll(bal));
+        base = __shfl(base, __ffsll((long long)bal) - 1, 64);
+        if (listed_later) job.unsure[(size_t)t * n_c + base + __popcll(bal & ((1ull << lane) - 1ull))] = it;
+    }
+    if (it >= 0 && !un) {
+        const unsigned long long key = s_key[lane];
+        int g = -1;
+        float d = INFINITY;
+        if (key != ~0ull) {
+            g = (int)(uint32_t)key;
+            if (job.open.ids != nullptr) g = job.open.ids[(size_t)t * K + g];  // column -> centroid
+            const float v = from_ordered((uint32_t)(key >> 32));
+            d = EXACT_MFMA ? fmaxf(v + xx, 0.0f) : v;
+        }
+        job.assign[(size_t)t * n_c + it] = g;
+        if (want_dist) job.dist[(size_t)t * n_c + it] = d;
+        if (job.counting.counts != nullptr && g >= 0) count_item(job.counting, t, K, n_c, g, it);
+    }
+}
+
+template <typename T, int KS, bool LISTED, bool EXACT_MFMA>
+__global__ __launch_bounds__(kAssignThreads, 2) void k_assign_approx(const AssignJob job, const int Kt,
+                                                                     const int tag_bits) {
+    // (trees in the fast index: the workgroups of a tree run behind the same L2s, which hold its tiles)
+    const int t = blockIdx.x;
+    constexpr int RI = KS <= 4 ? 4 : 2;
+    const int n_items = LISTED ? job.list_count[t] : job.n_c;
+    if (LISTED && EXACT_MFMA && !approx_takes(n_items, gridDim.x)) return;  // (k_assign_split's)
+    const bool narrow = LISTED && !EXACT_MFMA && !approx_takes(n_items, gridDim.x);
+    const int per_block = (kAssignThreads / 64) * 16 * (narrow ? 1 : RI);
+    if (!EXACT_MFMA && job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t] = 0;
+    for (int b = blockIdx.y; b * per_block < n_items; b += gridDim.y) {  // uniform
+        if (b != (int)blockIdx.y) __syncthreads();
+        if (LISTED && !EXACT_MFMA && narrow) approx_items<T, KS, 1, LISTED, EXACT_MFMA>(job, Kt, tag_bits, n_items, b);
+        else approx_items<T, KS, RI, LISTED, EXACT_MFMA>(job, Kt, tag_bits, n_items, b);
+    }
 }
 
 // ---- the centroids with room, side by side ---------------------------------------------------
-// one workgroup per tree: which centroids are not full, in order
-__global__ __launch_bounds__(256) void k_open_scan(const int32_t* fill, int K, int bf, int32_t* ids,
-                                                   int32_t* count) {
-    const int t = blockIdx.x;
-    const int32_t* ft = fill + (size_t)t * K;
-    int32_t* it = ids + (size_t)t * K;
-    const int total = block_exclusive_scan(
-        K, [&](int k) { return ft[k] < bf ? 1 : 0; },
-        [&](int k, int v) {
-            if (ft[k] < bf) it[v] = k;
-        });
-    if (threadIdx.x == 0) count[t] = total;
-}
-
-// one wave per tile of the side-by-side arrays: column i of tile c is centroid ids[16 c + i]; the
-// columns behind the last one, up to the end of the stage, are zeros with norm +inf
+// A workgroup per four tiles of the side-by-side arrays: column i of tile c is the centroid that is the
+// (16 c + i)-th not full; the columns behind the last one, up to the end of the stage, are zeros
+// that take no items.  Every workgroup counts for itself which centroids those are (a walk over the
+// tree's fill counts, 16 KiB at 4096 centroids, instead of a launch of its own ahead: 4.7 us).
 template <int KS>
-__global__ __launch_bounds__(64) void k_open_gather(const uint4* tiles, const float* cn2,
-                                                    const int32_t* ids, const int32_t* count, int K,
-                                                    int Kt, uint4* otiles, float* ocn2) {
+__global__ __launch_bounds__(256) void k_open_gather(const CentroidTiles ct, const int32_t* fill, int K,
+                                                     int bf, int Kt, int32_t* ids, int32_t* count,
+                                                     const CentroidTiles open) {
     constexpr int TILE_CHUNKS = 2 * KS * 64;
     constexpr int TPS = assign_stage(KS);
-    const int tile = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
-    const int no = count[t];
-    const int need = min((((no + 15) / 16 + TPS - 1) / TPS) * TPS, Kt);  // tiles the assignment will walk
+    __shared__ int s_ids[64];
+    __shared__ int s_w[4];
+    const int t = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int first = blockIdx.x * 64;  // my columns: [first, first + 64)
+    const int32_t* ft = fill + (size_t)t * K;
+    if (threadIdx.x < 64) s_ids[threadIdx.x] = -1;
+    int before = 0;  // open centroids ahead of the stretch
+    for (int k0 = 0; k0 < K; k0 += 1024) {  // uniform
+        int open_mask = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int k = k0 + (int)threadIdx.x * 4 + j;
+            if (k < K && ft[k] < bf) open_mask |= 1 << j;
+        }
+        const int mine = __popc(open_mask);
+        int inc = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += o;
+        }
+        if (lane == 63) s_w[wave] = inc;
+        __syncthreads();
+        int at = before + inc - mine;
+        for (int w = 0; w < wave; ++w) at += s_w[w];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if ((open_mask >> j) & 1) {
+                const int k = k0 + (int)threadIdx.x * 4 + j;
+                if (blockIdx.x == 0) ids[(size_t)t * K + at] = k;
+                if (at >= first && at < first + 64) s_ids[at - first] = k;
+                ++at;
+            }
+        before += s_w[0] + s_w[1] + s_w[2] + s_w[3];
+        __syncthreads();
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) count[t] = before;
+    const int need = min((((before + 15) / 16 + TPS - 1) / TPS) * TPS, Kt);  // tiles the assignment will walk
+    const int tile = blockIdx.x * 4 + wave;
     if (tile >= need) return;
-    const uint4* src = tiles + (size_t)t * Kt * TILE_CHUNKS;
-    uint4* dst = otiles + ((size_t)t * Kt + tile) * TILE_CHUNKS;
+    const uint4* src = ct.tiles + (size_t)t * Kt * TILE_CHUNKS;
+    uint4* dst = open.tiles + ((size_t)t * Kt + tile) * TILE_CHUNKS;
     const int i = lane & 15;
-    const int col = tile * 16 + i;
-    const int k = col < no ? ids[(size_t)t * K + col] : -1;
+    const int k = s_ids[wave * 16 + i];
 #pragma unroll
     for (int c0 = 0; c0 < TILE_CHUNKS; c0 += 64) {
         const int ci = c0 + lane;  // (ci % 16 == i: a lane always moves chunks of its own column)
@@ -317,22 +910,23 @@ __global__ __launch_bounds__(64) void k_open_gather(const uint4* tiles, const fl
         if (k >= 0) v = src[(size_t)(k >> 4) * TILE_CHUNKS + (ci - i) + (k & 15)];
         dst[ci] = v;
     }
-    if (lane < 16) ocn2[((size_t)t * Kt + tile) * 16 + i] = k >= 0 ? cn2[(size_t)t * Kt * 16 + k] : INFINITY;
+    if (lane < 16) {
+        const size_t o = ((size_t)t * Kt + tile) * 16 + i, c = (size_t)t * Kt * 16 + max(k, 0);
+        open.n2[o] = k >= 0 ? ct.n2[c] : INFINITY;
+        open.lo[o] = k >= 0 ? ct.lo[c] : 0.0f;
+    }
 }
 
-int launch_open_centroids(int dim, const void* tiles, const float* cn2, const int32_t* fill, int bf,
-                          int K, int num_trees, int32_t* open_ids, int32_t* open_count,
-                          void* open_tiles, float* open_cn2, hipStream_t s) {
+int launch_open_centroids(int KS, const CentroidTiles& ct, const int32_t* fill, int bf, int K,
+                          int num_trees, int32_t* open_ids, int32_t* open_count,
+                          const CentroidTiles& open, hipStream_t s) {
     const int Kt = assign_tiles(K);
-    hipLaunchKernelGGL(k_open_scan, dim3(num_trees), dim3(256), 0, s, fill, K, bf, open_ids, open_count);
-    const dim3 grid(Kt, num_trees);
-    const uint4* tl = reinterpret_cast<const uint4*>(tiles);
-    uint4* ot = reinterpret_cast<uint4*>(open_tiles);
-    switch (dim) {
-        case 64: hipLaunchKernelGGL((k_open_gather<2>), grid, dim3(64), 0, s, tl, cn2, open_ids, open_count, K, Kt, ot, open_cn2); break;
-        case 128: hipLaunchKernelGGL((k_open_gather<4>), grid, dim3(64), 0, s, tl, cn2, open_ids, open_count, K, Kt, ot, open_cn2); break;
-        case 256: hipLaunchKernelGGL((k_open_gather<8>), grid, dim3(64), 0, s, tl, cn2, open_ids, open_count, K, Kt, ot, open_cn2); break;
-        default: return fail(HIRA_EINVAL, "MFMA assignment: dim %d", dim);
+    const dim3 grid((Kt + 3) / 4, num_trees);
+    switch (KS) {
+        case 2: hipLaunchKernelGGL((k_open_gather<2>), grid, dim3(256), 0, s, ct, fill, K, bf, Kt, open_ids, open_count, open); break;
+        case 4: hipLaunchKernelGGL((k_open_gather<4>), grid, dim3(256), 0, s, ct, fill, K, bf, Kt, open_ids, open_count, open); break;
+        case 8: hipLaunchKernelGGL((k_open_gather<8>), grid, dim3(256), 0, s, ct, fill, K, bf, Kt, open_ids, open_count, open); break;
+        default: return fail(HIRA_EINVAL, "open centroids: KS %d", KS);
     }
     return HIRA_OK;
 }
@@ -342,6 +936,11 @@ int assign_tiles(int K) {
     const int kt = (K + 15) / 16;
     return (kt + kAssignStage - 1) / kAssignStage * kAssignStage;
 }
+
+int assign_ks(int dtype, int D) { return D <= 64 ? 2 : D <= 128 ? 4 : D <= 256 ? 8 : 0; }
+
+// bf16 rows of 64, 128 or 256 columns have an exact kernel on the matrix cores
+bool assign_exact_on_mfma(int dtype, int D) { return dtype == HIRA_BF16 && (D == 64 || D == 128 || D == 256); }
 
 // hi/lo tiles and norms of the centroids of every tree
 int launch_cent_prep(int dim, const float* cent, int K, int num_trees, const int32_t* fill, int bf,
@@ -358,48 +957,108 @@ int launch_cent_prep(int dim, const float* cent, int K, int num_trees, const int
     return HIRA_OK;
 }
 
-// nearest usable centroid of every item (or of the items list[0 .. *list_count) of each tree)
-int launch_assign_mfma(int dim, const void* x, int n_c, size_t x_tree_stride, const void* tiles,
-                       const float* cn2, int K, int num_trees, const int32_t* list,
-                       const int32_t* list_count, size_t list_stride, int32_t* assign, float* dist,
-                       const AssignCounting& counting, const AssignOpen& open, hipStream_t s) {
-    const int Kt = assign_tiles(K);
-    // (a launch over a list: workgroups for the narrow shape, see kAssignNarrowItems)
-    const int per_block = (kAssignThreads / 64) * (list != nullptr ? 1 : kAssignRI) * 16;
-    const int tps = assign_stage(dim / 32);
-    const size_t smem = 2 * (size_t)tps * (2 * (dim / 32) * 64) * sizeof(uint4) + 2 * (size_t)tps * 16 * sizeof(float);
-    const dim3 grid((n_c + per_block - 1) / per_block, num_trees);
-    const uint4* tl = reinterpret_cast<const uint4*>(tiles);
-    constexpr int kMaxDevices = 64;
+// The current device, for what is asked once per kernel and device.
+constexpr int kMaxDevices = 64;
+static int current_device() {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
-        return fail(HIRA_ELAUNCH, "MFMA assignment: no current device");
-    switch (dim) {
-#define HIRA_ASSIGN_MFMA_L(KS, LISTED)                                                              \
-    {                                                                                               \
-        /* more than 64 KiB of dynamic LDS has to be asked for: once per kernel and device */       \
-        static int asked[kMaxDevices];                                                              \
-        if (__atomic_load_n(&asked[dev], __ATOMIC_RELAXED) == 0) {                                  \
-            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_assign_mfma<KS, LISTED>),      \
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) \
-                return fail(HIRA_ELAUNCH, "MFMA assignment: %zu bytes of LDS refused", smem);          \
-            __atomic_store_n(&asked[dev], 1, __ATOMIC_RELAXED);                                     \
-        }                                                                                           \
-        hipLaunchKernelGGL((k_assign_mfma<KS, LISTED>), grid, dim3(kAssignThreads), smem, s, x, n_c, \
-                           x_tree_stride, tl, cn2, Kt, list, list_count, list_stride, assign, dist, \
-                           K, counting, open);                                                      \
-    }
-#define HIRA_ASSIGN_MFMA(KS)                                                                        \
-    if (list != nullptr) HIRA_ASSIGN_MFMA_L(KS, true) else HIRA_ASSIGN_MFMA_L(KS, false)            \
-    break;
-        case 64: HIRA_ASSIGN_MFMA(2)
-        case 128: HIRA_ASSIGN_MFMA(4)
-        case 256: HIRA_ASSIGN_MFMA(8)
-#undef HIRA_ASSIGN_MFMA
-#undef HIRA_ASSIGN_MFMA_L
-        default: return fail(HIRA_EINVAL, "MFMA assignment: dim %d", dim);
+    return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices ? dev : -1;
+}
+// (more than 64 KiB of dynamic LDS has to be asked for: once per kernel and device)
+static int ask_for_lds(const void* kernel, size_t smem, int* asked, int dev) {
+    if (dev < 0) return fail(HIRA_ELAUNCH, "assignment: no current device");
+    if (__atomic_load_n(&asked[dev], __ATOMIC_RELAXED) == 0) {
+        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+            return fail(HIRA_ELAUNCH, "assignment: %zu bytes of LDS refused", smem);
+        __atomic_store_n(&asked[dev], 1, __ATOMIC_RELAXED);
     }
     return HIRA_OK;
+}
+
+template <int KS>
+static int launch_exact(const AssignJob& job, hipStream_t s) {
+    const int Kt = assign_tiles(job.K);
+    // Many items walk the centroids 256 a workgroup, every tile read once for all of them; lists, whose
+    // length only the device knows, and few items, which would leave the chip idle, 64 a workgroup.
+    if (job.list != nullptr || job.after_approx || (long long)job.n_c * job.num_trees <= kApproxListItems) {
+        const int per_block = split_ri(KS) * 16, blocks = (job.n_c + per_block - 1) / per_block;
+        hipLaunchKernelGGL((k_assign_split<KS>), dim3(job.num_trees, blocks < kSplitBlocks ? blocks : kSplitBlocks),
+                           dim3(kSplitThreads), 0, s, job, Kt);
+        return HIRA_OK;
+    }
+    static int asked[kMaxDevices];
+    constexpr int TPS = assign_stage(KS);
+    constexpr size_t smem = 2 * (size_t)TPS * (2 * KS * 64) * sizeof(uint4) + 2 * (size_t)TPS * 16 * sizeof(float);
+    if (const int rc = ask_for_lds(reinterpret_cast<const void*>(&k_assign_mfma<KS>), smem, asked, current_device()))
+        return rc;
+    const int per_block = (kAssignThreads / 64) * kAssignRI * 16;
+    hipLaunchKernelGGL((k_assign_mfma<KS>), dim3((job.n_c + per_block - 1) / per_block, job.num_trees),
+                       dim3(kAssignThreads), smem, s, job, Kt);
+    return HIRA_OK;
+}
+
+// nearest usable centroid of every item, or of the items list[0 .. *list_count) of each tree, or of those
+// the approximate pass over either left
+int launch_assign_mfma(const AssignJob& job, hipStream_t s) {
+    switch (job.D) {
+        case 64: return launch_exact<2>(job, s);
+        case 128: return launch_exact<4>(job, s);
+        case 256: return launch_exact<8>(job, s);
+        default: return fail(HIRA_EINVAL, "MFMA assignment: dim %d", job.D);
+    }
+}
+
+template <typename T, int KS, bool LISTED, bool EXACT_MFMA>
+static int launch_approx(const AssignJob& job, hipStream_t s) {
+    static int asked[kMaxDevices];
+    constexpr int TPS = assign_stage(KS);
+    // (the pairs lie where the tiles were)
+    constexpr size_t tiles = 2 * (size_t)TPS * KS * 64 * sizeof(uint4) + (2 * (size_t)TPS * 16 + 8) * sizeof(float);
+    constexpr size_t pairs = 4 * (64 * 8 + kApproxPairs * 8), smem = tiles > pairs ? tiles : pairs;
+    if (const int rc = ask_for_lds(reinterpret_cast<const void*>(&k_assign_approx<T, KS, LISTED, EXACT_MFMA>), smem, asked,
+                                   current_device()))
+        return rc;
+    constexpr int RI = KS <= 4 ? 4 : 2;
+    const int per_block = (kAssignThreads / 64) * (LISTED && !EXACT_MFMA ? 1 : RI) * 16;
+    const int blocks = min((job.n_c + per_block - 1) / per_block, 65535);  // (they go on in strides)
+    const int Kt = assign_tiles(job.K);
+    int tag_bits = 1;
+    while ((1 << tag_bits) < Kt * 4) ++tag_bits;
+    if (tag_bits > kMaxTagBits) return fail(HIRA_EINVAL, "approximate assignment: %d centroids", job.K);
+    hipLaunchKernelGGL((k_assign_approx<T, KS, LISTED, EXACT_MFMA>), dim3(job.num_trees, blocks), dim3(kAssignThreads),
+                       smem, s, job, Kt, tag_bits);
+    return HIRA_OK;
+}
+
+template <typename T, int KS, bool EXACT_MFMA>
+static int launch_approx_l(const AssignJob& job, hipStream_t s) {
+    return job.list != nullptr ? launch_approx<T, KS, true, EXACT_MFMA>(job, s)
+                               : launch_approx<T, KS, false, EXACT_MFMA>(job, s);
+}
+
+int launch_assign_approx(const AssignJob& job, hipStream_t s) {
+    const int KS = assign_ks(job.dtype, job.D);
+    if (assign_exact_on_mfma(job.dtype, job.D)) {
+        if (KS == 2) return launch_approx_l<bf16_t, 2, true>(job, s);
+        if (KS == 4) return launch_approx_l<bf16_t, 4, true>(job, s);
+        return launch_approx_l<bf16_t, 8, true>(job, s);
+    }
+    if (job.dtype == HIRA_BF16) {
+        if (KS == 2) return launch_approx_l<bf16_t, 2, false>(job, s);
+        if (KS == 4) return launch_approx_l<bf16_t, 4, false>(job, s);
+        if (KS == 8) return launch_approx_l<bf16_t, 8, false>(job, s);
+    } else {
+        if (KS == 2) return launch_approx_l<float, 2, false>(job, s);
+        if (KS == 4) return launch_approx_l<float, 4, false>(job, s);
+        if (KS == 8) return launch_approx_l<float, 8, false>(job, s);
+    }
+    return fail(HIRA_EINVAL, "approximate assignment: %d columns", job.D);
+}
+
+// whether the approximate pass can take a level of K centroids over rows of D columns, and pays: it
+// costs a launch for the items it is unsure of, so the exact kernel must have something to lose
+bool assign_approx_pays(int dtype, int D, int K) {
+    if (assign_ks(dtype, D) == 0 || assign_tiles(K) * 4 > (1 << kMaxTagBits)) return false;
+    return K >= (assign_exact_on_mfma(dtype, D) ? kApproxMinMfma : kApproxMinSimple);
 }
 
 }  // namespace hira

@@ -33,6 +33,10 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 
+// what the phases of a level count, per tree: workgroups that are done, items on the two lists, items
+// behind the buckets (of this round, of the next), items the approximate assignment leaves
+constexpr int kBuildCounters = 6;
+
 __global__ void k_fill_i32(int32_t* p, size_t n, int32_t v) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
@@ -47,17 +51,14 @@ __global__ void k_fill_i32(int32_t* p, size_t n, int32_t v) {
 // ------------------------------------------------------------------------------------
 __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_t* n_live,
                              int32_t* placed, int32_t* fill, int32_t* slots, int32_t* counts,
-                             int32_t* done, int32_t* list_count /* (2, T) */, uint4* tiles,
-                             float* cn2) {
+                             int32_t* counters /* (kBuildCounters, T) */, CentroidTiles ct, int KS) {
     const int t = blockIdx.y, T = gridDim.y;
     const int n_t = n_live ? min(max(n_live[t], 0), n_c) : n_c;
     const int K_t = n_live ? max((n_t + bf - 1) / bf, 1) : K;
     const int stride = gridDim.x * blockDim.x;
     const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
     if (i0 == 0) {
-        done[t] = 0;
-        list_count[t] = 0;
-        list_count[T + t] = 0;
+        for (int c = 0; c < kBuildCounters; ++c) counters[c * T + t] = 0;
     }
     for (int i = i0; i < n_c; i += stride) placed[(size_t)t * n_c + i] = i >= n_t ? 1 : 0;
     for (int i = i0; i < K; i += stride) {
@@ -65,16 +66,18 @@ __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_
         counts[(size_t)t * K + i] = 0;
     }
     for (size_t i = i0; i < (size_t)K * bf; i += stride) slots[(size_t)t * K * bf + i] = -1;
-    if (tiles != nullptr) {
-        const int pad = Kt * 16 - K, cpc = D / 4;  // chunks of a column: hi and lo halves
-        const int KS = D / 32;
+    if (ct.tiles != nullptr) {
+        const int pad = Kt * 16 - K, cpc = KS * 8;  // chunks of a column: hi and lo halves
         for (int i = i0; i < pad * cpc; i += stride) {
             const int k = K + i / cpc, c = i % cpc;
-            const int half = c / (D / 8), j = c % (D / 8);
-            tiles[((size_t)t * Kt + (k >> 4)) * (size_t)(2 * KS * 64) + half * KS * 64 + (j >> 2) * 64 +
-                  (j & 3) * 16 + (k & 15)] = make_uint4(0, 0, 0, 0);
+            const int half = c / (KS * 4), j = c % (KS * 4);
+            ct.tiles[((size_t)t * Kt + (k >> 4)) * (size_t)(2 * KS * 64) + half * KS * 64 + (j >> 2) * 64 +
+                     (j & 3) * 16 + (k & 15)] = make_uint4(0, 0, 0, 0);
         }
-        for (int i = i0; i < pad; i += stride) cn2[(size_t)t * Kt * 16 + K + i] = INFINITY;
+        for (int i = i0; i < pad; i += stride) {
+            ct.n2[(size_t)t * Kt * 16 + K + i] = INFINITY;
+            ct.lo[(size_t)t * Kt * 16 + K + i] = 0.0f;
+        }
     }
 }
 
@@ -82,14 +85,13 @@ __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_
 // 1. initial centroids: item floor((k + u_k) * n_c / K), u_k in [0,1) from the seed
 // ------------------------------------------------------------------------------------
 //    (n_live != NULL: tree t holds n_live[t] <= n_c items, the first ones of its rows)
-//    tiles != NULL: the centroid also goes into its operand tile (fill: the centroids that
+//    ct.tiles != NULL: the centroid also goes into its operand tile (fill: the centroids that
 //    count as full from the start take no items)
 template <typename T>
 __global__ __launch_bounds__(64) void k_init_centroids(const void* x, int n_c, size_t x_tree_stride,
                                                        int K, int D, uint64_t seed, float* cent,
                                                        const int32_t* n_live, int bf, int Kt,
-                                                       const int32_t* fill, uint4* tiles,
-                                                       float* cn2) {
+                                                       const int32_t* fill, CentroidTiles ct, int KS) {
     __shared__ float s_c[256];
     const int k = blockIdx.x, t = blockIdx.y;
     const uint64_t h = mix64(seed ^ mix64((uint64_t)t * 0x100000001b3ull + (uint64_t)k));
@@ -104,11 +106,11 @@ __global__ __launch_bounds__(64) void k_init_centroids(const void* x, int n_c, s
     for (int j = threadIdx.x; j < D; j += blockDim.x) {
         const float v = load_elem<T>(x, src + j);
         dst[j] = v;
-        if (tiles != nullptr) s_c[j] = v;  // (the matrix-core path has D <= 256)
+        if (ct.tiles != nullptr) s_c[j] = v;  // (tiles are for D <= 256)
     }
-    if (tiles != nullptr) {
+    if (ct.tiles != nullptr) {
         __syncthreads();
-        emit_centroid(s_c, D, Kt, t, k, fill[(size_t)t * K + k] < bf, tiles, cn2);
+        emit_centroid(s_c, D, KS, Kt, t, k, fill[(size_t)t * K + k] < bf, ct);
     }
 }
 
@@ -134,7 +136,6 @@ __global__ __launch_bounds__(256) void k_assign_simple(
     const int n_items = list ? list_count[t] : n_c;
     const int wave_global = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int first = wave_global * (RPW * kPPG);
-    if (ac.counts == nullptr && first >= n_items) return;
     if (ac.zero != nullptr && blockIdx.x == 0 && threadIdx.x == 0) ac.zero[t] = 0;
     const bool chunk_ok = ch * EPL < D;
 
@@ -197,32 +198,30 @@ __global__ __launch_bounds__(256) void k_assign_simple(
             for (int p = 0; p < kPPG; ++p) {
                 if (item[p] >= 0) {
                     assign[(size_t)t * n_c + item[p]] = arg[p];
-                    dist[(size_t)t * n_c + item[p]] = best[p];
-                    if (ac.counts != nullptr && arg[p] >= 0)
-                        ac.pos[(size_t)t * n_c + item[p]] =
-                            atomicAdd(&ac.counts[(size_t)t * K + arg[p]], 1);
+                    if (dist != nullptr) dist[(size_t)t * n_c + item[p]] = best[p];
+                    if (ac.counts != nullptr && arg[p] >= 0) count_item(ac, t, K, n_c, arg[p], item[p]);
                 }
             }
         }
     }
-    if (ac.counts != nullptr) finish_counts(ac, t, K, (int)gridDim.x);
 }
 
 // ------------------------------------------------------------------------------------
-// 3. the items of a round bucketed by the centroid they were assigned to: item i of bucket a
-//    goes to members[offsets[a] + pos[i]] (offsets and pos come out of the assignment launch)
+// 3. the buckets of a round: what the assignment left of it (assign.h)
 // ------------------------------------------------------------------------------------
-__global__ void k_bucket_fill(const int32_t* assign, const int32_t* pos, const int32_t* offsets,
-                              int n_c, const int32_t* list, const int32_t* list_count,
-                              size_t list_stride, int K, int32_t* members) {
-    const int t = blockIdx.y;
-    const int n_items = list ? list_count[t] : n_c;
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n_items) return;
-    const int i = list ? list[(size_t)t * list_stride + p] : p;
-    const int a = assign[(size_t)t * n_c + i];
-    if (a < 0) return;
-    members[(size_t)t * n_c + offsets[(size_t)t * (K + 1) + a] + pos[(size_t)t * n_c + i]] = i;
+struct Buckets {
+    int32_t* counts;          // (T, K); every kernel here leaves it zero for the round after it
+    const int32_t* members;   // (T, K, kBucketCap)
+    const int2* more;         // (T, n_c)
+    const int32_t* more_count;  // (T)
+    int32_t* next_more_count;   // (T): the round after this one counts here; cleared by these kernels
+    int32_t* unsure_count;      // (T): cleared by these kernels
+};
+
+// item e of the ones that do not lie in `members` of the tree: its id if it is of bucket k, else -1
+__device__ __forceinline__ int more_of(const Buckets& b, int t, int n_c, int k, int e) {
+    const int2 v = b.more[(size_t)t * n_c + e];
+    return v.x == k ? v.y : -1;
 }
 
 // The order in which a bucket's members arrive depends on the run; everything that follows works
@@ -256,11 +255,14 @@ __device__ __forceinline__ int pow2_at_least(int n) {
     return p;
 }
 
-// (what every workgroup of the per-bucket kernels does for the round after it)
-__device__ __forceinline__ void reset_counters(int t, int k, int K, int32_t* counts, int32_t* done) {
+// (what every workgroup of the per-bucket kernels does for the round after it, having read the count)
+__device__ __forceinline__ void reset_counters(const Buckets& b, int t, int k, int K) {
     if (threadIdx.x == 0) {
-        counts[(size_t)t * K + k] = 0;
-        if (k == 0) done[t] = 0;
+        b.counts[(size_t)t * K + k] = 0;
+        if (k == 0) {
+            b.next_more_count[t] = 0;
+            b.unsure_count[t] = 0;
+        }
     }
 }
 
@@ -268,29 +270,44 @@ __device__ __forceinline__ void reset_counters(int t, int k, int K, int32_t* cou
 // 4. Lloyd round: centroid = mean of the member rows.  One workgroup per centroid: the members
 //    in the order of their item ids, row e summed by row group e % R, the R sums added in order:
 //    the result does not depend on the order of arrival.  An empty centroid keeps its value.
-//    tiles != NULL: the new centroid also goes into its operand tile.
+//    ct.tiles != NULL: the new centroid also goes into its operand tile.
 // ------------------------------------------------------------------------------------
 constexpr int kMeanSort = 4096;      // members ordered in LDS; more: through a bit map of item ids
 constexpr int kMeanMapBits = kMeanSort * 32;
 
 template <typename T>
 __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
-    const void* x, size_t x_tree_stride, int n_c, int K, int D, const int32_t* offsets,
-    const int32_t* members, int32_t* ordered /* (T, n_c): buckets too large for LDS */,
-    const int32_t* fill, int bf, float* cent, int Kt, uint4* tiles, float* cn2, int32_t* counts,
-    int32_t* done) {
+    const void* x, size_t x_tree_stride, int n_c, int K, int D, const Buckets bk,
+    const int32_t* fill, int bf, float* cent, int Kt, const CentroidTiles ct, int KS) {
     constexpr int EPL = Elem<T>::kPerChunk;
     __shared__ uint32_t s_ord[kMeanSort];            // (as a bit map: kMeanMapBits ids)
     __shared__ float s_part[kBucketThreads * EPL];   // (R, D) partial sums, R * D <= 256 * EPL
     __shared__ int32_t s_small[kBucketThreads];
+    __shared__ int32_t s_n;
     const int k = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
-    reset_counters(t, k, K, counts, done);
-    const int b0 = offsets[(size_t)t * (K + 1) + k];
-    const int m = offsets[(size_t)t * (K + 1) + k + 1] - b0;
+    const int m = bk.counts[(size_t)t * K + k];
+    const int32_t* mem = bk.members + ((size_t)t * K + k) * kBucketCap;
+    if (tid == 0) s_n = kBucketCap;
+    __syncthreads();  // (every thread has read the count)
+    reset_counters(bk, t, k, K);
     if (m <= 0) return;
-    const int32_t* mem = members + (size_t)t * n_c + b0;
-    const int32_t* ord_g = nullptr;  // the ordered members: in LDS, or here
-    if (m <= kBucketThreads) {
+    // ---- sums: CPR threads a row, R rows at a time -------------------------------------------
+    const int CPR = D / EPL, R = kBucketThreads / CPR;
+    const int r = tid / CPR, c = tid % CPR;
+    float acc[EPL];
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) acc[e] = 0.0f;
+    // rows [e0, e0 + n) in order, their ids at ids[0 .. n)
+    auto add_rows = [&](const uint32_t* ids, int e0, int n) {
+        if (r < R)
+            for (int e = e0 + (r - e0 % R + R) % R; e < e0 + n; e += R) {
+                float f[EPL];
+                unpack<T>(load_chunk<T>(x, ((size_t)t * x_tree_stride + (int)ids[e - e0]) * D, c), f);
+#pragma unroll
+                for (int q = 0; q < EPL; ++q) acc[q] += f[q];
+            }
+    };
+    if (m <= kBucketCap) {
         const int mine = tid < m ? mem[tid] : 0x7fffffff;
         s_small[tid] = mine;
         __syncthreads();
@@ -298,62 +315,64 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
         for (int j = 0; j < m; ++j) rank += s_small[j] < mine;
         if (tid < m) s_ord[rank] = (uint32_t)mine;
         __syncthreads();
+        add_rows(s_ord, 0, m);
     } else if (m <= kMeanSort) {
-        const int P = pow2_at_least(m);
-        for (int e = tid; e < P; e += kBucketThreads) s_ord[e] = e < m ? (uint32_t)mem[e] : 0xffffffffu;
+        const int P = pow2_at_least(m), others = bk.more_count[t];
+        for (int e = tid; e < P; e += kBucketThreads) s_ord[e] = e < kBucketCap ? (uint32_t)mem[e] : 0xffffffffu;
+        __syncthreads();
+        for (int e = tid; e < others; e += kBucketThreads) {
+            const int it = more_of(bk, t, n_c, k, e);
+            if (it >= 0) s_ord[atomicAdd(&s_n, 1)] = (uint32_t)it;
+        }
         bitonic_sort(s_ord, P);
+        add_rows(s_ord, 0, m);
     } else {
-        // ids in ranges of kMeanMapBits: a bit per member, then the set bits in order
-        int32_t* out = ordered + (size_t)t * n_c + b0;
+        // ids in ranges of kMeanMapBits: a bit per member, then the set bits in order, as many of them
+        // at a time as there is room for in s_part
+        constexpr int kPiece = kBucketThreads * EPL;
+        uint32_t* piece = reinterpret_cast<uint32_t*>(s_part);
+        const int others = bk.more_count[t];
         int written = 0;
         for (int lo = 0; lo < n_c; lo += kMeanMapBits) {
             __syncthreads();
             for (int w = tid; w < kMeanSort; w += kBucketThreads) s_ord[w] = 0;
             __syncthreads();
-            for (int e = tid; e < m; e += kBucketThreads) {
-                const int d = mem[e] - lo;
-                if (d >= 0 && d < kMeanMapBits) atomicOr(&s_ord[d >> 5], 1u << (d & 31));
-            }
+            auto mark = [&](int it) {
+                const int d = it - lo;
+                if (it >= 0 && d >= 0 && d < kMeanMapBits) atomicOr(&s_ord[d >> 5], 1u << (d & 31));
+            };
+            if (tid < kBucketCap) mark(mem[tid]);
+            for (int e = tid; e < others; e += kBucketThreads) mark(more_of(bk, t, n_c, k, e));
             __syncthreads();
             // thread `tid` owns the words [tid * W, (tid + 1) * W)
             constexpr int W = kMeanSort / kBucketThreads;
             const int in_range = block_exclusive_scan(
                 kBucketThreads, [&](int i) {
-                    int c = 0;
-                    for (int w = 0; w < W; ++w) c += __popc(s_ord[i * W + w]);
-                    return c;
+                    int n = 0;
+                    for (int w = 0; w < W; ++w) n += __popc(s_ord[i * W + w]);
+                    return n;
                 },
                 [&](int i, int v) { s_small[i] = v; });
             __syncthreads();
-            int at = written + s_small[tid];
-            for (int w = 0; w < W; ++w) {
-                uint32_t bits = s_ord[tid * W + w];
-                while (bits) {
-                    const int b = __ffs(bits) - 1;
-                    bits &= bits - 1;
-                    out[at++] = lo + (tid * W + w) * 32 + b;
+            for (int p0 = 0; p0 < in_range; p0 += kPiece) {
+                int at = s_small[tid];
+                for (int w = 0; w < W; ++w) {
+                    uint32_t bits = s_ord[tid * W + w];
+                    while (bits) {
+                        const int b = __ffs(bits) - 1;
+                        bits &= bits - 1;
+                        if (at >= p0 && at < p0 + kPiece) piece[at - p0] = (uint32_t)(lo + (tid * W + w) * 32 + b);
+                        ++at;
+                    }
                 }
+                __syncthreads();
+                add_rows(piece, written + p0, min(kPiece, in_range - p0));
+                __syncthreads();
             }
             written += in_range;
         }
-        __threadfence_block();
-        __syncthreads();
-        ord_g = out;
     }
-    // ---- sums: CPR threads a row, R rows at a time -------------------------------------------
-    const int CPR = D / EPL, R = kBucketThreads / CPR;
-    const int r = tid / CPR, c = tid % CPR;
-    float acc[EPL];
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] = 0.0f;
     if (r < R) {
-        for (int e = r; e < m; e += R) {
-            const int it = ord_g ? ord_g[e] : (int)s_ord[e];
-            float f[EPL];
-            unpack<T>(load_chunk<T>(x, ((size_t)t * x_tree_stride + it) * D, c), f);
-#pragma unroll
-            for (int q = 0; q < EPL; ++q) acc[q] += f[q];
-        }
 #pragma unroll
         for (int q = 0; q < EPL; ++q) s_part[r * D + c * EPL + q] = acc[q];
     }
@@ -366,13 +385,12 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
         v = s / (float)m;
         cent[((size_t)t * K + k) * D + j] = v;
     }
-    if (tiles != nullptr) {  // (D <= 256: column tid)
+    if (ct.tiles != nullptr) {  // (D <= 256: column tid)
         __syncthreads();
         if (tid < D) s_part[tid] = v;
         __syncthreads();
         if (tid < 64)
-            emit_centroid(s_part, D, Kt, t, k, !(fill != nullptr && fill[(size_t)t * K + k] >= bf),
-                          tiles, cn2);
+            emit_centroid(s_part, D, KS, Kt, t, k, !(fill != nullptr && fill[(size_t)t * K + k] >= bf), ct);
     }
 }
 
@@ -430,27 +448,25 @@ __global__ __launch_bounds__(64) void k_block_mean(const void* x, size_t x_tree_
 // slots of the block in that order; the others go on the list of the next round.  A block that
 // is full now takes no more items: its norm in the operand tiles becomes +inf.
 constexpr int kAcceptSort = 2048;  // keys sorted at a time; larger buckets in several goes, the
-                                   // best `take` so far carried along
+                                   // best `take` (at most 64) so far carried along
 
 __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
-    const int32_t* members, const int32_t* offsets, const float* dist, int n_c, int K, int bf,
-    int32_t* fill, int32_t* slots, int32_t* placed, int32_t* next_list, int32_t* next_count,
-    int Kt, float* cn2, int32_t* counts, int32_t* done) {
+    const Buckets bk, const float* dist, int n_c, int K, int bf, int32_t* fill, int32_t* slots,
+    int32_t* placed, int32_t* next_list, int32_t* next_count, int Kt, float* cn2) {
     __shared__ uint64_t s_keys[kAcceptSort];
-    __shared__ int32_t s_base, s_rej;
+    __shared__ int32_t s_base, s_rej, s_n;
     const int k = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
-    reset_counters(t, k, K, counts, done);
-    const int b0 = offsets[(size_t)t * (K + 1) + k];
-    const int m = offsets[(size_t)t * (K + 1) + k + 1] - b0;
-    if (m <= 0) return;
-    const int32_t* mem = members + (size_t)t * n_c + b0;
+    const int m = bk.counts[(size_t)t * K + k];
+    const int32_t* mem = bk.members + ((size_t)t * K + k) * kBucketCap;
     const float* dt = dist + (size_t)t * n_c;
     const int f = fill[(size_t)t * K + k];
     const int take = max(min(m, bf - f), 0);
     int32_t* my_slots = slots + ((size_t)t * K + k) * bf + f;
     int32_t* pl = placed + (size_t)t * n_c;
     int32_t* nl = next_list + (size_t)t * n_c;
-    __syncthreads();  // (every thread has read the block's fill)
+    __syncthreads();  // (every thread has read the block's fill and the bucket's count)
+    reset_counters(bk, t, k, K);
+    if (m <= 0) return;
     if (tid == 0) {
         s_base = m > take ? atomicAdd(&next_count[t], m - take) : 0;
         s_rej = 0;
@@ -458,7 +474,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
         if (cn2 != nullptr && f + take >= bf) cn2[(size_t)t * Kt * 16 + k] = INFINITY;
     }
     auto key_of = [&](int it) { return ((uint64_t)__float_as_uint(dt[it]) << 32) | (uint32_t)it; };
-    if (m <= kBucketThreads) {
+    if (m <= kBucketCap) {
         int it = -1;
         uint64_t mine = ~0ull;
         if (tid < m) {
@@ -479,17 +495,25 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
         }
         return;
     }
-    int kept = 0;  // s_keys[0 .. kept): the best so far, in order
-    for (int e0 = 0; e0 < m;) {
-        const int cn = min(kAcceptSort - kept, m - e0);
-        const int P = pow2_at_least(kept + cn);
+    // s_keys[0 .. n): the best so far and those not looked at yet; a kAcceptStep of the others at a
+    // time is searched for the bucket's items
+    constexpr int kAcceptStep = kAcceptSort - kBucketCap - 64;
+    const int others = bk.more_count[t];
+    if (tid < kBucketCap) s_keys[tid] = key_of(mem[tid]);
+    if (tid == 0) s_n = kBucketCap;
+    for (int e0 = 0; e0 < others; e0 += kAcceptStep) {
         __syncthreads();
-        for (int e = kept + tid; e < P; e += kBucketThreads)
-            s_keys[e] = e < kept + cn ? key_of(mem[e0 + e - kept]) : ~0ull;
+        for (int e = e0 + tid; e < min(e0 + kAcceptStep, others); e += kBucketThreads) {
+            const int it = more_of(bk, t, n_c, k, e);
+            if (it >= 0) s_keys[atomicAdd(&s_n, 1)] = key_of(it);
+        }
+        __syncthreads();
+        const int n = s_n, P = pow2_at_least(n);
+        for (int e = n + tid; e < P; e += kBucketThreads) s_keys[e] = ~0ull;
         bitonic_sort(s_keys, P);
-        kept = min(take, kept + cn);
-        e0 += cn;
+        if (tid == 0) s_n = min(take, n);
     }
+    __syncthreads();
     for (int r = tid; r < take; r += kBucketThreads) {
         const int it = (int)(uint32_t)s_keys[r];
         my_slots[r] = it;
@@ -497,10 +521,11 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
     }
     if (m > take) {  // whoever lies behind the last one taken tries again
         const uint64_t last = take > 0 ? s_keys[take - 1] : 0ull;
-        for (int e = tid; e < m; e += kBucketThreads) {
-            const int it = mem[e];
-            if (take == 0 || key_of(it) > last) nl[s_base + atomicAdd(&s_rej, 1)] = it;
-        }
+        auto again = [&](int it) {
+            if (it >= 0 && (take == 0 || key_of(it) > last)) nl[s_base + atomicAdd(&s_rej, 1)] = it;
+        };
+        if (tid < kBucketCap) again(mem[tid]);
+        for (int e = tid; e < others; e += kBucketThreads) again(more_of(bk, t, n_c, k, e));
     }
 }
 
@@ -728,16 +753,15 @@ struct Carver {
 
 struct BuildWs {
     float* cent_f32;
-    void* cent_tiles;  // centroids as bf16 operand tiles (matrix-core assignment), or NULL
-    float* cent_n2;
-    void* open_tiles;  // the same for the centroids with room, side by side (later packing rounds)
-    float* open_n2;
+    CentroidTiles ct;    // centroids as operand tiles (matrix cores), or NULL
+    CentroidTiles open;  // the same for the centroids with room, side by side (later packing rounds)
     int32_t *open_ids, *open_count;
-    int32_t *assign, *pos, *placed, *members, *ordered;
+    int32_t *assign, *placed, *members, *unsure;
+    int2* more;
     int32_t* list[2];     // the items of a packing round, and those of the round after it
-    int32_t* list_count;  // (2, T)
+    int32_t* counters;    // (kBuildCounters, T)
     float* dist;
-    int32_t *counts, *offsets, *done, *fill, *free_pre, *chunk_pre;
+    int32_t *counts, *fill, *free_pre, *chunk_pre;
     int32_t* slots[HIRA_MAX_LEVELS];
     void* cent_t[HIRA_MAX_LEVELS];
     int32_t* order[HIRA_MAX_LEVELS];
@@ -746,9 +770,10 @@ struct BuildWs {
 
 static int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// bf16 rows of 64, 128 or 256 columns are assigned on the matrix cores
-static bool assign_on_mfma(const HiraTree* t) {
-    return t->dtype == HIRA_BF16 && (t->dim == 64 || t->dim == 128 || t->dim == 256);
+// whether the matrix cores take the assignment of a level of K centroids (the exact kernel or the
+// approximate one)
+static bool assign_on_mfma(const HiraTree* t, int K) {
+    return assign_exact_on_mfma(t->dtype, t->dim) || assign_approx_pays(t->dtype, t->dim, K);
 }
 
 // cluster counts per level: K[0] = n, K[l] = ceil(K[l-1] / bf)
@@ -765,32 +790,29 @@ static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
     Carver c{reinterpret_cast<char*>(ws), 0};
     const size_t k1 = L >= 2 ? (size_t)K[1] : 1;
     b->cent_f32 = c.take<float>((size_t)T * k1 * D);
-    b->cent_tiles = nullptr;
-    b->cent_n2 = nullptr;
-    b->open_tiles = nullptr;
-    b->open_n2 = nullptr;
+    b->ct = b->open = CentroidTiles{nullptr, nullptr, nullptr};
     b->open_ids = b->open_count = nullptr;
-    if (assign_on_mfma(t)) {
+    if (assign_on_mfma(t, (int)k1)) {
         const size_t kpad = (size_t)assign_tiles((int)k1) * 16;
-        b->cent_tiles = c.take<char>((size_t)T * kpad * D * 4);  // hi and lo halves, 2 bytes each
-        b->cent_n2 = c.take<float>((size_t)T * kpad);
-        b->open_tiles = c.take<char>((size_t)T * kpad * D * 4);
-        b->open_n2 = c.take<float>((size_t)T * kpad);
+        const size_t chunks = kpad * assign_ks(t->dtype, D) * 8;  // hi and lo halves
+        for (CentroidTiles* ct : {&b->ct, &b->open}) {
+            ct->tiles = c.take<uint4>((size_t)T * chunks);
+            ct->n2 = c.take<float>((size_t)T * kpad);
+            ct->lo = c.take<float>((size_t)T * kpad);
+        }
         b->open_ids = c.take<int32_t>((size_t)T * k1);
         b->open_count = c.take<int32_t>((size_t)T);
     }
     b->assign = c.take<int32_t>((size_t)T * n);
-    b->pos = c.take<int32_t>((size_t)T * n);
     b->placed = c.take<int32_t>((size_t)T * n);
-    b->members = c.take<int32_t>((size_t)T * n);
-    b->ordered = c.take<int32_t>((size_t)T * n);
+    b->members = c.take<int32_t>((size_t)T * k1 * kBucketCap);
+    b->more = c.take<int2>((size_t)T * n);
+    b->unsure = c.take<int32_t>((size_t)T * n);
     b->list[0] = c.take<int32_t>((size_t)T * n);
     b->list[1] = c.take<int32_t>((size_t)T * n);
-    b->list_count = c.take<int32_t>((size_t)T * 2);
+    b->counters = c.take<int32_t>((size_t)T * kBuildCounters);
     b->dist = c.take<float>((size_t)T * n);
     b->counts = c.take<int32_t>((size_t)T * k1);
-    b->offsets = c.take<int32_t>((size_t)T * (k1 + 1));
-    b->done = c.take<int32_t>((size_t)T);
     b->fill = c.take<int32_t>((size_t)T * k1);
     b->free_pre = c.take<int32_t>((size_t)T * (k1 + 1));
     b->chunk_pre = c.take<int32_t>((size_t)T * ((size_t)ceil_div(n, 256) + 1));
@@ -808,7 +830,7 @@ static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
 }
 
 template <typename T>
-static int launch_assign(int lpr, dim3 grid, hipStream_t s, const void* x, int n_c,
+static int launch_assign_simple(int lpr, dim3 grid, hipStream_t s, const void* x, int n_c,
                          size_t x_stride, const float* cent, int K, int D, const int32_t* fill,
                          int bf, const int32_t* list, const int32_t* list_count,
                          size_t list_stride, int32_t* assign, float* dist,
@@ -849,14 +871,21 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
     int K[HIRA_MAX_LEVELS];
     cluster_counts(n, bf, L, K);
 
-    const bool on_mfma = w.cent_tiles != nullptr;
-    uint4* tiles = reinterpret_cast<uint4*>(w.cent_tiles);
+    int32_t* const done = w.counters;
+    int32_t* const list_count = w.counters + (size_t)NT;         // (2, T)
+    int32_t* const more_count = w.counters + (size_t)3 * NT;     // (2, T)
+    int32_t* const unsure_count = w.counters + (size_t)5 * NT;
+    const int KS = assign_ks(t->dtype, D);
     for (int l = 1; l < L; ++l) {
         const void* x = l == 1 ? keys_in : w.cent_t[l - 1];
         const int n_c = K[l - 1];
         const size_t xs = (size_t)n_c;  // rows per tree in x
         const int Kl = K[l];
+        const bool on_mfma = assign_on_mfma(t, Kl), approx = assign_approx_pays(t->dtype, D, Kl);
         const int Kt = on_mfma ? assign_tiles(Kl) : 0;
+        const CentroidTiles tiles = on_mfma ? w.ct : CentroidTiles{nullptr, nullptr, nullptr};
+        const long long all_items = (long long)n_c * NT;
+        int round = 0;  // of the level, Lloyd and packing together
         const int items_per_block = 4 * (64 / lpr) * kPPG;
         const dim3 g_assign(ceil_div(n_c, items_per_block), NT);
         const dim3 g_items(ceil_div(n_c, 256), NT);
@@ -867,66 +896,72 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
         const bool ragged = n_live != nullptr && l == 1;
         hipLaunchKernelGGL(k_level_init, dim3(min(ceil_div(max(n_c, Kl * bf), 256), 2048), NT),
                            dim3(256), 0, s, n_c, Kl, bf, D, Kt, ragged ? n_live : nullptr, w.placed,
-                           w.fill, w.slots[l], w.counts, w.done, w.list_count, tiles, w.cent_n2);
+                           w.fill, w.slots[l], w.counts, w.counters, tiles, KS);
         const int32_t* live = nullptr;
         const int32_t* live_cnt = nullptr;
         if (ragged) {
             hipLaunchKernelGGL(k_collect_unplaced, g_items, dim3(256), 0, s, w.placed, n_c,
-                               w.list[0], w.list_count);
+                               w.list[0], list_count);
             live = w.list[0];
-            live_cnt = w.list_count;
+            live_cnt = list_count;
         }
         hipLaunchKernelGGL((k_init_centroids<T>), g_cent, dim3(64), 0, s, x, n_c, xs, Kl, D,
                            seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, bf,
-                           Kt, w.fill, tiles, w.cent_n2);
-        // a round: the assignment (which also counts the items of every centroid and turns the
-        // counts into offsets), the buckets, and what the round does with every bucket
-        auto assign_round = [&](const int32_t* list, const int32_t* lcnt, const int32_t* fill,
-                                int32_t* zero, bool only_open) -> int {
-            const AssignCounting ac{w.counts, w.pos, w.done, w.offsets, zero};
-            int rc;
-            if (on_mfma && only_open) {
-                rc = launch_open_centroids(D, w.cent_tiles, w.cent_n2, w.fill, bf, Kl, NT, w.open_ids,
-                                           w.open_count, w.open_tiles, w.open_n2, s);
-                if (rc == HIRA_OK)
-                    rc = launch_assign_mfma(D, x, n_c, xs, w.open_tiles, w.open_n2, Kl, NT, list, lcnt,
-                                            (size_t)n_c, w.assign, w.dist, ac,
-                                            AssignOpen{w.open_count, w.open_ids}, s);
-            } else if (on_mfma)
-                rc = launch_assign_mfma(D, x, n_c, xs, w.cent_tiles, w.cent_n2, Kl, NT, list, lcnt,
-                                        (size_t)n_c, w.assign, w.dist, ac, AssignOpen{nullptr, nullptr}, s);
-            else
-                rc = launch_assign<T>(lpr, g_assign, s, x, n_c, xs, w.cent_f32, Kl, D, fill, bf, list,
-                                      lcnt, (size_t)n_c, w.assign, w.dist, ac);
-            if (rc != HIRA_OK) return rc;
-            hipLaunchKernelGGL(k_bucket_fill, g_items, dim3(256), 0, s, w.assign, w.pos, w.offsets,
-                               n_c, list, lcnt, (size_t)n_c, Kl, w.members);
-            return HIRA_OK;
+                           Kt, w.fill, tiles, KS);
+        // a round: the assignment (which also puts the items into buckets), then what the round does
+        // with every bucket.  A Lloyd round asks for no distances.
+        auto buckets = [&]() {
+            return Buckets{w.counts, w.members, w.more, more_count + (size_t)(round & 1) * NT,
+                           more_count + (size_t)((round + 1) & 1) * NT, unsure_count};
         };
-        for (int it = 0; it < niter; ++it) {
-            const int rc = assign_round(live, live_cnt, ragged ? w.fill : nullptr, nullptr, false);
+        auto assign_round = [&](const int32_t* list, const int32_t* lcnt, const int32_t* fill, float* dist,
+                                int32_t* zero, bool only_open, long long expected) -> int {
+            AssignJob job{x, n_c, xs, t->dtype, D, NT, tiles, w.cent_f32, Kl, list, lcnt, w.assign, dist,
+                          AssignCounting{w.counts, w.members, w.more, more_count + (size_t)(round & 1) * NT, zero},
+                          AssignOpen{nullptr, nullptr}, 0, w.unsure, unsure_count};
+            int rc = HIRA_OK;
+            if (on_mfma && only_open) {
+                rc = launch_open_centroids(KS, w.ct, w.fill, bf, Kl, NT, w.open_ids, w.open_count, w.open, s);
+                job.ct = w.open;
+                job.open = AssignOpen{w.open_count, w.open_ids};
+            }
+            const bool exact_mfma = assign_exact_on_mfma(t->dtype, D);
+            // (the lists of the packing about halve from round to round: the later ones are none of
+            // the approximate pass's, and spared its launch)
+            if (rc == HIRA_OK && approx && (!exact_mfma || expected > kApproxListItems)) {
+                rc = launch_assign_approx(job, s);
+                job.after_approx = 1;
+            }
             if (rc != HIRA_OK) return rc;
-            hipLaunchKernelGGL((k_bucket_mean<T>), g_cent, dim3(kBucketThreads), 0, s, x, xs, n_c,
-                               Kl, D, w.offsets, w.members, w.ordered, ragged ? w.fill : nullptr, bf,
-                               w.cent_f32, Kt, tiles, w.cent_n2, w.counts, w.done);
+            if (exact_mfma) return launch_assign_mfma(job, s);
+            if (job.after_approx) {
+                job.list = w.unsure;
+                job.list_count = unsure_count;
+            }
+            return launch_assign_simple<T>(lpr, g_assign, s, x, n_c, xs, w.cent_f32, Kl, D, fill, bf, job.list,
+                                           job.list_count, (size_t)n_c, w.assign, dist, job.counting);
+        };
+        for (int it = 0; it < niter; ++it, ++round) {
+            const int rc = assign_round(live, live_cnt, ragged ? w.fill : nullptr, nullptr, nullptr, false, all_items);
+            if (rc != HIRA_OK) return rc;
+            hipLaunchKernelGGL((k_bucket_mean<T>), g_cent, dim3(kBucketThreads), 0, s, x, xs, n_c, Kl, D, buckets(),
+                               ragged ? w.fill : nullptr, bf, w.cent_f32, Kt, tiles, KS);
         }
         // capacity packing: round r walks list r % 2 (the first one all items, or the items the
         // trees hold) and leaves those it could not place on the other list
-        for (int r = 0; r < pack_rounds; ++r) {
+        for (int r = 0; r < pack_rounds; ++r, ++round) {
             const int32_t* list = r == 0 ? live : w.list[r & 1];
-            const int32_t* lcnt = r == 0 ? live_cnt : w.list_count + (size_t)(r & 1) * NT;
-            int32_t* next_cnt = w.list_count + (size_t)((r + 1) & 1) * NT;
+            const int32_t* lcnt = r == 0 ? live_cnt : list_count + (size_t)(r & 1) * NT;
+            int32_t* next_cnt = list_count + (size_t)((r + 1) & 1) * NT;
             // (from the second round on most blocks are full: the assignment then sees only the
-            // centroids with room, side by side; worth its two small launches from 32 tiles on)
-            const int rc = assign_round(list, lcnt, w.fill, next_cnt, r >= 1 && Kl >= 512);
+            // centroids with room, side by side; worth its launch from 32 tiles on)
+            const int rc = assign_round(list, lcnt, w.fill, w.dist, next_cnt, r >= 1 && Kl >= 512, all_items >> r);
             if (rc != HIRA_OK) return rc;
-            hipLaunchKernelGGL(k_bucket_accept, g_cent, dim3(kBucketThreads), 0, s, w.members,
-                               w.offsets, w.dist, n_c, Kl, bf, w.fill, w.slots[l], w.placed,
-                               w.list[(r + 1) & 1], next_cnt, Kt, on_mfma ? w.cent_n2 : nullptr,
-                               w.counts, w.done);
+            hipLaunchKernelGGL(k_bucket_accept, g_cent, dim3(kBucketThreads), 0, s, buckets(), w.dist, n_c, Kl, bf,
+                               w.fill, w.slots[l], w.placed, w.list[(r + 1) & 1], next_cnt, Kt, tiles.n2);
         }
         hipLaunchKernelGGL(k_leftover_count, g_items, dim3(256), 0, s, w.placed, n_c, Kl, bf, w.fill,
-                           w.chunk_pre, w.free_pre, w.done);
+                           w.chunk_pre, w.free_pre, done);
         hipLaunchKernelGGL(k_leftover_place, g_items, dim3(256), 0, s, n_c, Kl, bf, w.fill,
                            w.chunk_pre, w.free_pre, w.slots[l], w.placed);
         // block centre = mean of what is in the block, rounded to the storage type
@@ -1092,7 +1127,7 @@ static void carve_nearest(int dtype, int T, int m, int D, bool masked, void* ws,
     Carver c{reinterpret_cast<char*>(ws), 0};
     b->tiles = nullptr;
     b->n2 = nullptr;
-    if (dtype == HIRA_BF16 && (D == 64 || D == 128 || D == 256)) {
+    if (assign_exact_on_mfma(dtype, D)) {
         const size_t kpad = (size_t)assign_tiles(m) * 16;
         b->tiles = c.take<char>((size_t)T * kpad * D * 4);
         b->n2 = c.take<float>((size_t)T * kpad);
@@ -1142,18 +1177,27 @@ extern "C" int hira_nearest(const void* x, int32_t dtype, int32_t num_trees, int
     fill_i32(reinterpret_cast<int32_t*>(dist2), (size_t)num_trees * n, 0x7f800000, s);
     if (b.tiles != nullptr) {
         rc = launch_cent_prep(dim, centers, m, num_trees, b.fill, 1, b.tiles, b.n2, s);
-        if (rc == HIRA_OK)
-            rc = launch_assign_mfma(dim, x, n, (size_t)n, b.tiles, b.n2, m, num_trees, nullptr,
-                                    nullptr, 0, idx, dist2, AssignCounting{}, AssignOpen{nullptr, nullptr}, s);
+        AssignJob job{};
+        job.x = x;
+        job.n_c = n;
+        job.x_tree_stride = (size_t)n;
+        job.dtype = dtype;
+        job.D = dim;
+        job.num_trees = num_trees;
+        job.ct = CentroidTiles{reinterpret_cast<uint4*>(b.tiles), b.n2, nullptr};
+        job.K = m;
+        job.assign = idx;
+        job.dist = dist2;
+        if (rc == HIRA_OK) rc = launch_assign_mfma(job, s);
     } else {
         const int epl = dtype == HIRA_F32 ? 4 : 8;
         int lpr = 2;
         while (lpr * epl < dim) lpr <<= 1;
         const dim3 grid(ceil_div(n, 4 * (64 / lpr) * kPPG), num_trees);
         rc = dtype == HIRA_F32
-                 ? launch_assign<float>(lpr, grid, s, x, n, (size_t)n, centers, m, dim, b.fill, 1,
+                 ? launch_assign_simple<float>(lpr, grid, s, x, n, (size_t)n, centers, m, dim, b.fill, 1,
                                         nullptr, nullptr, 0, idx, dist2, AssignCounting{})
-                 : launch_assign<bf16_t>(lpr, grid, s, x, n, (size_t)n, centers, m, dim, b.fill, 1,
+                 : launch_assign_simple<bf16_t>(lpr, grid, s, x, n, (size_t)n, centers, m, dim, b.fill, 1,
                                          nullptr, nullptr, 0, idx, dist2, AssignCounting{});
     }
     if (rc != HIRA_OK) return rc;
