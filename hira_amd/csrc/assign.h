@@ -10,35 +10,56 @@ namespace hira {
 // Bucketing fused into an assignment launch (counts NULL: the launch only assigns).
 //   counts  (T, K)       zero when the round starts; counts[a] += 1 for every item assigned to a.  The
 //                        value the item's increment returned is its place in the bucket:
-//   members (T, K, kBucketCap)  the first kBucketCap items of every bucket, in order of arrival
-//   more    (T, n_c)     (centroid, item) of the items behind those, more_count (T) of them.  Such
-//                        buckets are rare (a few seeds of a Lloyd round); what works on them looks for
-//                        their items here.
+//   members (T, K, kBucketCap)  the first kBucketCap items of every bucket, in order of arrival, and
+//   dists   (T, K, kBucketCap)  their distances (NULL: a Lloyd round, which asks for none)
+//   big     (T, K)       the buckets with more than kWaveBucket members, big_count (T) of them
+//   more    (T, n_c)     (centroid, item) of the items behind those, more_count (T) of them, their
+//   more_dist (T, n_c)   distances by item.  Such buckets are rare (a few seeds of a Lloyd round);
+//                        what works on them looks for their items here.
+//   lost    (T, n_c), lost_count (T)  packing: the items that have no nearest centroid (not numbers)
 // With the places fixed there is no prefix sum over the counts, no tail of a launch that waits for
 // it and no launch that sorts the items into buckets (4.3 + 5 us a round at 8 x 32768 items).
 //   zero    (T)          a counter the launch clears (the list of the round after it), or NULL
+// Counters of trees (big_count, more_count, lost_count, zero, and the lists' lengths) lie kCounterStride apart: at
+// one address, or in one line of memory, an addition waits for the one before it (9 ns each; 8 x 1024
+// workgroups adding to eight neighbours took 67 us).
 constexpr int kBucketCap = 256;
+constexpr int kWaveBucket = 64;
+constexpr int kCounterStride = 32;
 struct AssignCounting {
     int32_t* counts;
     int32_t* members;
+    float* dists;
+    int32_t* big;
+    int32_t* big_count;
     int2* more;
     int32_t* more_count;
+    float* more_dist;
+    int32_t* lost;
+    int32_t* lost_count;
     int32_t* zero;
 };
 
-// item `it` of tree t was assigned to centroid k >= 0
-__device__ __forceinline__ void count_item(const AssignCounting& ac, int t, int K, int n_c, int k, int it) {
+// item `it` of tree t was assigned to centroid k, at distance d (k < 0: to none)
+__device__ __forceinline__ void count_item(const AssignCounting& ac, int t, int K, int n_c, int k, int it, float d) {
+    if (k < 0) {
+        if (ac.dists != nullptr) ac.lost[(size_t)t * n_c + atomicAdd(&ac.lost_count[t * kCounterStride], 1)] = it;
+        return;
+    }
     const size_t b = (size_t)t * K + k;
     const int pos = atomicAdd(&ac.counts[b], 1);
     if (pos < kBucketCap) {
         ac.members[b * kBucketCap + pos] = it;
+        if (ac.dists != nullptr) ac.dists[b * kBucketCap + pos] = d;
+        if (pos == kWaveBucket) ac.big[(size_t)t * K + atomicAdd(&ac.big_count[t * kCounterStride], 1)] = k;
     } else {  // (one atomic for the lanes of the wave that are here)
         const unsigned long long here = __ballot(1);
         const int lane = threadIdx.x & 63, leader = __ffsll((long long)here) - 1;
         int base = 0;
-        if (lane == leader) base = atomicAdd(&ac.more_count[t], __popcll(here));
+        if (lane == leader) base = atomicAdd(&ac.more_count[t * kCounterStride], __popcll(here));
         base = __shfl(base, leader, 64);
         ac.more[(size_t)t * n_c + base + __popcll(here & ((1ull << lane) - 1ull))] = make_int2(k, it);
+        if (ac.dists != nullptr) ac.more_dist[(size_t)t * n_c + it] = d;
     }
 }
 
@@ -88,11 +109,6 @@ __device__ __forceinline__ int block_exclusive_scan(int n, Load load, Store stor
         __syncthreads();
     }
     return s_carry;
-}
-
-// a value another workgroup wrote or counted up during this launch, read where it is coherent
-__device__ __forceinline__ int32_t load_agent(const int32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---- centroids as operands of v_mfma_f32_16x16x32_bf16 --------------------------------------
@@ -153,6 +169,7 @@ __device__ __forceinline__ void emit_centroid(const float* c, int D, int KS, int
 struct AssignJob {
     const void* x;          // (T, n_c, D) items
     int n_c;
+    const int32_t* n_live;  // (T): the first so many of them only, or NULL
     size_t x_tree_stride;
     int dtype, D, num_trees;
     CentroidTiles ct;       // centroids as operand tiles (all, or the open ones)
@@ -160,8 +177,8 @@ struct AssignJob {
     int K;
     const int32_t* list;    // NULL: all items, else the items list[0 .. *list_count) of each tree
     const int32_t* list_count;
-    int32_t* assign;        // (T, n_c)
-    float* dist;            // (T, n_c), or NULL: nobody asks for the distances
+    int32_t* assign;        // (T, n_c) and
+    float* dist;            // (T, n_c): where the result goes if nothing is counted
     AssignCounting counting;
     AssignOpen open;
     int after_approx;       // the approximate pass has been over it: only what it left is left
@@ -171,6 +188,20 @@ struct AssignJob {
 
 // (all trees together) more items than this on a list, and the approximate pass takes it
 constexpr int kApproxListItems = 256 * 256;
+
+__device__ __forceinline__ int items_of(const AssignJob& job, int t) {
+    if (job.list != nullptr) return job.list_count[t * kCounterStride];
+    return job.n_live != nullptr ? min(max(job.n_live[t], 0), job.n_c) : job.n_c;
+}
+// what was found for item `it`: into its bucket, or as it is
+__device__ __forceinline__ void put_result(const AssignJob& job, int t, int it, int k, float d) {
+    if (job.counting.counts != nullptr) {
+        count_item(job.counting, t, job.K, job.n_c, k, it, d);
+    } else {
+        job.assign[(size_t)t * job.n_c + it] = k;
+        job.dist[(size_t)t * job.n_c + it] = d;
+    }
+}
 
 // assign_mfma.hip
 int assign_ks(int dtype, int D);        // KS of the operand tiles for rows of D columns, 0: none

@@ -95,9 +95,9 @@ __global__ __launch_bounds__(kAssignThreads, 2) void k_assign_mfma(const AssignJ
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, kb = lane >> 4;  // operand row / centroid column, column block
-    const int t = blockIdx.y, n_c = job.n_c, K = job.K;
+    const int t = blockIdx.y, n_items = items_of(job, t);
     const int first = (blockIdx.x * (kAssignThreads / 64) + wave) * (RI * 16);
-    if (job.counting.zero != nullptr && blockIdx.x == 0 && threadIdx.x == 0) job.counting.zero[t] = 0;
+    if (job.counting.zero != nullptr && blockIdx.x == 0 && threadIdx.x == 0) job.counting.zero[t * kCounterStride] = 0;
 
     // ---- my items: operand tiles in registers, ||x||^2 of row lane % 16 ------------------
     int item[RI];
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kAssignThreads, 2) void k_assign_mfma(const AssignJ
 #pragma unroll
     for (int ri = 0; ri < RI; ++ri) {
         const int pos = first + ri * 16 + n;
-        item[ri] = pos < n_c ? pos : -1;
+        item[ri] = pos < n_items ? pos : -1;
         float ss = 0.0f;
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
@@ -237,9 +237,7 @@ __global__ __launch_bounds__(kAssignThreads, 2) void k_assign_mfma(const AssignJ
                 xx = x2[ri];
             }
         if (it >= 0) {
-            job.assign[(size_t)t * n_c + it] = g;
-            if (job.dist != nullptr) job.dist[(size_t)t * n_c + it] = fmaxf(s_b[lane] + xx, 0.0f);
-            if (job.counting.counts != nullptr && g >= 0) count_item(job.counting, t, K, n_c, g, it);
+            put_result(job, t, it, g, fmaxf(s_b[lane] + xx, 0.0f));
         }
     }
 }
@@ -389,21 +387,19 @@ __device__ __forceinline__ void split_items(const AssignJob& job, int Kt, const 
         }
     if (it < 0) return;
     if (job.open.ids != nullptr && g >= 0) g = job.open.ids[(size_t)t * K + g];  // column -> centroid
-    job.assign[(size_t)t * n_c + it] = g;
-    if (job.dist != nullptr) job.dist[(size_t)t * n_c + it] = fmaxf(b + xx, 0.0f);
-    if (job.counting.counts != nullptr && g >= 0) count_item(job.counting, t, K, n_c, g, it);
+    put_result(job, t, it, g, fmaxf(b + xx, 0.0f));
 }
 
 template <int KS>
 __global__ __launch_bounds__(kSplitThreads, 2) void k_assign_split(const AssignJob job, const int Kt) {
     const int t = blockIdx.x;
     const int32_t* list = job.list;
-    int n_items = list ? job.list_count[t] : job.n_c;
+    int n_items = items_of(job, t);
     if (job.after_approx && (list == nullptr || approx_takes(n_items, gridDim.x))) {
         list = job.unsure;
-        n_items = job.unsure_count[t];
+        n_items = job.unsure_count[t * kCounterStride];
     }
-    if (job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t] = 0;
+    if (job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t * kCounterStride] = 0;
     for (int b = blockIdx.y; b * split_ri(KS) * 16 < n_items; b += gridDim.y) {  // uniform
         if (b != (int)blockIdx.y) __syncthreads();  // (the results of the stride before are out of LDS)
         split_items<KS>(job, Kt, list, n_items, b);
@@ -652,7 +648,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     }
 
     // ---- who is still in the running (LDS is free behind the loop's last barrier) -------------------
-    const bool want_dist = job.dist != nullptr;  // uniform: then every item's distance is needed
+    const bool want_dist = job.counting.dists != nullptr;  // uniform: then every item's distance is needed
     constexpr int WAVE_BYTES = 64 * 8 + kApproxPairs * 8;
     char* mine = reinterpret_cast<char*>(s_dyn) + wave * WAVE_BYTES;
     unsigned long long* s_key = reinterpret_cast<unsigned long long*>(mine);  // (64) best (distance, column)
@@ -810,7 +806,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     if (__ballot(listed_later) != 0ull) {
         const unsigned long long bal = __ballot(listed_later);
         int base = 0;
-        if (lane == __ffsll((long long)bal) - 1) base = atomicAdd(&job.unsure_count[t], __popcll(bal));
+        if (lane == __ffsll((long long)bal) - 1) base = atomicAdd(&job.unsure_count[t * kCounterStride], __popcll(bal));
         base = __shfl(base, __ffsll((long long)bal) - 1, 64);
         if (listed_later) job.unsure[(size_t)t * n_c + base + __popcll(bal & ((1ull << lane) - 1ull))] = it;
     }
@@ -824,9 +820,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
             const float v = from_ordered((uint32_t)(key >> 32));
             d = EXACT_MFMA ? fmaxf(v + xx, 0.0f) : v;
         }
-        job.assign[(size_t)t * n_c + it] = g;
-        if (want_dist) job.dist[(size_t)t * n_c + it] = d;
-        if (job.counting.counts != nullptr && g >= 0) count_item(job.counting, t, K, n_c, g, it);
+        put_result(job, t, it, g, d);
     }
 }
 
@@ -836,11 +830,11 @@ __global__ __launch_bounds__(kAssignThreads, 2) void k_assign_approx(const Assig
     // (trees in the fast index: the workgroups of a tree run behind the same L2s, which hold its tiles)
     const int t = blockIdx.x;
     constexpr int RI = KS <= 4 ? 4 : 2;
-    const int n_items = LISTED ? job.list_count[t] : job.n_c;
+    const int n_items = items_of(job, t);
     if (LISTED && EXACT_MFMA && !approx_takes(n_items, gridDim.x)) return;  // (k_assign_split's)
     const bool narrow = LISTED && !EXACT_MFMA && !approx_takes(n_items, gridDim.x);
     const int per_block = (kAssignThreads / 64) * 16 * (narrow ? 1 : RI);
-    if (!EXACT_MFMA && job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t] = 0;
+    if (!EXACT_MFMA && job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t * kCounterStride] = 0;
     for (int b = blockIdx.y; b * per_block < n_items; b += gridDim.y) {  // uniform
         if (b != (int)blockIdx.y) __syncthreads();
         if (LISTED && !EXACT_MFMA && narrow) approx_items<T, KS, 1, LISTED, EXACT_MFMA>(job, Kt, tag_bits, n_items, b);

@@ -33,9 +33,10 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     return z ^ (z >> 31);
 }
 
-// what the phases of a level count, per tree: workgroups that are done, items on the two lists, items
-// behind the buckets (of this round, of the next), items the approximate assignment leaves
-constexpr int kBuildCounters = 6;
+// what the phases of a level count, per tree: items on the two lists, items behind the buckets (of
+// this round, of the next), items the approximate assignment leaves, items without a centroid, large
+// buckets (of this round, of the next)
+constexpr int kBuildCounters = 8;
 
 __global__ void k_fill_i32(int32_t* p, size_t n, int32_t v) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -43,14 +44,12 @@ __global__ void k_fill_i32(int32_t* p, size_t n, int32_t v) {
 }
 
 // ------------------------------------------------------------------------------------
-// 0. what a level starts from, in one launch: nothing placed, empty blocks, zero counters; the
-//    centroid columns that pad the last stage of operand tiles are zeros that take no items.
-//    n_live != NULL: tree t holds n_live[t] <= n_c items, the first ones of its rows; the items
-//    it does not hold count as placed from the start (no phase ever touches them), and it uses
-//    its first ceil(n_t / bf) centroids only: the others count as full.
+// 0. what a level starts from, in one launch: empty blocks, zero counters; the centroid columns that
+//    pad the last stage of operand tiles are zeros that take no items.
+//    n_live != NULL: tree t holds n_live[t] <= n_c items, the first ones of its rows, and uses its
+//    first ceil(n_t / bf) centroids only: the others count as full.
 // ------------------------------------------------------------------------------------
-__global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_t* n_live,
-                             int32_t* placed, int32_t* fill, int32_t* slots, int32_t* counts,
+__global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_t* n_live, int32_t* fill, int32_t* slots, int32_t* counts,
                              int32_t* counters /* (kBuildCounters, T) */, CentroidTiles ct, int KS) {
     const int t = blockIdx.y, T = gridDim.y;
     const int n_t = n_live ? min(max(n_live[t], 0), n_c) : n_c;
@@ -58,9 +57,8 @@ __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_
     const int stride = gridDim.x * blockDim.x;
     const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
     if (i0 == 0) {
-        for (int c = 0; c < kBuildCounters; ++c) counters[c * T + t] = 0;
+        for (int c = 0; c < kBuildCounters; ++c) counters[(c * T + t) * kCounterStride] = 0;
     }
-    for (int i = i0; i < n_c; i += stride) placed[(size_t)t * n_c + i] = i >= n_t ? 1 : 0;
     for (int i = i0; i < K; i += stride) {
         fill[(size_t)t * K + i] = i >= K_t ? bf : 0;
         counts[(size_t)t * K + i] = 0;
@@ -118,25 +116,21 @@ __global__ __launch_bounds__(64) void k_init_centroids(const void* x, int n_c, s
 // 2. nearest centroid (vector-ALU kernel): argmin_k ||x_i - c_k||^2, lowest k on ties.
 //    LPR lanes hold one item row; each lane group keeps PPG items in registers and walks
 //    all centroids.  fill != NULL: centroids with fill[k] >= bf are skipped.
-//    list != NULL: only the items list[0 .. *list_count) are processed.
-//    ac: the items a centroid takes are counted as they are assigned (assign.h).
 // ------------------------------------------------------------------------------------
 constexpr int kPPG = 4;
 
 template <typename T, int LPR>
 __global__ __launch_bounds__(256) void k_assign_simple(
-    const void* x, int n_c, size_t x_tree_stride, const float* cent, int K, int D,
-    const int32_t* fill, int bf, const int32_t* list, const int32_t* list_count, size_t list_stride,
-    int32_t* assign, float* dist, AssignCounting ac) {
+    const int32_t* fill, int bf, const AssignJob job) {
     constexpr int EPL = Elem<T>::kPerChunk;
     constexpr int RPW = kWave / LPR;
     const int lane = lane_id();
     const int rg = lane / LPR, ch = lane % LPR;
     const int t = blockIdx.y;
-    const int n_items = list ? list_count[t] : n_c;
+    const int n_items = items_of(job, t), n_c = job.n_c, D = job.D, K = job.K;
     const int wave_global = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int first = wave_global * (RPW * kPPG);
-    if (ac.zero != nullptr && blockIdx.x == 0 && threadIdx.x == 0) ac.zero[t] = 0;
+    if (job.counting.zero != nullptr && blockIdx.x == 0 && threadIdx.x == 0) job.counting.zero[t * kCounterStride] = 0;
     const bool chunk_ok = ch * EPL < D;
 
     if (first < n_items) {  // (wave-uniform; no barrier inside)
@@ -148,15 +142,15 @@ __global__ __launch_bounds__(256) void k_assign_simple(
         for (int p = 0; p < kPPG; ++p) {
             const int pos = first + p * RPW + rg;
             item[p] = -1;
-            if (pos < n_items) item[p] = list ? list[(size_t)t * list_stride + pos] : pos;
+            if (pos < n_items) item[p] = job.list ? job.list[(size_t)t * n_c + pos] : pos;
             uint4 raw = make_uint4(0, 0, 0, 0);
             if (item[p] >= 0 && chunk_ok)
-                raw = load_chunk<T>(x, ((size_t)t * x_tree_stride + item[p]) * D, ch);
+                raw = load_chunk<T>(job.x, ((size_t)t * job.x_tree_stride + item[p]) * D, ch);
             unpack<T>(raw, xf[p]);
             best[p] = INFINITY;
             arg[p] = -1;
         }
-        const float* ct = cent + (size_t)t * K * D;
+        const float* ct = job.cent + (size_t)t * K * D;
         const int32_t* ft = fill ? fill + (size_t)t * K : nullptr;
         for (int k = 0; k < K; ++k) {
             if (ft && ft[k] >= bf) continue;  // wave-uniform
@@ -196,11 +190,7 @@ __global__ __launch_bounds__(256) void k_assign_simple(
         if (ch == 0) {
 #pragma unroll
             for (int p = 0; p < kPPG; ++p) {
-                if (item[p] >= 0) {
-                    assign[(size_t)t * n_c + item[p]] = arg[p];
-                    if (dist != nullptr) dist[(size_t)t * n_c + item[p]] = best[p];
-                    if (ac.counts != nullptr && arg[p] >= 0) count_item(ac, t, K, n_c, arg[p], item[p]);
-                }
+                if (item[p] >= 0) put_result(job, t, item[p], arg[p], best[p]);
             }
         }
     }
@@ -212,22 +202,43 @@ __global__ __launch_bounds__(256) void k_assign_simple(
 struct Buckets {
     int32_t* counts;          // (T, K); every kernel here leaves it zero for the round after it
     const int32_t* members;   // (T, K, kBucketCap)
+    const float* dists;       // (T, K, kBucketCap)
+    const int32_t* big;       // (T, K)
+    const int32_t* big_count;   // (T)
     const int2* more;         // (T, n_c)
     const int32_t* more_count;  // (T)
-    int32_t* next_more_count;   // (T): the round after this one counts here; cleared by these kernels
+    const float* more_dist;     // (T, n_c)
+    int32_t* next_big_count;    // (T): the round after this one counts here; cleared by these kernels
+    int32_t* next_more_count;   // (T): the same
     int32_t* unsure_count;      // (T): cleared by these kernels
 };
 
-// item e of the ones that do not lie in `members` of the tree: its id if it is of bucket k, else -1
-__device__ __forceinline__ int more_of(const Buckets& b, int t, int n_c, int k, int e) {
-    const int2 v = b.more[(size_t)t * n_c + e];
-    return v.x == k ? v.y : -1;
+// f(item) for the items of bucket k among entries [e0, e1) of those that do not lie in `members`;
+// called by the whole workgroup
+template <typename F>
+__device__ __forceinline__ void for_more(const Buckets& b, int t, int n_c, int k, int e0, int e1, F f) {
+    constexpr int U = 8;  // entries on their way at a time
+    const int2* more = b.more + (size_t)t * n_c;
+    for (int e = e0 + (int)threadIdx.x; e < e1; e += U * (int)blockDim.x) {
+        int2 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = e + u * (int)blockDim.x < e1 ? more[e + u * (int)blockDim.x] : make_int2(-1, 0);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (v[u].x == k) f(v[u].y);
+    }
 }
 
 // The order in which a bucket's members arrive depends on the run; everything that follows works
-// on them in a fixed order, which a workgroup per bucket establishes in LDS:
-//   up to 256 members   every thread ranks its member against all others
-//   more                a bitonic sorting network over the next power of two
+// on them in a fixed order.  Most buckets have about `bf` members (32 or so): a wave has one to
+// itself, ranks each lane's member against the others' in registers and works on without a barrier
+// (kWaveBucket members at most; a workgroup per bucket spent its time on five barriers and on 224
+// idle threads).  The larger ones, which the assignment has listed, take a workgroup each; the
+// launch's first workgroups do those, so that the longest start first:
+//   up to kBucketCap    every thread ranks its member against all others
+//   more                a bit map of the members (means), a bitonic sorting network (packing)
+constexpr int kWaves = 4;  // of a workgroup of the per-bucket kernels
+static int large_blocks(int K) { return min(max(K / 8, 1), 256); }  // workgroups of a tree for large buckets
 constexpr int kBucketThreads = 256;
 
 template <typename Key>
@@ -255,142 +266,253 @@ __device__ __forceinline__ int pow2_at_least(int n) {
     return p;
 }
 
-// (what every workgroup of the per-bucket kernels does for the round after it, having read the count)
-__device__ __forceinline__ void reset_counters(const Buckets& b, int t, int k, int K) {
-    if (threadIdx.x == 0) {
-        b.counts[(size_t)t * K + k] = 0;
-        if (k == 0) {
-            b.next_more_count[t] = 0;
-            b.unsure_count[t] = 0;
+// rank of this lane's value among those of lanes 0 .. m - 1 (distinct; the other lanes hold the
+// largest number; m uniform in the wave).  Lane numbers are constants: a step is three or four
+// instructions.
+template <typename Key>
+__device__ __forceinline__ int wave_rank(Key mine, int m) {
+    int rank = 0;
+#pragma unroll
+    for (int j0 = 0; j0 < 64; j0 += 8) {
+        if (j0 >= m) break;
+#pragma unroll
+        for (int j = j0; j < j0 + 8; ++j) {
+            Key o;
+            if constexpr (sizeof(Key) == 8)
+                o = ((Key)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mine >> 32), j) << 32) |
+                    (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, j);
+            else
+                o = (Key)__builtin_amdgcn_readlane((int)mine, j);
+            rank += o < mine ? 1 : 0;
         }
     }
+    return rank;
+}
+
+// what the wave, or the workgroup, that has read the count of its bucket does for the round after it
+// (behind a barrier: the count is read through the scalar cache, and only the wait there keeps this
+// store from overtaking it; a bucket's other reader finds a large count, or none, and leaves it)
+__device__ __forceinline__ void reset_count(const Buckets& b, int t, int k, int K) {
+    b.counts[(size_t)t * K + k] = 0;
+}
+__device__ __forceinline__ void reset_round(const Buckets& b, int t) {  // (one thread of the tree)
+    b.next_big_count[t * kCounterStride] = 0;
+    b.next_more_count[t * kCounterStride] = 0;
+    b.unsure_count[t * kCounterStride] = 0;
 }
 
 // ------------------------------------------------------------------------------------
-// 4. Lloyd round: centroid = mean of the member rows.  One workgroup per centroid: the members
-//    in the order of their item ids, row e summed by row group e % R, the R sums added in order:
-//    the result does not depend on the order of arrival.  An empty centroid keeps its value.
+// 4. Lloyd round: centroid = mean of the member rows: the members in the order of their item ids,
+//    row e summed by row group e % R, the R sums added in order, so the result does not depend on the
+//    order of arrival.  (A row is CPR threads of 16 bytes, R = 256 / CPR rows at a time: 256 threads of a
+//    workgroup, or four times the 64 lanes of a wave.)  An empty centroid keeps its value.
 //    ct.tiles != NULL: the new centroid also goes into its operand tile.
+//    What bounds it is the gather of the rows and, to the end, the few largest buckets (1473 rows at
+//    8 x 131072 items, beside a mean of 32): 8 x 32768 rows of 256 bytes 71 -> 39 us, 8 x 131072
+//    200 -> 125 us.
 // ------------------------------------------------------------------------------------
-constexpr int kMeanSort = 4096;      // members ordered in LDS; more: through a bit map of item ids
-constexpr int kMeanMapBits = kMeanSort * 32;
+constexpr int kMeanMap = 4096;  // words of a bit map of item ids, for buckets beyond kBucketCap
+constexpr int kMeanMapBits = kMeanMap * 32;
 
 template <typename T>
 __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
     const void* x, size_t x_tree_stride, int n_c, int K, int D, const Buckets bk,
-    const int32_t* fill, int bf, float* cent, int Kt, const CentroidTiles ct, int KS) {
+    const int32_t* fill, int bf, float* cent, int Kt, const CentroidTiles ct, int KS, int large) {
     constexpr int EPL = Elem<T>::kPerChunk;
-    __shared__ uint32_t s_ord[kMeanSort];            // (as a bit map: kMeanMapBits ids)
-    __shared__ float s_part[kBucketThreads * EPL];   // (R, D) partial sums, R * D <= 256 * EPL
-    __shared__ int32_t s_small[kBucketThreads];
-    __shared__ int32_t s_n;
-    const int k = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
-    const int m = bk.counts[(size_t)t * K + k];
-    const int32_t* mem = bk.members + ((size_t)t * K + k) * kBucketCap;
-    if (tid == 0) s_n = kBucketCap;
-    __syncthreads();  // (every thread has read the count)
-    reset_counters(bk, t, k, K);
-    if (m <= 0) return;
-    // ---- sums: CPR threads a row, R rows at a time -------------------------------------------
+    constexpr int kPart = kBucketThreads * EPL;  // (R, D) partial sums, R * D <= 256 * EPL
+    constexpr int kPiece = 64 * EPL;             // a quarter of them
+    // one bucket: partial sums, ids in order or their bit map, counts of the bit map's stretches;
+    // or, a wave each: a quarter of the partial sums
+    __shared__ __attribute__((aligned(16))) float s_lds[kPart + kMeanMap + kBucketThreads];
+    __shared__ uint32_t s_ids[kWaves][kWaveBucket];
+    static_assert(kWaves * kPiece <= kPart, "a quarter for every wave");
+    const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int CPR = D / EPL, R = kBucketThreads / CPR;
-    const int r = tid / CPR, c = tid % CPR;
-    float acc[EPL];
+    auto usable = [&](int k) { return !(fill != nullptr && fill[(size_t)t * K + k] >= bf); };
+    if (blockIdx.x == 0 && tid == 0) reset_round(bk, t);
+    if ((int)blockIdx.x >= large) {
+        const int k = ((int)blockIdx.x - large) * kWaves + wave;
+        if (k >= K) return;
+        uint32_t id = (uint32_t)bk.members[((size_t)t * K + k) * kBucketCap + lane];  // (garbage from m on)
+        const int m = __builtin_amdgcn_readfirstlane(bk.counts[(size_t)t * K + k]);
+        if (m <= 0 || m > kWaveBucket) return;
+        if (lane >= m) id = 0xffffffffu;
+        const int rank = wave_rank(id, m);
+        if (lane < m) s_ids[wave][rank] = id;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (lane == 0) reset_count(bk, t, k, K);
+        float acc[4][EPL];
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] = 0.0f;
-    // rows [e0, e0 + n) in order, their ids at ids[0 .. n)
-    auto add_rows = [&](const uint32_t* ids, int e0, int n) {
-        if (r < R)
-            for (int e = e0 + (r - e0 % R + R) % R; e < e0 + n; e += R) {
-                float f[EPL];
-                unpack<T>(load_chunk<T>(x, ((size_t)t * x_tree_stride + (int)ids[e - e0]) * D, c), f);
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int q = 0; q < EPL; ++q) acc[q] += f[q];
-            }
-    };
-    if (m <= kBucketCap) {
-        const int mine = tid < m ? mem[tid] : 0x7fffffff;
-        s_small[tid] = mine;
-        __syncthreads();
-        int rank = 0;
-        for (int j = 0; j < m; ++j) rank += s_small[j] < mine;
-        if (tid < m) s_ord[rank] = (uint32_t)mine;
-        __syncthreads();
-        add_rows(s_ord, 0, m);
-    } else if (m <= kMeanSort) {
-        const int P = pow2_at_least(m), others = bk.more_count[t];
-        for (int e = tid; e < P; e += kBucketThreads) s_ord[e] = e < kBucketCap ? (uint32_t)mem[e] : 0xffffffffu;
-        __syncthreads();
-        for (int e = tid; e < others; e += kBucketThreads) {
-            const int it = more_of(bk, t, n_c, k, e);
-            if (it >= 0) s_ord[atomicAdd(&s_n, 1)] = (uint32_t)it;
+            for (int q = 0; q < EPL; ++q) acc[i][q] = 0.0f;
+        for (int e0 = 0; e0 < m; e0 += 2 * R) {  // uniform
+            uint4 raw[2][4];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int v = lane + 64 * i, e = e0 + h * R + v / CPR;
+                    raw[h][i] = make_uint4(0, 0, 0, 0);
+                    if (v < R * CPR && e < m)
+                        raw[h][i] = load_chunk<T>(x, ((size_t)t * x_tree_stride + s_ids[wave][e]) * D, v % CPR);
+                }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {  // (a row that is none adds zeros)
+                    float f[EPL];
+                    unpack<T>(raw[h][i], f);
+#pragma unroll
+                    for (int q = 0; q < EPL; ++q) acc[i][q] += f[q];
+                }
         }
-        bitonic_sort(s_ord, P);
-        add_rows(s_ord, 0, m);
-    } else {
-        // ids in ranges of kMeanMapBits: a bit per member, then the set bits in order, as many of them
-        // at a time as there is room for in s_part
-        constexpr int kPiece = kBucketThreads * EPL;
-        uint32_t* piece = reinterpret_cast<uint32_t*>(s_part);
-        const int others = bk.more_count[t];
-        int written = 0;
-        for (int lo = 0; lo < n_c; lo += kMeanMapBits) {
-            __syncthreads();
-            for (int w = tid; w < kMeanSort; w += kBucketThreads) s_ord[w] = 0;
-            __syncthreads();
-            auto mark = [&](int it) {
-                const int d = it - lo;
-                if (it >= 0 && d >= 0 && d < kMeanMapBits) atomicOr(&s_ord[d >> 5], 1u << (d & 31));
-            };
-            if (tid < kBucketCap) mark(mem[tid]);
-            for (int e = tid; e < others; e += kBucketThreads) mark(more_of(bk, t, n_c, k, e));
-            __syncthreads();
-            // thread `tid` owns the words [tid * W, (tid + 1) * W)
-            constexpr int W = kMeanSort / kBucketThreads;
-            const int in_range = block_exclusive_scan(
-                kBucketThreads, [&](int i) {
-                    int n = 0;
-                    for (int w = 0; w < W; ++w) n += __popc(s_ord[i * W + w]);
-                    return n;
-                },
-                [&](int i, int v) { s_small[i] = v; });
-            __syncthreads();
-            for (int p0 = 0; p0 < in_range; p0 += kPiece) {
-                int at = s_small[tid];
-                for (int w = 0; w < W; ++w) {
-                    uint32_t bits = s_ord[tid * W + w];
-                    while (bits) {
-                        const int b = __ffs(bits) - 1;
-                        bits &= bits - 1;
-                        if (at >= p0 && at < p0 + kPiece) piece[at - p0] = (uint32_t)(lo + (tid * W + w) * 32 + b);
-                        ++at;
+        // the partial sums as one row of R * D numbers pass through LDS a quarter at a time; a lane
+        // adds up its columns
+        float* piece = s_lds + wave * kPiece;
+        const int rows = min(R, m);
+        float sum[8];
+        int at[8];  // where the column's next partial sum lies
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            sum[u] = 0.0f;
+            at[u] = lane + 64 * u;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int q = 0; q < EPL; ++q) piece[lane * EPL + q] = acc[i][q];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int end = min((i + 1) * kPiece, rows * D);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (64 * u < D)  // uniform
+                    for (; at[u] < end; at[u] += D) sum[u] += piece[at[u] - i * kPiece];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int j = lane + 64 * u;
+            if (j < D) {
+                const float v = sum[u] / (float)m;
+                cent[((size_t)t * K + k) * D + j] = v;
+                piece[j] = v;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (ct.tiles != nullptr) emit_centroid(piece, D, KS, Kt, t, k, usable(k), ct);
+        return;
+    }
+    // ---- the large ones --------------------------------------------------------------------------
+    float* s_part = s_lds;
+    uint32_t* s_ord = reinterpret_cast<uint32_t*>(s_lds + kPart);
+    int32_t* s_small = reinterpret_cast<int32_t*>(s_lds + kPart + kMeanMap);
+    const int nbig = bk.big_count[t * kCounterStride];
+    for (int i = blockIdx.x; i < nbig; i += large) {  // uniform
+        const int k = bk.big[(size_t)t * K + i];
+        const int m = bk.counts[(size_t)t * K + k];
+        const int32_t* mem = bk.members + ((size_t)t * K + k) * kBucketCap;
+        __syncthreads();
+        if (tid == 0) reset_count(bk, t, k, K);
+        const int r = tid / CPR, c = tid % CPR;
+        float acc[EPL];
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[e] = 0.0f;
+        // rows [e0, e0 + n) in order, their ids at ids[0 .. n)
+        auto add_rows = [&](const uint32_t* ids, int e0, int n) {
+            constexpr int U = 8;  // rows on their way at a time
+            if (r < R)
+                for (int e = e0 + (r - e0 % R + R) % R; e < e0 + n; e += U * R) {
+                    uint4 raw[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        raw[u] = make_uint4(0, 0, 0, 0);
+                        if (e + u * R < e0 + n)
+                            raw[u] = load_chunk<T>(x, ((size_t)t * x_tree_stride + (int)ids[e + u * R - e0]) * D, c);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        float f[EPL];
+                        unpack<T>(raw[u], f);
+                        if (e + u * R < e0 + n) {
+#pragma unroll
+                            for (int q = 0; q < EPL; ++q) acc[q] += f[q];
+                        }
                     }
                 }
+        };
+        if (m <= kBucketCap) {
+            const int mine = tid < m ? mem[tid] : 0x7fffffff;
+            s_small[tid] = mine;
+            __syncthreads();
+            int rank = 0;
+            for (int j = 0; j < m; ++j) rank += s_small[j] < mine;
+            if (tid < m) s_ord[rank] = (uint32_t)mine;
+            __syncthreads();
+            add_rows(s_ord, 0, m);
+        } else {
+            // ids in ranges of kMeanMapBits: a bit per member, then the set bits in order, as many of
+            // them at a time as there is room for in s_part
+            uint32_t* piece = reinterpret_cast<uint32_t*>(s_part);
+            constexpr int W = kMeanMap / kBucketThreads;
+            const int others = bk.more_count[t * kCounterStride];
+            int written = 0;
+            for (int lo = 0; lo < n_c; lo += kMeanMapBits) {
                 __syncthreads();
-                add_rows(piece, written + p0, min(kPiece, in_range - p0));
+                const int per = min(W, (n_c - lo + 32 * kBucketThreads - 1) / (32 * kBucketThreads));
+                for (int i = tid; i < per * kBucketThreads; i += kBucketThreads) s_ord[i] = 0;
                 __syncthreads();
+                auto mark = [&](int it) {
+                    const int d = it - lo;
+                    if (d >= 0 && d < kMeanMapBits) atomicOr(&s_ord[d >> 5], 1u << (d & 31));
+                };
+                if (tid < kBucketCap) mark(mem[tid]);
+                for_more(bk, t, n_c, k, 0, others, mark);
+                __syncthreads();
+                // thread `tid` owns the words [tid * per, (tid + 1) * per)
+                const int in_range = block_exclusive_scan(
+                    kBucketThreads, [&](int i) {
+                        int n = 0;
+                        for (int u = 0; u < per; ++u) n += __popc(s_ord[i * per + u]);
+                        return n;
+                    },
+                    [&](int i, int v) { s_small[i] = v; });
+                __syncthreads();
+                for (int p0 = 0; p0 < in_range; p0 += kPart) {
+                    int at = s_small[tid];
+                    for (int u = 0; u < per; ++u) {
+                        uint32_t bits = s_ord[tid * per + u];
+                        while (bits) {
+                            const int b = __ffs(bits) - 1;
+                            bits &= bits - 1;
+                            if (at >= p0 && at < p0 + kPart) piece[at - p0] = (uint32_t)(lo + (tid * per + u) * 32 + b);
+                            ++at;
+                        }
+                    }
+                    __syncthreads();
+                    add_rows(piece, written + p0, min(kPart, in_range - p0));
+                    __syncthreads();
+                }
+                written += in_range;
             }
-            written += in_range;
         }
-    }
-    if (r < R) {
+        __syncthreads();
+        if (r < R) {
 #pragma unroll
-        for (int q = 0; q < EPL; ++q) s_part[r * D + c * EPL + q] = acc[q];
-    }
-    __syncthreads();
-    float v = 0.0f;
-    for (int j = tid; j < D; j += kBucketThreads) {  // (D <= 512: at most two columns a thread)
-        float s = 0.0f;
+            for (int q = 0; q < EPL; ++q) s_part[r * D + c * EPL + q] = acc[q];
+        }
+        __syncthreads();
         const int rows = min(R, m);
-        for (int q = 0; q < rows; ++q) s += s_part[q * D + j];
-        v = s / (float)m;
-        cent[((size_t)t * K + k) * D + j] = v;
-    }
-    if (ct.tiles != nullptr) {  // (D <= 256: column tid)
+        for (int j = tid; j < D; j += kBucketThreads) {
+            float s = 0.0f;
+            for (int q = 0; q < rows; ++q) s += s_part[q * D + j];
+            const float v = s / (float)m;
+            cent[((size_t)t * K + k) * D + j] = v;
+            s_part[j] = v;  // (nobody else reads column j)
+        }
         __syncthreads();
-        if (tid < D) s_part[tid] = v;
-        __syncthreads();
-        if (tid < 64)
-            emit_centroid(s_part, D, KS, Kt, t, k, !(fill != nullptr && fill[(size_t)t * K + k] >= bf), ct);
+        if (ct.tiles != nullptr && wave == 0) emit_centroid(s_part, D, KS, Kt, t, k, usable(k), ct);
     }
 }
 
@@ -444,177 +566,191 @@ __global__ __launch_bounds__(64) void k_block_mean(const void* x, size_t x_tree_
 // ------------------------------------------------------------------------------------
 // 5. capacity packing
 // ------------------------------------------------------------------------------------
-// One workgroup per bucket: the closest proposers (by distance, then item id) take the free
-// slots of the block in that order; the others go on the list of the next round.  A block that
-// is full now takes no more items: its norm in the operand tiles becomes +inf.
+// The closest proposers of a bucket (by distance, then item id) take the free slots of the block in
+// that order; the others go on the list of the next round.  A block that is full now takes no more
+// items: its norm in the operand tiles becomes +inf.  (One addition to the list's length per
+// workgroup: a tree's 1024 or 4096 buckets would queue up at it.)  What bounds it is the chain count,
+// members, place on the list; first round of 8 x 131072 items 159 -> 60 us, of 8 x 32768 45 -> 14.
 constexpr int kAcceptSort = 2048;  // keys sorted at a time; larger buckets in several goes, the
                                    // best `take` (at most 64) so far carried along
 
 __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
-    const Buckets bk, const float* dist, int n_c, int K, int bf, int32_t* fill, int32_t* slots,
-    int32_t* placed, int32_t* next_list, int32_t* next_count, int Kt, float* cn2) {
+    const Buckets bk, int n_c, int K, int bf, int32_t* fill, int32_t* slots, int32_t* next_list,
+    int32_t* next_count, int Kt, float* cn2, int large) {
     __shared__ uint64_t s_keys[kAcceptSort];
+    __shared__ int32_t s_back[kWaves];
     __shared__ int32_t s_base, s_rej, s_n;
-    const int k = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
-    const int m = bk.counts[(size_t)t * K + k];
-    const int32_t* mem = bk.members + ((size_t)t * K + k) * kBucketCap;
-    const float* dt = dist + (size_t)t * n_c;
-    const int f = fill[(size_t)t * K + k];
-    const int take = max(min(m, bf - f), 0);
-    int32_t* my_slots = slots + ((size_t)t * K + k) * bf + f;
-    int32_t* pl = placed + (size_t)t * n_c;
+    const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int32_t* nl = next_list + (size_t)t * n_c;
-    __syncthreads();  // (every thread has read the block's fill and the bucket's count)
-    reset_counters(bk, t, k, K);
-    if (m <= 0) return;
-    if (tid == 0) {
-        s_base = m > take ? atomicAdd(&next_count[t], m - take) : 0;
-        s_rej = 0;
-        fill[(size_t)t * K + k] = f + take;
-        if (cn2 != nullptr && f + take >= bf) cn2[(size_t)t * Kt * 16 + k] = INFINITY;
-    }
-    auto key_of = [&](int it) { return ((uint64_t)__float_as_uint(dt[it]) << 32) | (uint32_t)it; };
-    if (m <= kBucketCap) {
-        int it = -1;
-        uint64_t mine = ~0ull;
-        if (tid < m) {
-            it = mem[tid];
-            mine = key_of(it);
+    auto key_of = [](float d, int it) { return ((uint64_t)__float_as_uint(d) << 32) | (uint32_t)it; };
+    auto filled = [&](int k, int f) {  // (one thread)
+        fill[(size_t)t * K + k] = f;
+        if (cn2 != nullptr && f >= bf) cn2[(size_t)t * Kt * 16 + k] = INFINITY;
+    };
+    if (blockIdx.x == 0 && tid == 0) reset_round(bk, t);
+    if ((int)blockIdx.x >= large) {
+        const int k = ((int)blockIdx.x - large) * kWaves + wave;
+        int m = 0, f = 0, take = 0;
+        uint64_t mine = 0;
+        if (k < K) {
+            const size_t b = (size_t)t * K + k;
+            mine = key_of(bk.dists[b * kBucketCap + lane], bk.members[b * kBucketCap + lane]);  // (garbage from m on)
+            m = __builtin_amdgcn_readfirstlane(bk.counts[b]);
+            f = __builtin_amdgcn_readfirstlane(fill[b]);
+            if (m > kWaveBucket) m = 0;
+            take = max(min(m, bf - f), 0);
+            if (lane == 0 && take > 0) filled(k, f + take);
         }
-        s_keys[tid] = mine;
+        if (lane >= m) mine = ~0ull;
+        if (lane == 0) s_back[wave] = m - take;
         __syncthreads();
-        int rank = 0;
-        for (int j = 0; j < m; ++j) rank += s_keys[j] < mine;
-        if (tid < m) {
+        if (lane == 0 && m > 0) reset_count(bk, t, k, K);
+        if (tid == 0) {
+            const int back = s_back[0] + s_back[1] + s_back[2] + s_back[3];
+            s_base = back > 0 ? atomicAdd(&next_count[t * kCounterStride], back) : 0;
+        }
+        const int rank = wave_rank(mine, m);  // (the addition is on its way)
+        __syncthreads();
+        if (lane < m) {
             if (rank < take) {
-                my_slots[rank] = it;
-                pl[it] = 1;
+                slots[((size_t)t * K + k) * bf + f + rank] = (int)(uint32_t)mine;
             } else {
-                nl[s_base + rank - take] = it;
+                int at = s_base + rank - take;
+                for (int w = 0; w < wave; ++w) at += s_back[w];
+                nl[at] = (int)(uint32_t)mine;
             }
         }
         return;
     }
-    // s_keys[0 .. n): the best so far and those not looked at yet; a kAcceptStep of the others at a
-    // time is searched for the bucket's items
-    constexpr int kAcceptStep = kAcceptSort - kBucketCap - 64;
-    const int others = bk.more_count[t];
-    if (tid < kBucketCap) s_keys[tid] = key_of(mem[tid]);
-    if (tid == 0) s_n = kBucketCap;
-    for (int e0 = 0; e0 < others; e0 += kAcceptStep) {
-        __syncthreads();
-        for (int e = e0 + tid; e < min(e0 + kAcceptStep, others); e += kBucketThreads) {
-            const int it = more_of(bk, t, n_c, k, e);
-            if (it >= 0) s_keys[atomicAdd(&s_n, 1)] = key_of(it);
+    // ---- the large ones --------------------------------------------------------------------------
+    const int nbig = bk.big_count[t * kCounterStride];
+    for (int i = blockIdx.x; i < nbig; i += large) {  // uniform
+        const int k = bk.big[(size_t)t * K + i];
+        const size_t b = (size_t)t * K + k;
+        const int m = bk.counts[b], f = fill[b];
+        const int32_t* mem = bk.members + b * kBucketCap;
+        const float* md = bk.dists + b * kBucketCap;
+        const float* more_d = bk.more_dist + (size_t)t * n_c;
+        int32_t* my_slots = slots + b * bf + f;
+        const int take = max(min(m, bf - f), 0);
+        __syncthreads();  // (everybody has read; what the bucket before left in LDS is used)
+        if (tid == 0) {
+            s_rej = 0;
+            s_base = m > take ? atomicAdd(&next_count[t * kCounterStride], m - take) : 0;
+            reset_count(bk, t, k, K);
+            filled(k, f + take);
+        }
+        if (m <= kBucketCap) {
+            const uint64_t own = tid < m ? key_of(md[tid], mem[tid]) : ~0ull;
+            s_keys[tid] = own;
+            __syncthreads();
+            int r = 0;
+            for (int j = 0; j < m; ++j) r += s_keys[j] < own;
+            if (tid < m) {
+                if (r < take) my_slots[r] = (int)(uint32_t)own;
+                else nl[s_base + r - take] = (int)(uint32_t)own;
+            }
+            continue;
+        }
+        // s_keys[0 .. n): the best so far and those not looked at yet; a kAcceptStep of the others at
+        // a time is searched for the bucket's items
+        constexpr int kAcceptStep = kAcceptSort - kBucketCap - 64;
+        const int others = bk.more_count[t * kCounterStride];
+        if (tid < kBucketCap) s_keys[tid] = key_of(md[tid], mem[tid]);
+        if (tid == 0) s_n = kBucketCap;
+        for (int e0 = 0; e0 < others; e0 += kAcceptStep) {
+            __syncthreads();
+            for_more(bk, t, n_c, k, e0, min(e0 + kAcceptStep, others),
+                     [&](int it) { s_keys[atomicAdd(&s_n, 1)] = key_of(more_d[it], it); });
+            __syncthreads();
+            const int n = s_n, P = pow2_at_least(n);
+            for (int e = n + tid; e < P; e += kBucketThreads) s_keys[e] = ~0ull;
+            bitonic_sort(s_keys, P);
+            if (tid == 0) s_n = min(take, n);
         }
         __syncthreads();
-        const int n = s_n, P = pow2_at_least(n);
-        for (int e = n + tid; e < P; e += kBucketThreads) s_keys[e] = ~0ull;
-        bitonic_sort(s_keys, P);
-        if (tid == 0) s_n = min(take, n);
-    }
-    __syncthreads();
-    for (int r = tid; r < take; r += kBucketThreads) {
-        const int it = (int)(uint32_t)s_keys[r];
-        my_slots[r] = it;
-        pl[it] = 1;
-    }
-    if (m > take) {  // whoever lies behind the last one taken tries again
-        const uint64_t last = take > 0 ? s_keys[take - 1] : 0ull;
-        auto again = [&](int it) {
-            if (it >= 0 && (take == 0 || key_of(it) > last)) nl[s_base + atomicAdd(&s_rej, 1)] = it;
-        };
-        if (tid < kBucketCap) again(mem[tid]);
-        for (int e = tid; e < others; e += kBucketThreads) again(more_of(bk, t, n_c, k, e));
+        for (int r = tid; r < take; r += kBucketThreads) my_slots[r] = (int)(uint32_t)s_keys[r];
+        if (m > take) {  // whoever lies behind the last one taken tries again
+            const uint64_t last = take > 0 ? s_keys[take - 1] : 0ull;
+            auto again = [&](float d, int it) {
+                if (take == 0 || key_of(d, it) > last) nl[s_base + atomicAdd(&s_rej, 1)] = it;
+            };
+            if (tid < kBucketCap) again(md[tid], mem[tid]);
+            for_more(bk, t, n_c, k, 0, others, [&](int it) { again(more_d[it], it); });
+        }
     }
 }
 
-// (one atomic per workgroup of 256 items, not per wave: the tree's counter is one address)
-__global__ __launch_bounds__(256) void k_collect_unplaced(const int32_t* placed, int n_c,
-                                                          int32_t* list, int32_t* list_count) {
-    __shared__ int32_t s_cnt[4];
-    __shared__ int32_t s_base;
-    const int t = blockIdx.y;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool mine = i < n_c && placed[(size_t)t * n_c + i] == 0;
-    const unsigned long long bal = __ballot(mine);
-    const int lane = lane_id(), wave = threadIdx.x >> 6;
-    if (lane == 0) s_cnt[wave] = __popcll(bal);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int total = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-        s_base = total > 0 ? atomicAdd(&list_count[t], total) : 0;
+// Whatever is still unplaced -- the list the last round left, and items that have no nearest
+// centroid -- goes to the free slots in order: the u-th of them (by item id) takes the u-th free
+// slot (by block, then slot).  A workgroup per tree: the ids in order through a bit map, then a walk over
+// the blocks.  (Few or none are left as a rule.  Two launches over all items took 17 + 5 us at 8 x 32768
+// items and 56 + 10 us at 8 x 131072.)
+constexpr int kLeftThreads = 1024;
+constexpr int kLeftWords = 16 * 1024;  // of the bit map: 512K ids at a time
+
+// exclusive prefix sum over the workgroup; `total` is that of all
+__device__ __forceinline__ int leftover_scan(int mine, int* s_w, int* total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int inc = mine;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(inc, off, 64);
+        if (lane >= off) inc += o;
     }
     __syncthreads();
-    int before = s_base;
-    for (int w = 0; w < wave; ++w) before += s_cnt[w];
-    if (mine) list[(size_t)t * n_c + before + __popcll(bal & ((1ull << lane) - 1ull))] = i;
+    if (lane == 63) s_w[wave] = inc;
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int w = 0; w < kLeftThreads / 64; ++w) {
+        if (w < wave) before += s_w[w];
+        all += s_w[w];
+    }
+    *total = all;
+    return before + inc - mine;
 }
 
-// Whatever is still unplaced goes to the free slots in order: the u-th unplaced item (by
-// item id) takes the u-th free slot (by block, then slot).  Two launches: the unplaced items of
-// every 256 are counted, and the tree's last workgroup turns the counts, and the free slots
-// of the blocks, into prefix sums; then every item finds its slot by itself.
-__global__ __launch_bounds__(256) void k_leftover_count(const int32_t* placed, int n_c, int K,
-                                                        int bf, const int32_t* fill,
-                                                        int32_t* chunk_pre /* (T, chunks + 1) */,
-                                                        int32_t* free_pre /* (T, K + 1) */,
-                                                        int32_t* done) {
-    __shared__ int32_t s_cnt[4];
-    __shared__ int32_t s_last;
-    const int t = blockIdx.y, nb = gridDim.x;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool mine = i < n_c && placed[(size_t)t * n_c + i] == 0;
-    const unsigned long long bal = __ballot(mine);
-    if (lane_id() == 0) s_cnt[threadIdx.x >> 6] = __popcll(bal);
-    __syncthreads();
-    int32_t* cp = chunk_pre + (size_t)t * (nb + 1);
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(&cp[blockIdx.x], s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3],
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        hand_off_release();  // (the count is where every workgroup sees it before the ticket)
-        s_last = atomicAdd(&done[t], 1) == nb - 1 ? 1 : 0;
+__global__ __launch_bounds__(kLeftThreads) void k_leftover(
+    const int32_t* list, const int32_t* list_count, const int32_t* lost, const int32_t* lost_count, int n_c,
+    int K, int bf, const int32_t* fill, int32_t* sorted /* (T, n_c) */, int32_t* slots) {
+    __shared__ uint32_t s_map[kLeftWords];
+    __shared__ int s_w[kLeftThreads / 64];
+    const int t = blockIdx.x, tid = threadIdx.x;
+    const int nl = list_count[t * kCounterStride], total = nl + lost_count[t * kCounterStride];
+    if (total == 0) return;
+    const int32_t* lt = list + (size_t)t * n_c;
+    const int32_t* xt = lost + (size_t)t * n_c;
+    int32_t* st = sorted + (size_t)t * n_c;
+    int done = 0, sum;
+    for (int lo = 0; lo < n_c && done < total; lo += kLeftWords * 32) {  // uniform
+        const int words = min(kLeftWords, (n_c - lo + 31) / 32), per = (words + kLeftThreads - 1) / kLeftThreads;
+        __syncthreads();
+        for (int i = tid; i < words; i += kLeftThreads) s_map[i] = 0;
+        __syncthreads();
+        for (int e = tid; e < total; e += kLeftThreads) {
+            const int d = (e < nl ? lt[e] : xt[e - nl]) - lo;
+            if (d >= 0 && d < words * 32) atomicOr(&s_map[d >> 5], 1u << (d & 31));
+        }
+        __syncthreads();
+        int mine = 0;
+        for (int i = tid * per; i < min((tid + 1) * per, words); ++i) mine += __popc(s_map[i]);
+        int at = done + leftover_scan(mine, s_w, &sum);
+        for (int i = tid * per; i < min((tid + 1) * per, words); ++i)
+            for (uint32_t bits = s_map[i]; bits; bits &= bits - 1) st[at++] = lo + i * 32 + __ffs(bits) - 1;
+        done += sum;
     }
+    __threadfence_block();
     __syncthreads();
-    if (!s_last) return;
-    const int unplaced = block_exclusive_scan(
-        nb, [&](int b) { return load_agent(cp + b); }, [&](int b, int v) { cp[b] = v; });
-    int32_t* fp = free_pre + (size_t)t * (K + 1);
-    const int32_t* ft = fill + (size_t)t * K;
-    const int room = block_exclusive_scan(
-        K, [&](int k) { return bf - ft[k]; }, [&](int k, int v) { fp[k] = v; });
-    if (threadIdx.x == 0) {
-        cp[nb] = unplaced;
-        fp[K] = room;
-        done[t] = 0;
+    int before = 0;  // free slots ahead
+    for (int k0 = 0; k0 < K && before < total; k0 += kLeftThreads) {  // uniform
+        const int k = k0 + tid;
+        const int f = k < K ? fill[(size_t)t * K + k] : bf;
+        const int room = max(bf - f, 0);
+        const int at = before + leftover_scan(room, s_w, &sum);
+        for (int j = 0; j < room && at + j < total; ++j) slots[((size_t)t * K + k) * bf + f + j] = st[at + j];
+        before += sum;
     }
-}
-
-__global__ __launch_bounds__(256) void k_leftover_place(int n_c, int K, int bf, const int32_t* fill,
-                                                        const int32_t* chunk_pre,
-                                                        const int32_t* free_pre, int32_t* slots,
-                                                        int32_t* placed) {
-    __shared__ int32_t s_cnt[4];
-    const int t = blockIdx.y, nb = gridDim.x;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool mine = i < n_c && placed[(size_t)t * n_c + i] == 0;
-    const unsigned long long bal = __ballot(mine);
-    const int lane = lane_id(), wave = threadIdx.x >> 6;
-    if (lane == 0) s_cnt[wave] = __popcll(bal);
-    __syncthreads();
-    if (!mine) return;
-    int u = chunk_pre[(size_t)t * (nb + 1) + blockIdx.x] + __popcll(bal & ((1ull << lane) - 1ull));
-    for (int w = 0; w < wave; ++w) u += s_cnt[w];
-    // block k with free_pre[k] <= u < free_pre[k + 1]
-    const int32_t* fp = free_pre + (size_t)t * (K + 1);
-    int lo = 0, hi = K;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (fp[mid] <= u) lo = mid; else hi = mid;
-    }
-    const int j = fill[(size_t)t * K + lo] + (u - fp[lo]);
-    slots[((size_t)t * K + lo) * bf + j] = i;
-    placed[(size_t)t * n_c + i] = 1;
 }
 
 // ------------------------------------------------------------------------------------
@@ -756,12 +892,12 @@ struct BuildWs {
     CentroidTiles ct;    // centroids as operand tiles (matrix cores), or NULL
     CentroidTiles open;  // the same for the centroids with room, side by side (later packing rounds)
     int32_t *open_ids, *open_count;
-    int32_t *assign, *placed, *members, *unsure;
+    int32_t *members, *big, *unsure, *lost;
+    float *dists, *more_dist;
     int2* more;
     int32_t* list[2];     // the items of a packing round, and those of the round after it
-    int32_t* counters;    // (kBuildCounters, T)
-    float* dist;
-    int32_t *counts, *fill, *free_pre, *chunk_pre;
+    int32_t* counters;    // (kBuildCounters, T), kCounterStride apart
+    int32_t *counts, *fill;
     int32_t* slots[HIRA_MAX_LEVELS];
     void* cent_t[HIRA_MAX_LEVELS];
     int32_t* order[HIRA_MAX_LEVELS];
@@ -803,19 +939,18 @@ static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
         b->open_ids = c.take<int32_t>((size_t)T * k1);
         b->open_count = c.take<int32_t>((size_t)T);
     }
-    b->assign = c.take<int32_t>((size_t)T * n);
-    b->placed = c.take<int32_t>((size_t)T * n);
     b->members = c.take<int32_t>((size_t)T * k1 * kBucketCap);
+    b->dists = c.take<float>((size_t)T * k1 * kBucketCap);
+    b->big = c.take<int32_t>((size_t)T * k1);
     b->more = c.take<int2>((size_t)T * n);
+    b->more_dist = c.take<float>((size_t)T * n);
+    b->lost = c.take<int32_t>((size_t)T * n);
     b->unsure = c.take<int32_t>((size_t)T * n);
     b->list[0] = c.take<int32_t>((size_t)T * n);
     b->list[1] = c.take<int32_t>((size_t)T * n);
-    b->counters = c.take<int32_t>((size_t)T * kBuildCounters);
-    b->dist = c.take<float>((size_t)T * n);
+    b->counters = c.take<int32_t>((size_t)T * kBuildCounters * kCounterStride);
     b->counts = c.take<int32_t>((size_t)T * k1);
     b->fill = c.take<int32_t>((size_t)T * k1);
-    b->free_pre = c.take<int32_t>((size_t)T * (k1 + 1));
-    b->chunk_pre = c.take<int32_t>((size_t)T * ((size_t)ceil_div(n, 256) + 1));
     for (int l = 0; l < HIRA_MAX_LEVELS; ++l) {
         b->slots[l] = nullptr;
         b->cent_t[l] = nullptr;
@@ -830,16 +965,13 @@ static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
 }
 
 template <typename T>
-static int launch_assign_simple(int lpr, dim3 grid, hipStream_t s, const void* x, int n_c,
-                         size_t x_stride, const float* cent, int K, int D, const int32_t* fill,
-                         int bf, const int32_t* list, const int32_t* list_count,
-                         size_t list_stride, int32_t* assign, float* dist,
-                         const AssignCounting& counting) {
-#define HIRA_ASSIGN_CASE(N)                                                                   \
-    case N:                                                                                   \
-        hipLaunchKernelGGL((k_assign_simple<T, N>), grid, dim3(256), 0, s, x, n_c, x_stride,   \
-                           cent, K, D, fill, bf, list, list_count, list_stride, assign, dist, \
-                           counting);                                                          \
+static int launch_assign_simple(const AssignJob& job, const int32_t* fill, int bf, hipStream_t s) {
+    int lpr = 2;
+    while (lpr * Elem<T>::kPerChunk < job.D) lpr <<= 1;
+    const dim3 grid(ceil_div(job.n_c, 4 * (64 / lpr) * kPPG), job.num_trees);
+#define HIRA_ASSIGN_CASE(N)                                                                            \
+    case N:                                                                                            \
+        hipLaunchKernelGGL((k_assign_simple<T, N>), grid, dim3(256), 0, s, fill, bf, job);             \
         break;
     switch (lpr) {
         HIRA_ASSIGN_CASE(2)
@@ -871,10 +1003,12 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
     int K[HIRA_MAX_LEVELS];
     cluster_counts(n, bf, L, K);
 
-    int32_t* const done = w.counters;
-    int32_t* const list_count = w.counters + (size_t)NT;         // (2, T)
-    int32_t* const more_count = w.counters + (size_t)3 * NT;     // (2, T)
-    int32_t* const unsure_count = w.counters + (size_t)5 * NT;
+    const size_t ct = (size_t)NT * kCounterStride;
+    int32_t* const list_count = w.counters;           // (2, T)
+    int32_t* const more_count = w.counters + 2 * ct;  // (2, T)
+    int32_t* const unsure_count = w.counters + 4 * ct;
+    int32_t* const lost_count = w.counters + 5 * ct;
+    int32_t* const big_count = w.counters + 6 * ct;   // (2, T)
     const int KS = assign_ks(t->dtype, D);
     for (int l = 1; l < L; ++l) {
         const void* x = l == 1 ? keys_in : w.cent_t[l - 1];
@@ -886,39 +1020,43 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
         const CentroidTiles tiles = on_mfma ? w.ct : CentroidTiles{nullptr, nullptr, nullptr};
         const long long all_items = (long long)n_c * NT;
         int round = 0;  // of the level, Lloyd and packing together
-        const int items_per_block = 4 * (64 / lpr) * kPPG;
-        const dim3 g_assign(ceil_div(n_c, items_per_block), NT);
-        const dim3 g_items(ceil_div(n_c, 256), NT);
-        const dim3 g_cent(Kl, NT);
+        const int large = large_blocks(Kl);
+        const dim3 g_cent(Kl, NT), g_bucket(large + ceil_div(Kl, kWaves), NT);
 
-        // Trees with fewer items than rows (n_live): every phase walks the list of the items
-        // the tree holds, and the first packing round does too.
+        // Trees with fewer items than rows (n_live): the rounds over all items are over the first
+        // ones of every tree.
         const bool ragged = n_live != nullptr && l == 1;
-        hipLaunchKernelGGL(k_level_init, dim3(min(ceil_div(max(n_c, Kl * bf), 256), 2048), NT),
-                           dim3(256), 0, s, n_c, Kl, bf, D, Kt, ragged ? n_live : nullptr, w.placed,
-                           w.fill, w.slots[l], w.counts, w.counters, tiles, KS);
-        const int32_t* live = nullptr;
-        const int32_t* live_cnt = nullptr;
-        if (ragged) {
-            hipLaunchKernelGGL(k_collect_unplaced, g_items, dim3(256), 0, s, w.placed, n_c,
-                               w.list[0], list_count);
-            live = w.list[0];
-            live_cnt = list_count;
-        }
+        hipLaunchKernelGGL(k_level_init, dim3(min(ceil_div(Kl * bf, 256), 2048), NT), dim3(256), 0, s, n_c, Kl, bf,
+                           D, Kt, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters, tiles, KS);
         hipLaunchKernelGGL((k_init_centroids<T>), g_cent, dim3(64), 0, s, x, n_c, xs, Kl, D,
                            seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, bf,
                            Kt, w.fill, tiles, KS);
         // a round: the assignment (which also puts the items into buckets), then what the round does
         // with every bucket.  A Lloyd round asks for no distances.
         auto buckets = [&]() {
-            return Buckets{w.counts, w.members, w.more, more_count + (size_t)(round & 1) * NT,
-                           more_count + (size_t)((round + 1) & 1) * NT, unsure_count};
+            const int now = round & 1, next = now ^ 1;
+            return Buckets{w.counts, w.members, w.dists, w.big, big_count + now * ct, w.more, more_count + now * ct,
+                           w.more_dist, big_count + next * ct, more_count + next * ct, unsure_count};
         };
-        auto assign_round = [&](const int32_t* list, const int32_t* lcnt, const int32_t* fill, float* dist,
+        auto assign_round = [&](const int32_t* list, const int32_t* lcnt, const int32_t* fill, bool packing,
                                 int32_t* zero, bool only_open, long long expected) -> int {
-            AssignJob job{x, n_c, xs, t->dtype, D, NT, tiles, w.cent_f32, Kl, list, lcnt, w.assign, dist,
-                          AssignCounting{w.counts, w.members, w.more, more_count + (size_t)(round & 1) * NT, zero},
-                          AssignOpen{nullptr, nullptr}, 0, w.unsure, unsure_count};
+            AssignJob job{};
+            job.x = x;
+            job.n_c = n_c;
+            job.n_live = ragged ? n_live : nullptr;
+            job.x_tree_stride = xs;
+            job.dtype = t->dtype;
+            job.D = D;
+            job.num_trees = NT;
+            job.ct = tiles;
+            job.cent = w.cent_f32;
+            job.K = Kl;
+            job.list = list;
+            job.list_count = lcnt;
+            job.counting = AssignCounting{w.counts, w.members, packing ? w.dists : nullptr, w.big,
+                                          big_count + (round & 1) * ct, w.more, more_count + (round & 1) * ct, w.more_dist, w.lost, lost_count, zero};
+            job.unsure = w.unsure;
+            job.unsure_count = unsure_count;
             int rc = HIRA_OK;
             if (on_mfma && only_open) {
                 rc = launch_open_centroids(KS, w.ct, w.fill, bf, Kl, NT, w.open_ids, w.open_count, w.open, s);
@@ -938,32 +1076,30 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
                 job.list = w.unsure;
                 job.list_count = unsure_count;
             }
-            return launch_assign_simple<T>(lpr, g_assign, s, x, n_c, xs, w.cent_f32, Kl, D, fill, bf, job.list,
-                                           job.list_count, (size_t)n_c, w.assign, dist, job.counting);
+            return launch_assign_simple<T>(job, fill, bf, s);
         };
         for (int it = 0; it < niter; ++it, ++round) {
-            const int rc = assign_round(live, live_cnt, ragged ? w.fill : nullptr, nullptr, nullptr, false, all_items);
+            const int rc = assign_round(nullptr, nullptr, ragged ? w.fill : nullptr, false, nullptr, false, all_items);
             if (rc != HIRA_OK) return rc;
-            hipLaunchKernelGGL((k_bucket_mean<T>), g_cent, dim3(kBucketThreads), 0, s, x, xs, n_c, Kl, D, buckets(),
-                               ragged ? w.fill : nullptr, bf, w.cent_f32, Kt, tiles, KS);
+            hipLaunchKernelGGL((k_bucket_mean<T>), g_bucket, dim3(kBucketThreads), 0, s, x, xs, n_c, Kl, D, buckets(),
+                               ragged ? w.fill : nullptr, bf, w.cent_f32, Kt, tiles, KS, large);
         }
-        // capacity packing: round r walks list r % 2 (the first one all items, or the items the
-        // trees hold) and leaves those it could not place on the other list
+        // capacity packing: the first round is over all items, round r over list r % 2; it leaves those
+        // it could not place on the other list
         for (int r = 0; r < pack_rounds; ++r, ++round) {
-            const int32_t* list = r == 0 ? live : w.list[r & 1];
-            const int32_t* lcnt = r == 0 ? live_cnt : list_count + (size_t)(r & 1) * NT;
-            int32_t* next_cnt = list_count + (size_t)((r + 1) & 1) * NT;
+            const int32_t* list = r == 0 ? nullptr : w.list[r & 1];
+            const int32_t* lcnt = r == 0 ? nullptr : list_count + (r & 1) * ct;
+            int32_t* next_cnt = list_count + ((r + 1) & 1) * ct;
             // (from the second round on most blocks are full: the assignment then sees only the
             // centroids with room, side by side; worth its launch from 32 tiles on)
-            const int rc = assign_round(list, lcnt, w.fill, w.dist, next_cnt, r >= 1 && Kl >= 512, all_items >> r);
+            const int rc = assign_round(list, lcnt, w.fill, true, next_cnt, r >= 1 && Kl >= 512, all_items >> r);
             if (rc != HIRA_OK) return rc;
-            hipLaunchKernelGGL(k_bucket_accept, g_cent, dim3(kBucketThreads), 0, s, buckets(), w.dist, n_c, Kl, bf,
-                               w.fill, w.slots[l], w.placed, w.list[(r + 1) & 1], next_cnt, Kt, tiles.n2);
+            hipLaunchKernelGGL(k_bucket_accept, g_bucket, dim3(kBucketThreads), 0, s, buckets(), n_c, Kl, bf,
+                               w.fill, w.slots[l], w.list[(r + 1) & 1], next_cnt, Kt, tiles.n2, large);
         }
-        hipLaunchKernelGGL(k_leftover_count, g_items, dim3(256), 0, s, w.placed, n_c, Kl, bf, w.fill,
-                           w.chunk_pre, w.free_pre, done);
-        hipLaunchKernelGGL(k_leftover_place, g_items, dim3(256), 0, s, n_c, Kl, bf, w.fill,
-                           w.chunk_pre, w.free_pre, w.slots[l], w.placed);
+        hipLaunchKernelGGL(k_leftover, dim3(NT), dim3(kLeftThreads), 0, s, w.list[pack_rounds & 1],
+                           list_count + (pack_rounds & 1) * ct, w.lost, lost_count, n_c, Kl, bf, w.fill,
+                           w.unsure, w.slots[l]);
         // block centre = mean of what is in the block, rounded to the storage type
         hipLaunchKernelGGL((k_block_mean<T>), g_cent, dim3(64), 0, s, x, xs, Kl, D, w.slots[l], bf,
                            lpr, w.cent_f32, w.cent_t[l]);
@@ -1175,30 +1311,24 @@ extern "C" int hira_nearest(const void* x, int32_t dtype, int32_t num_trees, int
     // a row without any usable centre keeps idx -1 and an infinite distance
     fill_i32(idx, (size_t)num_trees * n, -1, s);
     fill_i32(reinterpret_cast<int32_t*>(dist2), (size_t)num_trees * n, 0x7f800000, s);
+    AssignJob job{};
+    job.x = x;
+    job.n_c = n;
+    job.x_tree_stride = (size_t)n;
+    job.dtype = dtype;
+    job.D = dim;
+    job.num_trees = num_trees;
+    job.cent = centers;
+    job.K = m;
+    job.assign = idx;
+    job.dist = dist2;
     if (b.tiles != nullptr) {
         rc = launch_cent_prep(dim, centers, m, num_trees, b.fill, 1, b.tiles, b.n2, s);
-        AssignJob job{};
-        job.x = x;
-        job.n_c = n;
-        job.x_tree_stride = (size_t)n;
-        job.dtype = dtype;
-        job.D = dim;
-        job.num_trees = num_trees;
         job.ct = CentroidTiles{reinterpret_cast<uint4*>(b.tiles), b.n2, nullptr};
-        job.K = m;
-        job.assign = idx;
-        job.dist = dist2;
         if (rc == HIRA_OK) rc = launch_assign_mfma(job, s);
     } else {
-        const int epl = dtype == HIRA_F32 ? 4 : 8;
-        int lpr = 2;
-        while (lpr * epl < dim) lpr <<= 1;
-        const dim3 grid(ceil_div(n, 4 * (64 / lpr) * kPPG), num_trees);
-        rc = dtype == HIRA_F32
-                 ? launch_assign_simple<float>(lpr, grid, s, x, n, (size_t)n, centers, m, dim, b.fill, 1,
-                                        nullptr, nullptr, 0, idx, dist2, AssignCounting{})
-                 : launch_assign_simple<bf16_t>(lpr, grid, s, x, n, (size_t)n, centers, m, dim, b.fill, 1,
-                                         nullptr, nullptr, 0, idx, dist2, AssignCounting{});
+        rc = dtype == HIRA_F32 ? launch_assign_simple<float>(job, b.fill, 1, s)
+                               : launch_assign_simple<bf16_t>(job, b.fill, 1, s);
     }
     if (rc != HIRA_OK) return rc;
     HIRA_CHECK_LAUNCH("nearest-centre kernel");

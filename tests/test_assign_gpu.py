@@ -76,3 +76,15 @@ def test_blocks_equal_exact_arithmetic(dtype, trees, n, d, bf, values, gpu_devic
         want = _blocks(torch.from_numpy(x[t]).to(gpu_device).double(), K, bf, 5 + 7919, t, 8)
         got = index.perm[t, :K * bf].cpu().numpy().reshape(K, bf)
         np.testing.assert_array_equal(got, want, err_msg=f"tree {t}")
+
+
+@pytest.mark.parametrize("dtype,n,d,bf", [(torch.bfloat16, 3000, 128, 8), (torch.float32, 700, 36, 16)])
+def test_keys_that_are_no_numbers_keep_a_slot(dtype, n, d, bf, gpu_device):
+    from hira_amd.indexer.hip import HIPIndexer
+
+    x = torch.randn(1, 2, n, d, generator=torch.Generator().manual_seed(n))
+    x[:, :, 5::97, 3] = float("nan")
+    index = HIPIndexer(2, 1, bf, seed=2).build(x.to(dtype), x.to(dtype))
+    perm = index.perm[:, :-(-n // bf) * bf].cpu().numpy()
+    for t in range(2):
+        assert sorted(perm[t][perm[t] >= 0].tolist()) == list(range(n))
