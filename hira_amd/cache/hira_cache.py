@@ -113,6 +113,13 @@ class HiraCacheLayer(CacheLayerMixin):
     def queued_values(self):
         return self._queue_v.narrow(2, 0, self.queued_len)
 
+    def _whole_rows(self, x, m: int, width: int, like) -> bool:
+        """Are x's rows (B, H_kv, m, width) -- or (H_kv, m, width) of one sequence --, one behind the
+        other, on `like`'s device and 16-byte aligned, as the launches that copy rows take them?"""
+        return x.ndim >= 3 and x.shape[-3:] == (self.H_kv, m, width) and \
+            x.numel() == self.batch * self.H_kv * m * width and \
+            x.get_device() == like.get_device() and x.is_contiguous() and x.data_ptr() % 16 == 0
+
     def _enqueue(self, key_states, value_states):
         m = key_states.shape[-2]
         if self.queued_len + m > self._queue_k.shape[-2]:  # (a step of many tokens)
@@ -123,8 +130,8 @@ class HiraCacheLayer(CacheLayerMixin):
         k, v = self._queue_k, self._queue_v
         if self._queue_type is not None and k.is_cuda and \
                 key_states.dtype is k.dtype and value_states.dtype is v.dtype and \
-                key_states.get_device() == value_states.get_device() == k.get_device() and \
-                key_states.is_contiguous() and value_states.is_contiguous():
+                self._whole_rows(key_states, m, self.dim, k) and \
+                self._whole_rows(value_states, m, self.vdim, v):
             # one launch for both
             _lib.check(_lib.lib().hira_enqueue(
                 k.data_ptr(), v.data_ptr(), self._queue_type, self.batch * self.H_kv, k.shape[2],
@@ -199,7 +206,8 @@ class HiraCacheLayer(CacheLayerMixin):
         k4 = key_states if key_states.ndim == 4 else key_states[None]
         # (in the index's storage dtype: the threshold kernel reads samples and queries alike)
         store = getattr(self.indexer, "dtype", None) or k4.dtype
-        if k4.is_cuda and k4.dtype is store and k4.is_contiguous() and self._queue_type is not None:
+        if k4.is_cuda and k4.dtype is store and self._queue_type is not None and \
+                self._whole_rows(k4, n, self.dim, self._queue_k):
             # the positions travel with the launches: nothing waits for the build
             self.samples = torch.empty((k4.shape[0] * k4.shape[1], s, self.dim), dtype=store, device=k4.device)
             self._replace_rows(self.samples, k4, n, n, range(s), pick.tolist())
@@ -247,14 +255,15 @@ class HiraCacheLayer(CacheLayerMixin):
             # behind the other and the heads evenly spaced, as the queue's and a model's do.)
             if src.dtype is not smp.dtype or src.get_device() != smp.get_device():
                 src = src.to(device=smp.device, dtype=smp.dtype)
+            b, h = src.shape[:2]
+            step = src.stride(1) if h > 1 else src.stride(0) if b > 1 else m * self.dim
             if src.stride(3) != 1 or (m > 1 and src.stride(2) != self.dim) or \
-                    src.stride(1) % self.dim or (src.shape[0] > 1 and
-                                                 src.stride(0) != src.stride(1) * src.shape[1]):
-                src = src.contiguous()
-            if src.shape[1] == 1 and src.shape[0] == 1:
-                stride = m
-            else:
-                stride = (src.stride(1) if src.shape[1] > 1 else src.stride(0)) // self.dim
+                    step % self.dim or step < m * self.dim or (b > 1 and src.stride(0) != step * h) or \
+                    src.data_ptr() % 16:
+                # (clone: contiguous() would hand back a misaligned tensor as it is)
+                src = src.clone(memory_format=torch.contiguous_format)
+                step = m * self.dim
+            stride = step // self.dim
             self._replace_rows(smp, src, m, stride, last.keys(), last.values())
             return
         rows = src.reshape(-1, m, self.dim).to(smp.dtype)

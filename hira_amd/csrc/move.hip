@@ -101,6 +101,10 @@ static int row_chunks(int32_t dtype, int32_t width) {  // 16-byte chunks of a ro
     return width >= 0 && bytes % 16 == 0 ? bytes / 16 : -1;
 }
 
+static bool aligned16(const void* a, const void* b) {  // (the kernels move 16 bytes a lane)
+    return (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
+}
+
 /* see include/hira_hip.h */
 extern "C" int hira_enqueue(void* queue_keys, void* queue_values, int32_t dtype, int32_t num_trees,
                             int32_t cap, int32_t at, int32_t m, int32_t dim, int32_t vdim,
@@ -113,6 +117,8 @@ extern "C" int hira_enqueue(void* queue_keys, void* queue_values, int32_t dtype,
                    "hira_enqueue: rows %d .. %d of %d", at, at + m, cap);
     HIRA_CHECK_ARG(queue_keys && new_keys && (vc == 0 || (queue_values && new_values)),
                    "hira_enqueue: null argument");
+    HIRA_CHECK_ARG(aligned16(queue_keys, new_keys) && (vc == 0 || aligned16(queue_values, new_values)),
+                   "hira_enqueue: rows must be 16-byte aligned");
     const int64_t total = (int64_t)num_trees * m * (kc + vc);
     HIRA_CHECK_ARG(total < (int64_t)1 << 31, "hira_enqueue: too many rows at once");
     if (total == 0) return HIRA_OK;
@@ -149,6 +155,7 @@ extern "C" int hira_replace_rows(void* rows, int32_t dtype, int32_t dim, int32_t
     HIRA_CHECK_ARG(chunks >= 1, "hira_replace_rows: dim %d: rows must be a multiple of 16 bytes", dim);
     HIRA_CHECK_ARG(num_trees >= 1 && n >= 0 && from_rows <= from_stride, "hira_replace_rows: bad counts");
     HIRA_CHECK_ARG(n == 0 || (rows && from && slot_host && from_host), "hira_replace_rows: null argument");
+    HIRA_CHECK_ARG(n == 0 || aligned16(rows, from), "hira_replace_rows: rows must be 16-byte aligned");
     for (int i = 0; i < n; ++i)
         HIRA_CHECK_ARG(slot_host[i] >= 0 && slot_host[i] < rows_per_tree && from_host[i] >= 0 &&
                            from_host[i] < from_rows,

@@ -766,7 +766,8 @@ class HIPIndexer(BaseIndexer):
 
     def _rows(self, x: torch.Tensor, t: int, m: int, width: int) -> torch.Tensor:
         """(T, m, width) rows, contiguous, in the storage type and on the index's device."""
-        if x.dtype is self.dtype and x.get_device() == self.keys_buf.get_device() and x.is_contiguous():
+        if x.dtype is self.dtype and x.get_device() == self.keys_buf.get_device() and \
+                x.is_contiguous() and x.numel() == t * m * width:
             return x
         return x.to(device=self.device, dtype=self.dtype).reshape(t, m, width).contiguous()
 

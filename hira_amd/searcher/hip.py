@@ -354,6 +354,9 @@ class HIPSearcher(BaseSearcher):
             qk = self._queue_rows(queue_keys, indexer, c.dev, indexer.dim)
             qv = self._queue_rows(queue_values, indexer, c.dev, indexer.vdim)
             rows = qk.numel() // (indexer.num_trees * indexer.dim)
+            if qv.numel() != rows * indexer.num_trees * indexer.vdim:
+                raise ValueError(f"queue: keys {tuple(queue_keys.shape)} and values "
+                                 f"{tuple(queue_values.shape)} hold different numbers of rows")
             qu = c.queue
             qu.keys, qu.values, qu.len, qu.cap = qk.data_ptr(), qv.data_ptr(), rows, rows
             keep = keep + (qk, qv)

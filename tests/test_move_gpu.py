@@ -86,3 +86,71 @@ def test_output_in_bf16_is_the_rounded_fp32_output(dtype, d, bf, group, gpu_devi
     plan.run(q, tau, a)
     plan.run(q, tau, b)
     assert bool((a != 0).any()) and torch.equal(b, a.to(torch.bfloat16))
+
+
+def _layer(update_every, prompt):
+    from hira_amd.cache.hira_cache import HiraCacheLayer
+    from hira_amd.cache.hira_config import DeviceMode
+
+    layer = HiraCacheLayer(DeviceMode.CUDA_ONLY, update_every,
+                           {"num_levels": 2, "max_iterations": 1, "branching_factor": 32}, {},
+                           {"method": "sample_mean_topk", "sample_size": 100, "topk": 4})
+    layer.update(prompt, prompt)
+    return layer
+
+
+def _misaligned(x):
+    """The same values, contiguous, one element past a 16-byte boundary."""
+    y = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)[1:].view(x.shape)
+    y.copy_(x)
+    assert y.is_contiguous() and y.data_ptr() % 16
+    return y
+
+
+@pytest.mark.parametrize("update_every,m", [(8, 3), (1, 1), (4, 64)])
+@pytest.mark.parametrize("form", [_misaligned, lambda x: x.transpose(1, 2).contiguous().transpose(1, 2),
+                                  lambda x: x[:, :1].contiguous().expand(x.shape)])
+def test_cache_layer_takes_rows_however_they_lie(form, update_every, m, gpu_device):
+    """Queue, sample and index are the same from misaligned, strided and expanded (head stride 0)
+    tensors as from plain ones."""
+    prompt = torch.randn(1, 2, 500, 64, device="cuda").to(torch.bfloat16)
+    tokens = torch.randn(6, 1, 2, m, 64, device="cuda").to(torch.bfloat16)
+    a = _layer(update_every, prompt.clone())
+    b = _layer(update_every, _misaligned(prompt))
+    assert torch.equal(a.samples, b.samples)
+    for t in tokens:
+        x = form(t)
+        a.update(x.clone(memory_format=torch.contiguous_format), -x.clone(memory_format=torch.contiguous_format), 0)
+        b.update(x, form(-t), 0)
+        assert torch.equal(a.queued_keys, b.queued_keys) and torch.equal(a.queued_values, b.queued_values)
+        assert torch.equal(a.samples, b.samples)
+    a.indexer.sync_sizes(), b.indexer.sync_sizes()
+    n = a.indexer.size[0]
+    assert torch.equal(a.indexer.perm[:, :n], b.indexer.perm[:, :n])
+    assert torch.equal(a.indexer.values_buf[:, :n], b.indexer.values_buf[:, :n])
+
+
+def test_rows_of_the_wrong_shape_are_refused(gpu_device):
+    """Too few heads or columns raise on the host, as a copy of them would; nothing is launched."""
+    from hira_amd import _lib
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    prompt = torch.randn(1, 2, 500, 64, device="cuda").to(torch.bfloat16)
+    row = prompt[:, :, :1].contiguous()
+    for every in (8, 1):
+        layer = _layer(every, prompt)
+        with pytest.raises((RuntimeError, ValueError)):
+            layer.update(row, row[..., :32].contiguous(), 0)
+        with pytest.raises((RuntimeError, ValueError)):
+            layer.update(row[..., :32].contiguous(), row, 0)
+    index = HIPIndexer(2, 1, 32).build(prompt, prompt)
+    with pytest.raises((RuntimeError, ValueError)):
+        index.update(row, row[..., :32].contiguous())
+    q, tau = torch.randn(2, 64, device="cuda").to(torch.bfloat16), torch.zeros(2, device="cuda")
+    with pytest.raises((RuntimeError, ValueError)):
+        HIPSearcher().search_attention(q, tau, index, queue_keys=prompt[:, :, :8], queue_values=prompt[:, :, :7])
+    odd = _misaligned(row)
+    with pytest.raises(ValueError):
+        _lib.check(_lib.lib().hira_enqueue(prompt.data_ptr(), prompt.data_ptr(), _lib.HIRA_BF16, 2, 500, 0, 1, 64, 64,
+                                           odd.data_ptr(), row.data_ptr(), _lib.current_stream(row.device)))
