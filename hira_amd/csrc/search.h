@@ -19,7 +19,6 @@ struct SearchParams {
     int32_t size[HIRA_MAX_LEVELS];
     int32_t cap[HIRA_MAX_LEVELS];
     int32_t num_levels, bf, dim, vdim;
-    uint32_t bf_magic;  // ceil(2^32 / bf): n / bf = the high word of n * bf_magic (bf > 1, n < 2^26)
     int32_t layout;  // of the centers: HIRA_ROW_MAJOR or HIRA_TILE16
     int32_t key_layout;  // of the keys
     const int8_t* keys8;  // HIRA_TILE16_Q8: the 8-bit shadow, its steps and error bounds
@@ -59,8 +58,9 @@ struct SearchParams {
     int32_t num_parts;  // P = gridDim.x
     int32_t gmax_state; // MFMA kernel: heads per pass its LDS state rows are sized for
     void* attn_out;     // (H_q, Dv): written by the kernel itself when `done` is set
-    int32_t out_bf16;   // its type: bf16, else fp32
     int32_t* done;      // (T, passes) arrival counters, zero between launches; NULL: no fold
+    int32_t out_bf16;   // attn_out's type: bf16, else fp32
+    uint32_t bf_magic;  // ceil(2^32 / bf): n / bf = the high word of n * bf_magic (bf > 1, n < 2^26)
     unsigned long long* stats;
 };
 
