@@ -19,20 +19,14 @@
 // indexer/cpu.py:286-309 / indexer/cuda.py:114-198, against the ROUNDED centres and
 // nudged up by a few ulp so that rounding never makes a ball too small.
 #include "assign.h"
-#include "rows.h"
+#include "cluster.h"
+#include "small_levels.h"
 
 namespace hira {
 
 // ------------------------------------------------------------------------------------
 // small helpers
 // ------------------------------------------------------------------------------------
-__device__ __forceinline__ uint64_t mix64(uint64_t z) {
-    z += 0x9E3779B97F4A7C15ull;
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    return z ^ (z >> 31);
-}
-
 // what the phases of a level count, per tree: items on the two lists, items behind the buckets (of
 // this round, of the next), items the approximate assignment leaves, items without a centroid, large
 // buckets (of this round, of the next)
@@ -92,13 +86,10 @@ __global__ __launch_bounds__(64) void k_init_centroids(const void* x, int n_c, s
                                                        const int32_t* fill, CentroidTiles ct, int KS) {
     __shared__ float s_c[256];
     const int k = blockIdx.x, t = blockIdx.y;
-    const uint64_t h = mix64(seed ^ mix64((uint64_t)t * 0x100000001b3ull + (uint64_t)k));
-    const double u = (double)(h >> 11) * (1.0 / 9007199254740992.0);
     const int n_t = n_live ? max(min(n_live[t], n_c), 1) : n_c;
     // (a tree with fewer items uses the first K_t = ceil(n_t / bf) centroids only)
     const int K_t = n_live ? min(max((n_t + bf - 1) / bf, 1), K) : K;
-    long long idx = (long long)(((double)min(k, K_t - 1) + u) * (double)n_t / (double)K_t);
-    if (idx >= n_t) idx = n_t - 1;
+    const long long idx = first_centroid(seed, t, k, n_t, K_t);
     const size_t src = ((size_t)t * x_tree_stride + (size_t)idx) * D;
     float* dst = cent + ((size_t)t * K + k) * D;
     for (int j = threadIdx.x; j < D; j += blockDim.x) {
@@ -266,29 +257,6 @@ __device__ __forceinline__ int pow2_at_least(int n) {
     return p;
 }
 
-// rank of this lane's value among those of lanes 0 .. m - 1 (distinct; the other lanes hold the
-// largest number; m uniform in the wave).  Lane numbers are constants: a step is three or four
-// instructions.
-template <typename Key>
-__device__ __forceinline__ int wave_rank(Key mine, int m) {
-    int rank = 0;
-#pragma unroll
-    for (int j0 = 0; j0 < 64; j0 += 8) {
-        if (j0 >= m) break;
-#pragma unroll
-        for (int j = j0; j < j0 + 8; ++j) {
-            Key o;
-            if constexpr (sizeof(Key) == 8)
-                o = ((Key)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mine >> 32), j) << 32) |
-                    (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, j);
-            else
-                o = (Key)__builtin_amdgcn_readlane((int)mine, j);
-            rank += o < mine ? 1 : 0;
-        }
-    }
-    return rank;
-}
-
 // what the wave, or the workgroup, that has read the count of its bucket does for the round after it
 // (behind a barrier: the count is read through the scalar cache, and only the wait there keeps this
 // store from overtaking it; a bucket's other reader finds a large count, or none, and leaves it)
@@ -320,7 +288,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
     const int32_t* fill, int bf, float* cent, int Kt, const CentroidTiles ct, int KS, int large) {
     constexpr int EPL = Elem<T>::kPerChunk;
     constexpr int kPart = kBucketThreads * EPL;  // (R, D) partial sums, R * D <= 256 * EPL
-    constexpr int kPiece = 64 * EPL;             // a quarter of them
+    constexpr int kPiece = kWaveMeanPiece<T>;    // a quarter of them
     // one bucket: partial sums, ids in order or their bit map, counts of the bit map's stretches;
     // or, a wave each: a quarter of the partial sums
     __shared__ __attribute__((aligned(16))) float s_lds[kPart + kMeanMap + kBucketThreads];
@@ -342,65 +310,9 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
         if (lane < m) s_ids[wave][rank] = id;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (lane == 0) reset_count(bk, t, k, K);
-        float acc[4][EPL];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int q = 0; q < EPL; ++q) acc[i][q] = 0.0f;
-        for (int e0 = 0; e0 < m; e0 += 2 * R) {  // uniform
-            uint4 raw[2][4];
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int v = lane + 64 * i, e = e0 + h * R + v / CPR;
-                    raw[h][i] = make_uint4(0, 0, 0, 0);
-                    if (v < R * CPR && e < m)
-                        raw[h][i] = load_chunk<T>(x, ((size_t)t * x_tree_stride + s_ids[wave][e]) * D, v % CPR);
-                }
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {  // (a row that is none adds zeros)
-                    float f[EPL];
-                    unpack<T>(raw[h][i], f);
-#pragma unroll
-                    for (int q = 0; q < EPL; ++q) acc[i][q] += f[q];
-                }
-        }
-        // the partial sums as one row of R * D numbers pass through LDS a quarter at a time; a lane
-        // adds up its columns
         float* piece = s_lds + wave * kPiece;
-        const int rows = min(R, m);
-        float sum[8];
-        int at[8];  // where the column's next partial sum lies
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            sum[u] = 0.0f;
-            at[u] = lane + 64 * u;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int q = 0; q < EPL; ++q) piece[lane * EPL + q] = acc[i][q];
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            const int end = min((i + 1) * kPiece, rows * D);
-#pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (64 * u < D)  // uniform
-                    for (; at[u] < end; at[u] += D) sum[u] += piece[at[u] - i * kPiece];
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int j = lane + 64 * u;
-            if (j < D) {
-                const float v = sum[u] / (float)m;
-                cent[((size_t)t * K + k) * D + j] = v;
-                piece[j] = v;
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        wave_mean<T, 2>(x, (size_t)t * x_tree_stride, [&](int e) { return s_ids[wave][e]; }, m, D, piece,
+                        cent + ((size_t)t * K + k) * D);
         if (ct.tiles != nullptr) emit_centroid(piece, D, KS, Kt, t, k, usable(k), ct);
         return;
     }
@@ -516,51 +428,14 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
     }
 }
 
-// block centre = mean of the items in the bf slots of the block, stored in fp32 and rounded to the
-// storage type.  One wave per block: `lpr` lanes (a power of two) hold a row in 16-byte chunks,
-// the 64 / lpr lane groups take every (64 / lpr)-th slot, and their sums are added pairwise in a
-// fixed order.  An empty block keeps its value.
+// a wave per block (wave_block_mean)
 template <typename T>
 __global__ __launch_bounds__(64) void k_block_mean(const void* x, size_t x_tree_stride, int K,
                                                    int D, const int32_t* slots, int bf, int lpr,
                                                    float* cent, void* out_t) {
-    constexpr int EPL = Elem<T>::kPerChunk;
     const int k = blockIdx.x, t = blockIdx.y;
-    const int lane = threadIdx.x;
-    const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
-    const bool chunk_ok = ch * EPL < D;
-    const int32_t* lst = slots + ((size_t)t * K + k) * bf;
-    float acc[EPL];
-#pragma unroll
-    for (int q = 0; q < EPL; ++q) acc[q] = 0.0f;
-    int cnt = 0;
-    for (int e = rg; e < bf; e += groups) {
-        const int it = lst[e];
-        if (it < 0) continue;
-        ++cnt;
-        if (!chunk_ok) continue;
-        float f[EPL];
-        unpack<T>(load_chunk<T>(x, ((size_t)t * x_tree_stride + it) * D, ch), f);
-#pragma unroll
-        for (int q = 0; q < EPL; ++q) acc[q] += f[q];
-    }
-    for (int off = lpr; off < 64; off <<= 1) {
-        cnt += __shfl_xor(cnt, off, 64);
-#pragma unroll
-        for (int q = 0; q < EPL; ++q) acc[q] += __shfl_xor(acc[q], off, 64);
-    }
-    if (rg == 0 && chunk_ok) {
-#pragma unroll
-        for (int q = 0; q < EPL; ++q) {
-            const size_t o = ((size_t)t * K + k) * D + ch * EPL + q;
-            float v = cent[o];
-            if (cnt > 0) {
-                v = acc[q] / (float)cnt;
-                cent[o] = v;
-            }
-            store_elem<T>(out_t, o, v);
-        }
-    }
+    wave_block_mean<T>(x, (size_t)t * x_tree_stride, D, slots + ((size_t)t * K + k) * bf, bf, lpr,
+                       ((size_t)t * K + k) * D, cent, out_t);
 }
 
 // ------------------------------------------------------------------------------------
@@ -918,6 +793,17 @@ static void cluster_counts(int n, int bf, int L, int* K) {
     for (int l = 1; l < L; ++l) K[l] = K[l - 1] <= 0 ? 0 : (ceil_div(K[l - 1], bf) > 0 ? ceil_div(K[l - 1], bf) : 1);
 }
 
+// Whether a workgroup a tree takes this level, and with it all above (small_levels.hip).  It spends on a
+// round what its items times its centroids take one compute unit, the launches what launches take.  Trees x
+// items x centroids, launches / one workgroup a tree: 8 x 512 x 16 (128 columns) 139 / 101 us, 8 x 512 x 32
+// 135 / 120, 8 x 1024 x 16 183 / 153, 64 x 512 x 32 168 / 130, 8 x 1024 x 32 163 / 164; a wave goes through
+// the centroids beyond its first two one after the other: 8 x 250 x 63 126 / 138, 2 x 400 x 40 (256 columns)
+// 136 / 167.
+static bool level_is_small(const HiraTree* t, int n_c, int K) {
+    return assign_exact_on_mfma(t->dtype, t->dim) && n_c <= kSmallItems && K <= kSmallCentroids &&
+           n_c * K <= (t->dim <= 128 ? 16384 : 8192);
+}
+
 static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
     const int L = t->num_levels, T = t->num_trees, D = t->dim, bf = t->bf;
     const size_t esize = t->dtype == HIRA_F32 ? 4 : 2;
@@ -1011,6 +897,28 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
     int32_t* const big_count = w.counters + 6 * ct;   // (2, T)
     const int KS = assign_ks(t->dtype, D);
     for (int l = 1; l < L; ++l) {
+        if (level_is_small(t, K[l - 1], K[l]) && n_live == nullptr) {  // this one and all above it in one launch
+            SmallLevels p{};
+            p.x = l == 1 ? keys_in : w.cent_t[l - 1];
+            p.first = l;
+            p.last = L;
+            for (int i = l - 1; i < L; ++i) {
+                p.K[i] = K[i];
+                p.Kt[i] = assign_tiles(K[i]);
+                p.slots[i] = w.slots[i];
+                p.cent_t[i] = w.cent_t[i];
+            }
+            p.cent = w.cent_f32;
+            p.ct = w.ct;
+            p.seed = seed;
+            p.niter = niter;
+            p.pack_rounds = pack_rounds;
+            p.bf = bf;
+            p.lpr = lpr;
+            if (const int rc = launch_small_levels(p, D, NT, s)) return rc;
+            HIRA_CHECK_LAUNCH("build, small levels");
+            break;
+        }
         const void* x = l == 1 ? keys_in : w.cent_t[l - 1];
         const int n_c = K[l - 1];
         const size_t xs = (size_t)n_c;  // rows per tree in x

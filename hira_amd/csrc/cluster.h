@@ -1,0 +1,167 @@
+// What the kernels of the index build share where a level is clustered: the per-bucket kernels of
+// build.hip and the one that takes whole small levels (small_levels.hip).  Both have to come to the
+// same numbers, bit for bit, whichever of them a level goes through.
+#pragma once
+
+#include "rows.h"
+
+namespace hira {
+
+__device__ __forceinline__ uint64_t mix64(uint64_t z) {
+    z += 0x9E3779B97F4A7C15ull;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
+
+// the item that centroid k of tree t starts from: floor((k + u) * n_t / K_t), u in [0, 1) from the seed;
+// a tree uses the first K_t centroids, the others start from an item of the last one's
+__device__ __forceinline__ long long first_centroid(uint64_t seed, int t, int k, int n_t, int K_t) {
+    const uint64_t h = mix64(seed ^ mix64((uint64_t)t * 0x100000001b3ull + (uint64_t)k));
+    const double u = (double)(h >> 11) * (1.0 / 9007199254740992.0);
+    const long long idx = (long long)(((double)min(k, K_t - 1) + u) * (double)n_t / (double)K_t);
+    return idx >= n_t ? n_t - 1 : idx;
+}
+
+// rank of this lane's value among those of lanes 0 .. m - 1 (distinct; the other lanes hold the
+// largest number; m uniform in the wave).  Lane numbers are constants: a step is three or four
+// instructions.
+template <typename Key>
+__device__ __forceinline__ int wave_rank(Key mine, int m) {
+    int rank = 0;
+#pragma unroll
+    for (int j0 = 0; j0 < 64; j0 += 8) {
+        if (j0 >= m) break;
+#pragma unroll
+        for (int j = j0; j < j0 + 8; ++j) {
+            Key o;
+            if constexpr (sizeof(Key) == 8)
+                o = ((Key)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(mine >> 32), j) << 32) |
+                    (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine, j);
+            else
+                o = (Key)__builtin_amdgcn_readlane((int)mine, j);
+            rank += o < mine ? 1 : 0;
+        }
+    }
+    return rank;
+}
+
+// Mean of the m > 0 rows row0 + ids(e) of x, by one wave: row e is summed by row group e % R, the R sums
+// added in order (a row is CPR = D / EPL threads of 16 bytes, R = 256 / CPR rows at a time: a wave
+// stands for 256 threads).  H steps of R rows are in flight.  piece: kWaveMeanPiece numbers of LDS of
+// the wave's own, the mean's D numbers lie there at the end; cent_row: where they go.
+template <typename T>
+constexpr int kWaveMeanPiece = 64 * Elem<T>::kPerChunk;
+
+template <typename T, int H, typename Ids>
+__device__ __forceinline__ void wave_mean(const void* x, size_t row0, Ids ids, int m, int D, float* piece,
+                                          float* cent_row) {
+    constexpr int EPL = Elem<T>::kPerChunk;
+    constexpr int kPiece = kWaveMeanPiece<T>;
+    const int lane = threadIdx.x & 63;
+    const int CPR = D / EPL, R = 256 / CPR;
+    float acc[4][EPL];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < EPL; ++q) acc[i][q] = 0.0f;
+    for (int e0 = 0; e0 < m; e0 += H * R) {  // uniform
+        uint4 raw[H][4];
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int v = lane + 64 * i, e = e0 + h * R + v / CPR;
+                raw[h][i] = make_uint4(0, 0, 0, 0);
+                if (v < R * CPR && e < m)
+                    raw[h][i] = load_chunk<T>(x, (row0 + ids(e)) * D, v % CPR);
+            }
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {  // (a row that is none adds zeros)
+                float f[EPL];
+                unpack<T>(raw[h][i], f);
+#pragma unroll
+                for (int q = 0; q < EPL; ++q) acc[i][q] += f[q];
+            }
+    }
+    // the partial sums as one row of R * D numbers pass through LDS a quarter at a time; a lane
+    // adds up its columns
+    const int rows = min(R, m);
+    float sum[8];
+    int at[8];  // where the column's next partial sum lies
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        sum[u] = 0.0f;
+        at[u] = lane + 64 * u;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int q = 0; q < EPL; ++q) piece[lane * EPL + q] = acc[i][q];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int end = min((i + 1) * kPiece, rows * D);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (64 * u < D)  // uniform
+                for (; at[u] < end; at[u] += D) sum[u] += piece[at[u] - i * kPiece];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int j = lane + 64 * u;
+        if (j < D) {
+            const float v = sum[u] / (float)m;
+            cent_row[j] = v;
+            piece[j] = v;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// block centre = mean of the items in the bf slots of the block, stored in fp32 and rounded to the
+// storage type.  One wave: `lpr` lanes (a power of two) hold a row in 16-byte chunks,
+// the 64 / lpr lane groups take every (64 / lpr)-th slot, and their sums are added pairwise in a
+// fixed order.  An empty block keeps its value.
+template <typename T>
+__device__ __forceinline__ void wave_block_mean(const void* x, size_t row0, int D, const int32_t* slots, int bf,
+                                                int lpr, size_t out, float* cent, void* out_t) {
+    constexpr int EPL = Elem<T>::kPerChunk;
+    const int lane = threadIdx.x & 63;
+    const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
+    const bool chunk_ok = ch * EPL < D;
+    float acc[EPL];
+#pragma unroll
+    for (int q = 0; q < EPL; ++q) acc[q] = 0.0f;
+    int cnt = 0;
+    for (int e = rg; e < bf; e += groups) {
+        const int it = slots[e];
+        if (it < 0) continue;
+        ++cnt;
+        if (!chunk_ok) continue;
+        float f[EPL];
+        unpack<T>(load_chunk<T>(x, (row0 + it) * D, ch), f);
+#pragma unroll
+        for (int q = 0; q < EPL; ++q) acc[q] += f[q];
+    }
+    for (int off = lpr; off < 64; off <<= 1) {
+        cnt += __shfl_xor(cnt, off, 64);
+#pragma unroll
+        for (int q = 0; q < EPL; ++q) acc[q] += __shfl_xor(acc[q], off, 64);
+    }
+    if (rg == 0 && chunk_ok) {
+#pragma unroll
+        for (int q = 0; q < EPL; ++q) {
+            const size_t o = out + ch * EPL + q;
+            float v = cent[o];
+            if (cnt > 0) {
+                v = acc[q] / (float)cnt;
+                cent[o] = v;
+            }
+            store_elem<T>(out_t, o, v);
+        }
+    }
+}
+
+}  // namespace hira
