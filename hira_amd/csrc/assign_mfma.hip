@@ -474,17 +474,6 @@ __device__ __forceinline__ float from_ordered(uint32_t u) {
     return __uint_as_float(u ^ ((u >> 31) ? 0x80000000u : 0xffffffffu));
 }
 
-// sum over each aligned group of `lpr` lanes, in the order of group_sum<lpr>
-__device__ __forceinline__ float group_sum_of(float v, int lpr) {
-    if (lpr >= 2) v += dpp_move<0xB1>(v);
-    if (lpr >= 4) v += dpp_move<0x4E>(v);
-    if (lpr >= 8) v += dpp_move<0x141>(v);
-    if (lpr >= 16) v += dpp_move<0x140>(v);
-    if (lpr >= 32) v += __shfl_xor(v, 16, 64);
-    if (lpr >= 64) v += __shfl_xor(v, 32, 64);
-    return v;
-}
-
 constexpr int kApproxPairs = 512;  // (item, candidate) pairs of a wave: 64 items, at most eight each
 
 template <typename T, int KS, int RI, bool LISTED, bool EXACT_MFMA>

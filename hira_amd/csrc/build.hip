@@ -37,6 +37,13 @@ __global__ void k_fill_i32(int32_t* p, size_t n, int32_t v) {
     if (i < n) p[i] = v;
 }
 
+// Kernels with a wave per node: four nodes a workgroup (a workgroup of one wave costs its dispatch).
+constexpr int kNodeThreads = 256;
+static dim3 node_grid(int nodes, int trees) { return dim3((nodes + kNodeThreads / 64 - 1) / (kNodeThreads / 64), trees); }
+__device__ __forceinline__ int node_of_wave() {
+    return __builtin_amdgcn_readfirstlane(blockIdx.x * (kNodeThreads / 64) + (threadIdx.x >> 6));
+}
+
 // ------------------------------------------------------------------------------------
 // 0. what a level starts from, in one launch: empty blocks, zero counters; the centroid columns that
 //    pad the last stage of operand tiles are zeros that take no items.
@@ -80,25 +87,27 @@ __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_
 //    ct.tiles != NULL: the centroid also goes into its operand tile (fill: the centroids that
 //    count as full from the start take no items)
 template <typename T>
-__global__ __launch_bounds__(64) void k_init_centroids(const void* x, int n_c, size_t x_tree_stride,
+__global__ __launch_bounds__(kNodeThreads) void k_init_centroids(const void* x, int n_c, size_t x_tree_stride,
                                                        int K, int D, uint64_t seed, float* cent,
                                                        const int32_t* n_live, int bf, int Kt,
                                                        const int32_t* fill, CentroidTiles ct, int KS) {
-    __shared__ float s_c[256];
-    const int k = blockIdx.x, t = blockIdx.y;
+    __shared__ float s_all[kNodeThreads / 64][256];
+    const int k = node_of_wave(), t = blockIdx.y, lane = threadIdx.x & 63;
+    float* s_c = s_all[threadIdx.x >> 6];
+    if (k >= K) return;  // (the whole wave)
     const int n_t = n_live ? max(min(n_live[t], n_c), 1) : n_c;
     // (a tree with fewer items uses the first K_t = ceil(n_t / bf) centroids only)
     const int K_t = n_live ? min(max((n_t + bf - 1) / bf, 1), K) : K;
     const long long idx = first_centroid(seed, t, k, n_t, K_t);
     const size_t src = ((size_t)t * x_tree_stride + (size_t)idx) * D;
     float* dst = cent + ((size_t)t * K + k) * D;
-    for (int j = threadIdx.x; j < D; j += blockDim.x) {
+    for (int j = lane; j < D; j += 64) {
         const float v = load_elem<T>(x, src + j);
         dst[j] = v;
         if (ct.tiles != nullptr) s_c[j] = v;  // (tiles are for D <= 256)
     }
     if (ct.tiles != nullptr) {
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         emit_centroid(s_c, D, KS, Kt, t, k, fill[(size_t)t * K + k] < bf, ct);
     }
 }
@@ -428,13 +437,15 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
     }
 }
 
-// a wave per block (wave_block_mean)
+// A wave per block (wave_block_mean).  Bound by the gather of the rows: 8 x 131072 rows of 256
+// bytes 74 -> 60 us
 template <typename T>
-__global__ __launch_bounds__(64) void k_block_mean(const void* x, size_t x_tree_stride, int K,
-                                                   int D, const int32_t* slots, int bf, int lpr,
-                                                   float* cent, void* out_t) {
-    const int k = blockIdx.x, t = blockIdx.y;
-    wave_block_mean<T>(x, (size_t)t * x_tree_stride, D, slots + ((size_t)t * K + k) * bf, bf, lpr,
+__global__ __launch_bounds__(kNodeThreads) void k_block_mean(const void* x, size_t x_tree_stride, int K,
+                                                             int D, const int32_t* slots, int bf, int lpr,
+                                                             float* cent, void* out_t) {
+    const int k = node_of_wave(), t = blockIdx.y;
+    if (k >= K) return;  // (the whole wave)
+    wave_block_mean<T, 8>(x, (size_t)t * x_tree_stride, D, slots + ((size_t)t * K + k) * bf, bf, lpr,
                        ((size_t)t * K + k) * D, cent, out_t);
 }
 
@@ -684,9 +695,11 @@ __global__ void k_gather_elems(const void* src, size_t src_tree_stride, const in
 
 // counts[p] = children in use; radii[p] = max over them of (||child - centre|| + r_child),
 // -inf when there is none.  One wave per node: `lpr` lanes (a power of two) hold a row in
-// 16-byte chunks (a chunk is contiguous in either layout), 64 / lpr children at a time.
+// 16-byte chunks (a chunk is contiguous in either layout), 64 / lpr children a step, eight steps on their
+// way.  Bound by the read of the children: 8 x 131072 rows of 256 bytes
+// 79 -> 75 us, 8 x 32768 18.6 -> 15
 template <typename T>
-__global__ __launch_bounds__(64) void k_radii(const void* child, size_t child_tree_stride,
+__global__ __launch_bounds__(kNodeThreads) void k_radii(const void* child, size_t child_tree_stride,
                                               const float* child_radii,
                                               size_t child_radii_stride,
                                               const int32_t* child_order, int size_child,
@@ -695,8 +708,9 @@ __global__ __launch_bounds__(64) void k_radii(const void* child, size_t child_tr
                                               int layout, float* radii, int32_t* counts,
                                               size_t out_stride) {
     constexpr int EPL = Elem<T>::kPerChunk;
-    const int p = blockIdx.x, t = blockIdx.y;
-    const int lane = threadIdx.x;
+    const int p = node_of_wave(), t = blockIdx.y;
+    if (p >= size) return;  // (the whole wave)
+    const int lane = threadIdx.x & 63;
     const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
     const bool chunk_ok = ch * EPL < D;
     float cf[EPL];
@@ -708,36 +722,48 @@ __global__ __launch_bounds__(64) void k_radii(const void* child, size_t child_tr
                 elem_index(layout, D, (size_t)p, ch * EPL));
         unpack<T>(raw, cf);
     }
+    // (the children's orders and radii in one load each, U rows a lane group in flight; size_child =
+    // size * bf, and bf <= 64)
+    constexpr int U = 8;
+    const size_t s0 = (size_t)p * bf;
+    const bool mine = lane < bf && s0 + lane < (size_t)size_child && child_order[(size_t)t * size_child + s0 + lane] >= 0;
+    const float my_radius = mine && child_radii ? child_radii[(size_t)t * child_radii_stride + s0 + lane] : 0.0f;
+    const unsigned long long live = __ballot(mine);
+    const int c = __popcll(live);
     float r = -INFINITY;
-    int c = 0;
-    for (int j0 = 0; j0 < bf; j0 += groups) {  // (uniform trip count: the sums meet in shuffles)
-        const int j = j0 + rg;
-        const int s = p * bf + j;
-        const bool have = j < bf && s < size_child && child_order[(size_t)t * size_child + s] >= 0;
-        uint4 raw = make_uint4(0, 0, 0, 0);
-        if (have && chunk_ok)
-            raw = *reinterpret_cast<const uint4*>(
-                reinterpret_cast<const T*>(child) + (size_t)t * child_tree_stride * D +
-                elem_index(child_layout, D, (size_t)s, ch * EPL));
-        float f[EPL];
-        unpack<T>(raw, f);
-        float ss = 0.0f;
+    for (int j0 = 0; j0 < bf; j0 += U * groups) {  // (uniform trip count: the sums meet in shuffles)
+        uint4 raw[U];
 #pragma unroll
-        for (int q = 0; q < EPL; ++q) {
-            const float df = f[q] - cf[q];
-            ss += df * df;
+        for (int u = 0; u < U; ++u) {  // (a child that is none: the first slot's row)
+            const int j = j0 + u * groups + rg;
+            const size_t row = s0 + (j < bf && ((live >> (j & 63)) & 1) ? j : 0);
+            raw[u] = *reinterpret_cast<const uint4*>(
+                reinterpret_cast<const T*>(child) + (size_t)t * child_tree_stride * D +
+                elem_index(child_layout, D, row, chunk_ok ? ch * EPL : 0));
         }
-        for (int off = 1; off < lpr; off <<= 1) ss += __shfl_xor(ss, off, 64);
-        if (have) {
-            ++c;
-            float v = sqrtf(ss);
-            if (child_radii) v += child_radii[(size_t)t * child_radii_stride + s];
-            r = fmaxf(r, v);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = j0 + u * groups + rg;
+            float f[EPL];
+            unpack<T>(raw[u], f);
+            float ss = 0.0f;
+#pragma unroll
+            for (int q = 0; q < EPL; ++q) {
+                const float df = f[q] - cf[q];
+                ss += df * df;
+            }
+            if (!chunk_ok) ss = 0.0f;
+            ss = group_sum_of(ss, lpr);
+            const float radius = __shfl(my_radius, j & 63, 64);
+            if (j < bf && ((live >> (j & 63)) & 1)) {
+                float v = sqrtf(ss);
+                if (child_radii) v += radius;
+                r = fmaxf(r, v);
+            }
         }
     }
     for (int off = lpr; off < 64; off <<= 1) {
         r = fmaxf(r, __shfl_xor(r, off, 64));
-        c += __shfl_xor(c, off, 64);
     }
     if (lane == 0) {
         // a few ulp of head room: the bound must survive fp32 rounding of this sum
@@ -929,14 +955,14 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
         const long long all_items = (long long)n_c * NT;
         int round = 0;  // of the level, Lloyd and packing together
         const int large = large_blocks(Kl);
-        const dim3 g_cent(Kl, NT), g_bucket(large + ceil_div(Kl, kWaves), NT);
+        const dim3 g_bucket(large + ceil_div(Kl, kWaves), NT);
 
         // Trees with fewer items than rows (n_live): the rounds over all items are over the first
         // ones of every tree.
         const bool ragged = n_live != nullptr && l == 1;
         hipLaunchKernelGGL(k_level_init, dim3(min(ceil_div(Kl * bf, 256), 2048), NT), dim3(256), 0, s, n_c, Kl, bf,
                            D, Kt, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters, tiles, KS);
-        hipLaunchKernelGGL((k_init_centroids<T>), g_cent, dim3(64), 0, s, x, n_c, xs, Kl, D,
+        hipLaunchKernelGGL((k_init_centroids<T>), node_grid(Kl, NT), dim3(kNodeThreads), 0, s, x, n_c, xs, Kl, D,
                            seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, bf,
                            Kt, w.fill, tiles, KS);
         // a round: the assignment (which also puts the items into buckets), then what the round does
@@ -1009,7 +1035,7 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
                            list_count + (pack_rounds & 1) * ct, w.lost, lost_count, n_c, Kl, bf, w.fill,
                            w.unsure, w.slots[l]);
         // block centre = mean of what is in the block, rounded to the storage type
-        hipLaunchKernelGGL((k_block_mean<T>), g_cent, dim3(64), 0, s, x, xs, Kl, D, w.slots[l], bf,
+        hipLaunchKernelGGL((k_block_mean<T>), node_grid(Kl, NT), dim3(kNodeThreads), 0, s, x, xs, Kl, D, w.slots[l], bf,
                            lpr, w.cent_f32, w.cent_t[l]);
         HIRA_CHECK_LAUNCH("build level");
     }
@@ -1058,7 +1084,7 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
     for (int l = 1; l < L; ++l) {
         const void* child = l == 1 ? t->keys : t->centers[l - 1];
         const float* crad = l == 1 ? nullptr : t->radii[l - 1];
-        hipLaunchKernelGGL((k_radii<T>), dim3(t->size[l], NT), dim3(64), 0, s, child,
+        hipLaunchKernelGGL((k_radii<T>), node_grid(t->size[l], NT), dim3(kNodeThreads), 0, s, child,
                            (size_t)t->cap[l - 1], crad, (size_t)t->cap[l - 1], w.order[l - 1],
                            t->size[l - 1], t->centers[l], (size_t)t->cap[l], t->size[l], bf, D, lpr,
                            l == 1 ? key_layout_of(t->layout) : center_layout_of(t->layout),

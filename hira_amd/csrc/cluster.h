@@ -124,26 +124,38 @@ __device__ __forceinline__ void wave_mean(const void* x, size_t row0, Ids ids, i
 // storage type.  One wave: `lpr` lanes (a power of two) hold a row in 16-byte chunks,
 // the 64 / lpr lane groups take every (64 / lpr)-th slot, and their sums are added pairwise in a
 // fixed order.  An empty block keeps its value.
-template <typename T>
+// (the slots in one load, U rows a lane group in flight: bf <= 64)
+template <typename T, int U>
 __device__ __forceinline__ void wave_block_mean(const void* x, size_t row0, int D, const int32_t* slots, int bf,
                                                 int lpr, size_t out, float* cent, void* out_t) {
     constexpr int EPL = Elem<T>::kPerChunk;
     const int lane = threadIdx.x & 63;
     const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
     const bool chunk_ok = ch * EPL < D;
+    const int slot = lane < bf ? slots[lane] : -1;
     float acc[EPL];
 #pragma unroll
     for (int q = 0; q < EPL; ++q) acc[q] = 0.0f;
     int cnt = 0;
-    for (int e = rg; e < bf; e += groups) {
-        const int it = slots[e];
-        if (it < 0) continue;
-        ++cnt;
-        if (!chunk_ok) continue;
-        float f[EPL];
-        unpack<T>(load_chunk<T>(x, (row0 + it) * D, ch), f);
+    for (int e0 = 0; e0 < bf; e0 += U * groups) {  // uniform: the slots come by shuffles
+        int it[U];
+        uint4 raw[U];
 #pragma unroll
-        for (int q = 0; q < EPL; ++q) acc[q] += f[q];
+        for (int u = 0; u < U; ++u) {
+            const int e = e0 + u * groups + rg;
+            it[u] = __shfl(slot, e & 63, 64);
+            if (e >= bf) it[u] = -1;
+            raw[u] = load_chunk<T>(x, (row0 + max(it[u], 0)) * D, chunk_ok ? ch : 0);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (it[u] >= 0) {
+                ++cnt;
+                float f[EPL];
+                unpack<T>(raw[u], f);
+#pragma unroll
+                for (int q = 0; q < EPL; ++q) acc[q] += f[q];
+            }
     }
     for (int off = lpr; off < 64; off <<= 1) {
         cnt += __shfl_xor(cnt, off, 64);

@@ -119,6 +119,17 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// sum over each aligned group of `lpr` lanes, in the order of group_sum<lpr>
+__device__ __forceinline__ float group_sum_of(float v, int lpr) {
+    if (lpr >= 2) v += dpp_move<0xB1>(v);
+    if (lpr >= 4) v += dpp_move<0x4E>(v);
+    if (lpr >= 8) v += dpp_move<0x141>(v);
+    if (lpr >= 16) v += dpp_move<0x140>(v);
+    if (lpr >= 32) v += __shfl_xor(v, 16, 64);
+    if (lpr >= 64) v += __shfl_xor(v, 32, 64);
+    return v;
+}
+
 // Reductions ACROSS the 64/LANES groups of a wave (lanes with equal lane % LANES).
 template <int LANES>
 __device__ __forceinline__ float cross_group_max(float v) {

@@ -387,7 +387,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
         __syncthreads();
         // ---- block centres ----------------------------------------------------------------------------
         for (int k = wave; k < K; k += kSmallWaves)
-            wave_block_mean<bf16_t>(x, row0, D, slots + (size_t)k * bf, bf, p.lpr, ((size_t)t * K + k) * D, p.cent, p.cent_t[l]);
+            wave_block_mean<bf16_t, 2>(x, row0, D, slots + (size_t)k * bf, bf, p.lpr, ((size_t)t * K + k) * D, p.cent, p.cent_t[l]);
         __syncthreads();  // (the next level reads them)
     }
 }
