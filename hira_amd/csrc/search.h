@@ -66,7 +66,7 @@ struct SearchParams {
 
 // element i of the attention output, in the type the caller asked for
 __device__ __forceinline__ void store_out(void* out, int bf16, size_t i, float v) {
-    if (bf16) reinterpret_cast<uint16_t*>(out)[i] = f32_to_bf16_bits(v);  // uniform
+    if (__builtin_expect(bf16, 0)) reinterpret_cast<uint16_t*>(out)[i] = f32_to_bf16_bits(v);  // uniform
     else reinterpret_cast<float*>(out)[i] = v;
 }
 
