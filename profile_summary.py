@@ -65,7 +65,7 @@ def build_table(path: str, which: int):
            "| kernel | calls | total us | avg us | min us | max us |", "|---|---|---|---|---|---|"]
     for k, v in sorted(agg.items(), key=lambda kv: -sum(kv[1])):
         out.append(f"| `{k[:70]}` | {len(v)} | {sum(v):.1f} | {sum(v) / len(v):.2f} | {min(v):.2f} | {max(v):.2f} |")
-    asg = [f"{dur(r):.0f}" for r in one if "k_assign_mfma" in r["Kernel_Name"]]
+    asg = [f"{dur(r):.0f}" for r in one if "k_assign_" in r["Kernel_Name"]]
     out += ["", "assignment launches in order (us): " + " ".join(asg)]
     return "\n".join(out)
 
