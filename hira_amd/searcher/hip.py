@@ -189,13 +189,11 @@ class HIPSearcher(BaseSearcher):
                 c = self._calls.get(key)
                 if c is None:
                     off, heads, gmax, group = self._head_map(h_q, indexer, None)
-                    # (through the host: the copy is complete for every stream when it returns)
-                    ones = torch.ones((h_q,)).to(indexer.keys_buf.device)
                     qs = _lib.HiraQuery(h_q, None, None, None, off.data_ptr(), heads.data_ptr(), gmax, group)
                     if len(self._calls) >= self._MAX_CALLS:
                         self._calls.clear()
                     c = self._calls[key] = _Call(tree, self.launch, qs, indexer.keys_buf.get_device(),
-                                                 (off, heads), ones)
+                                                 (off, heads), None)
                 if query.get_device() == c.dev:
                     dev, qs = c.dev, c.query
                     if isinstance(threshold, torch.Tensor) and threshold.dtype is torch.float32 and \
@@ -206,6 +204,8 @@ class HIPSearcher(BaseSearcher):
                         tau = self._coerce_threshold(threshold, h_q, indexer.device)
                     if scaling is None:
                         sc = c.ones
+                        if sc is None:
+                            sc = self._scale_of_one(c, h_q, indexer.keys_buf.device)
                     elif isinstance(scaling, torch.Tensor) and scaling.dtype is torch.float32 and \
                             scaling.numel() == h_q and scaling.get_device() == dev and \
                             scaling.is_contiguous():
@@ -217,6 +217,16 @@ class HIPSearcher(BaseSearcher):
         qs, keep = self._query_struct(query, threshold, indexer, q_head_to_kv, scaling)
         return (_Call(tree, self.launch, qs, indexer.keys_buf.get_device(), keep, None),
                 qs.num_q_heads, keep)
+
+    @staticmethod
+    def _scale_of_one(c: _Call, h_q: int, device) -> torch.Tensor:
+        """A scale of one per head, kept with the call description -- through the host: the copy is
+        complete for every stream when it returns.  A call that is being captured takes one of the
+        graph's own."""
+        if torch.cuda.is_current_stream_capturing():
+            return torch.ones((h_q,), dtype=torch.float32, device=device)
+        c.ones = torch.ones((h_q,), dtype=torch.float32).to(device)
+        return c.ones
 
     def _get_workspace(self, nbytes: int, device) -> torch.Tensor:
         if self._workspace is None or self._workspace.numel() < nbytes or \

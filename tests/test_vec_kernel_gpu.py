@@ -60,3 +60,27 @@ def test_trees_and_batches(n, levels, bf, group, gpu_device):
 @pytest.mark.parametrize("threads,npw", [(64, 1), (64, 70), (128, 3), (256, 33), (512, 9)])
 def test_workgroup_shapes(threads, npw, gpu_device):
     _check(2500, 80, torch.float32, 3, 7, 4, seed=threads + npw, queue=33, block_threads=threads, nodes_per_wave=npw)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_first_call_on_an_index_may_be_captured(dtype, gpu_device):
+    """No scale given, another index than the call before (same heads): nothing comes from the host."""
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    keys, vals = (torch.randn(2, 1, 2, 900, 64, device="cuda").to(dtype) for _ in range(2))
+    a, b = (HIPIndexer(2, 1, 32).build(k, v) for k, v in zip(keys, vals))
+    q, tau = torch.randn(4, 64, device="cuda").to(dtype), torch.full((4,), 6.0, device="cuda")
+    searcher = HIPSearcher()
+    searcher.search_attention(q, tau, a)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = searcher.search_attention(q, tau, b)
+    want = HIPSearcher().search_attention(q, tau, b, scaling=torch.ones(4, device="cuda"))
+    assert bool((want != 0).any())
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
