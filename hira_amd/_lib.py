@@ -220,7 +220,10 @@ def check(rc: int) -> None:
 
 
 def stream_of(index: int) -> int:
-    """Handle of torch's current HIP stream on device number `index`."""
+    """Handle of torch's current HIP stream on device number `index`, as a tensor's ``get_device()``
+    gives it: -1 is host memory, which torch would take for "the current device"."""
+    if index < 0:
+        raise ValueError("the arrays are in host memory: this call runs on the GPU")
     global _raw_stream
     if _raw_stream is None:
         import torch
@@ -240,7 +243,10 @@ def current_stream(device) -> int:
     per layer and decode step)."""
     import torch
 
-    idx = device.index if isinstance(device, torch.device) else torch.device(device).index
+    device = torch.device(device)
+    if device.type == "cpu":
+        raise ValueError("the arrays are in host memory: this call runs on the GPU")
+    idx = device.index
     if idx is None:
         idx = torch.cuda.current_device()
     raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)

@@ -58,7 +58,18 @@ _MINUS_INF = 0xFF800000  # the bits of an fp32 -inf
 
 def _fill_arrays(specs, trees: int) -> None:
     """One launch over several (T, rows, ...) arrays: (dst, src or None, rows to copy from src, first
-    row to fill, fill word).  What growing an index, or clearing its padding, takes."""
+    row to fill, fill word).  What growing an index, or clearing its padding, takes.  Arrays in host
+    memory (an index restored there) take tensor operations instead."""
+    if not specs[0][0].is_cuda:
+        for dst, src, rows, fill_from, word in specs:
+            if src is not None:
+                dst[:, :rows] = src[:, :rows]
+            tail = dst[:, fill_from:]
+            if word:  # (perm, radii: words of four bytes)
+                tail.view(torch.int32).fill_(word - (1 << 32))
+            else:
+                tail.zero_()
+        return
     arr = (_lib.HiraArray * len(specs))()
     for a, (dst, src, rows, fill_from, word) in zip(arr, specs):
         row = dst.element_size() * (dst.shape[2] if dst.ndim == 3 else 1)
@@ -810,6 +821,13 @@ class HIPIndexer(BaseIndexer):
         # nothing known yet)
         self._state = torch.empty((self.num_trees, _lib.HIRA_MAX_LEVELS + 2), dtype=torch.int32,
                                   device=self.device)
+        if not self._state.is_cuda:
+            row = [0] * (_lib.HIRA_MAX_LEVELS + 2)
+            row[0 if self.num_levels == 1 else 1:self.num_levels] = \
+                self.size[0 if self.num_levels == 1 else 1:]
+            row[_lib.HIRA_MAX_LEVELS] = self.num_keys
+            self._state[:] = torch.tensor(row, dtype=torch.int32)
+            return
         tree = self.tree_struct()
         _lib.check(_lib.lib().hira_update_state(C.byref(tree), self.num_keys, self._state.data_ptr(),
                                                 _lib.stream_of(self._state.get_device())))

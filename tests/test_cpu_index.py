@@ -1,0 +1,72 @@
+"""An index in host memory: restored, adopted, grown and saved without a GPU; what would launch a kernel
+on it is refused."""
+import numpy as np
+import pytest
+import torch
+
+from hira_amd import _lib
+from hira_amd.indexer.hip import HIPIndexer
+from oracle import hira_oracle as ho
+
+
+def _parts(dtype, bf=16, n=300, d=64, trees=2, seed=0):
+    rng = np.random.default_rng(seed)
+    keys = torch.from_numpy(rng.normal(size=(trees, n, d)).astype(np.float32)).to(dtype).float().numpy()
+    size = ho.fixed_fanout_sizes(n, bf, 3)
+    pad, perm = np.zeros((trees, size[0], d), np.float32), np.full((trees, size[0]), -1, np.int32)
+    pad[:, :n], perm[:, :n] = keys, np.arange(n)
+    k1, k2 = size[1], size[2]
+    counts1 = np.clip(n - np.arange(k1) * bf, 0, bf).astype(np.int32)
+    c1, c2 = (rng.normal(size=(trees, k, d)).astype(np.float32) for k in (k1, k2))
+    return dict(bf=bf, keys=pad, perm=perm, values=pad.copy(), dtype=dtype, centers=[None, c1, c2],
+                radii=[None, np.full((trees, k1), 20.0, np.float32), np.full((trees, k2), 40.0, np.float32)],
+                counts=[None, np.tile(counts1, (trees, 1)), np.full((trees, k2), bf, np.int32)])
+
+
+@pytest.mark.parametrize("dtype,layout", [(torch.float32, "row_major"), (torch.bfloat16, "row_major"),
+                                          (torch.bfloat16, "tiled")])
+@pytest.mark.parametrize("capacity", [None, 2000])
+def test_adopted_saved_loaded_and_grown(dtype, layout, capacity, tmp_path):
+    p = _parts(dtype)
+    a = HIPIndexer.from_layout(device="cpu", layout=layout, capacity=capacity, **p)
+    n = a.size[0]
+    keys = torch.from_numpy(p["keys"]).to(dtype)
+
+    def whole(x):
+        assert x.size == a.size and x.num_keys == 300 and all(c >= s for c, s in zip(x.cap, x.size))
+        assert torch.equal(x.keys_rowmajor(), keys) and torch.equal(x.values_buf[:, :n], keys)
+        assert torch.equal(x.perm[:, :n], torch.from_numpy(p["perm"]))
+        for l in (1, 2):
+            k = x.size[l]
+            assert torch.equal(x.centers_rowmajor(l), torch.from_numpy(p["centers"][l]).to(dtype))
+            assert torch.equal(x.radii[l][:, :k], torch.from_numpy(p["radii"][l]))
+            assert torch.equal(x.counts[l][:, :k], torch.from_numpy(p["counts"][l]))
+            # what lies behind the slots in use is empty
+            assert bool((x.radii[l][:, k:] == float("-inf")).all()) and not x.counts[l][:, k:].any()
+        assert bool((x.perm[:, n:] == -1).all()) and not x.values_buf[:, n:].any()
+
+    whole(a)
+    path = str(tmp_path / "index.safetensors")
+    a.save(path)
+    b = HIPIndexer.load(path, device="cpu", capacity=capacity)
+    whole(b)
+    b.reserve(5000)
+    assert b.cap[0] > n + 5000 - 300
+    whole(b)
+    b.begin_unsynced(10)
+    assert b._state.shape == (2, _lib.HIRA_MAX_LEVELS + 2)
+    assert b._state[0].tolist()[:3] == [0, a.size[1], a.size[2]] and int(b._state[1, _lib.HIRA_MAX_LEVELS]) == 300
+
+
+def test_no_kernel_is_launched_over_host_memory():
+    p = _parts(torch.float32)
+    a = HIPIndexer.from_layout(device="cpu", layout="row_major", **p)
+    new = torch.zeros((1, 2, 1, 64))
+    for call in (lambda: a.update(new, new), lambda: HIPIndexer(2, device="cpu").build(new, new),
+                 lambda: HIPIndexer.from_layout(device="cpu", layout="q8", **_parts(torch.bfloat16))):
+        with pytest.raises(ValueError, match="GPU"):
+            call()
+    with pytest.raises(ValueError, match="GPU"):
+        _lib.stream_of(-1)
+    with pytest.raises(ValueError, match="GPU"):
+        _lib.current_stream(torch.device("cpu"))
