@@ -208,7 +208,9 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
             const float l = i0 == 0 ? l0 : (i < P ? ld(pl + i) : 0.0f);
             const float w = m > -INFINITY ? exp2f(m - mx) : 0.0f;
             ls += w * l;
-            const bool nz = w > 0.0f && l > 0.0f;
+            // (whatever holds a selected key, however small its weight beside the others': zero times an
+            // infinite sum is no zero)
+            const bool nz = m > -INFINITY;
             const unsigned long long bal = __ballot(nz);
             if (nz) {
                 const int k = n + __popcll(bal & ((1ull << lane) - 1ull));
@@ -241,9 +243,11 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
             for (int k0 = grp; k0 < n; k0 += 8 * n_grp) {
                 u32x4 v[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u)  // (16: the device-scope bit)
-                    v[u] = __builtin_amdgcn_raw_buffer_load_b128(
-                        rsrc, col0 + (unsigned)list[g * P + min(k0 + u * n_grp, n - 1)] * (unsigned)(Dv * 4), 0, 16);
+                for (int u = 0; u < 8; ++u) {  // (16: the device-scope bit)
+                    // (beyond the list: an address beyond the buffer, which reads as zero)
+                    const unsigned at = col0 + (unsigned)list[g * P + min(k0 + u * n_grp, n - 1)] * (unsigned)(Dv * 4);
+                    v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, k0 + u * n_grp < n ? at : 0xfffffff0u, 0, 16);
+                }
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
                     const float w = k0 + u * n_grp < n ? wts[g * P + k0 + u * n_grp] : 0.0f;
@@ -261,7 +265,7 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
                 const float o[4] = {sx, sy, sz, sw};
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
-                    store_out(p.attn_out, p.out_bf16, (size_t)head * Dv + qd * 4 + c, L > 0.0f ? o[c] / L : 0.0f);
+                    store_out(p.attn_out, p.out_bf16, (size_t)head * Dv + qd * 4 + c, L == 0.0f ? 0.0f : o[c] / L);
             }
         }
     }
@@ -273,7 +277,7 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
         float sum = 0.0f;
         for (int r = 0; r < n_grp; ++r) sum += red[(size_t)r * items * 4 + e];
         const float L = s_l[g];
-        store_out(p.attn_out, p.out_bf16, (size_t)head * Dv + (e - g * Dv), L > 0.0f ? sum / L : 0.0f);
+        store_out(p.attn_out, p.out_bf16, (size_t)head * Dv + (e - g * Dv), L == 0.0f ? 0.0f : sum / L);
     }
 }
 
@@ -620,8 +624,12 @@ void search_kernel(const SearchParams p) {
             }
             if (owner) {
 #pragma unroll
-                for (int i = 0; i < KEPT; ++i)
-                    tab[(my_u * RPW + rg) * GMAX + my_g + i] = (sel >> i) & 1u ? s[i] * my_sc[i] * kLog2e : -INFINITY;
+                for (int i = 0; i < KEPT; ++i) {
+                    // (fminf: a logit that is no number becomes +inf.  A maximum does not see the former,
+                    // and what follows makes NaN of both, as a softmax does)
+                    const float z = fminf(s[i] * my_sc[i] * kLog2e, INFINITY);
+                    tab[(my_u * RPW + rg) * GMAX + my_g + i] = (sel >> i) & 1u ? z : -INFINITY;
+                }
             }
             // weights while the values are on their way: lane l takes the table's entries
             // l, l + 64, ..., all of head l % GMAX
@@ -640,8 +648,10 @@ void search_kernel(const SearchParams p) {
             m_run = mx;
 #pragma unroll
             for (int i = 0; i < NE; ++i) {
-                const float w = z[i] > -INFINITY ? exp2f(z[i] - mx) : 0.0f;
+                // (zero says "not selected": a selected row's weight stays above it)
+                float w = z[i] > -INFINITY ? exp2f(z[i] - mx) : 0.0f;
                 l_run += w;
+                if (GMAX > 1 && w == 0.0f && z[i] > -INFINITY) w = 1e-45f;
                 if (ROWS * GMAX >= 64 || lane < ROWS * GMAX) tab[i * 64 + lane] = w;
             }
             __builtin_amdgcn_wave_barrier();
@@ -651,17 +661,30 @@ void search_kernel(const SearchParams p) {
 #pragma unroll
                 for (int e = 0; e < EPL; ++e) acc[g][e] *= fg;
             }
+            // (a row's weights are asked for with the row before it.  The heads that did not select the row
+            // are masked out, not multiplied by zero: a value that is not finite stays with those that did.
+            // As masks on straight-line code it costs nothing to be seen with up to four heads a pass and 2 %
+            // with eight -- 2 trees x 20000 rows of 64 bf16 25.8 -> 26.2 us --, as branches 2 and 7 %)
+            float wt[GMAX];
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) wt[g] = tab[rg * GMAX + g];
 #pragma unroll
             for (int u = 0; u < KU; ++u) {
-                if ((B & LANES.row[u]) == 0ull) continue;  // uniform in the wave
-                float vf[EPL];
-                unpack<T>(vraw[u], vf);
+                float next[GMAX];
 #pragma unroll
-                for (int g = 0; g < GMAX; ++g) {
-                    const float w = tab[(u * RPW + rg) * GMAX + g];
+                for (int g = 0; g < GMAX; ++g) next[g] = tab[(min(u + 1, KU - 1) * RPW + rg) * GMAX + g];
+                if ((B & LANES.row[u]) != 0ull) {  // uniform in the wave
+                    float vf[EPL];
+                    unpack<T>(vraw[u], vf);
 #pragma unroll
-                    for (int e = 0; e < EPL; ++e) acc[g][e] += w * vf[e];
+                    for (int g = 0; g < GMAX; ++g)
+                        if (GMAX == 1 || __builtin_expect(wt[g] != 0.0f, 1)) {
+#pragma unroll
+                            for (int e = 0; e < EPL; ++e) acc[g][e] += wt[g] * vf[e];
+                        }
                 }
+#pragma unroll
+                for (int g = 0; g < GMAX; ++g) wt[g] = next[g];
             }
         }
     }
