@@ -387,9 +387,10 @@ __device__ __attribute__((noinline)) void update_one_key_called(const UpdatePara
 //   rows       of the 64 keys to their slots, 16 bytes a thread.
 // Radii wait until the list is given up: R = max over the keys of what each asks for, and that
 // grows with the distance, so the largest distance a candidate saw gives the radius that key by
-// key would have reached, to the last bit, and so up the levels.  A key that finds no candidate
-// opens a node the general way (all candidates are full then: the new node becomes the list).  A
-// tree with more nodes with room than the list holds goes the general way altogether.  Same
+// key would have reached, to the last bit, and so up the levels.  A key that finds all candidates
+// full opens a node, which becomes the list.  A key that has no finite distance to any candidate opens
+// one too, but the others still have room: it ends its chunk, and the nodes with room are listed anew.
+// A tree with more nodes with room than the list holds goes the general way altogether.  Same
 // placement, slots and radii as key by key (the replaced kernels:
 // kernels/triton_update_kernels.py:85-123 nearest centre for a whole window at once, :126-235 slots,
 // :238-326 radii).
@@ -725,6 +726,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
     __shared__ WindowLds w;
     __shared__ int s_slot[kWinKeys];  // where the chunk's keys went (-1: placed the general way, or dropped)
     __shared__ int s_done;            // keys of the chunk dealt with so far
+    __shared__ bool s_room;           // a listed node has room
     __shared__ int s_used[HIRA_MAX_LEVELS];  // slots in use per level
     constexpr int EPL = Elem<T>::kPerChunk;
     const int tree = blockIdx.x;
@@ -769,8 +771,9 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
         for (int i = 0; i < p.m; ++i) update_one_key_called<T>(p, tree, i, sm, red_f, red_i, s_dist, s_rad);
         return;
     }
-    for (int i0 = 0; i0 < p.m; i0 += kWinKeys) {  // uniform
-        const int nk = min(kWinKeys, p.m - i0);
+    for (int i0 = 0; i0 < p.m;) {  // uniform
+        int nk = min(kWinKeys, p.m - i0);
+        bool list_anew = false;  // behind this chunk
         const int position0 = position;
         if (i0 > 0) {
             stage(i0);  // (behind the barrier that ends the chunk before: nobody needs its rows any more)
@@ -828,8 +831,10 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
                     w.cnt[lane] = cnt;
                     w.far[lane] = far;
                 }
+                const bool room = __ballot(cnt < bf) != 0ull;
                 if (lane == 0) {
                     s_done = kk;
+                    s_room = room;
                     if (kk < nk) s_slot[kk] = -1;
                 }
             }
@@ -838,11 +843,16 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
             position += kd - k;
             k = kd;
             if (k < nk) {
-                // key k found no node with room: it opens one.  All listed nodes are full, so the
-                // new one is the whole list from here on.
+                // key k found no node with room, or none at a distance that is a finite number: it opens one
+                list_anew = s_room;
                 window_flush(p, tree, w);
                 const int node = open_node<T>(p, tree, i0 + k, position, s_used, rows + (size_t)k * D, sm, red_f, red_i, s_dist, s_rad);
                 if (node >= 0) ++position;
+                if (list_anew) {  // uniform
+                    nk = k + 1;
+                    break;
+                }
+                // (all listed nodes are full: the new one is the whole list from here on)
                 if (t == 0) {
                     w.n = node >= 0 ? 1 : 0;
                     w.id[0] = node;
@@ -918,7 +928,17 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
                 if (lane == 0) atomicMax(reinterpret_cast<int*>(p.keps + b1 + slot / bf), __float_as_int(worst));
             }
         }
-        if (i0 + kWinKeys < p.m) __syncthreads();
+        i0 += nk;
+        if (list_anew) {  // uniform
+            __syncthreads();
+            if (!window_candidates<T>(p, tree, w, cen)) {
+                if (t == 0) st[HIRA_MAX_LEVELS] = position;
+                __syncthreads();
+                for (; i0 < p.m; ++i0) update_one_key_called<T>(p, tree, i0, sm, red_f, red_i, s_dist, s_rad);
+                return;
+            }
+        }
+        if (i0 < p.m) __syncthreads();
     }
     window_flush(p, tree, w);
     if (wave == 0) {

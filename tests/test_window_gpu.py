@@ -90,3 +90,56 @@ def test_window_equals_key_by_key_on_half_full_trees(k2, bf, m, d, dtype, layout
     for i in range(6):
         b.update(N[:, :, i:i + 1], N[:, :, i:i + 1])
     assert torch.equal(a.perm[:, :a.size[0]], b.perm[:, :b.size[0]])
+
+
+@pytest.mark.parametrize("k2,bf,m,d,dtype,layout,bad", [
+    (1, 8, 30, 64, torch.float32, "row_major", {5: "nan", 11: "inf", 12: "huge"}),
+    (3, 8, 64, 128, torch.bfloat16, "row_major", {0: "huge", 63: "nan"}),            # first and last of a chunk
+    (2, 16, 130, 128, torch.bfloat16, "tiled", {64: "inf", 65: "nan", 128: "huge"}),  # at the seams of chunks
+    (3, 16, 80, 64, torch.bfloat16, "tiled", {3: "nan", 9: "inf"}),  # then more nodes with room than the list holds
+    (1, 16, 40, 128, torch.bfloat16, "q8", {7: "huge"}),
+])
+def test_window_with_keys_that_have_no_distance(k2, bf, m, d, dtype, layout, bad, gpu_device):
+    """A key whose distances are not finite opens a node of its own; the nodes with room stay known:
+    the keys behind it, and the next windows, fill them as key by key."""
+    from hira_amd.indexer.hip import HIPIndexer
+
+    parts, held = _half_full(1, k2, bf, d, dtype, seed=m)
+    rng = np.random.default_rng(m)
+    c1 = parts["centers"][1]
+    new = (c1[:, rng.integers(0, c1.shape[1], size=m)] + 0.3 * rng.normal(size=(1, m, d))).astype(np.float32)
+    for i, what in bad.items():
+        new[0, i, 3] = {"nan": np.nan, "inf": np.inf, "huge": 1e30}[what]  # (huge: its square overflows)
+    N = torch.from_numpy(new)[None].to(dtype).cuda()
+    a, b = (HIPIndexer.from_layout(layout=layout, num_keys=int(held[0]), **parts) for _ in range(2))
+    for x in (a, b):
+        x.graft_min = 1 << 30
+        x.reserve(64 * bf * bf)  # (every such key may take a node of each level)
+    free = int((bf - a.counts[1][:, :k2 * bf]).sum())
+    bits = {torch.float32: torch.int32, torch.bfloat16: torch.int16}[dtype]
+
+    def same():
+        assert a.size == b.size and torch.equal(a._state[:, 1:], b._state[:, 1:])
+        n = a.size[0]
+        assert torch.equal(a.perm[:, :n], b.perm[:, :n])
+        assert torch.equal(a.keys_buf.view(bits), b.keys_buf.view(bits))
+        assert torch.equal(a.values_buf.view(bits)[:, :n], b.values_buf.view(bits)[:, :n])
+        for l in (1, 2):
+            k = a.size[l]
+            assert torch.equal(a.counts[l][:, :k], b.counts[l][:, :k])
+            assert torch.equal(a.radii[l][:, :k], b.radii[l][:, :k])
+            assert torch.equal(a.centers_rowmajor(l).view(bits), b.centers_rowmajor(l).view(bits))
+
+    a.update(N, N)
+    for i in range(m):
+        b.update(N[:, :, i:i + 1], N[:, :, i:i + 1])
+    same()
+    good = [i for i in range(m) if i not in bad]
+    if len(good) <= free:  # the nodes that had room took them all
+        assert int((bf - a.counts[1][:, :k2 * bf]).sum()) == free - len(good)
+    for lo in (0, 6):  # the next windows find what room is left
+        w = N[:, :, good[lo:lo + 6]].contiguous()
+        a.update(w, w)
+        for i in range(6):
+            b.update(w[:, :, i:i + 1], w[:, :, i:i + 1])
+        same()
