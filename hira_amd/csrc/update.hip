@@ -396,8 +396,12 @@ __device__ __attribute__((noinline)) void update_one_key_called(const UpdatePara
 // :238-326 radii).
 constexpr int kCandMax = 48;
 constexpr int kWinKeys = 64;  // keys of a window taken together
-constexpr int kWinCols = 4;   // columns of a row a lane holds, at most (rows of up to 256)
-constexpr size_t kWinLds = 128 * 1024;  // dynamic LDS of a workgroup, at most (256 fp32 columns: 126 KiB)
+// COLS, below: columns of a row a lane holds, at most.  Rows of fp32, and of bf16 up to 256, take four;
+// wider ones five (320 columns): 8 trees x 64 keys of 288 columns, which went key by key, 358 -> 61 us.
+// Five for all rows would cost those of 128 columns 0.8 us of 33.
+constexpr int kWinColsMax = 5;
+constexpr size_t kWinLds = 128 * 1024;  // dynamic LDS of a workgroup, at most (256 fp32 columns: 126 KiB; 320
+                                        // bf16 columns: 115)
 
 struct WindowLds {
     int n;                                  // candidates listed (may exceed kCandMax: then unusable)
@@ -514,7 +518,7 @@ __device__ __forceinline__ float win_sum_across(float v) {
 // each, and goes through the candidates: the eight sums over the lanes halve in number with every
 // one of the first three steps (lanes with the bit set go on with the other half).  The additions are those of a butterfly of lane ^ 1, ^ 2,
 // ..., ^ 32, in that order: the general way's, to the last bit.
-template <typename T>
+template <typename T, int COLS>
 __device__ __forceinline__ void window_distances(const int D, const WindowLds& w, const float* cen, const T* rows,
                                  const int k0, const int k1, float* table) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -523,12 +527,12 @@ __device__ __forceinline__ void window_distances(const int D, const WindowLds& w
     const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
     const int mine = (b0 ? 4 : 0) + (b1 ? 2 : 0) + (b2 ? 1 : 0);  // the key (of eight) I end up with
     for (int k = k0 + wave * 8; k < k1; k += kUpdThreads / 64 * 8) {  // uniform in the wave
-        float x[8][kWinCols];
+        float x[8][COLS];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const size_t src = (size_t)min(k + u, k1 - 1) * D;
 #pragma unroll
-            for (int i = 0; i < kWinCols; ++i)
+            for (int i = 0; i < COLS; ++i)
                 if (i * 64 < D) {  // (uniform)
                     const float xi = load_elem<T>(rows, src + min(i * 64 + lane, D - 1));
                     x[u][i] = i * 64 + lane < D ? xi : 0.0f;
@@ -539,7 +543,7 @@ __device__ __forceinline__ void window_distances(const int D, const WindowLds& w
 #pragma unroll
             for (int u = 0; u < 8; ++u) v[u] = 0.0f;
 #pragma unroll
-            for (int i = 0; i < kWinCols; ++i)
+            for (int i = 0; i < COLS; ++i)
                 if (i * 64 < D) {  // uniform
                     const float ci = cen[(size_t)c * D + min(i * 64 + lane, D - 1)];
                     const float cj = i * 64 + lane < D ? ci : 0.0f;
@@ -716,7 +720,7 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
     return node1;
 }
 
-template <typename T>
+template <typename T, int COLS>
 __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParams p) {
     // 2 D floats of the general way, kCandMax centres, the table of distances, a chunk of key rows
     extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -779,7 +783,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
             stage(i0);  // (behind the barrier that ends the chunk before: nobody needs its rows any more)
             __syncthreads();
         }
-        window_distances<T>(D, w, cen, rows, 0, nk, table);
+        window_distances<T, COLS>(D, w, cen, rows, 0, nk, table);
         for (int k = 0; k < nk;) {  // uniform
             __syncthreads();
             if (wave == 0) {
@@ -869,7 +873,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
                 for (int j = t; j < D; j += kUpdThreads) cen[j] = sm[j];  // (its centre is the key)
                 __syncthreads();
                 ++k;
-                window_distances<T>(D, w, cen, rows, k, nk, table);
+                window_distances<T, COLS>(D, w, cen, rows, k, nk, table);
             }
         }
         // ---- the rows of the keys placed from the list, 16 bytes a thread -----------------------
@@ -1007,10 +1011,10 @@ static int update_arguments(const HiraTree* tree, const void* new_keys, const vo
     p.state = state;
     *smem = 2 * (size_t)tree->dim * sizeof(float);
     // windows of a few keys and more: the nodes with room are listed in LDS (where they fit: 48 centres
-    // of up to 256 columns beside the table of distances and a chunk of rows)
+    // of up to 256 columns, bf16 320, beside the table of distances and a chunk of rows)
     *smem_w = *smem + (size_t)kCandMax * (tree->dim + kWinKeys) * sizeof(float) +
               (size_t)kWinKeys * tree->dim * (tree->dtype == HIRA_F32 ? 4 : 2);
-    *window = m >= 4 && tree->num_levels >= 2 && tree->dim <= 64 * kWinCols && *smem_w <= kWinLds;
+    *window = m >= 4 && tree->num_levels >= 2 && tree->dim <= 64 * (tree->dtype == HIRA_F32 ? 4 : kWinColsMax) && *smem_w <= kWinLds;
     const size_t vrow = (size_t)tree->vdim * (tree->dtype == HIRA_F32 ? 4 : 2);
     if (new_values != nullptr && vrow % 16 == 0 && *smem_w + kWinKeys * vrow <= kWinLds) {
         p.stage_values = 1;
@@ -1021,7 +1025,7 @@ static int update_arguments(const HiraTree* tree, const void* new_keys, const vo
 
 // The window kernel's LDS, its own lists beside the dynamic part, can exceed what a launch gets
 // without asking: asked for once per kernel and device.
-template <typename T>
+template <typename T, int COLS>
 static int launch_update_window(const UpdateParams& p, int trees, size_t smem, hipStream_t s) {
     constexpr int kMaxDevices = 64;
     static int asked[kMaxDevices];
@@ -1029,12 +1033,12 @@ static int launch_update_window(const UpdateParams& p, int trees, size_t smem, h
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
         return fail(HIRA_ELAUNCH, "update: no current device");
     if (__atomic_load_n(&asked[dev], __ATOMIC_RELAXED) == 0) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_update_window<T>),
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_update_window<T, COLS>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWinLds) != hipSuccess)
             return fail(HIRA_ELAUNCH, "update: %zu bytes of LDS refused", kWinLds);
         __atomic_store_n(&asked[dev], 1, __ATOMIC_RELAXED);
     }
-    hipLaunchKernelGGL(k_update_window<T>, dim3(trees), dim3(kUpdThreads), smem, s, p);
+    hipLaunchKernelGGL((k_update_window<T, COLS>), dim3(trees), dim3(kUpdThreads), smem, s, p);
     return HIRA_OK;
 }
 
@@ -1075,8 +1079,10 @@ extern "C" int hira_update(const HiraTree* tree, const void* new_keys, const voi
     if (m == 0) return HIRA_OK;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (window) {
-        const int rc = tree->dtype == HIRA_F32 ? launch_update_window<float>(p, tree->num_trees, smem_w, s)
-                                               : launch_update_window<bf16_t>(p, tree->num_trees, smem_w, s);
+        const int rc = tree->dtype == HIRA_F32
+                           ? launch_update_window<float, 4>(p, tree->num_trees, smem_w, s)
+                           : tree->dim <= 256 ? launch_update_window<bf16_t, 4>(p, tree->num_trees, smem_w, s)
+                                              : launch_update_window<bf16_t, kWinColsMax>(p, tree->num_trees, smem_w, s);
         if (rc != HIRA_OK) return rc;
     } else if (tree->dtype == HIRA_F32) {
         hipLaunchKernelGGL(k_update<float>, dim3(tree->num_trees), dim3(kUpdThreads), smem, s, p);

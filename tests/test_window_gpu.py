@@ -143,3 +143,36 @@ def test_window_with_keys_that_have_no_distance(k2, bf, m, d, dtype, layout, bad
         for i in range(6):
             b.update(w[:, :, i:i + 1], w[:, :, i:i + 1])
         same()
+
+
+@pytest.mark.parametrize("d,dv,dtype", [(260, 260, torch.float32), (264, 264, torch.bfloat16),
+                                        (288, 288, torch.bfloat16), (312, 0, torch.bfloat16),
+                                        (320, 320, torch.bfloat16), (320, 64, torch.bfloat16),
+                                        (328, 328, torch.bfloat16)])
+def test_windows_of_rows_beyond_256_columns(d, dv, dtype, gpu_device):
+    """Around the widest rows that the list of nodes and a chunk of keys have room for."""
+    from hira_amd.indexer.hip import HIPIndexer
+
+    parts, held = _half_full(1, 2, 8, d, dtype, seed=d)
+    parts["values"] = parts["keys"][:, :, :dv].copy() if dv <= d and dv else None
+    rng = np.random.default_rng(d)
+    m = 70
+    c1 = parts["centers"][1]
+    new = (c1[:, rng.integers(0, c1.shape[1], size=m)] + 0.3 * rng.normal(size=(1, m, d))).astype(np.float32)
+    N = torch.from_numpy(new)[None].to(dtype).cuda()
+    V = N[..., :dv].contiguous() if dv else None
+    a, b = (HIPIndexer.from_layout(layout="row_major", num_keys=int(held[0]), **parts) for _ in range(2))
+    a.graft_min = b.graft_min = 1 << 30
+    a.update(N, V)
+    for i in range(m):
+        b.update(N[:, :, i:i + 1], None if V is None else V[:, :, i:i + 1])
+    assert a.size == b.size
+    n = a.size[0]
+    assert torch.equal(a.perm[:, :n], b.perm[:, :n]) and torch.equal(a.keys_buf[:, :n], b.keys_buf[:, :n])
+    if V is not None:
+        assert torch.equal(a.values_buf[:, :n], b.values_buf[:, :n])
+    for l in (1, 2):
+        k = a.size[l]
+        assert torch.equal(a.counts[l][:, :k], b.counts[l][:, :k])
+        assert torch.equal(a.radii[l][:, :k], b.radii[l][:, :k])
+        assert torch.equal(a.centers[l][:, :k], b.centers[l][:, :k])
