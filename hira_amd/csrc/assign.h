@@ -10,8 +10,9 @@ namespace hira {
 // Bucketing fused into an assignment launch (counts NULL: the launch only assigns).
 //   counts  (T, K)       zero when the round starts; counts[a] += 1 for every item assigned to a.  The
 //                        value the item's increment returned is its place in the bucket:
-//   members (T, K, kBucketCap)  the first kBucketCap items of every bucket, in order of arrival, and
-//   dists   (T, K, kBucketCap)  their distances (NULL: a Lloyd round, which asks for none)
+//   members (T, K, places)  the first `places` items of every bucket, in order of arrival, and
+//   dists   (T, K, places)  their distances (NULL: a Lloyd round, which asks for none)
+//   places_log2             bucket_places_log2 of the fan-out
 //   big     (T, K)       the buckets with more than kWaveBucket members, big_count (T) of them
 //   more    (T, n_c)     (centroid, item) of the items behind those, more_count (T) of them, their
 //   more_dist (T, n_c)   distances by item.  Such buckets are rare (a few seeds of a Lloyd round);
@@ -23,8 +24,14 @@ namespace hira {
 // Counters of trees (big_count, more_count, lost_count, zero, and the lists' lengths) lie kCounterStride apart: at
 // one address, or in one line of memory, an addition waits for the one before it (9 ns each; 8 x 1024
 // workgroups adding to eight neighbours took 67 us).
+// places = sixteen times the fan-out, the mean of a bucket, rounded up to a power of two between
+// kWaveBucket and kBucketCap: 128 bytes a key of workspace at fan-outs of 4, 8 and 16, 64 at 32, less than
+// 256 from 3 on.  (256 places whatever the fan-out took 512 bytes a key at 4 and 2 KiB at 1.  Eight times
+// the fan-out: what lies behind the places costs 8 x 20000 rows at a fan-out of 16 2 %.)
 constexpr int kBucketCap = 256;
 constexpr int kWaveBucket = 64;
+static_assert(kWaveBucket == 1 << 6 && kBucketCap == 1 << 8, "bucket_places_log2");
+static inline int bucket_places_log2(int bf) { return bf <= 4 ? 6 : bf <= 8 ? 7 : 8; }
 constexpr int kCounterStride = 32;
 struct AssignCounting {
     int32_t* counts;
@@ -38,6 +45,7 @@ struct AssignCounting {
     int32_t* lost;
     int32_t* lost_count;
     int32_t* zero;
+    int places_log2;
 };
 
 // item `it` of tree t was assigned to centroid k, at distance d (k < 0: to none)
@@ -48,10 +56,10 @@ __device__ __forceinline__ void count_item(const AssignCounting& ac, int t, int 
     }
     const size_t b = (size_t)t * K + k;
     const int pos = atomicAdd(&ac.counts[b], 1);
-    if (pos < kBucketCap) {
-        ac.members[b * kBucketCap + pos] = it;
-        if (ac.dists != nullptr) ac.dists[b * kBucketCap + pos] = d;
-        if (pos == kWaveBucket) ac.big[(size_t)t * K + atomicAdd(&ac.big_count[t * kCounterStride], 1)] = k;
+    if (pos == kWaveBucket) ac.big[(size_t)t * K + atomicAdd(&ac.big_count[t * kCounterStride], 1)] = k;
+    if (pos < 1 << ac.places_log2) {
+        ac.members[(b << ac.places_log2) + pos] = it;
+        if (ac.dists != nullptr) ac.dists[(b << ac.places_log2) + pos] = d;
     } else {  // (one atomic for the lanes of the wave that are here)
         const unsigned long long here = __ballot(1);
         const int lane = threadIdx.x & 63, leader = __ffsll((long long)here) - 1;

@@ -201,8 +201,8 @@ __global__ __launch_bounds__(256) void k_assign_simple(
 // ------------------------------------------------------------------------------------
 struct Buckets {
     int32_t* counts;          // (T, K); every kernel here leaves it zero for the round after it
-    const int32_t* members;   // (T, K, kBucketCap)
-    const float* dists;       // (T, K, kBucketCap)
+    const int32_t* members;   // (T, K, places)
+    const float* dists;       // (T, K, places)
     const int32_t* big;       // (T, K)
     const int32_t* big_count;   // (T)
     const int2* more;         // (T, n_c)
@@ -211,6 +211,9 @@ struct Buckets {
     int32_t* next_big_count;    // (T): the round after this one counts here; cleared by these kernels
     int32_t* next_more_count;   // (T): the same
     int32_t* unsure_count;      // (T): cleared by these kernels
+    int places_log2;
+    __device__ int places() const { return 1 << places_log2; }
+    __device__ size_t first(size_t b) const { return b << places_log2; }  // place of bucket b (of all trees)
 };
 
 // f(item) for the items of bucket k among entries [e0, e1) of those that do not lie in `members`;
@@ -235,7 +238,7 @@ __device__ __forceinline__ void for_more(const Buckets& b, int t, int n_c, int k
 // (kWaveBucket members at most; a workgroup per bucket spent its time on five barriers and on 224
 // idle threads).  The larger ones, which the assignment has listed, take a workgroup each; the
 // launch's first workgroups do those, so that the longest start first:
-//   up to kBucketCap    every thread ranks its member against all others
+//   up to its places    every thread ranks its member against all others
 //   more                a bit map of the members (means), a bitonic sorting network (packing)
 constexpr int kWaves = 4;  // of a workgroup of the per-bucket kernels
 static int large_blocks(int K) { return min(max(K / 8, 1), 256); }  // workgroups of a tree for large buckets
@@ -288,7 +291,7 @@ __device__ __forceinline__ void reset_round(const Buckets& b, int t) {  // (one 
 //    8 x 131072 items, beside a mean of 32): 8 x 32768 rows of 256 bytes 71 -> 39 us, 8 x 131072
 //    200 -> 125 us.
 // ------------------------------------------------------------------------------------
-constexpr int kMeanMap = 4096;  // words of a bit map of item ids, for buckets beyond kBucketCap
+constexpr int kMeanMap = 4096;  // words of a bit map of item ids, for buckets beyond their places
 constexpr int kMeanMapBits = kMeanMap * 32;
 
 template <typename T>
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
     if ((int)blockIdx.x >= large) {
         const int k = ((int)blockIdx.x - large) * kWaves + wave;
         if (k >= K) return;
-        uint32_t id = (uint32_t)bk.members[((size_t)t * K + k) * kBucketCap + lane];  // (garbage from m on)
+        uint32_t id = (uint32_t)bk.members[bk.first((size_t)t * K + k) + lane];  // (garbage from m on)
         const int m = __builtin_amdgcn_readfirstlane(bk.counts[(size_t)t * K + k]);
         if (m <= 0 || m > kWaveBucket) return;
         if (lane >= m) id = 0xffffffffu;
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
     for (int i = blockIdx.x; i < nbig; i += large) {  // uniform
         const int k = bk.big[(size_t)t * K + i];
         const int m = bk.counts[(size_t)t * K + k];
-        const int32_t* mem = bk.members + ((size_t)t * K + k) * kBucketCap;
+        const int32_t* mem = bk.members + bk.first((size_t)t * K + k);
         __syncthreads();
         if (tid == 0) reset_count(bk, t, k, K);
         const int r = tid / CPR, c = tid % CPR;
@@ -363,7 +366,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
                     }
                 }
         };
-        if (m <= kBucketCap) {
+        if (m <= bk.places()) {
             const int mine = tid < m ? mem[tid] : 0x7fffffff;
             s_small[tid] = mine;
             __syncthreads();
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
                     const int d = it - lo;
                     if (d >= 0 && d < kMeanMapBits) atomicOr(&s_ord[d >> 5], 1u << (d & 31));
                 };
-                if (tid < kBucketCap) mark(mem[tid]);
+                if (tid < bk.places()) mark(mem[tid]);
                 for_more(bk, t, n_c, k, 0, others, mark);
                 __syncthreads();
                 // thread `tid` owns the words [tid * per, (tid + 1) * per)
@@ -481,7 +484,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
         uint64_t mine = 0;
         if (k < K) {
             const size_t b = (size_t)t * K + k;
-            mine = key_of(bk.dists[b * kBucketCap + lane], bk.members[b * kBucketCap + lane]);  // (garbage from m on)
+            mine = key_of(bk.dists[bk.first(b) + lane], bk.members[bk.first(b) + lane]);  // (garbage from m on)
             m = __builtin_amdgcn_readfirstlane(bk.counts[b]);
             f = __builtin_amdgcn_readfirstlane(fill[b]);
             if (m > kWaveBucket) m = 0;
@@ -515,8 +518,8 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
         const int k = bk.big[(size_t)t * K + i];
         const size_t b = (size_t)t * K + k;
         const int m = bk.counts[b], f = fill[b];
-        const int32_t* mem = bk.members + b * kBucketCap;
-        const float* md = bk.dists + b * kBucketCap;
+        const int32_t* mem = bk.members + bk.first(b);
+        const float* md = bk.dists + bk.first(b);
         const float* more_d = bk.more_dist + (size_t)t * n_c;
         int32_t* my_slots = slots + b * bf + f;
         const int take = max(min(m, bf - f), 0);
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
             reset_count(bk, t, k, K);
             filled(k, f + take);
         }
-        if (m <= kBucketCap) {
+        if (m <= bk.places()) {
             const uint64_t own = tid < m ? key_of(md[tid], mem[tid]) : ~0ull;
             s_keys[tid] = own;
             __syncthreads();
@@ -543,8 +546,8 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
         // a time is searched for the bucket's items
         constexpr int kAcceptStep = kAcceptSort - kBucketCap - 64;
         const int others = bk.more_count[t * kCounterStride];
-        if (tid < kBucketCap) s_keys[tid] = key_of(md[tid], mem[tid]);
-        if (tid == 0) s_n = kBucketCap;
+        if (tid < bk.places()) s_keys[tid] = key_of(md[tid], mem[tid]);
+        if (tid == 0) s_n = bk.places();
         for (int e0 = 0; e0 < others; e0 += kAcceptStep) {
             __syncthreads();
             for_more(bk, t, n_c, k, e0, min(e0 + kAcceptStep, others),
@@ -562,7 +565,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
             auto again = [&](float d, int it) {
                 if (take == 0 || key_of(d, it) > last) nl[s_base + atomicAdd(&s_rej, 1)] = it;
             };
-            if (tid < kBucketCap) again(md[tid], mem[tid]);
+            if (tid < bk.places()) again(md[tid], mem[tid]);
             for_more(bk, t, n_c, k, 0, others, [&](int it) { again(more_d[it], it); });
         }
     }
@@ -851,8 +854,8 @@ static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
         b->open_ids = c.take<int32_t>((size_t)T * k1);
         b->open_count = c.take<int32_t>((size_t)T);
     }
-    b->members = c.take<int32_t>((size_t)T * k1 * kBucketCap);
-    b->dists = c.take<float>((size_t)T * k1 * kBucketCap);
+    b->members = c.take<int32_t>((size_t)T * k1 << bucket_places_log2(bf));
+    b->dists = c.take<float>((size_t)T * k1 << bucket_places_log2(bf));
     b->big = c.take<int32_t>((size_t)T * k1);
     b->more = c.take<int2>((size_t)T * n);
     b->more_dist = c.take<float>((size_t)T * n);
@@ -970,7 +973,7 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
         auto buckets = [&]() {
             const int now = round & 1, next = now ^ 1;
             return Buckets{w.counts, w.members, w.dists, w.big, big_count + now * ct, w.more, more_count + now * ct,
-                           w.more_dist, big_count + next * ct, more_count + next * ct, unsure_count};
+                           w.more_dist, big_count + next * ct, more_count + next * ct, unsure_count, bucket_places_log2(bf)};
         };
         auto assign_round = [&](const int32_t* list, const int32_t* lcnt, const int32_t* fill, bool packing,
                                 int32_t* zero, bool only_open, long long expected) -> int {
@@ -988,7 +991,8 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
             job.list = list;
             job.list_count = lcnt;
             job.counting = AssignCounting{w.counts, w.members, packing ? w.dists : nullptr, w.big,
-                                          big_count + (round & 1) * ct, w.more, more_count + (round & 1) * ct, w.more_dist, w.lost, lost_count, zero};
+                                          big_count + (round & 1) * ct, w.more, more_count + (round & 1) * ct, w.more_dist, w.lost, lost_count, zero,
+                                          bucket_places_log2(bf)};
             job.unsure = w.unsure;
             job.unsure_count = unsure_count;
             int rc = HIRA_OK;

@@ -130,3 +130,23 @@ def test_launch_plan_fills_the_compute_units():
     assert _partials_per_head(1, 131072, 4) == 128          # 256 tiles, one tree
     assert _partials_per_head(1, 8192, 4) == 16             # fewer tiles than compute units
     assert _partials_per_head(128, 32768, 4) == 4           # several rounds: 16 tiles a workgroup
+
+
+@pytest.mark.parametrize("bf", [1, 2, 4, 8, 10, 16, 32, 64])
+@pytest.mark.parametrize("dtype,dim", [(_lib.HIRA_F32, 36), (_lib.HIRA_BF16, 128)])
+def test_build_workspace_follows_the_number_of_keys(bf, dtype, dim):
+    """Bytes a key, beside the centroids themselves: lists and orders (48 bytes, and a slot a level),
+    places of the buckets (64 to 256, eight bytes each, sixteen times the fan-out in between)."""
+    from hira_amd.indexer.hip import level_sizes
+
+    n, trees = 1 << 20, 8
+    t = _lib.HiraTree()
+    t.num_trees, t.num_levels, t.bf, t.dim, t.vdim, t.dtype = trees, 2, bf, dim, dim, dtype
+    for l, s in enumerate(level_sizes(n, bf, 2)):
+        t.size[l] = t.cap[l] = s
+    need = _lib.lib().hira_build_workspace_bytes(ctypes.byref(t), n)
+    # per centroid: fp32, two sets of operand tiles (hi and lo bf16, columns padded to 32, and eight bytes), and
+    # counters; the tiles' number is rounded up to whole stages
+    centroid = dim * 4 + 2 * (4 * -(-dim // 32) * 32 + 8) + dim * 4 + 24
+    places = {1: 64, 2: 64, 4: 64, 8: 128}.get(bf, 256) * 8 / bf
+    assert 0 < need / (trees * n) < centroid / bf * 1.02 + 48 + places + 8

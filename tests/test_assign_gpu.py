@@ -88,3 +88,25 @@ def test_keys_that_are_no_numbers_keep_a_slot(dtype, n, d, bf, gpu_device):
     perm = index.perm[:, :-(-n // bf) * bf].cpu().numpy()
     for t in range(2):
         assert sorted(perm[t][perm[t] >= 0].tolist()) == list(range(n))
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 64), (torch.float32, 36)])
+@pytest.mark.parametrize("bf,places", [(1, 64), (4, 64), (5, 128), (8, 128), (9, 256), (32, 256), (64, 256)])
+@pytest.mark.parametrize("more", [-1, 0, 1, 3])
+def test_buckets_around_the_places_they_have(dtype, d, bf, places, more, gpu_device):
+    """The largest bucket one item below, at and beyond the places that a fan-out gives each."""
+    from hira_amd.indexer.hip import HIPIndexer
+
+    n = 70 * bf + 400
+    rng = np.random.default_rng(bf)
+    x = rng.integers(-4, 5, size=(1, n, d)).astype(np.float32)
+    x[:, 1:places + more] = x[:, :1]  # (row 0 is the first centroid)
+    keys = torch.from_numpy(x)[None].to(dtype)
+    index = HIPIndexer(2, 0, bf, seed=5).build(keys, keys.clone())
+    K = -(-n // bf)
+    want = _blocks(torch.from_numpy(x[0]).to(gpu_device).double(), K, bf, 5 + 7919, 0, 8)
+    np.testing.assert_array_equal(index.perm[0, :K * bf].cpu().numpy().reshape(K, bf), want)
+    # with Lloyd rounds: means over the same buckets, in a fixed order
+    a, b = (HIPIndexer(2, 2, bf, seed=5).build(keys, keys.clone()) for _ in range(2))
+    assert torch.equal(a.perm, b.perm) and torch.equal(a.radii[1], b.radii[1])
+    assert sorted(a.perm[a.perm >= 0].tolist()) == list(range(n))
