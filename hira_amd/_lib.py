@@ -17,7 +17,8 @@ HIRA_MAX_LEVELS = 8
 HIRA_STATS_COLS = HIRA_MAX_LEVELS + 3  # counters per tree a search can fill in
 HIRA_F32, HIRA_BF16 = 0, 1
 HIRA_ROW_MAJOR, HIRA_TILE16, HIRA_TILE16_Q8 = 0, 1, 2
-HIRA_ABI_VERSION = 8
+HIRA_ABI_VERSION = 9
+HIRA_UNIT_SCALE_HEADS = 4096
 
 _vp = C.c_void_p
 
@@ -105,6 +106,7 @@ def out_dtype_of(query: HiraQuery) -> C.c_int32:
 SYMBOLS = {
     "hira_abi_version": (C.c_int, []),
     "hira_last_error": (C.c_char_p, []),
+    "hira_unit_scale": (_vp, []),
     "hira_search_workspace_bytes": (
         C.c_size_t,
         [C.POINTER(HiraTree), C.POINTER(HiraQuery), C.POINTER(HiraQueue), C.POINTER(HiraLaunch)],

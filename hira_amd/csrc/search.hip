@@ -395,18 +395,19 @@ constexpr int kMaxDevices = 64;
 static __device__ __align__(256) unsigned char scratch[hira::kScratchBytes];
 static void* g_scratch_ptr[hira::kMaxDevices];  // per device; written once (same value from any thread)
 
-static int scratch_for_current_device(void** out) {
+// The device address of a symbol of this file on the current device, kept in `kept` (one per device).
+static int symbol_on_current_device(const void* symbol, const char* name, void** kept, void** out) {
     int dev = -1;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return fail(HIRA_ELAUNCH, "hipGetDevice: %s", hipGetErrorString(e));
     HIRA_CHECK_ARG(dev >= 0 && dev < kMaxDevices, "device %d: at most %d devices", dev, kMaxDevices);
-    void* ptr = __atomic_load_n(&g_scratch_ptr[dev], __ATOMIC_ACQUIRE);
+    void* ptr = __atomic_load_n(&kept[dev], __ATOMIC_ACQUIRE);
     if (ptr == nullptr) {
-        e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+        e = hipGetSymbolAddress(&ptr, symbol);
         if (e != hipSuccess || ptr == nullptr)
-            return fail(HIRA_ELAUNCH, "hipGetSymbolAddress(scratch) on device %d: %s", dev,
+            return fail(HIRA_ELAUNCH, "hipGetSymbolAddress(%s) on device %d: %s", name, dev,
                         hipGetErrorString(e));
-        __atomic_store_n(&g_scratch_ptr[dev], ptr, __ATOMIC_RELEASE);
+        __atomic_store_n(&kept[dev], ptr, __ATOMIC_RELEASE);
     }
     *out = ptr;
     return HIRA_OK;
@@ -416,7 +417,23 @@ extern "C" int hira_search_noalloc(const HiraTree* tree, const HiraQuery* query,
                                    const HiraQueue* queue, const HiraSearchOut* out,
                                    const HiraLaunch* launch, void* stream) {
     void* ptr = nullptr;
-    const int rc = scratch_for_current_device(&ptr);
+    const int rc = symbol_on_current_device(HIP_SYMBOL(scratch), "scratch", g_scratch_ptr, &ptr);
     if (rc != HIRA_OK) return rc;
     return search_impl(tree, query, queue, out, launch, ptr, kScratchBytes, kScratchCounters, stream);
+}
+
+// ---- a scale of one per head for callers that have none ----------------------------------------
+#define HIRA_ONES_8 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f
+#define HIRA_ONES_64 HIRA_ONES_8, HIRA_ONES_8, HIRA_ONES_8, HIRA_ONES_8, HIRA_ONES_8, HIRA_ONES_8, HIRA_ONES_8, HIRA_ONES_8
+#define HIRA_ONES_512 HIRA_ONES_64, HIRA_ONES_64, HIRA_ONES_64, HIRA_ONES_64, HIRA_ONES_64, HIRA_ONES_64, HIRA_ONES_64, HIRA_ONES_64
+static __device__ __align__(256) float unit_scale[] = {HIRA_ONES_512, HIRA_ONES_512, HIRA_ONES_512, HIRA_ONES_512,
+                                                       HIRA_ONES_512, HIRA_ONES_512, HIRA_ONES_512, HIRA_ONES_512};
+static_assert(sizeof(unit_scale) == HIRA_UNIT_SCALE_HEADS * sizeof(float), "a one per head");
+static void* g_unit_scale_ptr[hira::kMaxDevices];
+
+/* see include/hira_hip.h */
+extern "C" const float* hira_unit_scale(void) {
+    void* ptr = nullptr;
+    if (symbol_on_current_device(HIP_SYMBOL(unit_scale), "unit_scale", g_unit_scale_ptr, &ptr) != HIRA_OK) return nullptr;
+    return static_cast<const float*>(ptr);
 }

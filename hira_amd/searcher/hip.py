@@ -39,18 +39,19 @@ def _on(t: torch.Tensor, device) -> bool:
 
 class _Call:
     """What a call on one tree with one number of heads needs and does not change from call to
-    call: the C structs (only this thread fills them in), the head map, a scale of one per head,
-    the workspace's size.  Made on first use and kept by the searcher: a call that comes with ready
-    tensors (the storage type, on the index's device, contiguous) then allocates and copies nothing
-    and its host side is a handful of attribute reads around one library call (21 -> 8 us for
-    ``search``, 25 -> 11 us for ``search_attention``, which the kernels of small indexes are shorter
-    than)."""
+    call: the C structs (only this thread fills them in), the head map, the address of a scale of one
+    per head (the library's own; None: not asked for yet), the workspace's size.  Made on first use and
+    kept by the searcher: a call that comes with ready tensors (the storage type, on the index's device,
+    contiguous) then allocates and copies nothing and its host side is a handful of attribute reads
+    around one library call (21 -> 8 us for ``search``, 25 -> 11 us for ``search_attention``, which the
+    kernels of small indexes are shorter than).  That holds from the second call on a tree whose level
+    sizes stay: the first on an index, and the first after an append that moved them, makes it anew."""
 
     __slots__ = ("tree", "query", "out", "queue", "dev", "keep", "ones", "ws_bytes", "ws_rows",
                  "tree_ref", "query_ref", "out_ref", "queue_ref", "launch_ref")
 
-    def __init__(self, tree, launch, query, dev, keep, ones):
-        self.tree, self.query, self.dev, self.keep, self.ones = tree, query, dev, keep, ones
+    def __init__(self, tree, launch, query, dev, keep):
+        self.tree, self.query, self.dev, self.keep, self.ones = tree, query, dev, keep, None
         self.out = _lib.HiraSearchOut()
         self.queue = _lib.HiraQueue()
         self.ws_bytes, self.ws_rows = 0, -1  # the workspace, and the queue rows it was sized for
@@ -193,7 +194,7 @@ class HIPSearcher(BaseSearcher):
                     if len(self._calls) >= self._MAX_CALLS:
                         self._calls.clear()
                     c = self._calls[key] = _Call(tree, self.launch, qs, indexer.keys_buf.get_device(),
-                                                 (off, heads), None)
+                                                 (off, heads))
                 if query.get_device() == c.dev:
                     dev, qs = c.dev, c.query
                     if isinstance(threshold, torch.Tensor) and threshold.dtype is torch.float32 and \
@@ -202,30 +203,30 @@ class HIPSearcher(BaseSearcher):
                         tau = threshold
                     else:
                         tau = self._coerce_threshold(threshold, h_q, indexer.device)
+                    one = None
                     if scaling is None:
-                        sc = c.ones
-                        if sc is None:
-                            sc = self._scale_of_one(c, h_q, indexer.keys_buf.device)
+                        one = c.ones or self._unit_scale(c, h_q)
+                        sc = None if one else self._coerce_scaling(None, h_q, indexer.device)
                     elif isinstance(scaling, torch.Tensor) and scaling.dtype is torch.float32 and \
                             scaling.numel() == h_q and scaling.get_device() == dev and \
                             scaling.is_contiguous():
                         sc = scaling
                     else:
                         sc = self._coerce_scaling(scaling, h_q, indexer.device)
-                    qs.q, qs.tau, qs.scaling = query.data_ptr(), tau.data_ptr(), sc.data_ptr()
+                    qs.q, qs.tau, qs.scaling = query.data_ptr(), tau.data_ptr(), one or sc.data_ptr()
                     return c, h_q, (query, tau, sc)
         qs, keep = self._query_struct(query, threshold, indexer, q_head_to_kv, scaling)
-        return (_Call(tree, self.launch, qs, indexer.keys_buf.get_device(), keep, None),
+        return (_Call(tree, self.launch, qs, indexer.keys_buf.get_device(), keep),
                 qs.num_q_heads, keep)
 
     @staticmethod
-    def _scale_of_one(c: _Call, h_q: int, device) -> torch.Tensor:
-        """A scale of one per head, kept with the call description -- through the host: the copy is
-        complete for every stream when it returns.  A call that is being captured takes one of the
-        graph's own."""
-        if torch.cuda.is_current_stream_capturing():
-            return torch.ones((h_q,), dtype=torch.float32, device=device)
-        c.ones = torch.ones((h_q,), dtype=torch.float32).to(device)
+    def _unit_scale(c: _Call, h_q: int) -> Optional[int]:
+        """Address of the library's scale of one per head, or None: more heads than it holds, or a
+        capture is the first to ask on this device (then a tensor of the call's own is used)."""
+        if c.dev < 0 or h_q > _lib.HIRA_UNIT_SCALE_HEADS or torch.cuda.is_current_stream_capturing():
+            return None
+        with torch.cuda.device(c.dev):
+            c.ones = _lib.lib().hira_unit_scale()
         return c.ones
 
     def _get_workspace(self, nbytes: int, device) -> torch.Tensor:

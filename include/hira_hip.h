@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define HIRA_ABI_VERSION 8
+#define HIRA_ABI_VERSION 9
 #define HIRA_MAX_LEVELS 8
 #define HIRA_STATS_COLS (HIRA_MAX_LEVELS + 3) /* counters per tree a search can fill in */
 
@@ -164,6 +164,12 @@ typedef struct HiraLaunch {
 
 int hira_abi_version(void);
 const char* hira_last_error(void);
+
+/* Device address of HIRA_UNIT_SCALE_HEADS ones on the current device, for HiraQuery.scaling where the
+ * caller has no scale: part of the library's device image, so complete for every stream and there
+ * until the process ends.  NULL on failure (hira_last_error). */
+#define HIRA_UNIT_SCALE_HEADS 4096
+const float* hira_unit_scale(void);
 
 /* Bytes of workspace hira_search needs for this tree/query (arrival counters, one per tree
  * and head pass, at the start; attention partials after them).  The workspace must be ZERO

@@ -70,3 +70,14 @@ def test_no_kernel_is_launched_over_host_memory():
         _lib.stream_of(-1)
     with pytest.raises(ValueError, match="GPU"):
         _lib.current_stream(torch.device("cpu"))
+
+
+def test_no_search_is_launched_over_host_memory():
+    from hira_amd.searcher.hip import HIPSearcher
+
+    a = HIPIndexer.from_layout(device="cpu", layout="row_major", **_parts(torch.float32))
+    q, tau = torch.zeros((4, 64)), torch.zeros((4,))
+    for call in (HIPSearcher().search, HIPSearcher().search_attention, HIPSearcher().search_compact):
+        for scaling in (None, torch.ones(4)):
+            with pytest.raises(ValueError, match="GPU"):
+                call(q, tau, a, scaling=scaling)

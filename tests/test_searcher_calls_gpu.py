@@ -1,0 +1,58 @@
+"""What HIPSearcher keeps between calls: no wait where an index has grown, launch options and outputs as
+they are at the time of the call."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _index(n=3000, d=64, dtype=torch.float32, trees=2, seed=0, **kw):
+    from hira_amd.indexer import HIPIndexer
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    k, v = (torch.randn((1, trees, n, d), generator=g, device="cuda").to(dtype) for _ in range(2))
+    return HIPIndexer(3, 1, 8, **kw).build(k, v), g
+
+
+def test_a_search_without_a_scale_does_not_wait(gpu_device):
+    from hira_amd.searcher import HIPSearcher
+
+    idx, g = _index()
+    idx.reserve(100)
+    q, tau = torch.randn((4, 64), generator=g, device="cuda"), torch.full((4,), 8.0, device="cuda")
+    new = torch.randn((1, 2, 1, 64), generator=g, device="cuda")
+    se = HIPSearcher()
+    for call in (lambda: se.search(q, tau, idx), lambda: se.search_attention(q, tau, idx)):
+        call()
+        idx.update(new, new, sync=False)
+        call()  # (code and memory of a first call)
+        torch.cuda.synchronize()
+        size = list(idx.size)
+        while idx.size == size:  # appends until the level sizes, and with them the call, are others
+            idx.update(new, new, sync=False)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(1_000_000_000)
+        slept = torch.cuda.Event()
+        slept.record()
+        got = call()
+        assert not slept.query(), "the host waited for what was enqueued before the search"
+        torch.cuda.synchronize()
+        want = HIPSearcher()
+        ones = torch.ones((4,), device="cuda")
+        ref = want.search(q, tau, idx, scaling=ones) if got.shape[1] == idx.size[0] else \
+            want.search_attention(q, tau, idx, scaling=ones)
+        assert torch.equal(got, ref) and bool((got != 0).any())
+
+
+@pytest.mark.parametrize("trees,group", [(2, 4), (512, 8), (512, 9)])  # 8, 4096 and 4608 heads
+def test_a_missing_scale_is_one(trees, group, gpu_device):
+    from hira_amd.searcher import HIPSearcher
+
+    idx, g = _index(n=40, trees=trees)
+    h = trees * group
+    q, tau = torch.randn((h, 64), generator=g, device="cuda"), torch.full((h,), 3.0, device="cuda")
+    ones = torch.ones((h,), device="cuda")
+    for _ in range(2):
+        a = HIPSearcher()
+        assert torch.equal(a.search(q, tau, idx).clone(), HIPSearcher().search(q, tau, idx, scaling=ones))
+        assert torch.equal(a.search_attention(q, tau, idx), a.search_attention(q, tau, idx, scaling=ones))
