@@ -47,16 +47,17 @@ class _Call:
     kernels of small indexes are shorter than).  That holds from the second call on a tree whose level
     sizes stay: the first on an index, and the first after an append that moved them, makes it anew."""
 
-    __slots__ = ("tree", "query", "out", "queue", "dev", "keep", "ones", "ws_bytes", "ws_rows",
-                 "tree_ref", "query_ref", "out_ref", "queue_ref", "launch_ref")
+    __slots__ = ("tree", "query", "out", "queue", "dev", "keep", "ones", "ws_bytes", "ws_for",
+                 "launch", "tree_ref", "query_ref", "out_ref", "queue_ref", "launch_ref")
 
-    def __init__(self, tree, launch, query, dev, keep):
+    def __init__(self, tree, query, dev, keep):
         self.tree, self.query, self.dev, self.keep, self.ones = tree, query, dev, keep, None
         self.out = _lib.HiraSearchOut()
         self.queue = _lib.HiraQueue()
-        self.ws_bytes, self.ws_rows = 0, -1  # the workspace, and the queue rows it was sized for
+        self.ws_bytes, self.ws_for = 0, (-1, b"")  # the workspace; the queue rows and launch options it is for
         self.tree_ref, self.query_ref = C.byref(tree), C.byref(query)
-        self.out_ref, self.queue_ref, self.launch_ref = C.byref(self.out), C.byref(self.queue), C.byref(launch)
+        self.out_ref, self.queue_ref = C.byref(self.out), C.byref(self.queue)
+        self.launch = self.launch_ref = None
 
 
 class HIPSearcher(BaseSearcher):
@@ -193,8 +194,7 @@ class HIPSearcher(BaseSearcher):
                     qs = _lib.HiraQuery(h_q, None, None, None, off.data_ptr(), heads.data_ptr(), gmax, group)
                     if len(self._calls) >= self._MAX_CALLS:
                         self._calls.clear()
-                    c = self._calls[key] = _Call(tree, self.launch, qs, indexer.keys_buf.get_device(),
-                                                 (off, heads))
+                    c = self._calls[key] = _Call(tree, qs, indexer.keys_buf.get_device(), (off, heads))
                 if query.get_device() == c.dev:
                     dev, qs = c.dev, c.query
                     if isinstance(threshold, torch.Tensor) and threshold.dtype is torch.float32 and \
@@ -216,8 +216,7 @@ class HIPSearcher(BaseSearcher):
                     qs.q, qs.tau, qs.scaling = query.data_ptr(), tau.data_ptr(), one or sc.data_ptr()
                     return c, h_q, (query, tau, sc)
         qs, keep = self._query_struct(query, threshold, indexer, q_head_to_kv, scaling)
-        return (_Call(tree, self.launch, qs, indexer.keys_buf.get_device(), keep),
-                qs.num_q_heads, keep)
+        return (_Call(tree, qs, indexer.keys_buf.get_device(), keep), qs.num_q_heads, keep)
 
     @staticmethod
     def _unit_scale(c: _Call, h_q: int) -> Optional[int]:
@@ -251,11 +250,15 @@ class HIPSearcher(BaseSearcher):
         lib = _lib.lib()
         ws_ptr, ws_bytes = None, 0
         queue_ref = c.queue_ref if queue_rows else None
+        launch = self.launch  # (as it is now: callers may replace it, or change its fields)
+        if c.launch is not launch:
+            c.launch, c.launch_ref = launch, C.byref(launch)
         if attn:
-            if queue_rows > c.ws_rows:  # (more rows in the queue may mean more partials)
-                c.ws_rows = queue_rows
-                c.ws_bytes = lib.hira_search_workspace_bytes(c.tree_ref, c.query_ref, queue_ref,
-                                                             c.launch_ref)
+            rows, options = c.ws_for
+            now = bytes(launch)
+            if queue_rows > rows or options != now:  # (more rows in the queue may mean more partials)
+                c.ws_for = queue_rows, now
+                c.ws_bytes = lib.hira_search_workspace_bytes(c.tree_ref, c.query_ref, queue_ref, c.launch_ref)
             ws_bytes = c.ws_bytes
             ws = self._workspace
             if ws is None or ws.get_device() != c.dev or ws.numel() < ws_bytes:

@@ -56,3 +56,27 @@ def test_a_missing_scale_is_one(trees, group, gpu_device):
         a = HIPSearcher()
         assert torch.equal(a.search(q, tau, idx).clone(), HIPSearcher().search(q, tau, idx, scaling=ones))
         assert torch.equal(a.search_attention(q, tau, idx), a.search_attention(q, tau, idx, scaling=ones))
+
+
+def test_launch_options_are_those_of_the_call(gpu_device):
+    from hira_amd import _lib
+    from hira_amd.searcher import HIPSearcher
+
+    idx, g = _index(n=9000, layout="row_major")
+    q, tau = torch.randn((8, 64), generator=g, device="cuda"), torch.full((8,), 12.0, device="cuda")
+    sc = torch.full((8,), 0.125, device="cuda")
+    se = HIPSearcher(nodes_per_wave=200)
+    ref = se.search_attention(q, tau, idx, scaling=sc).clone()
+    dense = se.search(q, tau, idx, scaling=sc).clone()
+    se.launch.nodes_per_wave = 1  # many more partials: a larger workspace
+    assert torch.allclose(se.search_attention(q, tau, idx, scaling=sc), ref, rtol=1e-4, atol=1e-5)
+    se.launch = _lib.HiraLaunch(64, 1, 1, 1)  # the same, folded by a second launch
+    st = torch.zeros((2, _lib.HIRA_STATS_COLS), dtype=torch.int64, device="cuda")
+    assert torch.allclose(se.search_attention(q, tau, idx, scaling=sc, stats=st), ref, rtol=1e-4, atol=1e-5)
+    assert torch.equal(se.search(q, tau, idx, scaling=sc), dense)
+    se.launch.kernel = 3
+    for call in (se.search, se.search_attention):
+        with pytest.raises(ValueError, match="kernel"):
+            call(q, tau, idx, scaling=sc)
+    se.launch = _lib.HiraLaunch(0, 0, 0, 0)
+    assert torch.allclose(se.search_attention(q, tau, idx, scaling=sc), ref, rtol=1e-4, atol=1e-5)
