@@ -111,6 +111,9 @@ SYMBOLS = {
         C.c_size_t,
         [C.POINTER(HiraTree), C.POINTER(HiraQuery), C.POINTER(HiraQueue), C.POINTER(HiraLaunch)],
     ),
+    "hira_search_counter_bytes": (
+        C.c_size_t, [C.POINTER(HiraTree), C.POINTER(HiraQuery), C.POINTER(HiraLaunch)],
+    ),
     "hira_search": (
         C.c_int,
         [C.POINTER(HiraTree), C.POINTER(HiraQuery), C.POINTER(HiraQueue),

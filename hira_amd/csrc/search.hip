@@ -226,6 +226,13 @@ extern "C" size_t hira_search_workspace_bytes(const HiraTree* tree, const HiraQu
     return workspace_need(query->num_q_heads, P, tree->vdim, tree->num_trees, plan.head_chunks);
 }
 
+/* see include/hira_hip.h */
+extern "C" size_t hira_search_counter_bytes(const HiraTree* tree, const HiraQuery* query, const HiraLaunch* launch) {
+    SearchPlan plan;
+    if (make_plan(tree, query, nullptr, launch, true, &plan) != HIRA_OK) return 0;
+    return counter_bytes(tree->num_trees, plan.head_chunks);
+}
+
 // The search behind both entry points.  Attention needs arrival counters (one int32 per tree
 // and head pass, zero between calls) and room for the partials; `fixed_counters` > 0: the
 // counters live in a region of that many entries of their own (the entry point that allocates

@@ -25,6 +25,10 @@ from .base import BaseSearcher
 
 DEFAULT_OUTPUT_FILL_VALUE = 0.0
 
+# The workspace's first bytes hold nothing but arrival counters, zero between calls, whatever index a
+# call is on: its counters end where this part ends (16384 trees x passes of heads).
+_COUNTERS = 64 * 1024
+
 
 def _on(t: torch.Tensor, device) -> bool:
     """Is tensor `t` on `device`?  ("cuda" without an index means the current device, which a
@@ -47,14 +51,15 @@ class _Call:
     kernels of small indexes are shorter than).  That holds from the second call on a tree whose level
     sizes stay: the first on an index, and the first after an append that moved them, makes it anew."""
 
-    __slots__ = ("tree", "query", "out", "queue", "dev", "keep", "ones", "ws_bytes", "ws_for",
+    __slots__ = ("tree", "query", "out", "queue", "dev", "keep", "ones", "ws_bytes", "ws_at", "ws_for",
                  "launch", "tree_ref", "query_ref", "out_ref", "queue_ref", "launch_ref")
 
     def __init__(self, tree, query, dev, keep):
         self.tree, self.query, self.dev, self.keep, self.ones = tree, query, dev, keep, None
         self.out = _lib.HiraSearchOut()
         self.queue = _lib.HiraQueue()
-        self.ws_bytes, self.ws_for = 0, (-1, b"")  # the workspace; the queue rows and launch options it is for
+        # the workspace and the place in it; the queue rows and launch options it is for
+        self.ws_bytes, self.ws_at, self.ws_for = 0, 0, (-1, b"")
         self.tree_ref, self.query_ref = C.byref(tree), C.byref(query)
         self.out_ref, self.queue_ref = C.byref(self.out), C.byref(self.queue)
         self.launch = self.launch_ref = None
@@ -259,11 +264,15 @@ class HIPSearcher(BaseSearcher):
             if queue_rows > rows or options != now:  # (more rows in the queue may mean more partials)
                 c.ws_for = queue_rows, now
                 c.ws_bytes = lib.hira_search_workspace_bytes(c.tree_ref, c.query_ref, queue_ref, c.launch_ref)
-            ws_bytes = c.ws_bytes
+                c.ws_at = _COUNTERS - lib.hira_search_counter_bytes(c.tree_ref, c.query_ref, c.launch_ref)
+            ws_bytes, at = c.ws_bytes, c.ws_at
             ws = self._workspace
-            if ws is None or ws.get_device() != c.dev or ws.numel() < ws_bytes:
-                ws = self._get_workspace(ws_bytes, indexer.device)
-            ws_ptr = ws.data_ptr()
+            if at < 0:  # more counters than are kept apart: a workspace of the call's own
+                at = 0
+                ws = torch.zeros(ws_bytes, dtype=torch.uint8, device=indexer.device)
+            elif ws is None or ws.get_device() != c.dev or ws.numel() < at + ws_bytes:
+                ws = self._get_workspace(at + ws_bytes, indexer.device)
+            ws_ptr = ws.data_ptr() + at
         rc = lib.hira_search(c.tree_ref, c.query_ref, queue_ref, c.out_ref, c.launch_ref, ws_ptr,
                              ws_bytes, _lib.stream_of(c.dev))
         if rc:

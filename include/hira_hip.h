@@ -176,8 +176,12 @@ const float* hira_unit_scale(void);
  * before its first use; every completed call leaves the counters zero again, and they sit
  * at an offset that depends only on the number of trees and head passes, so a workspace can
  * be reused without clearing by any later call with the same trees and heads that needs no
- * more bytes (a tree that grew, a queue that came or went).  Two calls that may run
- * concurrently need separate workspaces. */
+ * more bytes (a tree that grew, a queue that came or went).  Calls with other numbers of
+ * trees or head passes have partials where this one has counters: they share a workspace if
+ * hira_search_counter_bytes, the counters' part of these bytes, is the same for both, or if each is
+ * given the address that lies that far below one place where the partials of all begin.  Two calls that
+ * may run concurrently need separate workspaces. */
+size_t hira_search_counter_bytes(const HiraTree* tree, const HiraQuery* query, const HiraLaunch* launch);
 size_t hira_search_workspace_bytes(const HiraTree* tree, const HiraQuery* query,
                                    const HiraQueue* queue, const HiraLaunch* launch);
 

@@ -80,3 +80,21 @@ def test_launch_options_are_those_of_the_call(gpu_device):
             call(q, tau, idx, scaling=sc)
     se.launch = _lib.HiraLaunch(0, 0, 0, 0)
     assert torch.allclose(se.search_attention(q, tau, idx, scaling=sc), ref, rtol=1e-4, atol=1e-5)
+
+
+def test_one_searcher_serves_indexes_of_any_number_of_trees(gpu_device):
+    """The arrival counters of many trees lie where the partials of few did not write."""
+    from hira_amd.searcher import HIPSearcher
+
+    few, g = _index(n=9000, trees=2)
+    many = [_index(n=n, trees=t, seed=t)[0] for t, n in ((300, 200), (96, 700), (9000, 40))]  # (18000 counters)
+    se = HIPSearcher()
+    for kernel in (0, 1):
+        for idx in [few, many[0], few, many[1], many[2], many[0]]:
+            h = idx.num_trees * 9
+            q, tau = torch.randn((h, 64), generator=g, device="cuda"), torch.full((h,), 6.0, device="cuda")
+            sc = torch.full((h,), 0.125, device="cuda")
+            se.launch.kernel = kernel
+            out = torch.full((h, 64), 7.0, device="cuda")
+            se.search_attention(q, tau, idx, scaling=sc, out=out)
+            assert torch.equal(out, HIPSearcher(kernel=kernel).search_attention(q, tau, idx, scaling=sc))
