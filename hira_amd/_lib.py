@@ -48,8 +48,12 @@ class HiraTree(C.Structure):
 
 
 class HiraQuery(C.Structure):
+    """`out_dtype` (HIRA_F32 or HIRA_BF16: the type hira_search writes attn_out in) lies in what was
+    padding once, and comes last by position: structs filled in by position keep their meaning."""
+
     _fields_ = [
         ("num_q_heads", C.c_int32),
+        ("out_dtype", C.c_int32),
         ("q", _vp),
         ("tau", _vp),
         ("scaling", _vp),
@@ -58,6 +62,11 @@ class HiraQuery(C.Structure):
         ("max_group", C.c_int32),
         ("group_size", C.c_int32),
     ]
+
+    def __init__(self, num_q_heads=0, q=None, tau=None, scaling=None, tree_q_off=None, tree_q_heads=None,
+                 max_group=0, group_size=0, out_dtype=HIRA_F32):
+        super().__init__(num_q_heads, out_dtype, q, tau, scaling, tree_q_off, tree_q_heads, max_group,
+                         group_size)
 
 
 class HiraQueue(C.Structure):
@@ -93,13 +102,6 @@ class HiraArray(C.Structure):
     _fields_ = [("dst", _vp), ("src", _vp), ("dst_stride", C.c_int64), ("src_stride", C.c_int64),
                 ("copy_bytes", C.c_int64), ("fill_from", C.c_int64), ("fill", C.c_uint32),
                 ("reserved_", C.c_int32)]
-
-
-def out_dtype_of(query: HiraQuery) -> C.c_int32:
-    """The struct's `out_dtype` (HIRA_F32 or HIRA_BF16: the type hira_search writes attn_out in).
-    It lies between `num_q_heads` and `q`, in what was padding before; ``_fields_`` leaves it out so
-    that structs filled in by position keep their meaning."""
-    return C.c_int32.from_buffer(query, 4)
 
 
 # every symbol include/hira_hip.h declares: (restype, argtypes)

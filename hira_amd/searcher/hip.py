@@ -41,6 +41,23 @@ def _on(t: torch.Tensor, device) -> bool:
     return t.device.index == device.index
 
 
+_OUT_TYPES = {torch.float32: _lib.HIRA_F32, torch.bfloat16: _lib.HIRA_BF16}
+
+
+def _refuse_out(out: torch.Tensor):
+    raise ValueError(f"out is {out.dtype}: attention is written as float32, or rounded once to bfloat16")
+
+
+def _out_type(out: torch.Tensor, numel: int, dev: int) -> int:
+    """The type that attention is written to `out` in; ValueError where it cannot be written there."""
+    if out.dtype not in _OUT_TYPES:
+        _refuse_out(out)
+    if out.numel() < numel or out.get_device() != dev or not out.is_contiguous():
+        raise ValueError(f"out {tuple(out.shape)} on {out.device}: expected {numel} numbers or more, contiguous, "
+                         "on the index's device")
+    return _OUT_TYPES[out.dtype]
+
+
 class _Call:
     """What a call on one tree with one number of heads needs and does not change from call to
     call: the C structs (only this thread fills them in), the head map, the address of a scale of one
@@ -330,7 +347,7 @@ class HIPSearcher(BaseSearcher):
                          indexer, q_head_to_kv=None, scaling=None,
                          out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """softmax(scaling * score) V over given lists (``search_compact`` in the slot index
-        space, possibly edited): index (H_q, cap) int32 key slots, score (H_q, cap) fp32 raw
+        space, possibly edited), fp32: index (H_q, cap) int32 key slots, score (H_q, cap) fp32 raw
         q.k, count (H_q,) int32.  Returns (H_q, Dv) fp32; zeros where a list is empty."""
         if indexer.values_buf is None:
             raise ValueError("the index was built without values: nothing to attend to")
@@ -348,6 +365,8 @@ class HIPSearcher(BaseSearcher):
                             gmax, group)
         if out is None:
             out = torch.empty((h_q, indexer.vdim), dtype=torch.float32, device=dev)
+        elif _out_type(out, h_q * indexer.vdim, indexer.keys_buf.get_device()) != _lib.HIRA_F32:
+            raise ValueError("sparse_attention writes float32")
         tree = indexer.tree_struct()
         stream = _lib.current_stream(dev)
         _lib.check(_lib.lib().hira_sparse_attention(
@@ -361,12 +380,16 @@ class HIPSearcher(BaseSearcher):
                          out: Optional[torch.Tensor] = None,
                          stats: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Fused search + softmax(scaling * q.K_S^T) V_S over the selected keys and, when
-        given, every queued key (T, m, D) / value (T, m, Dv).  Returns (H_q, Dv) fp32."""
+        given, every queued key (T, m, D) / value (T, m, Dv).  Returns (H_q, Dv) fp32, or ``out``:
+        contiguous, fp32 or bf16 (the fp32 sums are then rounded where they are written)."""
         if indexer.values_buf is None:
             raise ValueError("the index was built without values: nothing to attend to")
         c, h_q, keep = self._call(query, threshold, indexer, q_head_to_kv, scaling)
         if out is None:
             out = torch.empty((h_q, indexer.vdim), dtype=torch.float32, device=indexer.keys_buf.device)
+            c.query.out_dtype = _lib.HIRA_F32
+        else:
+            c.query.out_dtype = _out_type(out, h_q * indexer.vdim, c.dev)
         so = c.out
         so.dense = so.sel_index = so.sel_score = so.sel_count = None
         so.dense_by_position = so.dense_fill = 0
@@ -435,7 +458,6 @@ class DecodePlan:
         self._keep = (off, heads, stats)
         self.query = _lib.HiraQuery(num_q_heads, None, None, self.scaling.data_ptr(),
                                     off.data_ptr(), heads.data_ptr(), gmax, group)
-        self._out_type = _lib.out_dtype_of(self.query)
         self.out = _lib.HiraSearchOut()
         self.out.stats = None if stats is None else stats.data_ptr()
         self.launch = searcher.launch
@@ -478,7 +500,7 @@ class DecodePlan:
         q.q = query.data_ptr()
         q.tau = threshold.data_ptr()
         self.out.attn_out = out.data_ptr()
-        self._out_type.value = _lib.HIRA_BF16 if out.dtype is torch.bfloat16 else _lib.HIRA_F32
+        q.out_dtype = _OUT_TYPES[out.dtype] if out.dtype in _OUT_TYPES else _refuse_out(out)
         if stream is None:
             stream = _lib.stream_of(self._dev)
         qu = None

@@ -65,6 +65,15 @@ def test_struct_layout_matches_header():
     assert ctypes.sizeof(_lib.HiraSearchOut) == 72
 
 
+def test_query_by_position_and_by_name():
+    q = _lib.HiraQuery(4, 1, 2, 3, 5, 6, 7, 8)
+    assert (q.num_q_heads, q.out_dtype, q.q, q.tau, q.scaling, q.tree_q_off, q.tree_q_heads, q.max_group,
+            q.group_size) == (4, _lib.HIRA_F32, 1, 2, 3, 5, 6, 7, 8)
+    assert _lib.HiraQuery(out_dtype=_lib.HIRA_BF16).out_dtype == _lib.HIRA_BF16
+    assert _lib.HiraQuery.out_dtype.offset == 4 and _lib.HiraQuery.q.offset == 8
+    assert ctypes.sizeof(_lib.HiraQuery) == 56
+
+
 def test_new_entry_points_validate_without_a_gpu():
     """hira_threshold and hira_sparse_attention reject bad arguments before any launch."""
     lib = _lib.lib()

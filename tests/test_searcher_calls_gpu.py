@@ -98,3 +98,34 @@ def test_one_searcher_serves_indexes_of_any_number_of_trees(gpu_device):
             out = torch.full((h, 64), 7.0, device="cuda")
             se.search_attention(q, tau, idx, scaling=sc, out=out)
             assert torch.equal(out, HIPSearcher(kernel=kernel).search_attention(q, tau, idx, scaling=sc))
+
+
+@pytest.mark.parametrize("layout", ["row_major", "tiled"])
+def test_output_of_the_callers_own(layout, gpu_device):
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    g = torch.Generator(device="cuda").manual_seed(1)
+    k = torch.randn((1, 2, 3000, 64), generator=g, device="cuda").to(torch.bfloat16)
+    idx = HIPIndexer(3, 1, 16, layout=layout).build(k, k)
+    q, tau = torch.randn((8, 64), generator=g, device="cuda").to(torch.bfloat16), torch.full((8,), 12.0, device="cuda")
+    sc = torch.full((8,), 0.125, device="cuda")
+    se = HIPSearcher()
+    ref = se.search_attention(q, tau, idx, scaling=sc)
+    out = torch.full((2, 8, 64), 7.0, dtype=torch.bfloat16, device="cuda")  # (twice as much as is written)
+    assert se.search_attention(q, tau, idx, scaling=sc, out=out) is out
+    assert torch.equal(out[0], ref.to(torch.bfloat16)) and bool((out[1] == 7.0).all())
+    assert torch.equal(se.search_attention(q, tau, idx, scaling=sc), ref)  # (fp32 again)
+    assert torch.equal(se.search_attention(q, tau, idx, scaling=sc, out=torch.empty_like(ref)), ref)
+    lists = se.search_compact(q, tau, idx)
+    plan = se.plan_attention(idx, 8, scaling=sc)
+    for bad in (torch.empty((8, 64), dtype=torch.float16, device="cuda"), torch.empty((8, 64)),
+                torch.empty((8, 63), device="cuda"), torch.empty((64, 8), device="cuda").t()):
+        with pytest.raises(ValueError):
+            se.search_attention(q, tau, idx, scaling=sc, out=bad)
+        with pytest.raises(ValueError):
+            se.sparse_attention(*lists, idx, scaling=sc, out=bad)
+    with pytest.raises(ValueError):
+        se.sparse_attention(*lists, idx, scaling=sc, out=out)
+    with pytest.raises(ValueError):
+        plan.run(q, tau, torch.empty((8, 64), dtype=torch.float16, device="cuda"))
