@@ -12,7 +12,9 @@
 //   scan    the survivors' key slots, end to end, are dealt out over the waves in blocks of up to 64
 //           rows; the values of a block's selected rows are asked for together.
 // So a launch is a chain of four trips to memory (arguments, gates, keys, values) plus the hand-off
-// of the partials, whatever the fan-out, and a pruned node costs nothing behind its gate.  No
+// of the partials, whatever the fan-out, and a pruned node costs nothing behind its gate.  (4 trees x
+// 5003 rows of 80 fp32, three heads, as the work falls away: 15.6 us; with a key a head selected 13.4;
+// with every node pruned 10.6; without the attention 8.8, 8.6 and 5.6.)  No
 // global frontier is exchanged between workgroups.  (Before, every wave walked nodes of its own:
 // each gate repeated the ancestors' rows, and short nodes left most lanes without a row.)
 //
