@@ -29,6 +29,7 @@ namespace hira {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 abf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float af32x4_t;
+typedef __attribute__((ext_vector_type(8))) float af32x8_t;
 
 constexpr int kAssignRI = 4;       // operand tiles of 16 items per wave
 constexpr int kAssignThreads = 256;
@@ -424,8 +425,10 @@ __global__ __launch_bounds__(kSplitThreads, 2) void k_assign_split(const AssignJ
 // four centroids of ONE item, so best and second are one pair per item tile instead of four, and the
 // start values are a 16-byte read from LDS.
 // What bounds it is the matrix cores: 8 x 131072 items x 4096 centroids take 1690-1740 us with the
-// exact kernel and 890 us with this one, 1010 us where the distances are asked for (1.2 PFLOP/s, what
-// a large matrix product reaches on this card); 8 x 32768 x 1024: 165 -> 84 / 114 us.
+// exact kernel and 875 us with this one, 950 us where the distances are asked for; 8 x 32768 x 1024:
+// 165 -> 80 / 89 us.  Of a workgroup's 102 / 111 us its walk of the tiles takes 90 (1.5 PFLOP/s; a large
+// matrix product reaches 1.6 on this card), its items 6, its end 6 / 12.  (930 / 1060 us with a barrier every
+// 64 products of a wave and an end that looked rows up in operand tiles.)
 constexpr float kNoScore = -1e37f;  // start value of a centroid that takes no items
 constexpr int kMaxTagBits = 14;     // centroid numbers inside a lane: Kt * 4 of them
 
@@ -436,23 +439,24 @@ __device__ __forceinline__ void load_to_lds(const uint4* src, uint4* dst) {
                                      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 // (ahead of the barrier behind which the others read them)
-__device__ __forceinline__ void arrived_in_lds() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void arrived_in_lds() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
 
+// columns [c0, c0 + 8) of a row: what `raw` holds of them (zeros where there is nothing) as an operand chunk,
+// and the sums of squares of the row and of what bf16 drops
 template <typename T>
-__device__ __forceinline__ void approx_row(const AssignJob& job, size_t row, int c0, bool have,
-                                           uint4& packed, float& x2, float& l2) {
-    // columns [c0, c0 + 8) of a row: bf16 operand chunk, sums of squares of the row and of what bf16 drops
+__device__ __forceinline__ void approx_row(const uint4 (&raw)[8 / Elem<T>::kPerChunk], uint4& packed, float& x2, float& l2) {
     constexpr int EPL = Elem<T>::kPerChunk;
     float f[8];
 #pragma unroll
     for (int h = 0; h < 8 / EPL; ++h) {
-        uint4 raw = make_uint4(0, 0, 0, 0);
-        if (have && c0 + h * EPL < job.D) raw = load_chunk<T>(job.x, row * job.D, c0 / EPL + h);
         float g[EPL];
-        unpack<T>(raw, g);
+        unpack<T>(raw[h], g);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) f[h * EPL + e] = g[e];
-        if (EPL == 8) packed = raw;
+        if (EPL == 8) packed = raw[h];
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) x2 += f[e] * f[e];
@@ -474,18 +478,23 @@ __device__ __forceinline__ float from_ordered(uint32_t u) {
     return __uint_as_float(u ^ ((u >> 31) ? 0x80000000u : 0xffffffffu));
 }
 
+constexpr int kApproxThreads = 256;
+// Tiles of a stage: two of the stages that the tiles are padded to.  (A barrier every 64 products of a wave
+// had the matrix cores wait a third of the time; eight waves a workgroup instead of four were no better.)
+constexpr int approx_stage(int KS) { return 2 * assign_stage(KS); }
 constexpr int kApproxPairs = 512;  // (item, candidate) pairs of a wave: 64 items, at most eight each
 
 template <typename T, int KS, int RI, bool LISTED, bool EXACT_MFMA>
 __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int tag_bits, int n_items, int block) {
     constexpr int HALF = KS * 64;                       // chunks of the hi half of 16 centroids
     constexpr int TILE_CHUNKS = 2 * HALF;
-    constexpr int TPS = assign_stage(KS);
+    constexpr int TPS = approx_stage(KS);
     constexpr int STAGE = TPS * HALF;
-    constexpr int CPT = STAGE / kAssignThreads;
+    constexpr int CPT = STAGE / kApproxThreads;
     constexpr int ITEMS = RI * 16;                      // of a wave
+    constexpr int WAVES = kApproxThreads / 64;
     constexpr bool SPLIT = sizeof(T) == 4;              // items lose something in bf16
-    static_assert(STAGE % kAssignThreads == 0, "stage does not split over the workgroup");
+    static_assert(STAGE % kApproxThreads == 0, "stage does not split over the workgroup");
     extern __shared__ uint4 s_dyn[];
     uint4* s_c = s_dyn;                                             // (2, STAGE)
     float* s_start = reinterpret_cast<float*>(s_dyn + 2 * STAGE);   // (2, TPS * 16)
@@ -495,8 +504,36 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const int n = lane & 15, kb = lane >> 4;
     const int t = blockIdx.x, n_c = job.n_c, K = job.K;
-    const int first = (block * (kAssignThreads / 64) + wave) * ITEMS;
+    const int first = (block * (kApproxThreads / 64) + wave) * ITEMS;
 
+    // ---- the first stage of tiles: on its way while the items come ---------------------------------
+    // (whole stages of assign_stage(KS) tiles are there; the walk's last stage may have no second half: it
+    // takes a tile there is, whose centroids take no items)
+    const int tiles = job.open.count ? min(((job.open.count[t] + 15) / 16 + TPS / 2 - 1) / (TPS / 2) * (TPS / 2), Kt) : Kt;
+    const int Ks = (tiles + TPS - 1) / TPS;
+    const uint4* tt = job.ct.tiles + (size_t)t * Kt * TILE_CHUNKS;
+    const float* n2t = job.ct.n2 + (size_t)t * Kt * 16;
+    const float* lot = job.ct.lo + (size_t)t * Kt * 16;
+    const int q = threadIdx.x & (TPS * 16 - 1);
+    // (of a tile only the hi half is fetched)
+    auto fetch = [&](int st, int buf) {
+        const int last = tiles - 1 - st * TPS;  // of the stage
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) {
+            constexpr int PER = HALF / kApproxThreads;  // steps of the workgroup a tile (0: several tiles a step)
+            const int ci = c * kApproxThreads + (int)threadIdx.x;
+            const int tile = PER > 0 ? c / max(PER, 1) : ci / HALF;
+            const uint4* src = tt + (size_t)(st * TPS + min(tile, last)) * TILE_CHUNKS + ci % HALF;
+            load_to_lds(src, s_c + buf * STAGE + c * kApproxThreads + wave_u * 64);
+        }
+    };
+    auto norms_at = [&](int st) { return min(st * (TPS * 16) + q, tiles * 16 - 1); };
+    float first_n2 = 0.0f, first_lo = 0.0f;
+    if (Ks > 0) {
+        fetch(0, 0);
+        first_n2 = n2t[norms_at(0)];
+        first_lo = lot[norms_at(0)];
+    }
     // ---- my items ----------------------------------------------------------------------------
     int item[RI];
     uint4 b[RI][KS];
@@ -506,14 +543,12 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     for (int ri = 0; ri < RI; ++ri) {
         const int pos = first + ri * 16 + n;
         item[ri] = -1;
-        if (pos < n_items) item[ri] = LISTED ? job.list[(size_t)t * n_c + pos] : pos;
+        const int at = min(pos, n_items - 1);  // (n_items > 0: the workgroup has work)
+        item[ri] = LISTED ? job.list[(size_t)t * n_c + at] : at;
+        if (pos >= n_items) item[ri] = -1;
     }
-#pragma unroll
-    for (int ri = 0; ri < RI; ++ri) {
-        float ss = 0.0f, ls = 0.0f;
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-            approx_row<T>(job, (size_t)t * job.x_tree_stride + max(item[ri], 0), s * 32 + kb * 8, item[ri] >= 0, b[ri][s], ss, ls);
+    constexpr int EPL = Elem<T>::kPerChunk;
+    auto norms = [&](int ri, float ss, float ls) {  // (of this lane's columns)
         ss += __shfl_xor(ss, 16, 64);
         ss += __shfl_xor(ss, 32, 64);
         x2[ri] = ss;
@@ -523,6 +558,44 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
             ls += __shfl_xor(ls, 32, 64);
             Xl = fmaxf(Xl, ls);
         }
+    };
+    if constexpr (EXACT_MFMA) {
+        // whole operands: all rows on their way under no condition (a load under one is waited for where
+        // the condition ends, one item tile after the other)
+        uint4 raw[RI][KS][1];
+#pragma unroll
+        for (int ri = 0; ri < RI; ++ri)
+#pragma unroll
+            for (int s = 0; s < KS; ++s)
+                raw[ri][s][0] = load_chunk<T>(job.x, ((size_t)t * job.x_tree_stride + max(item[ri], 0)) * (32 * KS), s * 4 + kb);
+#pragma unroll
+        for (int ri = 0; ri < RI; ++ri) {
+            float ss = 0.0f, ls = 0.0f;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                if (item[ri] < 0) raw[ri][s][0] = make_uint4(0, 0, 0, 0);
+                approx_row<T>(raw[ri][s], b[ri][s], ss, ls);
+            }
+            norms(ri, ss, ls);
+        }
+    } else {
+#pragma unroll
+        for (int ri = 0; ri < RI; ++ri) {
+            float ss = 0.0f, ls = 0.0f;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                const int c0 = s * 32 + kb * 8;
+                uint4 raw[8 / EPL];
+#pragma unroll
+                for (int h = 0; h < 8 / EPL; ++h) {
+                    raw[h] = make_uint4(0, 0, 0, 0);
+                    if (item[ri] >= 0 && c0 + h * EPL < job.D)
+                        raw[h] = load_chunk<T>(job.x, ((size_t)t * job.x_tree_stride + item[ri]) * job.D, c0 / EPL + h);
+                }
+                approx_row<T>(raw, b[ri][s], ss, ls);
+            }
+            norms(ri, ss, ls);
+        }
     }
 #pragma unroll
     for (int off = 1; off < 16; off <<= 1) {
@@ -531,15 +604,26 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     }
     if (lane == 0) {
         s_x[wave] = X;
-        s_x[4 + wave] = Xl;
+        s_x[WAVES + wave] = Xl;
     }
     __syncthreads();
-    X = fmaxf(fmaxf(s_x[0], s_x[1]), fmaxf(s_x[2], s_x[3]));
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        X = fmaxf(X, s_x[w]);
+        if (SPLIT) Xl = fmaxf(Xl, s_x[WAVES + w]);
+    }
     X = sqrtf(X) * 1.0001f;
     if (SPLIT) {
-        Xl = fmaxf(fmaxf(s_x[4], s_x[5]), fmaxf(s_x[6], s_x[7]));
         Xl = sqrtf(Xl) * 1.0001f;
     }
+
+    auto put_start = [&](int st, int buf, float n2, float lo) {
+        // (1e-5 of the squared norm: what the rounding of the norm can be worth)
+        float v = fmaf(X, lo, -0.5f * n2 + 1e-5f * n2);
+        if (SPLIT) v = fmaf(Xl, sqrtf(n2), v);
+        if (!(n2 < INFINITY) || st * TPS * 16 + q >= tiles * 16) v = kNoScore;
+        s_start[buf * TPS * 16 + q] = v;  // (the same by every wave that has the column: no branch)
+    };
 
     float best[2][RI], second[2][RI];  // of the even tiles, of the odd ones
 #pragma unroll
@@ -547,36 +631,8 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     const uint32_t keep = ~((1u << tag_bits) - 1u);
 
     // ---- all centroid tiles --------------------------------------------------------------------
-    const int Ks_all = (Kt + TPS - 1) / TPS;
-    const int Ks = job.open.count ? min(((job.open.count[t] + 15) / 16 + TPS - 1) / TPS, Ks_all) : Ks_all;
-    const uint4* tt = job.ct.tiles + (size_t)t * Ks_all * TPS * TILE_CHUNKS;
-    const float* n2t = job.ct.n2 + (size_t)t * Ks_all * (TPS * 16);
-    const float* lot = job.ct.lo + (size_t)t * Ks_all * (TPS * 16);
-    const int q = threadIdx.x & (TPS * 16 - 1);
-    auto put_start = [&](int buf, float n2, float lo) {
-        // (1e-5 of the squared norm: what the rounding of the norm can be worth)
-        float v = fmaf(X, lo, -0.5f * n2 + 1e-5f * n2);
-        if (SPLIT) v = fmaf(Xl, sqrtf(n2), v);
-        s_start[buf * TPS * 16 + q] = n2 < INFINITY ? v : kNoScore;  // (every wave the same: no branch)
-    };
-    // (of a tile only the hi half is fetched)
-    uint32_t from[CPT];
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-        const int ci = c * kAssignThreads + (int)threadIdx.x;
-        from[c] = (uint32_t)(ci / HALF * TILE_CHUNKS + ci % HALF);
-    }
-    auto fetch = [&](int st, int buf) {
-        const uint4* src = tt + (size_t)st * (TPS * TILE_CHUNKS);
-#pragma unroll
-        for (int c = 0; c < CPT; ++c) load_to_lds(src + from[c], s_c + buf * STAGE + c * kAssignThreads + wave_u * 64);
-    };
-    if (Ks > 0) {
-        fetch(0, 0);
-        put_start(0, n2t[q], lot[q]);
-    }
+    if (Ks > 0) put_start(0, 0, first_n2, first_lo);
     arrived_in_lds();
-    __syncthreads();
     // The results of a tile are looked at while the next tile's products are made: a product keeps the
     // matrix cores busy for the time of four vector instructions, three of which deal with a result.
     // The order is the one written here (left to itself the compiler makes all products of a stage
@@ -586,20 +642,36 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     for (int ri = 0; ri < RI; ++ri) acc[1][ri] = af32x4_t{-3e38f, -3e38f, -3e38f, -3e38f};
     uint32_t keep_v;  // (in a vector register: with `tag` in a scalar one the bits are one instruction)
     asm volatile("v_mov_b32 %0, %1" : "=v"(keep_v) : "s"(keep));
+    // The four results of an item tile in nine steps: tagged, then two at a time into best and second.  With
+    // best >= second the two largest of {best, second, u, v} are max3(best, u, v) and
+    // max(med3(best, u, v), second), and the maxima of `second` of both pairs are one instruction.
+    // (Asm: fmaxf quiets its operands first, an instruction each.)
+    constexpr int LOOKS = 8, PRODUCTS = KS * RI, RESULTS = LOOKS * RI;
+    float m3[RI];
     auto look = [&](int of, uint32_t tag, int o) {
-        const int j = o / RI, ri = o % RI;
-        const float v = __uint_as_float((__float_as_uint(acc[of][ri][j]) & keep_v) | (tag + j));
-        second[of][ri] = __builtin_amdgcn_fmed3f(best[of][ri], second[of][ri], v);
-        asm("v_max_f32 %0, %0, %1" : "+v"(best[of][ri]) : "v"(v));  // (fmaxf is two: it quiets v first)
+        const int ri = o / LOOKS, k = o % LOOKS;
+        float(&r)[RI] = best[of];
+        auto tagged = [&](int j) { acc[of][ri][j] = __uint_as_float((__float_as_uint(acc[of][ri][j]) & keep_v) | (tag + j)); };
+        auto max3 = [](float& a, float u, float v) { asm("v_max3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(u), "v"(v)); };
+        if (k == 0) tagged(0);
+        if (k == 1) tagged(1);
+        if (k == 2) m3[ri] = __builtin_amdgcn_fmed3f(r[ri], acc[of][ri][0], acc[of][ri][1]);
+        if (k == 3) max3(r[ri], acc[of][ri][0], acc[of][ri][1]);
+        if (k == 4) tagged(2);
+        if (k == 5) tagged(3);
+        if (k == 6) {
+            const float m = __builtin_amdgcn_fmed3f(r[ri], acc[of][ri][2], acc[of][ri][3]);
+            max3(second[of][ri], m3[ri], m);
+        }
+        if (k == 7) max3(r[ri], acc[of][ri][2], acc[of][ri][3]);
     };
-    constexpr int PRODUCTS = KS * RI, RESULTS = 4 * RI;
     for (int st = 0; st < Ks; ++st) {
         const int buf = st & 1;
         const uint4* cbuf = s_c + buf * STAGE + lane;
         const float* sbuf = s_start + buf * TPS * 16 + 4 * kb;
         const int nst = min(st + 1, Ks - 1);
+        const float next_n2 = n2t[norms_at(nst)], next_lo = lot[norms_at(nst)];
         fetch(nst, buf ^ 1);
-        const float next_n2 = n2t[nst * (TPS * 16) + q], next_lo = lot[nst * (TPS * 16) + q];
         abf16x8_t a[2][KS];
         af32x4_t start[2];
 #pragma unroll
@@ -626,9 +698,8 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        put_start(buf ^ 1, next_n2, next_lo);
+        put_start(nst, buf ^ 1, next_n2, next_lo);
         arrived_in_lds();
-        __syncthreads();
     }
     if (Ks > 0) {
         static_assert(TPS % 2 == 0, "the last tile's results are in acc[1]");
@@ -647,34 +718,56 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     s_key[lane] = ~0ull;
     int npairs = 0;      // uniform in the wave
     bool unsure[RI];
+    int top[RI];         // the column with the largest value among the item's lanes
+    bool scored[RI];     // its exact distance is needed, and those of the others in the running
+    unsigned long long ask = 0;  // (uniform) not zero: some are
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // The largest value among the item's lanes, less what it can be too large by, is what the exact score of
+    // the nearest reaches at least.  (One lookup an item, for all item tiles at once: a lookup of every lane's
+    // own two columns is 64 lines of memory a load, 4.4 us at the end of a workgroup's 106.)
+    int col[2][RI];
+    float top_v[RI], top_n2[RI], top_lo[RI];
 #pragma unroll
     for (int ri = 0; ri < RI; ++ri) {
-        int col[2];
-        bool any[2];
-        float floor_of = -INFINITY;  // the exact score of the best is at least this
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
+        for (int e = 0; e < 2; ++e) {  // (a value that is no number holds any tag)
             const uint32_t tag = __float_as_uint(best[e][ri]) & ~keep;
-            col[e] = (int)(tag >> 2) * 16 + 4 * kb + (int)(tag & 3u);
-            any[e] = best[e][ri] > 0.5f * kNoScore && item[ri] >= 0;
-            if (any[e]) {
-                const float n2 = n2t[col[e]], lo = lot[col[e]];
-                float off = 2.0f * (X * lo + 1e-5f * n2);
-                if (SPLIT) off += 2.0f * Xl * sqrtf(n2);
-                if (!EXACT_MFMA) off += 1e-5f * X * X;  // (rounding of sums of squared differences)
-                floor_of = fmaxf(floor_of, best[e][ri] - off - fabsf(best[e][ri]) * shift);
+            col[e][ri] = min((int)(tag >> 2) * 16 + 4 * kb + (int)(tag & 3u), Kt * 16 - 1);
+        }
+        const float v0 = best[0][ri] > 0.5f * kNoScore ? best[0][ri] : -INFINITY;
+        const float v1 = best[1][ri] > 0.5f * kNoScore ? best[1][ri] : -INFINITY;
+        const bool second_is = v1 > v0;
+        float tv = second_is ? v1 : v0;
+        int tc = second_is ? col[1][ri] : col[0][ri];
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            const float ov = __shfl_xor(tv, off, 64);
+            const int oc = __shfl_xor(tc, off, 64);
+            if (ov > tv || (ov == tv && oc < tc)) {
+                tv = ov;
+                tc = oc;
             }
         }
-        floor_of = fmaxf(floor_of, __shfl_xor(floor_of, 16, 64));
-        floor_of = fmaxf(floor_of, __shfl_xor(floor_of, 32, 64));
+        top_v[ri] = tv;
+        top[ri] = tc;
+        top_n2[ri] = n2t[tc];
+        top_lo[ri] = lot[tc];
+    }
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+        const bool have = item[ri] >= 0 && top_v[ri] > 0.5f * kNoScore;
+        float off = 2.0f * (X * top_lo[ri] + 1e-5f * top_n2[ri]);
+        if (SPLIT) off += 2.0f * Xl * sqrtf(top_n2[ri]);
+        if (!EXACT_MFMA) off += 1e-5f * X * X;  // (rounding of sums of squared differences)
+        const float floor_of = top_v[ri] - off - fabsf(top_v[ri]) * shift;
         bool in[2];
         int un = 0, cands = 0;
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            in[e] = any[e] && best[e][ri] + fabsf(best[e][ri]) * shift >= floor_of;
+            const bool any = have && best[e][ri] > 0.5f * kNoScore;  // (not a number: no)
+            in[e] = any && best[e][ri] + fabsf(best[e][ri]) * shift >= floor_of;
             // (a value next to zero does not hold its tag)
-            un |= any[e] && (!(second[e][ri] + fabsf(second[e][ri]) * shift < floor_of) || fabsf(best[e][ri]) < 1e-30f);
+            un |= any && (!(second[e][ri] + fabsf(second[e][ri]) * shift < floor_of) || fabsf(best[e][ri]) < 1e-30f);
             cands += in[e];
         }
         un |= __shfl_xor(un, 16, 64);
@@ -683,25 +776,73 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
         cands += __shfl_xor(cands, 32, 64);
         un |= cands == 0;  // (rows with numbers that are none: as the exact kernel has it)
         unsure[ri] = un;
+        scored[ri] = !un && (want_dist || cands > 1);
+        ask |= __ballot(scored[ri]);
+        if (!un && !scored[ri] && kb == 0) s_key[ri * 16 + n] = (unsigned long long)(uint32_t)top[ri];  // (the only one)
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const bool score = in[e] && !un && (want_dist || cands > 1);
+            const bool score = in[e] && scored[ri] && !(EXACT_MFMA && col[e][ri] == top[ri]);
             const unsigned long long bal = __ballot(score);
             if (score) {
                 const int at = npairs + __popcll(bal & ((1ull << lane) - 1ull));
                 s_item[at] = ri * 16 + n;
-                s_col[at] = col[e];
+                s_col[at] = col[e][ri];
             }
             npairs += __popcll(bal);
-            if (in[e] && !un && !score) s_key[ri * 16 + n] = (unsigned long long)(uint32_t)col[e];  // (the only one)
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 
     // ---- the candidates' exact distances ---------------------------------------------------------
     if constexpr (EXACT_MFMA) {
-        // sixteen pairs at a time: row i of the A operand is the pair's centroid, column i of B its
-        // item, the result on the diagonal; the products in the exact kernel's order
+        // Row i of the A operand is a centroid, column i of B an item, the result on the diagonal; the
+        // products in the exact kernel's order.  First the largest of every item, whose operands are still in
+        // registers: the centroids' rows of all item tiles are asked for at once.  Then the others,
+        // sixteen pairs at a time.  The rows come from the fp32 centroids and are split here as emit_centroid
+        // splits them: sixteen lines of memory a load.  (Out of sixteen operand tiles they are 64, and the end of
+        // a workgroup that asks for distances took 9.3 of its 125 us.)
+        auto cent_row = [&](int c) {
+            const int k = job.open.ids != nullptr ? job.open.ids[(size_t)t * K + c] : c;  // column -> centroid
+            return reinterpret_cast<const uint4*>(job.cent + ((size_t)t * K + k) * (32 * KS) + kb * 8);
+        };
+        auto halves = [](const uint4& lo4, const uint4& hi4, abf16x8_t& h, abf16x8_t& l) {
+            const af32x8_t v = {__uint_as_float(lo4.x), __uint_as_float(lo4.y), __uint_as_float(lo4.z), __uint_as_float(lo4.w),
+                                __uint_as_float(hi4.x), __uint_as_float(hi4.y), __uint_as_float(hi4.z), __uint_as_float(hi4.w)};
+            h = __builtin_convertvector(v, abf16x8_t);
+            l = __builtin_convertvector(v - __builtin_convertvector(h, af32x8_t), abf16x8_t);
+        };
+        auto put_diagonal = [&](const af32x4_t& d4, float n2, int c, int it_local, bool have) {
+            if (kb == (n >> 2) && have) {  // row n = 4 * kb + j of column n
+                const int j = n & 3;
+                const float d = j == 0 ? d4[0] : j == 1 ? d4[1] : j == 2 ? d4[2] : d4[3];
+                const float v = n2 - 2.0f * d;
+                atomicMin(&s_key[it_local], ((unsigned long long)ordered_bits(v) << 32) | (uint32_t)c);
+            }
+        };
+        if (ask != 0) {  // uniform
+            uint4 rows[RI][KS][2];
+#pragma unroll
+            for (int ri = 0; ri < RI; ++ri) {
+                const uint4* row = cent_row(scored[ri] ? top[ri] : 0);  // (column 0: there is one)
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    rows[ri][s][0] = row[s * 8];
+                    rows[ri][s][1] = row[s * 8 + 1];
+                }
+            }
+#pragma unroll
+            for (int ri = 0; ri < RI; ++ri) {
+                af32x4_t d4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    abf16x8_t h, l;
+                    halves(rows[ri][s][0], rows[ri][s][1], h, l);
+                    d4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h, __builtin_bit_cast(abf16x8_t, b[ri][s]), d4, 0, 0, 0);
+                    d4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l, __builtin_bit_cast(abf16x8_t, b[ri][s]), d4, 0, 0, 0);
+                }
+                put_diagonal(d4, top_n2[ri], top[ri], ri * 16 + n, scored[ri]);
+            }
+        }
         for (int p0 = 0; p0 < npairs; p0 += 16) {  // uniform in the wave
             const int pi = min(p0 + n, npairs - 1);
             const int it_local = s_item[pi], col = s_col[pi];
@@ -711,30 +852,26 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
                 const int o = __shfl(item[ri], it_local & 15, 64);
                 if ((it_local >> 4) == ri) it = o;
             }
-            const uint4* ct = tt + (size_t)(col >> 4) * TILE_CHUNKS + kb * 16 + (col & 15);
+            const uint4* row = cent_row(col);
             const uint4* xt = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(job.x) +
                                                              ((size_t)t * job.x_tree_stride + it) * (32 * KS) + kb * 8);
-            uint4 ch[KS], cl[KS], xr[KS];
+            uint4 rows[KS][2], xr[KS];
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
-                ch[s] = ct[s * 64];
-                cl[s] = ct[HALF + s * 64];
+                rows[s][0] = row[s * 8];
+                rows[s][1] = row[s * 8 + 1];
                 xr[s] = xt[s * 4];
             }
             const float n2 = n2t[col];
             af32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < KS; ++s) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(abf16x8_t, ch[s]), __builtin_bit_cast(abf16x8_t, xr[s]), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(abf16x8_t, cl[s]), __builtin_bit_cast(abf16x8_t, xr[s]), acc, 0, 0, 0);
+                abf16x8_t h, l;
+                halves(rows[s][0], rows[s][1], h, l);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h, __builtin_bit_cast(abf16x8_t, xr[s]), acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l, __builtin_bit_cast(abf16x8_t, xr[s]), acc, 0, 0, 0);
             }
-            // the diagonal: row n = 4 * kb + j of column n
-            if (kb == (n >> 2) && p0 + n < npairs) {
-                const int j = n & 3;
-                const float d = j == 0 ? acc[0] : j == 1 ? acc[1] : j == 2 ? acc[2] : acc[3];
-                const float v = n2 - 2.0f * d;
-                atomicMin(&s_key[it_local], ((unsigned long long)ordered_bits(v) << 32) | (uint32_t)col);
-            }
+            put_diagonal(acc, n2, col, it_local, p0 + n < npairs);
         }
     } else {
         // LPR lanes a pair, as the vector-ALU kernel holds an item and a centroid
@@ -814,7 +951,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
 }
 
 template <typename T, int KS, bool LISTED, bool EXACT_MFMA>
-__global__ __launch_bounds__(kAssignThreads, 2) void k_assign_approx(const AssignJob job, const int Kt,
+__global__ __launch_bounds__(kApproxThreads, 2) void k_assign_approx(const AssignJob job, const int Kt,
                                                                      const int tag_bits) {
     // (trees in the fast index: the workgroups of a tree run behind the same L2s, which hold its tiles)
     const int t = blockIdx.x;
@@ -822,7 +959,7 @@ __global__ __launch_bounds__(kAssignThreads, 2) void k_assign_approx(const Assig
     const int n_items = items_of(job, t);
     if (LISTED && EXACT_MFMA && !approx_takes(n_items, gridDim.x)) return;  // (k_assign_split's)
     const bool narrow = LISTED && !EXACT_MFMA && !approx_takes(n_items, gridDim.x);
-    const int per_block = (kAssignThreads / 64) * 16 * (narrow ? 1 : RI);
+    const int per_block = (kApproxThreads / 64) * 16 * (narrow ? 1 : RI);
     if (!EXACT_MFMA && job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t * kCounterStride] = 0;
     for (int b = blockIdx.y; b * per_block < n_items; b += gridDim.y) {  // uniform
         if (b != (int)blockIdx.y) __syncthreads();
@@ -993,21 +1130,21 @@ int launch_assign_mfma(const AssignJob& job, hipStream_t s) {
 template <typename T, int KS, bool LISTED, bool EXACT_MFMA>
 static int launch_approx(const AssignJob& job, hipStream_t s) {
     static int asked[kMaxDevices];
-    constexpr int TPS = assign_stage(KS);
+    constexpr int TPS = approx_stage(KS);
     // (the pairs lie where the tiles were)
-    constexpr size_t tiles = 2 * (size_t)TPS * KS * 64 * sizeof(uint4) + (2 * (size_t)TPS * 16 + 8) * sizeof(float);
-    constexpr size_t pairs = 4 * (64 * 8 + kApproxPairs * 8), smem = tiles > pairs ? tiles : pairs;
+    constexpr size_t tiles = 2 * (size_t)TPS * (KS * 64 * sizeof(uint4) + 16 * sizeof(float)) + 2 * (kApproxThreads / 64) * sizeof(float);
+    constexpr size_t pairs = kApproxThreads / 64 * (64 * 8 + kApproxPairs * 8), smem = tiles > pairs ? tiles : pairs;
     if (const int rc = ask_for_lds(reinterpret_cast<const void*>(&k_assign_approx<T, KS, LISTED, EXACT_MFMA>), smem, asked,
                                    current_device()))
         return rc;
     constexpr int RI = KS <= 4 ? 4 : 2;
-    const int per_block = (kAssignThreads / 64) * (LISTED && !EXACT_MFMA ? 1 : RI) * 16;
+    const int per_block = (kApproxThreads / 64) * (LISTED && !EXACT_MFMA ? 1 : RI) * 16;
     const int blocks = min((job.n_c + per_block - 1) / per_block, 65535);  // (they go on in strides)
     const int Kt = assign_tiles(job.K);
     int tag_bits = 1;
     while ((1 << tag_bits) < Kt * 4) ++tag_bits;
     if (tag_bits > kMaxTagBits) return fail(HIRA_EINVAL, "approximate assignment: %d centroids", job.K);
-    hipLaunchKernelGGL((k_assign_approx<T, KS, LISTED, EXACT_MFMA>), dim3(job.num_trees, blocks), dim3(kAssignThreads),
+    hipLaunchKernelGGL((k_assign_approx<T, KS, LISTED, EXACT_MFMA>), dim3(job.num_trees, blocks), dim3(kApproxThreads),
                        smem, s, job, Kt, tag_bits);
     return HIRA_OK;
 }
