@@ -243,21 +243,45 @@ __global__ __launch_bounds__(kAssignThreads, 2) void k_assign_mfma(const AssignJ
     }
 }
 
-// ---- every product with both halves, few items: 64 a workgroup, its waves share out the centroids ----
+// ---- every product with both halves, few items: 64 a wave, or a few waves -----------------------
 // Lists (the packing's, or what the approximate pass leaves) and small levels leave most of the chip
-// idle if a wave walks all centroids for items of its own: here the 8 waves of a workgroup hold the
-// same items and walk every eighth tile, straight from memory to registers (nobody shares a tile
-// inside the workgroup), the next one on its way while one is used.  Centroids are the rows of a
+// idle if 256 items go together.  Here a wave holds 64 items and walks the tiles straight from memory to
+// registers, the next one on its way while one is used; `share` waves of the workgroup hold the same items
+// and walk every share-th tile, as many as there are waves for on the chip (split_share).  Centroids are the rows of a
 // product, so a lane's results are four centroids of one item per item tile, and what is left at the
-// end is a minimum over four lanes and eight waves.
-// (1024 centroids, 8 x ~1000 items: 52 us with a walk of all tiles per wave, now 13.)
+// end is a minimum over four lanes and `share` waves.
+// What bounds it is the chain items, tiles, bucket, and for long lists the matrix cores.  Eight waves to 64 items
+// whatever their number: a workgroup's items and its end were most of its time where lists are long and
+// centroids few (8 x 7200 items, 330 centroids: 40 us, now 24; 8 x 8300, 330: 58, now 48); one wave to
+// 64 items whatever their number: 8 x ~1000 items, 1024 centroids 52 us, now 9.
 constexpr int kSplitThreads = 512;
 constexpr int kSplitBlocks = 128;        // workgroups of a tree, at most: they go through a list in strides
+constexpr int kSplitWavesLog2 = 11;      // of the waves on the chip at a time: 256 compute units, 8 each
+static_assert(kSplitThreads == 64 << 3, "split_share_log2");
 
 constexpr int split_ri(int KS) { return KS <= 4 ? 4 : 2; }
 
+// Waves that share a set of items, of which each of `trees` trees has `sets` (as a power of two): the number
+// whose rounds of waves take least, a wave's items and its end as long as kSplitFixed tiles.
 template <int KS>
-__device__ __forceinline__ void split_items(const AssignJob& job, int Kt, const int32_t* list, int n_items, int block) {
+__device__ __forceinline__ int split_share_log2(int sets, int trees, int tiles) {
+    constexpr int kSplitFixed = 48 / KS, on_chip_log2 = KS <= 2 ? kSplitWavesLog2 + 1 : kSplitWavesLog2;
+    int best = 0;
+    long long least = 0;
+#pragma unroll
+    for (int s = 0; s <= 3; ++s) {
+        const long long rounds = (((long long)sets * trees << s) + (1 << on_chip_log2) - 1) >> on_chip_log2;
+        const long long cost = rounds * (kSplitFixed + ((tiles + (1 << s) - 1) >> s));
+        if (s == 0 || cost < least) {
+            best = s;
+            least = cost;
+        }
+    }
+    return best;
+}
+
+template <int KS>
+__device__ __forceinline__ void split_items(const AssignJob& job, int Kt, int tiles, const int32_t* list, int n_items, int share_log2, int block) {
     constexpr int D = 32 * KS, RI = split_ri(KS), ITEMS = RI * 16, WAVES = kSplitThreads / 64;
     constexpr int TILE_CHUNKS = 2 * KS * 64;
     __shared__ float s_b[WAVES][ITEMS];
@@ -269,7 +293,8 @@ __device__ __forceinline__ void split_items(const AssignJob& job, int Kt, const 
     // ---- the first tile of the wave, and the items ---------------------------------------------
     const uint4* tt = job.ct.tiles + (size_t)t * Kt * TILE_CHUNKS + lane;
     const float* n2t = job.ct.n2 + (size_t)t * Kt * 16 + 4 * kb;
-    const int tiles = job.open.count ? min((job.open.count[t] + 15) / 16, Kt) : (K + 15) / 16;
+    const int share = 1 << share_log2;
+    const int set = block * (WAVES >> share_log2) + (wave >> share_log2), part = wave & (share - 1);
     uint4 c[2][2 * KS];
     float4 c2[2];
     auto fetch = [&](int tile, uint4 (&to)[2 * KS], float4& n2) {
@@ -277,16 +302,17 @@ __device__ __forceinline__ void split_items(const AssignJob& job, int Kt, const 
 #pragma unroll
         for (int s = 0; s < 2 * KS; ++s) to[s] = src[s * 64];
         n2 = *reinterpret_cast<const float4*>(n2t + tile * 16);
+        __builtin_amdgcn_sched_barrier(0);  // (asked for here, not where the first product wants it)
     };
-    fetch(min(wave, Kt - 1), c[0], c2[0]);
+    fetch(min(part, Kt - 1), c[0], c2[0]);
     int item[RI];
     uint4 x[RI][KS];
     float x2[RI];
 #pragma unroll
     for (int ri = 0; ri < RI; ++ri) {
-        const int pos = block * ITEMS + ri * 16 + n;
-        item[ri] = -1;
-        if (pos < n_items) item[ri] = list ? list[(size_t)t * n_c + pos] : pos;
+        const int pos = set * ITEMS + ri * 16 + n, at = min(pos, n_items - 1);  // (n_items > 0)
+        item[ri] = list ? list[(size_t)t * n_c + at] : at;
+        if (pos >= n_items) item[ri] = -1;
     }
 #pragma unroll
     for (int ri = 0; ri < RI; ++ri)
@@ -340,16 +366,16 @@ __device__ __forceinline__ void split_items(const AssignJob& job, int Kt, const 
                 }
             }
     };
-    int tile = wave;
-    for (; tile + WAVES < tiles; tile += 2 * WAVES) {  // uniform in the wave; no barrier inside
-        fetch(tile + WAVES, c[1], c2[1]);
+    int tile = set * ITEMS < n_items ? part : tiles;  // (a wave without items walks none)
+    for (; tile + share < tiles; tile += 2 * share) {  // uniform in the wave; no barrier inside
+        fetch(tile + share, c[1], c2[1]);
         use(tile, c[0], c2[0]);
-        fetch(min(tile + 2 * WAVES, Kt - 1), c[0], c2[0]);
-        use(tile + WAVES, c[1], c2[1]);
+        fetch(min(tile + 2 * share, Kt - 1), c[0], c2[0]);
+        use(tile + share, c[1], c2[1]);
     }
     if (tile < tiles) use(tile, c[0], c2[0]);
 
-    // ---- one of the four lanes, then of the eight waves, of an item ------------------------------
+    // ---- one of the four lanes, then of the waves, of an item ------------------------------------
     auto better = [](float b, int g, float ob, int og) { return og >= 0 && (g < 0 || ob < b || (ob == b && og < g)); };
 #pragma unroll
     for (int ri = 0; ri < RI; ++ri) {
@@ -368,12 +394,11 @@ __device__ __forceinline__ void split_items(const AssignJob& job, int Kt, const 
         }
     }
     __syncthreads();
-    if (wave != 0 || lane >= ITEMS) return;
+    if (part != 0 || lane >= ITEMS) return;
     // lane (kb, n) takes item n of tile kb
-    float b = s_b[0][lane];
-    int g = s_g[0][lane];
-#pragma unroll
-    for (int w = 1; w < WAVES; ++w)
+    float b = s_b[wave][lane];
+    int g = s_g[wave][lane];
+    for (int w = wave + 1; w < wave + share; ++w)  // uniform
         if (better(b, g, s_b[w][lane], s_g[w][lane])) {
             b = s_b[w][lane];
             g = s_g[w][lane];
@@ -401,9 +426,12 @@ __global__ __launch_bounds__(kSplitThreads, 2) void k_assign_split(const AssignJ
         n_items = job.unsure_count[t * kCounterStride];
     }
     if (job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t * kCounterStride] = 0;
-    for (int b = blockIdx.y; b * split_ri(KS) * 16 < n_items; b += gridDim.y) {  // uniform
+    constexpr int ITEMS = split_ri(KS) * 16;
+    const int tiles = job.open.count ? min((job.open.count[t] + 15) / 16, Kt) : (job.K + 15) / 16;
+    const int sets = (n_items + ITEMS - 1) / ITEMS, share_log2 = split_share_log2<KS>(sets, gridDim.x, tiles);
+    for (int b = blockIdx.y; b * (kSplitThreads / 64 >> share_log2) < sets; b += gridDim.y) {  // uniform
         if (b != (int)blockIdx.y) __syncthreads();  // (the results of the stride before are out of LDS)
-        split_items<KS>(job, Kt, list, n_items, b);
+        split_items<KS>(job, Kt, tiles, list, n_items, share_log2, b);
     }
 }
 
@@ -413,14 +441,14 @@ __global__ __launch_bounds__(kSplitThreads, 2) void k_assign_split(const AssignJ
 //   |x.c - xh.hi| <= ||x|| lo_k + ||xl|| ||c_k||      (lo_k: assign.h, rounding of the sums included)
 // so the products with `hi` alone, started from  -||c_k||^2 / 2 + X lo_k + Xl ||c_k||  (X, Xl: the
 // largest norms among the workgroup's items), are never below the exact score, and above it by at most
-// twice that allowance.  A lane keeps its best and second best of them per item, for even and for
-// odd tiles, the centroid's number in the low bits of the value (one instruction, against a comparison and two selections that
-// a separate index takes; what the bits shift the value by counts as error).  Per item the best lower
-// bound decides who is still in the running: of the four lanes that share the item, and their two
-// bests each, those that reach it.  One candidate: that is the nearest.  Several: each is scored by the exact kernel's own
-// arithmetic, and the smallest distance wins, the lowest centroid on ties -- the exact kernel's
+// twice that allowance.  A lane keeps its best and second best of them per item and
+// class of tiles, the centroid's number in the low bits of the value (one instruction, against a comparison
+// and two selections that a separate index takes; what the bits shift the value by counts as error).  Per item
+// the lower bound of the largest decides who is still in the running: of the four lanes that share the item, and
+// their bests, those that reach it.  One candidate: that is the nearest.  Several: each is scored by the
+// exact kernel's own arithmetic, and the smallest distance wins, the lowest centroid on ties -- the exact kernel's
 // result bit for bit.  Where a SECOND best is in the running too, a third could be as well, which
-// nobody noted: such items (1-2 % on normal keys) go on a list that the exact kernel takes.
+// nobody noted: such items (about 1 % on normal keys) go on a list that the exact kernel takes.
 // Operands: centroids are the rows (A), items the columns (B): a lane's four results of a product are
 // four centroids of ONE item, so best and second are one pair per item tile instead of four, and the
 // start values are a 16-byte read from LDS.
@@ -482,7 +510,11 @@ constexpr int kApproxThreads = 256;
 // Tiles of a stage: two of the stages that the tiles are padded to.  (A barrier every 64 products of a wave
 // had the matrix cores wait a third of the time; eight waves a workgroup instead of four were no better.)
 constexpr int approx_stage(int KS) { return 2 * assign_stage(KS); }
-constexpr int kApproxPairs = 512;  // (item, candidate) pairs of a wave: 64 items, at most eight each
+// Classes of tiles (by number) that a lane keeps a best and a second best of: the more, the fewer items of which
+// two candidates share a class.  (Two classes instead of four: twice the items the exact kernel has to take,
+// 109 us for it instead of 58 after the packing's full pass over 8 x 131072 items.)
+constexpr int kApproxClasses = 4;
+constexpr int kApproxPairs = 64 * 4 * kApproxClasses;  // (item, candidate) pairs of a wave, at most
 
 template <typename T, int KS, int RI, bool LISTED, bool EXACT_MFMA>
 __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int tag_bits, int n_items, int block) {
@@ -492,7 +524,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     constexpr int STAGE = TPS * HALF;
     constexpr int CPT = STAGE / kApproxThreads;
     constexpr int ITEMS = RI * 16;                      // of a wave
-    constexpr int WAVES = kApproxThreads / 64;
+    constexpr int WAVES = kApproxThreads / 64, CLS = kApproxClasses;
     constexpr bool SPLIT = sizeof(T) == 4;              // items lose something in bf16
     static_assert(STAGE % kApproxThreads == 0, "stage does not split over the workgroup");
     extern __shared__ uint4 s_dyn[];
@@ -625,9 +657,11 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
         s_start[buf * TPS * 16 + q] = v;  // (the same by every wave that has the column: no branch)
     };
 
-    float best[2][RI], second[2][RI];  // of the even tiles, of the odd ones
+    float best[CLS][RI], second[CLS][RI];  // of the tiles 0, CLS, 2 CLS, ..., of 1, CLS + 1, ..., ...
 #pragma unroll
-    for (int ri = 0; ri < RI; ++ri) best[0][ri] = second[0][ri] = best[1][ri] = second[1][ri] = -INFINITY;
+    for (int ri = 0; ri < RI; ++ri)
+#pragma unroll
+        for (int e = 0; e < CLS; ++e) best[e][ri] = second[e][ri] = -INFINITY;
     const uint32_t keep = ~((1u << tag_bits) - 1u);
 
     // ---- all centroid tiles --------------------------------------------------------------------
@@ -648,9 +682,9 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     // (Asm: fmaxf quiets its operands first, an instruction each.)
     constexpr int LOOKS = 8, PRODUCTS = KS * RI, RESULTS = LOOKS * RI;
     float m3[RI];
-    auto look = [&](int of, uint32_t tag, int o) {
+    auto look = [&](int of, int cls, uint32_t tag, int o) {
         const int ri = o / LOOKS, k = o % LOOKS;
-        float(&r)[RI] = best[of];
+        float(&r)[RI] = best[cls];
         auto tagged = [&](int j) { acc[of][ri][j] = __uint_as_float((__float_as_uint(acc[of][ri][j]) & keep_v) | (tag + j)); };
         auto max3 = [](float& a, float u, float v) { asm("v_max3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(u), "v"(v)); };
         if (k == 0) tagged(0);
@@ -661,7 +695,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
         if (k == 5) tagged(3);
         if (k == 6) {
             const float m = __builtin_amdgcn_fmed3f(r[ri], acc[of][ri][2], acc[of][ri][3]);
-            max3(second[of][ri], m3[ri], m);
+            max3(second[cls][ri], m3[ri], m);
         }
         if (k == 7) max3(r[ri], acc[of][ri][2], acc[of][ri][3]);
     };
@@ -688,7 +722,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
                 acc[me][ri] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     a[me][s], __builtin_bit_cast(abf16x8_t, b[ri][s]), s == 0 ? start[me] : acc[me][ri], 0, 0, 0);
 #pragma unroll
-                for (int o = p * RESULTS / PRODUCTS; o < (p + 1) * RESULTS / PRODUCTS; ++o) look(me ^ 1, tag, o);
+                for (int o = p * RESULTS / PRODUCTS; o < (p + 1) * RESULTS / PRODUCTS; ++o) look(me ^ 1, (ti + CLS - 1) % CLS, tag, o);
                 if (p == 1 && ti + 1 < TPS) {  // the next tile's operands
 #pragma unroll
                     for (int s2 = 0; s2 < KS; ++s2)
@@ -702,9 +736,9 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
         arrived_in_lds();
     }
     if (Ks > 0) {
-        static_assert(TPS % 2 == 0, "the last tile's results are in acc[1]");
+        static_assert(TPS % 2 == 0 && TPS % CLS == 0, "the last tile's results are in acc[1]");
 #pragma unroll
-        for (int o = 0; o < RESULTS; ++o) look(1, (uint32_t)(Ks * TPS - 1) * 4u, o);
+        for (int o = 0; o < RESULTS; ++o) look(1, CLS - 1, (uint32_t)(Ks * TPS - 1) * 4u, o);
     }
 
     // ---- who is still in the running (LDS is free behind the loop's last barrier) -------------------
@@ -725,20 +759,21 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     // The largest value among the item's lanes, less what it can be too large by, is what the exact score of
     // the nearest reaches at least.  (One lookup an item, for all item tiles at once: a lookup of every lane's
     // own two columns is 64 lines of memory a load, 4.4 us at the end of a workgroup's 106.)
-    int col[2][RI];
+    int col[CLS][RI];
     float top_v[RI], top_n2[RI], top_lo[RI];
 #pragma unroll
     for (int ri = 0; ri < RI; ++ri) {
+        float tv = -INFINITY;
+        int tc = Kt * 16 - 1;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {  // (a value that is no number holds any tag)
+        for (int e = 0; e < CLS; ++e) {  // (a value that is no number holds any tag, and is none of the largest)
             const uint32_t tag = __float_as_uint(best[e][ri]) & ~keep;
             col[e][ri] = min((int)(tag >> 2) * 16 + 4 * kb + (int)(tag & 3u), Kt * 16 - 1);
+            if (best[e][ri] > 0.5f * kNoScore && best[e][ri] > tv) {
+                tv = best[e][ri];
+                tc = col[e][ri];
+            }
         }
-        const float v0 = best[0][ri] > 0.5f * kNoScore ? best[0][ri] : -INFINITY;
-        const float v1 = best[1][ri] > 0.5f * kNoScore ? best[1][ri] : -INFINITY;
-        const bool second_is = v1 > v0;
-        float tv = second_is ? v1 : v0;
-        int tc = second_is ? col[1][ri] : col[0][ri];
 #pragma unroll
         for (int off = 16; off < 64; off <<= 1) {
             const float ov = __shfl_xor(tv, off, 64);
@@ -760,10 +795,10 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
         if (SPLIT) off += 2.0f * Xl * sqrtf(top_n2[ri]);
         if (!EXACT_MFMA) off += 1e-5f * X * X;  // (rounding of sums of squared differences)
         const float floor_of = top_v[ri] - off - fabsf(top_v[ri]) * shift;
-        bool in[2];
+        bool in[CLS];
         int un = 0, cands = 0;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
+        for (int e = 0; e < CLS; ++e) {
             const bool any = have && best[e][ri] > 0.5f * kNoScore;  // (not a number: no)
             in[e] = any && best[e][ri] + fabsf(best[e][ri]) * shift >= floor_of;
             // (a value next to zero does not hold its tag)
@@ -780,7 +815,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
         ask |= __ballot(scored[ri]);
         if (!un && !scored[ri] && kb == 0) s_key[ri * 16 + n] = (unsigned long long)(uint32_t)top[ri];  // (the only one)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
+        for (int e = 0; e < CLS; ++e) {
             const bool score = in[e] && scored[ri] && !(EXACT_MFMA && col[e][ri] == top[ri]);
             const unsigned long long bal = __ballot(score);
             if (score) {
