@@ -194,6 +194,17 @@ struct AssignJob {
     int32_t* unsure_count;
 };
 
+// Grids of `blocks` workgroups to each of `trees` trees, trees in the fast index: workgroups go to the eight XCDs in
+// turn by their number, so a tree's run behind the same L2s in one launch after the other, and what a launch
+// wrote is there for the next.  (Trees in the slow index: every tile and bucket came from another XCD's L2 or
+// from memory; 8 x 32768 keys NEW us a build.)
+static inline dim3 tree_grid(long long blocks, int trees) {
+    const long long y = blocks < 32768 ? (blocks > 0 ? blocks : 1) : 32768;
+    return dim3((unsigned)trees, (unsigned)y, (unsigned)((blocks + y - 1) / y > 0 ? (blocks + y - 1) / y : 1));
+}
+__device__ __forceinline__ int tree_block() { return (int)(blockIdx.y + blockIdx.z * gridDim.y); }
+__device__ __forceinline__ int tree_blocks() { return (int)(gridDim.y * gridDim.z); }
+
 // (all trees together) more items than this on a list, and the approximate pass takes it
 constexpr int kApproxListItems = 256 * 256;
 

@@ -1016,8 +1016,8 @@ __global__ __launch_bounds__(256) void k_open_gather(const CentroidTiles ct, con
     constexpr int TPS = assign_stage(KS);
     __shared__ int s_ids[64];
     __shared__ int s_w[4];
-    const int t = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int first = blockIdx.x * 64;  // my columns: [first, first + 64)
+    const int t = blockIdx.x, block = tree_block(), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int first = block * 64;  // my columns: [first, first + 64)
     const int32_t* ft = fill + (size_t)t * K;
     if (threadIdx.x < 64) s_ids[threadIdx.x] = -1;
     int before = 0;  // open centroids ahead of the stretch
@@ -1043,16 +1043,16 @@ __global__ __launch_bounds__(256) void k_open_gather(const CentroidTiles ct, con
         for (int j = 0; j < 4; ++j)
             if ((open_mask >> j) & 1) {
                 const int k = k0 + (int)threadIdx.x * 4 + j;
-                if (blockIdx.x == 0) ids[(size_t)t * K + at] = k;
+                if (block == 0) ids[(size_t)t * K + at] = k;
                 if (at >= first && at < first + 64) s_ids[at - first] = k;
                 ++at;
             }
         before += s_w[0] + s_w[1] + s_w[2] + s_w[3];
         __syncthreads();
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) count[t] = before;
+    if (block == 0 && threadIdx.x == 0) count[t] = before;
     const int need = min((((before + 15) / 16 + TPS - 1) / TPS) * TPS, Kt);  // tiles the assignment will walk
-    const int tile = blockIdx.x * 4 + wave;
+    const int tile = block * 4 + wave;
     if (tile >= need) return;
     const uint4* src = ct.tiles + (size_t)t * Kt * TILE_CHUNKS;
     uint4* dst = open.tiles + ((size_t)t * Kt + tile) * TILE_CHUNKS;
@@ -1076,7 +1076,7 @@ int launch_open_centroids(int KS, const CentroidTiles& ct, const int32_t* fill, 
                           int num_trees, int32_t* open_ids, int32_t* open_count,
                           const CentroidTiles& open, hipStream_t s) {
     const int Kt = assign_tiles(K);
-    const dim3 grid((Kt + 3) / 4, num_trees);
+    const dim3 grid = tree_grid((Kt + 3) / 4, num_trees);
     switch (KS) {
         case 2: hipLaunchKernelGGL((k_open_gather<2>), grid, dim3(256), 0, s, ct, fill, K, bf, Kt, open_ids, open_count, open); break;
         case 4: hipLaunchKernelGGL((k_open_gather<4>), grid, dim3(256), 0, s, ct, fill, K, bf, Kt, open_ids, open_count, open); break;

@@ -39,9 +39,9 @@ __global__ void k_fill_i32(int32_t* p, size_t n, int32_t v) {
 
 // Kernels with a wave per node: four nodes a workgroup (a workgroup of one wave costs its dispatch).
 constexpr int kNodeThreads = 256;
-static dim3 node_grid(int nodes, int trees) { return dim3((nodes + kNodeThreads / 64 - 1) / (kNodeThreads / 64), trees); }
+static dim3 node_grid(int nodes, int trees) { return tree_grid((nodes + kNodeThreads / 64 - 1) / (kNodeThreads / 64), trees); }
 __device__ __forceinline__ int node_of_wave() {
-    return __builtin_amdgcn_readfirstlane(blockIdx.x * (kNodeThreads / 64) + (threadIdx.x >> 6));
+    return __builtin_amdgcn_readfirstlane(tree_block() * (kNodeThreads / 64) + (threadIdx.x >> 6));
 }
 
 // ------------------------------------------------------------------------------------
@@ -52,11 +52,11 @@ __device__ __forceinline__ int node_of_wave() {
 // ------------------------------------------------------------------------------------
 __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_t* n_live, int32_t* fill, int32_t* slots, int32_t* counts,
                              int32_t* counters /* (kBuildCounters, T) */, CentroidTiles ct, int KS) {
-    const int t = blockIdx.y, T = gridDim.y;
+    const int t = blockIdx.x, T = gridDim.x;
     const int n_t = n_live ? min(max(n_live[t], 0), n_c) : n_c;
     const int K_t = n_live ? max((n_t + bf - 1) / bf, 1) : K;
-    const int stride = gridDim.x * blockDim.x;
-    const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
+    const int stride = tree_blocks() * blockDim.x;
+    const int i0 = tree_block() * blockDim.x + threadIdx.x;
     if (i0 == 0) {
         for (int c = 0; c < kBuildCounters; ++c) counters[(c * T + t) * kCounterStride] = 0;
     }
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_init_centroids(const void* x, 
                                                        const int32_t* n_live, int bf, int Kt,
                                                        const int32_t* fill, CentroidTiles ct, int KS) {
     __shared__ float s_all[kNodeThreads / 64][256];
-    const int k = node_of_wave(), t = blockIdx.y, lane = threadIdx.x & 63;
+    const int k = node_of_wave(), t = blockIdx.x, lane = threadIdx.x & 63;
     float* s_c = s_all[threadIdx.x >> 6];
     if (k >= K) return;  // (the whole wave)
     const int n_t = n_live ? max(min(n_live[t], n_c), 1) : n_c;
@@ -306,13 +306,13 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
     __shared__ __attribute__((aligned(16))) float s_lds[kPart + kMeanMap + kBucketThreads];
     __shared__ uint32_t s_ids[kWaves][kWaveBucket];
     static_assert(kWaves * kPiece <= kPart, "a quarter for every wave");
-    const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int t = blockIdx.x, block = tree_block(), tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int CPR = D / EPL, R = kBucketThreads / CPR;
     auto usable = [&](int k) { return !(fill != nullptr && fill[(size_t)t * K + k] >= bf); };
-    if (blockIdx.x == 0 && tid == 0) reset_round(bk, t);
-    if ((int)blockIdx.x >= large) {
-        const int k = ((int)blockIdx.x - large) * kWaves + wave;
+    if (block == 0 && tid == 0) reset_round(bk, t);
+    if (block >= large) {
+        const int k = (block - large) * kWaves + wave;
         if (k >= K) return;
         uint32_t id = (uint32_t)bk.members[bk.first((size_t)t * K + k) + lane];  // (garbage from m on)
         const int m = __builtin_amdgcn_readfirstlane(bk.counts[(size_t)t * K + k]);
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
     uint32_t* s_ord = reinterpret_cast<uint32_t*>(s_lds + kPart);
     int32_t* s_small = reinterpret_cast<int32_t*>(s_lds + kPart + kMeanMap);
     const int nbig = bk.big_count[t * kCounterStride];
-    for (int i = blockIdx.x; i < nbig; i += large) {  // uniform
+    for (int i = block; i < nbig; i += large) {  // uniform
         const int k = bk.big[(size_t)t * K + i];
         const int m = bk.counts[(size_t)t * K + k];
         const int32_t* mem = bk.members + bk.first((size_t)t * K + k);
@@ -446,7 +446,7 @@ template <typename T>
 __global__ __launch_bounds__(kNodeThreads) void k_block_mean(const void* x, size_t x_tree_stride, int K,
                                                              int D, const int32_t* slots, int bf, int lpr,
                                                              float* cent, void* out_t) {
-    const int k = node_of_wave(), t = blockIdx.y;
+    const int k = node_of_wave(), t = blockIdx.x;
     if (k >= K) return;  // (the whole wave)
     wave_block_mean<T, 8>(x, (size_t)t * x_tree_stride, D, slots + ((size_t)t * K + k) * bf, bf, lpr,
                        ((size_t)t * K + k) * D, cent, out_t);
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
     __shared__ uint64_t s_keys[kAcceptSort];
     __shared__ int32_t s_back[kWaves];
     __shared__ int32_t s_base, s_rej, s_n;
-    const int t = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int t = blockIdx.x, block = tree_block(), tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int32_t* nl = next_list + (size_t)t * n_c;
     auto key_of = [](float d, int it) { return ((uint64_t)__float_as_uint(d) << 32) | (uint32_t)it; };
@@ -477,9 +477,9 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
         fill[(size_t)t * K + k] = f;
         if (cn2 != nullptr && f >= bf) cn2[(size_t)t * Kt * 16 + k] = INFINITY;
     };
-    if (blockIdx.x == 0 && tid == 0) reset_round(bk, t);
-    if ((int)blockIdx.x >= large) {
-        const int k = ((int)blockIdx.x - large) * kWaves + wave;
+    if (block == 0 && tid == 0) reset_round(bk, t);
+    if (block >= large) {
+        const int k = (block - large) * kWaves + wave;
         int m = 0, f = 0, take = 0;
         uint64_t mine = 0;
         if (k < K) {
@@ -514,7 +514,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
     }
     // ---- the large ones --------------------------------------------------------------------------
     const int nbig = bk.big_count[t * kCounterStride];
-    for (int i = blockIdx.x; i < nbig; i += large) {  // uniform
+    for (int i = block; i < nbig; i += large) {  // uniform
         const int k = bk.big[(size_t)t * K + i];
         const size_t b = (size_t)t * K + k;
         const int m = bk.counts[b], f = fill[b];
@@ -648,8 +648,8 @@ __global__ __launch_bounds__(kLeftThreads) void k_leftover(
 // order_child[s*bf + j] = slots[order_parent[s]][j]  (or -1); order_parent == NULL: identity
 __global__ void k_compose_order(const int32_t* order_parent, int size_parent, int K_parent,
                                 const int32_t* slots, int bf, int32_t* order_child) {
-    const int t = blockIdx.y;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x;
+    const int i = tree_block() * blockDim.x + threadIdx.x;
     if (i >= size_parent * bf) return;
     const int s = i / bf, j = i % bf;
     int node = order_parent ? order_parent[(size_t)t * size_parent + s] : (s < K_parent ? s : -1);
@@ -668,9 +668,9 @@ __global__ void k_gather_rows(const void* src, size_t src_tree_stride, const int
                               int size, int D, void* dst, size_t dst_tree_stride, int dst_layout,
                               int32_t* perm_out, size_t perm_tree_stride) {
     constexpr int EPL = Elem<T>::kPerChunk;
-    const int t = blockIdx.y;
+    const int t = blockIdx.x;
     const int chunks = D / EPL;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t i = (size_t)tree_block() * blockDim.x + threadIdx.x;
     if (i >= (size_t)size * chunks) return;
     const int s = (int)(i / chunks), c = (int)(i % chunks);
     const int o = order[(size_t)t * size + s];
@@ -686,8 +686,8 @@ __global__ void k_gather_rows(const void* src, size_t src_tree_stride, const int
 template <typename T>
 __global__ void k_gather_elems(const void* src, size_t src_tree_stride, const int32_t* order,
                                int size, int D, void* dst, size_t dst_tree_stride) {
-    const int t = blockIdx.y;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x;
+    const size_t i = (size_t)tree_block() * blockDim.x + threadIdx.x;
     if (i >= (size_t)size * D) return;
     const int s = (int)(i / D), j = (int)(i % D);
     const int o = order[(size_t)t * size + s];
@@ -711,7 +711,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_radii(const void* child, size_
                                               int layout, float* radii, int32_t* counts,
                                               size_t out_stride) {
     constexpr int EPL = Elem<T>::kPerChunk;
-    const int p = node_of_wave(), t = blockIdx.y;
+    const int p = node_of_wave(), t = blockIdx.x;
     if (p >= size) return;  // (the whole wave)
     const int lane = threadIdx.x & 63;
     const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
@@ -958,12 +958,12 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
         const long long all_items = (long long)n_c * NT;
         int round = 0;  // of the level, Lloyd and packing together
         const int large = large_blocks(Kl);
-        const dim3 g_bucket(large + ceil_div(Kl, kWaves), NT);
+        const dim3 g_bucket = tree_grid(large + ceil_div(Kl, kWaves), NT);
 
         // Trees with fewer items than rows (n_live): the rounds over all items are over the first
         // ones of every tree.
         const bool ragged = n_live != nullptr && l == 1;
-        hipLaunchKernelGGL(k_level_init, dim3(min(ceil_div(Kl * bf, 256), 2048), NT), dim3(256), 0, s, n_c, Kl, bf,
+        hipLaunchKernelGGL(k_level_init, tree_grid(min(ceil_div(Kl * bf, 256), 2048), NT), dim3(256), 0, s, n_c, Kl, bf,
                            D, Kt, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters, tiles, KS);
         hipLaunchKernelGGL((k_init_centroids<T>), node_grid(Kl, NT), dim3(kNodeThreads), 0, s, x, n_c, xs, Kl, D,
                            seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, bf,
@@ -1047,39 +1047,39 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
     // layout, top-down
     if (L == 1) {
         // keys stay in insertion order
-        hipLaunchKernelGGL(k_compose_order, dim3(ceil_div(n, 256), NT), dim3(256), 0, s, nullptr, n,
+        hipLaunchKernelGGL(k_compose_order, tree_grid(ceil_div(n, 256), NT), dim3(256), 0, s, nullptr, n,
                            n, nullptr, 1, w.order[0]);
     }
     for (int l = L - 1; l >= 1; --l) {
         const int32_t* po = l == L - 1 ? nullptr : w.order[l];
-        hipLaunchKernelGGL(k_compose_order, dim3(ceil_div(t->size[l] * bf, 256), NT), dim3(256), 0,
+        hipLaunchKernelGGL(k_compose_order, tree_grid(ceil_div(t->size[l] * bf, 256), NT), dim3(256), 0,
                            s, po, t->size[l], K[l], w.slots[l], bf, w.order[l - 1]);
         if (l == L - 1)  // identity order of the root, needed by the gathers below
-            hipLaunchKernelGGL(k_compose_order, dim3(ceil_div(t->size[l], 256), NT), dim3(256), 0,
+            hipLaunchKernelGGL(k_compose_order, tree_grid(ceil_div(t->size[l], 256), NT), dim3(256), 0,
                                s, nullptr, t->size[l], K[l], nullptr, 1, w.order[l]);
     }
     // gathers
     {
         const size_t tot = (size_t)t->size[0] * (D / Elem<T>::kPerChunk);
-        hipLaunchKernelGGL((k_gather_rows<T>), dim3((unsigned)((tot + 255) / 256), NT), dim3(256),
+        hipLaunchKernelGGL((k_gather_rows<T>), tree_grid((long long)((tot + 255) / 256), NT), dim3(256),
                            0, s, keys_in, (size_t)n, w.order[0], t->size[0], D, t->keys,
                            (size_t)t->cap[0], key_layout_of(t->layout), t->perm, (size_t)t->cap[0]);
         if (values_in && t->values) {
             if (t->vdim % Elem<T>::kPerChunk == 0) {
                 const size_t totv = (size_t)t->size[0] * (t->vdim / Elem<T>::kPerChunk);
-                hipLaunchKernelGGL((k_gather_rows<T>), dim3((unsigned)((totv + 255) / 256), NT),
+                hipLaunchKernelGGL((k_gather_rows<T>), tree_grid((long long)((totv + 255) / 256), NT),
                                    dim3(256), 0, s, values_in, (size_t)n, w.order[0], t->size[0],
                                    t->vdim, t->values, (size_t)t->cap[0], (int)HIRA_ROW_MAJOR, nullptr, (size_t)0);
             } else {
                 const size_t totv = (size_t)t->size[0] * t->vdim;
-                hipLaunchKernelGGL((k_gather_elems<T>), dim3((unsigned)((totv + 255) / 256), NT),
+                hipLaunchKernelGGL((k_gather_elems<T>), tree_grid((long long)((totv + 255) / 256), NT),
                                    dim3(256), 0, s, values_in, (size_t)n, w.order[0], t->size[0],
                                    t->vdim, t->values, (size_t)t->cap[0]);
             }
         }
         for (int l = 1; l < L; ++l) {
             const size_t totc = (size_t)t->size[l] * (D / Elem<T>::kPerChunk);
-            hipLaunchKernelGGL((k_gather_rows<T>), dim3((unsigned)((totc + 255) / 256), NT),
+            hipLaunchKernelGGL((k_gather_rows<T>), tree_grid((long long)((totc + 255) / 256), NT),
                                dim3(256), 0, s, w.cent_t[l], (size_t)K[l], w.order[l], t->size[l], D,
                                t->centers[l], (size_t)t->cap[l], center_layout_of(t->layout), nullptr, (size_t)0);
         }
