@@ -51,7 +51,7 @@ __device__ __forceinline__ int node_of_wave() {
 //    first ceil(n_t / bf) centroids only: the others count as full.
 // ------------------------------------------------------------------------------------
 __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_t* n_live, int32_t* fill, int32_t* slots, int32_t* counts,
-                             int32_t* counters /* (kBuildCounters, T) */, CentroidTiles ct, int KS) {
+                             int32_t* counters /* (kBuildCounters, T) */, float* absmax /* (T, kAbsCopies, D) or NULL */, CentroidTiles ct, int KS) {
     const int t = blockIdx.x, T = gridDim.x;
     const int n_t = n_live ? min(max(n_live[t], 0), n_c) : n_c;
     const int K_t = n_live ? max((n_t + bf - 1) / bf, 1) : K;
@@ -60,6 +60,8 @@ __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_
     if (i0 == 0) {
         for (int c = 0; c < kBuildCounters; ++c) counters[(c * T + t) * kCounterStride] = 0;
     }
+    if (absmax != nullptr)
+        for (int i = i0; i < kAbsCopies * D; i += stride) absmax[(size_t)t * kAbsCopies * D + i] = 0.0f;
     for (int i = i0; i < K; i += stride) {
         fill[(size_t)t * K + i] = i >= K_t ? bf : 0;
         counts[(size_t)t * K + i] = 0;
@@ -645,135 +647,199 @@ __global__ __launch_bounds__(kLeftThreads) void k_leftover(
 // ------------------------------------------------------------------------------------
 // 6. final layout
 // ------------------------------------------------------------------------------------
-// order_child[s*bf + j] = slots[order_parent[s]][j]  (or -1); order_parent == NULL: identity
-__global__ void k_compose_order(const int32_t* order_parent, int size_parent, int K_parent,
-                                const int32_t* slots, int bf, int32_t* order_child) {
-    const int t = blockIdx.x;
-    const int i = tree_block() * blockDim.x + threadIdx.x;
-    if (i >= size_parent * bf) return;
-    const int s = i / bf, j = i % bf;
-    int node = order_parent ? order_parent[(size_t)t * size_parent + s] : (s < K_parent ? s : -1);
-    int v = -1;
-    if (slots == nullptr)
-        v = node;  // bf == 1: plain copy / identity
-    else if (node >= 0)
-        v = slots[((size_t)t * K_parent + node) * bf + j];
-    order_child[(size_t)t * size_parent * bf + i] = v;
+// One level: every node of level l gets its children's rows (keys and values, or block centres of level
+// l - 1) into their slots, its radius and its count:
+//   radius = max over children (||child - centre|| + r_child), -inf when there is none.
+// A wave per node.  Which cluster lies in a slot is followed from the root down (the clusters of the top level
+// lie in order; slots[i][k] are the children of cluster k of level i): a chain of l' < L loads that no launch
+// has to prepare.  `lpr` lanes (a power of two) hold a row in 16-byte chunks (a chunk is contiguous in either
+// layout), 64 / lpr children a step, eight steps on their way.  The rows are read once for all of it: bound
+// by the bytes moved, 8 x 131072 keys and values of 256 bytes with their radii and the largest magnitude
+// per channel 214 us, 5.0 TB/s.  (As launches of their own -- orders, keys, values, centres, radii,
+// magnitudes -- a level-4 index of those took 360 us, now 235; 8 x 32768 keys, three levels, 82, now 50.)
+struct PlaceLevel {
+    const void* rows;                // (T, rows_stride, D) what the children are: keys as they came, or block centres
+    size_t rows_stride;
+    const int32_t* slots[HIRA_MAX_LEVELS];  // (T, K[i], bf)
+    int32_t K[HIRA_MAX_LEVELS];
+    int32_t num_levels, level, size, bf, D, lpr;
+    void* child;                     // (T, child_stride, D) where they go
+    size_t child_stride;
+    int32_t child_layout, center_layout;
+    const float* child_radii;        // (T, child_stride), or NULL: keys have none
+    const void* cent;                // (T, K[level], D) the level's block centres
+    void* top;                       // top level: where those go themselves, (T, out_stride, D)
+    float* radii;                    // (T, out_stride)
+    int32_t* counts;
+    size_t out_stride;
+    int32_t* perm;                   // level 1: (T, child_stride)
+    const void* values_in;           // level 1: (T, rows_stride, vdim) -> (T, child_stride, vdim), or NULL
+    void* values;
+    int32_t vdim, lpr_v;             // (a value row in steps of lpr_v <= 64 lanes)
+    float* absmax;                   // ABSMAX: (T, kAbsCopies, D) joined by the largest finite magnitudes per channel
+};
+
+// 16 bytes that nothing reads for a while: they push nothing out of the caches on their way
+__device__ __forceinline__ void store_once(void* p, const uint4& v) {
+    typedef __attribute__((ext_vector_type(4))) uint32_t vec4;
+    __builtin_nontemporal_store(vec4{v.x, v.y, v.z, v.w}, reinterpret_cast<vec4*>(p));
 }
 
-// dst[t][s] = src[t][order[t][s]] (zero row for -1), a thread per 16-byte chunk of a row (a chunk
-// is contiguous in either layout).  perm_out != NULL: also writes perm.
-template <typename T>
-__global__ void k_gather_rows(const void* src, size_t src_tree_stride, const int32_t* order,
-                              int size, int D, void* dst, size_t dst_tree_stride, int dst_layout,
-                              int32_t* perm_out, size_t perm_tree_stride) {
+template <typename T, bool ABSMAX>
+__global__ __launch_bounds__(kNodeThreads) void k_place(const PlaceLevel pl) {
     constexpr int EPL = Elem<T>::kPerChunk;
-    const int t = blockIdx.x;
-    const int chunks = D / EPL;
+    constexpr int U = 8;
+    __shared__ float s_abs[ABSMAX ? kNodeThreads / 64 : 1][256];
+    const int p = node_of_wave(), t = blockIdx.x, lane = threadIdx.x & 63;
+    const int bf = pl.bf, D = pl.D, lpr = pl.lpr;
+    const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
+    const bool chunk_ok = ch * EPL < D;
+    float big[EPL];
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) big[e] = 0.0f;
+    if (p < pl.size) {  // (uniform in the wave)
+        int id = p;  // the cluster that lies in slot p
+        for (int i = pl.level; i < pl.num_levels - 1; ++i) id /= bf;
+        for (int i = pl.num_levels - 1; i > pl.level; --i) {  // (from cluster `id` of level i to one of level i - 1)
+            int at = p;
+            for (int j = pl.level; j < i - 1; ++j) at /= bf;
+            id = id >= 0 ? pl.slots[i][((size_t)t * pl.K[i] + id) * bf + at % bf] : -1;
+        }
+        const int own = max(id, 0);
+        const int mine = lane < bf && id >= 0 ? pl.slots[pl.level][((size_t)t * pl.K[pl.level] + own) * bf + lane] : -1;
+        const unsigned long long live = __ballot(mine >= 0);
+        const size_t s0 = (size_t)t * pl.child_stride + (size_t)p * bf;  // slots of the children
+        const float my_radius = mine >= 0 && pl.child_radii ? pl.child_radii[s0 + lane] : 0.0f;
+        if (pl.perm && lane < bf) pl.perm[s0 + lane] = mine;
+        const uint4 craw = load_chunk<T>(pl.cent, ((size_t)t * pl.K[pl.level] + own) * D, chunk_ok ? ch : 0);
+        float cf[EPL];
+        unpack<T>(craw, cf);
+        if (pl.top && rg == 0 && chunk_ok)
+            *reinterpret_cast<uint4*>(reinterpret_cast<T*>(pl.top) + (size_t)t * pl.out_stride * D +
+                                      elem_index(pl.center_layout, D, (size_t)p, ch * EPL)) = craw;
+        T* const child = reinterpret_cast<T*>(pl.child) + (size_t)t * pl.child_stride * D;
+        float r = -INFINITY;
+        for (int j0 = 0; j0 < bf; j0 += U * groups) {  // (uniform trip count: the sums meet in shuffles)
+            uint4 raw[U];
+            int it[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {  // (a child that is none: row 0)
+                const int j = j0 + u * groups + rg;
+                it[u] = __shfl(mine, j & 63, 64);
+                raw[u] = load_chunk<T>(pl.rows, ((size_t)t * pl.rows_stride + max(it[u], 0)) * D, chunk_ok ? ch : 0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int j = j0 + u * groups + rg;
+                const bool have = j < bf && it[u] >= 0;
+                if (j < bf && chunk_ok)
+                    *reinterpret_cast<uint4*>(child + elem_index(pl.child_layout, D, (size_t)p * bf + j, ch * EPL)) =
+                        make_uint4(have ? raw[u].x : 0u, have ? raw[u].y : 0u, have ? raw[u].z : 0u, have ? raw[u].w : 0u);
+                float f[EPL];
+                unpack<T>(raw[u], f);
+                float ss = 0.0f;
+#pragma unroll
+                for (int q = 0; q < EPL; ++q) {
+                    const float df = f[q] - cf[q];
+                    ss += df * df;
+                }
+                if (!chunk_ok) ss = 0.0f;
+                ss = group_sum_of(ss, lpr);
+                const float radius = __shfl(my_radius, j & 63, 64);
+                if (have) {
+                    float v = sqrtf(ss);
+                    if (pl.child_radii) v += radius;
+                    r = fmaxf(r, v);
+                }
+                if constexpr (ABSMAX) {
+#pragma unroll
+                    for (int q = 0; q < EPL; ++q) {
+                        const float a = fabsf(f[q]);
+                        big[q] = have && a < INFINITY && a > big[q] ? a : big[q];
+                    }
+                }
+            }
+        }
+        if (pl.values) {
+            const int lpr_v = pl.lpr_v, rg_v = lane / lpr_v, ch_v = lane % lpr_v, groups_v = 64 / lpr_v;
+            T* const values = reinterpret_cast<T*>(pl.values);
+            for (int c0 = 0; c0 * EPL < pl.vdim; c0 += lpr_v) {
+                const int c = c0 + ch_v;
+                const bool ok_v = c * EPL < pl.vdim;
+                for (int j0 = 0; j0 < bf; j0 += U * groups_v) {
+                    uint4 raw[U];
+                    int it[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        it[u] = __shfl(mine, (j0 + u * groups_v + rg_v) & 63, 64);
+                        raw[u] = load_chunk<T>(pl.values_in, ((size_t)t * pl.rows_stride + max(it[u], 0)) * pl.vdim, ok_v ? c : 0);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int j = j0 + u * groups_v + rg_v;
+                        const bool have = it[u] >= 0;
+                        if (j < bf && ok_v)
+                            store_once(values + (s0 + j) * pl.vdim + c * EPL, have ? raw[u] : make_uint4(0, 0, 0, 0));
+                    }
+                }
+            }
+        }
+        for (int off = lpr; off < 64; off <<= 1) r = fmaxf(r, __shfl_xor(r, off, 64));
+        if (lane == 0) {
+            // a few ulp of head room: the bound must survive fp32 rounding of this sum
+            if (r > 0.0f) r = r * (1.0f + 4.0f * 1.1920929e-7f) + 1e-30f;
+            pl.radii[(size_t)t * pl.out_stride + p] = r;
+            pl.counts[(size_t)t * pl.out_stride + p] = __popcll(live);
+        }
+    }
+    if constexpr (ABSMAX) {
+        // integer maxima: the bits of non-negative floats order like unsigned integers, and a maximum does not
+        // depend on the order of arrival.  (Into kAbsCopies places in turn: workgroups of a tree that all join
+        // the same 128 numbers wait for each other, 236 us for this launch instead of 214.)
+        const int wave = threadIdx.x >> 6;
+#pragma unroll
+        for (int q = 0; q < EPL; ++q) {
+            float m = big[q];
+            for (int off = lpr; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+            if (rg == 0 && chunk_ok) s_abs[wave][ch * EPL + q] = m;
+        }
+        __syncthreads();
+        for (int j = threadIdx.x; j < D; j += kNodeThreads) {
+            float m = s_abs[0][j];
+#pragma unroll
+            for (int w = 1; w < kNodeThreads / 64; ++w) m = fmaxf(m, s_abs[w][j]);
+            atomicMax(reinterpret_cast<unsigned*>(pl.absmax) + ((size_t)t * kAbsCopies + tree_block() % kAbsCopies) * D + j, __float_as_uint(m));
+        }
+    }
+}
+
+// An index of one level: keys and values as they came, perm the numbers in order; a thread per 16-byte chunk
+// of a row (a chunk is contiguous in either layout).
+template <typename T>
+__global__ void k_copy_rows(const void* src, int size, int D, void* dst, size_t dst_tree_stride, int dst_layout, int32_t* perm) {
+    constexpr int EPL = Elem<T>::kPerChunk;
+    const int t = blockIdx.x, chunks = D / EPL;
     const size_t i = (size_t)tree_block() * blockDim.x + threadIdx.x;
     if (i >= (size_t)size * chunks) return;
     const int s = (int)(i / chunks), c = (int)(i % chunks);
-    const int o = order[(size_t)t * size + s];
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (o >= 0) v = load_chunk<T>(src, ((size_t)t * src_tree_stride + o) * D, c);
-    T* out = reinterpret_cast<T*>(dst) + (size_t)t * dst_tree_stride * D +
-             elem_index(dst_layout, D, (size_t)s, c * EPL);
-    *reinterpret_cast<uint4*>(out) = v;
-    if (perm_out && c == 0) perm_out[(size_t)t * perm_tree_stride + s] = o;
+    *reinterpret_cast<uint4*>(reinterpret_cast<T*>(dst) + (size_t)t * dst_tree_stride * D + elem_index(dst_layout, D, (size_t)s, c * EPL)) =
+        load_chunk<T>(src, ((size_t)t * size + s) * D, c);
+    if (perm && c == 0) perm[(size_t)t * dst_tree_stride + s] = s;
 }
 
-// the same, a thread per element: value rows whose length is not a multiple of 16 bytes
+// dst[t][s] = src[t][perm[t][s]] (zero row for -1), a thread per element: value rows whose length is not a
+// multiple of 16 bytes
 template <typename T>
-__global__ void k_gather_elems(const void* src, size_t src_tree_stride, const int32_t* order,
+__global__ void k_gather_elems(const void* src, size_t src_tree_stride, const int32_t* perm,
                                int size, int D, void* dst, size_t dst_tree_stride) {
     const int t = blockIdx.x;
     const size_t i = (size_t)tree_block() * blockDim.x + threadIdx.x;
     if (i >= (size_t)size * D) return;
     const int s = (int)(i / D), j = (int)(i % D);
-    const int o = order[(size_t)t * size + s];
+    const int o = perm[(size_t)t * dst_tree_stride + s];
     float v = 0.0f;
     if (o >= 0) v = load_elem<T>(src, ((size_t)t * src_tree_stride + o) * D + j);
     store_elem<T>(dst, ((size_t)t * dst_tree_stride + s) * D + j, v);
-}
-
-// counts[p] = children in use; radii[p] = max over them of (||child - centre|| + r_child),
-// -inf when there is none.  One wave per node: `lpr` lanes (a power of two) hold a row in
-// 16-byte chunks (a chunk is contiguous in either layout), 64 / lpr children a step, eight steps on their
-// way.  Bound by the read of the children: 8 x 131072 rows of 256 bytes
-// 79 -> 75 us, 8 x 32768 18.6 -> 15
-template <typename T>
-__global__ __launch_bounds__(kNodeThreads) void k_radii(const void* child, size_t child_tree_stride,
-                                              const float* child_radii,
-                                              size_t child_radii_stride,
-                                              const int32_t* child_order, int size_child,
-                                              const void* centers, size_t center_tree_stride,
-                                              int size, int bf, int D, int lpr, int child_layout,
-                                              int layout, float* radii, int32_t* counts,
-                                              size_t out_stride) {
-    constexpr int EPL = Elem<T>::kPerChunk;
-    const int p = node_of_wave(), t = blockIdx.x;
-    if (p >= size) return;  // (the whole wave)
-    const int lane = threadIdx.x & 63;
-    const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
-    const bool chunk_ok = ch * EPL < D;
-    float cf[EPL];
-    {
-        uint4 raw = make_uint4(0, 0, 0, 0);
-        if (chunk_ok)
-            raw = *reinterpret_cast<const uint4*>(
-                reinterpret_cast<const T*>(centers) + (size_t)t * center_tree_stride * D +
-                elem_index(layout, D, (size_t)p, ch * EPL));
-        unpack<T>(raw, cf);
-    }
-    // (the children's orders and radii in one load each, U rows a lane group in flight; size_child =
-    // size * bf, and bf <= 64)
-    constexpr int U = 8;
-    const size_t s0 = (size_t)p * bf;
-    const bool mine = lane < bf && s0 + lane < (size_t)size_child && child_order[(size_t)t * size_child + s0 + lane] >= 0;
-    const float my_radius = mine && child_radii ? child_radii[(size_t)t * child_radii_stride + s0 + lane] : 0.0f;
-    const unsigned long long live = __ballot(mine);
-    const int c = __popcll(live);
-    float r = -INFINITY;
-    for (int j0 = 0; j0 < bf; j0 += U * groups) {  // (uniform trip count: the sums meet in shuffles)
-        uint4 raw[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {  // (a child that is none: the first slot's row)
-            const int j = j0 + u * groups + rg;
-            const size_t row = s0 + (j < bf && ((live >> (j & 63)) & 1) ? j : 0);
-            raw[u] = *reinterpret_cast<const uint4*>(
-                reinterpret_cast<const T*>(child) + (size_t)t * child_tree_stride * D +
-                elem_index(child_layout, D, row, chunk_ok ? ch * EPL : 0));
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int j = j0 + u * groups + rg;
-            float f[EPL];
-            unpack<T>(raw[u], f);
-            float ss = 0.0f;
-#pragma unroll
-            for (int q = 0; q < EPL; ++q) {
-                const float df = f[q] - cf[q];
-                ss += df * df;
-            }
-            if (!chunk_ok) ss = 0.0f;
-            ss = group_sum_of(ss, lpr);
-            const float radius = __shfl(my_radius, j & 63, 64);
-            if (j < bf && ((live >> (j & 63)) & 1)) {
-                float v = sqrtf(ss);
-                if (child_radii) v += radius;
-                r = fmaxf(r, v);
-            }
-        }
-    }
-    for (int off = lpr; off < 64; off <<= 1) {
-        r = fmaxf(r, __shfl_xor(r, off, 64));
-    }
-    if (lane == 0) {
-        // a few ulp of head room: the bound must survive fp32 rounding of this sum
-        if (r > 0.0f) r = r * (1.0f + 4.0f * 1.1920929e-7f) + 1e-30f;
-        radii[(size_t)t * out_stride + p] = r;
-        counts[(size_t)t * out_stride + p] = c;
-    }
 }
 
 // ------------------------------------------------------------------------------------
@@ -804,7 +870,7 @@ struct BuildWs {
     int32_t *counts, *fill;
     int32_t* slots[HIRA_MAX_LEVELS];
     void* cent_t[HIRA_MAX_LEVELS];
-    int32_t* order[HIRA_MAX_LEVELS];
+    float* absmax;  // (T, kAbsCopies, D), zero: an index with an 8-bit shadow; else NULL
     size_t total;
 };
 
@@ -869,13 +935,12 @@ static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
     for (int l = 0; l < HIRA_MAX_LEVELS; ++l) {
         b->slots[l] = nullptr;
         b->cent_t[l] = nullptr;
-        b->order[l] = nullptr;
     }
     for (int l = 1; l < L; ++l) {
         b->slots[l] = c.take<int32_t>((size_t)T * K[l] * bf);
         b->cent_t[l] = c.take<char>((size_t)T * K[l] * D * esize);
     }
-    for (int l = 0; l < L; ++l) b->order[l] = c.take<int32_t>((size_t)T * t->size[l]);
+    b->absmax = t->layout == HIRA_TILE16_Q8 ? c.take<float>((size_t)T * kAbsCopies * D) : nullptr;
     b->total = (c.used + 255) & ~(size_t)255;
 }
 
@@ -927,6 +992,7 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
     const int KS = assign_ks(t->dtype, D);
     for (int l = 1; l < L; ++l) {
         if (level_is_small(t, K[l - 1], K[l]) && n_live == nullptr) {  // this one and all above it in one launch
+            if (l == 1 && w.absmax != nullptr) fill_i32(reinterpret_cast<int32_t*>(w.absmax), (size_t)NT * kAbsCopies * D, 0, s);
             SmallLevels p{};
             p.x = l == 1 ? keys_in : w.cent_t[l - 1];
             p.first = l;
@@ -964,7 +1030,7 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
         // ones of every tree.
         const bool ragged = n_live != nullptr && l == 1;
         hipLaunchKernelGGL(k_level_init, tree_grid(min(ceil_div(Kl * bf, 256), 2048), NT), dim3(256), 0, s, n_c, Kl, bf,
-                           D, Kt, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters, tiles, KS);
+                           D, Kt, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters, l == 1 ? w.absmax : nullptr, tiles, KS);
         hipLaunchKernelGGL((k_init_centroids<T>), node_grid(Kl, NT), dim3(kNodeThreads), 0, s, x, n_c, xs, Kl, D,
                            seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, bf,
                            Kt, w.fill, tiles, KS);
@@ -1044,59 +1110,65 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
         HIRA_CHECK_LAUNCH("build level");
     }
 
-    // layout, top-down
+    // layout and radii, bottom-up
+    const bool whole_v = t->vdim % EPL == 0, have_v = values_in && t->values;
     if (L == 1) {
-        // keys stay in insertion order
-        hipLaunchKernelGGL(k_compose_order, tree_grid(ceil_div(n, 256), NT), dim3(256), 0, s, nullptr, n,
-                           n, nullptr, 1, w.order[0]);
-    }
-    for (int l = L - 1; l >= 1; --l) {
-        const int32_t* po = l == L - 1 ? nullptr : w.order[l];
-        hipLaunchKernelGGL(k_compose_order, tree_grid(ceil_div(t->size[l] * bf, 256), NT), dim3(256), 0,
-                           s, po, t->size[l], K[l], w.slots[l], bf, w.order[l - 1]);
-        if (l == L - 1)  // identity order of the root, needed by the gathers below
-            hipLaunchKernelGGL(k_compose_order, tree_grid(ceil_div(t->size[l], 256), NT), dim3(256), 0,
-                               s, nullptr, t->size[l], K[l], nullptr, 1, w.order[l]);
-    }
-    // gathers
-    {
-        const size_t tot = (size_t)t->size[0] * (D / Elem<T>::kPerChunk);
-        hipLaunchKernelGGL((k_gather_rows<T>), tree_grid((long long)((tot + 255) / 256), NT), dim3(256),
-                           0, s, keys_in, (size_t)n, w.order[0], t->size[0], D, t->keys,
-                           (size_t)t->cap[0], key_layout_of(t->layout), t->perm, (size_t)t->cap[0]);
-        if (values_in && t->values) {
-            if (t->vdim % Elem<T>::kPerChunk == 0) {
-                const size_t totv = (size_t)t->size[0] * (t->vdim / Elem<T>::kPerChunk);
-                hipLaunchKernelGGL((k_gather_rows<T>), tree_grid((long long)((totv + 255) / 256), NT),
-                                   dim3(256), 0, s, values_in, (size_t)n, w.order[0], t->size[0],
-                                   t->vdim, t->values, (size_t)t->cap[0], (int)HIRA_ROW_MAJOR, nullptr, (size_t)0);
-            } else {
-                const size_t totv = (size_t)t->size[0] * t->vdim;
-                hipLaunchKernelGGL((k_gather_elems<T>), tree_grid((long long)((totv + 255) / 256), NT),
-                                   dim3(256), 0, s, values_in, (size_t)n, w.order[0], t->size[0],
-                                   t->vdim, t->values, (size_t)t->cap[0]);
-            }
-        }
-        for (int l = 1; l < L; ++l) {
-            const size_t totc = (size_t)t->size[l] * (D / Elem<T>::kPerChunk);
-            hipLaunchKernelGGL((k_gather_rows<T>), tree_grid((long long)((totc + 255) / 256), NT),
-                               dim3(256), 0, s, w.cent_t[l], (size_t)K[l], w.order[l], t->size[l], D,
-                               t->centers[l], (size_t)t->cap[l], center_layout_of(t->layout), nullptr, (size_t)0);
+        const size_t tot = (size_t)n * (D / EPL);
+        hipLaunchKernelGGL((k_copy_rows<T>), tree_grid((long long)((tot + 255) / 256), NT), dim3(256), 0, s, keys_in, n, D,
+                           t->keys, (size_t)t->cap[0], key_layout_of(t->layout), t->perm);
+        if (have_v && whole_v) {
+            const size_t totv = (size_t)n * (t->vdim / EPL);
+            hipLaunchKernelGGL((k_copy_rows<T>), tree_grid((long long)((totv + 255) / 256), NT), dim3(256), 0, s, values_in,
+                               n, t->vdim, t->values, (size_t)t->cap[0], (int)HIRA_ROW_MAJOR, nullptr);
         }
     }
-    // radii and counts, bottom-up
     for (int l = 1; l < L; ++l) {
-        const void* child = l == 1 ? t->keys : t->centers[l - 1];
-        const float* crad = l == 1 ? nullptr : t->radii[l - 1];
-        hipLaunchKernelGGL((k_radii<T>), node_grid(t->size[l], NT), dim3(kNodeThreads), 0, s, child,
-                           (size_t)t->cap[l - 1], crad, (size_t)t->cap[l - 1], w.order[l - 1],
-                           t->size[l - 1], t->centers[l], (size_t)t->cap[l], t->size[l], bf, D, lpr,
-                           l == 1 ? key_layout_of(t->layout) : center_layout_of(t->layout),
-                           center_layout_of(t->layout), t->radii[l], t->counts[l], (size_t)t->cap[l]);
+        PlaceLevel p{};
+        p.rows = l == 1 ? keys_in : w.cent_t[l - 1];
+        p.rows_stride = (size_t)K[l - 1];
+        for (int i = l; i < L; ++i) {
+            p.slots[i] = w.slots[i];
+            p.K[i] = K[i];
+        }
+        p.num_levels = L;
+        p.level = l;
+        p.size = t->size[l];
+        p.bf = bf;
+        p.D = D;
+        p.lpr = lpr;
+        p.child = l == 1 ? t->keys : t->centers[l - 1];
+        p.child_stride = (size_t)t->cap[l - 1];
+        p.child_layout = l == 1 ? key_layout_of(t->layout) : center_layout_of(t->layout);
+        p.center_layout = center_layout_of(t->layout);
+        p.child_radii = l == 1 ? nullptr : t->radii[l - 1];
+        p.cent = w.cent_t[l];
+        p.top = l == L - 1 ? t->centers[l] : nullptr;
+        p.radii = t->radii[l];
+        p.counts = t->counts[l];
+        p.out_stride = (size_t)t->cap[l];
+        if (l == 1) {
+            p.perm = t->perm;
+            if (have_v && whole_v) {
+                p.values_in = values_in;
+                p.values = t->values;
+                p.vdim = t->vdim;
+                p.lpr_v = 2;
+                while (p.lpr_v < 64 && p.lpr_v * EPL < t->vdim) p.lpr_v <<= 1;
+            }
+            p.absmax = w.absmax;
+        }
+        if (l == 1 && w.absmax != nullptr)
+            hipLaunchKernelGGL((k_place<T, true>), node_grid(t->size[l], NT), dim3(kNodeThreads), 0, s, p);
+        else
+            hipLaunchKernelGGL((k_place<T, false>), node_grid(t->size[l], NT), dim3(kNodeThreads), 0, s, p);
+    }
+    if (have_v && !whole_v) {
+        const size_t totv = (size_t)t->size[0] * t->vdim;
+        hipLaunchKernelGGL((k_gather_elems<T>), tree_grid((long long)((totv + 255) / 256), NT), dim3(256), 0, s, values_in,
+                           (size_t)n, t->perm, t->size[0], t->vdim, t->values, (size_t)t->cap[0]);
     }
     HIRA_CHECK_LAUNCH("build layout");
-    if (t->layout == HIRA_TILE16_Q8)  // steps from all keys, then the 8-bit shadow
-        return hira_quantize(t, 0, t->size[0], 1, s);
+    if (w.absmax != nullptr) return quantize_with(t, w.absmax, kAbsCopies, s);  // the 8-bit shadow, its steps from all keys
     return HIRA_OK;
 }
 

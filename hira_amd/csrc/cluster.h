@@ -7,6 +7,11 @@
 
 namespace hira {
 
+// quantize.hip: the 8-bit shadow of all keys, its steps from the largest magnitudes per channel,
+// (T, copies, D)
+int quantize_with(const HiraTree* tree, const float* absmax, int copies, hipStream_t s);
+constexpr int kAbsCopies = 32;
+
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     z += 0x9E3779B97F4A7C15ull;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;

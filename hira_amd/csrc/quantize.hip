@@ -61,9 +61,14 @@ __global__ void k_zero_f32(float* p, size_t n) {
     if (i < n) p[i] = 0.0f;
 }
 
-__global__ void k_step_from_absmax(float* kscale, size_t n) {
+// n steps of D channels a tree; absmax: `copies` maxima a channel, (n / D, copies, D)
+__global__ void k_step_from_absmax(float* kscale, const float* absmax, int copies, int D, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) kscale[i] = fmaxf(kscale[i] / 127.0f, kMinStep);
+    if (i >= n) return;
+    const float* at = absmax + i / D * copies * D + i % D;
+    float m = 0.0f;
+    for (int c = 0; c < copies; ++c) m = fmaxf(m, at[(size_t)c * D]);
+    kscale[i] = fmaxf(m / 127.0f, kMinStep);
 }
 
 // one wave per level-1 node: its bf key slots -> shadow bytes, error bound of the node.  A lane takes
@@ -120,6 +125,21 @@ __global__ __launch_bounds__(kQuantThreads) void k_quantize(const uint16_t* keys
     if (lane == 0) keps[(size_t)t * cap1 + node] = worst;
 }
 
+static void quantize_nodes(const HiraTree* tree, int node_first, int nodes, hipStream_t s) {
+    hipLaunchKernelGGL(k_quantize, dim3((nodes + kQuantWaves - 1) / kQuantWaves, tree->num_trees), dim3(kQuantThreads), 0, s,
+                       reinterpret_cast<const uint16_t*>(tree->keys), tree->keys8, tree->kscale, tree->perm, tree->keps,
+                       (size_t)tree->cap[0], (size_t)tree->cap[1], node_first, nodes, tree->bf, tree->dim);
+}
+
+int quantize_with(const HiraTree* tree, const float* absmax, int copies, hipStream_t s) {
+    const size_t n = (size_t)tree->num_trees * tree->dim;
+    hipLaunchKernelGGL(k_step_from_absmax, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, tree->kscale, absmax, copies,
+                       tree->dim, n);
+    quantize_nodes(tree, 0, tree->size[1], s);
+    HIRA_CHECK_LAUNCH("quantize kernel");
+    return HIRA_OK;
+}
+
 }  // namespace hira
 
 using namespace hira;
@@ -155,13 +175,10 @@ extern "C" int hira_quantize(const HiraTree* tree, int32_t slot_first, int32_t s
             hipLaunchKernelGGL(k_absmax, dim3(parts, T), dim3(kQuantThreads), 0, s, keys,
                                (size_t)tree->cap[0], rows, D, tree->kscale);
         hipLaunchKernelGGL(k_step_from_absmax, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           tree->kscale, n);
+                           tree->kscale, tree->kscale, 1, D, n);
     }
     if (slot_count == 0) return HIRA_OK;
-    const int nodes = slot_count / bf;
-    hipLaunchKernelGGL(k_quantize, dim3((nodes + kQuantWaves - 1) / kQuantWaves, T), dim3(kQuantThreads), 0, s, keys,
-                       tree->keys8, tree->kscale, tree->perm, tree->keps, (size_t)tree->cap[0],
-                       (size_t)tree->cap[1], slot_first / bf, nodes, bf, D);
+    quantize_nodes(tree, slot_first / bf, slot_count / bf, s);
     HIRA_CHECK_LAUNCH("quantize kernel");
     return HIRA_OK;
 }
