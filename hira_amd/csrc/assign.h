@@ -222,6 +222,23 @@ __device__ __forceinline__ void put_result(const AssignJob& job, int t, int it, 
     }
 }
 
+// The current device, for what is asked once per kernel and device.
+constexpr int kMaxDevices = 64;
+static inline int current_device() {
+    int dev = 0;
+    return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices ? dev : -1;
+}
+// (more than 64 KiB of dynamic LDS has to be asked for: once per kernel and device)
+static inline int ask_for_lds(const void* kernel, size_t smem, int* asked, int dev) {
+    if (dev < 0) return fail(HIRA_ELAUNCH, "assignment: no current device");
+    if (__atomic_load_n(&asked[dev], __ATOMIC_RELAXED) == 0) {
+        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
+            return fail(HIRA_ELAUNCH, "assignment: %zu bytes of LDS refused", smem);
+        __atomic_store_n(&asked[dev], 1, __ATOMIC_RELAXED);
+    }
+    return HIRA_OK;
+}
+
 // assign_mfma.hip
 int assign_ks(int dtype, int D);        // KS of the operand tiles for rows of D columns, 0: none
 bool assign_exact_on_mfma(int dtype, int D);

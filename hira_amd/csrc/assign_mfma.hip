@@ -1112,23 +1112,6 @@ int launch_cent_prep(int dim, const float* cent, int K, int num_trees, const int
     return HIRA_OK;
 }
 
-// The current device, for what is asked once per kernel and device.
-constexpr int kMaxDevices = 64;
-static int current_device() {
-    int dev = 0;
-    return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices ? dev : -1;
-}
-// (more than 64 KiB of dynamic LDS has to be asked for: once per kernel and device)
-static int ask_for_lds(const void* kernel, size_t smem, int* asked, int dev) {
-    if (dev < 0) return fail(HIRA_ELAUNCH, "assignment: no current device");
-    if (__atomic_load_n(&asked[dev], __ATOMIC_RELAXED) == 0) {
-        if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess)
-            return fail(HIRA_ELAUNCH, "assignment: %zu bytes of LDS refused", smem);
-        __atomic_store_n(&asked[dev], 1, __ATOMIC_RELAXED);
-    }
-    return HIRA_OK;
-}
-
 template <int KS>
 static int launch_exact(const AssignJob& job, hipStream_t s) {
     const int Kt = assign_tiles(job.K);

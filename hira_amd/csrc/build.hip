@@ -450,8 +450,9 @@ __global__ __launch_bounds__(kNodeThreads) void k_block_mean(const void* x, size
                                                              float* cent, void* out_t) {
     const int k = node_of_wave(), t = blockIdx.x;
     if (k >= K) return;  // (the whole wave)
-    wave_block_mean<T, 8>(x, (size_t)t * x_tree_stride, D, slots + ((size_t)t * K + k) * bf, bf, lpr,
-                       ((size_t)t * K + k) * D, cent, out_t);
+    wave_block_mean<T, 8>(x, (size_t)t * x_tree_stride, D,
+                          (threadIdx.x & 63) < bf ? slots[((size_t)t * K + k) * bf + (threadIdx.x & 63)] : -1, bf, lpr,
+                          ((size_t)t * K + k) * D, cent, out_t);
 }
 
 // ------------------------------------------------------------------------------------
@@ -889,14 +890,13 @@ static void cluster_counts(int n, int bf, int L, int* K) {
 }
 
 // Whether a workgroup a tree takes this level, and with it all above (small_levels.hip).  It spends on a
-// round what its items times its centroids take one compute unit, the launches what launches take.  Trees x
-// items x centroids, launches / one workgroup a tree: 8 x 512 x 16 (128 columns) 139 / 101 us, 8 x 512 x 32
-// 135 / 120, 8 x 1024 x 16 183 / 153, 64 x 512 x 32 168 / 130, 8 x 1024 x 32 163 / 164; a wave goes through
-// the centroids beyond its first two one after the other: 8 x 250 x 63 126 / 138, 2 x 400 x 40 (256 columns)
-// 136 / 167.
+// round what its items take one compute unit, the launches what launches take.  Trees x items x centroids (128
+// columns), launches / one workgroup a tree, of a build of that level alone: 8 x 1024 x 32 164 / 126 us,
+// 64 x 1024 x 32 203 / 141, 8 x 512 x 16 139 / 69, 8 x 1024 x 16 183 / 105.  With more centroids a wave
+// takes them in turns (8 x 512 x 64: 134 / 147); rows of 256 columns: no gain left at 1024 x 32 (174 / 175).
 static bool level_is_small(const HiraTree* t, int n_c, int K) {
     return assign_exact_on_mfma(t->dtype, t->dim) && n_c <= kSmallItems && K <= kSmallCentroids &&
-           n_c * K <= (t->dim <= 128 ? 16384 : 8192);
+           n_c * K <= (t->dim <= 128 ? small_pairs(t->dim) : 8192);
 }
 
 static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
@@ -999,12 +999,10 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
             p.last = L;
             for (int i = l - 1; i < L; ++i) {
                 p.K[i] = K[i];
-                p.Kt[i] = assign_tiles(K[i]);
                 p.slots[i] = w.slots[i];
                 p.cent_t[i] = w.cent_t[i];
             }
             p.cent = w.cent_f32;
-            p.ct = w.ct;
             p.seed = seed;
             p.niter = niter;
             p.pack_rounds = pack_rounds;

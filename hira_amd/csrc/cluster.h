@@ -129,15 +129,14 @@ __device__ __forceinline__ void wave_mean(const void* x, size_t row0, Ids ids, i
 // storage type.  One wave: `lpr` lanes (a power of two) hold a row in 16-byte chunks,
 // the 64 / lpr lane groups take every (64 / lpr)-th slot, and their sums are added pairwise in a
 // fixed order.  An empty block keeps its value.
-// (the slots in one load, U rows a lane group in flight: bf <= 64)
+// (slot: what lies in slot `lane` of the block, -1 from bf on; U rows a lane group in flight: bf <= 64)
 template <typename T, int U>
-__device__ __forceinline__ void wave_block_mean(const void* x, size_t row0, int D, const int32_t* slots, int bf,
+__device__ __forceinline__ void wave_block_mean(const void* x, size_t row0, int D, int slot, int bf,
                                                 int lpr, size_t out, float* cent, void* out_t) {
     constexpr int EPL = Elem<T>::kPerChunk;
     const int lane = threadIdx.x & 63;
     const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
     const bool chunk_ok = ch * EPL < D;
-    const int slot = lane < bf ? slots[lane] : -1;
     float acc[EPL];
 #pragma unroll
     for (int q = 0; q < EPL; ++q) acc[q] = 0.0f;

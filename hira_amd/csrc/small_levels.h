@@ -8,16 +8,15 @@ namespace hira {
 
 constexpr int kSmallItems = 1024;      // what its LDS has room for
 constexpr int kSmallCentroids = 32;
+constexpr int small_pairs(int D) { return D <= 128 ? 32768 : 16384; }  // items times centroids
 
 struct SmallLevels {
     const void* x;                     // (T, K[first - 1], D) bf16 items of level `first`
     int32_t first, last;               // levels first .. last - 1
     int32_t K[HIRA_MAX_LEVELS];        // K[l - 1] items are clustered into K[l] blocks
-    int32_t Kt[HIRA_MAX_LEVELS];       // operand tiles of a tree (assign_tiles)
     int32_t* slots[HIRA_MAX_LEVELS];   // (T, K[l], bf)
     void* cent_t[HIRA_MAX_LEVELS];     // (T, K[l], D) block centres in bf16
     float* cent;                       // (T, K[l], D)
-    CentroidTiles ct;
     uint64_t seed;
     int32_t niter, pack_rounds, bf, lpr;
 };

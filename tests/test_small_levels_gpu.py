@@ -65,3 +65,10 @@ def test_levels_above_cluster_the_centres_below(h, n, d, levels, bf, gpu_device)
                     mean = child[t, k * bf: k * bf + c].mean(0)
                     # (one rounding to bf16, 2^-9 of a number, and fp32 sums)
                     assert torch.allclose(centre[t, k], mean, rtol=2 ** -8, atol=1e-5)
+
+
+@pytest.mark.parametrize("kind", ["normal", "hub"])
+@pytest.mark.parametrize("h,n,d,bf,niter", [(1, 1024, 128, 32, 1), (2, 1023, 64, 32, 2), (1, 993, 128, 32, 0), (1, 512, 256, 32, 1),
+                                            (2, 97, 128, 3, 1), (2, 1009, 128, 32, 1)])
+def test_as_many_pairs_as_the_scores_have_room_for(kind, h, n, d, bf, niter, gpu_device):
+    test_a_small_level_is_clustered_as_a_large_one(kind, h, n, d, bf, niter, gpu_device)
