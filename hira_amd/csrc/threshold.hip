@@ -4,9 +4,10 @@
 // One workgroup of sixteen waves per query head; with whole groups of heads per tree the
 // workgroups of a tree are a multiple of eight apart in the launch, so that they run behind the
 // same L2 (workgroups go to the eight L2s in turn) and the tree's sample is fetched from memory
-// once.  Up to 1024 samples and k <= 16: every wave sorts its 64 scores in registers, the
-// sixteen best of every wave meet in LDS, and one wave picks the k best of those 256 one by one.  Scores: 16 lanes share a sample row (16 bytes
-// each per step), eight rows per lane group in flight.  Then either a maximum, or a bitonic sort
+// once.  Scores of bf16 rows of 64 or 128 columns: tau_dot_scores, one a thread.  Other rows: 16 lanes share a
+// sample row (16 bytes each per step), sixteen rows per lane group in flight, scores to LDS.  Up to 1024 samples and
+// k <= 16: every wave sorts its 64 scores in registers, the sixteen best of every wave meet in LDS, and one wave
+// merges them.  Else either a maximum, or a bitonic sort
 // by the first four waves with the scores in registers (entry e*256 + thread of the padded
 // array lives in register e of that thread: partners 256 or more apart are a register swap,
 // partners inside a wave a cross-lane move, only the two distances in between go through LDS)

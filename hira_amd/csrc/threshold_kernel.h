@@ -2,6 +2,8 @@
 // one workgroup: the kernel of hira_threshold runs it in every workgroup, the kernel of
 // hira_update_threshold in the workgroups behind those that append.
 #pragma once
+#include <type_traits>
+
 #include "common.hip.h"
 
 namespace hira {
@@ -146,6 +148,79 @@ struct TauSortFrom {
     }
 };
 
+// Scores of the kTauThreads sample rows from r0 on, one a thread, bf16 rows of 8 * LPR columns: LPR lanes hold a row
+// in 16-byte chunks, LPR passes of kTauThreads / LPR rows are on their way at once, two products an instruction
+// (v_dot2_f32_bf16: fp32 sums, error against 64 bits 0.96 of a chain of fmas' over 128 normal columns, 0.75 with some of
+// them twenty times as large), and the sums over the lanes halve in number as they go, so that lane i ends with pass
+// i's row.  With an fma a product, a sum over all lanes a row and the scores through LDS a wave has some 400 vector
+// instructions and not 130, four waves a SIMD: a launch of 32 heads, 1000 samples of 128 columns 8.8 us, now
+// 6.2 (with the merge below), 8 heads, 64 columns 8.7, now 5.1.  What bounds it is the launch, one trip to memory
+// and 256 KB through a compute unit's L1 at 64 bytes a clock, 1.8 us.
+// (On the matrix cores, rows as the A operand, a load is half lines of sixteen rows, and what is on its way is
+// more than the L1: 11.2 us.)
+// Loads: buffer loads, the tree's sample behind one scalar descriptor, the pass in a scalar offset, one
+// address register for all of them.  The range check of a buffer load looks at the vector offset only, so the
+// scalar one must stay inside the sample by itself: a pass that reaches past the end is moved back to end with
+// the sample, and its rows that an earlier pass has are none here (row -1, score -INFINITY).
+template <int LPR>
+__device__ __forceinline__ float tau_dot_scores(const void* xs, const void* qh, int r0, int S, bool rot4_first, int& row) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int D = 8 * LPR, PASS = kTauThreads / LPR;
+    const int tid = threadIdx.x, sub = tid % LPR, grp = tid / LPR;
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(xs), 0, S * D * 2, 0x00020000);
+    const unsigned voff = (unsigned)(grp * D + sub * 8) * 2u;
+    const int last_pass = max(S - PASS, 0);
+    u32x4 raw[LPR];
+#pragma unroll
+    for (int u = 0; u < LPR; ++u) {
+        raw[u] = u32x4{0, 0, 0, 0};
+        if (r0 + u * PASS < S)  // uniform
+            raw[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, (unsigned)(min(r0 + u * PASS, last_pass) * (D * 2)), 0);
+    }
+    const u32x4 b = reinterpret_cast<const u32x4*>(qh)[sub];
+    float dot[LPR];
+#pragma unroll
+    for (int u = 0; u < LPR; ++u) {
+        float d = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t x = raw[u][e], y = b[e];  // (an element of a vector cannot be bit-cast where it is)
+            d = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, x), __builtin_bit_cast(bf16x2, y), d, false);
+        }
+        dot[u] = d;
+    }
+    auto halve = [&](auto step) {
+        constexpr int J = decltype(step)::value;
+        const bool high = (sub & J) != 0;
+#pragma unroll
+        for (int u = 0; u < J; ++u) {
+            const float keep = high ? dot[u + J] : dot[u], give = high ? dot[u] : dot[u + J];
+            dot[u] = keep + tau_partner<J>(give, rot4_first);
+        }
+    };
+    if constexpr (LPR == 16) halve(std::integral_constant<int, 8>{});
+    halve(std::integral_constant<int, 4>{});
+    halve(std::integral_constant<int, 2>{});
+    halve(std::integral_constant<int, 1>{});
+    const int base = r0 + sub * PASS;
+    row = min(base, last_pass) + grp;
+    if (base >= S || row < base || row >= S) row = -1;
+    return row >= 0 ? dot[0] : -INFINITY;
+}
+
+// The 16 largest of two rows of 16 lanes, each sorted largest first, sorted the same way.
+__device__ __forceinline__ float tau_merge16(float a, float b, int ln, bool rot4_first) {
+    float m = fmaxf(a, dpp_move<0x140>(b));  // (the row mirrored)
+    auto step = [&](float o, bool lower) { m = lower ? fmaxf(m, o) : fminf(m, o); };
+    step(tau_partner<8>(m, rot4_first), (ln & 8) == 0);
+    step(tau_partner<4>(m, rot4_first), (ln & 4) == 0);
+    step(tau_partner<2>(m, rot4_first), (ln & 2) == 0);
+    step(tau_partner<1>(m, rot4_first), (ln & 1) == 0);
+    return m;
+}
+
 // E = registers per thread of the sort: the padded array has 1024 * E entries
 // The work of one workgroup of kTauThreads threads: the threshold of the head that place `pos`
 // of the launch stands for.
@@ -172,6 +247,47 @@ __device__ __forceinline__ void threshold_block(
         head = tree_q_heads[pos];
     }
 
+    // ---- few of up to 1024, a score a thread: every wave sorts its 64, largest first; the sixteen best of every
+    // wave meet in LDS, and one wave merges them, two sorted rows of 16 lanes at a time, down to sixteen.
+    // (Picking the k best of those 256 one maximum at a time: 0.7 us more.)
+    auto few_best = [&](float x) {
+        const int ln = tid & 63, wv = tid >> 6;
+        const bool rot4 = __builtin_amdgcn_update_dpp(0, ln, 0x124, 0xF, 0xF, true) == (ln ^ 4);
+        tau_wave_stage<2, 1>(x, ln, rot4);
+        tau_wave_stage<4, 2>(x, ln, rot4);
+        tau_wave_stage<8, 4>(x, ln, rot4);
+        tau_wave_stage<16, 8>(x, ln, rot4);
+        tau_wave_stage<32, 16>(x, ln, rot4);
+        tau_wave_stage<64, 32>(x, ln, rot4);
+        if (ln < 16) s_sc[1][wv * 16 + ln] = x;
+        __syncthreads();
+        if (wv != 0) return;
+        float c[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[e] = s_sc[1][e * 64 + ln];
+        float m = tau_merge16(tau_merge16(c[0], c[1], ln, rot4), tau_merge16(c[2], c[3], ln, rot4), ln, rot4);
+        m = tau_merge16(m, __shfl_xor(m, 16, 64), ln, rot4);
+        m = tau_merge16(m, __shfl_xor(m, 32, 64), ln, rot4);
+        float sum = 0.0f;
+        for (int r = 0; r < k; ++r)  // uniform
+            sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), r));
+        if (ln == 0) tau[head] = sum / (float)k;
+    };
+    const T* xs = samples + (size_t)tree * S * D;
+    const T* qh = q + (size_t)head * D;
+    if (sizeof(T) == 2 && (D == 64 || D == 128)) {
+        const int ln = tid & 63;
+        const bool rot4 = __builtin_amdgcn_update_dpp(0, ln, 0x124, 0xF, 0xF, true) == (ln ^ 4);
+        for (int r0 = 0; r0 < S; r0 += kTauThreads) {  // uniform
+            int row;
+            const float x = D == 64 ? tau_dot_scores<8>(xs, qh, r0, S, rot4, row) : tau_dot_scores<16>(xs, qh, r0, S, rot4, row);
+            if (E == 1 && k <= 16 && method != HIRA_TAU_SAMPLE_MAX) {
+                few_best(x);
+                return;
+            }
+            if (row >= 0) s_sc[0][row] = x;
+        }
+    } else {
     // ---- scores: 16 lanes per sample row, 64 rows per pass, kTauRows passes at a time ---------
     // (buffer loads: the tree's sample behind one scalar descriptor, the pass in a scalar offset,
     // one address register for all the rows a lane has in flight -- which is what lets sixteen of
@@ -181,8 +297,6 @@ __device__ __forceinline__ void threshold_block(
     // says which lanes have none.)
     const int sub = tid & 15, grp = tid >> 4;
     const int chunks = D / EPL;
-    const T* xs = samples + (size_t)tree * S * D;
-    const T* qh = q + (size_t)head * D;
     constexpr int PASS = kTauThreads / 16;
     const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<T*>(xs), 0, (int)((size_t)S * D * sizeof(T)), 0x00020000);
@@ -221,6 +335,7 @@ __device__ __forceinline__ void threshold_block(
             if (sub == 0 && r0 + u * PASS < S && row < S) s_sc[0][row] = d;
         }
     }
+    }
     __syncthreads();
     // ---- from here on only the first four waves hold data; the others keep the barriers company
     constexpr int ST = kTauSorters;
@@ -242,39 +357,7 @@ __device__ __forceinline__ void threshold_block(
     }
 
     if (E == 1 && k <= 16) {
-        // ---- few of up to 1024: every wave sorts its 64 scores, largest first ------------------
-        const int ln = tid & 63, wv = tid >> 6;
-        const bool rot4 = __builtin_amdgcn_update_dpp(0, ln, 0x124, 0xF, 0xF, true) == (ln ^ 4);
-        float x = tid < S ? s_sc[0][tid] : -INFINITY;
-        tau_wave_stage<2, 1>(x, ln, rot4);
-        tau_wave_stage<4, 2>(x, ln, rot4);
-        tau_wave_stage<8, 4>(x, ln, rot4);
-        tau_wave_stage<16, 8>(x, ln, rot4);
-        tau_wave_stage<32, 16>(x, ln, rot4);
-        tau_wave_stage<64, 32>(x, ln, rot4);
-        __syncthreads();  // everybody has read its score
-        if (ln < 16) s_sc[1][wv * 16 + ln] = x;
-        __syncthreads();
-        if (wv != 0) return;
-        // the k best of the 256 that are left, one at a time: the wave's maximum, taken out of
-        // the one place (lowest lane, lowest register) that holds it
-        float c[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) c[e] = s_sc[1][e * 64 + ln];
-        float sum = 0.0f;
-        for (int r = 0; r < k; ++r) {  // uniform
-            const float mine = fmaxf(fmaxf(c[0], c[1]), fmaxf(c[2], c[3]));
-            const float best = tau_wave_max(mine, rot4);
-            sum += best;
-            const unsigned long long has = __ballot(mine == best);
-            if (ln == __ffsll((long long)has) - 1) {
-                if (c[0] == best) c[0] = -INFINITY;
-                else if (c[1] == best) c[1] = -INFINITY;
-                else if (c[2] == best) c[2] = -INFINITY;
-                else c[3] = -INFINITY;
-            }
-        }
-        if (ln == 0) tau[head] = sum / (float)k;
+        few_best(tid < S ? s_sc[0][tid] : -INFINITY);
         return;
     }
 
