@@ -17,7 +17,7 @@ HIRA_MAX_LEVELS = 8
 HIRA_STATS_COLS = HIRA_MAX_LEVELS + 3  # counters per tree a search can fill in
 HIRA_F32, HIRA_BF16 = 0, 1
 HIRA_ROW_MAJOR, HIRA_TILE16, HIRA_TILE16_Q8 = 0, 1, 2
-HIRA_ABI_VERSION = 9
+HIRA_ABI_VERSION = 10
 HIRA_UNIT_SCALE_HEADS = 4096
 
 _vp = C.c_void_p
@@ -73,6 +73,11 @@ class HiraQueue(C.Structure):
     _fields_ = [("keys", _vp), ("values", _vp), ("len", C.c_int32), ("cap", C.c_int32)]
 
 
+class HiraSample(C.Structure):
+    _fields_ = [("rows", _vp), ("num_rows", C.c_int32), ("method", C.c_int32), ("k", C.c_int32),
+                ("reserved_", C.c_int32), ("tau", _vp)]
+
+
 class HiraSearchOut(C.Structure):
     _fields_ = [
         ("dense", _vp),
@@ -119,6 +124,11 @@ SYMBOLS = {
     "hira_search": (
         C.c_int,
         [C.POINTER(HiraTree), C.POINTER(HiraQuery), C.POINTER(HiraQueue),
+         C.POINTER(HiraSearchOut), C.POINTER(HiraLaunch), _vp, C.c_size_t, _vp],
+    ),
+    "hira_search_sampled": (
+        C.c_int,
+        [C.POINTER(HiraTree), C.POINTER(HiraQuery), C.POINTER(HiraSample), C.POINTER(HiraQueue),
          C.POINTER(HiraSearchOut), C.POINTER(HiraLaunch), _vp, C.c_size_t, _vp],
     ),
     "hira_search_noalloc": (

@@ -104,6 +104,10 @@ class HiraCacheLayer(CacheLayerMixin):
         esize = self._queue_k.element_size()
         if dt not in (torch.float32, torch.bfloat16) or self.dim * esize % 16 or self.vdim * esize % 16:
             self._queue_type = None
+        # what a launch is told of the buffers: they are the layer's own, and stay until the next allocation
+        self._queue_at = (self._queue_k.data_ptr(), self._queue_v.data_ptr(), self._queue_type,
+                          self.batch * self.H_kv, rows)
+        self._queue_dev = self._queue_k.get_device()
 
     @property
     def queued_keys(self):
@@ -116,8 +120,9 @@ class HiraCacheLayer(CacheLayerMixin):
     def _whole_rows(self, x, m: int, width: int, like) -> bool:
         """Are x's rows (B, H_kv, m, width) -- or (H_kv, m, width) of one sequence --, one behind the
         other, on `like`'s device and 16-byte aligned, as the launches that copy rows take them?"""
-        return x.ndim >= 3 and x.shape[-3:] == (self.H_kv, m, width) and \
-            x.numel() == self.batch * self.H_kv * m * width and \
+        return (x.shape == (self.batch, self.H_kv, m, width) or (
+            x.ndim >= 3 and x.shape[-3:] == (self.H_kv, m, width) and
+            x.numel() == self.batch * self.H_kv * m * width)) and \
             x.get_device() == like.get_device() and x.is_contiguous() and x.data_ptr() % 16 == 0
 
     def _enqueue(self, key_states, value_states):
@@ -128,15 +133,16 @@ class HiraCacheLayer(CacheLayerMixin):
             self._queue_k[:, :, :n] = old_k[:, :, :n]
             self._queue_v[:, :, :n] = old_v[:, :, :n]
         k, v = self._queue_k, self._queue_v
-        if self._queue_type is not None and k.is_cuda and \
-                key_states.dtype is k.dtype and value_states.dtype is v.dtype and \
+        if self._queue_type is not None and self._queue_dev >= 0 and \
+                key_states.dtype is k.dtype and value_states.dtype is k.dtype and \
                 self._whole_rows(key_states, m, self.dim, k) and \
                 self._whole_rows(value_states, m, self.vdim, v):
             # one launch for both
-            _lib.check(_lib.lib().hira_enqueue(
-                k.data_ptr(), v.data_ptr(), self._queue_type, self.batch * self.H_kv, k.shape[2],
-                self.queued_len, m, self.dim, self.vdim, key_states.data_ptr(),
-                value_states.data_ptr(), _lib.stream_of(k.get_device())))
+            rc = _lib.lib().hira_enqueue(
+                *self._queue_at, self.queued_len, m, self.dim, self.vdim, key_states.data_ptr(),
+                value_states.data_ptr(), _lib.stream_of(self._queue_dev))
+            if rc:
+                _lib.check(rc)
             self.queued_len += m
             return
         if key_states.ndim != 4:

@@ -389,6 +389,19 @@ extern "C" int hira_search(const HiraTree* tree, const HiraQuery* query, const H
     return search_impl(tree, query, queue, out, launch, workspace, workspace_bytes, 0, stream);
 }
 
+/* see include/hira_hip.h */
+extern "C" int hira_search_sampled(const HiraTree* tree, const HiraQuery* query, const HiraSample* sample,
+                                   const HiraQueue* queue, const HiraSearchOut* out, const HiraLaunch* launch,
+                                   void* workspace, size_t workspace_bytes, void* stream) {
+    HIRA_CHECK_ARG(tree && query && sample, "hira_search_sampled: null argument");
+    const int rc = hira_threshold(sample->rows, tree->dtype, tree->num_trees, sample->num_rows, tree->dim, query,
+                                  sample->method, sample->k, sample->tau, stream);
+    if (rc != HIRA_OK) return rc;
+    HiraQuery with = *query;
+    with.tau = sample->tau;
+    return hira_search(tree, &with, queue, out, launch, workspace, workspace_bytes, stream);
+}
+
 // ---- the same search for callers that cannot allocate ----------------------------------------
 // Its scratch (arrival counters, then attention partials) is this array in the library's own
 // device image: every GPU the library runs on holds a copy until the process ends.  Host code

@@ -463,6 +463,8 @@ class DecodePlan:
         self.launch = searcher.launch
         self.tree = indexer.tree_struct()
         self.queue = _lib.HiraQueue()
+        self.sample = _lib.HiraSample()
+        self._sample_ref = C.byref(self.sample)
         self.tau_buf: Optional[torch.Tensor] = None  # (H_q,) thresholds written by run_sampled
         self._ws_rows = 1  # queue rows the workspace is sized for
         self.ws_bytes = self._workspace_need()
@@ -494,32 +496,38 @@ class DecodePlan:
         leading dimensions amounting to T trees: keys not in the index yet, attended by every
         head of their tree; the first `queue_len` rows of every tree are in use (all `cap`
         when not given)."""
-        if self.indexer.tree_struct() is not self.tree:
-            self._follow_index()
-        q = self.query
-        q.q = query.data_ptr()
-        q.tau = threshold.data_ptr()
-        self.out.attn_out = out.data_ptr()
-        q.out_dtype = _OUT_TYPES[out.dtype] if out.dtype in _OUT_TYPES else _refuse_out(out)
+        qu = self._step(query, out, queue_keys, queue_values, queue_len)
+        self.query.tau = threshold.data_ptr()
         if stream is None:
             stream = _lib.stream_of(self._dev)
-        qu = None
-        if queue_keys is not None and queue_keys.shape[-2] > 0 and queue_len != 0:
-            cap = int(queue_keys.shape[-2])
-            m = cap if queue_len is None else int(queue_len)
-            if not 0 < m <= cap or queue_values.shape[-2] != cap:
-                raise ValueError(f"queue: {m} rows in use of {cap} "
-                                 f"(values hold {queue_values.shape[-2]})")
-            qs = self.queue
-            qs.keys, qs.values, qs.len, qs.cap = queue_keys.data_ptr(), queue_values.data_ptr(), m, cap
-            if m > self._ws_rows:
-                self._ws_rows = m
-                self._follow_index()
-            qu = self._refs[4]
         t, q, o, l, _ = self._refs
         rc = self.lib.hira_search(t, q, qu, o, l, self.ws.data_ptr(), self.ws_bytes, stream)
         if rc:
             _lib.check(rc)
+
+    def _step(self, query, out, queue_keys, queue_values, queue_len):
+        """Query, output and queue of a step into the call's structs; the queue's reference, or None."""
+        if self.indexer.tree_struct() is not self.tree:
+            self._follow_index()
+        q = self.query
+        q.q = query.data_ptr()
+        self.out.attn_out = out.data_ptr()
+        q.out_dtype = _OUT_TYPES[out.dtype] if out.dtype in _OUT_TYPES else _refuse_out(out)
+        if queue_keys is None or queue_len == 0:
+            return None
+        cap = int(queue_keys.shape[-2])
+        if cap == 0:
+            return None
+        m = cap if queue_len is None else int(queue_len)
+        if not 0 < m <= cap or queue_values.shape[-2] != cap:
+            raise ValueError(f"queue: {m} rows in use of {cap} "
+                             f"(values hold {queue_values.shape[-2]})")
+        qs = self.queue
+        qs.keys, qs.values, qs.len, qs.cap = queue_keys.data_ptr(), queue_values.data_ptr(), m, cap
+        if m > self._ws_rows:
+            self._ws_rows = m
+            self._follow_index()
+        return self._refs[4]
 
     def run_sampled(self, query: torch.Tensor, samples: torch.Tensor, method: str, k: int,
                     out: torch.Tensor, stream: Optional[int] = None,
@@ -527,40 +535,45 @@ class DecodePlan:
                     queue_values: Optional[torch.Tensor] = None,
                     queue_len: Optional[int] = None, append=None) -> torch.Tensor:
         """A decode step whose thresholds come from a key sample (T, S, D), tree dtype,
-        contiguous: ``hira_threshold`` ("sample_max" or "sample_mean_topk" with k) writes them
-        into a buffer of the plan, ``run`` follows on the same stream.  Returns that buffer.
+        contiguous: ``hira_search_sampled`` ("sample_max" or "sample_mean_topk" with k) writes them
+        into a buffer of the plan and searches with them, two launches of one call.  Returns that buffer.
         ``append`` = (new_keys (T, m, D), new_values (T, m, Dv) or None, state): the step first
         appends these rows to the index (``hira_update``'s arguments), in the launch that takes
         the thresholds (``hira_update_threshold``)."""
-        if self.tau_buf is None:
-            self.tau_buf = torch.empty((self.query.num_q_heads,), dtype=torch.float32,
-                                       device=self.indexer.device)
-        if samples.ndim != 3 or samples.shape[0] != self.tree.num_trees or \
-                samples.shape[2] != self.tree.dim or samples.dtype != self.indexer.dtype or \
-                not samples.is_contiguous():
-            raise ValueError(f"samples {tuple(samples.shape)} {samples.dtype}: expected contiguous "
-                             f"({self.tree.num_trees}, S, {self.tree.dim}) {self.indexer.dtype}")
+        tau = self.tau_buf
+        if tau is None:
+            tau = self.tau_buf = torch.empty((self.query.num_q_heads,), dtype=torch.float32,
+                                             device=self.indexer.device)
+        tree, shape = self.tree, samples.shape
+        if len(shape) != 3 or shape[0] != tree.num_trees or shape[2] != tree.dim or \
+                samples.dtype != self.indexer.dtype or not samples.is_contiguous():
+            raise ValueError(f"samples {tuple(shape)} {samples.dtype}: expected contiguous "
+                             f"({tree.num_trees}, S, {tree.dim}) {self.indexer.dtype}")
         if stream is None:
             stream = _lib.stream_of(self._dev)
-        if self.indexer.tree_struct() is not self.tree:
-            self._follow_index()
-        self.query.q = query.data_ptr()
         rule = 0 if method == "sample_max" else 1
         if append is not None:
+            if self.indexer.tree_struct() is not self.tree:
+                self._follow_index()
+            self.query.q = query.data_ptr()
             new_keys, new_values, state = append
             rc = self.lib.hira_update_threshold(
                 self._refs[0], new_keys.data_ptr(),
                 new_values.data_ptr() if new_values is not None else None,
                 int(new_keys.shape[-2]), state.data_ptr(), samples.data_ptr(),
-                int(samples.shape[1]), self._refs[1], rule, int(k), self.tau_buf.data_ptr(), stream)
-        else:
-            rc = self.lib.hira_threshold(
-                samples.data_ptr(), self.tree.dtype, self.tree.num_trees, int(samples.shape[1]),
-                self.tree.dim, self._refs[1], rule, int(k), self.tau_buf.data_ptr(), stream)
+                int(shape[1]), self._refs[1], rule, int(k), tau.data_ptr(), stream)
+            if rc:
+                _lib.check(rc)
+            self.run(query, tau, out, stream, queue_keys, queue_values, queue_len)
+            return tau
+        qu = self._step(query, out, queue_keys, queue_values, queue_len)
+        sm = self.sample
+        sm.rows, sm.num_rows, sm.method, sm.k, sm.tau = samples.data_ptr(), shape[1], rule, int(k), tau.data_ptr()
+        t, q, o, l, _ = self._refs
+        rc = self.lib.hira_search_sampled(t, q, self._sample_ref, qu, o, l, self.ws.data_ptr(), self.ws_bytes, stream)
         if rc:
             _lib.check(rc)
-        self.run(query, self.tau_buf, out, stream, queue_keys, queue_values, queue_len)
-        return self.tau_buf
+        return tau
 
 
 class StreamingStep:

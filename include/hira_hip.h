@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define HIRA_ABI_VERSION 9
+#define HIRA_ABI_VERSION 10
 #define HIRA_MAX_LEVELS 8
 #define HIRA_STATS_COLS (HIRA_MAX_LEVELS + 3) /* counters per tree a search can fill in */
 
@@ -329,6 +329,23 @@ enum { HIRA_TAU_SAMPLE_MAX = 0, HIRA_TAU_SAMPLE_MEAN_TOPK = 1 };
 int hira_threshold(const void* samples, int32_t dtype, int32_t num_trees, int32_t num_samples,
                    int32_t dim, const HiraQuery* query, int32_t method, int32_t k,
                    float* tau_out, void* stream);
+
+/*
+ * hira_threshold and hira_search of one decode step as one call (two launches on the stream): the thresholds
+ * are written to sample->tau and searched with; query->tau is not read.  Results are those of the two calls.
+ * The samples have the tree's dtype, dim and tree count.
+ */
+typedef struct HiraSample {
+    const void* rows;     /* (T, num_rows, D) */
+    int32_t num_rows;
+    int32_t method;       /* HIRA_TAU_* */
+    int32_t k;
+    int32_t reserved_;
+    float* tau;           /* (H_q,) */
+} HiraSample;
+int hira_search_sampled(const HiraTree* tree, const HiraQuery* query, const HiraSample* sample,
+                        const HiraQueue* queue, const HiraSearchOut* out, const HiraLaunch* launch,
+                        void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * hira_update and hira_threshold of one decode step as ONE launch, for a step that appends a key
