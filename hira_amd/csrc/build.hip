@@ -677,6 +677,10 @@ struct PlaceLevel {
     const void* values_in;           // level 1: (T, rows_stride, vdim) -> (T, child_stride, vdim), or NULL
     void* values;
     int32_t vdim, lpr_v;             // (a value row in steps of lpr_v <= 64 lanes)
+    // a subtree (level 1 of 2): nodes with children first, to slots from slot0 and nodes from node0 on; perm takes
+    // pos[child], (T, rows_stride)
+    const int32_t* pos;
+    int32_t slot0, node0;
     float* absmax;                   // ABSMAX: (T, kAbsCopies, D) joined by the largest finite magnitudes per channel
 };
 
@@ -706,18 +710,26 @@ __global__ __launch_bounds__(kNodeThreads) void k_place(const PlaceLevel pl) {
             for (int j = pl.level; j < i - 1; ++j) at /= bf;
             id = id >= 0 ? pl.slots[i][((size_t)t * pl.K[i] + id) * bf + at % bf] : -1;
         }
+        if (pl.pos) {  // block p, if those with children come first (size = bf <= 64 blocks, filled from the first slot on)
+            const unsigned long long full = __ballot(lane < bf && pl.slots[1][((size_t)t * bf + min(lane, bf - 1)) * bf] >= 0);
+            const int n_full = __popcll(full);
+            unsigned long long left = p < n_full ? full : ~full;
+            for (int i = p < n_full ? p : p - n_full; i > 0; --i) left &= left - 1ull;
+            id = __ffsll((long long)left) - 1;
+        }
         const int own = max(id, 0);
         const int mine = lane < bf && id >= 0 ? pl.slots[pl.level][((size_t)t * pl.K[pl.level] + own) * bf + lane] : -1;
         const unsigned long long live = __ballot(mine >= 0);
-        const size_t s0 = (size_t)t * pl.child_stride + (size_t)p * bf;  // slots of the children
+        const size_t s0 = (size_t)t * pl.child_stride + pl.slot0 + (size_t)p * bf;  // slots of the children
         const float my_radius = mine >= 0 && pl.child_radii ? pl.child_radii[s0 + lane] : 0.0f;
-        if (pl.perm && lane < bf) pl.perm[s0 + lane] = mine;
+        if (pl.perm && lane < bf)
+            pl.perm[s0 + lane] = mine >= 0 && pl.pos ? pl.pos[(size_t)t * pl.rows_stride + mine] : mine;
         const uint4 craw = load_chunk<T>(pl.cent, ((size_t)t * pl.K[pl.level] + own) * D, chunk_ok ? ch : 0);
         float cf[EPL];
         unpack<T>(craw, cf);
         if (pl.top && rg == 0 && chunk_ok)
             *reinterpret_cast<uint4*>(reinterpret_cast<T*>(pl.top) + (size_t)t * pl.out_stride * D +
-                                      elem_index(pl.center_layout, D, (size_t)p, ch * EPL)) = craw;
+                                      elem_index(pl.center_layout, D, (size_t)pl.node0 + p, ch * EPL)) = craw;
         T* const child = reinterpret_cast<T*>(pl.child) + (size_t)t * pl.child_stride * D;
         float r = -INFINITY;
         for (int j0 = 0; j0 < bf; j0 += U * groups) {  // (uniform trip count: the sums meet in shuffles)
@@ -734,7 +746,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_place(const PlaceLevel pl) {
                 const int j = j0 + u * groups + rg;
                 const bool have = j < bf && it[u] >= 0;
                 if (j < bf && chunk_ok)
-                    *reinterpret_cast<uint4*>(child + elem_index(pl.child_layout, D, (size_t)p * bf + j, ch * EPL)) =
+                    *reinterpret_cast<uint4*>(child + elem_index(pl.child_layout, D, (size_t)pl.slot0 + (size_t)p * bf + j, ch * EPL)) =
                         make_uint4(have ? raw[u].x : 0u, have ? raw[u].y : 0u, have ? raw[u].z : 0u, have ? raw[u].w : 0u);
                 float f[EPL];
                 unpack<T>(raw[u], f);
@@ -789,8 +801,8 @@ __global__ __launch_bounds__(kNodeThreads) void k_place(const PlaceLevel pl) {
         if (lane == 0) {
             // a few ulp of head room: the bound must survive fp32 rounding of this sum
             if (r > 0.0f) r = r * (1.0f + 4.0f * 1.1920929e-7f) + 1e-30f;
-            pl.radii[(size_t)t * pl.out_stride + p] = r;
-            pl.counts[(size_t)t * pl.out_stride + p] = __popcll(live);
+            pl.radii[(size_t)t * pl.out_stride + pl.node0 + p] = r;
+            pl.counts[(size_t)t * pl.out_stride + pl.node0 + p] = __popcll(live);
         }
     }
     if constexpr (ABSMAX) {
@@ -972,14 +984,19 @@ static void fill_i32(int32_t* p, size_t n, int32_t v, hipStream_t s) {
     hipLaunchKernelGGL(k_fill_i32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n, v);
 }
 
-template <typename T>
-static int build_impl(const HiraTree* t, const void* keys_in, const void* values_in, int n,
-                      const int32_t* n_live, int niter, int pack_rounds, uint64_t seed,
-                      const BuildWs& w, hipStream_t s) {
-    const int L = t->num_levels, NT = t->num_trees, D = t->dim, bf = t->bf;
-    constexpr int EPL = Elem<T>::kPerChunk;
+static int lanes_per_row(int dtype, int D) {  // a power of two, 16 bytes a lane
     int lpr = 2;
-    while (lpr * EPL < D) lpr <<= 1;
+    while (lpr * (dtype == HIRA_F32 ? 4 : 8) < D) lpr <<= 1;
+    return lpr;
+}
+
+// Levels 1 .. L - 1: slots and block centres of every cluster, to the workspace.
+// small_ragged: two levels of trees with key counts may go through small_levels.hip too (a subtree: 105 us for 8 x
+// 1024 x 32, the launches 164; a build with counts stays with the launches, whatever its sizes).
+template <typename T>
+static int cluster_levels(const HiraTree* t, const void* keys_in, int n, const int32_t* n_live, int niter,
+                          int pack_rounds, uint64_t seed, const BuildWs& w, bool small_ragged, hipStream_t s) {
+    const int L = t->num_levels, NT = t->num_trees, D = t->dim, bf = t->bf, lpr = lanes_per_row(t->dtype, D);
     int K[HIRA_MAX_LEVELS];
     cluster_counts(n, bf, L, K);
 
@@ -991,10 +1008,11 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
     int32_t* const big_count = w.counters + 6 * ct;   // (2, T)
     const int KS = assign_ks(t->dtype, D);
     for (int l = 1; l < L; ++l) {
-        if (level_is_small(t, K[l - 1], K[l]) && n_live == nullptr) {  // this one and all above it in one launch
+        if (level_is_small(t, K[l - 1], K[l]) && (n_live == nullptr || (small_ragged && L == 2))) {  // this one and all above it in one launch
             if (l == 1 && w.absmax != nullptr) fill_i32(reinterpret_cast<int32_t*>(w.absmax), (size_t)NT * kAbsCopies * D, 0, s);
             SmallLevels p{};
             p.x = l == 1 ? keys_in : w.cent_t[l - 1];
+            p.n_live = n_live;
             p.first = l;
             p.last = L;
             for (int i = l - 1; i < L; ++i) {
@@ -1107,6 +1125,19 @@ static int build_impl(const HiraTree* t, const void* keys_in, const void* values
                            lpr, w.cent_f32, w.cent_t[l]);
         HIRA_CHECK_LAUNCH("build level");
     }
+
+    return HIRA_OK;
+}
+
+template <typename T>
+static int build_impl(const HiraTree* t, const void* keys_in, const void* values_in, int n,
+                      const int32_t* n_live, int niter, int pack_rounds, uint64_t seed,
+                      const BuildWs& w, hipStream_t s) {
+    const int L = t->num_levels, NT = t->num_trees, D = t->dim, bf = t->bf, lpr = lanes_per_row(t->dtype, D);
+    constexpr int EPL = Elem<T>::kPerChunk;
+    int K[HIRA_MAX_LEVELS];
+    cluster_counts(n, bf, L, K);
+    if (const int rc = cluster_levels<T>(t, keys_in, n, n_live, niter, pack_rounds, seed, w, false, s)) return rc;
 
     // layout and radii, bottom-up
     const bool whole_v = t->vdim % EPL == 0, have_v = values_in && t->values;
@@ -1250,6 +1281,228 @@ extern "C" int hira_build_ragged(const HiraTree* tree, const void* keys_in, cons
     return tree->dtype == HIRA_F32
                ? build_impl<float>(tree, keys_in, values_in, n, n_live, niter, pack_rounds, seed, b, s)
                : build_impl<bf16_t>(tree, keys_in, values_in, n, n_live, niter, pack_rounds, seed, b, s);
+}
+
+// ---- one level-2 subtree of every tree clustered anew -----------------------------------------
+// Four launches: the subtree's rows to the front of a workspace, the two levels over them, the nodes with keys
+// into their places, the radii above.  8 trees x 1024 rows of 128 columns, keys and values, bf16: 11 + 105 + 9 + 9 us
+// on the GPU, 21 on the host.  (As gathers, sorts and copies of a tensor library around a build of its own some fifty
+// launches: 557 us of the host, which the GPU waited for.)  The clustering bounds it, a chain of rounds.
+namespace hira {
+
+constexpr int kTakeSlots = 64;
+
+// The subtree's rows of every tree, those in use first, in slot order: rows (T, nsub, D) row-major, values, the
+// insertion positions (-1: no key), how many a tree holds.  A workgroup per 64 slots; each counts for
+// itself how many are in use ahead of its own.
+template <typename T>
+__global__ __launch_bounds__(256) void k_subtree_take(const HiraTree tree, int slot0, int nsub, T* rows, T* vals, int32_t* pos,
+                                                      int32_t* counts) {
+    constexpr int EPL = Elem<T>::kPerChunk;
+    __shared__ int s_before[4], s_total[4], s_dst[kTakeSlots];
+    const int t = blockIdx.x, first = tree_block() * kTakeSlots, tid = threadIdx.x, lane = tid & 63;
+    const size_t cap0 = (size_t)tree.cap[0];
+    const int32_t* perm = tree.perm + (size_t)t * cap0 + slot0;
+    int before = 0, total = 0;
+    for (int i = tid; i < nsub; i += 256) {
+        const int live = perm[i] >= 0 ? 1 : 0;
+        total += live;
+        before += i < first ? live : 0;
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        before += __shfl_xor(before, off, 64);
+        total += __shfl_xor(total, off, 64);
+    }
+    if (lane == 0) {
+        s_before[tid >> 6] = before;
+        s_total[tid >> 6] = total;
+    }
+    __syncthreads();
+    if (tid < kTakeSlots) {
+        before = s_before[0] + s_before[1] + s_before[2] + s_before[3];
+        total = s_total[0] + s_total[1] + s_total[2] + s_total[3];
+        const int slot = first + tid, at = slot < nsub ? perm[slot] : -1;
+        const unsigned long long live = __ballot(at >= 0);
+        const int ahead = before + __popcll(live & ((1ull << tid) - 1ull));
+        const int dst = at >= 0 ? ahead : total + slot - ahead;
+        s_dst[tid] = dst;
+        if (slot < nsub) pos[(size_t)t * nsub + dst] = at;
+        if (first == 0 && tid == 0) counts[t] = total;
+    }
+    __syncthreads();
+    const int kc = tree.dim / EPL, vc = vals ? tree.vdim / EPL : 0, per = kc + vc, here = min(kTakeSlots, nsub - first);
+    const int layout = key_layout_of(tree.layout);
+    for (int e = tid; e < here * per; e += 256) {
+        const int r = e / per, c = e % per;
+        const size_t slot = (size_t)slot0 + first + r, dst = (size_t)t * nsub + s_dst[r];
+        if (c < kc)
+            *reinterpret_cast<uint4*>(rows + dst * tree.dim + c * EPL) =
+                load_row_chunk<T>(tree.keys, layout, tree.dim, (size_t)t * cap0, slot, c);
+        else
+            *reinterpret_cast<uint4*>(vals + dst * tree.vdim + (c - kc) * EPL) =
+                load_chunk<T>(tree.values, ((size_t)t * cap0 + slot) * tree.vdim, c - kc);
+    }
+}
+
+// The level-2 node keeps its centre and gets the radius its new children need; its ancestors cover it where it grew
+// (with a little head room: fp32 norms).  A number that is none stays one.  A workgroup per tree.
+template <typename T>
+__global__ __launch_bounds__(256) void k_subtree_up(const HiraTree tree, int node, int32_t* state) {
+    __shared__ float s_r[4], s_d[HIRA_MAX_LEVELS];
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int D = tree.dim, bf = tree.bf, L = tree.num_levels, n0 = node * bf, layout = center_layout_of(tree.layout);
+    auto at = [&](int l, size_t p, int j) {
+        return load_elem<T>(tree.centers[l], (size_t)t * tree.cap[l] * D + elem_index(layout, D, p, j));
+    };
+    auto distance = [&](int l, size_t p, size_t q) {  // of node p of level l - 1 and node q of level l (one wave)
+        float ss = 0.0f;
+        for (int j = lane; j < D; j += 64) {
+            const float df = at(l - 1, p, j) - at(l, q, j);
+            ss += df * df;
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+        return sqrtf(ss);
+    };
+    auto larger = [](float a, float b) { return b > a || b != b ? b : a; };
+    float r = -INFINITY;
+    for (int p = wave; p < bf; p += 4)
+        r = larger(r, distance(2, (size_t)n0 + p, (size_t)node) + tree.radii[1][(size_t)t * tree.cap[1] + n0 + p]);
+    if (lane == 0) s_r[wave] = r;
+    size_t child = (size_t)node;
+    for (int l = 3; l < L; ++l, child /= (size_t)bf)
+        if ((l & 3) == wave) {
+            const float d = distance(l, child, child / (size_t)bf);
+            if (lane == 0) s_d[l] = d;
+        }
+    __syncthreads();
+    const unsigned long long full = __ballot(lane < bf && tree.counts[1][(size_t)t * tree.cap[1] + n0 + min(lane, bf - 1)] > 0);
+    if (tid != 0) return;
+    constexpr float kRoom = 1.0f + 1e-6f;
+    r = larger(larger(larger(s_r[0], s_r[1]), s_r[2]), s_r[3]) * kRoom;
+    tree.radii[2][(size_t)t * tree.cap[2] + node] = r;
+    tree.counts[2][(size_t)t * tree.cap[2] + node] = __popcll(full);
+    child = (size_t)node;
+    for (int l = 3; l < L; ++l) {
+        child /= (size_t)bf;
+        float* out = tree.radii[l] + (size_t)t * tree.cap[l] + child;
+        r = larger(*out, (s_d[l] + r) * kRoom);
+        *out = r;
+    }
+    if (state) state[(size_t)t * (HIRA_MAX_LEVELS + 2)] = 0;  // (the rebuilt nodes may have room again)
+}
+
+struct RebuildWs {
+    BuildWs build;
+    HiraTree sub;
+    void *rows, *vals;
+    int32_t *pos, *counts;
+    size_t total;
+};
+
+static int carve_rebuild(const HiraTree* t, void* ws, RebuildWs* b) {
+    HIRA_CHECK_ARG(t != nullptr && t->num_trees >= 1 && t->num_levels >= 3 && t->num_levels <= HIRA_MAX_LEVELS,
+                   "a subtree of level 2 needs at least three levels");
+    HIRA_CHECK_ARG(t->bf >= 1 && t->bf <= 64, "branching factor %d not in 1..64", t->bf);
+    HIRA_CHECK_ARG(t->layout == HIRA_ROW_MAJOR || t->bf % 16 == 0, "tiled layout: fan-out %d, a subtree must start on a tile", t->bf);
+    const int nsub = t->bf * t->bf;
+    HiraTree& sub = b->sub;
+    memset(&sub, 0, sizeof(sub));
+    sub.num_trees = t->num_trees;
+    sub.num_levels = 2;
+    sub.bf = t->bf;
+    sub.dim = t->dim;
+    sub.vdim = t->vdim;
+    sub.dtype = t->dtype;
+    sub.layout = HIRA_ROW_MAJOR;
+    sub.size[0] = sub.cap[0] = nsub;
+    sub.size[1] = sub.cap[1] = t->bf;
+    if (const int rc = check_build_args(&sub, nsub)) return rc;
+    const size_t esize = t->dtype == HIRA_F32 ? 4 : 2, T = (size_t)t->num_trees;
+    Carver c{reinterpret_cast<char*>(ws), 0};
+    b->rows = c.take<char>(T * nsub * t->dim * esize);
+    b->vals = t->values ? c.take<char>(T * nsub * t->vdim * esize) : nullptr;
+    b->pos = c.take<int32_t>(T * nsub);
+    b->counts = c.take<int32_t>(T);
+    const size_t own = (c.used + 255) & ~(size_t)255;
+    carve(&sub, nsub, ws ? reinterpret_cast<char*>(ws) + own : nullptr, &b->build);
+    b->total = own + b->build.total;
+    return HIRA_OK;
+}
+
+template <typename T>
+static int rebuild_impl(const HiraTree* t, int node, int niter, int pack_rounds, uint64_t seed, int32_t* state, const RebuildWs& w,
+                        hipStream_t s) {
+    const int bf = t->bf, nsub = bf * bf, NT = t->num_trees;
+    hipLaunchKernelGGL((k_subtree_take<T>), tree_grid((nsub + kTakeSlots - 1) / kTakeSlots, NT), dim3(256), 0, s, *t, node * nsub,
+                       nsub, reinterpret_cast<T*>(w.rows), reinterpret_cast<T*>(w.vals), w.pos, w.counts);
+    if (const int rc = cluster_levels<T>(&w.sub, w.rows, nsub, w.counts, niter, pack_rounds, seed, w.build, true, s)) return rc;
+    PlaceLevel p{};
+    p.rows = w.rows;
+    p.rows_stride = (size_t)nsub;
+    p.slots[1] = w.build.slots[1];
+    p.K[1] = bf;
+    p.num_levels = 2;
+    p.level = 1;
+    p.size = bf;
+    p.bf = bf;
+    p.D = t->dim;
+    p.lpr = lanes_per_row(t->dtype, t->dim);
+    p.child = t->keys;
+    p.child_stride = (size_t)t->cap[0];
+    p.child_layout = key_layout_of(t->layout);
+    p.center_layout = center_layout_of(t->layout);
+    p.cent = w.build.cent_t[1];
+    p.top = t->centers[1];
+    p.radii = t->radii[1];
+    p.counts = t->counts[1];
+    p.out_stride = (size_t)t->cap[1];
+    p.perm = t->perm;
+    if (w.vals) {
+        p.values_in = w.vals;
+        p.values = t->values;
+        p.vdim = t->vdim;
+        p.lpr_v = min(lanes_per_row(t->dtype, t->vdim), 64);
+    }
+    p.pos = w.pos;
+    p.slot0 = node * nsub;
+    p.node0 = node * bf;
+    hipLaunchKernelGGL((k_place<T, false>), node_grid(bf, NT), dim3(kNodeThreads), 0, s, p);
+    hipLaunchKernelGGL((k_subtree_up<T>), dim3(NT), dim3(256), 0, s, *t, node, state);
+    HIRA_CHECK_LAUNCH("subtree rebuild");
+    return t->layout == HIRA_TILE16_Q8 ? hira_quantize(t, node * nsub, nsub, 0, s) : HIRA_OK;
+}
+
+}  // namespace hira
+
+/* see include/hira_hip.h */
+extern "C" size_t hira_rebuild_workspace_bytes(const HiraTree* tree) {
+    RebuildWs w;
+    return carve_rebuild(tree, nullptr, &w) == HIRA_OK ? w.total : 0;
+}
+
+/* see include/hira_hip.h */
+extern "C" int hira_rebuild_subtree(const HiraTree* tree, int32_t node, int32_t niter, int32_t pack_rounds, uint64_t seed,
+                                    int32_t* state, void* workspace, size_t workspace_bytes, void* stream) {
+    RebuildWs w;
+    if (const int rc = carve_rebuild(tree, workspace, &w)) return rc;
+    if (workspace == nullptr || workspace_bytes < w.total)
+        return fail(HIRA_EWORKSPACE, "workspace %zu bytes, need %zu", workspace_bytes, w.total);
+    const long long bf = tree->bf;
+    HIRA_CHECK_ARG(node >= 0 && node < tree->cap[2] && (node + 1) * bf <= tree->cap[1] && (node + 1) * bf * bf <= tree->cap[0],
+                   "level-2 node %d: its slots lie beyond the capacity of the index", node);
+    HIRA_CHECK_ARG(tree->keys && tree->perm, "keys / perm missing");
+    HIRA_CHECK_ARG(niter >= 0 && pack_rounds >= 1, "niter %d, pack_rounds %d", niter, pack_rounds);
+    for (int l = 1; l < tree->num_levels; ++l)
+        HIRA_CHECK_ARG(tree->centers[l] && tree->radii[l] && tree->counts[l], "level %d arrays missing", l);
+    HIRA_CHECK_ARG(!tree->values || tree->vdim % (tree->dtype == HIRA_F32 ? 4 : 8) == 0, "vdim %d: rows must be a multiple of 16 bytes",
+                   tree->vdim);
+    if (tree->layout == HIRA_TILE16_Q8)
+        HIRA_CHECK_ARG(tree->keys8 && tree->kscale && tree->keps, "keys8 / kscale / keps missing");
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    return tree->dtype == HIRA_F32 ? rebuild_impl<float>(tree, node, niter, pack_rounds, seed, state, w, s)
+                                   : rebuild_impl<bf16_t>(tree, node, niter, pack_rounds, seed, state, w, s);
 }
 
 // ---- nearest centre as a call of its own -------------------------------------------------

@@ -12,6 +12,7 @@ constexpr int small_pairs(int D) { return D <= 128 ? 32768 : 16384; }  // items 
 
 struct SmallLevels {
     const void* x;                     // (T, K[first - 1], D) bf16 items of level `first`
+    const int32_t* n_live;             // (T) how many of them a tree holds, the first ones (then first = 1, last = 2); or NULL
     int32_t first, last;               // levels first .. last - 1
     int32_t K[HIRA_MAX_LEVELS];        // K[l - 1] items are clustered into K[l] blocks
     int32_t* slots[HIRA_MAX_LEVELS];   // (T, K[l], bf)

@@ -287,18 +287,24 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int bf = p.bf;
     for (int l = p.first; l < p.last; ++l) {  // uniform, and so are the loops over rounds
-        const int n_c = p.K[l - 1], K = p.K[l];
+        const int K = p.K[l];
+        // (a tree with fewer items uses its first K_t centroids only: the others count as full)
+        const int n_c = p.n_live == nullptr ? p.K[l - 1] : min(max(p.n_live[t], 0), p.K[l - 1]);
+        const int K_t = p.n_live == nullptr ? K : min(max((n_c + bf - 1) / bf, 1), K);
         const void* x = l == p.first ? p.x : p.cent_t[l - 1];
-        const size_t row0 = (size_t)t * n_c;
+        const size_t row0 = (size_t)t * p.K[l - 1];
         int32_t* slots = p.slots[l] + (size_t)t * K * bf;
         float* cent = p.cent + (size_t)t * K * D;
         float* piece = s.piece[wave];
 
         // ---- empty blocks, first centroids -------------------------------------------------------
-        for (int i = tid; i < K; i += kSmallThreads) s.fill[i] = s.count[i] = 0;
+        for (int i = tid; i < K; i += kSmallThreads) {
+            s.fill[i] = i >= K_t ? bf : 0;
+            s.count[i] = 0;
+        }
         if (tid == 0) s.n_big = 0;
         for (int k = wave; k < K; k += kSmallWaves) {
-            const size_t src = (row0 + (size_t)first_centroid(p.seed + 7919ull * (uint64_t)l, t, k, n_c, K)) * D;
+            const size_t src = (row0 + (size_t)first_centroid(p.seed + 7919ull * (uint64_t)l, t, k, max(n_c, 1), K_t)) * D;
             for (int j = lane; j < D; j += 64) {
                 const float v = load_elem<bf16_t>(x, src + j);
                 cent[(size_t)k * D + j] = v;
@@ -306,6 +312,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             small_emit<KS>(s, piece, k);
+            if (lane == 0 && k >= K_t) s.n2[k] = INFINITY;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
         __syncthreads();

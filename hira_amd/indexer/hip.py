@@ -987,9 +987,8 @@ class HIPIndexer(BaseIndexer):
         keys now and then.  The keys stay in the subtree's own slots [node*bf*bf,
         (node+1)*bf*bf); its level-1 nodes get new centres, radii and counts; the level-2
         node keeps its centre, gets the radius its new children need, and its ancestors are
-        inflated where that radius grew.  One build over all trees (hira_build_ragged: the trees
-        hold different numbers of keys there) and a few batched tensor operations; nothing is
-        read back to the host."""
+        inflated where that radius grew.  One call of the library for all trees, whatever numbers of
+        keys they hold there; nothing is read back to the host."""
         if self.keys_buf is None:
             raise ValueError("Indexer is not built: call build() first.")
         if self.num_levels < 3:
@@ -1005,71 +1004,17 @@ class HIPIndexer(BaseIndexer):
         s0, n0 = node * nsub, node * bf
         if s0 + nsub > self.cap[0] or n0 + bf > self.cap[1]:
             raise ValueError("the subtree's slots lie beyond the capacity of the index")
-        # the subtree's keys of every tree, those it holds first (in slot order); how many each
-        # tree holds stays on the device: nothing here waits for the GPU
-        perm_sub = self.perm[:, s0:s0 + nsub]
-        live = perm_sub >= 0
-        order = torch.sort((~live).to(torch.uint8), dim=1, stable=True).indices  # (T, nsub)
-        counts = live.sum(dim=1, dtype=torch.int32).contiguous()
-        rows = self.keys_buf[:, s0:s0 + nsub]
-        rows = from_tiled(rows) if self.keys_tiled else rows
-        rows = torch.gather(rows, 1, order[:, :, None].expand(-1, -1, self.dim))
-        vals = None
-        if self.values_buf is not None:
-            vals = torch.gather(self.values_buf[:, s0:s0 + nsub], 1,
-                                order[:, :, None].expand(-1, -1, self.vdim))
-        pos = torch.gather(perm_sub, 1, order)  # insertion positions, the missing ones (-1) last
-        # one build over all trees: two levels, bf nodes of bf slots, fewer keys in some trees
-        sub = HIPIndexer(2, self.max_iterations, bf, seed=self.seed + node,
-                         device=str(self.device), pack_rounds=self.pack_rounds,
-                         layout=self.layout_name)
-        sub.build(rows.reshape(self.batch, self.num_heads, nsub, self.dim),
-                  None if vals is None else vals.reshape(self.batch, self.num_heads, nsub, self.vdim),
-                  key_counts=counts)
-        if sub.size[0] != nsub or sub.size[1] != bf or sub.tiled != self.tiled or sub.q8 != self.q8:
-            raise RuntimeError("sub-tree layout differs from the index's")
-        # a node's children fill its slots from the first one on (appends open the next child
-        # behind them): the new level-1 nodes that hold keys go first, whole nodes moving with
-        # their bf key slots (a node's rows are whole tiles, so tiled rows move as they are)
-        cnt1 = sub.counts[1][:, :bf]
-        nodes = torch.sort((cnt1 == 0).to(torch.uint8), dim=1, stable=True).indices  # (T, bf)
-
-        def by_node(x, width):  # (T, bf * bf, width) in slot order -> nodes in the new order
-            idx = nodes[:, :, None].expand(-1, -1, bf * width)
-            return torch.gather(x.reshape(T, bf, bf * width), 1, idx).reshape(T, nsub, width)
-
-        self.keys_buf[:, s0:s0 + nsub] = by_node(sub.keys_buf[:, :nsub], self.dim)
-        if vals is not None:
-            self.values_buf[:, s0:s0 + nsub] = by_node(sub.values_buf[:, :nsub], self.vdim)
-        sp = by_node(sub.perm[:, :nsub, None], 1)[:, :, 0].long()
-        self.perm[:, s0:s0 + nsub] = torch.where(
-            sp >= 0, torch.gather(pos, 1, sp.clamp(min=0)), torch.full_like(pos, -1))
-        c1 = torch.gather(sub.centers_rowmajor(1)[:, :bf], 1,
-                          nodes[:, :, None].expand(-1, -1, self.dim))     # (T, bf, D), storage type
-        r1 = torch.gather(sub.radii[1][:, :bf], 1, nodes)                  # (T, bf), -inf: empty
-        cnt1 = torch.gather(cnt1, 1, nodes)
-        self.centers[1][:, n0:n0 + bf] = to_tiled(c1) if self.tiled else c1
-        self.radii[1][:, n0:n0 + bf] = r1
-        self.counts[1][:, n0:n0 + bf] = cnt1
-        # level 2: same centre, the radius its new children need; ancestors cover it where it grew
-        c1 = c1.float()
-        child, c_child, r_child = node, None, None
-        for l in range(2, self.num_levels):
-            tile0 = child // 16 * 16  # (de-tiling needs whole tiles)
-            cl = self.centers[l][:, tile0:tile0 + 16]
-            cl = (from_tiled(cl) if self.tiled else cl)[:, child - tile0].float()  # (T, D)
-            if l == 2:
-                r = ((c1 - cl[:, None]).norm(dim=2) + r1).amax(dim=1) * (1 + 1e-6)
-                self.counts[2][:, child] = (cnt1 > 0).sum(dim=1, dtype=torch.int32)
-            else:
-                r = torch.maximum(self.radii[l][:, child],
-                                  ((c_child - cl).norm(dim=1) + r_child) * (1 + 1e-6))
-            self.radii[l][:, child] = r
-            c_child, r_child, child = cl, r, child // bf
-        if self._state is not None:
-            self._state[:, 0] = 0  # the rebuilt nodes may have room again
-        self._tree_struct = None
-        self.quantize(s0, nsub)
+        lib, tree = _lib.lib(), self.tree_struct()
+        stream = _lib.stream_of(self.keys_buf.get_device())
+        need = lib.hira_rebuild_workspace_bytes(C.byref(tree))
+        if need == 0:
+            _lib.check(-1)
+        ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+        rc = lib.hira_rebuild_subtree(
+            C.byref(tree), node, self.max_iterations, self.pack_rounds, self.seed + node,
+            None if self._state is None else self._state.data_ptr(), ws.data_ptr(), need, stream)
+        if rc:
+            _lib.check(rc)
         return self
 
 

@@ -257,6 +257,18 @@ int hira_build_ragged(const HiraTree* tree, const void* keys_in, const void* val
                       void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The subtree under node `node` of level 2 of EVERY tree clustered anew (three levels or more): its keys in two
+ * levels as hira_build_ragged would, nodes with keys first, the level-2 node's radius and its ancestors'; what the
+ * reference does to a node that has grown uneven by building an index over its keys (indexer/cuda.py:544-701).
+ * Slots [node * bf * bf, +bf * bf) and level-1 nodes [node * bf, +bf) must lie inside cap[].
+ *   state   hira_update's, or NULL: told that the rebuilt nodes may have room again
+ * Enqueues on the stream, nothing is read back.  Tiled layouts: bf a multiple of 16.
+ */
+size_t hira_rebuild_workspace_bytes(const HiraTree* tree);
+int hira_rebuild_subtree(const HiraTree* tree, int32_t node, int32_t niter, int32_t pack_rounds, uint64_t seed,
+                         int32_t* state, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Nearest centre of every row, the distance step of the build (every Lloyd round and every
  * packing round of hira_build runs these kernels) as a call of its own:
  *   idx[t][i] = argmin_k ||x[t][i] - centers[t][k]||^2 over the centres with valid[t][k] != 0,
