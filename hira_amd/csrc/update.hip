@@ -387,7 +387,9 @@ __device__ __attribute__((noinline)) void update_one_key_called(const UpdatePara
 //   rows       of the 64 keys to their slots, 16 bytes a thread.
 // What bounds it is latency in one workgroup a tree (its waves wait 69 % of their cycles).  A launch, 8 trees
 // of 128 bf16 columns: with 48 nodes to list, 48 us for 4 keys, 52 for 16, 60 for 32, 87 for 64; with one
-// node, full after 32 keys, and then another: 14 us for 4, 20 for 32, 31 for 64, 57 for 128, 110 for 256.
+// node, full after 32 keys, and then another: 16 us for 4, 19 for 32, 27 for 64, 47 for 128, 93 for 255 (33, 59 and
+// 119 for the last three when a key that opens a node looked for its parent in memory, the distances to the new node
+// were taken of keys that it has no room for, and the 8-bit shadow was written a byte at a time).
 // Radii wait until the list is given up: R = max over the keys of what each asks for, and that
 // grows with the distance, so the largest distance a candidate saw gives the radius that key by
 // key would have reached, to the last bit, and so up the levels.  A key that finds all candidates
@@ -401,10 +403,15 @@ constexpr int kCandMax = 48;
 constexpr int kWinKeys = 64;  // keys of a window taken together
 // COLS, below: columns of a row a lane holds, at most.  Rows of fp32, and of bf16 up to 256, take four;
 // wider ones five (320 columns): 8 trees x 64 keys of 288 columns, which went key by key, 358 -> 61 us.
-// Five for all rows would cost those of 128 columns 0.8 us of 33.
+// Five for all rows would cost those of 128 columns 0.8 us a launch.
 constexpr int kWinColsMax = 5;
-constexpr size_t kWinLds = 128 * 1024;  // dynamic LDS of a workgroup, at most (256 fp32 columns: 126 KiB; 320
-                                        // bf16 columns: 115)
+constexpr size_t kWinLds = 144 * 1024;  // dynamic LDS of a workgroup, at most (256 fp32 columns: 142 KiB; 320
+                                        // bf16 columns: 135)
+// Level-2 nodes with room, listed like those of level 1, so that a key that opens a node finds its parent without a
+// trip to memory.  More than the list holds, or more nodes to look through than one trip reads: no list.
+template <typename T>
+constexpr int kParents = 64 / (int)sizeof(T);
+constexpr int kParentsMax = 32, kParentCounts = 4;  // (counts a thread reads)
 
 struct WindowLds {
     int n;                                  // candidates listed (may exceed kCandMax: then unusable)
@@ -418,6 +425,9 @@ struct WindowLds {
     int anc_rep[HIRA_MAX_LEVELS][kCandMax];     // [l][c]: the first candidate with the same ancestor at level l
     float anc_rad[HIRA_MAX_LEVELS][kCandMax];   // [l][rep]: that ancestor's radius
     float anc_step[HIRA_MAX_LEVELS][kCandMax];  // [l][c]: distance between c's ancestors at levels l-1 and l
+    int n2;                                 // level-2 nodes listed (more than kParents: no list)
+    int id2[kParentsMax], cnt2[kParentsMax];
+    float d2[kParentsMax];                  // squared distances of a key to them
 };
 
 // level-l ancestor of level-1 node `node1` (l >= 1)
@@ -426,18 +436,27 @@ __device__ __forceinline__ size_t ancestor_of(size_t node1, int l, int bf) {
     return node1;
 }
 
-// Reads the tree's level-1 nodes with room into LDS.  cen: (kCandMax, D) floats.  Returns false
-// (uniform) when there are more than the list holds.
+// Reads the tree's level-1 nodes with room into LDS, and those of level 2.  cen: (kCandMax, D) floats, par:
+// (kParents, D).  Returns false (uniform) when there are more of level 1 than the list holds.
 template <typename T>
-__device__ bool window_candidates(const UpdateParams& p, const int tree, WindowLds& w, float* cen) {
+__device__ bool window_candidates(const UpdateParams& p, const int tree, WindowLds& w, float* cen, T* par) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int D = p.dim, L = p.num_levels, bf = p.bf;
     int32_t* st = p.state + (size_t)tree * (HIRA_MAX_LEVELS + 2);
     const int used = st[1], first = min(max(st[0], 0), used);
+    const int used2 = L > 2 ? st[2] : 0;
+    const bool look2 = used2 <= kParentCounts * kUpdThreads;
     const size_t b1 = (size_t)tree * p.cap[1];
     if (t == 0) {
         w.n = 0;
         w.low_empty = used;
+        w.n2 = look2 ? 0 : kParents<T> + 1;
+    }
+    int c2[kParentCounts];  // (on their way beside level 1's)
+#pragma unroll
+    for (int u = 0; u < kParentCounts; ++u) {
+        const int n = u * kUpdThreads + t;
+        c2[u] = look2 && n < used2 ? p.counts[2][(size_t)tree * p.cap[2] + n] : bf;
     }
     __syncthreads();
     for (int nb = first & ~63; nb < used; nb += kUpdThreads) {  // uniform
@@ -456,9 +475,20 @@ __device__ bool window_candidates(const UpdateParams& p, const int tree, WindowL
             w.far[at] = -1.0f;
         }
     }
+#pragma unroll
+    for (int u = 0; u < kParentCounts; ++u)
+        if (c2[u] > 0 && c2[u] < bf) {
+            const int at = atomicAdd(&w.n2, 1);
+            if (at < kParents<T>) {
+                w.id2[at] = u * kUpdThreads + t;
+                w.cnt2[at] = c2[u];
+            }
+        }
     __syncthreads();
-    const int nc = w.n;
+    const int nc = w.n, n2 = w.n2 <= kParents<T> ? w.n2 : 0;
     if (nc > kCandMax) return false;
+    for (int e = t; e < n2 * D; e += kUpdThreads)
+        store_elem<T>(par, e, load_elem<T>(p.centers[2], (size_t)tree * p.cap[2] * D + elem_index(p.layout, D, (size_t)w.id2[e / D], e % D)));
     // (the order in which the waves listed their nodes does not matter: ties between candidates
     // are decided by the node's id)
     for (int c = wave; c < nc; c += kUpdThreads / 64) {  // uniform in the wave
@@ -723,9 +753,104 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
     return node1;
 }
 
+// The same from the list of level-2 nodes, where one of them has room: the new level-1 node gets its place, its centre
+// (also to cen) and its parent's count, the path above its radii, and it becomes the list of candidates; the key's row
+// goes the way of all others (its slot to *slot).  Returns the node, or -1 (uniform, and nothing is changed): no node
+// of the list takes the key, or the slot lies behind the capacity.
+template <typename T>
+__device__ __forceinline__ int open_listed(const UpdateParams& p, const int tree, int* s_used, int* slot, const T* key, const T* par,
+                                           WindowLds& w, float* cen, float* s_dist, float* s_rad) {
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int D = p.dim, L = p.num_levels, bf = p.bf, n2 = w.n2;
+    const size_t b1 = (size_t)tree * p.cap[1];
+    for (int e = wave; e < n2; e += kUpdThreads / 64) {  // uniform in the wave
+        float ss = 0.0f;
+        for (int j = lane; j < D; j += 64) {
+            const float df = load_elem<T>(key, j) - load_elem<T>(par, (size_t)e * D + j);
+            ss += df * df;
+        }
+        ss += win_partner<1>(ss);
+        ss += win_partner<2>(ss);
+        ss += win_partner<4>(ss);
+        ss += win_partner<8>(ss);
+        ss = win_sum_across<16>(ss);
+        ss = win_sum_across<32>(ss);
+        if (lane == 0) w.d2[e] = w.cnt2[e] < bf && ss < INFINITY ? ss : INFINITY;
+    }
+    __syncthreads();
+    const float d = lane < n2 ? w.d2[lane] : INFINITY;
+    const float best = win_min(d);
+    if (best == INFINITY) return -1;
+    int low = d == best ? w.id2[min(lane, kParentsMax - 1)] : 0x7fffffff;  // (ties: the lowest node)
+    unsigned long long who = __ballot(d == best);
+    if (who & (who - 1ull)) {
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
+        who = __ballot(d == best && w.id2[min(lane, kParentsMax - 1)] == low);
+    }
+    const int c = __ffsll((long long)who) - 1, parent = w.id2[c], pcount = w.cnt2[c];
+    const long long idx = (long long)parent * bf + pcount;
+    if (idx >= p.cap[1] || idx * bf >= p.cap[0]) return -1;
+    for (int j = t; j < D; j += kUpdThreads) {
+        const float x = load_elem<T>(key, j);
+        store_elem<T>(p.centers[1], b1 * D + elem_index(p.layout, D, (size_t)idx, j), x);
+        cen[j] = x;
+    }
+    for (int l = 2 + wave; l < L; l += kUpdThreads / 64) {  // the path above: a wave per level
+        const size_t node = ancestor_of((size_t)parent, l - 1, bf);
+        const float rad_now = p.radii[l][(size_t)tree * p.cap[l] + node];
+        float ss = best;
+        if (l > 2) {
+            const size_t child = ancestor_of((size_t)parent, l - 2, bf);
+            const size_t bl = (size_t)tree * p.cap[l], bc = (size_t)tree * p.cap[l - 1];
+            ss = 0.0f;
+            for (int j = lane; j < D; j += 64) {
+                const float a = load_elem<T>(p.centers[l - 1], bc * D + elem_index(p.layout, D, child, j));
+                const float b = load_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, node, j));
+                ss += (a - b) * (a - b);
+            }
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+        }
+        if (lane == 0) {
+            s_dist[l] = sqrtf(ss);
+            s_rad[l] = rad_now;
+        }
+    }
+    if (t == 0) {
+        p.radii[1][b1 + idx] = 0.0f;
+        p.counts[1][b1 + idx] = 1;
+        p.counts[2][(size_t)tree * p.cap[2] + parent] = pcount + 1;
+        if (p.keps != nullptr) p.keps[b1 + idx] = 0.0f;  // (its keys' rows raise it)
+        if (idx + 1 > s_used[1]) s_used[1] = p.state[(size_t)tree * (HIRA_MAX_LEVELS + 2) + 1] = (int)(idx + 1);
+        *slot = (int)(idx * bf);
+        w.n = 1;
+        w.id[0] = (int)idx;
+        w.cnt[0] = w.cnt0[0] = 1;
+        w.rad[0] = 0.0f;
+        w.far[0] = -1.0f;
+    }
+    __syncthreads();
+    if (t == 0) {  // (nobody reads this until the next barrier)
+        w.cnt2[c] = pcount + 1;
+        float r_child = 0.0f;
+        for (int l = 2; l < L; ++l) {
+            const size_t node = ancestor_of((size_t)parent, l - 1, bf);
+            const float rn = fmaxf(s_rad[l], pad_up(s_dist[l] + r_child));
+            if (rn != s_rad[l]) p.radii[l][(size_t)tree * p.cap[l] + node] = rn;
+            r_child = rn;
+            w.anc_id[l][0] = (int)node;
+            w.anc_rep[l][0] = 0;
+            w.anc_step[l][0] = s_dist[l];
+            w.anc_rad[l][0] = rn;
+        }
+    }
+    return (int)idx;
+}
+
 template <typename T, int COLS>
 __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParams p) {
-    // 2 D floats of the general way, kCandMax centres, the table of distances, a chunk of key rows
+    // 2 D floats of the general way, kCandMax centres, the table of distances, kParents centres, a chunk of key rows
     extern __shared__ __attribute__((aligned(16))) float sm[];
     __shared__ float red_f[4];
     __shared__ int red_i[4];
@@ -741,7 +866,8 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
     const int D = p.dim, Dv = p.vdim, L = p.num_levels, bf = p.bf;
     float* cen = sm + 2 * (size_t)D;
     float* table = cen + (size_t)kCandMax * D;
-    T* rows = reinterpret_cast<T*>(table + (size_t)kCandMax * kWinKeys);  // (kWinKeys, D): the chunk's keys
+    T* par = reinterpret_cast<T*>(table + (size_t)kCandMax * kWinKeys);
+    T* rows = par + (size_t)kParents<T> * D;  // (kWinKeys, D): the chunk's keys
     uint4* vals = p.stage_values ? reinterpret_cast<uint4*>(rows + (size_t)kWinKeys * D) : nullptr;  // its values
     int32_t* st = p.state + (size_t)tree * (HIRA_MAX_LEVELS + 2);
     const size_t base0 = (size_t)tree * p.cap[0], b1 = (size_t)tree * p.cap[1];
@@ -774,7 +900,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
     int position = st[HIRA_MAX_LEVELS];  // of the next key (every thread carries it along)
     stage(0);
     if (t >= 1 && t < L) s_used[t] = st[t];
-    if (!window_candidates<T>(p, tree, w, cen)) {  // uniform: the tree's keys go the general way, all of them
+    if (!window_candidates<T>(p, tree, w, cen, par)) {  // uniform: the tree's keys go the general way, all of them
         for (int i = 0; i < p.m; ++i) update_one_key_called<T>(p, tree, i, sm, red_f, red_i, s_dist, s_rad);
         return;
     }
@@ -853,33 +979,59 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
                 // key k found no node with room, or none at a distance that is a finite number: it opens one
                 list_anew = s_room;
                 window_flush(p, tree, w);
-                const int node = open_node<T>(p, tree, i0 + k, position, s_used, rows + (size_t)k * D, sm, red_f, red_i, s_dist, s_rad);
-                if (node >= 0) ++position;
-                if (list_anew) {  // uniform
-                    nk = k + 1;
-                    break;
-                }
-                // (all listed nodes are full: the new one is the whole list from here on)
-                if (t == 0) {
-                    w.n = node >= 0 ? 1 : 0;
-                    w.id[0] = node;
-                    w.cnt[0] = w.cnt0[0] = 1;
-                    w.rad[0] = s_rad[1];
-                    w.far[0] = -1.0f;
-                    for (int l = 2; l < L; ++l) {
-                        w.anc_id[l][0] = (int)ancestor_of((size_t)max(node, 0), l, bf);
-                        w.anc_rep[l][0] = 0;
-                        w.anc_step[l][0] = s_dist[l];
-                        w.anc_rad[l][0] = s_rad[l];
+                const T* key = rows + (size_t)k * D;
+                int node = -1;
+                if (!list_anew && L > 2 && w.n2 <= kParents<T>)  // uniform
+                    node = open_listed<T>(p, tree, s_used, &s_slot[k], key, par, w, cen, s_dist, s_rad);
+                if (node >= 0) {
+                    ++position;
+                } else {
+                    // (with no room left in the list a node of level 2 is opened too, the only one there with room then)
+                    bool none2 = w.n2 <= kParents<T>;
+                    for (int e = 0; none2 && e < w.n2; ++e) none2 = w.cnt2[e] >= bf;
+                    node = open_node<T>(p, tree, i0 + k, position, s_used, key, sm, red_f, red_i, s_dist, s_rad);
+                    if (node >= 0) ++position;
+                    if (list_anew) {  // uniform
+                        nk = k + 1;
+                        break;
                     }
+                    // (all listed nodes are full: the new one is the whole list from here on)
+                    if (t == 0) {
+                        w.n = node >= 0 ? 1 : 0;
+                        w.id[0] = node;
+                        w.cnt[0] = w.cnt0[0] = 1;
+                        w.rad[0] = s_rad[1];
+                        w.far[0] = -1.0f;
+                        for (int l = 2; l < L; ++l) {
+                            w.anc_id[l][0] = (int)ancestor_of((size_t)max(node, 0), l, bf);
+                            w.anc_rep[l][0] = 0;
+                            w.anc_step[l][0] = s_dist[l];
+                            w.anc_rad[l][0] = s_rad[l];
+                        }
+                        w.n2 = none2 && node >= 0 ? 1 : kParents<T> + 1;
+                        w.id2[0] = node / bf;
+                        w.cnt2[0] = 1;
+                    }
+                    for (int j = t; j < D; j += kUpdThreads) {  // (its centre is the key)
+                        cen[j] = sm[j];
+                        par[j] = key[j];
+                    }
+                    __syncthreads();
                 }
-                for (int j = t; j < D; j += kUpdThreads) cen[j] = sm[j];  // (its centre is the key)
-                __syncthreads();
                 ++k;
-                window_distances<T, COLS>(D, w, cen, rows, k, nk, table);
+                // (of the keys that it has room for: those behind them find it full, whatever the distance)
+                window_distances<T, COLS>(D, w, cen, rows, k, min(nk, k + bf - 1), table);
             }
         }
         // ---- the rows of the keys placed from the list, 16 bytes a thread -----------------------
+        float step[16];  // of a chunk of the 8-bit shadow: a thread's columns are the same for all its keys
+        const int sc = D / 16, my_chunk = t % max(sc, 1);
+        if (p.keys8 != nullptr)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 v = reinterpret_cast<const float4*>(p.kscale + (size_t)tree * D + my_chunk * 16)[q];
+                step[q * 4] = v.x, step[q * 4 + 1] = v.y, step[q * 4 + 2] = v.z, step[q * 4 + 3] = v.w;
+            }
         const bool v_chunks = with_values && Dv % EPL == 0;
         const int vc = v_chunks ? Dv / EPL : 0, per = kc + vc;
         constexpr int RU = 4;  // chunks a thread has in flight
@@ -920,25 +1072,38 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
         }
         if (p.keys8 != nullptr) {
             // the keys' 8-bit shadow with the tree's steps; a component beyond +-127 steps clips,
-            // and the node's error bound then covers it.  A wave per key.
-            for (int q = wave; q < nk; q += kUpdThreads / 64) {  // uniform in the wave
-                const int slot = s_slot[q];
-                if (slot < 0) continue;
+            // and the node's error bound then covers it.  Sixteen columns a thread, 4 or 8 threads a key.
+            if (wave == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (thread 0's bounds of nodes opened here, ahead of
+            __syncthreads();                                                // the maxima that raise them)
+            for (int e0 = 0; e0 < nk * sc; e0 += kUpdThreads) {  // uniform
+                const int q = min((e0 + t) / sc, nk - 1), slot = e0 + t < nk * sc ? s_slot[q] : -1;
                 float worst = 0.0f;
-                for (int j = lane; j < D; j += 64) {
-                    const float u = load_elem<T>(rows, (size_t)q * D + j) / p.kscale[(size_t)tree * D + j];
-                    const float k8 = fminf(fmaxf(rintf(u), -127.0f), 127.0f);
-                    worst = fmaxf(worst, fabsf(u - k8));
-                    p.keys8[base0 * D + shadow_index(D, (size_t)slot, j)] = (int8_t)(int)k8;
+                uint32_t out[4];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    out[g] = 0;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float u = load_elem<T>(rows, (size_t)q * D + my_chunk * 16 + g * 4 + e) / step[g * 4 + e];
+                        const float k8 = fminf(fmaxf(rintf(u), -127.0f), 127.0f);
+                        worst = fmaxf(worst, fabsf(u - k8));
+                        out[g] |= (uint32_t)(uint8_t)(int8_t)(int)k8 << (8 * e);
+                    }
                 }
-                worst = wave_max(worst);
-                if (lane == 0) atomicMax(reinterpret_cast<int*>(p.keps + b1 + slot / bf), __float_as_int(worst));
+                worst = fmaxf(worst, win_partner<1>(worst));
+                worst = fmaxf(worst, win_partner<2>(worst));
+                if (sc > 4) worst = fmaxf(worst, win_partner<4>(worst));  // uniform
+                if (slot >= 0) {
+                    *reinterpret_cast<uint4*>(p.keys8 + base0 * D + shadow_index(D, (size_t)slot, my_chunk * 16)) =
+                        make_uint4(out[0], out[1], out[2], out[3]);
+                    if (my_chunk == 0) atomicMax(reinterpret_cast<int*>(p.keps + b1 + slot / bf), __float_as_int(worst));
+                }
             }
         }
         i0 += nk;
         if (list_anew) {  // uniform
             __syncthreads();
-            if (!window_candidates<T>(p, tree, w, cen)) {
+            if (!window_candidates<T>(p, tree, w, cen, par)) {
                 if (t == 0) st[HIRA_MAX_LEVELS] = position;
                 __syncthreads();
                 for (; i0 < p.m; ++i0) update_one_key_called<T>(p, tree, i0, sm, red_f, red_i, s_dist, s_rad);
@@ -1014,8 +1179,8 @@ static int update_arguments(const HiraTree* tree, const void* new_keys, const vo
     p.state = state;
     *smem = 2 * (size_t)tree->dim * sizeof(float);
     // windows of a few keys and more: the nodes with room are listed in LDS (where they fit: 48 centres
-    // of up to 256 columns, bf16 320, beside the table of distances and a chunk of rows)
-    *smem_w = *smem + (size_t)kCandMax * (tree->dim + kWinKeys) * sizeof(float) +
+    // of up to 256 columns, bf16 320, and those of level 2 beside the table of distances and a chunk of rows)
+    *smem_w = *smem + (size_t)kCandMax * (tree->dim + kWinKeys) * sizeof(float) + (size_t)64 * tree->dim +
               (size_t)kWinKeys * tree->dim * (tree->dtype == HIRA_F32 ? 4 : 2);
     *window = m >= 4 && tree->num_levels >= 2 && tree->dim <= 64 * (tree->dtype == HIRA_F32 ? 4 : kWinColsMax) && *smem_w <= kWinLds;
     const size_t vrow = (size_t)tree->vdim * (tree->dtype == HIRA_F32 ? 4 : 2);
