@@ -29,7 +29,8 @@
 
 namespace hira {
 
-constexpr int kUpdThreads = 256;
+constexpr int kUpdThreads = 256;  // of a workgroup that takes key after key
+constexpr int kWinThreads = 512;  // of one that takes a window (the functions of both: NT)
 
 struct UpdateParams {
     void* keys;
@@ -59,8 +60,8 @@ __device__ __forceinline__ float pad_up(float r) { return r > 0.0f ? r * (1.0f +
 // costs one count read.  Ties go to the lowest id.  *not_full (if given) receives the lowest
 // index from `first` on whose node is not full (`used` if there is none).
 constexpr int kCountsInFlight = 16;  // reads of child counts a lane has in flight
-template <typename T>
-__device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int first, int used,
+template <typename T, int NT>
+__device__ __forceinline__ int nearest_with_room(const UpdateParams& p, int tree, int l, int first, int used,
                                  const float* x, float* red_f, int* red_i, int* not_full,
                                  int* count_of = nullptr, float* dist2_of = nullptr,
                                  float* radius_of = nullptr) {
@@ -72,24 +73,24 @@ __device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int fir
     int arg = -1, argc = 0;  // the best node so far and its child count
     float argr = 0.0f;       // (its radius, asked for with the centre)
     int low = used;  // lowest index of a node that is not full, among those I have seen
-    for (int nb = (first & ~63) + wave * 64; nb < used; nb += kCountsInFlight * 4 * 64) {
+    for (int nb = (first & ~63) + wave * 64; nb < used; nb += kCountsInFlight * NT) {
         // the reads of the child counts in flight together (a wave's nodes still come in
         // increasing order): one trip to memory for 4096 nodes
         int c4[kCountsInFlight];
 #pragma unroll
         for (int u = 0; u < kCountsInFlight; ++u) {
-            const int n = nb + u * 4 * 64 + lane;
+            const int n = nb + u * NT + lane;
             c4[u] = n < used ? cnt[n] : p.bf;
         }
 #pragma unroll
         for (int u = 0; u < kCountsInFlight; ++u) {
-            if (nb + u * 4 * 64 >= used) break;  // uniform
-            if (c4[u] < p.bf) low = min(low, nb + u * 4 * 64 + lane);
+            if (nb + u * NT >= used) break;  // uniform
+            if (c4[u] < p.bf) low = min(low, nb + u * NT + lane);
             // a node in use with a free slot; count 0 marks a pad slot, which is not a node yet
             unsigned long long bal = __ballot(c4[u] > 0 && c4[u] < p.bf);
             while (bal != 0ull) {  // uniform in the wave
                 const int src = __ffsll((long long)bal) - 1;
-                const int node = nb + u * 4 * 64 + src;
+                const int node = nb + u * NT + src;
                 const int node_c = __shfl(c4[u], src, 64);
                 bal &= bal - 1ull;
                 float ss = 0.0f;
@@ -115,7 +116,11 @@ __device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int fir
         for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
         if (lane == 0) red_i[wave] = low;
         __syncthreads();
-        if (threadIdx.x == 0) *not_full = max(min(min(red_i[0], red_i[1]), min(red_i[2], red_i[3])), first);
+        if (threadIdx.x == 0) {
+#pragma unroll
+            for (int w = 1; w < NT / 64; ++w) low = min(low, red_i[w]);
+            *not_full = max(low, first);
+        }
         __syncthreads();
     }
     if (lane == 0) {
@@ -126,7 +131,7 @@ __device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int fir
     float b = red_f[0];
     int a = red_i[0], aw_of = 0;
 #pragma unroll
-    for (int w = 1; w < 4; ++w) {
+    for (int w = 1; w < NT / 64; ++w) {
         const float bw = red_f[w];
         const int aw = red_i[w];
         if (aw >= 0 && (a < 0 || bw < b || (bw == b && aw < a))) {
@@ -154,8 +159,8 @@ __device__ int nearest_with_room(const UpdateParams& p, int tree, int l, int fir
 
 // One key of the window, placed the general way: key i of the tree's new keys.
 //   sm: 2 D floats (the key, the centre of a node being attached upwards).
-template <typename T>
-__device__ void update_one_key(const UpdateParams& p, const int tree, const int i, float* sm, float* red_f,
+template <typename T, int NT>
+__device__ __forceinline__ void update_one_key(const UpdateParams& p, const int tree, const int i, float* sm, float* red_f,
                                int* red_i, float* s_dist, float* s_rad) {
     float* x = sm;              // (D) the new key, fp32
     float* cbuf = sm + p.dim;   // (D) centre of the node being attached upwards
@@ -165,7 +170,7 @@ __device__ void update_one_key(const UpdateParams& p, const int tree, const int 
     const size_t base0 = (size_t)tree * p.cap[0];
 
     const size_t src = ((size_t)tree * p.m + i) * D;
-    for (int j = t; j < D; j += kUpdThreads) x[j] = load_elem<T>(p.new_keys, src + j);
+    for (int j = t; j < D; j += NT) x[j] = load_elem<T>(p.new_keys, src + j);
     __syncthreads();
     const int position = st[HIRA_MAX_LEVELS];
 
@@ -175,12 +180,12 @@ __device__ void update_one_key(const UpdateParams& p, const int tree, const int 
     if (L == 1) {
         slot = position < p.cap[0] ? position : -1;
     } else {
-        node1 = nearest_with_room<T>(p, tree, 1, min(max(st[0], 0), st[1]), st[1], x, red_f, red_i, &st[0],
+        node1 = nearest_with_room<T, NT>(p, tree, 1, min(max(st[0], 0), st[1]), st[1], x, red_f, red_i, &st[0],
                                          &count1);
         if (node1 < 0) {
             // ---- open a new level-1 node; attach it upwards -----------------------
             // child_c = centre of the node being attached (the key itself at level 1)
-            for (int j = t; j < D; j += kUpdThreads) cbuf[j] = x[j];
+            for (int j = t; j < D; j += NT) cbuf[j] = x[j];
             __syncthreads();
             int lvl = 1;          // level of the node that needs a parent
             int parent = -1;      // node of level lvl+1 that takes it
@@ -191,7 +196,7 @@ __device__ void update_one_key(const UpdateParams& p, const int tree, const int 
                     parent = -1;
                     break;
                 }
-                parent = nearest_with_room<T>(p, tree, lvl + 1, 0, st[lvl + 1], cbuf, red_f, red_i, nullptr);
+                parent = nearest_with_room<T, NT>(p, tree, lvl + 1, 0, st[lvl + 1], cbuf, red_f, red_i, nullptr);
                 if (parent >= 0) break;
                 ++lvl;
             }
@@ -220,7 +225,7 @@ __device__ void update_one_key(const UpdateParams& p, const int tree, const int 
             id = idx;
             for (int l = opened_top; l >= 1; --l) {
                 const size_t bl = (size_t)tree * p.cap[l];
-                for (int j = t; j < D; j += kUpdThreads)
+                for (int j = t; j < D; j += NT)
                     store_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, (size_t)id, j), x[j]);
                 if (t == 0) {
                     p.radii[l][bl + id] = 0.0f;
@@ -252,13 +257,13 @@ __device__ void update_one_key(const UpdateParams& p, const int tree, const int 
     {
         const T* dummy = nullptr;
         (void)dummy;
-        for (int j = t; j < D; j += kUpdThreads)
+        for (int j = t; j < D; j += NT)
             store_elem<T>(p.keys, base0 * D + elem_index(p.key_layout, D, (size_t)slot, j), x[j]);
         if (p.keys8 != nullptr) {
             // the key's 8-bit shadow with the tree's steps; a component beyond +-127 steps
             // clips, and the node's error bound then covers it
             float worst = 0.0f;
-            for (int j = t; j < D; j += kUpdThreads) {
+            for (int j = t; j < D; j += NT) {
                 const float u = x[j] / p.kscale[(size_t)tree * D + j];
                 const float r = fminf(fmaxf(rintf(u), -127.0f), 127.0f);
                 worst = fmaxf(worst, fabsf(u - r));
@@ -269,7 +274,9 @@ __device__ void update_one_key(const UpdateParams& p, const int tree, const int 
             __syncthreads();
             if (t == 0) {
                 float* e = p.keps + (size_t)tree * p.cap[1] + node1;
-                const float w = fmaxf(fmaxf(red_f[0], red_f[1]), fmaxf(red_f[2], red_f[3]));
+                float w = red_f[0];
+#pragma unroll
+                for (int i = 1; i < NT / 64; ++i) w = fmaxf(w, red_f[i]);
                 // a node that just opened holds no other key: its bound starts here
                 const bool fresh = count1 == 0;
                 *e = fresh ? w : fmaxf(*e, w);
@@ -278,7 +285,7 @@ __device__ void update_one_key(const UpdateParams& p, const int tree, const int 
         }
         if (p.new_values && p.values) {
             const size_t vs = ((size_t)tree * p.m + i) * Dv;
-            for (int j = t; j < Dv; j += kUpdThreads)
+            for (int j = t; j < Dv; j += NT)
                 store_elem<T>(p.values, (base0 + slot) * Dv + j, load_elem<T>(p.new_values, vs + j));
         }
         if (t == 0) {
@@ -292,7 +299,7 @@ __device__ void update_one_key(const UpdateParams& p, const int tree, const int 
     // the chain R_l = max(R_l, d_l + R_{l-1}). ---------------------------------------------
     if (L >= 2) {
         const int lane = t & 63;
-        for (int l = 1 + (t >> 6); l < L; l += kUpdThreads / 64) {  // uniform in the wave
+        for (int l = 1 + (t >> 6); l < L; l += NT / 64) {  // uniform in the wave
             size_t child = (size_t)node1;  // node of level l - 1 on the key's path (l >= 2)
             for (int i = 2; i < l; ++i) child /= (size_t)bf;
             const size_t node = l == 1 ? (size_t)node1 : child / (size_t)bf;
@@ -335,7 +342,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update(const UpdateParams p) {
     __shared__ int red_i[4];
     __shared__ float s_dist[HIRA_MAX_LEVELS], s_rad[HIRA_MAX_LEVELS];
     for (int i = 0; i < p.m; ++i)
-        update_one_key<T>(p, (int)blockIdx.x, i, sm, red_f, red_i, s_dist, s_rad);
+        update_one_key<T, kUpdThreads>(p, (int)blockIdx.x, i, sm, red_f, red_i, s_dist, s_rad);
 }
 
 // An append of a few keys per tree and the thresholds of a decode step in one launch: the first
@@ -355,7 +362,7 @@ __global__ __launch_bounds__(kTauThreads) void k_update_threshold(
     if ((int)blockIdx.x < trees) {  // uniform in the workgroup
         if (threadIdx.x >= kUpdThreads) return;
         for (int i = 0; i < p.m; ++i)
-            update_one_key<T>(p, (int)blockIdx.x, i, sm, red_f, red_i, s_dist, s_rad);
+            update_one_key<T, kUpdThreads>(p, (int)blockIdx.x, i, sm, red_f, red_i, s_dist, s_rad);
         return;
     }
     threshold_block<T, E>(samples, S, p.dim, q, tree_q_off, tree_q_heads, group_size, trees, method, k,
@@ -364,13 +371,6 @@ __global__ __launch_bounds__(kTauThreads) void k_update_threshold(
 
 // The general way as a call (the kernel below needs it now and then: its loop stays small, and the
 // compiler keeps the loop's values in registers instead of asking for them again every key).
-template <typename T>
-__device__ __attribute__((noinline)) void update_one_key_called(const UpdateParams& p, const int tree, const int i,
-                                                             float* sm, float* red_f, int* red_i, float* s_dist,
-                                                             float* s_rad) {
-    update_one_key<T>(p, tree, i, sm, red_f, red_i, s_dist, s_rad);
-}
-
 // ---- windows of several keys ---------------------------------------------------------------
 // Placing a key the general way costs a handful of dependent trips to memory (child counts,
 // the centres of the nodes with room, the ancestors' centres and radii): 4-5 us a key, one key
@@ -386,10 +386,12 @@ __device__ __attribute__((noinline)) void update_one_key_called(const UpdatePara
 //              the other;
 //   rows       of the 64 keys to their slots, 16 bytes a thread.
 // What bounds it is latency in one workgroup a tree (its waves wait 69 % of their cycles).  A launch, 8 trees
-// of 128 bf16 columns: with 48 nodes to list, 48 us for 4 keys, 52 for 16, 60 for 32, 87 for 64; with one
-// node, full after 32 keys, and then another: 16 us for 4, 19 for 32, 27 for 64, 47 for 128, 93 for 255 (33, 59 and
-// 119 for the last three when a key that opens a node looked for its parent in memory, the distances to the new node
-// were taken of keys that it has no room for, and the 8-bit shadow was written a byte at a time).
+// of 128 bf16 columns: with 45 nodes to list, 39 us for 4 keys, 42 for 16, 49 for 32, 57 for 64 (48, 52, 60, 87); with one
+// node, full after 32 keys, and then another: 13 us for 4, 15 for 32, 21 for 64, 35 for 128, 68 for 255 (16, 21, 33, 59
+// and 119 when a key that opens a node looked for its parent in memory, the distances to the new node were taken of
+// keys that it has no room for, the 8-bit shadow was written a byte at a time, and the general way was a call: a
+// kernel that calls needs scratch memory, and its launch then took 4 us more).  256 threads instead of 512: 13, 15,
+// 21, 37, 76.
 // Radii wait until the list is given up: R = max over the keys of what each asks for, and that
 // grows with the distance, so the largest distance a candidate saw gives the radius that key by
 // key would have reached, to the last bit, and so up the levels.  A key that finds all candidates
@@ -411,7 +413,7 @@ constexpr size_t kWinLds = 144 * 1024;  // dynamic LDS of a workgroup, at most (
 // trip to memory.  More than the list holds, or more nodes to look through than one trip reads: no list.
 template <typename T>
 constexpr int kParents = 64 / (int)sizeof(T);
-constexpr int kParentsMax = 32, kParentCounts = 4;  // (counts a thread reads)
+constexpr int kParentsMax = 32, kParentCounts = 2;  // (counts a thread reads)
 
 struct WindowLds {
     int n;                                  // candidates listed (may exceed kCandMax: then unusable)
@@ -438,14 +440,14 @@ __device__ __forceinline__ size_t ancestor_of(size_t node1, int l, int bf) {
 
 // Reads the tree's level-1 nodes with room into LDS, and those of level 2.  cen: (kCandMax, D) floats, par:
 // (kParents, D).  Returns false (uniform) when there are more of level 1 than the list holds.
-template <typename T>
-__device__ bool window_candidates(const UpdateParams& p, const int tree, WindowLds& w, float* cen, T* par) {
+template <typename T, int NT>
+__device__ __forceinline__ bool window_candidates(const UpdateParams& p, const int tree, WindowLds& w, float* cen, T* par) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int D = p.dim, L = p.num_levels, bf = p.bf;
     int32_t* st = p.state + (size_t)tree * (HIRA_MAX_LEVELS + 2);
     const int used = st[1], first = min(max(st[0], 0), used);
     const int used2 = L > 2 ? st[2] : 0;
-    const bool look2 = used2 <= kParentCounts * kUpdThreads;
+    const bool look2 = used2 <= kParentCounts * NT;
     const size_t b1 = (size_t)tree * p.cap[1];
     if (t == 0) {
         w.n = 0;
@@ -455,11 +457,11 @@ __device__ bool window_candidates(const UpdateParams& p, const int tree, WindowL
     int c2[kParentCounts];  // (on their way beside level 1's)
 #pragma unroll
     for (int u = 0; u < kParentCounts; ++u) {
-        const int n = u * kUpdThreads + t;
+        const int n = u * NT + t;
         c2[u] = look2 && n < used2 ? p.counts[2][(size_t)tree * p.cap[2] + n] : bf;
     }
     __syncthreads();
-    for (int nb = first & ~63; nb < used; nb += kUpdThreads) {  // uniform
+    for (int nb = first & ~63; nb < used; nb += NT) {  // uniform
         const int n = nb + t;
         const int c = (n >= first && n < used) ? p.counts[1][b1 + n] : bf;
         if (c <= 0) atomicMin(&w.low_empty, n);
@@ -480,18 +482,18 @@ __device__ bool window_candidates(const UpdateParams& p, const int tree, WindowL
         if (c2[u] > 0 && c2[u] < bf) {
             const int at = atomicAdd(&w.n2, 1);
             if (at < kParents<T>) {
-                w.id2[at] = u * kUpdThreads + t;
+                w.id2[at] = u * NT + t;
                 w.cnt2[at] = c2[u];
             }
         }
     __syncthreads();
     const int nc = w.n, n2 = w.n2 <= kParents<T> ? w.n2 : 0;
     if (nc > kCandMax) return false;
-    for (int e = t; e < n2 * D; e += kUpdThreads)
+    for (int e = t; e < n2 * D; e += NT)
         store_elem<T>(par, e, load_elem<T>(p.centers[2], (size_t)tree * p.cap[2] * D + elem_index(p.layout, D, (size_t)w.id2[e / D], e % D)));
     // (the order in which the waves listed their nodes does not matter: ties between candidates
     // are decided by the node's id)
-    for (int c = wave; c < nc; c += kUpdThreads / 64) {  // uniform in the wave
+    for (int c = wave; c < nc; c += NT / 64) {  // uniform in the wave
         const size_t node = (size_t)w.id[c];
         for (int j = lane; j < D; j += 64)
             cen[(size_t)c * D + j] = load_elem<T>(p.centers[1], b1 * D + elem_index(p.layout, D, node, j));
@@ -515,7 +517,7 @@ __device__ bool window_candidates(const UpdateParams& p, const int tree, WindowL
         }
     }
     __syncthreads();
-    for (int k = t; k < nc * HIRA_MAX_LEVELS; k += kUpdThreads) {
+    for (int k = t; k < nc * HIRA_MAX_LEVELS; k += NT) {
         const int c = k % nc, l = k / nc;
         if (l < 2 || l >= L) continue;
         const int anc = w.anc_id[l][c];
@@ -551,7 +553,7 @@ __device__ __forceinline__ float win_sum_across(float v) {
 // each, and goes through the candidates: the eight sums over the lanes halve in number with every
 // one of the first three steps (lanes with the bit set go on with the other half).  The additions are those of a butterfly of lane ^ 1, ^ 2,
 // ..., ^ 32, in that order: the general way's, to the last bit.
-template <typename T, int COLS>
+template <typename T, int COLS, int NT>
 __device__ __forceinline__ void window_distances(const int D, const WindowLds& w, const float* cen, const T* rows,
                                  const int k0, const int k1, float* table) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -559,7 +561,7 @@ __device__ __forceinline__ void window_distances(const int D, const WindowLds& w
     if (nc == 0) return;
     const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4;
     const int mine = (b0 ? 4 : 0) + (b1 ? 2 : 0) + (b2 ? 1 : 0);  // the key (of eight) I end up with
-    for (int k = k0 + wave * 8; k < k1; k += kUpdThreads / 64 * 8) {  // uniform in the wave
+    for (int k = k0 + wave * 8; k < k1; k += NT / 64 * 8) {  // uniform in the wave
         float x[8][COLS];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
@@ -612,7 +614,7 @@ __device__ __forceinline__ float win_min(float v) {  // over the wave, the same 
 
 // The list is given up: child counts and radii of the candidates that took keys, and their
 // ancestors' radii, go to memory.  By wave 0, a candidate a lane.
-__device__ void window_flush(const UpdateParams& p, const int tree, WindowLds& w) {
+__device__ __forceinline__ void window_flush(const UpdateParams& p, const int tree, WindowLds& w) {
     const int c = threadIdx.x, L = p.num_levels;
     if (c >= 64) return;
     const bool took = c < w.n && w.cnt[c] != w.cnt0[c];
@@ -648,7 +650,7 @@ __device__ void window_flush(const UpdateParams& p, const int tree, WindowLds& w
 // chosen one), the key and the level sizes (s_used) being in LDS.  Returns the node (-1: dropped for
 // lack of capacity); x (LDS) then holds the key in fp32, s_dist[l] the distance between the node's
 // ancestors at levels l - 1 and l, s_rad[l] the radius of the latter.
-template <typename T>
+template <typename T, int NT>
 __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, const int i,
                                                  const int position, int* s_used, const T* key, float* x,
                                                  float* red_f, int* red_i, float* s_dist, float* s_rad) {
@@ -656,13 +658,13 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
     const int D = p.dim, Dv = p.vdim, L = p.num_levels, bf = p.bf;
     int32_t* st = p.state + (size_t)tree * (HIRA_MAX_LEVELS + 2);
     const size_t base0 = (size_t)tree * p.cap[0];
-    for (int j = t; j < D; j += kUpdThreads) x[j] = load_elem<T>(key, j);
+    for (int j = t; j < D; j += NT) x[j] = load_elem<T>(key, j);
     __syncthreads();
     int top = 1;  // levels 1 .. top get a new node
     int parent = -1, pcount = 0;
     float pdist = 0.0f, prad = 0.0f;
     for (; top < L - 1; ++top) {  // uniform
-        parent = nearest_with_room<T>(p, tree, top + 1, 0, s_used[top + 1], x, red_f, red_i, nullptr, &pcount, &pdist,
+        parent = nearest_with_room<T, NT>(p, tree, top + 1, 0, s_used[top + 1], x, red_f, red_i, nullptr, &pcount, &pdist,
                                       &prad);
         if (parent >= 0) break;
     }
@@ -681,7 +683,7 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
         return -1;  // uniform
     }
     // the path above the new nodes: radii, and the distances between centres (a wave per level)
-    for (int l = top + 1 + wave; l < L; l += kUpdThreads / 64) {  // uniform in the wave
+    for (int l = top + 1 + wave; l < L; l += NT / 64) {  // uniform in the wave
         float d = sqrtf(pdist), rad_now = prad;
         if (l > top + 1) {
             const size_t node = ancestor_of((size_t)parent, l - top, bf);
@@ -707,7 +709,7 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
     id = idx;
     for (int l = top; l >= 1; --l) {
         const size_t bl = (size_t)tree * p.cap[l];
-        for (int j = t; j < D; j += kUpdThreads)
+        for (int j = t; j < D; j += NT)
             store_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, (size_t)id, j), x[j]);
         if (t == 0) {
             p.radii[l][bl + id] = 0.0f;
@@ -719,14 +721,14 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
     }
     const size_t slot = (size_t)id;
     const int node1 = (int)(id / bf);
-    for (int j = t; j < D; j += kUpdThreads)
+    for (int j = t; j < D; j += NT)
         store_elem<T>(p.keys, base0 * D + elem_index(p.key_layout, D, slot, j), x[j]);
     if (p.new_values && p.values)
-        for (int j = t; j < Dv; j += kUpdThreads)
+        for (int j = t; j < Dv; j += NT)
             store_elem<T>(p.values, (base0 + slot) * Dv + j, load_elem<T>(p.new_values, ((size_t)tree * p.m + i) * Dv + j));
     float worst = 0.0f;
     if (p.keys8 != nullptr) {
-        for (int j = t; j < D; j += kUpdThreads) {
+        for (int j = t; j < D; j += NT) {
             const float u = x[j] / p.kscale[(size_t)tree * D + j];
             const float r = fminf(fmaxf(rintf(u), -127.0f), 127.0f);
             worst = fmaxf(worst, fabsf(u - r));
@@ -737,8 +739,12 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
     }
     __syncthreads();
     if (t == 0) {
-        if (p.keys8 != nullptr)  // (the node holds no other key: its bound starts here)
-            p.keps[(size_t)tree * p.cap[1] + node1] = fmaxf(fmaxf(red_f[0], red_f[1]), fmaxf(red_f[2], red_f[3]));
+        if (p.keys8 != nullptr) {  // (the node holds no other key: its bound starts here)
+            float w = red_f[0];
+#pragma unroll
+            for (int i = 1; i < NT / 64; ++i) w = fmaxf(w, red_f[i]);
+            p.keps[(size_t)tree * p.cap[1] + node1] = w;
+        }
         p.perm[base0 + slot] = position;
         st[HIRA_MAX_LEVELS] = position + 1;
         if (parent >= 0) p.counts[top + 1][(size_t)tree * p.cap[top + 1] + parent] = pcount + 1;
@@ -757,13 +763,14 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
 // (also to cen) and its parent's count, the path above its radii, and it becomes the list of candidates; the key's row
 // goes the way of all others (its slot to *slot).  Returns the node, or -1 (uniform, and nothing is changed): no node
 // of the list takes the key, or the slot lies behind the capacity.
-template <typename T>
+template <typename T, int NT>
 __device__ __forceinline__ int open_listed(const UpdateParams& p, const int tree, int* s_used, int* slot, const T* key, const T* par,
                                            WindowLds& w, float* cen, float* s_dist, float* s_rad) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int D = p.dim, L = p.num_levels, bf = p.bf, n2 = w.n2;
     const size_t b1 = (size_t)tree * p.cap[1];
-    for (int e = wave; e < n2; e += kUpdThreads / 64) {  // uniform in the wave
+    const int known = w.n == 1 ? w.anc_id[2][0] : -1;  // the level-2 node whose path the list still has
+    for (int e = wave; e < n2; e += NT / 64) {  // uniform in the wave
         float ss = 0.0f;
         for (int j = lane; j < D; j += 64) {
             const float df = load_elem<T>(key, j) - load_elem<T>(par, (size_t)e * D + j);
@@ -791,12 +798,13 @@ __device__ __forceinline__ int open_listed(const UpdateParams& p, const int tree
     const int c = __ffsll((long long)who) - 1, parent = w.id2[c], pcount = w.cnt2[c];
     const long long idx = (long long)parent * bf + pcount;
     if (idx >= p.cap[1] || idx * bf >= p.cap[0]) return -1;
-    for (int j = t; j < D; j += kUpdThreads) {
+    for (int j = t; j < D; j += NT) {
         const float x = load_elem<T>(key, j);
         store_elem<T>(p.centers[1], b1 * D + elem_index(p.layout, D, (size_t)idx, j), x);
         cen[j] = x;
     }
-    for (int l = 2 + wave; l < L; l += kUpdThreads / 64) {  // the path above: a wave per level
+    const bool same_path = known == parent;
+    for (int l = same_path ? L : 2 + wave; l < L; l += NT / 64) {  // the path above: a wave per level
         const size_t node = ancestor_of((size_t)parent, l - 1, bf);
         const float rad_now = p.radii[l][(size_t)tree * p.cap[l] + node];
         float ss = best;
@@ -834,26 +842,30 @@ __device__ __forceinline__ int open_listed(const UpdateParams& p, const int tree
     if (t == 0) {  // (nobody reads this until the next barrier)
         w.cnt2[c] = pcount + 1;
         float r_child = 0.0f;
+        size_t node = (size_t)parent;
         for (int l = 2; l < L; ++l) {
-            const size_t node = ancestor_of((size_t)parent, l - 1, bf);
-            const float rn = fmaxf(s_rad[l], pad_up(s_dist[l] + r_child));
-            if (rn != s_rad[l]) p.radii[l][(size_t)tree * p.cap[l] + node] = rn;
+            const float have = same_path ? w.anc_rad[l][0] : s_rad[l];
+            const float step = l == 2 ? sqrtf(best) : (same_path ? w.anc_step[l][0] : s_dist[l]);
+            const float rn = fmaxf(have, pad_up(step + r_child));
+            if (rn != have) p.radii[l][(size_t)tree * p.cap[l] + node] = rn;
             r_child = rn;
             w.anc_id[l][0] = (int)node;
             w.anc_rep[l][0] = 0;
-            w.anc_step[l][0] = s_dist[l];
+            w.anc_step[l][0] = step;
             w.anc_rad[l][0] = rn;
+            node /= (size_t)bf;
         }
     }
     return (int)idx;
 }
 
 template <typename T, int COLS>
-__global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParams p) {
+__global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParams p) {
     // 2 D floats of the general way, kCandMax centres, the table of distances, kParents centres, a chunk of key rows
     extern __shared__ __attribute__((aligned(16))) float sm[];
-    __shared__ float red_f[4];
-    __shared__ int red_i[4];
+    constexpr int NT = kWinThreads;
+    __shared__ float red_f[NT / 64];
+    __shared__ int red_i[NT / 64];
     __shared__ float s_dist[HIRA_MAX_LEVELS], s_rad[HIRA_MAX_LEVELS];
     __shared__ WindowLds w;
     __shared__ int s_slot[kWinKeys];  // where the chunk's keys went (-1: placed the general way, or dropped)
@@ -880,31 +892,30 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
         const uint4* vsrc = vals == nullptr ? nullptr
                                             : reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(p.new_values) +
                                                                              ((size_t)tree * p.m + i0) * Dv);
-        constexpr int SU = 8;
+        typedef uint32_t vec4 __attribute__((ext_vector_type(4)));  // (an array of uint4 stays in memory here)
+        constexpr int SU = 2048 / NT;
         const int nc = nk * kc, nv = vals == nullptr ? 0 : nk * (Dv / EPL);
-        for (int e0 = t; e0 < nc + nv; e0 += SU * kUpdThreads) {
-            uint4 raw[SU];
+        for (int e0 = t; e0 < nc + nv; e0 += SU * NT) {
+            vec4 raw[SU];
 #pragma unroll
             for (int u = 0; u < SU; ++u) {
-                const int e = min(e0 + u * kUpdThreads, nc + nv - 1);
-                raw[u] = e < nc ? src[e] : vsrc[e - nc];
+                const int e = min(e0 + u * NT, nc + nv - 1);
+                raw[u] = *reinterpret_cast<const vec4*>(e < nc ? src + e : vsrc + (e - nc));
             }
 #pragma unroll
             for (int u = 0; u < SU; ++u) {
-                const int e = e0 + u * kUpdThreads;
-                if (e < nc) reinterpret_cast<uint4*>(rows)[e] = raw[u];
-                else if (e < nc + nv) vals[e - nc] = raw[u];
+                const int e = e0 + u * NT;
+                if (e < nc) reinterpret_cast<vec4*>(rows)[e] = raw[u];
+                else if (e < nc + nv) reinterpret_cast<vec4*>(vals)[e - nc] = raw[u];
             }
         }
     };
     int position = st[HIRA_MAX_LEVELS];  // of the next key (every thread carries it along)
     stage(0);
     if (t >= 1 && t < L) s_used[t] = st[t];
-    if (!window_candidates<T>(p, tree, w, cen, par)) {  // uniform: the tree's keys go the general way, all of them
-        for (int i = 0; i < p.m; ++i) update_one_key_called<T>(p, tree, i, sm, red_f, red_i, s_dist, s_rad);
-        return;
-    }
-    for (int i0 = 0; i0 < p.m;) {  // uniform
+    int i0 = 0;
+    bool general = !window_candidates<T, NT>(p, tree, w, cen, par);  // uniform: what is left goes the general way
+    while (i0 < p.m && !general) {  // uniform
         int nk = min(kWinKeys, p.m - i0);
         bool list_anew = false;  // behind this chunk
         const int position0 = position;
@@ -912,7 +923,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
             stage(i0);  // (behind the barrier that ends the chunk before: nobody needs its rows any more)
             __syncthreads();
         }
-        window_distances<T, COLS>(D, w, cen, rows, 0, nk, table);
+        window_distances<T, COLS, NT>(D, w, cen, rows, 0, nk, table);
         for (int k = 0; k < nk;) {  // uniform
             __syncthreads();
             if (wave == 0) {
@@ -982,14 +993,14 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
                 const T* key = rows + (size_t)k * D;
                 int node = -1;
                 if (!list_anew && L > 2 && w.n2 <= kParents<T>)  // uniform
-                    node = open_listed<T>(p, tree, s_used, &s_slot[k], key, par, w, cen, s_dist, s_rad);
+                    node = open_listed<T, NT>(p, tree, s_used, &s_slot[k], key, par, w, cen, s_dist, s_rad);
                 if (node >= 0) {
                     ++position;
                 } else {
                     // (with no room left in the list a node of level 2 is opened too, the only one there with room then)
                     bool none2 = w.n2 <= kParents<T>;
                     for (int e = 0; none2 && e < w.n2; ++e) none2 = w.cnt2[e] >= bf;
-                    node = open_node<T>(p, tree, i0 + k, position, s_used, key, sm, red_f, red_i, s_dist, s_rad);
+                    node = open_node<T, NT>(p, tree, i0 + k, position, s_used, key, sm, red_f, red_i, s_dist, s_rad);
                     if (node >= 0) ++position;
                     if (list_anew) {  // uniform
                         nk = k + 1;
@@ -1012,7 +1023,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
                         w.id2[0] = node / bf;
                         w.cnt2[0] = 1;
                     }
-                    for (int j = t; j < D; j += kUpdThreads) {  // (its centre is the key)
+                    for (int j = t; j < D; j += NT) {  // (its centre is the key)
                         cen[j] = sm[j];
                         par[j] = key[j];
                     }
@@ -1020,10 +1031,14 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
                 }
                 ++k;
                 // (of the keys that it has room for: those behind them find it full, whatever the distance)
-                window_distances<T, COLS>(D, w, cen, rows, k, min(nk, k + bf - 1), table);
+                window_distances<T, COLS, NT>(D, w, cen, rows, k, min(nk, k + bf - 1), table);
             }
         }
         // ---- the rows of the keys placed from the list, 16 bytes a thread -----------------------
+        if (p.keys8 != nullptr) {  // thread 0's bounds of nodes opened here, ahead of the maxima that raise them
+            if (wave == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        }
         float step[16];  // of a chunk of the 8-bit shadow: a thread's columns are the same for all its keys
         const int sc = D / 16, my_chunk = t % max(sc, 1);
         if (p.keys8 != nullptr)
@@ -1036,19 +1051,19 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
         const int vc = v_chunks ? Dv / EPL : 0, per = kc + vc;
         constexpr int RU = 4;  // chunks a thread has in flight
         const float inv_per = 1.0f / (float)per;  // (at most 64 x 128 chunks: the float quotient is exact)
-        for (int e0 = t; e0 < nk * per; e0 += RU * kUpdThreads) {
+        for (int e0 = t; e0 < nk * per; e0 += RU * NT) {
             uint4 raw[RU];
             T* dst[RU];
 #pragma unroll
             for (int u = 0; u < RU; ++u) {
-                const int e = min(e0 + u * kUpdThreads, nk * per - 1);
+                const int e = min(e0 + u * NT, nk * per - 1);
                 const int q = (int)(((float)e + 0.5f) * inv_per), c = e - q * per, slot = s_slot[q];
                 const size_t r = (size_t)tree * p.m + i0 + q;
                 const bool key = c < kc;
                 if (key) raw[u] = reinterpret_cast<const uint4*>(rows)[q * kc + c];
                 else if (vals != nullptr) raw[u] = vals[q * vc + c - kc];
                 else raw[u] = load_chunk<T>(p.new_values, r * Dv, c - kc);
-                dst[u] = slot < 0 || e0 + u * kUpdThreads >= nk * per
+                dst[u] = slot < 0 || e0 + u * NT >= nk * per
                              ? nullptr
                              : (key ? reinterpret_cast<T*>(p.keys) + base0 * D + elem_index(p.key_layout, D, (size_t)slot, c * EPL)
                                     : reinterpret_cast<T*>(p.values) + (base0 + slot) * Dv + (c - kc) * EPL);
@@ -1058,7 +1073,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
                 if (dst[u] != nullptr) *reinterpret_cast<uint4*>(dst[u]) = raw[u];
         }
         if (with_values && !v_chunks)  // (value rows that are not made of chunks)
-            for (int e = t; e < nk * Dv; e += kUpdThreads) {
+            for (int e = t; e < nk * Dv; e += NT) {
                 const int q = e / Dv, j = e - q * Dv;
                 if (s_slot[q] >= 0)
                     store_elem<T>(p.values, (base0 + s_slot[q]) * Dv + j,
@@ -1073,9 +1088,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
         if (p.keys8 != nullptr) {
             // the keys' 8-bit shadow with the tree's steps; a component beyond +-127 steps clips,
             // and the node's error bound then covers it.  Sixteen columns a thread, 4 or 8 threads a key.
-            if (wave == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (thread 0's bounds of nodes opened here, ahead of
-            __syncthreads();                                                // the maxima that raise them)
-            for (int e0 = 0; e0 < nk * sc; e0 += kUpdThreads) {  // uniform
+            for (int e0 = 0; e0 < nk * sc; e0 += NT) {  // uniform
                 const int q = min((e0 + t) / sc, nk - 1), slot = e0 + t < nk * sc ? s_slot[q] : -1;
                 float worst = 0.0f;
                 uint32_t out[4];
@@ -1103,14 +1116,15 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_window(const UpdateParam
         i0 += nk;
         if (list_anew) {  // uniform
             __syncthreads();
-            if (!window_candidates<T>(p, tree, w, cen, par)) {
-                if (t == 0) st[HIRA_MAX_LEVELS] = position;
-                __syncthreads();
-                for (; i0 < p.m; ++i0) update_one_key_called<T>(p, tree, i0, sm, red_f, red_i, s_dist, s_rad);
-                return;
-            }
+            general = !window_candidates<T, NT>(p, tree, w, cen, par);
         }
         if (i0 < p.m) __syncthreads();
+    }
+    if (general) {
+        if (t == 0) st[HIRA_MAX_LEVELS] = position;
+        __syncthreads();
+        for (; i0 < p.m; ++i0) update_one_key<T, NT>(p, tree, i0, sm, red_f, red_i, s_dist, s_rad);
+        return;
     }
     window_flush(p, tree, w);
     if (wave == 0) {
@@ -1206,7 +1220,7 @@ static int launch_update_window(const UpdateParams& p, int trees, size_t smem, h
             return fail(HIRA_ELAUNCH, "update: %zu bytes of LDS refused", kWinLds);
         __atomic_store_n(&asked[dev], 1, __ATOMIC_RELAXED);
     }
-    hipLaunchKernelGGL((k_update_window<T, COLS>), dim3(trees), dim3(kUpdThreads), smem, s, p);
+    hipLaunchKernelGGL((k_update_window<T, COLS>), dim3(trees), dim3(kWinThreads), smem, s, p);
     return HIRA_OK;
 }
 
