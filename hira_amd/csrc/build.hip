@@ -289,15 +289,17 @@ __device__ __forceinline__ void reset_round(const Buckets& b, int t) {  // (one 
 //    order of arrival.  (A row is CPR threads of 16 bytes, R = 256 / CPR rows at a time: 256 threads of a
 //    workgroup, or four times the 64 lanes of a wave.)  An empty centroid keeps its value.
 //    ct.tiles != NULL: the new centroid also goes into its operand tile.
-//    What bounds it is the gather of the rows and, to the end, the few largest buckets (1473 rows at
-//    8 x 131072 items, beside a mean of 32): 8 x 32768 rows of 256 bytes 71 -> 39 us, 8 x 131072
-//    200 -> 125 us.
+//    What bounds it is the latency of each bucket's chain (count, members, rows, sums): 6 us a workgroup of four
+//    small ones, 20 to 45 us a large one (up to 1473 rows at 8 x 131072 items, beside a mean of 32), so what
+//    counts is how many are on a compute unit: six workgroups (76 registers, 18 KiB), with fewer rows on their way in
+//    each.  8 x 32768 rows of 256 bytes 28 us, 8 x 131072 72 us (33 and 92 with four workgroups of 108 registers, twice the
+//    rows on their way and a quarter of the sums added up one load after the other).
 // ------------------------------------------------------------------------------------
-constexpr int kMeanMap = 4096;  // words of a bit map of item ids, for buckets beyond their places
+constexpr int kMeanMap = 2048;  // words of a bit map of item ids, for buckets beyond their places
 constexpr int kMeanMapBits = kMeanMap * 32;
 
 template <typename T>
-__global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
+__global__ __launch_bounds__(kBucketThreads, 6) void k_bucket_mean(
     const void* x, size_t x_tree_stride, int n_c, int K, int D, const Buckets bk,
     const int32_t* fill, int bf, float* cent, int Kt, const CentroidTiles ct, int KS, int large) {
     constexpr int EPL = Elem<T>::kPerChunk;
@@ -325,7 +327,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         if (lane == 0) reset_count(bk, t, k, K);
         float* piece = s_lds + wave * kPiece;
-        wave_mean<T, 2>(x, (size_t)t * x_tree_stride, [&](int e) { return s_ids[wave][e]; }, m, D, piece,
+        wave_mean<T, 1>(x, (size_t)t * x_tree_stride, [&](int e) { return s_ids[wave][e]; }, m, D, piece,
                         cent + ((size_t)t * K + k) * D);
         if (ct.tiles != nullptr) emit_centroid(piece, D, KS, Kt, t, k, usable(k), ct);
         return;
@@ -347,7 +349,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_mean(
         for (int e = 0; e < EPL; ++e) acc[e] = 0.0f;
         // rows [e0, e0 + n) in order, their ids at ids[0 .. n)
         auto add_rows = [&](const uint32_t* ids, int e0, int n) {
-            constexpr int U = 8;  // rows on their way at a time
+            constexpr int U = 4;  // rows on their way at a time
             if (r < R)
                 for (int e = e0 + (r - e0 % R + R) % R; e < e0 + n; e += U * R) {
                     uint4 raw[U];

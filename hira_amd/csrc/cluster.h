@@ -94,6 +94,40 @@ __device__ __forceinline__ void wave_mean(const void* x, size_t row0, Ids ids, i
     // the partial sums as one row of R * D numbers pass through LDS a quarter at a time; a lane
     // adds up its columns
     const int rows = min(R, m);
+    if (const int nc = D / 64; D % 64 == 0 && (nc == 1 || nc == 2 || nc == 4)) {  // uniform
+        // (64 lanes are whole columns: what a lane reads of a quarter is all on its way together.  Partial sums of
+        // rows that are none are zeros, and a sum that began as +0 stays what it is when a zero is added.)
+        float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int q = 0; q < EPL; ++q) piece[lane * EPL + q] = acc[i][q];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            float v[EPL];
+#pragma unroll
+            for (int q = 0; q < EPL; ++q) v[q] = piece[lane + 64 * q];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (nc == 1) {
+#pragma unroll
+                for (int q = 0; q < EPL; ++q) sum[0] += v[q];
+            } else if (nc == 2) {
+#pragma unroll
+                for (int q = 0; q < EPL; ++q) sum[q % 2] += v[q];
+            } else {
+#pragma unroll
+                for (int q = 0; q < EPL; ++q) sum[q % 4] += v[q];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (u < nc) {
+                const float v = sum[u] / (float)m;
+                cent_row[lane + 64 * u] = v;
+                piece[lane + 64 * u] = v;
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        return;
+    }
     float sum[8];
     int at[8];  // where the column's next partial sum lies
 #pragma unroll

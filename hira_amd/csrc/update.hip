@@ -389,9 +389,8 @@ __global__ __launch_bounds__(kTauThreads) void k_update_threshold(
 // of 128 bf16 columns: with 45 nodes to list, 39 us for 4 keys, 42 for 16, 49 for 32, 57 for 64 (48, 52, 60, 87); with one
 // node, full after 32 keys, and then another: 13 us for 4, 15 for 32, 21 for 64, 35 for 128, 68 for 255 (16, 21, 33, 59
 // and 119 when a key that opens a node looked for its parent in memory, the distances to the new node were taken of
-// keys that it has no room for, the 8-bit shadow was written a byte at a time, and the general way was a call: a
-// kernel that calls needs scratch memory, and its launch then took 4 us more).  256 threads instead of 512: 13, 15,
-// 21, 37, 76.
+// keys that it has no room for, the 8-bit shadow was written a byte at a time, and the general way was a call, around which
+// values lay in scratch memory: 4 us of any launch).  256 threads instead of 512: 13, 15, 21, 37, 76.
 // Radii wait until the list is given up: R = max over the keys of what each asks for, and that
 // grows with the distance, so the largest distance a candidate saw gives the radius that key by
 // key would have reached, to the last bit, and so up the levels.  A key that finds all candidates
