@@ -198,9 +198,10 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
         const int head = p.group_size > 0 ? hoff + g : p.tree_q_heads[hoff + g];
         const float* pm = p.part_m + (size_t)head * P;
         const float* pl = p.part_l + (size_t)head * P;
-        float mx = -INFINITY;
-        for (int i = lane; i < P; i += 64) mx = fmaxf(mx, ld(pm + i));
+        // (the first 64 partials' in one trip: up to there nothing is asked for twice)
         const float m0 = lane < P ? ld(pm + lane) : -INFINITY, l0 = lane < P ? ld(pl + lane) : 0.0f;
+        float mx = m0;
+        for (int i = lane + 64; i < P; i += 64) mx = fmaxf(mx, ld(pm + i));
         mx = wave_max(mx);
         float ls = 0.0f;
         int n = 0;
@@ -713,17 +714,26 @@ void search_kernel(const SearchParams p) {
     __syncthreads();
     for (int t = threadIdx.x; t < G * Dv; t += blockDim.x) {
         const int g = t / Dv, e = t % Dv;
-        float mall = -INFINITY;
-        for (int w = 0; w < nwaves; ++w)
-            mall = fmaxf(mall, smem[((size_t)w * GMAX + g) * (DVP + 2) + DVP]);
+        // (what every wave has, read at once: one wave's after the other's was a chain of 16 reads, and with the fold's
+        // maxima asked for twice 0.3 us of 15.9 at 4 trees x 5003 rows of 80 columns, 3 heads each)
+        float mw[WAVES], aw[WAVES], lw[WAVES], mall = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float* ws = smem + ((size_t)min(w, nwaves - 1) * GMAX + g) * (DVP + 2);
+            mw[w] = w < nwaves ? ws[DVP] : -INFINITY;
+            aw[w] = ws[e];  // (anything, where the wave has no selected key)
+            lw[w] = ws[DVP + 1];
+        }
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) mall = fmaxf(mall, mw[w]);
         float a = 0.0f, lsum = 0.0f;
-        for (int w = 0; w < nwaves; ++w) {
-            const float* ws = smem + ((size_t)w * GMAX + g) * (DVP + 2);
-            const float mw = ws[DVP];
-            if (mw == -INFINITY) continue;
-            const float f = exp2f(mw - mall);
-            a += ws[e] * f;
-            lsum += ws[DVP + 1] * f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float f = exp2f(mw[w] - mall);
+            if (mw[w] != -INFINITY) {
+                a += aw[w] * f;
+                lsum += lw[w] * f;
+            }
         }
         const size_t slot = (size_t)head_of(g) * p.num_parts + blockIdx.x;
         // device-scope stores: written through, so that the workgroup that folds the partials
