@@ -303,13 +303,21 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
             s.count[i] = 0;
         }
         if (tid == 0) s.n_big = 0;
-        for (int k = wave; k < K; k += kSmallWaves) {
+        constexpr int kMine = (kSmallCentroids + kSmallWaves - 1) / kSmallWaves, NJ = D / 64;
+        float first[kMine][NJ];  // (a wave's centroids, asked for together)
+#pragma unroll
+        for (int i = 0; i < kMine; ++i) {
+            const int k = min(wave + i * kSmallWaves, K - 1);
             const size_t src = (row0 + (size_t)first_centroid(p.seed + 7919ull * (uint64_t)l, t, k, max(n_c, 1), K_t)) * D;
-            for (int j = lane; j < D; j += 64) {
-                const float v = load_elem<bf16_t>(x, src + j);
-                cent[(size_t)k * D + j] = v;
-                piece[j] = v;
-            }
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) first[i][j] = load_elem<bf16_t>(x, src + j * 64 + lane);
+        }
+#pragma unroll
+        for (int i = 0; i < kMine; ++i) {
+            const int k = wave + i * kSmallWaves;
+            if (k >= K) break;  // uniform
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) cent[(size_t)k * D + j * 64 + lane] = piece[j * 64 + lane] = first[i][j];
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             small_emit<KS>(s, piece, k);
             if (lane == 0 && k >= K_t) s.n2[k] = INFINITY;
