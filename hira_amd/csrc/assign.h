@@ -136,24 +136,22 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
     return (uint32_t)f32_to_bf16_bits(a) | ((uint32_t)f32_to_bf16_bits(b) << 16);
 }
 
-// Centroid k of tree t, D fp32 numbers at c (LDS or memory), into its tile; called by the 64
-// lanes of one wave.
-__device__ __forceinline__ void emit_centroid(const float* c, int D, int KS, int Kt, int t, int k,
-                                              bool usable, const CentroidTiles& ct) {
-    const int j = threadIdx.x & 63;
+// Columns 8 j .. 8 j + 7 of centroid k of tree t (zeros behind the last one) into its tile; `lanes` (a power of two, at
+// least 4 KS) consecutive lanes hold a centroid.
+__device__ __forceinline__ void emit_columns(const float (&v)[8], int j, int lanes, bool have, int KS, int Kt, int t, int k,
+                                             bool usable, const CentroidTiles& ct) {
     float ss = 0.0f, ls = 0.0f;
-    if (j < KS * 4) {
+    if (have && j < KS * 4) {
         const int s = j >> 2, kb = j & 3, i = k & 15;
         uint4* out = ct.tiles + ((size_t)t * Kt + (k >> 4)) * (size_t)(2 * KS * 64);
         float hi[8], lo[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float v = j * 8 + e < D ? c[j * 8 + e] : 0.0f;
-            hi[e] = bf16_bits_to_f32(f32_to_bf16_bits(v));
-            lo[e] = bf16_bits_to_f32(f32_to_bf16_bits(v - hi[e]));
+            hi[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e]));
+            lo[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e] - hi[e]));
             const float w = hi[e] + lo[e];
             ss += w * w;
-            ls += (v - hi[e]) * (v - hi[e]);
+            ls += (v[e] - hi[e]) * (v[e] - hi[e]);
         }
         out[s * 64 + kb * 16 + i] = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]),
                                                pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
@@ -161,16 +159,26 @@ __device__ __forceinline__ void emit_centroid(const float* c, int D, int KS, int
             make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]),
                        pack_bf16(lo[6], lo[7]));
     }
-#pragma unroll
-    for (int off = 1; off < 32; off <<= 1) {
+    for (int off = 1; off < lanes; off <<= 1) {
         ss += __shfl_xor(ss, off, 64);
         ls += __shfl_xor(ls, off, 64);
     }
-    if (j == 0) {
+    if (have && j == 0) {
         ct.n2[(size_t)t * Kt * 16 + k] = usable ? ss : INFINITY;
         // (1e-5 of ||c|| per 32 columns: what the roundings of two sums of products can be worth)
         ct.lo[(size_t)t * Kt * 16 + k] = sqrtf(ls) * 1.0001f + (float)KS * 1e-5f * sqrtf(ss);
     }
+}
+
+// Centroid k of tree t, D fp32 numbers at c (LDS or memory), into its tile; called by the 64
+// lanes of one wave.
+__device__ __forceinline__ void emit_centroid(const float* c, int D, int KS, int Kt, int t, int k,
+                                              bool usable, const CentroidTiles& ct) {
+    const int j = threadIdx.x & 63;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = j < KS * 4 && j * 8 + e < D ? c[j * 8 + e] : 0.0f;
+    emit_columns(v, j, 32, true, KS, Kt, t, k, usable, ct);
 }
 
 // What an assignment launch works on.

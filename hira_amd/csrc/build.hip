@@ -88,30 +88,37 @@ __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_
 //    (n_live != NULL: tree t holds n_live[t] <= n_c items, the first ones of its rows)
 //    ct.tiles != NULL: the centroid also goes into its operand tile (fill: the centroids that
 //    count as full from the start take no items)
+//    `lanes` (a power of two) hold a centroid, eight columns each, so that a wave takes several: bound by its
+//    instructions (the random number, the split into halves), 8 x 4096 centroids of 128 columns 13.5 us, 27 with a
+//    centroid a wave, most of whose lanes had no columns.
 template <typename T>
 __global__ __launch_bounds__(kNodeThreads) void k_init_centroids(const void* x, int n_c, size_t x_tree_stride,
                                                        int K, int D, uint64_t seed, float* cent,
                                                        const int32_t* n_live, int bf, int Kt,
-                                                       const int32_t* fill, CentroidTiles ct, int KS) {
-    __shared__ float s_all[kNodeThreads / 64][256];
-    const int k = node_of_wave(), t = blockIdx.x, lane = threadIdx.x & 63;
-    float* s_c = s_all[threadIdx.x >> 6];
-    if (k >= K) return;  // (the whole wave)
+                                                       const int32_t* fill, CentroidTiles ct, int KS, int lanes) {
+    constexpr int EPL = Elem<T>::kPerChunk, CH = 8 / EPL;
+    const int t = blockIdx.x, lane = threadIdx.x & 63, j = lane % lanes;
+    const int k = node_of_wave() * (64 / lanes) + lane / lanes, own = min(k, K - 1);
     const int n_t = n_live ? max(min(n_live[t], n_c), 1) : n_c;
     // (a tree with fewer items uses the first K_t = ceil(n_t / bf) centroids only)
     const int K_t = n_live ? min(max((n_t + bf - 1) / bf, 1), K) : K;
-    const long long idx = first_centroid(seed, t, k, n_t, K_t);
+    const long long idx = first_centroid(seed, t, own, n_t, K_t);
     const size_t src = ((size_t)t * x_tree_stride + (size_t)idx) * D;
-    float* dst = cent + ((size_t)t * K + k) * D;
-    for (int j = lane; j < D; j += 64) {
-        const float v = load_elem<T>(x, src + j);
-        dst[j] = v;
-        if (ct.tiles != nullptr) s_c[j] = v;  // (tiles are for D <= 256)
+    float v[8];
+#pragma unroll
+    for (int h = 0; h < CH; ++h) {
+        uint4 raw = make_uint4(0, 0, 0, 0);
+        if ((j * CH + h) * EPL < D) raw = load_chunk<T>(x, src, j * CH + h);
+        float f[EPL];
+        unpack<T>(raw, f);
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) v[h * EPL + e] = f[e];
     }
-    if (ct.tiles != nullptr) {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        emit_centroid(s_c, D, KS, Kt, t, k, fill[(size_t)t * K + k] < bf, ct);
-    }
+    float* dst = cent + ((size_t)t * K + own) * D + j * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)  // (rows are whole fours)
+        if (k < K && j * 8 + h * 4 < D) *reinterpret_cast<float4*>(dst + h * 4) = make_float4(v[h * 4], v[h * 4 + 1], v[h * 4 + 2], v[h * 4 + 3]);
+    if (ct.tiles != nullptr) emit_columns(v, j, lanes, k < K, KS, Kt, t, own, fill[(size_t)t * K + own] < bf, ct);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1049,9 +1056,11 @@ static int cluster_levels(const HiraTree* t, const void* keys_in, int n, const i
         const bool ragged = n_live != nullptr && l == 1;
         hipLaunchKernelGGL(k_level_init, tree_grid(min(ceil_div(Kl * bf, 256), 2048), NT), dim3(256), 0, s, n_c, Kl, bf,
                            D, Kt, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters, l == 1 ? w.absmax : nullptr, tiles, KS);
-        hipLaunchKernelGGL((k_init_centroids<T>), node_grid(Kl, NT), dim3(kNodeThreads), 0, s, x, n_c, xs, Kl, D,
+        int lanes = 1;
+        while (lanes * 8 < D || (on_mfma && lanes < KS * 4)) lanes <<= 1;
+        hipLaunchKernelGGL((k_init_centroids<T>), node_grid(ceil_div(Kl, 64 / lanes), NT), dim3(kNodeThreads), 0, s, x, n_c, xs, Kl, D,
                            seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, bf,
-                           Kt, w.fill, tiles, KS);
+                           Kt, w.fill, tiles, KS, lanes);
         // a round: the assignment (which also puts the items into buckets), then what the round does
         // with every bucket.  A Lloyd round asks for no distances.
         auto buckets = [&]() {
