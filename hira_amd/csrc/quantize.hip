@@ -67,7 +67,13 @@ __global__ void k_step_from_absmax(float* kscale, const float* absmax, int copie
     if (i >= n) return;
     const float* at = absmax + i / D * copies * D + i % D;
     float m = 0.0f;
-    for (int c = 0; c < copies; ++c) m = fmaxf(m, at[(size_t)c * D]);
+    for (int c0 = 0; c0 < copies; c0 += 16) {  // (16 on their way: one after the other, 32 copies were 10 us)
+        float v[16];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) v[c] = at[(size_t)min(c0 + c, copies - 1) * D];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) m = fmaxf(m, v[c]);
+    }
     kscale[i] = fmaxf(m / 127.0f, kMinStep);
 }
 
