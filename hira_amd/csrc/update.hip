@@ -52,6 +52,25 @@ struct UpdateParams {
     int32_t stage_values;  // windows: the values' rows have room in LDS too
 };
 
+// The kernels' arguments lie in six 64-byte lines of memory: all of them asked for at once (touch_kernel_arguments
+// of search.h, for its kernels' nine): a window of 64 keys 21 -> 19.7 us, a single key 7.6 -> 7.2.
+__device__ __forceinline__ void touch_update_arguments() {
+    static_assert(sizeof(UpdateParams) > 5 * 64 + 4 && sizeof(UpdateParams) <= 6 * 64, "one load per 64-byte line of the arguments");
+    auto ka = __builtin_amdgcn_kernarg_segment_ptr();
+    uint32_t d0, d1, d2, d3, d4, d5;
+    asm volatile(
+        "s_load_dword %0, %6, 0x0\n\t"
+        "s_load_dword %1, %6, 0x40\n\t"
+        "s_load_dword %2, %6, 0x80\n\t"
+        "s_load_dword %3, %6, 0xc0\n\t"
+        "s_load_dword %4, %6, 0x100\n\t"
+        "s_load_dword %5, %6, 0x140\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&s"(d0), "=&s"(d1), "=&s"(d2), "=&s"(d3), "=&s"(d4), "=&s"(d5)
+        : "s"(ka)
+        : "memory");
+}
+
 // a bound must survive the fp32 rounding of the sums that produced it
 __device__ __forceinline__ float pad_up(float r) { return r > 0.0f ? r * (1.0f + 4.0f * 1.1920929e-7f) + 1e-30f : r; }
 
@@ -341,6 +360,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update(const UpdateParams p) {
     __shared__ float red_f[4];
     __shared__ int red_i[4];
     __shared__ float s_dist[HIRA_MAX_LEVELS], s_rad[HIRA_MAX_LEVELS];
+    touch_update_arguments();
     for (int i = 0; i < p.m; ++i)
         update_one_key<T, kUpdThreads>(p, (int)blockIdx.x, i, sm, red_f, red_i, s_dist, s_rad);
 }
@@ -387,7 +407,7 @@ __global__ __launch_bounds__(kTauThreads) void k_update_threshold(
 //   rows       of the 64 keys to their slots, 16 bytes a thread.
 // What bounds it is latency in one workgroup a tree (its waves wait 69 % of their cycles).  A launch, 8 trees
 // of 128 bf16 columns: with 45 nodes to list, 39 us for 4 keys, 42 for 16, 49 for 32, 57 for 64 (48, 52, 60, 87); with one
-// node, full after 32 keys, and then another: 13 us for 4, 15 for 32, 21 for 64, 35 for 128, 68 for 255 (16, 21, 33, 59
+// node, full after 32 keys, and then another: 12 us for 4, 14 for 32, 20 for 64, 34 for 128, 66 for 255 (16, 21, 33, 59
 // and 119 when a key that opens a node looked for its parent in memory, the distances to the new node were taken of
 // keys that it has no room for, the 8-bit shadow was written a byte at a time, and the general way was a call, around which
 // values lay in scratch memory: 4 us of any launch).  256 threads instead of 512: 13, 15, 21, 37, 76.
@@ -871,6 +891,7 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
     __shared__ int s_done;            // keys of the chunk dealt with so far
     __shared__ bool s_room;           // a listed node has room
     __shared__ int s_used[HIRA_MAX_LEVELS];  // slots in use per level
+    touch_update_arguments();
     constexpr int EPL = Elem<T>::kPerChunk;
     const int tree = blockIdx.x;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
