@@ -495,3 +495,69 @@ def test_attention_over_given_lists(h_kv, h_q, n, d, bf, nl, dtype, gpu_device):
     assert rel_err(got2[1:], ref2[1:]) <= tol
     with pytest.raises(ValueError):
         se.sparse_attention(idx, sco[:, :-1], cnt, c["idx"], scaling=sc)
+
+
+SMALL_MFMA_CASES = [
+    # trees, heads a tree, keys, width, fan-out, levels, queued rows: tiles of 16 nodes -> partials a head
+    (2, 4, 200, 128, 32, 3, 0),      # one tile
+    (2, 3, 500, 64, 16, 2, 0),       # two
+    (1, 8, 1537, 128, 32, 2, 5),     # four, and the queue's
+    (3, 4, 2048, 128, 32, 2, 0),     # four, all nodes full
+    (2, 16, 2500, 128, 32, 2, 0),    # five, sixteen heads
+    (2, 4, 1990, 256, 16, 2, 0),     # eight
+    (2, 4, 2050, 128, 16, 2, 0),     # nine
+    (1, 5, 3900, 64, 16, 3, 1),      # sixteen, and the queue's
+    (1, 4, 4000, 128, 16, 2, 0),     # sixteen
+    (1, 17, 2000, 128, 64, 2, 0),    # two passes of heads, nodes of four tiles
+]
+
+
+@pytest.mark.parametrize("t,g,n,d,bf,nl,m", SMALL_MFMA_CASES)
+def test_small_trees_on_the_matrix_cores(t, g, n, d, bf, nl, m, gpu_device):
+    """A few workgroups a tree: attention against softmax over the selected keys in float64 and against
+    the fold of a second launch, with a head that selects nothing and one that selects a single key
+    (partials without a key), the workspace full of NaN before the first call."""
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+    from hira_amd.searcher.hip import _COUNTERS
+
+    print(f"case {t} {g} {n} {d} {bf} {nl} {m}", flush=True)
+    gen = torch.Generator().manual_seed(n + g)
+    K = torch.randn(1, t, n, d, generator=gen).bfloat16()
+    V = torch.randn(1, t, n, d, generator=gen).bfloat16()
+    q = torch.randn(t * g, d, generator=gen).bfloat16()
+    s = torch.matmul(q.reshape(t, g, d).double(), K[0].double().transpose(1, 2).contiguous())  # (t, g, n)
+    keep = max(2, n // 60)
+    top = s.topk(keep + 1, dim=-1).values
+    tau = (0.5 * (top[..., keep - 1] + top[..., keep])).float()
+    tau[0, 0] = 1e9
+    tau[-1, -1] = (0.5 * (top[-1, -1, 0] + top[-1, -1, 1])).float()
+    idx = HIPIndexer(nl, 1, bf).build(K.cuda(), V.cuda())
+    assert idx.tiled
+    sel = s >= tau.double()[..., None]
+    z, vals = s * d ** -0.5, V[0].double()
+    qk = qv = None
+    if m:
+        qk, qv = torch.randn(t, m, d, generator=gen).bfloat16(), torch.randn(t, m, d, generator=gen).bfloat16()
+        zq = torch.matmul(q.reshape(t, g, d).double(), qk.double().transpose(1, 2).contiguous()) * d ** -0.5
+        z, sel = torch.cat([z, zq], -1), torch.cat([sel, torch.ones(t, g, m, dtype=torch.bool)], -1)
+        vals = torch.cat([vals, qv.double()], 1)
+        qk, qv = qk.cuda(), qv.cuda()
+    w = torch.softmax(z.masked_fill(~sel, float("-inf")), -1).nan_to_num(0.0)
+    ref = torch.matmul(w, vals).reshape(t * g, d)
+    args = (q.cuda(), tau.reshape(-1).cuda(), idx)
+    kw = dict(scaling=torch.full((t * g,), d ** -0.5, device="cuda"), queue_keys=qk, queue_values=qv)
+    fused, apart = HIPSearcher(kernel=2), HIPSearcher(kernel=2, separate_merge=True)
+    for se in (fused, apart):
+        se.search_attention(*args, **kw)
+        se._workspace[_COUNTERS:] = 0xFF
+    a, b = fused.search_attention(*args, **kw).cpu(), apart.search_attention(*args, **kw).cpu()
+    if not m:
+        assert not a[0].any()
+    den = ref.abs().amax(1, keepdim=True).clamp_min(1e-30)
+    # (scores and sums in fp32 over bf16 rows; the folds differ in the order of their sums)
+    assert float(((a.double() - ref).abs() / den).max()) <= 2e-5
+    assert float(((a - b).abs() / den).max()) <= 2e-6
+    stats = torch.zeros((t, 11), dtype=torch.int64, device="cuda")
+    fused.search_attention(*args, **kw, stats=stats)
+    assert int(stats[:, 8].sum()) == int(sel[..., :n].any(dim=1).sum())
