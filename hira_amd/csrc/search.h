@@ -78,6 +78,7 @@ struct SearchPlan {
     int nodes_per_wave;
     int num_nodes, num_queue_blocks;
     int tree_blocks, queue_blocks, head_chunks;
+    bool ahead;       // MFMA kernel: key tiles are asked for together with the gates' operands
     size_t smem;
 };
 

@@ -88,6 +88,7 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
             HIRA_CHECK_ARG(t->cap[l] % 16 == 0, "tiled layout: cap[%d]=%d not a multiple of 16",
                            l, t->cap[l]);
     }
+    plan->ahead = false;
     plan->num_queue_blocks = 0;
     if (queue && queue->keys && queue->len > 0) {
         HIRA_CHECK_ARG(queue->len <= queue->cap, "queue len %d > cap %d", queue->len,
@@ -154,6 +155,13 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
             if (blocks > max_parts) blocks = max_parts;
             if (blocks > plan->tree_blocks) plan->tree_blocks = (int)blocks;
         }
+        // key tiles asked for ahead of the gates: for workgroups of one tile, and where reading the keys of
+        // nodes that the gates would have pruned costs less than the trip.  8 trees x 4 heads, keys of random
+        // rows / of boosted channels, whose balls prune half: 4 MiB of keys 11.3 -> 9.9 / 12.2 -> 10.9 us
+        // (indexes taking turns), 16 MiB 12.9 -> 11.4 / 13.0 -> 11.7, 24 MiB 14.5 -> 12.9 / 14.0 -> 12.5;
+        // 32 MiB in 32 trees 13.8 -> 12.7 / 12.8 -> 13.1
+        plan->ahead = plan->threads == kMfmaThreads && plan->nodes_per_wave == 1 &&
+                      (size_t)t->num_trees * (size_t)t->size[0] * (size_t)t->dim * 2 <= ((size_t)28 << 20);
         plan->queue_blocks = plan->num_queue_blocks > 0 ? 1 : 0;  // one workgroup takes the whole queue
         plan->smem = 0;
         // every workgroup that walks the tree must own at least one tile: one without a tile

@@ -22,6 +22,8 @@
 //          against the lane's own threshold).  A tile with a selected row writes the scaled
 //          scores of its rows to the wave's stretch of a table in LDS (-inf: not selected) and
 //          appends the selected rows to the wave's row list.
+//          (A small launch, whose workgroups own one tile: the waves ask for the key tiles of their two
+//          nodes each beside the gates' operands, see AHEAD below.)
 //   gather the wave raises its running maximum per head, turns the listed scores into weights
 //          2^(z - m) with lane = (row, head), and fetches the value rows of its list, kVBatch
 //          in flight, each row once however many heads selected it:
@@ -242,6 +244,9 @@ __device__ __forceinline__ void gate_issue(const SearchParams& p, int tree, int 
     }
 }
 
+// nodes of a wave of the instantiations that ask for key tiles ahead of the gates: a tile's 16 over 8 waves
+constexpr int kAheadNodes = 16 / kMfmaWaves;
+
 // OUT: the launch also wants dense scores or selection lists (kept out of the attention-only
 // instantiation, whose registers are all spoken for).
 // Q8: the index keeps an 8-bit shadow of its keys (HIRA_TILE16_Q8).  The scan then reads the
@@ -254,11 +259,15 @@ __device__ __forceinline__ void gate_issue(const SearchParams& p, int tree, int 
 // around it, in which the compiler's waits count the loads still in flight and a node's products
 // start when ITS tiles have arrived; at the head of a loop they fall back to waiting for
 // everything asked for so far.
-template <int KS, int MT, int GS, bool OUT, bool Q8, int POL, int HV, bool ONE>
+// AHEAD: (small launches) a workgroup owns one tile, and its waves ask for the key tiles of their two
+// nodes each together with the gates' operands, whether the nodes survive or not: a trip to memory less,
+// and no list of survivors.
+template <int KS, int MT, int GS, bool OUT, bool Q8, int POL, int HV, bool ONE, bool AHEAD = false>
 __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const SearchParams p) {
     using S = MfmaShape<KS, MT, GS, Q8>;
     constexpr int D = S::D;
-    constexpr int NB = S::NB;
+    constexpr int NB = AHEAD ? kAheadNodes : S::NB;
+    static_assert(!AHEAD || (ONE && !OUT && !Q8 && HV == 1 && NB <= S::NB), "");
     constexpr int KA = S::KA;          // 16-byte chunks per lane of a scanned tile
     constexpr int KS8 = Q8 ? KS / 2 : 1;
     constexpr int VPL = KS / 2;        // value elements per lane: Dv = D = 64 * VPL
@@ -429,12 +438,27 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         float tau = p.tau[qh];
         float sc = p.scaling[qh];
         GateLoads<KS> gl;
+        uint4 a[NB][MT][KA];  // key tiles of the nodes that a wave takes in a round
         if (tl_mine < ntile) {
 #pragma unroll
             for (int s = 0; s < KS; ++s)
                 qraw[s] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.q) +
                                                           (size_t)qh * D + s * 32 + kb * 8);
             gate_issue<KS, Q8>(p, tree, tile_of(tl_mine), lane, kb, gl);
+        }
+        if constexpr (AHEAD) {
+            // (slots beyond the capacity, under nodes that pad the tile or a last node of 48: zeros, no memory
+            // access)
+            const size_t r0 = (size_t)tree * p.cap[0];
+            const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(
+                reinterpret_cast<const uint16_t*>(p.keys) + r0 * (size_t)D, (size_t)p.cap[0] * D * 2);
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+#pragma unroll
+                for (int tt = 0; tt < MT; ++tt)
+                    load_tile_buf<KA, POL != 0>(
+                        rsrc, (unsigned)lane * 16u,
+                        ((unsigned)(node_of(u * kMfmaWaves + wave) * bf) / 16u + tt) * (unsigned)(KA * 1024), a[u][tt]);
         }
         __builtin_amdgcn_sched_barrier(0);  // (nothing that uses a load moves above this line)
         tline.stamp(kTlGateIssued);
@@ -641,8 +665,8 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         tline.stamp(kTlBarrier);
 
         // ---- the surviving nodes of my tiles in order, dealt round-robin to the waves ----------
-        int rounds, alive = 0;
-        {
+        int rounds = 1, alive = 0;
+        if constexpr (!AHEAD) {
             const int n_info = ntile * 16;
             const unsigned long long lt = (1ull << lane) - 1ull;
 #pragma unroll
@@ -699,7 +723,6 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         int nx_node[NB], nx_cnt[NB], nx_half[NB];
         uint32_t nx_mask[NB];
         float nx_eps[Q8 ? NB : 1];
-        uint4 a[NB][MT][KA];
         auto fetch = [&](int round, int u_only) {  // u_only < 0: all NB nodes of the round
             // my nodes of the round: entries (round*NB + u) * nw + wave of the survivors
             uint32_t ent[NB];
@@ -738,7 +761,19 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                 }
             }
         };
-        if (rounds > 0) fetch(0, -1);
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                const int n = u * kMfmaWaves + wave;
+                const uint32_t info = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_ninfo[n]);
+                nx_node[u] = n;
+                nx_half[u] = 0;
+                nx_mask[u] = info & 0xFFFFu;
+                nx_cnt[u] = nx_mask[u] != 0u ? (int)(info >> 16) : 0;
+            }
+        } else {
+            if (rounds > 0) fetch(0, -1);
+        }
         tline.stamp(kTlFetched);
 
         constexpr int KB0 = KS <= 4 ? 2 : 1;      // batches of 16 key rows asked for ahead
@@ -879,6 +914,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                         nsel += __popc(rowmask);
                     }
                 } else {
+                if (AHEAD && cnt[u] == 0) continue;  // uniform
                 f32x4_t sco_u[MT];
 #pragma unroll
                 for (int tt = 0; tt < MT; ++tt)  // (a tile that is not there came as zeros)
@@ -1536,12 +1572,21 @@ void launch_mfma_one(const SearchPlan& plan, const SearchParams& p, dim3 grid, h
     const bool one = plan.nodes_per_wave * 16 * HV <= (plan.threads / 64) * MfmaShape<KS, MT, GS, Q8>::NB;
     if (out) {
         hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, true, Q8, POL, HV, false>), grid, block, 0, s, p);
-    } else if constexpr (!Q8) {
-        if (one) hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, Q8, POL, HV, true>), grid, block, 0, s, p);
-        else hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, Q8, POL, HV, false>), grid, block, 0, s, p);
-    } else {
-        hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, Q8, POL, HV, false>), grid, block, 0, s, p);
+        return;
     }
+    if constexpr (!Q8 && POL == 0 && HV == 1 && KS <= 4 && MfmaShape<KS, MT, GS>::NB >= kAheadNodes) {
+        if (plan.ahead) {
+            hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, false, 0, 1, true, true>), grid, block, 0, s, p);
+            return;
+        }
+    }
+    if constexpr (!Q8) {
+        if (one) {
+            hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, Q8, POL, HV, true>), grid, block, 0, s, p);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, Q8, POL, HV, false>), grid, block, 0, s, p);
 }
 
 template <int KS, int MT, bool Q8, int POL, int HV = 1>

@@ -509,6 +509,8 @@ SMALL_MFMA_CASES = [
     (1, 5, 3900, 64, 16, 3, 1),      # sixteen, and the queue's
     (1, 4, 4000, 128, 16, 2, 0),     # sixteen
     (1, 17, 2000, 128, 64, 2, 0),    # two passes of heads, nodes of four tiles
+    (2, 4, 3000, 128, 48, 2, 0),     # nodes of three tiles
+    (1, 4, 777, 64, 48, 3, 0),
 ]
 
 
