@@ -499,7 +499,10 @@ def test_attention_over_given_lists(h_kv, h_q, n, d, bf, nl, dtype, gpu_device):
 
 SMALL_MFMA_CASES = [
     # trees, heads a tree, keys, width, fan-out, levels, queued rows: tiles of 16 nodes -> partials a head
-    (2, 4, 200, 128, 32, 3, 0),      # one tile
+    (2, 4, 500, 128, 32, 2, 0),      # one tile: the tree's only workgroup
+    (3, 11, 130, 64, 16, 2, 0),
+    (2, 4, 500, 128, 32, 2, 7),      # one, and the queue's
+    (2, 4, 200, 128, 32, 3, 0),      # two, one without a node in use
     (2, 3, 500, 64, 16, 2, 0),       # two
     (1, 8, 1537, 128, 32, 2, 5),     # four, and the queue's
     (3, 4, 2048, 128, 32, 2, 0),     # four, all nodes full
