@@ -335,19 +335,6 @@ void search_kernel(const SearchParams p) {
     const int node_first = blk * nwaves * p.nodes_per_wave;
     const int node_last = min(node_first + nwaves * p.nodes_per_wave, n_nodes);
 
-    // ---- queries of the group: this lane's chunk of each (asked for here, first used at the gates) ----
-    uint4 qraw[GMAX];
-    float tau[GMAX];
-#pragma unroll
-    for (int g = 0; g < GMAX; ++g) {
-        qraw[g] = make_uint4(0, 0, 0, 0);
-        tau[g] = INFINITY;
-        if (g < G) {
-            const int h = head_of(g);
-            if (chunk_ok) qraw[g] = load_chunk<T>(p.q, (size_t)h * D, ch);
-            tau[g] = p.tau[h];
-        }
-    }
     // threshold, scale and head of the values whose sums this lane ends up with
     int vfirst = 0;  // vec_value_of(ch)
     {
@@ -360,14 +347,33 @@ void search_kernel(const SearchParams p) {
             }
     }
     const int my_u = vfirst / GMAX, my_g = vfirst % GMAX;  // row of the block, first head
-    float my_tau[KEPT], my_sc[KEPT];
-    int my_h[KEPT];
+    // ---- queries of the group: this lane's chunk of each (asked for here, first used at the gates).
+    // Heads first, then straight-line loads, those of a head or a chunk that is not there the last one's
+    // again, dropped where they are used: with a condition around each head's (its number, `g < G`) the
+    // waits at the joins made them a trip to memory after the other ahead of the gates (4 trees x 5003 rows of 80 fp32, three heads each:
+    // 15.6 -> 15.25 us, seven heads of 64 16.95 -> 16.55) ----
+    int hd[GMAX], my_h[KEPT];
+#pragma unroll
+    for (int g = 0; g < GMAX; ++g) hd[g] = hoff + min(g, G - 1);
+#pragma unroll
+    for (int i = 0; i < KEPT; ++i) my_h[i] = hoff + min(my_g + i % GMAX, G - 1);
+    if (!by_group) {  // uniform
+#pragma unroll
+        for (int g = 0; g < GMAX; ++g) hd[g] = p.tree_q_heads[hd[g]];
+#pragma unroll
+        for (int i = 0; i < KEPT; ++i) my_h[i] = p.tree_q_heads[my_h[i]];
+    }
+    uint4 qraw[GMAX];
+    float tau[GMAX], my_tau[KEPT], my_sc[KEPT];
+#pragma unroll
+    for (int g = 0; g < GMAX; ++g) {
+        qraw[g] = load_chunk<T>(p.q, (size_t)hd[g] * D, chunk_ok ? ch : 0);
+        tau[g] = p.tau[hd[g]];
+    }
 #pragma unroll
     for (int i = 0; i < KEPT; ++i) {
-        const int g = my_g + i % GMAX;
-        my_h[i] = g < G ? head_of(g) : 0;
-        my_tau[i] = g < G ? p.tau[my_h[i]] : INFINITY;
-        my_sc[i] = g < G ? p.scaling[my_h[i]] : 0.0f;
+        my_tau[i] = p.tau[my_h[i]];
+        my_sc[i] = p.scaling[my_h[i]];
     }
 
     const void* kbase = is_queue ? p.queue_keys : p.keys;
@@ -424,7 +430,7 @@ void search_kernel(const SearchParams p) {
             float qn[GMAX];
 #pragma unroll
             for (int g = 0; g < GMAX; ++g) {
-                unpack<T>(qraw[g], qf[g]);
+                unpack<T>(chunk_ok ? qraw[g] : make_uint4(0, 0, 0, 0), qf[g]);
                 float ss = 0.0f;
 #pragma unroll
                 for (int e = 0; e < EPL; ++e) ss += qf[g][e] * qf[g][e];
@@ -473,7 +479,7 @@ void search_kernel(const SearchParams p) {
             }
         } else {
 #pragma unroll
-            for (int g = 0; g < GMAX; ++g) unpack<T>(qraw[g], qf[g]);
+            for (int g = 0; g < GMAX; ++g) unpack<T>(chunk_ok ? qraw[g] : make_uint4(0, 0, 0, 0), qf[g]);
         }
         // The dense output's stretch under the batch starts out as the fill value; the scores of
         // selected keys follow behind the barriers.
