@@ -36,7 +36,10 @@ struct SearchParams {
     const void* queue_values;
     int32_t queue_len, queue_cap;
     // work split
-    int32_t nodes_per_wave;  // vector-ALU kernel: level-1 nodes (or pseudo blocks) a workgroup walks, per wave of it; MFMA kernel: tiles per workgroup
+    union {
+        int32_t nodes_per_wave;  // MFMA kernel: tiles per workgroup
+        int32_t nodes_per_wg;    // vector-ALU kernel: level-1 nodes (or pseudo blocks) a workgroup walks
+    };
     int32_t tree_blocks;     // workgroups that walk the tree; the rest scan the queue
     int32_t key_policy;      // MFMA kernel: which cache policy the scan's loads use (0: default,
                              // 1: key tiles non-temporal, 2: value rows too), by the launch's size
@@ -56,7 +59,7 @@ struct SearchParams {
     float* part_l;    // (H_q, P)
     float* part_acc;  // (H_q, P, Dv)
     int32_t num_parts;  // P = gridDim.x
-    int32_t gmax_state; // MFMA kernel: heads per pass its LDS state rows are sized for
+    int32_t queue_nodes;  // vector-ALU kernel: pseudo blocks of the queue a workgroup takes
     void* attn_out;     // (H_q, Dv): written by the kernel itself when `done` is set
     int32_t* done;      // (T, passes) arrival counters, zero between launches; NULL: no fold
     int32_t out_bf16;   // attn_out's type: bf16, else fp32
@@ -75,10 +78,11 @@ struct SearchPlan {
     int lpr;          // lanes per row (vector-ALU kernel)
     int gmax;         // heads per pass
     int threads;      // workgroup size
-    int nodes_per_wave;
+    int nodes_per_wave;  // MFMA kernel: tiles per workgroup
+    int nodes_per_wg, queue_nodes;  // vector-ALU kernel: as in SearchParams
     int num_nodes, num_queue_blocks;
     int tree_blocks, queue_blocks, head_chunks;
-    bool ahead;       // MFMA kernel: key tiles are asked for together with the gates' operands
+    int ahead;        // > 0: keys are asked for together with the gates' operands (vector-ALU kernel: as many elements a lane)
     size_t smem;
 };
 

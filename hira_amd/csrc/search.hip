@@ -89,6 +89,7 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
                            l, t->cap[l]);
     }
     plan->ahead = false;
+    plan->nodes_per_wg = plan->queue_nodes = 0;
     plan->num_queue_blocks = 0;
     if (queue && queue->keys && queue->len > 0) {
         HIRA_CHECK_ARG(queue->len <= queue->cap, "queue len %d > cap %d", queue->len,
@@ -197,10 +198,33 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
         if (per < least) per = least;
         npw = (int)((per + waves - 1) / waves);
     }
-    plan->nodes_per_wave = npw;
-    const int per_block = waves * npw;
-    plan->tree_blocks = (plan->num_nodes + per_block - 1) / per_block;
-    plan->queue_blocks = (plan->num_queue_blocks + per_block - 1) / per_block;
+    plan->nodes_per_wg = plan->queue_nodes = waves * npw;
+    if (t->num_levels >= 2 && threads == kVecThreads && !(launch && launch->nodes_per_wave)) {
+        // One batch of nodes a workgroup and one block of rows a wave, its keys asked for beside the gates'
+        // operands (search_kernel's ONE): where the workgroups of the smaller block, else of the larger, are no
+        // more than above, and the keys of nodes that the gates would have pruned are few.  us, general way /
+        // larger / smaller block: 4 trees x 1000 rows of 80 fp32, three heads, 14.55 / 11.5 / 10.5 (twice as
+        // many workgroups as compute units lose: x 5003 15.3 / 12.4 / 14.6); rows of 96 bf16 x 5003 15.1 / 13.0;
+        // a search without attention of 10000 rows of 128 fp32 5.5 / 4.25 / 3.9, of 40000, 85 % of them
+        // pruned, 8.4 / 7.0 (indexes taking turns 10.3 / 8.7)
+        const int rpw = kWave / lpr;
+        const size_t key_bytes = (size_t)t->num_trees * (size_t)t->size[0] * (size_t)t->dim * esize;
+        for (int elems = kOneSmall; elems <= (plan->gmax <= 4 ? kOneLarge : kOneSmall) && !plan->ahead; elems *= 2) {
+            const int rows = kVecThreads / 64 * vec_one_rows(rpw, epl, elems);
+            int per = rows / t->bf;
+            if (per > kBatch) per = kBatch;
+            if (per > kOneGateRows * kVecThreads / 64 * rpw) per = kOneGateRows * kVecThreads / 64 * rpw;
+            if (per < 1 || rows < kPseudoBlock || key_bytes > ((size_t)28 << 20)) continue;
+            if ((int64_t)((plan->num_nodes + per - 1) / per) * t->num_trees * plan->head_chunks >
+                (attn ? 1 : 2) * compute_units())
+                continue;
+            plan->ahead = elems;
+            plan->nodes_per_wg = per;
+            plan->queue_nodes = rows / kPseudoBlock;
+        }
+    }
+    plan->tree_blocks = (plan->num_nodes + plan->nodes_per_wg - 1) / plan->nodes_per_wg;
+    plan->queue_blocks = (plan->num_queue_blocks + plan->queue_nodes - 1) / plan->queue_nodes;
     plan->smem = (size_t)(threads / 64) * state;
     {   // the fold of the last workgroup reuses the same LDS
         const size_t heads_parts = (size_t)plan->gmax * (plan->tree_blocks + plan->queue_blocks);
@@ -309,7 +333,9 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
         p.queue_len = queue->len;
         p.queue_cap = queue->cap;
     }
-    p.nodes_per_wave = plan.nodes_per_wave;
+    if (plan.kernel == 2) p.nodes_per_wave = plan.nodes_per_wave;
+    else p.nodes_per_wg = plan.nodes_per_wg;
+    p.queue_nodes = plan.queue_nodes;
     p.tree_blocks = plan.tree_blocks;
     {   // up to what the eight L2s hold together (32 MiB) the default policy; up to 512 MiB the
         // key tiles and the value rows non-temporal; beyond, the key tiles only
@@ -370,7 +396,6 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
 
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     dim3 grid(P, tree->num_trees, plan.head_chunks);
-    p.gmax_state = plan.gmax;
     if (plan.kernel == 2)
         rc = launch_search_mfma(plan, p, dim3(tree->num_trees, P, plan.head_chunks), s);
     else

@@ -13,8 +13,9 @@
 //           rows; the values of a block's selected rows are asked for together.
 // So a launch is a chain of four trips to memory (arguments, gates, keys, values) plus the hand-off
 // of the partials, whatever the fan-out, and a pruned node costs nothing behind its gate.  (4 trees x
-// 5003 rows of 80 fp32, three heads, as the work falls away: 15.6 us; with a key a head selected 13.4;
-// with every node pruned 10.6; without the attention 8.8, 8.6 and 5.6.)  No
+// 5003 rows of 80 fp32, three heads, as the work falls away: 15.25 us; with a key a head selected 13.4;
+// with every node pruned 10.6; without the attention 8.8, 8.6 and 5.6.)  Small launches ask for gates and
+// keys at once, in straight-line code (ONE, below): 12.4 us for that one.  No
 // global frontier is exchanged between workgroups.  (Before, every wave walked nodes of its own:
 // each gate repeated the ancestors' rows, and short nodes left most lanes without a row.)
 //
@@ -33,10 +34,18 @@ namespace hira {
 
 constexpr int kVecThreads = 512;  // workgroup size, at most
 constexpr int kBatch = 64;        // level-1 nodes a workgroup gates together
+constexpr int kOneGateRows = 2;   // level-1 rows a lane group asks for where there is one batch (ONE, below)
 // rows of a block that a wave scans at once: eight loads a lane (with eight heads a pass as many as
 // the registers have room for: four, two of bf16), at most 64 rows
 constexpr int vec_rows(int rpw, int gmax, int epl) {
     const int r = (gmax <= 4 ? 8 : 16 / epl) * rpw;
+    return r < 64 ? r : 64;
+}
+// rows of a wave's block where it has only one (ONE, below), for `elems` elements a lane: a block is as much
+// work whatever it holds, so the smaller one is taken where the workgroups then still fit
+constexpr int kOneSmall = 16, kOneLarge = 32;
+constexpr int vec_one_rows(int rpw, int epl, int elems) {
+    const int r = elems / epl * rpw;
     return r < 64 ? r : 64;
 }
 
@@ -284,13 +293,18 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
     }
 }
 
-template <typename T, int LPR, int GMAX>
+// ONE > 0: every workgroup of the launch has one batch of nodes whose key slots are one block of rows for
+// each of its eight waves (of ONE elements a lane).  A wave then asks for its block together with the gates'
+// operands of all levels, whether the nodes survive or not: no list, two trips to memory and a barrier less,
+// and no loop, at whose head the waits would be for everything asked for so far.  Every row being in some
+// wave's block, a dense output's fill value goes out with the scores.
+template <typename T, int LPR, int GMAX, int ONE>
 __global__ __launch_bounds__(kVecThreads) __attribute__((amdgpu_waves_per_eu(GMAX == 1 ? 3 : 2)))
 void search_kernel(const SearchParams p) {
     constexpr int EPL = Elem<T>::kPerChunk;
     constexpr int RPW = kWave / LPR;  // rows per wave-wide load
     constexpr int DVP = LPR * EPL;    // widest row a lane group can hold
-    constexpr int KU = vec_rows(RPW, GMAX, EPL) / RPW;  // row loads in flight per lane
+    constexpr int KU = (ONE ? vec_one_rows(RPW, EPL, ONE) : vec_rows(RPW, GMAX, EPL)) / RPW;  // row loads in flight per lane
     constexpr int ROWS = KU * RPW;
     constexpr int NV = KU * GMAX;                  // scores a lane group makes of a block
     constexpr int KEPT = vec_kept(NV, LPR);
@@ -332,8 +346,9 @@ void search_kernel(const SearchParams p) {
     const int blk = is_queue ? (int)blockIdx.x - p.tree_blocks : (int)blockIdx.x;
     const int n_nodes = is_queue ? p.num_queue_blocks : p.num_nodes;
     const bool real_nodes = !is_queue && L >= 2;
-    const int node_first = blk * nwaves * p.nodes_per_wave;
-    const int node_last = min(node_first + nwaves * p.nodes_per_wave, n_nodes);
+    const int wg_nodes = is_queue ? p.queue_nodes : p.nodes_per_wg;
+    const int node_first = blk * wg_nodes;
+    const int node_last = min(node_first + wg_nodes, n_nodes);
 
     // threshold, scale and head of the values whose sums this lane ends up with
     int vfirst = 0;  // vec_value_of(ch)
@@ -400,6 +415,316 @@ void search_kernel(const SearchParams p) {
         for (int e = 0; e < EPL; ++e) acc[g][e] = 0.0f;
     float qf[GMAX][EPL];
 
+    // ---- a wave's block of rows once it has arrived: scores, sums over the lanes, the selection, outputs, the
+    // selected rows' values.  slot[u]: key slot of row u of the lane group; mine(): slot of the row
+    // whose sums this lane ends up with, whether it is one, the heads it may be selected for --------
+    float* tab = s_tab[wave];
+    auto take = [&](const uint4 (&raw)[KU], const int (&slot)[KU], auto mine) {
+        float s[NV];
+#pragma unroll
+        for (int u = 0; u < KU; ++u) {
+            float kf[EPL];
+            unpack<T>(raw[u], kf);
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) {
+                float d = 0.0f;
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
+                s[u * GMAX + g] = d;
+            }
+        }
+        reduce_scatter<NV, LPR / 2>(s, lane);
+        int my_slot;
+        bool my_row;
+        const unsigned my_am = mine(my_slot, my_row);
+        unsigned sel = 0;  // bit i: value i
+#pragma unroll
+        for (int i = 0; i < KEPT; ++i)
+            if (((my_am >> (my_g + i)) & 1u) && (is_queue || s[i] >= my_tau[i])) sel |= 1u << i;
+        const bool owner = LANES.any == ~0ull || ((LANES.any >> lane) & 1ull);
+        const uint64_t B = __ballot(owner && sel != 0u);  // lanes that hold a selected score
+        if constexpr (ONE) {
+            // (every row of the workgroup's nodes is in some wave's block: fill value or score)
+            if (p.dense != nullptr && p.dense_fill && !is_queue && owner && my_row) {
+#pragma unroll
+                for (int i = 0; i < KEPT; ++i)
+                    if (my_g + i < G)
+                        p.dense[(int64_t)my_h[i] * p.dense_stride + my_slot] =
+                            (sel >> i) & 1u ? s[i] * my_sc[i] : p.dense_fill_value;
+            }
+        }
+        if (B == 0ull) return;  // uniform in the wave
+        if (p.stats) {
+            // a key is selected where any of its heads is: every row once
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                const uint64_t lanes = B & LANES.row[u];
+                for (int r = 0; r < RPW; ++r) {
+                    const uint64_t group = LPR == 64 ? ~0ull : ((1ull << (LPR & 63)) - 1ull) << (r * LPR);
+                    if (lane == 0 && (lanes & group)) count(HIRA_MAX_LEVELS, 1);
+                }
+            }
+            if (owner && sel) count(HIRA_MAX_LEVELS + 1, (unsigned)__popc(sel));
+        }
+        if (!is_queue && (p.dense != nullptr || p.sel_count != nullptr)) {
+            int idx = my_slot;
+            if (owner && sel && p.dense_by_position) idx = p.perm[krow0 + my_slot];
+            if (p.dense != nullptr && owner && !(ONE && p.dense_fill)) {
+#pragma unroll
+                for (int i = 0; i < KEPT; ++i)
+                    if ((sel >> i) & 1u) p.dense[(int64_t)my_h[i] * p.dense_stride + idx] = s[i] * my_sc[i];
+            }
+            if (p.sel_count != nullptr) {
+#pragma unroll
+                for (int i = 0; i < KEPT; ++i) {
+                    const uint64_t Bi = __ballot(owner && ((sel >> i) & 1u));
+#pragma unroll
+                    for (int g = 0; g < GMAX; ++g) {
+                        // (a head's entries of the wave go side by side: one atomic)
+                        const bool mine = owner && ((sel >> i) & 1u) && my_g + i == g;
+                        const uint64_t bal = __ballot(mine);
+                        if (Bi == 0ull || bal == 0ull) continue;  // uniform
+                        int base = 0;
+                        if (mine && (bal & ((1ull << lane) - 1ull)) == 0ull)
+                            base = atomicAdd(&p.sel_count[my_h[i]], __popcll(bal));
+                        base = __shfl(base, __ffsll((long long)bal) - 1, 64);
+                        const int pos = base + __popcll(bal & ((1ull << lane) - 1ull));
+                        if (mine && pos < p.sel_cap) {
+                            p.sel_index[(int64_t)my_h[i] * p.sel_cap + pos] = idx;
+                            p.sel_score[(int64_t)my_h[i] * p.sel_cap + pos] = s[i];
+                        }
+                    }
+                }
+            }
+        }
+        if (!want_attn) return;  // uniform
+        // ---- the values of the rows that some head selected -------------------------------
+        uint4 vraw[KU];
+#pragma unroll
+        for (int u = 0; u < KU; ++u) {
+            vraw[u] = make_uint4(0, 0, 0, 0);
+            const uint64_t lanes = B & LANES.row[u];
+            const uint64_t group = LPR == 64 ? ~0ull : ((1ull << (LPR & 63)) - 1ull) << (rg * LPR);
+            if ((lanes & group) != 0ull && vchunk_ok) vraw[u] = load_chunk<T>(vbase, (krow0 + slot[u]) * Dv, ch);
+        }
+        if (owner) {
+#pragma unroll
+            for (int i = 0; i < KEPT; ++i) {
+                // (fminf: a logit that is no number becomes +inf.  A maximum does not see the former,
+                // and what follows makes NaN of both, as a softmax does)
+                const float z = fminf(s[i] * my_sc[i] * kLog2e, INFINITY);
+                tab[(my_u * RPW + rg) * GMAX + my_g + i] = (sel >> i) & 1u ? z : -INFINITY;
+            }
+        }
+        // weights while the values are on their way: lane l takes the table's entries
+        // l, l + 64, ..., all of head l % GMAX
+        constexpr int NE = (ROWS * GMAX + 63) / 64;
+        __builtin_amdgcn_wave_barrier();
+        float z[NE], mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            const bool mine = ROWS * GMAX >= 64 || lane < ROWS * GMAX;
+            z[i] = mine ? tab[i * 64 + lane] : -INFINITY;
+            mx = fmaxf(mx, z[i]);
+        }
+        mx = fmaxf(cross_group_max<GMAX>(mx), m_run);
+        const float f = m_run == -INFINITY ? 0.0f : exp2f(m_run - mx);
+        l_run *= f;
+        m_run = mx;
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+            // (zero says "not selected": a selected row's weight stays above it)
+            float w = z[i] > -INFINITY ? exp2f(z[i] - mx) : 0.0f;
+            l_run += w;
+            if (GMAX > 1 && w == 0.0f && z[i] > -INFINITY) w = 1e-45f;
+            if (ROWS * GMAX >= 64 || lane < ROWS * GMAX) tab[i * 64 + lane] = w;
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int g = 0; g < GMAX; ++g) {
+            const float fg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), g));
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[g][e] *= fg;
+        }
+        // (a row's weights are asked for with the row before it.  The heads that did not select the row
+        // are masked out, not multiplied by zero: a value that is not finite stays with those that did.
+        // As masks on straight-line code it costs nothing to be seen with up to four heads a pass and 2 %
+        // with eight -- 2 trees x 20000 rows of 64 bf16 25.8 -> 26.2 us --, as branches 2 and 7 %)
+        float wt[GMAX];
+#pragma unroll
+        for (int g = 0; g < GMAX; ++g) wt[g] = tab[rg * GMAX + g];
+#pragma unroll
+        for (int u = 0; u < KU; ++u) {
+            float next[GMAX];
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) next[g] = tab[(min(u + 1, KU - 1) * RPW + rg) * GMAX + g];
+            if ((B & LANES.row[u]) != 0ull) {  // uniform in the wave
+                float vf[EPL];
+                unpack<T>(vraw[u], vf);
+#pragma unroll
+                for (int g = 0; g < GMAX; ++g)
+                    if (GMAX == 1 || __builtin_expect(wt[g] != 0.0f, 1)) {
+#pragma unroll
+                        for (int e = 0; e < EPL; ++e) acc[g][e] += wt[g] * vf[e];
+                    }
+            }
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) wt[g] = next[g];
+        }
+    };
+    if constexpr (ONE) {
+        float qn[GMAX];
+        auto queries = [&]() {
+    #pragma unroll
+            for (int g = 0; g < GMAX; ++g) {
+                unpack<T>(chunk_ok ? qraw[g] : make_uint4(0, 0, 0, 0), qf[g]);
+                float ss = 0.0f;
+    #pragma unroll
+                for (int e = 0; e < EPL; ++e) ss += qf[g][e] * qf[g][e];
+                qn[g] = sqrtf(group_sum<LPR>(ss));
+            }
+        };
+        // row r of level l's rows of the batch: which heads pass, and is there a node at all
+        auto judge = [&](int l, int rows, int r, const uint4& raw, float rad) {
+            float kf[EPL];
+            unpack<T>(raw, kf);
+            unsigned pass = 0;
+    #pragma unroll
+            for (int g = 0; g < GMAX; ++g) {
+                float d = 0.0f;
+    #pragma unroll
+                for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
+                d = group_sum<LPR>(d);
+                if (d + qn[g] * rad >= tau[g]) pass |= 1u << g;
+            }
+            if (ch == 0 && r < rows) s_pass[l][r] = pass | (rad > -INFINITY ? 0x80000000u : 0u);
+        };
+        auto ask = [&](int l, int first, int rows, int r, uint4& raw, float& rad) {
+            raw = make_uint4(0, 0, 0, 0);
+            rad = -INFINITY;
+            if (r < rows) {
+                const size_t t0 = (size_t)tree * p.cap[l];
+                if (chunk_ok) raw = load_row_chunk<T>(p.centers[l], p.layout, D, t0, first + r, ch);
+                rad = p.radii[l][t0 + first + r];
+            }
+        };
+        // a level-1 node, lane `lane` of the batch: a node counts where a head is alive above it, by its
+        // first level-1 descendant
+        auto count_nodes = [&](int n0) {
+            unsigned a = gmask;
+            for (int l = L - 1; l >= 1; --l) {
+                unsigned id = (unsigned)(n0 + lane), fl = (unsigned)n0;
+                bool lead = true;
+                for (int i = 1; i < l; ++i) {
+                    const unsigned up = over_bf(id);
+                    lead = lead && up * (unsigned)p.bf == id;
+                    id = up;
+                    fl = over_bf(fl);
+                }
+                const uint32_t w = s_pass[l][id - fl];
+                if (a && (w >> 31) && lead) count(l, 1);
+                a &= w;
+            }
+        };
+        const int n0 = node_first, nb = node_last - node_first;  // (never empty, kBatch at most)
+        const int cc = chunk_ok ? ch : 0;
+        auto row_at = [&](const void* base, int layout, size_t row0, int row) {
+            const T* b = reinterpret_cast<const T*>(base) + row0 * (size_t)D;
+            const size_t at = sizeof(T) == 4 || layout == HIRA_ROW_MAJOR ? (size_t)row * D + cc * EPL
+                                                                         : elem_index(HIRA_TILE16, D, (size_t)row, cc * EPL);
+            return *reinterpret_cast<const uint4*>(b + at);
+        };
+        const uint4 none = make_uint4(0, 0, 0, 0);
+        // gates: rows of levels 1 and 2 over all waves, every level above on a wave of its own; a row that
+        // is not there is the last one again, a level that is not there level 1
+        constexpr int KA = kOneGateRows;
+        const int r0 = wave * RPW + rg, rstep = nwaves * RPW;
+        const int l2 = L > 2 ? 2 : 1, l3w = 2 + (wave == 0 ? nwaves : wave), l3 = l3w < L ? l3w : 1;
+        int first2 = 0, rows2 = 0, first3 = 0, rows3 = 0, cnt = 0;
+        uint4 raw1[KA], raw2 = none, raw3 = none, kraw[KU];
+        float rad1[KA], rad2 = 0.0f, rad3 = 0.0f;
+        const int i0 = wave * ROWS, wg_rows = nb * block_rows;  // my block's first row
+        const int slot0 = n0 * block_rows + i0 + rg;
+        if (real_nodes) {  // uniform
+            first2 = (int)over_bf((unsigned)n0);
+            int last2 = (int)over_bf((unsigned)(n0 + nb - 1));
+            rows2 = L > 2 ? last2 - first2 + 1 : 0;
+            first3 = first2;
+            int last3 = last2;
+            for (int l = 3; l <= l3; ++l) {
+                first3 = (int)over_bf((unsigned)first3);
+                last3 = (int)over_bf((unsigned)last3);
+            }
+            rows3 = l3w < L ? last3 - first3 + 1 : 0;
+            const size_t t1 = (size_t)tree * p.cap[1], t2 = (size_t)tree * p.cap[l2], t3 = (size_t)tree * p.cap[l3];
+#pragma unroll
+            for (int k = 0; k < KA; ++k) {
+                const int row = n0 + min(r0 + k * rstep, nb - 1);
+                raw1[k] = row_at(p.centers[1], p.layout, t1, row);
+                rad1[k] = p.radii[1][t1 + row];
+            }
+            const int row2 = rows2 > 0 ? first2 + min(r0, rows2 - 1) : 0;
+            raw2 = row_at(p.centers[l2], p.layout, t2, row2);
+            rad2 = p.radii[l2][t2 + row2];
+            const int row3 = rows3 > 0 ? first3 + min(rg, rows3 - 1) : 0;
+            raw3 = row_at(p.centers[l3], p.layout, t3, row3);
+            rad3 = p.radii[l3][t3 + row3];
+            cnt = p.counts[1][t1 + n0 + min(lane, nb - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < KU; ++u) kraw[u] = row_at(kbase, klayout, krow0, min(slot0 + u * RPW, n_rows - 1));
+        __builtin_amdgcn_sched_barrier(0);  // (nothing that uses a load moves above this line)
+        queries();
+        unsigned alive = gmask;
+        if (real_nodes) {  // uniform
+            if (wave * RPW < rows2) judge(2, rows2, r0, chunk_ok ? raw2 : none, rad2);  // (uniform in the wave)
+            if (rows3 > 0) judge(l3, rows3, rg, chunk_ok ? raw3 : none, rad3);
+#pragma unroll
+            for (int k = 0; k < KA; ++k)
+                if (wave * RPW + k * rstep < nb) judge(1, nb, r0 + k * rstep, chunk_ok ? raw1[k] : none, rad1[k]);
+#pragma unroll 1
+            for (int r = r0 + rstep; r - rg < rows2; r += rstep) {  // (fan-outs of two or three)
+                ask(2, first2, rows2, r, raw2, rad2);
+                judge(2, rows2, r, raw2, rad2);
+            }
+#pragma unroll 1
+            for (int r = rg + RPW; r - rg < rows3; r += RPW) {
+                ask(l3, first3, rows3, r, raw2, rad2);
+                judge(l3, rows3, r, raw2, rad2);
+            }
+            __syncthreads();
+            // a node is alive for the heads that it and all its ancestors pass for (every wave for itself: no
+            // second barrier)
+            alive = lane < nb && cnt > 0 ? gmask & s_pass[1][lane] : 0u;
+            unsigned id = (unsigned)(n0 + min(lane, nb - 1)), fl = (unsigned)n0;
+#pragma unroll 1
+            for (int l = 2; l < L; ++l) {
+                id = over_bf(id);
+                fl = over_bf(fl);
+                alive &= s_pass[l][id - fl];
+            }
+            if (p.stats && wave == 0) {
+                if (lane < nb) count_nodes(n0);
+                if (alive) count(0, (unsigned)cnt);
+            }
+        }
+        if (i0 < wg_rows) {  // uniform in the wave
+            int slot[KU];
+#pragma unroll
+            for (int u = 0; u < KU; ++u) {
+                slot[u] = min(slot0 + u * RPW, n_rows - 1);
+                if (!chunk_ok) kraw[u] = none;
+            }
+            take(kraw, slot, [&](int& my_slot, bool& my_row) -> unsigned {
+                const int row = i0 + my_u * RPW + rg, k = (int)(((float)row + 0.5f) * inv_rows);
+                const int node = __shfl((int)(alive | ((unsigned)cnt << 16)), min(k, 63), 64);
+                my_slot = n0 * block_rows + row;
+                my_row = row < wg_rows && my_slot < n_rows;
+                if (!real_nodes) return my_row ? gmask : 0u;
+                return my_row && row - k * block_rows < (node >> 16) ? (unsigned)node & 0xFFFFu : 0u;
+            });
+        }
+    } else {
     for (int n0 = node_first; n0 < node_last; n0 += kBatch) {  // uniform in the workgroup
         const int nb = min(kBatch, node_last - n0);
         if (n0 > node_first) __syncthreads();  // (the list of the batch before is done with)
@@ -534,7 +859,6 @@ void search_kernel(const SearchParams p) {
         __syncthreads();
         // ---- scan ---------------------------------------------------------------------------
         const int nrows = s_count * block_rows;
-        float* tab = s_tab[wave];
         // row `row` of the survivors' rows: its key slot, the heads it may be selected for (0: none)
         auto row_info = [&](int row, int& slot) -> unsigned {
             // (rows of a batch stay far below 2^22: the float quotient is exact enough)
@@ -554,149 +878,10 @@ void search_kernel(const SearchParams p) {
                 raw[u] = make_uint4(0, 0, 0, 0);
                 if (am != 0u && chunk_ok) raw[u] = load_row_chunk<T>(kbase, klayout, D, krow0, slot[u], ch);
             }
-            float s[NV];
-#pragma unroll
-            for (int u = 0; u < KU; ++u) {
-                float kf[EPL];
-                unpack<T>(raw[u], kf);
-#pragma unroll
-                for (int g = 0; g < GMAX; ++g) {
-                    float d = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < EPL; ++e) d += kf[e] * qf[g][e];
-                    s[u * GMAX + g] = d;
-                }
-            }
-            reduce_scatter<NV, LPR / 2>(s, lane);
-            // this lane's sums: row my_u of its group's block, heads my_g ...
-            int my_slot;
-            const unsigned my_am = row_info(i0 + my_u * RPW + rg, my_slot);
-            unsigned sel = 0;  // bit i: value i
-#pragma unroll
-            for (int i = 0; i < KEPT; ++i)
-                if (((my_am >> (my_g + i)) & 1u) && (is_queue || s[i] >= my_tau[i])) sel |= 1u << i;
-            const bool owner = LANES.any == ~0ull || ((LANES.any >> lane) & 1ull);
-            const uint64_t B = __ballot(owner && sel != 0u);  // lanes that hold a selected score
-            if (B == 0ull) continue;  // uniform in the wave
-            if (p.stats) {
-                // a key is selected where any of its heads is: every row once
-#pragma unroll
-                for (int u = 0; u < KU; ++u) {
-                    const uint64_t lanes = B & LANES.row[u];
-                    for (int r = 0; r < RPW; ++r) {
-                        const uint64_t group = LPR == 64 ? ~0ull : ((1ull << (LPR & 63)) - 1ull) << (r * LPR);
-                        if (lane == 0 && (lanes & group)) count(HIRA_MAX_LEVELS, 1);
-                    }
-                }
-                if (owner && sel) count(HIRA_MAX_LEVELS + 1, (unsigned)__popc(sel));
-            }
-            if (!is_queue && (p.dense != nullptr || p.sel_count != nullptr)) {
-                int idx = my_slot;
-                if (owner && sel && p.dense_by_position) idx = p.perm[krow0 + my_slot];
-                if (p.dense != nullptr && owner) {
-#pragma unroll
-                    for (int i = 0; i < KEPT; ++i)
-                        if ((sel >> i) & 1u) p.dense[(int64_t)my_h[i] * p.dense_stride + idx] = s[i] * my_sc[i];
-                }
-                if (p.sel_count != nullptr) {
-#pragma unroll
-                    for (int i = 0; i < KEPT; ++i) {
-                        const uint64_t Bi = __ballot(owner && ((sel >> i) & 1u));
-#pragma unroll
-                        for (int g = 0; g < GMAX; ++g) {
-                            // (a head's entries of the wave go side by side: one atomic)
-                            const bool mine = owner && ((sel >> i) & 1u) && my_g + i == g;
-                            const uint64_t bal = __ballot(mine);
-                            if (Bi == 0ull || bal == 0ull) continue;  // uniform
-                            int base = 0;
-                            if (mine && (bal & ((1ull << lane) - 1ull)) == 0ull)
-                                base = atomicAdd(&p.sel_count[my_h[i]], __popcll(bal));
-                            base = __shfl(base, __ffsll((long long)bal) - 1, 64);
-                            const int pos = base + __popcll(bal & ((1ull << lane) - 1ull));
-                            if (mine && pos < p.sel_cap) {
-                                p.sel_index[(int64_t)my_h[i] * p.sel_cap + pos] = idx;
-                                p.sel_score[(int64_t)my_h[i] * p.sel_cap + pos] = s[i];
-                            }
-                        }
-                    }
-                }
-            }
-            if (!want_attn) continue;  // uniform
-            // ---- the values of the rows that some head selected -------------------------------
-            uint4 vraw[KU];
-#pragma unroll
-            for (int u = 0; u < KU; ++u) {
-                vraw[u] = make_uint4(0, 0, 0, 0);
-                const uint64_t lanes = B & LANES.row[u];
-                const uint64_t group = LPR == 64 ? ~0ull : ((1ull << (LPR & 63)) - 1ull) << (rg * LPR);
-                if ((lanes & group) != 0ull && vchunk_ok) vraw[u] = load_chunk<T>(vbase, (krow0 + slot[u]) * Dv, ch);
-            }
-            if (owner) {
-#pragma unroll
-                for (int i = 0; i < KEPT; ++i) {
-                    // (fminf: a logit that is no number becomes +inf.  A maximum does not see the former,
-                    // and what follows makes NaN of both, as a softmax does)
-                    const float z = fminf(s[i] * my_sc[i] * kLog2e, INFINITY);
-                    tab[(my_u * RPW + rg) * GMAX + my_g + i] = (sel >> i) & 1u ? z : -INFINITY;
-                }
-            }
-            // weights while the values are on their way: lane l takes the table's entries
-            // l, l + 64, ..., all of head l % GMAX
-            constexpr int NE = (ROWS * GMAX + 63) / 64;
-            __builtin_amdgcn_wave_barrier();
-            float z[NE], mx = -INFINITY;
-#pragma unroll
-            for (int i = 0; i < NE; ++i) {
-                const bool mine = ROWS * GMAX >= 64 || lane < ROWS * GMAX;
-                z[i] = mine ? tab[i * 64 + lane] : -INFINITY;
-                mx = fmaxf(mx, z[i]);
-            }
-            mx = fmaxf(cross_group_max<GMAX>(mx), m_run);
-            const float f = m_run == -INFINITY ? 0.0f : exp2f(m_run - mx);
-            l_run *= f;
-            m_run = mx;
-#pragma unroll
-            for (int i = 0; i < NE; ++i) {
-                // (zero says "not selected": a selected row's weight stays above it)
-                float w = z[i] > -INFINITY ? exp2f(z[i] - mx) : 0.0f;
-                l_run += w;
-                if (GMAX > 1 && w == 0.0f && z[i] > -INFINITY) w = 1e-45f;
-                if (ROWS * GMAX >= 64 || lane < ROWS * GMAX) tab[i * 64 + lane] = w;
-            }
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int g = 0; g < GMAX; ++g) {
-                const float fg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), g));
-#pragma unroll
-                for (int e = 0; e < EPL; ++e) acc[g][e] *= fg;
-            }
-            // (a row's weights are asked for with the row before it.  The heads that did not select the row
-            // are masked out, not multiplied by zero: a value that is not finite stays with those that did.
-            // As masks on straight-line code it costs nothing to be seen with up to four heads a pass and 2 %
-            // with eight -- 2 trees x 20000 rows of 64 bf16 25.8 -> 26.2 us --, as branches 2 and 7 %)
-            float wt[GMAX];
-#pragma unroll
-            for (int g = 0; g < GMAX; ++g) wt[g] = tab[rg * GMAX + g];
-#pragma unroll
-            for (int u = 0; u < KU; ++u) {
-                float next[GMAX];
-#pragma unroll
-                for (int g = 0; g < GMAX; ++g) next[g] = tab[(min(u + 1, KU - 1) * RPW + rg) * GMAX + g];
-                if ((B & LANES.row[u]) != 0ull) {  // uniform in the wave
-                    float vf[EPL];
-                    unpack<T>(vraw[u], vf);
-#pragma unroll
-                    for (int g = 0; g < GMAX; ++g)
-                        if (GMAX == 1 || __builtin_expect(wt[g] != 0.0f, 1)) {
-#pragma unroll
-                            for (int e = 0; e < EPL; ++e) acc[g][e] += wt[g] * vf[e];
-                        }
-                }
-#pragma unroll
-                for (int g = 0; g < GMAX; ++g) wt[g] = next[g];
-            }
+            take(raw, slot, [&](int& my_slot, bool&) { return row_info(i0 + my_u * RPW + rg, my_slot); });
         }
     }
+    }  // ONE or loops
 
     if (!want_attn) return;  // uniform
 
@@ -768,20 +953,23 @@ void search_kernel(const SearchParams p) {
     fold_heads(p, hoff, G, smem);
 }
 
+template <typename T, int LPR, int GMAX>
+inline void launch_search(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s) {
+    const size_t smem = p.part_acc ? plan.smem : 0;
+    const dim3 block(plan.threads);
+    // (a block of the larger kind holds more scores a lane than eight heads leave registers for)
+    if (plan.ahead == kOneSmall) hipLaunchKernelGGL((search_kernel<T, LPR, GMAX, kOneSmall>), grid, block, smem, s, p);
+    else if (plan.ahead) hipLaunchKernelGGL((search_kernel<T, LPR, GMAX, (GMAX <= 4 ? kOneLarge : kOneSmall)>), grid, block, smem, s, p);
+    else hipLaunchKernelGGL((search_kernel<T, LPR, GMAX, 0>), grid, block, smem, s, p);
+}
+
 template <typename T, int LPR>
 inline void launch_search(const SearchPlan& plan, const SearchParams& p, dim3 grid,
                           hipStream_t s) {
-    const size_t smem = p.part_acc ? plan.smem : 0;
     switch (plan.gmax) {
-        case 1:
-            hipLaunchKernelGGL((search_kernel<T, LPR, 1>), grid, dim3(plan.threads), smem, s, p);
-            break;
-        case 4:
-            hipLaunchKernelGGL((search_kernel<T, LPR, 4>), grid, dim3(plan.threads), smem, s, p);
-            break;
-        default:
-            hipLaunchKernelGGL((search_kernel<T, LPR, 8>), grid, dim3(plan.threads), smem, s, p);
-            break;
+        case 1: launch_search<T, LPR, 1>(plan, p, grid, s); break;
+        case 4: launch_search<T, LPR, 4>(plan, p, grid, s); break;
+        default: launch_search<T, LPR, 8>(plan, p, grid, s); break;
     }
 }
 

@@ -84,3 +84,66 @@ def test_first_call_on_an_index_may_be_captured(dtype, gpu_device):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+ONE_CASES = [
+    # trees, heads a tree, keys, key width, value width, fan-out, levels, type, layout, queued rows
+    (1, 1, 9, 16, 16, 1, 3, torch.float32, "row_major", 0),      # fan-out 1: as many nodes as keys
+    (2, 1, 500, 128, 64, 2, 5, torch.float32, "row_major", 0),   # more rows of level 2 than a load brings
+    (2, 3, 777, 64, 128, 3, 7, torch.bfloat16, "row_major", 40),
+    (1, 4, 2100, 80, 80, 7, 4, torch.float32, "row_major", 129),
+    (3, 5, 600, 256, 256, 64, 2, torch.float32, "row_major", 3),   # a node is half a workgroup's rows
+    (2, 8, 640, 512, 512, 16, 3, torch.bfloat16, "row_major", 0),  # 64 lanes a row, eight heads
+    (2, 12, 1500, 96, 96, 10, 3, torch.bfloat16, "tiled", 9),
+    (2, 4, 3000, 64, 64, 4, 2, torch.bfloat16, "tiled", 0),
+    (1, 2, 1300, 8, 8, 5, 4, torch.bfloat16, "row_major", 1),
+]
+
+
+@pytest.mark.parametrize("t,g,n,d,dv,bf,nl,dtype,layout,m", ONE_CASES)
+def test_one_block_a_wave_equals_the_general_way(t, g, n, d, dv, bf, nl, dtype, layout, m, gpu_device):
+    """Launches whose workgroups ask for their keys beside the gates, against the batches and lists that
+    launch options still take: the same scores, lists and counters, attention but for the order of its
+    sums, also with heads in an order of the caller's, key and value rows that are not finite, a head
+    that selects everything and one that selects nothing."""
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    print(f"case {t} {g} {n} {d} {dv} {bf} {nl} {dtype} {layout} {m}", flush=True)
+    gen = torch.Generator().manual_seed(n + d)
+    k = torch.randn(1, t, n, d, generator=gen).to(dtype).cuda()
+    v = torch.randn(1, t, n, dv, generator=gen).to(dtype).cuda()
+    q = torch.randn(t * g, d, generator=gen).to(dtype).cuda()
+    idx = HIPIndexer(nl, 1, bf, layout=layout).build(k, v)
+    s = torch.matmul(q.reshape(t, g, d).float(), k[0].float().transpose(1, 2).contiguous()).reshape(t * g, n)
+    tau = s.topk(max(1, n // 20), dim=1).values[:, -1].contiguous()
+    tau[0] = float("inf") if t * g > 1 else tau[0]
+    tau[-1] = float("-inf")
+    qk = qv = None
+    if m:
+        qk, qv = (torch.randn(t, m, w, generator=gen).to(dtype).cuda() for w in (d, dv))
+    sc = torch.full((t * g,), d ** -0.5, device="cuda")
+    one, gen_way = HIPSearcher(kernel=1), HIPSearcher(kernel=1, nodes_per_wave=3)
+    turned = torch.arange(t).repeat(g) if t > 1 else None
+    for q2kv in (None, turned):
+        out = []
+        for se in (one, gen_way):
+            st = torch.zeros((t, 11), dtype=torch.int64, device="cuda")
+            dense = se.search(q, tau, idx, q_head_to_kv=q2kv, scaling=sc, stats=st).clone()
+            pos = se.search(q, tau, idx, q_head_to_kv=q2kv, index_space="position").clone()
+            at, score, count = (x.clone() for x in se.search_compact(q, tau, idx, q_head_to_kv=q2kv))
+            by = torch.full((t * g, idx.size[0]), -9.0, device="cuda")
+            for h in range(t * g):
+                by[h, at[h, : count[h]].long()] = score[h, : count[h]]
+            att = se.search_attention(q, tau, idx, q_head_to_kv=q2kv, scaling=sc, queue_keys=qk, queue_values=qv)
+            out.append((dense, pos, by, count, st, att))
+        for a, b in zip(out[0][:5], out[1][:5]):
+            assert torch.equal(a, b)
+        a, b = out[0][5], out[1][5]
+        assert float((a - b).abs().max()) <= 1e-5 * float(b.abs().max())  # (sums of fp32 in another order)
+    slot = int((idx.perm[0] >= 0).nonzero()[0])
+    idx.values_buf[0, slot] = float("inf")
+    if not idx.tiled:
+        idx.keys_buf[0, slot + (idx.perm[0, slot + 1] >= 0).int().item()] = float("nan")
+    a, b = (se.search_attention(q, tau, idx, scaling=sc, queue_keys=qk, queue_values=qv) for se in (one, gen_way))
+    assert torch.equal(a.isfinite(), b.isfinite()) and torch.equal(a.isnan(), b.isnan())
