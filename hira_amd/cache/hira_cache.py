@@ -90,7 +90,7 @@ class HiraCacheLayer(CacheLayerMixin):
             raise NotImplementedError(f"Device mode {self.device_mode} not supported yet")
         self.indexed_len = 0
         self.queued_len = 0
-        self._update_takes_sync = None
+        self._update_takes = None
 
     def _alloc_queue(self, rows: int):
         """Room for `rows` queued keys and values per head, allocated once (the reference
@@ -228,34 +228,38 @@ class HiraCacheLayer(CacheLayerMixin):
             dst.data_ptr(), self._queue_type, self.dim, dst.shape[0], dst.shape[1], src.data_ptr(), rows,
             stride, arr(*slots), arr(*which), len(which), _lib.stream_of(dst.get_device())))
 
-    def _refresh_samples(self, new_keys, seen: int):
+    def _sample_pairs(self, new_keys, seen: int):
         """Keep the sample uniform over all indexed keys as the index grows (reservoir
         sampling, the same positions for every head): key number i (0-based) of the sequence
         joins with probability S/(i+1) in place of a random member; while the sample is still
-        smaller than S every new key joins."""
+        smaller than S every new key joins.  Returns the members to replace and the new keys that
+        do, a member each at most."""
         if self.samples is None:
-            return
+            return (), ()
         k4 = new_keys if new_keys.ndim == 4 else new_keys[None]
-        m = k4.shape[-2]
+        m, first = k4.shape[-2], 0
         room = self._sample_target - self.samples.shape[1]
         if room > 0:  # a short prompt: the sample holds every key so far
-            take = min(room, m)
-            rows = k4.narrow(2, 0, take).reshape(-1, take, self.dim).to(self.samples.dtype)
+            first = min(room, m)
+            rows = k4.narrow(2, 0, first).reshape(-1, first, self.dim).to(self.samples.dtype)
             self.samples = torch.cat([self.samples, rows], dim=1).contiguous()
             self._sample_facts()
-            if take == m:
-                return
-            k4, seen, m = k4.narrow(2, take, m - take), seen + take, m - take
-        s = self.samples.shape[1]
-        draws = torch.rand(m, generator=self._sample_gen).tolist()
-        who = [i for i, u in enumerate(draws) if u < s / (seen + i + 1)]
+            if first == m:
+                return (), ()
+        s, seen = self.samples.shape[1], seen + first
+        draws = torch.rand(m - first, generator=self._sample_gen).tolist()
+        who = [first + i for i, u in enumerate(draws) if u < s / (seen + i + 1)]
         if not who:
-            return
+            return (), ()
         slots = torch.randint(0, s, (len(who),), generator=self._sample_gen).tolist()
         # a slot drawn twice keeps its last arrival
         last = dict(zip(slots, who))
-        smp = self.samples
-        src = k4
+        return tuple(last.keys()), tuple(last.values())
+
+    def _replace_sampled(self, new_keys, slots, which):
+        """The members `slots` of the sample replaced by rows `which` of the new keys."""
+        src = new_keys if new_keys.ndim == 4 else new_keys[None]
+        m, smp = src.shape[-2], self.samples
         if smp.is_cuda and self._queue_type is not None:
             # one launch, the lists travel with its arguments.  (The rows of a head must lie one
             # behind the other and the heads evenly spaced, as the queue's and a model's do.)
@@ -269,11 +273,10 @@ class HiraCacheLayer(CacheLayerMixin):
                 # (clone: contiguous() would hand back a misaligned tensor as it is)
                 src = src.clone(memory_format=torch.contiguous_format)
                 step = m * self.dim
-            stride = step // self.dim
-            self._replace_rows(smp, src, m, stride, last.keys(), last.values())
+            self._replace_rows(smp, src, m, step // self.dim, slots, which)
             return
         rows = src.reshape(-1, m, self.dim).to(smp.dtype)
-        smp[:, torch.tensor(list(last.keys()))] = rows[:, torch.tensor(list(last.values()))].to(smp.device)
+        smp[:, torch.tensor(slots)] = rows[:, torch.tensor(which)].to(smp.device)
 
     def _sample_facts(self):
         """The rule as every output of the layer carries it."""
@@ -301,15 +304,22 @@ class HiraCacheLayer(CacheLayerMixin):
         # no read-back of the level sizes: the host carries their bounds (HIPIndexer.update,
         # sync=False), so folding the queue into the index does not wait for the GPU; a
         # one-level index has no node counts to bound with and keeps the synchronous form
-        if self._update_takes_sync is None:
+        if self._update_takes is None:
             import inspect
 
-            self._update_takes_sync = "sync" in inspect.signature(self.indexer.update).parameters
-        if self._update_takes_sync:
-            self.indexer.update(keys, values, sync=getattr(self.indexer, "num_levels", 1) < 2)
-        else:  # an indexer with the reference's two-argument update
-            self.indexer.update(keys, values)
-        self._refresh_samples(keys, self.indexed_len)
+            self._update_takes = inspect.signature(self.indexer.update).parameters.keys()
+        kw = {}
+        if "sync" in self._update_takes:  # (an indexer with the reference's update takes the rows alone)
+            kw["sync"] = getattr(self.indexer, "num_levels", 1) < 2
+        slots, which = self._sample_pairs(keys, self.indexed_len)
+        if slots and "sample" in self._update_takes and self.samples.is_cuda and \
+                self.samples.dtype is getattr(self.indexer, "dtype", None):
+            # the sample's new members go with the append
+            kw["sample"] = (self.samples, slots, which)
+            slots = ()
+        self.indexer.update(keys, values, **kw)
+        if slots:
+            self._replace_sampled(keys, slots, which)
         self.indexed_len += keys.shape[-2]
 
     def get_mask_sizes(self, cache_position):

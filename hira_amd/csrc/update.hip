@@ -71,6 +71,28 @@ __device__ __forceinline__ void touch_update_arguments() {
         : "memory");
 }
 
+// Rows of a key sample that new keys of the same call take the place of, in workgroups behind the trees':
+// dst[t][slot[i]] = new_keys[t][from[i]].  They share nothing with the append, and a launch of their own costs
+// the host and the GPU more than they do (a token that goes into the index at once, 2 trees of 64 bf16 columns:
+// 6.9 us for the append and, behind a gap of 1.2, 2.0 for the sample; together 7.0).  The pairs travel with the
+// arguments.
+constexpr int kSamplePairs = 32;
+struct SampleRows {
+    uint4* dst;
+    int32_t trees, chunks, rows_per_tree, n;  // trees: the workgroups that append
+    int32_t slot[kSamplePairs], from[kSamplePairs];
+};
+
+template <int NT>
+__device__ __forceinline__ void replace_sample(const UpdateParams& p, const SampleRows& r) {
+    const int i = ((int)blockIdx.x - r.trees) * NT + (int)threadIdx.x;
+    if (i >= r.trees * r.n * r.chunks) return;
+    const int row = i / r.chunks, c = i - row * r.chunks;  // row: tree * n + pair
+    const int t = row / r.n, k = row - t * r.n;
+    r.dst[((size_t)t * r.rows_per_tree + r.slot[k]) * r.chunks + c] =
+        reinterpret_cast<const uint4*>(p.new_keys)[((size_t)t * p.m + r.from[k]) * r.chunks + c];
+}
+
 // a bound must survive the fp32 rounding of the sums that produced it
 __device__ __forceinline__ float pad_up(float r) { return r > 0.0f ? r * (1.0f + 4.0f * 1.1920929e-7f) + 1e-30f : r; }
 
@@ -355,12 +377,16 @@ __device__ __forceinline__ void update_one_key(const UpdateParams& p, const int 
 }
 
 template <typename T>
-__global__ __launch_bounds__(kUpdThreads) void k_update(const UpdateParams p) {
+__global__ __launch_bounds__(kUpdThreads) void k_update(const UpdateParams p, const SampleRows sample) {
     extern __shared__ float sm[];
     __shared__ float red_f[4];
     __shared__ int red_i[4];
     __shared__ float s_dist[HIRA_MAX_LEVELS], s_rad[HIRA_MAX_LEVELS];
     touch_update_arguments();
+    if ((int)blockIdx.x >= sample.trees) {  // uniform in the workgroup
+        replace_sample<kUpdThreads>(p, sample);
+        return;
+    }
     for (int i = 0; i < p.m; ++i)
         update_one_key<T, kUpdThreads>(p, (int)blockIdx.x, i, sm, red_f, red_i, s_dist, s_rad);
 }
@@ -879,7 +905,7 @@ __device__ __forceinline__ int open_listed(const UpdateParams& p, const int tree
 }
 
 template <typename T, int COLS>
-__global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParams p) {
+__global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParams p, const SampleRows sample) {
     // 2 D floats of the general way, kCandMax centres, the table of distances, kParents centres, a chunk of key rows
     extern __shared__ __attribute__((aligned(16))) float sm[];
     constexpr int NT = kWinThreads;
@@ -892,6 +918,10 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
     __shared__ bool s_room;           // a listed node has room
     __shared__ int s_used[HIRA_MAX_LEVELS];  // slots in use per level
     touch_update_arguments();
+    if ((int)blockIdx.x >= sample.trees) {  // uniform in the workgroup
+        replace_sample<kWinThreads>(p, sample);
+        return;
+    }
     constexpr int EPL = Elem<T>::kPerChunk;
     const int tree = blockIdx.x;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -1225,10 +1255,15 @@ static int update_arguments(const HiraTree* tree, const void* new_keys, const vo
     return HIRA_OK;
 }
 
+// workgroups: one a tree, and as many as the sample's rows take
+static unsigned update_grid(const SampleRows& r, int threads) {
+    return (unsigned)(r.trees + (r.trees * r.n * r.chunks + threads - 1) / threads);
+}
+
 // The window kernel's LDS, its own lists beside the dynamic part, can exceed what a launch gets
 // without asking: asked for once per kernel and device.
 template <typename T, int COLS>
-static int launch_update_window(const UpdateParams& p, int trees, size_t smem, hipStream_t s) {
+static int launch_update_window(const UpdateParams& p, const SampleRows& sample, size_t smem, hipStream_t s) {
     constexpr int kMaxDevices = 64;
     static int asked[kMaxDevices];
     int dev = 0;
@@ -1240,7 +1275,8 @@ static int launch_update_window(const UpdateParams& p, int trees, size_t smem, h
             return fail(HIRA_ELAUNCH, "update: %zu bytes of LDS refused", kWinLds);
         __atomic_store_n(&asked[dev], 1, __ATOMIC_RELAXED);
     }
-    hipLaunchKernelGGL((k_update_window<T, COLS>), dim3(trees), dim3(kWinThreads), smem, s, p);
+    hipLaunchKernelGGL((k_update_window<T, COLS>), dim3(update_grid(sample, kWinThreads)), dim3(kWinThreads), smem, s, p,
+                       sample);
     return HIRA_OK;
 }
 
@@ -1270,28 +1306,62 @@ extern "C" int hira_update_state(const HiraTree* tree, int32_t num_keys, int32_t
     return HIRA_OK;
 }
 
+static int update_launch(const HiraTree* tree, const UpdateParams& p, const SampleRows& sample, bool window, size_t smem,
+                         size_t smem_w, hipStream_t s) {
+    if (window) {
+        const int rc = tree->dtype == HIRA_F32
+                           ? launch_update_window<float, 4>(p, sample, smem_w, s)
+                           : tree->dim <= 256 ? launch_update_window<bf16_t, 4>(p, sample, smem_w, s)
+                                              : launch_update_window<bf16_t, kWinColsMax>(p, sample, smem_w, s);
+        if (rc != HIRA_OK) return rc;
+    } else {
+        const dim3 grid(update_grid(sample, kUpdThreads)), block(kUpdThreads);
+        if (tree->dtype == HIRA_F32) hipLaunchKernelGGL(k_update<float>, grid, block, smem, s, p, sample);
+        else hipLaunchKernelGGL(k_update<bf16_t>, grid, block, smem, s, p, sample);
+    }
+    HIRA_CHECK_LAUNCH("update kernel");
+    return HIRA_OK;
+}
+
 /* see include/hira_hip.h */
 extern "C" int hira_update(const HiraTree* tree, const void* new_keys, const void* new_values,
                            int32_t m, int32_t* state, void* stream) {
+    return hira_update_sample(tree, new_keys, new_values, m, state, nullptr, 0, nullptr, nullptr, 0, stream);
+}
+
+/* see include/hira_hip.h */
+extern "C" int hira_update_sample(const HiraTree* tree, const void* new_keys, const void* new_values, int32_t m,
+                                  int32_t* state, void* sample, int32_t rows_per_tree, const int32_t* slot_host,
+                                  const int32_t* from_host, int32_t n, void* stream) {
     UpdateParams p;
     bool window;
     size_t smem, smem_w;
     if (const int rc = update_arguments(tree, new_keys, new_values, m, state, &p, &window, &smem, &smem_w))
         return rc;
-    if (m == 0) return HIRA_OK;
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (window) {
-        const int rc = tree->dtype == HIRA_F32
-                           ? launch_update_window<float, 4>(p, tree->num_trees, smem_w, s)
-                           : tree->dim <= 256 ? launch_update_window<bf16_t, 4>(p, tree->num_trees, smem_w, s)
-                                              : launch_update_window<bf16_t, kWinColsMax>(p, tree->num_trees, smem_w, s);
-        if (rc != HIRA_OK) return rc;
-    } else if (tree->dtype == HIRA_F32) {
-        hipLaunchKernelGGL(k_update<float>, dim3(tree->num_trees), dim3(kUpdThreads), smem, s, p);
-    } else {
-        hipLaunchKernelGGL(k_update<bf16_t>, dim3(tree->num_trees), dim3(kUpdThreads), smem, s, p);
+    SampleRows r;
+    memset(&r, 0, sizeof(r));
+    r.trees = tree->num_trees;
+    HIRA_CHECK_ARG(n >= 0 && (n == 0 || (sample && slot_host && from_host)), "hira_update_sample: null argument");
+    for (int i = 0; i < n; ++i)
+        HIRA_CHECK_ARG(slot_host[i] >= 0 && slot_host[i] < rows_per_tree && from_host[i] >= 0 && from_host[i] < m,
+                       "hira_update_sample: row %d from %d", slot_host[i], from_host[i]);
+    const int row = tree->dim * (tree->dtype == HIRA_F32 ? 4 : 2);
+    // (the launch takes a few rows, whole and aligned, each slot once; otherwise a launch of their own behind it)
+    const bool along = n > 0 && n <= kSamplePairs && row % 16 == 0 && (((uintptr_t)sample | (uintptr_t)new_keys) & 15) == 0 &&
+                       (int64_t)tree->num_trees * n * (row / 16) < (int64_t)1 << 31;
+    if (along) {
+        r.dst = static_cast<uint4*>(sample);
+        r.chunks = row / 16;
+        r.rows_per_tree = rows_per_tree;
+        r.n = n;
+        memcpy(r.slot, slot_host, n * sizeof(int32_t));
+        memcpy(r.from, from_host, n * sizeof(int32_t));
     }
-    HIRA_CHECK_LAUNCH("update kernel");
+    if (m > 0)
+        if (const int rc = update_launch(tree, p, r, window, smem, smem_w, reinterpret_cast<hipStream_t>(stream))) return rc;
+    if (n > 0 && !along)
+        return hira_replace_rows(sample, tree->dtype, tree->dim, tree->num_trees, rows_per_tree, new_keys, m, m, slot_host,
+                                 from_host, n, stream);
     return HIRA_OK;
 }
 

@@ -782,6 +782,31 @@ class HIPIndexer(BaseIndexer):
             return x
         return x.to(device=self.device, dtype=self.dtype).reshape(t, m, width).contiguous()
 
+    def _sample_args(self, sample):
+        """(address, rows a tree, slots, which, their number) of ``update``'s sample for the library."""
+        if sample is None:
+            return None, 0, None, None, 0
+        rows, slots, which = sample
+        if rows.dtype is not self.dtype or rows.get_device() != self.keys_buf.get_device() or \
+                rows.ndim != 3 or rows.shape[0] != self.num_trees or rows.shape[2] != self.dim or \
+                not rows.is_contiguous() or len(slots) != len(which):
+            raise ValueError(f"sample must be contiguous ({self.num_trees}, S, {self.dim}) {self.dtype} rows "
+                             "on the index's device with as many slots as keys")
+        n = len(slots)
+        arr = C.c_int32 * n
+        return rows.data_ptr(), rows.shape[1], arr(*slots), arr(*which), n
+
+    def _replace_sample(self, sample, new_keys: torch.Tensor, m: int) -> "HIPIndexer":
+        rows, per_tree, slots, which, n = self._sample_args(sample)
+        if n:
+            kin = self._rows(new_keys, self.num_trees, m, self.dim)
+            if kin.data_ptr() % 16:
+                kin = kin.clone()
+            _lib.check(_lib.lib().hira_replace_rows(
+                rows, _DTYPES[self.dtype], self.dim, self.num_trees, per_tree, kin.data_ptr(), m, m, slots,
+                which, n, _lib.stream_of(self.keys_buf.get_device())))
+        return self
+
     def reserve(self, appends: int) -> "HIPIndexer":
         """Room for `appends` more keys per tree, so that updates up to that many do not
         re-allocate: device pointers (and with them captured graphs and plans) stay valid."""
@@ -856,7 +881,7 @@ class HIPIndexer(BaseIndexer):
             self._sizes_changed()
 
     def update(self, new_keys: torch.Tensor, new_values: Optional[torch.Tensor] = None, *,
-               sync: bool = True):
+               sync: bool = True, sample=None):
         """Append new_keys (1, H, m, D) (and new_values (1, H, m, Dv)) in order
         (indexer/cuda.py:544-701).  One launch; afterwards the level sizes are read back
         (one small device-to-host copy), as the next search needs them.
@@ -865,7 +890,11 @@ class HIPIndexer(BaseIndexer):
         sizes (slots past a tree's real size hold nodes without children, which every search
         prunes at once), nothing waits for the stream, and with ``reserve`` called beforehand
         the call is a single launch on fixed pointers, fit for a captured graph.
-        ``sync_sizes`` (or the next update with ``sync=True``) brings the exact sizes back."""
+        ``sync_sizes`` (or the next update with ``sync=True``) brings the exact sizes back.
+
+        ``sample`` = (rows (T, S, D) of the index's type on its device, contiguous; slots; which): row
+        slots[i] of every tree's key sample is replaced by new key which[i], beside the append (no
+        slot twice)."""
         if self.keys_buf is None:
             raise ValueError("Indexer is not built: call build() first.")
         if new_keys.ndim != 4 or new_keys.shape[0] != self.batch or \
@@ -888,14 +917,17 @@ class HIPIndexer(BaseIndexer):
             full = self.graft_min if self.graft_min is not None else max(256, bf ** (nl - 1) // 2)
             part = self.graft_min if self.graft_min is not None else max(256, bf ** (nl - 2) // 2)
             if m >= full:
-                return self._graft(new_keys, new_values, m, nl, None)
+                self._graft(new_keys, new_values, m, nl, None)
+                return self._replace_sample(sample, new_keys, m)
             if nl >= 3 and m >= part:
                 # a mid-size window: further children of an existing root where every tree has
                 # one with room, else a new root (whose free child slots take the next ones)
                 where = self._room_under_a_root(new_keys, m)
                 if where is not None:
-                    return self._graft(new_keys, new_values, m, nl - 1, where)
-                return self._graft(new_keys, new_values, m, nl, None)
+                    self._graft(new_keys, new_values, m, nl - 1, where)
+                else:
+                    self._graft(new_keys, new_values, m, nl, None)
+                return self._replace_sample(sample, new_keys, m)
         if not sync and 0 < self._unsynced_room < m:  # (checked before anything is launched)
             raise RuntimeError("more appends than begin_unsynced made room for")
         need = self._needed_caps(m)
@@ -906,9 +938,13 @@ class HIPIndexer(BaseIndexer):
         kin = self._rows(new_keys, t, m, self.dim)
         vin = None if new_values is None else self._rows(new_values, t, m, self.vdim)
         tree = self.tree_struct()
-        rc = _lib.lib().hira_update(C.byref(tree), kin.data_ptr(),
-                                    None if vin is None else vin.data_ptr(), m,
-                                    self._state.data_ptr(), _lib.stream_of(self.keys_buf.get_device()))
+        rows, per_tree, slots, which, n = self._sample_args(sample)
+        if n and kin.data_ptr() % 16:  # (whole chunks of rows move there)
+            kin = kin.clone()
+        rc = _lib.lib().hira_update_sample(C.byref(tree), kin.data_ptr(),
+                                           None if vin is None else vin.data_ptr(), m,
+                                           self._state.data_ptr(), rows, per_tree, slots, which, n,
+                                           _lib.stream_of(self.keys_buf.get_device()))
         if rc:
             _lib.check(rc)
         self.num_keys += m

@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define HIRA_ABI_VERSION 10
+#define HIRA_ABI_VERSION 11
 #define HIRA_MAX_LEVELS 8
 #define HIRA_STATS_COLS (HIRA_MAX_LEVELS + 3) /* counters per tree a search can fill in */
 
@@ -308,6 +308,17 @@ int hira_nearest(const void* x, int32_t dtype, int32_t num_trees, int32_t n,
  */
 int hira_update(const HiraTree* tree, const void* new_keys, const void* new_values, int32_t m,
                 int32_t* state, void* stream);
+
+/*
+ * hira_update, and beside it a few rows of every tree's key sample replaced by new keys (as
+ * hira_replace_rows does, which the reservoir of the cache layer's thresholds needs after every
+ * append): sample[t][slot_host[i]] = new_keys[t][from_host[i]] for i < n, the sample (T,
+ * rows_per_tree, D) in the tree's dtype, every slot at most once.  Up to 32 rows go with the
+ * append's launch.  n = 0: hira_update.
+ */
+int hira_update_sample(const HiraTree* tree, const void* new_keys, const void* new_values, int32_t m,
+                       int32_t* state, void* sample, int32_t rows_per_tree, const int32_t* slot_host,
+                       const int32_t* from_host, int32_t n, void* stream);
 
 /* The initial state of every tree, as described above, from tree->size and the number of keys
  * inserted so far: on the stream, without a copy from the host that would wait for it. */

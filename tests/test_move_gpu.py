@@ -154,3 +154,27 @@ def test_rows_of_the_wrong_shape_are_refused(gpu_device):
     with pytest.raises(ValueError):
         _lib.check(_lib.lib().hira_enqueue(prompt.data_ptr(), prompt.data_ptr(), _lib.HIRA_BF16, 2, 500, 0, 1, 64, 64,
                                            odd.data_ptr(), row.data_ptr(), _lib.current_stream(row.device)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,n,d", [(1, 1, 64), (3, 3, 72), (4, 1, 128), (40, 32, 128), (40, 33, 64), (600, 50, 64)])
+def test_an_append_replaces_members_of_a_sample(dtype, m, n, d, gpu_device):
+    """The same index as an append alone, and the sample's rows replaced: key by key, as a window, more rows
+    than go with the launch, a window that is grafted."""
+    from hira_amd.indexer import HIPIndexer
+
+    k, v = torch.randn(2, 1, 3, 900 + m, d, device="cuda").to(dtype)
+    alone, both = (HIPIndexer(3, 1, 16).build(k[:, :, :900], v[:, :, :900]) for _ in range(2))
+    sample = torch.randn(3, 70, d, device="cuda").to(dtype)
+    slots, which = torch.randperm(70)[:n].tolist(), torch.randint(0, m, (n,)).tolist()
+    want = sample.clone()
+    want[:, slots] = k[0, :, 900:][:, which]
+    alone.update(k[:, :, 900:], v[:, :, 900:])
+    both.update(k[:, :, 900:], v[:, :, 900:], sample=(sample, slots, which))
+    assert torch.equal(sample, want)
+    assert both.size == alone.size
+    for a, b in zip([alone.perm, alone.keys_buf, alone.values_buf] + alone.centers[1:] + alone.radii[1:] + alone.counts[1:],
+                    [both.perm, both.keys_buf, both.values_buf] + both.centers[1:] + both.radii[1:] + both.counts[1:]):
+        assert torch.equal(a, b)
+    with pytest.raises(ValueError):
+        both.update(k[:, :, 900:], v[:, :, 900:], sample=(sample, [70], [0]))
