@@ -13,7 +13,9 @@ releases are provided: ``get_max_cache_shape`` (reference, cache/hira_cache.py:1
 from __future__ import annotations
 
 import ctypes as C
+import inspect
 from dataclasses import dataclass
+from functools import lru_cache
 from typing import Any
 
 import torch
@@ -27,6 +29,15 @@ from hira_amd.searcher import HIPSearcher
 # names the reference binds in this module (tests patch them there)
 CUDAIndexer = HIPIndexer
 CUDASearcher = HIPSearcher
+
+
+@lru_cache(maxsize=64)
+def _parameters(function) -> frozenset:
+    """Names of a function's parameters (looked up once: the look costs as much as a token's launches)."""
+    try:
+        return frozenset(inspect.signature(function).parameters)
+    except (TypeError, ValueError):
+        return frozenset()
 
 
 @dataclass
@@ -216,17 +227,17 @@ class HiraCacheLayer(CacheLayerMixin):
                 self._whole_rows(k4, n, self.dim, self._queue_k):
             # the positions travel with the launches: nothing waits for the build
             self.samples = torch.empty((k4.shape[0] * k4.shape[1], s, self.dim), dtype=store, device=k4.device)
-            self._replace_rows(self.samples, k4, n, n, range(s), pick.tolist())
+            at = torch.arange(s, dtype=torch.int32), pick.to(torch.int32)
+            self._replace_rows(self.samples, k4, n, n, *(C.cast(x.data_ptr(), C.POINTER(C.c_int32)) for x in at), s)
             return
         self.samples = k4[:, :, pick.to(k4.device)].reshape(-1, s, self.dim).to(store).contiguous()
 
-    def _replace_rows(self, dst, src, rows: int, stride: int, slots, which):
-        """dst[t][slots[i]] = src[t][which[i]] for every tree t; src holds `rows` rows a tree, `stride`
-        rows apart."""
-        arr = C.c_int32 * len(which)
+    def _replace_rows(self, dst, src, rows: int, stride: int, slots, which, n: int):
+        """dst[t][slots[i]] = src[t][which[i]] for every tree t and i < n (arrays of 32-bit numbers in host
+        memory, read before the call returns); src holds `rows` rows a tree, `stride` rows apart."""
         _lib.check(_lib.lib().hira_replace_rows(
             dst.data_ptr(), self._queue_type, self.dim, dst.shape[0], dst.shape[1], src.data_ptr(), rows,
-            stride, arr(*slots), arr(*which), len(which), _lib.stream_of(dst.get_device())))
+            stride, slots, which, n, _lib.stream_of(dst.get_device())))
 
     def _sample_pairs(self, new_keys, seen: int):
         """Keep the sample uniform over all indexed keys as the index grows (reservoir
@@ -273,7 +284,8 @@ class HiraCacheLayer(CacheLayerMixin):
                 # (clone: contiguous() would hand back a misaligned tensor as it is)
                 src = src.clone(memory_format=torch.contiguous_format)
                 step = m * self.dim
-            self._replace_rows(smp, src, m, step // self.dim, slots, which)
+            arr = C.c_int32 * len(which)
+            self._replace_rows(smp, src, m, step // self.dim, arr(*slots), arr(*which), len(which))
             return
         rows = src.reshape(-1, m, self.dim).to(smp.dtype)
         smp[:, torch.tensor(slots)] = rows[:, torch.tensor(which)].to(smp.device)
@@ -305,9 +317,8 @@ class HiraCacheLayer(CacheLayerMixin):
         # sync=False), so folding the queue into the index does not wait for the GPU; a
         # one-level index has no node counts to bound with and keeps the synchronous form
         if self._update_takes is None:
-            import inspect
-
-            self._update_takes = inspect.signature(self.indexer.update).parameters.keys()
+            update = self.indexer.update
+            self._update_takes = _parameters(getattr(update, "__func__", update))
         kw = {}
         if "sync" in self._update_takes:  # (an indexer with the reference's update takes the rows alone)
             kw["sync"] = getattr(self.indexer, "num_levels", 1) < 2
@@ -389,16 +400,10 @@ class HiraCache(Cache):
     def _indexer_kwargs(hira_config: HiraConfig, group):
         """The configuration's indexer arguments, plus the heads per tree where the indexer in
         use takes them (one with the reference's constructor does not)."""
-        import inspect
-
         import hira_amd.cache.hira_cache as me
 
         kw = dict(hira_config.get_indexer_kwargs())
-        try:
-            params = inspect.signature(me.CUDAIndexer.__init__).parameters
-        except (TypeError, ValueError):
-            params = {}
-        if group is not None and "heads_per_tree" in params:
+        if group is not None and "heads_per_tree" in _parameters(me.CUDAIndexer.__init__):
             kw["heads_per_tree"] = group
         return kw
 

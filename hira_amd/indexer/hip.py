@@ -53,6 +53,7 @@ def from_tiled(x: torch.Tensor) -> torch.Tensor:
     return v.contiguous().reshape(t, r, d)
 
 
+_NO_SAMPLE = (None, 0, None, None, 0)
 _MINUS_INF = 0xFF800000  # the bits of an fp32 -inf
 
 
@@ -124,6 +125,14 @@ def choose_layout(request: str, dtype: torch.dtype, dim: int, vdim: int, num_lev
         and heads_per_tree >= Q8_AUTO_MIN_HEADS and n >= Q8_AUTO_MIN_KEYS)
     tiled = tile_ok and (request in ("tiled", "q8") or auto_tiled)
     return tiled, q8
+
+
+class _Append:
+    """What an append without a read-back found out and the next one of as many keys finds again: while the
+    tree's struct is the same (its arrays, capacities and size bounds) and `left` calls are not used
+    up, the bounds of the level sizes do not move and the capacities suffice."""
+
+    __slots__ = ("tree", "ref", "state", "dev", "m", "kshape", "vshape", "left")
 
 
 class HIPIndexer(BaseIndexer):
@@ -208,6 +217,7 @@ class HIPIndexer(BaseIndexer):
         self.counts: List[Optional[torch.Tensor]] = []
         self._tree_struct = None
         self._state: Optional[torch.Tensor] = None  # device-side bookkeeping of update()
+        self._append: Optional[_Append] = None
 
     # ------------------------------------------------------------------ reference views
     @property
@@ -351,7 +361,7 @@ class HIPIndexer(BaseIndexer):
         if specs:
             _fill_arrays(specs, t)
         self._tree_struct = None
-        self._state = None
+        self._state = self._append = None
 
     def tree_struct(self) -> _lib.HiraTree:
         """The C view of the tree; valid while this indexer's tensors are alive."""
@@ -629,7 +639,10 @@ class HIPIndexer(BaseIndexer):
     def _grow(self, need: List[int]) -> None:
         """Re-allocate the level arrays with at least `need` slots (doubling), keeping the
         contents.  A tile of 16 rows is contiguous, so a tiled matrix grows by rows too."""
-        if all(n <= c for n, c in zip(need, self.cap)):
+        for n, c in zip(need, self.cap):
+            if n > c:
+                break
+        else:
             return
         caps = []
         for l, (c, n) in enumerate(zip(self.cap, need)):
@@ -785,7 +798,7 @@ class HIPIndexer(BaseIndexer):
     def _sample_args(self, sample):
         """(address, rows a tree, slots, which, their number) of ``update``'s sample for the library."""
         if sample is None:
-            return None, 0, None, None, 0
+            return _NO_SAMPLE
         rows, slots, which = sample
         if rows.dtype is not self.dtype or rows.get_device() != self.keys_buf.get_device() or \
                 rows.ndim != 3 or rows.shape[0] != self.num_trees or rows.shape[2] != self.dim or \
@@ -895,6 +908,22 @@ class HIPIndexer(BaseIndexer):
         ``sample`` = (rows (T, S, D) of the index's type on its device, contiguous; slots; which): row
         slots[i] of every tree's key sample is replaced by new key which[i], beside the append (no
         slot twice)."""
+        a = self._append
+        if a is not None and not sync and a.tree is self._tree_struct and a.left > 0 and \
+                new_keys.shape == a.kshape and new_values is not None and new_values.shape == a.vshape and \
+                new_keys.dtype is self.dtype and new_values.dtype is self.dtype and \
+                new_keys.get_device() == a.dev and new_values.get_device() == a.dev and \
+                new_keys.is_contiguous() and new_values.is_contiguous() and \
+                (sample is None or new_keys.data_ptr() % 16 == 0):
+            rc = _lib.lib().hira_update_sample(
+                a.ref, new_keys.data_ptr(), new_values.data_ptr(), a.m, a.state, *self._sample_args(sample),
+                _lib.stream_of(a.dev))
+            if rc:
+                _lib.check(rc)
+            a.left -= 1
+            self.num_keys += a.m
+            self._pending += a.m
+            return self
         if self.keys_buf is None:
             raise ValueError("Indexer is not built: call build() first.")
         if new_keys.ndim != 4 or new_keys.shape[0] != self.batch or \
@@ -962,6 +991,13 @@ class HIPIndexer(BaseIndexer):
         if bound != self.size:
             self.size = bound
             self._sizes_changed()
+        self._append = None
+        if self._unsynced_room == 0 and new_values is not None:
+            a = self._append = _Append()
+            a.tree, a.state, a.dev, a.m = self.tree_struct(), self._state.data_ptr(), self.keys_buf.get_device(), m
+            a.ref, a.kshape, a.vshape = C.byref(a.tree), new_keys.shape, new_values.shape
+            # (a new level-1 node at most every `bf` keys: the bounds move when the next one may be)
+            a.left = -self._pending % self.branching_factor // m
         return self
 
     _warmed: set = set()

@@ -155,21 +155,21 @@ class HIPSearcher(BaseSearcher):
         hit = self._map_cache.get(key)
         if hit is not None:
             return hit
-        group = 0
         if q_head_to_kv is None:
             if h_q % batch:
                 raise ValueError(f"H_q={h_q} not divisible by batch={batch}")
             per_seq = h_q // batch
-            if per_seq == h_kv:
-                local = torch.arange(per_seq)
-            else:
-                if per_seq % h_kv:
-                    raise ValueError(
-                        f"Unsupported head mapping: H_q={per_seq} must equal or be divisible "
-                        f"by H_kv={h_kv}")
-                local = torch.arange(per_seq) // (per_seq // h_kv)
-            m = (torch.arange(batch)[:, None] * h_kv + local[None, :]).reshape(-1)
-            group = per_seq // h_kv  # head h of the launch belongs to tree h // group
+            if per_seq % h_kv:
+                raise ValueError(
+                    f"Unsupported head mapping: H_q={per_seq} must equal or be divisible "
+                    f"by H_kv={h_kv}")
+            # head h of the launch belongs to tree h // group: made on the device, nothing is copied there
+            group = per_seq // h_kv
+            val = (torch.arange(0, h_q + 1, group, dtype=torch.int32, device=indexer.device),
+                   torch.arange(h_q, dtype=torch.int32, device=indexer.device), group, group)
+            if not (val[0].is_cuda and torch.cuda.is_current_stream_capturing()):  # (its fill has not run yet)
+                self._map_cache = {key: val}
+            return val
         else:
             if not torch.is_tensor(q_head_to_kv):
                 raise TypeError(
@@ -184,7 +184,7 @@ class HIPSearcher(BaseSearcher):
         off = torch.zeros(t + 1, dtype=torch.int32)
         off[1:] = counts.cumsum(0).to(torch.int32)
         dev = indexer.device
-        val = (off.to(dev), order.to(torch.int32).to(dev), int(counts.max().item()), group)
+        val = (off.to(dev), order.to(torch.int32).to(dev), int(counts.max().item()), 0)
         self._map_cache = {key: val}
         return val
 

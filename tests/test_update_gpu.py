@@ -561,3 +561,35 @@ def test_warm_up_runs_the_first_use_paths_and_leaves_the_index_alone(dtype, d, b
     for l in range(1, nl):
         assert torch.equal(a.radii[l][:, : a.size[l]], b.radii[l][:, : a.size[l]])
     _check_tree(a, keys, keys)
+
+
+@pytest.mark.parametrize("bf,levels,m", [(4, 3, 1), (10, 5, 1), (16, 2, 5), (32, 3, 7)])
+def test_appends_that_describe_the_last_one_again(bf, levels, m, gpu_device):
+    """Appends without a read-back keep what the one before found out; against an index that finds out
+    anew every time: the same bounds after every call, and the same trees, with a window of another length,
+    a read-back and a stretch with fixed bounds in between."""
+    from hira_amd.indexer import HIPIndexer
+
+    k, v = torch.randn(2, 1, 2, 700 + 80 * m, 64, device="cuda").to(torch.bfloat16)
+    kept, anew = (HIPIndexer(levels, 1, bf).build(k[:, :, :700], v[:, :, :700]) for _ in range(2))
+    at = 700
+    for i in range(60):
+        w = 3 * m if i == 20 else m
+        for x in (kept, anew):
+            if x is anew:
+                x._append = None
+            if i == 30:
+                x.sync_sizes()
+            if i == 40:
+                x.begin_unsynced(6 * m)
+            if i == 46:
+                x.sync_sizes()
+            x.update(k[:, :, at:at + w].contiguous(), v[:, :, at:at + w].contiguous(), sync=False)
+        at += w
+        assert kept.size == anew.size and kept.cap == anew.cap and kept._pending == anew._pending
+    for x in (kept, anew):
+        x.sync_sizes()
+    assert kept.size == anew.size and kept.num_keys == anew.num_keys
+    for a, b in zip([kept.perm, kept.keys_buf, kept.values_buf] + kept.centers[1:] + kept.radii[1:] + kept.counts[1:],
+                    [anew.perm, anew.keys_buf, anew.values_buf] + anew.centers[1:] + anew.radii[1:] + anew.counts[1:]):
+        assert torch.equal(a, b)
