@@ -486,12 +486,12 @@ __device__ __forceinline__ size_t ancestor_of(size_t node1, int l, int bf) {
 // Reads the tree's level-1 nodes with room into LDS, and those of level 2.  cen: (kCandMax, D) floats, par:
 // (kParents, D).  Returns false (uniform) when there are more of level 1 than the list holds.
 template <typename T, int NT>
-__device__ __forceinline__ bool window_candidates(const UpdateParams& p, const int tree, WindowLds& w, float* cen, T* par) {
+__device__ __forceinline__ bool window_candidates(const UpdateParams& p, const int tree, const int st0, const int st1,
+                                                  const int st2, WindowLds& w, float* cen, T* par) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int D = p.dim, L = p.num_levels, bf = p.bf;
-    int32_t* st = p.state + (size_t)tree * (HIRA_MAX_LEVELS + 2);
-    const int used = st[1], first = min(max(st[0], 0), used);
-    const int used2 = L > 2 ? st[2] : 0;
+    const int used = st1, first = min(max(st0, 0), used);
+    const int used2 = L > 2 ? st2 : 0;
     const bool look2 = used2 <= kParentCounts * NT;
     const size_t b1 = (size_t)tree * p.cap[1];
     if (t == 0) {
@@ -804,104 +804,185 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
     return node1;
 }
 
-// The same from the list of level-2 nodes, where one of them has room: the new level-1 node gets its place, its centre
-// (also to cen) and its parent's count, the path above its radii, and it becomes the list of candidates; the key's row
-// goes the way of all others (its slot to *slot).  Returns the node, or -1 (uniform, and nothing is changed): no node
-// of the list takes the key, or the slot lies behind the capacity.
+// All that is left of a chunk, keys [k, nk), once no listed node has room: from there on a key opens a node, the
+// bf - 1 behind it fill that one, whatever their distance, and the next opens another.  So everything is known but
+// the parents, and what was a chain of openings (parent, distances to the new node, choice: 4.6 us each) is one pass:
+// the openers' distances to the listed level-2 nodes and everybody's to its opener at once, the parents one after
+// the other by one wave, the paths above them together.  A window of 64 keys, two openings, 18.5 -> 12.3 us (with what the other waves do beside wave 0).
+// The new nodes then stand in the list as candidates do, take their counts and radii to memory as they do, and the
+// last one stays as the list.  The keys' rows go the way of all others (s_slot).  Returns the first key that is
+// left (k: none was placed): at one that no listed parent takes, whose node's slot lies behind the capacity, or
+// whose distance is no finite number.
 template <typename T, int NT>
-__device__ __forceinline__ int open_listed(const UpdateParams& p, const int tree, int* s_used, int* slot, const T* key, const T* par,
-                                           WindowLds& w, float* cen, float* s_dist, float* s_rad) {
+__device__ __forceinline__ int open_run(const UpdateParams& p, const int tree, int* s_used, int* s_slot, int* s_stop, const T* rows,
+                                        const T* par, WindowLds& w, float* cen, float* table, const int k, const int nk) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int D = p.dim, L = p.num_levels, bf = p.bf, n2 = w.n2;
     const size_t b1 = (size_t)tree * p.cap[1];
-    const int known = w.n == 1 ? w.anc_id[2][0] : -1;  // the level-2 node whose path the list still has
-    for (int e = wave; e < n2; e += NT / 64) {  // uniform in the wave
-        float ss = 0.0f;
-        for (int j = lane; j < D; j += 64) {
-            const float df = load_elem<T>(key, j) - load_elem<T>(par, (size_t)e * D + j);
-            ss += df * df;
-        }
+    const int most = min((nk - k + bf - 1) / bf, kCandMax);  // openers: keys k, k + bf, ...
+    const int end = min(nk, k + most * bf);
+    float* far = table + kCandMax * kParentsMax;  // (kWinKeys) squared distances to the openers
+    // (the additions are those of a butterfly of lane ^ 1, ^ 2, ..., ^ 32, the general way's)
+    auto total = [&](float ss) {
         ss += win_partner<1>(ss);
         ss += win_partner<2>(ss);
         ss += win_partner<4>(ss);
         ss += win_partner<8>(ss);
         ss = win_sum_across<16>(ss);
-        ss = win_sum_across<32>(ss);
-        if (lane == 0) w.d2[e] = w.cnt2[e] < bf && ss < INFINITY ? ss : INFINITY;
+        return win_sum_across<32>(ss);
+    };
+    auto apart = [&](const T* x, const T* y) {
+        float ss = 0.0f;
+        for (int j = lane; j < D; j += 64) {
+            const float df = load_elem<T>(x, j) - load_elem<T>(y, j);
+            ss += df * df;
+        }
+        return ss;
+    };
+    // (numbers below a few thousand: the float quotients are exact)
+    const float inv_bf = 1.0f / (float)bf, inv_n2 = 1.0f / (float)max(n2, 1);
+    auto over = [](int x, float inv) { return (int)(((float)x + 0.5f) * inv); };
+    // (wave 0 comes from taking the list before to memory, and asks for the parents' radii meanwhile)
+    constexpr int NW = NT / 64 - 1;
+    float rad2 = 0.0f;
+    if (wave == 0 && lane < n2) rad2 = p.radii[2][(size_t)tree * p.cap[2] + w.id2[min(lane, kParentsMax - 1)]];
+    for (int e = wave - 1; e < most * n2 && wave > 0; e += NW) {  // uniform in the wave
+        const int i = over(e, inv_n2), c = e - i * n2;
+        const float ss = total(apart(rows + (size_t)(k + i * bf) * D, par + (size_t)c * D));
+        if (lane == 0) table[i * kParentsMax + c] = ss;
+    }
+    for (int q0 = k + wave - 1; q0 < end && wave > 0; q0 += NW * 5) {  // uniform in the wave; five keys at a time
+        float ss[5];
+#pragma unroll
+        for (int u = 0; u < 5; ++u) {
+            const int q = min(q0 + u * NW, end - 1);
+            ss[u] = apart(rows + (size_t)q * D, rows + (size_t)(k + over(q - k, inv_bf) * bf) * D);
+        }
+#pragma unroll
+        for (int u = 0; u < 5; ++u) {
+            const int q = q0 + u * NW;
+            const float d = total(ss[u]);
+            if (lane == 0 && q < end) far[q - k] = over(q - k, inv_bf) * bf == q - k ? 0.0f : d;
+        }
     }
     __syncthreads();
-    const float d = lane < n2 ? w.d2[lane] : INFINITY;
-    const float best = win_min(d);
-    if (best == INFINITY) return -1;
-    int low = d == best ? w.id2[min(lane, kParentsMax - 1)] : 0x7fffffff;  // (ties: the lowest node)
-    unsigned long long who = __ballot(d == best);
-    if (who & (who - 1ull)) {
+    if (wave == 0) {
+        int cnt2 = lane < n2 ? w.cnt2[lane] : bf;
+        const int id2 = lane < n2 ? w.id2[min(lane, kParentsMax - 1)] : 0x7fffffff, had2 = cnt2;
+        const int grp = over(lane, inv_bf);  // of key k + lane
+        const float mine = lane < end - k ? far[lane] : 0.0f;
+        const unsigned long long bad = __ballot(!(mine < INFINITY));
+        int stop = bad != 0ull ? k + __ffsll((long long)bad) - 1 : end;
+        int n = 0, used = s_used[1];
+        for (; n < most && k + n * bf < stop; ++n) {
+            const float have = lane < n2 && cnt2 < bf ? table[n * kParentsMax + min(lane, kParentsMax - 1)] : INFINITY;
+            const float d = have < INFINITY ? have : INFINITY;
+            const float best = win_min(d);
+            if (best == INFINITY) break;
+            unsigned long long who = __ballot(d == best);
+            if (who & (who - 1ull)) {  // ties: the lowest node
+                int low = d == best ? id2 : 0x7fffffff;
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
-        who = __ballot(d == best && w.id2[min(lane, kParentsMax - 1)] == low);
-    }
-    const int c = __ffsll((long long)who) - 1, parent = w.id2[c], pcount = w.cnt2[c];
-    const long long idx = (long long)parent * bf + pcount;
-    if (idx >= p.cap[1] || idx * bf >= p.cap[0]) return -1;
-    for (int j = t; j < D; j += NT) {
-        const float x = load_elem<T>(key, j);
-        store_elem<T>(p.centers[1], b1 * D + elem_index(p.layout, D, (size_t)idx, j), x);
-        cen[j] = x;
-    }
-    const bool same_path = known == parent;
-    for (int l = same_path ? L : 2 + wave; l < L; l += NT / 64) {  // the path above: a wave per level
-        const size_t node = ancestor_of((size_t)parent, l - 1, bf);
-        const float rad_now = p.radii[l][(size_t)tree * p.cap[l] + node];
-        float ss = best;
-        if (l > 2) {
-            const size_t child = ancestor_of((size_t)parent, l - 2, bf);
-            const size_t bl = (size_t)tree * p.cap[l], bc = (size_t)tree * p.cap[l - 1];
-            ss = 0.0f;
-            for (int j = lane; j < D; j += 64) {
-                const float a = load_elem<T>(p.centers[l - 1], bc * D + elem_index(p.layout, D, child, j));
-                const float b = load_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, node, j));
-                ss += (a - b) * (a - b);
+                for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
+                who = __ballot(d == best && id2 == low);
             }
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+            const int c = __ffsll((long long)who) - 1;
+            const int parent = __builtin_amdgcn_readlane(id2, c);
+            const long long idx = (long long)parent * bf + __builtin_amdgcn_readlane(cnt2, c);
+            if (idx >= p.cap[1] || idx * bf >= p.cap[0]) break;
+            if (lane == c) ++cnt2;
+            used = max(used, (int)(idx + 1));
+            if (lane == 0) {
+                w.id[n] = (int)idx;
+                w.anc_id[2][n] = parent;
+                w.anc_step[2][n] = sqrtf(best);
+                w.anc_rad[2][n] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(rad2), c));
+            }
+        }
+        stop = min(stop, k + n * bf);
+        if (lane < n) {
+            w.cnt[lane] = min(bf, stop - k - lane * bf);
+            w.cnt0[lane] = 0;  // (memory has neither count nor radius of it)
+            w.rad[lane] = -INFINITY;
+            w.far[lane] = 0.0f;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        if (lane < stop - k) {
+            s_slot[k + lane] = w.id[grp] * bf + (lane - grp * bf);
+            atomicMax(reinterpret_cast<int*>(&w.far[grp]), __float_as_int(mine));  // (not negative: ordered as integers)
+        }
+        if (lane < n2 && cnt2 != had2) {
+            w.cnt2[lane] = cnt2;
+            p.counts[2][(size_t)tree * p.cap[2] + id2] = cnt2;
         }
         if (lane == 0) {
-            s_dist[l] = sqrtf(ss);
-            s_rad[l] = rad_now;
+            if (used != s_used[1]) s_used[1] = p.state[(size_t)tree * (HIRA_MAX_LEVELS + 2) + 1] = used;
+            w.n = n;
+            *s_stop = stop;
         }
-    }
-    if (t == 0) {
-        p.radii[1][b1 + idx] = 0.0f;
-        p.counts[1][b1 + idx] = 1;
-        p.counts[2][(size_t)tree * p.cap[2] + parent] = pcount + 1;
-        if (p.keps != nullptr) p.keps[b1 + idx] = 0.0f;  // (its keys' rows raise it)
-        if (idx + 1 > s_used[1]) s_used[1] = p.state[(size_t)tree * (HIRA_MAX_LEVELS + 2) + 1] = (int)(idx + 1);
-        *slot = (int)(idx * bf);
-        w.n = 1;
-        w.id[0] = (int)idx;
-        w.cnt[0] = w.cnt0[0] = 1;
-        w.rad[0] = 0.0f;
-        w.far[0] = -1.0f;
     }
     __syncthreads();
-    if (t == 0) {  // (nobody reads this until the next barrier)
-        w.cnt2[c] = pcount + 1;
-        float r_child = 0.0f;
-        size_t node = (size_t)parent;
-        for (int l = 2; l < L; ++l) {
-            const float have = same_path ? w.anc_rad[l][0] : s_rad[l];
-            const float step = l == 2 ? sqrtf(best) : (same_path ? w.anc_step[l][0] : s_dist[l]);
-            const float rn = fmaxf(have, pad_up(step + r_child));
-            if (rn != have) p.radii[l][(size_t)tree * p.cap[l] + node] = rn;
-            r_child = rn;
-            w.anc_id[l][0] = (int)node;
-            w.anc_rep[l][0] = 0;
-            w.anc_step[l][0] = step;
-            w.anc_rad[l][0] = rn;
-            node /= (size_t)bf;
+    const int n = w.n, stop = *s_stop;
+    if (n == 0) return k;  // uniform
+    for (int i = wave - 1; i < n && wave > 0; i += NW)  // uniform in the wave
+        for (int j = lane; j < D; j += 64) {
+            const float x = load_elem<T>(rows, (size_t)(k + i * bf) * D + j);
+            store_elem<T>(p.centers[1], b1 * D + elem_index(p.layout, D, (size_t)w.id[i], j), x);
+            if (i == n - 1) cen[j] = x;
+        }
+    if (p.keps != nullptr && t < n) p.keps[b1 + w.id[t]] = 0.0f;  // (its keys' rows raise it)
+    for (int e = wave; e < n * (L - 3); e += NT / 64) {  // the paths above level 2: a wave per node and level
+        const int i = e % n, l = 3 + e / n;
+        const size_t parent = (size_t)w.anc_id[2][i], node = ancestor_of(parent, l - 1, bf);
+        const size_t bl = (size_t)tree * p.cap[l];
+        const float rad_now = p.radii[l][bl + node];
+        const size_t child = ancestor_of(parent, l - 2, bf), bc = (size_t)tree * p.cap[l - 1];
+        float ss = 0.0f;
+        for (int j = lane; j < D; j += 64) {
+            const float a = load_elem<T>(p.centers[l - 1], bc * D + elem_index(p.layout, D, child, j));
+            const float b = load_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, node, j));
+            ss += (a - b) * (a - b);
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+        if (lane == 0) {
+            w.anc_id[l][i] = (int)node;
+            w.anc_step[l][i] = sqrtf(ss);
+            w.anc_rad[l][i] = rad_now;
         }
     }
-    return (int)idx;
+    if (L > 3) __syncthreads();  // uniform
+    if (wave == 0) {
+        for (int l = 2; l < L; ++l)
+            if (lane < n) {
+                const int anc = w.anc_id[l][lane];
+                int first = lane;
+                for (int o = lane - 1; o >= 0; --o) first = w.anc_id[l][o] == anc ? o : first;
+                w.anc_rep[l][lane] = first;
+            }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        window_flush(p, tree, w);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        if (lane == 0) {  // the last one is the list
+            const int c = n - 1;
+            w.n = 1;
+            w.id[0] = w.id[c];
+            w.cnt[0] = w.cnt0[0] = w.cnt[c];
+            w.rad[0] = pad_up(sqrtf(w.far[c]));
+            w.far[0] = -1.0f;
+            for (int l = 2; l < L; ++l) {
+                w.anc_id[l][0] = w.anc_id[l][c];
+                w.anc_step[l][0] = w.anc_step[l][c];
+                w.anc_rad[l][0] = w.anc_rad[l][w.anc_rep[l][c]];
+                w.anc_rep[l][0] = 0;
+            }
+        }
+    }
+    __syncthreads();
+    return stop;
 }
 
 template <typename T, int COLS>
@@ -961,10 +1042,13 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
         }
     };
     int position = st[HIRA_MAX_LEVELS];  // of the next key (every thread carries it along)
+    // (the state is asked for with the first rows, not behind them)
+    const int st0 = st[0], st1 = st[1], st2 = st[2], my_used = t < HIRA_MAX_LEVELS ? st[t] : 0;
     stage(0);
-    if (t >= 1 && t < L) s_used[t] = st[t];
+    if (t >= 1 && t < L) s_used[t] = my_used;
     int i0 = 0;
-    bool general = !window_candidates<T, NT>(p, tree, w, cen, par);  // uniform: what is left goes the general way
+    bool flushed = false;  // (wave 0's)
+    bool general = !window_candidates<T, NT>(p, tree, st0, st1, st2, w, cen, par);  // uniform: what is left goes the general way
     while (i0 < p.m && !general) {  // uniform
         int nk = min(kWinKeys, p.m - i0);
         bool list_anew = false;  // behind this chunk
@@ -1041,16 +1125,20 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
                 list_anew = s_room;
                 window_flush(p, tree, w);
                 const T* key = rows + (size_t)k * D;
-                int node = -1;
-                if (!list_anew && L > 2 && w.n2 <= kParents<T>)  // uniform
-                    node = open_listed<T, NT>(p, tree, s_used, &s_slot[k], key, par, w, cen, s_dist, s_rad);
-                if (node >= 0) {
-                    ++position;
-                } else {
+                if (!list_anew && L > 2 && w.n2 <= kParents<T>) {  // uniform
+                    const int k1 = open_run<T, NT>(p, tree, s_used, s_slot, &s_done, rows, par, w, cen, table, k, nk);
+                    if (k1 > k) {
+                        position += k1 - k;
+                        k = k1;
+                        if (k < nk) window_distances<T, COLS, NT>(D, w, cen, rows, k, nk, table);
+                        continue;
+                    }
+                }
+                {
                     // (with no room left in the list a node of level 2 is opened too, the only one there with room then)
                     bool none2 = w.n2 <= kParents<T>;
                     for (int e = 0; none2 && e < w.n2; ++e) none2 = w.cnt2[e] >= bf;
-                    node = open_node<T, NT>(p, tree, i0 + k, position, s_used, key, sm, red_f, red_i, s_dist, s_rad);
+                    const int node = open_node<T, NT>(p, tree, i0 + k, position, s_used, key, sm, red_f, red_i, s_dist, s_rad);
                     if (node >= 0) ++position;
                     if (list_anew) {  // uniform
                         nk = k + 1;
@@ -1099,21 +1187,28 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
             }
         const bool v_chunks = with_values && Dv % EPL == 0;
         const int vc = v_chunks ? Dv / EPL : 0, per = kc + vc;
+        // (behind the last chunk wave 0 takes the list to memory meanwhile)
+        const bool last = i0 + nk >= p.m && !list_anew;  // uniform
+        const int rt = last ? t - 64 : t, rn = last ? NT - 64 : NT;
+        if (last && wave == 0) {
+            window_flush(p, tree, w);
+            flushed = true;
+        }
         constexpr int RU = 4;  // chunks a thread has in flight
         const float inv_per = 1.0f / (float)per;  // (at most 64 x 128 chunks: the float quotient is exact)
-        for (int e0 = t; e0 < nk * per; e0 += RU * NT) {
+        for (int e0 = rt; e0 < nk * per && rt >= 0; e0 += RU * rn) {
             uint4 raw[RU];
             T* dst[RU];
 #pragma unroll
             for (int u = 0; u < RU; ++u) {
-                const int e = min(e0 + u * NT, nk * per - 1);
+                const int e = min(e0 + u * rn, nk * per - 1);
                 const int q = (int)(((float)e + 0.5f) * inv_per), c = e - q * per, slot = s_slot[q];
                 const size_t r = (size_t)tree * p.m + i0 + q;
                 const bool key = c < kc;
                 if (key) raw[u] = reinterpret_cast<const uint4*>(rows)[q * kc + c];
                 else if (vals != nullptr) raw[u] = vals[q * vc + c - kc];
                 else raw[u] = load_chunk<T>(p.new_values, r * Dv, c - kc);
-                dst[u] = slot < 0 || e0 + u * NT >= nk * per
+                dst[u] = slot < 0 || e0 + u * rn >= nk * per
                              ? nullptr
                              : (key ? reinterpret_cast<T*>(p.keys) + base0 * D + elem_index(p.key_layout, D, (size_t)slot, c * EPL)
                                     : reinterpret_cast<T*>(p.values) + (base0 + slot) * Dv + (c - kc) * EPL);
@@ -1166,7 +1261,7 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
         i0 += nk;
         if (list_anew) {  // uniform
             __syncthreads();
-            general = !window_candidates<T, NT>(p, tree, w, cen, par);
+            general = !window_candidates<T, NT>(p, tree, st[0], st[1], st[2], w, cen, par);
         }
         if (i0 < p.m) __syncthreads();
     }
@@ -1176,7 +1271,7 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
         for (; i0 < p.m; ++i0) update_one_key<T, NT>(p, tree, i0, sm, red_f, red_i, s_dist, s_rad);
         return;
     }
-    window_flush(p, tree, w);
+    if (!flushed) window_flush(p, tree, w);
     if (wave == 0) {
         // the bound of the next search for room: the lowest listed node that still has some, or
         // the lowest slot that was no node when the list was made
