@@ -159,10 +159,8 @@ __device__ __forceinline__ void emit_columns(const float (&v)[8], int j, int lan
             make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]),
                        pack_bf16(lo[6], lo[7]));
     }
-    for (int off = 1; off < lanes; off <<= 1) {
-        ss += __shfl_xor(ss, off, 64);
-        ls += __shfl_xor(ls, off, 64);
-    }
+    ss = group_sum_of(ss, lanes);
+    ls = group_sum_of(ls, lanes);
     if (have && j == 0) {
         ct.n2[(size_t)t * Kt * 16 + k] = usable ? ss : INFINITY;
         // (1e-5 of ||c|| per 32 columns: what the roundings of two sums of products can be worth)

@@ -71,8 +71,7 @@ __global__ __launch_bounds__(64) void k_cent_prep(const float* cent, int K, cons
             make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]),
                        pack_bf16(lo[6], lo[7]));
     }
-    ss += __shfl_xor(ss, 16, 64);
-    ss += __shfl_xor(ss, 32, 64);
+    ss = cross_group_sum<16>(ss);
     if (kb == 0) {
         const bool usable = k < K && !(fill != nullptr && fill[(size_t)t * K + k] >= bf);
         cn2[((size_t)t * Kt + tile) * 16 + i] = usable ? ss : INFINITY;
@@ -121,8 +120,7 @@ __global__ __launch_bounds__(kAssignThreads, 2) void k_assign_mfma(const AssignJ
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
         }
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
+        ss = cross_group_sum<16>(ss);
         x2[ri] = ss;
     }
     float best[RI][4];
@@ -331,8 +329,7 @@ __device__ __forceinline__ void split_items(const AssignJob& job, int Kt, int ti
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
         }
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
+        ss = cross_group_sum<16>(ss);
         x2[ri] = ss;
     }
     float best[RI];
@@ -581,13 +578,11 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     }
     constexpr int EPL = Elem<T>::kPerChunk;
     auto norms = [&](int ri, float ss, float ls) {  // (of this lane's columns)
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
+        ss = cross_group_sum<16>(ss);
         x2[ri] = ss;
         X = fmaxf(X, ss);
         if (SPLIT) {
-            ls += __shfl_xor(ls, 16, 64);
-            ls += __shfl_xor(ls, 32, 64);
+            ls = cross_group_sum<16>(ls);
             Xl = fmaxf(Xl, ls);
         }
     };
@@ -629,11 +624,8 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
             norms(ri, ss, ls);
         }
     }
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) {
-        X = fmaxf(X, __shfl_xor(X, off, 64));
-        if (SPLIT) Xl = fmaxf(Xl, __shfl_xor(Xl, off, 64));
-    }
+    X = lanes_fold<1, 16>(X, OpMax{});
+    if (SPLIT) Xl = lanes_fold<1, 16>(Xl, OpMax{});
     if (lane == 0) {
         s_x[wave] = X;
         s_x[WAVES + wave] = Xl;

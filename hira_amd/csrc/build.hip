@@ -806,7 +806,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_place(const PlaceLevel pl) {
                 }
             }
         }
-        for (int off = lpr; off < 64; off <<= 1) r = fmaxf(r, __shfl_xor(r, off, 64));
+        r = cross_group(r, lpr, OpMax{});
         if (lane == 0) {
             // a few ulp of head room: the bound must survive fp32 rounding of this sum
             if (r > 0.0f) r = r * (1.0f + 4.0f * 1.1920929e-7f) + 1e-30f;
@@ -822,7 +822,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_place(const PlaceLevel pl) {
 #pragma unroll
         for (int q = 0; q < EPL; ++q) {
             float m = big[q];
-            for (int off = lpr; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+            m = cross_group(m, lpr, OpMax{});
             if (rg == 0 && chunk_ok) s_abs[wave][ch * EPL + q] = m;
         }
         __syncthreads();
@@ -1320,11 +1320,8 @@ __global__ __launch_bounds__(256) void k_subtree_take(const HiraTree tree, int s
         total += live;
         before += i < first ? live : 0;
     }
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        before += __shfl_xor(before, off, 64);
-        total += __shfl_xor(total, off, 64);
-    }
+    before = lanes_fold<1, 64>(before, OpSum{});
+    total = lanes_fold<1, 64>(total, OpSum{});
     if (lane == 0) {
         s_before[tid >> 6] = before;
         s_total[tid >> 6] = total;
@@ -1372,8 +1369,7 @@ __global__ __launch_bounds__(256) void k_subtree_up(const HiraTree tree, int nod
             const float df = at(l - 1, p, j) - at(l, q, j);
             ss += df * df;
         }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+        ss = wave_sum(ss);
         return sqrtf(ss);
     };
     auto larger = [](float a, float b) { return b > a || b != b ? b : a; };

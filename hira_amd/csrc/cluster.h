@@ -195,11 +195,9 @@ __device__ __forceinline__ void wave_block_mean(const void* x, size_t row0, int 
                 for (int q = 0; q < EPL; ++q) acc[q] += f[q];
             }
     }
-    for (int off = lpr; off < 64; off <<= 1) {
-        cnt += __shfl_xor(cnt, off, 64);
+    cnt = cross_group(cnt, lpr, OpSum{});
 #pragma unroll
-        for (int q = 0; q < EPL; ++q) acc[q] += __shfl_xor(acc[q], off, 64);
-    }
+    for (int q = 0; q < EPL; ++q) acc[q] = cross_group(acc[q], lpr, OpSum{});
     if (rg == 0 && chunk_ok) {
 #pragma unroll
         for (int q = 0; q < EPL; ++q) {

@@ -402,8 +402,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     float sdot = 0.0f;
 #pragma unroll
                     for (int e = 0; e < VPL; ++e) sdot += bf16_lo((uint32_t)kraw[i][e]) * qf[g][e];
-#pragma unroll
-                    for (int off = 1; off < 64; off <<= 1) sdot += __shfl_xor(sdot, off, 64);
+                    sdot = wave_sum(sdot);
                     const float z = sdot * sc2g[g];
                     const float mnew = fmaxf(mq[g], z);
                     const float f = exp2f(mq[g] - mnew);  // 0 the first time
@@ -510,10 +509,8 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                         asum += fabsf(uf[s][e]);
                     }
                 }
-                umax = fmaxf(umax, __shfl_xor(umax, 16, 64));
-                umax = fmaxf(umax, __shfl_xor(umax, 32, 64));
-                asum += __shfl_xor(asum, 16, 64);
-                asum += __shfl_xor(asum, 32, 64);
+                umax = cross_group_max<16>(umax);
+                asum = cross_group_sum<16>(asum);
                 const float su = fmaxf(umax, 1e-30f) / kQ8Steps;
                 const float inv = kQ8Steps / fmaxf(umax, 1e-30f);  // (u * inv: within 0.004 of u / su)
 #pragma unroll
@@ -553,8 +550,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
         }
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
+        ss = cross_group_sum<16>(ss);
         const float qn = sqrtf(ss);
         if (wave == 0) {
 #pragma unroll
@@ -1051,8 +1047,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             // weights are computed with lane = (row, head), head = lane % GS -----------------------
             float m_lane = 0.0f;  // the running maximum of head lane % GS (a finite stand-in for -inf)
             auto raise_max = [&]() {
-                zmax = fmaxf(zmax, __shfl_xor(zmax, 16, 64));
-                zmax = fmaxf(zmax, __shfl_xor(zmax, 32, 64));
+                zmax = cross_group_max<16>(zmax);
                 const float mnew = fmaxf(m_run, zmax);
                 const float f = (m_run == mnew) ? 1.0f : exp2f(m_run - mnew);
                 m_run = mnew;
@@ -1292,8 +1287,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         }
         m_run = m_all;
     }
-#pragma unroll
-    for (int off = GS; off < 64; off <<= 1) l_mine += __shfl_xor(l_mine, off, 64);
+    l_mine = cross_group_sum<GS>(l_mine);
     if (lane < GS) s_lw[wave * 16 + lane] = l_mine;
     if (wave == 0 && kb == 0) s_mh[col] = m_run;
     int tid = threadIdx.x;  // (opaque, like lane_o above: nothing of the merge is computed early)
@@ -1461,8 +1455,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             }
             nc += __popcll(bal);
         }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) ls += __shfl_xor(ls, off, 64);
+        ls = wave_sum(ls);
         if (lane == 0) {
             s_red[2 * g] = mx;
             s_red[2 * g + 1] = ls;

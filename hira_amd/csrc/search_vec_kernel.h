@@ -231,8 +231,7 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
             }
             n += __popcll(bal);
         }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) ls += __shfl_xor(ls, off, 64);
+        ls = wave_sum(ls);
         if (lane == 0) {
             s_l[g] = ls;
             s_n[g] = n;

@@ -83,8 +83,7 @@ __device__ __forceinline__ void small_emit(SmallLds<KS>& s, const float* c, int 
         out[0] = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]), pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
         out[KS * 64] = make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]), pack_bf16(lo[6], lo[7]));
     }
-#pragma unroll
-    for (int off = 1; off < 32; off <<= 1) ss += __shfl_xor(ss, off, 64);
+    ss = group_sum<32>(ss);
     if (j == 0) s.n2[k] = ss;
 }
 
@@ -115,8 +114,7 @@ __device__ __forceinline__ void small_assign(SmallLds<KS>& s, const void* x, siz
 #pragma unroll
                     for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
                 }
-                ss += __shfl_xor(ss, 16, 64);
-                ss += __shfl_xor(ss, 32, 64);
+                ss = cross_group_sum<16>(ss);
                 x2[ri] = ss;
             }
         }

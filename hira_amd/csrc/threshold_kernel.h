@@ -15,11 +15,7 @@ constexpr int kTauRows = 16;  // sample rows a lane group has in flight
 
 __device__ __forceinline__ float tau_block_reduce(float v, bool is_max, float* s_red) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const float o = __shfl_xor(v, off, 64);
-        v = is_max ? fmaxf(v, o) : v + o;
-    }
+    v = is_max ? wave_max(v) : wave_sum(v);
     if (lane == 0) s_red[wave] = v;
     __syncthreads();
     float r = s_red[0];
@@ -31,11 +27,13 @@ __device__ __forceinline__ float tau_block_reduce(float v, bool is_max, float* s
 constexpr int kTauSorters = 256;  // threads that hold the scores during the sort
 
 // The value that lane ^ J holds: moves inside a row of 16 lanes (J < 16) are data-path moves,
-// only J = 16 and 32 go through the LDS crossbar.  rot4_first: which rotation by 4 brings lane ^ 4.
+// J = 16 and 32 swaps of rows and halves.  rot4_first: which rotation by 4 brings lane ^ 4.
 template <int J>
 __device__ __forceinline__ float tau_partner(float v, bool rot4_first) {
-    if constexpr (J >= 16) {
-        return __shfl_xor(v, J, 64);
+    if constexpr (J >= 16) {  // a swap leaves the lower and the upper row's (half's) value in either
+        const auto r = J == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false)
+                               : __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return __uint_as_float((threadIdx.x & J) != 0 ? r[0] : r[1]);
     } else if constexpr (J == 8) {
         return dpp_move<0x128>(v);  // row rotate by 8
     } else if constexpr (J == 4) {
@@ -115,7 +113,7 @@ __device__ __forceinline__ void tau_sort_step(float (&v)[EE], float* s0, float* 
             // (whole waves: the steps inside a wave are not theirs to spend issue slots on)
         } else if constexpr (J >= 16) {
 #pragma unroll
-            for (int e = 0; e < EE; ++e) meet(e, __shfl_xor(v[e], J, 64));
+            for (int e = 0; e < EE; ++e) meet(e, tau_partner<J>(v[e], rot4_first));
         } else if constexpr (J == 8) {
 #pragma unroll
             for (int e = 0; e < EE; ++e) meet(e, dpp_move<0x128>(v[e]));  // row rotate by 8
@@ -266,8 +264,8 @@ __device__ __forceinline__ void threshold_block(
 #pragma unroll
         for (int e = 0; e < 4; ++e) c[e] = s_sc[1][e * 64 + ln];
         float m = tau_merge16(tau_merge16(c[0], c[1], ln, rot4), tau_merge16(c[2], c[3], ln, rot4), ln, rot4);
-        m = tau_merge16(m, __shfl_xor(m, 16, 64), ln, rot4);
-        m = tau_merge16(m, __shfl_xor(m, 32, 64), ln, rot4);
+        m = tau_merge16(m, tau_partner<16>(m, rot4), ln, rot4);
+        m = tau_merge16(m, tau_partner<32>(m, rot4), ln, rot4);
         float sum = 0.0f;
         for (int r = 0; r < k; ++r)  // uniform
             sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(m), r));

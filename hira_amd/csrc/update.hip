@@ -140,8 +140,7 @@ __device__ __forceinline__ int nearest_with_room(const UpdateParams& p, int tree
                     const float df = x[j] - load_elem<T>(p.centers[l], base * D + elem_index(p.layout, D, (size_t)node, j));
                     ss += df * df;
                 }
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+                ss = wave_sum(ss);
                 if (ss < best) {
                     best = ss;
                     arg = node;
@@ -153,8 +152,7 @@ __device__ __forceinline__ int nearest_with_room(const UpdateParams& p, int tree
     }
     __syncthreads();
     if (not_full != nullptr) {  // uniform
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
+        low = wave_min(low);
         if (lane == 0) red_i[wave] = low;
         __syncthreads();
         if (threadIdx.x == 0) {
@@ -354,8 +352,7 @@ __device__ __forceinline__ void update_one_key(const UpdateParams& p, const int 
                 const float b = load_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, node, j));
                 ss += (a - b) * (a - b);
             }
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+            ss = wave_sum(ss);
             if (lane == 0) {
                 s_dist[l] = sqrtf(ss);
                 s_rad[l] = rad_now;
@@ -552,8 +549,7 @@ __device__ __forceinline__ bool window_candidates(const UpdateParams& p, const i
                 const float b = load_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, anc, j));
                 ss += (a - b) * (a - b);
             }
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+            ss = wave_sum(ss);
             if (lane == 0) {
                 w.anc_id[l][c] = (int)anc;
                 w.anc_step[l][c] = sqrtf(ss);
@@ -741,8 +737,7 @@ __device__ __forceinline__ int open_node(const UpdateParams& p, const int tree, 
                 const float b = load_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, node, j));
                 ss += (a - b) * (a - b);
             }
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+            ss = wave_sum(ss);
             d = sqrtf(ss);
         }
         if (lane == 0) {
@@ -882,8 +877,7 @@ __device__ __forceinline__ int open_run(const UpdateParams& p, const int tree, i
             unsigned long long who = __ballot(d == best);
             if (who & (who - 1ull)) {  // ties: the lowest node
                 int low = d == best ? id2 : 0x7fffffff;
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
+                low = wave_min(low);
                 who = __ballot(d == best && id2 == low);
             }
             const int c = __ffsll((long long)who) - 1;
@@ -944,8 +938,7 @@ __device__ __forceinline__ int open_run(const UpdateParams& p, const int tree, i
             const float b = load_elem<T>(p.centers[l], bl * D + elem_index(p.layout, D, node, j));
             ss += (a - b) * (a - b);
         }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off, 64);
+        ss = wave_sum(ss);
         if (lane == 0) {
             w.anc_id[l][i] = (int)node;
             w.anc_step[l][i] = sqrtf(ss);
@@ -1095,8 +1088,7 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
                     unsigned long long who = __ballot(d == best);
                     if (who & (who - 1ull)) {  // ties: the lowest node
                         int low = d == best ? id : 0x7fffffff;
-#pragma unroll
-                        for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
+                        low = wave_min(low);
                         who = __ballot(d == best && id == low);
                     }
                     if (lane == __ffsll((long long)who) - 1) {
@@ -1276,8 +1268,7 @@ __global__ __launch_bounds__(kWinThreads) void k_update_window(const UpdateParam
         // the bound of the next search for room: the lowest listed node that still has some, or
         // the lowest slot that was no node when the list was made
         int low = lane < w.n && w.cnt[lane] < bf ? w.id[lane] : 0x7fffffff;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) low = min(low, __shfl_xor(low, off, 64));
+        low = wave_min(low);
         if (lane == 0) {
             st[0] = min(low, min(w.low_empty, s_used[1]));
             st[HIRA_MAX_LEVELS] = position;
