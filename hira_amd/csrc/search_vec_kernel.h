@@ -320,7 +320,9 @@ void search_kernel(const SearchParams p) {
 
     touch_kernel_arguments();
     const int lane = lane_id();
-    const int wave = threadIdx.x >> 6;
+    // (uniform, as the compiler would not know: a level picked by it has its arguments read by vector loads otherwise,
+    // a trip to memory ahead of the rows')
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int nwaves = blockDim.x >> 6;
     const int rg = lane / LPR;
     const int ch = lane % LPR;
