@@ -174,6 +174,19 @@ __device__ __forceinline__ float row_score(const f32x4_t& acc, int i, int col) {
     return __shfl(pick4(acc, i & 3), col + 16 * (i >> 2), 64);
 }
 
+// What lane % GS of my row of 16 holds.
+template <int GS>
+__device__ __forceinline__ float of_head(float v) {
+    int x = __float_as_int(v);
+    if constexpr (GS == 8) {  // the row's upper half takes the lower's
+        x = __builtin_amdgcn_update_dpp(x, x, 0x118, 0xF, 0xC, false);
+    } else if constexpr (GS == 4) {  // the second quad the first's, then the upper half the lower's
+        x = __builtin_amdgcn_update_dpp(x, x, 0x114, 0xF, 0x2, false);
+        x = __builtin_amdgcn_update_dpp(x, x, 0x118, 0xF, 0xC, false);
+    }
+    return __int_as_float(x);
+}
+
 __device__ __forceinline__ void stat_add(unsigned long long* st, int slot, unsigned v) {
     if (v) atomicAdd(&st[slot], (unsigned long long)v);
 }
@@ -206,8 +219,8 @@ template <int KS>
 struct GateLoads {
     uint4 a1[KS];      // the tile of level-1 centres
     float4 r4;         // radii of rows 4*kb .. 4*kb+3
-    int4 c4;           // child counts of the same rows
-    float4 e4;         // (8-bit shadow) error bounds of the same rows
+    int cn;            // child count of row lane % 16
+    float en;          // (8-bit shadow) error bound of that row
     uint4 anc[2][KS];  // tiles holding the ancestors at levels min(L-1,3) and the one below
     float arad[2];
     unsigned aid[2];
@@ -226,8 +239,8 @@ __device__ __forceinline__ void gate_issue(const SearchParams& p, int tree, int 
     const size_t row1 = (size_t)tree * p.cap[1];
     load_tile<KS>(tile_ptr<KS>(p.centers[1], row1, (size_t)t1, lane), g.a1);
     g.r4 = *reinterpret_cast<const float4*>(p.radii[1] + row1 + (size_t)t1 * 16 + 4 * kb);
-    g.c4 = *reinterpret_cast<const int4*>(p.counts[1] + row1 + (size_t)t1 * 16 + 4 * kb);
-    if (Q8) g.e4 = *reinterpret_cast<const float4*>(p.keps + row1 + (size_t)t1 * 16 + 4 * kb);
+    g.cn = p.counts[1][row1 + (size_t)t1 * 16 + (lane & 15)];
+    if (Q8) g.en = p.keps[row1 + (size_t)t1 * 16 + (lane & 15)];
     const int n_par = min(max(L - 2, 0), 2);
     const unsigned id2 = node_over_bf(p, (unsigned)t1 * 16u);
 #pragma unroll
@@ -614,7 +627,6 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
 
             // level-1 gates: 16 nodes at once
             unsigned alive4 = 0u;
-            const int cc[4] = {gl.c4.x, gl.c4.y, gl.c4.z, gl.c4.w};
             if (tile_live) {
                 const f32x4_t g1 = tile_scores<KS>(gl.a1, bq);
                 const float rr[4] = {gl.r4.x, gl.r4.y, gl.r4.z, gl.r4.w};
@@ -630,28 +642,14 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
 #pragma unroll
             for (int j = 0; j < 4; ++j) nb[j] = __ballot((alive4 >> j) & 1u);
             // node n = 4*kb' + j of the tile: its heads are field kb' of nb[j]
-            // (its child count sits in lane 16*kb', element j, of cc)
-            int cnt_n = 0;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int c = __shfl(cc[j], 16 * ((lane >> 2) & 3), 64);
-                if ((lane & 3) == j) cnt_n = c;
-            }
             if (lane < 16) {
                 const int jn = lane & 3;
                 const unsigned long long bits = jn == 0 ? nb[0] : (jn == 1 ? nb[1] : (jn == 2 ? nb[2] : nb[3]));
                 s_ninfo[tl_mine * 16 + lane] =
-                    (uint32_t)((bits >> (16 * (lane >> 2))) & 0xFFFFull) | ((uint32_t)cnt_n << 16);
+                    (uint32_t)((bits >> (16 * (lane >> 2))) & 0xFFFFull) | ((uint32_t)gl.cn << 16);
             }
-            if constexpr (Q8) {  // the error bounds of the tile's nodes travel like the counts
-                const float ee[4] = {gl.e4.x, gl.e4.y, gl.e4.z, gl.e4.w};
-                float eps_n = 0.0f;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float e = __shfl(ee[j], 16 * ((lane >> 2) & 3), 64);
-                    if ((lane & 3) == j) eps_n = e;
-                }
-                if (lane < 16) s_keps[tl_mine * 16 + lane] = eps_n;
+            if constexpr (Q8) {
+                if (lane < 16) s_keps[tl_mine * 16 + lane] = gl.en;
             }
             tl_mine += nw;
             if (tl_mine < ntile) gate_issue<KS, Q8>(p, tree, tile_of(tl_mine), lane, kb, gl);
@@ -1052,9 +1050,9 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                 const float f = (m_run == mnew) ? 1.0f : exp2f(m_run - mnew);
                 m_run = mnew;
                 // a head without a selected key has m = -inf and only z = -inf: any finite stand-in
-                m_lane = __shfl(mnew == -INFINITY ? 0.0f : mnew, lane_o & (GS - 1), 64);
+                m_lane = of_head<GS>(mnew == -INFINITY ? 0.0f : mnew);
                 if (__ballot(f != 1.0f) != 0ull) {  // uniform
-                    l_mine *= __shfl(f, lane_o & (GS - 1), 64);
+                    l_mine *= of_head<GS>(f);
 #pragma unroll
                     for (int g = 0; g < GS; ++g) {
                         const float fg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), g));
@@ -1274,7 +1272,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         float m_all = -INFINITY;
         for (int w = 0; w < nw; ++w) m_all = fmaxf(m_all, s_mxw[w * 16 + col]);
         const float fw = m_run == -INFINITY ? 0.0f : exp2f(m_run - m_all);
-        l_mine *= __shfl(fw, lane & (GS - 1), 64);
+        l_mine *= of_head<GS>(fw);
 #pragma unroll
         for (int g = 0; g < GS; ++g) {
             const float fg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fw), g));
