@@ -239,11 +239,15 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
     }
     __syncthreads();
     const int quads = Dv / 4, items = G * quads;
-    const int n_grp = max((int)blockDim.x / items, 1);
+    // (quotients of small numbers as products with a reciprocal, exact for numbers of a few thousand: a division is
+    // thirty instructions of a chain)
+    const float inv_items = 1.0f / (float)items, inv_quads = 1.0f / (float)quads, inv_dv = 1.0f / (float)Dv;
+    auto over = [](int x, float inv) { return (int)(((float)x + 0.5f) * inv); };
+    const int n_grp = max(over((int)blockDim.x, inv_items), 1);
     for (int i0 = 0; i0 < items; i0 += blockDim.x) {  // uniform; once unless G * Dv > 4 threads
-        const int item = n_grp > 1 ? t % items : i0 + t, grp = n_grp > 1 ? t / items : 0;
+        const int grp = n_grp > 1 ? over(t, inv_items) : 0, item = n_grp > 1 ? t - grp * items : i0 + t;
         if (item < items && grp < n_grp) {
-            const int g = item / quads, qd = item % quads;
+            const int g = over(item, inv_quads), qd = item - g * quads;
             const int head = p.group_size > 0 ? hoff + g : p.tree_q_heads[hoff + g];
             typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
             const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -283,7 +287,7 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
     if (n_grp == 1) return;
     __syncthreads();
     for (int e = t; e < items * 4; e += blockDim.x) {
-        const int g = e / Dv;
+        const int g = over(e, inv_dv);
         const int head = p.group_size > 0 ? hoff + g : p.tree_q_heads[hoff + g];
         float sum = 0.0f;
         for (int r = 0; r < n_grp; ++r) sum += red[(size_t)r * items * 4 + e];
@@ -904,8 +908,9 @@ void search_kernel(const SearchParams p) {
         }
     }
     __syncthreads();
+    const float inv_dv = 1.0f / (float)Dv;  // (quotients below some thousands: exact)
     for (int t = threadIdx.x; t < G * Dv; t += blockDim.x) {
-        const int g = t / Dv, e = t % Dv;
+        const int g = (int)(((float)t + 0.5f) * inv_dv), e = t - g * Dv;
         // (what every wave has, read at once: one wave's after the other's was a chain of 16 reads, and with the fold's
         // maxima asked for twice 0.3 us of 15.9 at 4 trees x 5003 rows of 80 columns, 3 heads each)
         float mw[WAVES], aw[WAVES], lw[WAVES], mall = -INFINITY;
