@@ -1174,7 +1174,6 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             } else {
                 if constexpr (WIDE) {
                     if (want_attn && tot > 0) {  // uniform in the launch / in the wave
-                        raise_max();
                         constexpr int NLD = kVBatch / RPI;  // load instructions of a batch
                         for (int e0 = 0; e0 < tot; e0 += kVBatch) {  // uniform in the wave
                             // the batch's rows in the score table: for the weights (lane = (row of
@@ -1202,6 +1201,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                             }
                             if (r == 0 && e0 == 0) tline.stamp_wave(kTlWaveIssued);
                             __builtin_amdgcn_sched_barrier(0);
+                            if (e0 == 0) raise_max();  // (while the first values are on their way)
                             // scores -> weights, in place, 64 (row, head) pairs at a time
 #pragma unroll
                             for (int ps = 0; ps < NPASS; ++ps) {
