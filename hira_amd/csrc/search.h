@@ -26,7 +26,7 @@ struct SearchParams {
     const float* keps;
     // queries
     const void* q;
-    const float* tau;
+    const float* tau;  // (SAMPLED: written by the launch, threshold_join)
     const float* scaling;
     const int32_t* tree_q_off;
     const int32_t* tree_q_heads;
@@ -41,20 +41,36 @@ struct SearchParams {
         int32_t nodes_per_wg;    // vector-ALU kernel: level-1 nodes (or pseudo blocks) a workgroup walks
     };
     int32_t tree_blocks;     // workgroups that walk the tree; the rest scan the queue
-    int32_t key_policy;      // MFMA kernel: which cache policy the scan's loads use (0: default,
-                             // 1: key tiles non-temporal, 2: value rows too), by the launch's size
+    int32_t sample_wgs;      // > 0: that many workgroups a tree, ahead of the searching ones, make the thresholds
+                             // (instantiations SAMPLED; attention only: what a sample needs shares its
+                             // place with what a dense output and lists need)
     int32_t num_nodes;       // level-1 nodes (or pseudo blocks over the keys when L == 1)
     int32_t num_queue_blocks;
     // outputs
-    float* dense;
-    int64_t dense_stride;
-    int32_t dense_by_position;
+    union {
+        float* dense;
+        float* sample_best;  // threshold_stretch
+    };
+    union {
+        int64_t dense_stride;
+        const void* sample;  // (T, sample_rows, D)
+    };
+    union {
+        int32_t dense_by_position;
+        int32_t sample_wait;  // looks at the counter before a workgroup makes its thresholds itself
+    };
     int32_t dense_fill;       // the kernels write dense_fill_value wherever no score goes
-    float dense_fill_value;
+    union {
+        float dense_fill_value;
+        int32_t sample_rows;
+    };
     int32_t* sel_index;
     float* sel_score;
     int32_t* sel_count;
-    int32_t sel_cap;
+    union {
+        int32_t sel_cap;
+        int32_t sample_k;
+    };
     float* part_m;    // (H_q, P)
     float* part_l;    // (H_q, P)
     float* part_acc;  // (H_q, P, Dv)
@@ -80,6 +96,8 @@ struct SearchPlan {
     int threads;      // workgroup size
     int nodes_per_wave;  // MFMA kernel: tiles per workgroup
     int nodes_per_wg, queue_nodes;  // vector-ALU kernel: as in SearchParams
+    int key_policy;   // MFMA kernel: which cache policy the scan's loads use (0: default, 1: key tiles
+                      // non-temporal, 2: value rows too), by the launch's size
     int num_nodes, num_queue_blocks;
     int tree_blocks, queue_blocks, head_chunks;
     int ahead;        // > 0: keys are asked for together with the gates' operands (vector-ALU kernel: as many elements a lane)
@@ -91,6 +109,8 @@ int launch_vec_f32(const SearchPlan& plan, const SearchParams& p, dim3 grid, hip
 int launch_vec_bf16(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
 
 // search_mfma.hip
+// thresholds in the search's launch: fan-outs of up to two key tiles (with four the kernel's registers spill)
+constexpr int kSampledTiles = 2;
 bool mfma_search_supported(const HiraTree* t, const HiraQueue* queue);
 constexpr int kMfmaThreads = 512;       // workgroup size of the MFMA kernel (8 waves), at most
 constexpr int kMfmaMaxTilesPerWg = 16;  // tiles of 16 level-1 nodes one workgroup walks, at most

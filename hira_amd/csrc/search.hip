@@ -2,6 +2,7 @@
 // the partials as a launch of its own.  The kernel is in search_vec_kernel.h, instantiated per
 // element type in search_vec_f32.hip and search_vec_bf16.hip.
 #include "search_vec_kernel.h"
+#include "threshold_kernel.h"
 
 namespace hira {
 
@@ -238,16 +239,17 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
 
 using namespace hira;
 
-// partials (acc, m, l) followed by the arrival counters of the fused fold
-// bytes of the arrival counters, which come first: their place does not depend on the
-// number of partials, so a workspace stays usable when the tree grows or a queue comes and goes
-static size_t counter_bytes(int trees, int passes) {
+// The arrival counters of the fused fold and the scores that a launch with its own thresholds hands over, both zero
+// between calls, then the partials (acc, m, l).  The former come first: their place does not depend on the
+// number of partials, so a workspace stays usable when the tree grows or a queue comes and goes.
+constexpr int kSampledHeads = 128;  // (two workgroups a head and a compute unit each: more heads make no such launch)
+static size_t arrival_bytes(int trees, int passes) {
     return (((size_t)trees * passes * sizeof(int32_t)) + 255) & ~(size_t)255;
 }
-
-static size_t workspace_need(int h_q, size_t P, int vdim, int trees, int passes) {
-    return counter_bytes(trees, passes) + (size_t)h_q * P * (size_t)(vdim + 2) * sizeof(float);
+static size_t counter_bytes(int trees, int passes, int h_q) {
+    return arrival_bytes(trees, passes) + (h_q <= kSampledHeads ? ((size_t)h_q * 32 * sizeof(float) + 255) & ~(size_t)255 : 0);
 }
+static size_t partial_bytes(int h_q, size_t P, int vdim) { return (size_t)h_q * P * (size_t)(vdim + 2) * sizeof(float); }
 
 extern "C" size_t hira_search_workspace_bytes(const HiraTree* tree, const HiraQuery* query,
                                               const HiraQueue* queue,
@@ -255,14 +257,27 @@ extern "C" size_t hira_search_workspace_bytes(const HiraTree* tree, const HiraQu
     SearchPlan plan;
     if (make_plan(tree, query, queue, launch, true, &plan) != HIRA_OK) return 0;
     const size_t P = (size_t)plan.tree_blocks + plan.queue_blocks;
-    return workspace_need(query->num_q_heads, P, tree->vdim, tree->num_trees, plan.head_chunks);
+    return counter_bytes(tree->num_trees, plan.head_chunks, query->num_q_heads) + partial_bytes(query->num_q_heads, P, tree->vdim);
 }
 
 /* see include/hira_hip.h */
 extern "C" size_t hira_search_counter_bytes(const HiraTree* tree, const HiraQuery* query, const HiraLaunch* launch) {
     SearchPlan plan;
     if (make_plan(tree, query, nullptr, launch, true, &plan) != HIRA_OK) return 0;
-    return counter_bytes(tree->num_trees, plan.head_chunks);
+    return counter_bytes(tree->num_trees, plan.head_chunks, query->num_q_heads);
+}
+
+// Does this search make its thresholds itself (threshold_stretch)?  What that is written for, under a
+// kernel of one tile a workgroup that asks for its keys ahead, the fold in the launch, nothing but attention, and a
+// compute unit for every workgroup: the kernel runs one at a time on a compute unit, and one that had to wait for a
+// place would begin when the stretches are done, as in a launch of its own.
+constexpr int kSampleWait = 1 << 14;  // looks at the counter; one takes about a microsecond
+static bool sampled_in_one(const SearchPlan& plan, const SearchParams& p, const HiraTree* tree, const HiraSample* sample) {
+    if (p.group_size * tree->num_trees > kSampledHeads) return false;
+    return plan.kernel == 2 && plan.ahead && plan.tree_blocks > 0 && plan.key_policy == 0 && p.keys8 == nullptr && tree->bf <= 16 * kSampledTiles &&
+           tree->dim <= 128 && p.done != nullptr && p.dense == nullptr && p.sel_count == nullptr && plan.head_chunks == 1 &&
+           p.group_size > 0 && p.group_size <= 16 && sample->method == HIRA_TAU_SAMPLE_MEAN_TOPK && sample->k <= 16 &&
+           sample->num_rows <= kTauFewRows && (2 * p.group_size + p.num_parts) * tree->num_trees <= compute_units();
 }
 
 // The search behind both entry points.  Attention needs arrival counters (one int32 per tree
@@ -271,7 +286,7 @@ extern "C" size_t hira_search_counter_bytes(const HiraTree* tree, const HiraQuer
 // nothing), else at the start of the caller's workspace, the partials right after them.
 static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQueue* queue,
                        const HiraSearchOut* out, const HiraLaunch* launch, void* workspace,
-                       size_t workspace_bytes, size_t fixed_counters, void* stream) {
+                       size_t workspace_bytes, size_t fixed_counters, void* stream, const HiraSample* sample = nullptr) {
     SearchPlan plan;
     HIRA_CHECK_ARG(out != nullptr, "out is NULL");
     const bool attn = out->attn_out != nullptr;
@@ -340,7 +355,7 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
     {   // up to what the eight L2s hold together (32 MiB) the default policy; up to 512 MiB the
         // key tiles and the value rows non-temporal; beyond, the key tiles only
         const size_t key_bytes = (size_t)tree->num_trees * (size_t)tree->size[0] * (size_t)tree->dim * 2;
-        p.key_policy = key_bytes <= ((size_t)32 << 20) ? 0 : (key_bytes <= ((size_t)512 << 20) ? 2 : 1);
+        plan.key_policy = key_bytes <= ((size_t)32 << 20) ? 0 : (key_bytes <= ((size_t)512 << 20) ? 2 : 1);
     }
     p.num_nodes = plan.num_nodes;
     p.num_queue_blocks = use_queue ? plan.num_queue_blocks : 0;
@@ -353,13 +368,18 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
     p.sel_score = out->sel_score;
     p.sel_count = out->sel_count;
     p.sel_cap = out->sel_cap;
+    static_assert(sizeof(p.sample) == sizeof(p.dense_stride), "");
     p.stats = out->stats;
 
     const int P = plan.tree_blocks + (use_queue ? plan.queue_blocks : 0);
-    if (P == 0) return HIRA_OK;
+    auto thresholds_ahead = [&] {
+        return hira_threshold(sample->rows, tree->dtype, tree->num_trees, sample->num_rows, tree->dim, query,
+                              sample->method, sample->k, sample->tau, stream);
+    };
+    if (P == 0) return sample ? thresholds_ahead() : HIRA_OK;
     p.num_parts = P;
     if (attn) {
-        size_t ctr_bytes = counter_bytes(tree->num_trees, plan.head_chunks);
+        size_t ctr_bytes = counter_bytes(tree->num_trees, plan.head_chunks, query->num_q_heads);
         if (fixed_counters > 0) {
             if ((size_t)tree->num_trees * plan.head_chunks > fixed_counters)
                 return fail(HIRA_EWORKSPACE, "%d trees x %d head passes: more than the %zu arrival "
@@ -367,7 +387,7 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
                             plan.head_chunks, fixed_counters);
             ctr_bytes = fixed_counters * sizeof(int32_t);
         }
-        const size_t need = ctr_bytes + workspace_need(query->num_q_heads, (size_t)P, tree->vdim, 0, 0);
+        const size_t need = ctr_bytes + partial_bytes(query->num_q_heads, (size_t)P, tree->vdim);
         if (workspace == nullptr || workspace_bytes < need)
             return fail(HIRA_EWORKSPACE, fixed_counters > 0
                             ? "the built-in scratch buffer holds %zu bytes, this search needs %zu"
@@ -395,9 +415,20 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
                        query->num_q_heads);
 
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (sample && sampled_in_one(plan, p, tree, sample)) {
+        p.sample_wgs = p.group_size * (sample->num_rows > kTauStretch ? 2 : 1);
+        p.sample_best = reinterpret_cast<float*>(static_cast<char*>(workspace) + arrival_bytes(tree->num_trees, plan.head_chunks));
+        p.sample = sample->rows;
+        p.sample_rows = sample->num_rows;
+        p.sample_k = sample->k;
+        p.sample_wait = sample->wait > 0 ? sample->wait : (sample->wait < 0 ? 0 : kSampleWait);
+    } else if (sample) {
+        rc = thresholds_ahead();
+        if (rc != HIRA_OK) return rc;
+    }
     dim3 grid(P, tree->num_trees, plan.head_chunks);
     if (plan.kernel == 2)
-        rc = launch_search_mfma(plan, p, dim3(tree->num_trees, P, plan.head_chunks), s);
+        rc = launch_search_mfma(plan, p, dim3(tree->num_trees, P + p.sample_wgs, plan.head_chunks), s);
     else
         rc = tree->dtype == HIRA_F32 ? launch_vec_f32(plan, p, grid, s)
                                      : launch_vec_bf16(plan, p, grid, s);
@@ -427,12 +458,12 @@ extern "C" int hira_search_sampled(const HiraTree* tree, const HiraQuery* query,
                                    const HiraQueue* queue, const HiraSearchOut* out, const HiraLaunch* launch,
                                    void* workspace, size_t workspace_bytes, void* stream) {
     HIRA_CHECK_ARG(tree && query && sample, "hira_search_sampled: null argument");
-    const int rc = hira_threshold(sample->rows, tree->dtype, tree->num_trees, sample->num_rows, tree->dim, query,
-                                  sample->method, sample->k, sample->tau, stream);
-    if (rc != HIRA_OK) return rc;
+    if (const int rc = check_threshold_arguments(sample->rows, tree->dtype, tree->num_trees, sample->num_rows, tree->dim, query,
+                                                 sample->method, sample->k, sample->tau))
+        return rc;
     HiraQuery with = *query;
     with.tau = sample->tau;
-    return hira_search(tree, &with, queue, out, launch, workspace, workspace_bytes, stream);
+    return search_impl(tree, &with, queue, out, launch, workspace, workspace_bytes, 0, stream, sample);
 }
 
 // ---- the same search for callers that cannot allocate ----------------------------------------

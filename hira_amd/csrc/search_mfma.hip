@@ -18,7 +18,7 @@ bool mfma_search_supported(const HiraTree* t, const HiraQueue* queue) {
 // grid: x = tree, y = tile of 16 level-1 nodes, z = pass of 16 heads
 int launch_search_mfma(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s) {
     const bool q8 = p.keys8 != nullptr;  // the scan reads the keys' 8-bit shadow
-    const int pol = q8 ? 0 : p.key_policy;  // cache policy of the bf16 tiles and the value rows
+    const int pol = q8 ? 0 : plan.key_policy;  // cache policy of the bf16 tiles and the value rows
     typedef void (*Launch)(const SearchPlan&, const SearchParams&, dim3, hipStream_t);
     static const Launch table[3][4] = {
         {launch_mfma_d64, launch_mfma_nt1_d64, launch_mfma_nt2_d64, launch_mfma_q8_d64},

@@ -43,6 +43,7 @@
 
 #include "search.h"
 #include "search_mfma_timeline.h"
+#include "threshold_kernel.h"
 
 namespace hira {
 
@@ -275,7 +276,8 @@ constexpr int kAheadNodes = 16 / kMfmaWaves;
 // AHEAD: (small launches) a workgroup owns one tile, and its waves ask for the key tiles of their two
 // nodes each together with the gates' operands, whether the nodes survive or not: a trip to memory less,
 // and no list of survivors.
-template <int KS, int MT, int GS, bool OUT, bool Q8, int POL, int HV, bool ONE, bool AHEAD = false>
+// SAMPLED: (with AHEAD) the launch makes its thresholds itself, in workgroups ahead of the searching ones.
+template <int KS, int MT, int GS, bool OUT, bool Q8, int POL, int HV, bool ONE, bool AHEAD = false, bool SAMPLED = false>
 __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const SearchParams p) {
     using S = MfmaShape<KS, MT, GS, Q8>;
     constexpr int D = S::D;
@@ -313,19 +315,31 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     const int tree = blockIdx.x;
     const int L = p.num_levels, bf = p.bf;
     const bool want_attn = p.part_acc != nullptr;
+    static_assert(!SAMPLED || (AHEAD && S::WORDS >= kTauFewRows), "");
+    __shared__ float s_tau[SAMPLED ? kHeadsPerPass : 1];
+    int wgs = gridDim.y, wg = blockIdx.y;  // searching workgroups of the tree, my number among them
+    if constexpr (SAMPLED) {
+        wgs -= p.sample_wgs;
+        wg -= p.sample_wgs;
+        if (wg < 0) {  // uniform
+            threshold_stretch<4 * KS>(p.sample, p.sample_rows, p.q, tree, p.group_size, (int)blockIdx.y, p.sample_best,
+                                      reinterpret_cast<float*>(s_words), p.done + tree, wgs + p.sample_wgs * kTauMade);
+            return;
+        }
+    }
     // Workgroup y of a tree owns the tree's tiles y, y + (workgroups of the tree), ...: a stride
     // apart, since neighbouring tiles hold sibling nodes, which tend to survive (and be selected
     // from) together.
     const int wg_tiles = (p.size[1] + 15) >> 4;
     const int n_groups = p.tree_blocks;
-    const int grp = (int)blockIdx.y;
-    const int ntile = (int)blockIdx.y < p.tree_blocks
+    const int grp = wg;
+    const int ntile = wg < p.tree_blocks
                           ? min(p.nodes_per_wave, (wg_tiles - grp + n_groups - 1) / n_groups)
                           : 0;
     auto tile_of = [&](int tl) { return grp + tl * n_groups; };
     // level-1 node behind entry n (tile n / 16 of mine, node n % 16 of the tile)
     auto node_of = [&](int n) { return tile_of(n >> 4) * 16 + (n & 15); };
-    const bool is_queue = (int)blockIdx.y >= p.tree_blocks;  // the workgroup after the tree's
+    const bool is_queue = wg >= p.tree_blocks;  // the workgroup after the tree's
     Timeline tline(p);  // (empty unless the library is built with time stamps)
     unsigned long long* stats =
         (p.stats && !Timeline::kOn) ? p.stats + (size_t)tree * HIRA_STATS_COLS : nullptr;
@@ -447,7 +461,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         uint4 qraw[KS];
 #pragma unroll
         for (int s = 0; s < KS; ++s) qraw[s] = make_uint4(0, 0, 0, 0);
-        float tau = p.tau[qh];
+        float tau = SAMPLED ? 0.0f : p.tau[qh];
         float sc = p.scaling[qh];
         GateLoads<KS> gl;
         uint4 a[NB][MT][KA];  // key tiles of the nodes that a wave takes in a round
@@ -570,6 +584,16 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             for (int s = 0; s < KS; ++s) s_bq[s * 64 + lane] = qraw[s];
         }
 
+        if constexpr (SAMPLED) {
+            // the thresholds: wave 0, which alone gates, waits for them and leaves them to the others
+            if (wave == 0) {
+                threshold_join<4 * KS, GS>(p.sample, p.sample_rows, p.q, tree, hoff, G, p.sample_k, p.sample_best, p.sample_wait, s_tau,
+                                           reinterpret_cast<float*>(s_words));
+                tau = head_ok ? s_tau[col] : INFINITY;
+                if (wg == 0 && lane < G) const_cast<float*>(p.tau)[hoff + lane] = s_tau[lane];
+            }
+        }
+
         // ---- gate: one tile per wave at a time ------------------------------------------------
         while (tl_mine < ntile) {  // uniform in the wave
             const int t1 = tile_of(tl_mine);
@@ -657,6 +681,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         tline.stamp(kTlGated);
         __syncthreads();
         tline.stamp(kTlBarrier);
+        if constexpr (SAMPLED) tau = head_ok ? s_tau[col] : INFINITY;
 
         // ---- the surviving nodes of my tiles in order, dealt round-robin to the waves ----------
         int rounds = 1, alive = 0;
@@ -1294,7 +1319,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     const int P = p.num_parts;
     // a tree's only workgroup writes the output itself: no partial, no ticket, no fold (8 trees x 500 keys in
     // two levels: 9.2 -> 7.5 us)
-    const bool alone = gridDim.y == 1 && p.done != nullptr;  // uniform
+    const bool alone = wgs == 1 && p.done != nullptr;  // uniform
 #pragma unroll
     for (int c = 0; c < GS / 4; ++c) {
         if (c * 4 >= G) continue;  // uniform (no break: the loop has to unroll)
@@ -1342,7 +1367,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                 store_out(p.attn_out, p.out_bf16, (size_t)head * D + e, lsum > 0.0f ? a_sum * (1.0f / lsum) : 0.0f);
                 continue;
             }
-            const size_t slot = (size_t)head * P + blockIdx.y;
+            const size_t slot = (size_t)head * P + wg;
             // device-scope stores: written through, so that the workgroup that folds the
             // partials (maybe on another L2 slice) reads them without cache-wide flushes;
             // a head without a selected key only says so (m = -inf)
@@ -1356,13 +1381,29 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         }
     }
     tline.stamp(kTlStoresIssued);
+    // (SAMPLED) my ticket, by wave 0; behind the last of all the tree's counter and scores go back to zero
+    auto sampled_ticket = [&] {
+        int before = 0;
+        if (lane == 0) before = __hip_atomic_fetch_add(p.done + tree, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        before = __builtin_amdgcn_readfirstlane(before);
+        if (before + 1 == wgs + p.sample_wgs * kTauMade) threshold_reset(p.sample_best + (size_t)hoff * 32, G * 32, p.done + tree);
+        return (before & (kTauMade - 1)) == wgs - 1;
+    };
+    if constexpr (SAMPLED) {
+        if (alone && wave == 0) sampled_ticket();
+    }
     if (p.done == nullptr || alone) return;  // the caller folds the partials in a second launch, or there is one
 
     // ---- the last workgroup of this tree (and pass) to arrive folds the tree's partials ----
     hand_off_release();
     tline.stamp(kTlStored);
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if constexpr (SAMPLED) {
+        if (wave == 0) {
+            const bool last = sampled_ticket();
+            if (lane == 0) s_last = last;
+        }
+    } else if (threadIdx.x == 0) {
         int* ctr = p.done + (size_t)tree * gridDim.z + blockIdx.z;
         const int ticket = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s_last = ticket == (int)gridDim.y - 1;
@@ -1564,7 +1605,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
 template <int KS, int MT, int GS, bool Q8, int POL, int HV>
 void launch_mfma_one(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s) {
     const dim3 block(plan.threads);
-    const bool out = p.dense != nullptr || p.sel_count != nullptr;
+    const bool out = p.sample_wgs == 0 && (p.dense != nullptr || p.sel_count != nullptr);
     // nodes (entries of the survivors' list) a workgroup's tiles hold at most, against those its
     // waves take in one round
     const bool one = plan.nodes_per_wave * 16 * HV <= (plan.threads / 64) * MfmaShape<KS, MT, GS, Q8>::NB;
@@ -1573,6 +1614,12 @@ void launch_mfma_one(const SearchPlan& plan, const SearchParams& p, dim3 grid, h
         return;
     }
     if constexpr (!Q8 && POL == 0 && HV == 1 && KS <= 4 && MfmaShape<KS, MT, GS>::NB >= kAheadNodes) {
+        if constexpr (MT <= kSampledTiles) {
+            if (plan.ahead && p.sample_wgs > 0) {
+                hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, false, 0, 1, true, true, true>), grid, block, 0, s, p);
+                return;
+            }
+        }
         if (plan.ahead) {
             hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, false, 0, 1, true, true>), grid, block, 0, s, p);
             return;

@@ -160,11 +160,12 @@ struct TauSortFrom {
 // address register for all of them.  The range check of a buffer load looks at the vector offset only, so the
 // scalar one must stay inside the sample by itself: a pass that reaches past the end is moved back to end with
 // the sample, and its rows that an earlier pass has are none here (row -1, score -INFINITY).
-template <int LPR>
+// (Workgroups of NT threads, at most 1024, score NT rows at a time.)
+template <int LPR, int NT = kTauThreads>
 __device__ __forceinline__ float tau_dot_scores(const void* xs, const void* qh, int r0, int S, bool rot4_first, int& row) {
     typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    constexpr int D = 8 * LPR, PASS = kTauThreads / LPR;
+    constexpr int D = 8 * LPR, PASS = NT / LPR;
     const int tid = threadIdx.x, sub = tid % LPR, grp = tid / LPR;
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(xs), 0, S * D * 2, 0x00020000);
@@ -219,6 +220,169 @@ __device__ __forceinline__ float tau_merge16(float a, float b, int ln, bool rot4
     return m;
 }
 
+// A wave's 64 values, one a lane, sorted largest first.
+__device__ __forceinline__ float tau_wave_sort(float x, int ln, bool rot4) {
+    tau_wave_stage<2, 1>(x, ln, rot4);
+    tau_wave_stage<4, 2>(x, ln, rot4);
+    tau_wave_stage<8, 4>(x, ln, rot4);
+    tau_wave_stage<16, 8>(x, ln, rot4);
+    tau_wave_stage<32, 16>(x, ln, rot4);
+    tau_wave_stage<64, 32>(x, ln, rot4);
+    return x;
+}
+
+// ---- thresholds in the launch that searches with them -------------------------------------------------
+// A search of few workgroups needs its thresholds only where its gates are compared, some 2.5 us after its start,
+// and a launch ahead of it is one more for the host and the queue.  So the first workgroups of the search's launch
+// score the sample, kTauStretch rows of a tree for a head each, and leave the stretch's 16 best in memory; every
+// workgroup of higher number looks for them behind its own loads (threshold_join).  Only those wait, for ones
+// that never do.  Up to kTauFewRows sample rows, the mean of at most 16 best, bf16 rows of 64 or 128 columns; the
+// arithmetic is threshold_block's, the same bits.
+// us, two launches / this, 8 trees x 4 heads, 1000 samples: 4001 rows of 128 columns 15.0 / 12.3 (waiting for a
+// counter and then asking for the scores 15.3), 8000 16.6 / 13.6, 1000 14.0 / 11.0, 4001 x 64 13.0 / 10.8;
+// 8 heads a tree 16.9 / 14.4; 300 rows, as many samples 12.0 / 9.4.  What bounds it is the chain: arguments, one trip and
+// half the sample through a compute unit's L1, the sorts (some 6 us from the start), two trips of the hand-over,
+// then the search from its gates on.
+//   best    (H_q, 2, 16) scores, largest first; 0 between launches, which says: not there yet (a score of 0 is
+//           left as -0, which adds up to the same).  So what is waited for is the scores themselves; behind a
+//           counter, two trips later, nothing was won
+//   ready   the tree's arrival counter: tickets of the searching workgroups in the low half, finished stretches in
+//           the high half.  Whoever comes last of all sets it and `best` back to zero (threshold_reset)
+constexpr int kTauFewRows = 1024, kTauStretch = 512;
+constexpr int kTauMade = 1 << 16;
+
+// By one wave: the tree's thresholds are used by all, its counter and its n words of `best` go back to zero.
+__device__ __forceinline__ void threshold_reset(float* best, int n, int* ready) {
+    for (int i = threadIdx.x & 63; i < n; i += 64) __hip_atomic_store(best + i, 0.0f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((threadIdx.x & 63) == 0) __hip_atomic_store(ready, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// heads: of a tree; all: the counter's value behind the last of all
+template <int LPR>
+__device__ __forceinline__ void threshold_stretch(const void* samples, int S, const void* q, int tree, int heads, int index,
+                                                  float* best, float* lds, int* ready, int all) {
+    const int head = tree * heads + index % heads, stretch = index / heads;
+    constexpr int D = 8 * LPR;
+    const int ln = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const bool rot4 = __builtin_amdgcn_update_dpp(0, ln, 0x124, 0xF, 0xF, true) == (ln ^ 4);
+    const uint16_t* xs = reinterpret_cast<const uint16_t*>(samples) + (size_t)tree * S * D;
+    const uint16_t* qh = reinterpret_cast<const uint16_t*>(q) + (size_t)head * D;
+    int row;
+    const float x = tau_wave_sort(tau_dot_scores<LPR, kTauStretch>(xs, qh, stretch * kTauStretch, S, rot4, row), ln, rot4);
+    if (ln < 16) lds[wv * 16 + ln] = x;  // 8 waves
+    __syncthreads();
+    if (wv != 0) return;
+    float m = tau_merge16(lds[ln], lds[64 + ln], ln, rot4);
+    m = tau_merge16(m, tau_partner<16>(m, rot4), ln, rot4);
+    m = tau_merge16(m, tau_partner<32>(m, rot4), ln, rot4);
+    if (ln < 16)
+        __hip_atomic_store(best + (head * 2 + stretch) * 16 + ln, m == 0.0f ? -0.0f : m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // (written through and complete before it is counted: the hand-off of search.h)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    int before = 0;
+    if (ln == 0) before = __hip_atomic_fetch_add(ready, kTauMade, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(before) + kTauMade == all) threshold_reset(best + (size_t)tree * heads * 32, heads * 32, ready);
+}
+
+// The mean of the k best of every row of 16 lanes, sorted largest first: added up in that order.
+__device__ __forceinline__ float tau_row_mean(float m, int k) {
+    float sum = 0.0f;
+    auto add = [&](auto at) {
+        constexpr int R = decltype(at)::value;
+        const float v = dpp_move<0x150 + R>(m);  // (lane R of the row to all of it)
+        if (R < k) sum += v;                     // uniform
+    };
+#define HIRA_TAU_ADD(R) add(std::integral_constant<int, R>{})
+    HIRA_TAU_ADD(0), HIRA_TAU_ADD(1), HIRA_TAU_ADD(2), HIRA_TAU_ADD(3), HIRA_TAU_ADD(4), HIRA_TAU_ADD(5), HIRA_TAU_ADD(6), HIRA_TAU_ADD(7);
+    HIRA_TAU_ADD(8), HIRA_TAU_ADD(9), HIRA_TAU_ADD(10), HIRA_TAU_ADD(11), HIRA_TAU_ADD(12), HIRA_TAU_ADD(13), HIRA_TAU_ADD(14), HIRA_TAU_ADD(15);
+#undef HIRA_TAU_ADD
+    return sum / (float)k;
+}
+
+// The threshold of a head by one wave, slowly and in few registers: for a workgroup that gave up waiting.
+// scores: kTauFewRows floats of LDS.
+template <int LPR>
+__device__ __forceinline__ float threshold_by_wave(const void* samples, int S, const void* q, int tree, int head, int k, float* scores) {
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    constexpr int D = 8 * LPR;
+    const int ln = threadIdx.x & 63;
+    const uint4* xs = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(samples) + (size_t)tree * S * D);
+    const uint4* qh = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(q) + (size_t)head * D);
+#pragma unroll 1
+    for (int r = ln; r < S; r += 64) {
+        float d[LPR];
+#pragma unroll
+        for (int c = 0; c < LPR; ++c) {
+            const uint4 a = xs[(size_t)r * LPR + c], b = qh[c];
+            const uint32_t u[4] = {a.x, a.y, a.z, a.w}, v[4] = {b.x, b.y, b.z, b.w};
+            d[c] = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                d[c] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, u[e]), __builtin_bit_cast(bf16x2, v[e]), d[c], false);
+        }
+#pragma unroll
+        for (int half = LPR / 2; half >= 1; half /= 2)
+#pragma unroll
+            for (int c = 0; c < half; ++c) d[c] += d[c + half];
+        scores[r] = d[0];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    float sum = 0.0f;
+#pragma unroll 1
+    for (int i = 0; i < k; ++i) {  // uniform: the largest one that is left
+        float best = -INFINITY;
+        int at = -1;
+        for (int r = ln; r < S; r += 64) {
+            const float v = scores[r];
+            if (v > best || at < 0) best = v, at = r;
+        }
+        const float top = wave_max(best);
+        const unsigned long long who = __ballot(at >= 0 && best == top);
+        if (ln == __ffsll((long long)who) - 1) scores[at] = -INFINITY;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        sum += top;
+    }
+    return sum / (float)k;
+}
+
+// By one wave of a workgroup that searches for the G <= GS heads from `head0` on of a tree: their thresholds to
+// s_tau, as soon as the stretches are there.  `limit` looks without success: it makes them itself.
+// scores: kTauFewRows floats of LDS.
+template <int LPR, int GS>
+__device__ __forceinline__ void threshold_join(const void* samples, int S, const void* q, int tree, int head0, int G, int k,
+                                               const float* best, int limit, float* s_tau, float* scores) {
+    const int ln = threadIdx.x & 63;
+    float a[GS / 4], b[GS / 4];  // of four heads at a time, a row of 16 lanes each
+    bool made = false;
+    for (int look = 0; look < limit && !made; ++look) {  // uniform
+        made = true;
+#pragma unroll
+        for (int i = 0; i < GS / 4; ++i) {
+            const float* at = best + (head0 + min(4 * i + ln / 16, G - 1)) * 32 + ln % 16;
+            a[i] = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            b[i] = -INFINITY;
+            if (S > kTauStretch) b[i] = __hip_atomic_load(at + 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // uniform
+        }
+#pragma unroll
+        for (int i = 0; i < GS / 4; ++i) made = made && __float_as_uint(a[i]) != 0u && __float_as_uint(b[i]) != 0u;
+        made = __ballot(!made) == 0ull;
+    }
+    if (made) {
+        const bool rot4 = __builtin_amdgcn_update_dpp(0, ln, 0x124, 0xF, 0xF, true) == (ln ^ 4);
+#pragma unroll
+        for (int i = 0; i < GS / 4; ++i) {
+            const float tau = tau_row_mean(tau_merge16(a[i], b[i], ln, rot4), k);
+            if (ln % 16 == 0 && 4 * i + ln / 16 < G) s_tau[4 * i + ln / 16] = tau;
+        }
+    } else {
+        for (int g = 0; g < G; ++g) {  // uniform
+            const float tau = threshold_by_wave<LPR>(samples, S, q, tree, head0 + g, k, scores);
+            if (ln == 0) s_tau[g] = tau;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+}
+
 // E = registers per thread of the sort: the padded array has 1024 * E entries
 // The work of one workgroup of kTauThreads threads: the threshold of the head that place `pos`
 // of the launch stands for.
@@ -251,12 +415,7 @@ __device__ __forceinline__ void threshold_block(
     auto few_best = [&](float x) {
         const int ln = tid & 63, wv = tid >> 6;
         const bool rot4 = __builtin_amdgcn_update_dpp(0, ln, 0x124, 0xF, 0xF, true) == (ln ^ 4);
-        tau_wave_stage<2, 1>(x, ln, rot4);
-        tau_wave_stage<4, 2>(x, ln, rot4);
-        tau_wave_stage<8, 4>(x, ln, rot4);
-        tau_wave_stage<16, 8>(x, ln, rot4);
-        tau_wave_stage<32, 16>(x, ln, rot4);
-        tau_wave_stage<64, 32>(x, ln, rot4);
+        x = tau_wave_sort(x, ln, rot4);
         if (ln < 16) s_sc[1][wv * 16 + ln] = x;
         __syncthreads();
         if (wv != 0) return;

@@ -536,7 +536,7 @@ class DecodePlan:
                     queue_len: Optional[int] = None, append=None) -> torch.Tensor:
         """A decode step whose thresholds come from a key sample (T, S, D), tree dtype,
         contiguous: ``hira_search_sampled`` ("sample_max" or "sample_mean_topk" with k) writes them
-        into a buffer of the plan and searches with them, two launches of one call.  Returns that buffer.
+        into a buffer of the plan and searches with them, one or two launches of one call.  Returns that buffer.
         ``append`` = (new_keys (T, m, D), new_values (T, m, Dv) or None, state): the step first
         appends these rows to the index (``hira_update``'s arguments), in the launch that takes
         the thresholds (``hira_update_threshold``)."""

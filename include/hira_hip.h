@@ -172,12 +172,13 @@ const char* hira_last_error(void);
 const float* hira_unit_scale(void);
 
 /* Bytes of workspace hira_search needs for this tree/query (arrival counters, one per tree
- * and head pass, at the start; attention partials after them).  The workspace must be ZERO
+ * and head pass, at the start, and for up to 128 query heads 128 bytes a head for hira_search_sampled;
+ * attention partials after them).  The workspace must be ZERO
  * before its first use; every completed call leaves the counters zero again, and they sit
  * at an offset that depends only on the number of trees and head passes, so a workspace can
  * be reused without clearing by any later call with the same trees and heads that needs no
  * more bytes (a tree that grew, a queue that came or went).  Calls with other numbers of
- * trees or head passes have partials where this one has counters: they share a workspace if
+ * trees, heads or head passes have partials where this one has counters: they share a workspace if
  * hira_search_counter_bytes, the counters' part of these bytes, is the same for both, or if each is
  * given the address that lies that far below one place where the partials of all begin.  Two calls that
  * may run concurrently need separate workspaces. */
@@ -354,7 +355,7 @@ int hira_threshold(const void* samples, int32_t dtype, int32_t num_trees, int32_
                    float* tau_out, void* stream);
 
 /*
- * hira_threshold and hira_search of one decode step as one call (two launches on the stream): the thresholds
+ * hira_threshold and hira_search of one decode step as one call (two launches on the stream, or one): the thresholds
  * are written to sample->tau and searched with; query->tau is not read.  Results are those of the two calls.
  * The samples have the tree's dtype, dim and tree count.
  */
@@ -363,7 +364,8 @@ typedef struct HiraSample {
     int32_t num_rows;
     int32_t method;       /* HIRA_TAU_* */
     int32_t k;
-    int32_t reserved_;
+    int32_t wait;         /* 0; where one launch does both: looks at its progress before a workgroup stops
+                             waiting for thresholds and makes them itself (< 0: at once), same results */
     float* tau;           /* (H_q,) */
 } HiraSample;
 int hira_search_sampled(const HiraTree* tree, const HiraQuery* query, const HiraSample* sample,

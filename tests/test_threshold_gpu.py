@@ -177,3 +177,43 @@ def test_decode_step_in_a_hip_graph(gpu_device):
         assert torch.equal(tau, plan.tau_buf), rep
         assert torch.equal(got, want), rep
         assert float(got.abs().max()) > 0
+
+
+@pytest.mark.parametrize("wait", [0, -1, 1])
+@pytest.mark.parametrize(
+    "t,n,d,bf,levels,group,s,k,q_rows",
+    [(8, 4001, 128, 32, 3, 4, 1000, 10, 9),     # sixteen score rounds, several partials a tree, a queue
+     (2, 500, 64, 16, 3, 1, 500, 16, 0),        # one round of scores
+     (1, 300, 128, 32, 2, 16, 1, 1, 0),         # a workgroup a tree, one sample row, a full pass of heads
+     (4, 900, 64, 32, 2, 3, 513, 2, 0),         # the second round holds one row
+     (2, 2000, 128, 16, 4, 8, 1024, 7, 64),     # the largest sample
+     (3, 700, 64, 32, 3, 5, 31, 16, 1)])        # less than a wave of rows
+def test_thresholds_in_the_launch_that_searches(t, n, d, bf, levels, group, s, k, q_rows, wait, gpu_device):
+    """The call that makes its thresholds in the search's launch against the two calls, bit for bit; with
+    workgroups that do not wait (-1) or hardly (1) and make the thresholds themselves as well."""
+    from hira_amd.cache import threshold_finder as tf
+    from hira_amd.indexer.hip import HIPIndexer
+    from hira_amd.searcher.hip import HIPSearcher
+
+    K = torch.from_numpy(bf16_round(clustered_keys(t, n, d, seed=n, clusters=20)))[None].to(torch.bfloat16).cuda()
+    idx = HIPIndexer(levels, 1, bf).build(K, K)
+    samples = K[0][:, torch.randperm(n, generator=torch.Generator().manual_seed(2))[:s].cuda()].contiguous() \
+        if s <= n else K[0].repeat(1, 2, 1)[:, :s].contiguous()
+    queue = dict(queue_keys=K[0][:, :q_rows].contiguous(), queue_values=K[0][:, :q_rows].contiguous()) if q_rows else {}
+    se, h = HIPSearcher(), t * group
+    scale = torch.full((h,), d ** -0.5)
+    plan, other = (se.plan_attention(idx, h, scaling=scale) for _ in range(2))
+    plan.sample.wait = wait
+    got, want = (torch.full((h, d), float("nan"), device="cuda") for _ in range(2))
+    for rep in range(3):
+        q = torch.from_numpy(bf16_round(random_query(h, d, seed=rep))).to(torch.bfloat16).cuda()
+        tau = plan.run_sampled(q, samples, "sample_mean_topk", k, got, **queue)
+        two = tf.sample_mean_topk(samples, q, k)
+        other.run(q, two, want, **queue)
+        torch.cuda.synchronize()
+        assert torch.equal(tau, two.view(-1)), rep
+        assert torch.equal(got, want), rep
+        plan.run(q, two, got, **queue)  # (the arrival counters are back at zero)
+        assert torch.equal(got, want), rep
+        assert int(plan.ws[: 256 + 128 * h].max()) == 0
+        assert torch.isfinite(got).all()
