@@ -75,7 +75,7 @@ class HiraQueue(C.Structure):
 
 class HiraSample(C.Structure):
     _fields_ = [("rows", _vp), ("num_rows", C.c_int32), ("method", C.c_int32), ("k", C.c_int32),
-                ("wait", C.c_int32), ("tau", _vp)]
+                ("wait", C.c_int32), ("tau", _vp), ("scratch", _vp)]
 
 
 class HiraSearchOut(C.Structure):

@@ -239,15 +239,10 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
 
 using namespace hira;
 
-// The arrival counters of the fused fold and the scores that a launch with its own thresholds hands over, both zero
-// between calls, then the partials (acc, m, l).  The former come first: their place does not depend on the
-// number of partials, so a workspace stays usable when the tree grows or a queue comes and goes.
-constexpr int kSampledHeads = 128;  // (two workgroups a head and a compute unit each: more heads make no such launch)
-static size_t arrival_bytes(int trees, int passes) {
+// The arrival counters of the fused fold, then the partials (acc, m, l).  The counters come first: their place does
+// not depend on the number of partials, so a workspace stays usable when the tree grows or a queue comes and goes.
+static size_t counter_bytes(int trees, int passes) {
     return (((size_t)trees * passes * sizeof(int32_t)) + 255) & ~(size_t)255;
-}
-static size_t counter_bytes(int trees, int passes, int h_q) {
-    return arrival_bytes(trees, passes) + (h_q <= kSampledHeads ? ((size_t)h_q * 32 * sizeof(float) + 255) & ~(size_t)255 : 0);
 }
 static size_t partial_bytes(int h_q, size_t P, int vdim) { return (size_t)h_q * P * (size_t)(vdim + 2) * sizeof(float); }
 
@@ -257,14 +252,14 @@ extern "C" size_t hira_search_workspace_bytes(const HiraTree* tree, const HiraQu
     SearchPlan plan;
     if (make_plan(tree, query, queue, launch, true, &plan) != HIRA_OK) return 0;
     const size_t P = (size_t)plan.tree_blocks + plan.queue_blocks;
-    return counter_bytes(tree->num_trees, plan.head_chunks, query->num_q_heads) + partial_bytes(query->num_q_heads, P, tree->vdim);
+    return counter_bytes(tree->num_trees, plan.head_chunks) + partial_bytes(query->num_q_heads, P, tree->vdim);
 }
 
 /* see include/hira_hip.h */
 extern "C" size_t hira_search_counter_bytes(const HiraTree* tree, const HiraQuery* query, const HiraLaunch* launch) {
     SearchPlan plan;
     if (make_plan(tree, query, nullptr, launch, true, &plan) != HIRA_OK) return 0;
-    return counter_bytes(tree->num_trees, plan.head_chunks, query->num_q_heads);
+    return counter_bytes(tree->num_trees, plan.head_chunks);
 }
 
 // Does this search make its thresholds itself (threshold_stretch)?  What that is written for, under a
@@ -273,7 +268,7 @@ extern "C" size_t hira_search_counter_bytes(const HiraTree* tree, const HiraQuer
 // place would begin when the stretches are done, as in a launch of its own.
 constexpr int kSampleWait = 1 << 14;  // looks at the counter; one takes about a microsecond
 static bool sampled_in_one(const SearchPlan& plan, const SearchParams& p, const HiraTree* tree, const HiraSample* sample) {
-    if (p.group_size * tree->num_trees > kSampledHeads) return false;
+    if (sample->scratch == nullptr) return false;
     return plan.kernel == 2 && plan.ahead && plan.tree_blocks > 0 && plan.key_policy == 0 && p.keys8 == nullptr && tree->bf <= 16 * kSampledTiles &&
            tree->dim <= 128 && p.done != nullptr && p.dense == nullptr && p.sel_count == nullptr && plan.head_chunks == 1 &&
            p.group_size > 0 && p.group_size <= 16 && sample->method == HIRA_TAU_SAMPLE_MEAN_TOPK && sample->k <= 16 &&
@@ -379,7 +374,7 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
     if (P == 0) return sample ? thresholds_ahead() : HIRA_OK;
     p.num_parts = P;
     if (attn) {
-        size_t ctr_bytes = counter_bytes(tree->num_trees, plan.head_chunks, query->num_q_heads);
+        size_t ctr_bytes = counter_bytes(tree->num_trees, plan.head_chunks);
         if (fixed_counters > 0) {
             if ((size_t)tree->num_trees * plan.head_chunks > fixed_counters)
                 return fail(HIRA_EWORKSPACE, "%d trees x %d head passes: more than the %zu arrival "
@@ -417,7 +412,7 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (sample && sampled_in_one(plan, p, tree, sample)) {
         p.sample_wgs = p.group_size * (sample->num_rows > kTauStretch ? 2 : 1);
-        p.sample_best = reinterpret_cast<float*>(static_cast<char*>(workspace) + arrival_bytes(tree->num_trees, plan.head_chunks));
+        p.sample_best = sample->scratch;
         p.sample = sample->rows;
         p.sample_rows = sample->num_rows;
         p.sample_k = sample->k;

@@ -469,6 +469,9 @@ class DecodePlan:
         self._ws_rows = 1  # queue rows the workspace is sized for
         self.ws_bytes = self._workspace_need()
         self.ws = torch.zeros(max(self.ws_bytes, 1), dtype=torch.uint8, device=dev)
+        # (zero once: a launch that makes its thresholds hands them over in it and leaves it at zero)
+        self.tau_scratch = torch.zeros((num_q_heads, 32), dtype=torch.float32, device=dev)
+        self.sample.scratch = self.tau_scratch.data_ptr()
         self._refs = (C.byref(self.tree), C.byref(self.query), C.byref(self.out),
                       C.byref(self.launch), C.byref(self.queue))
 

@@ -172,13 +172,12 @@ const char* hira_last_error(void);
 const float* hira_unit_scale(void);
 
 /* Bytes of workspace hira_search needs for this tree/query (arrival counters, one per tree
- * and head pass, at the start, and for up to 128 query heads 128 bytes a head for hira_search_sampled;
- * attention partials after them).  The workspace must be ZERO
+ * and head pass, at the start; attention partials after them).  The workspace must be ZERO
  * before its first use; every completed call leaves the counters zero again, and they sit
  * at an offset that depends only on the number of trees and head passes, so a workspace can
  * be reused without clearing by any later call with the same trees and heads that needs no
  * more bytes (a tree that grew, a queue that came or went).  Calls with other numbers of
- * trees, heads or head passes have partials where this one has counters: they share a workspace if
+ * trees or head passes have partials where this one has counters: they share a workspace if
  * hira_search_counter_bytes, the counters' part of these bytes, is the same for both, or if each is
  * given the address that lies that far below one place where the partials of all begin.  Two calls that
  * may run concurrently need separate workspaces. */
@@ -367,6 +366,9 @@ typedef struct HiraSample {
     int32_t wait;         /* 0; where one launch does both: looks at its progress before a workgroup stops
                              waiting for thresholds and makes them itself (< 0: at once), same results */
     float* tau;           /* (H_q,) */
+    float* scratch;       /* NULL: two launches; or (H_q, 32), ZERO before its first use and left zero by every
+                             completed call: small searches then make the thresholds in their own launch.  Two
+                             calls that may run concurrently need separate ones. */
 } HiraSample;
 int hira_search_sampled(const HiraTree* tree, const HiraQuery* query, const HiraSample* sample,
                         const HiraQueue* queue, const HiraSearchOut* out, const HiraLaunch* launch,

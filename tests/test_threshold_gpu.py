@@ -215,5 +215,5 @@ def test_thresholds_in_the_launch_that_searches(t, n, d, bf, levels, group, s, k
         assert torch.equal(got, want), rep
         plan.run(q, two, got, **queue)  # (the arrival counters are back at zero)
         assert torch.equal(got, want), rep
-        assert int(plan.ws[: 256 + 128 * h].max()) == 0
+        assert int(plan.ws[: 4 * t].max()) == 0 and not plan.tau_scratch.any()
         assert torch.isfinite(got).all()
