@@ -263,14 +263,16 @@ extern "C" size_t hira_search_counter_bytes(const HiraTree* tree, const HiraQuer
 }
 
 // Does this search make its thresholds itself (threshold_stretch)?  What that is written for, under a
-// kernel of one tile a workgroup that asks for its keys ahead, the fold in the launch, nothing but attention, and a
+// kernel that asks for its keys ahead, the fold in the launch, nothing but attention, and a
 // compute unit for every workgroup: the kernel runs one at a time on a compute unit, and one that had to wait for a
 // place would begin when the stretches are done, as in a launch of its own.
 constexpr int kSampleWait = 1 << 14;  // looks at the counter; one takes about a microsecond
 static bool sampled_in_one(const SearchPlan& plan, const SearchParams& p, const HiraTree* tree, const HiraSample* sample) {
     if (sample->scratch == nullptr) return false;
-    return plan.kernel == 2 && plan.ahead && plan.tree_blocks > 0 && plan.key_policy == 0 && p.keys8 == nullptr && tree->bf <= 16 * kSampledTiles &&
-           tree->dim <= 128 && p.done != nullptr && p.dense == nullptr && p.sel_count == nullptr && plan.head_chunks == 1 &&
+    const bool kernel = plan.kernel == 2 ? plan.key_policy == 0 && p.keys8 == nullptr && tree->bf <= 16 * kSampledTiles
+                                         : plan.lpr * 8 == tree->dim;
+    return kernel && plan.ahead && plan.tree_blocks > 0 && tree->dtype == HIRA_BF16 && (tree->dim == 64 || tree->dim == 128) &&
+           p.done != nullptr && p.dense == nullptr && p.sel_count == nullptr && plan.head_chunks == 1 &&
            p.group_size > 0 && p.group_size <= 16 && sample->method == HIRA_TAU_SAMPLE_MEAN_TOPK && sample->k <= 16 &&
            sample->num_rows <= kTauFewRows && (2 * p.group_size + p.num_parts) * tree->num_trees <= compute_units();
 }
@@ -421,7 +423,7 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
         rc = thresholds_ahead();
         if (rc != HIRA_OK) return rc;
     }
-    dim3 grid(P, tree->num_trees, plan.head_chunks);
+    dim3 grid(P + p.sample_wgs, tree->num_trees, plan.head_chunks);
     if (plan.kernel == 2)
         rc = launch_search_mfma(plan, p, dim3(tree->num_trees, P + p.sample_wgs, plan.head_chunks), s);
     else

@@ -1381,16 +1381,8 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         }
     }
     tline.stamp(kTlStoresIssued);
-    // (SAMPLED) my ticket, by wave 0; behind the last of all the tree's counter and scores go back to zero
-    auto sampled_ticket = [&] {
-        int before = 0;
-        if (lane == 0) before = __hip_atomic_fetch_add(p.done + tree, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        before = __builtin_amdgcn_readfirstlane(before);
-        if (before + 1 == wgs + p.sample_wgs * kTauMade) threshold_reset(p.sample_best + (size_t)hoff * 32, G * 32, p.done + tree);
-        return (before & (kTauMade - 1)) == wgs - 1;
-    };
     if constexpr (SAMPLED) {
-        if (alone && wave == 0) sampled_ticket();
+        if (alone && wave == 0) sampled_ticket(p, tree, wgs, hoff, G);
     }
     if (p.done == nullptr || alone) return;  // the caller folds the partials in a second launch, or there is one
 
@@ -1400,7 +1392,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     __syncthreads();
     if constexpr (SAMPLED) {
         if (wave == 0) {
-            const bool last = sampled_ticket();
+            const bool last = sampled_ticket(p, tree, wgs, hoff, G);
             if (lane == 0) s_last = last;
         }
     } else if (threadIdx.x == 0) {

@@ -29,6 +29,7 @@
 // select a key when q.k >= tau.
 #pragma once
 #include "search.h"
+#include "threshold_kernel.h"
 
 namespace hira {
 
@@ -301,7 +302,9 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
 // operands of all levels, whether the nodes survive or not: no list, two trips to memory and a barrier less,
 // and no loop, at whose head the waits would be for everything asked for so far.  Every row being in some
 // wave's block, a dense output's fill value goes out with the scores.
-template <typename T, int LPR, int GMAX, int ONE>
+// SAMPLED: (with ONE, bf16 rows of 8 * LPR columns) the launch makes its thresholds itself, in workgroups ahead of the
+// searching ones of a tree (threshold_stretch); a workgroup looks for them with its keys on their way.
+template <typename T, int LPR, int GMAX, int ONE, bool SAMPLED = false>
 __global__ __launch_bounds__(kVecThreads) __attribute__((amdgpu_waves_per_eu(GMAX == 1 ? 3 : 2)))
 void search_kernel(const SearchParams p) {
     constexpr int EPL = Elem<T>::kPerChunk;
@@ -321,6 +324,8 @@ void search_kernel(const SearchParams p) {
     __shared__ uint32_t s_pass[HIRA_MAX_LEVELS][kBatch + 1];  // heads a row passes for | 1 << 31: not empty
     __shared__ uint32_t s_list[kBatch];  // survivors: node - first | child count << 8 | heads << 16
     __shared__ int s_count;
+    static_assert(!SAMPLED || (ONE > 0 && sizeof(T) == 2 && kVecThreads == kTauStretch), "");
+    __shared__ float s_tau[SAMPLED ? GMAX : 1], s_scores[SAMPLED ? kTauFewRows : 1];
 
     touch_kernel_arguments();
     const int lane = lane_id();
@@ -344,11 +349,23 @@ void search_kernel(const SearchParams p) {
     const int hoff = (by_group ? tree * p.group_size : p.tree_q_off[tree]) + blockIdx.z * GMAX;
     const int G = min(GMAX, (by_group ? (tree + 1) * p.group_size : p.tree_q_off[tree + 1]) - hoff);
     if (G <= 0) return;  // uniform for the workgroup
+    int wgs = gridDim.x, wg = blockIdx.x;  // searching workgroups of the tree, my number among them
+    if constexpr (SAMPLED) {
+        wgs -= p.sample_wgs;
+        wg -= p.sample_wgs;
+        if (wg < 0) {  // uniform
+            threshold_stretch<LPR>(p.sample, p.sample_rows, p.q, tree, G, (int)blockIdx.x, p.sample_best, s_scores, p.done + tree,
+                                   wgs + p.sample_wgs * kTauMade);
+            return;
+        }
+    }
+    // (what a launch that makes its thresholds keeps lies where the others have their dense output)
+    const bool dense = !SAMPLED && p.dense != nullptr, lists = !SAMPLED && p.sel_count != nullptr;
     const unsigned gmask = (1u << G) - 1u;
     auto head_of = [&](int g) { return by_group ? hoff + g : p.tree_q_heads[hoff + g]; };
 
-    const bool is_queue = (int)blockIdx.x >= p.tree_blocks;
-    const int blk = is_queue ? (int)blockIdx.x - p.tree_blocks : (int)blockIdx.x;
+    const bool is_queue = wg >= p.tree_blocks;
+    const int blk = is_queue ? wg - p.tree_blocks : wg;
     const int n_nodes = is_queue ? p.num_queue_blocks : p.num_nodes;
     const bool real_nodes = !is_queue && L >= 2;
     const int wg_nodes = is_queue ? p.queue_nodes : p.nodes_per_wg;
@@ -388,11 +405,11 @@ void search_kernel(const SearchParams p) {
 #pragma unroll
     for (int g = 0; g < GMAX; ++g) {
         qraw[g] = load_chunk<T>(p.q, (size_t)hd[g] * D, chunk_ok ? ch : 0);
-        tau[g] = p.tau[hd[g]];
+        tau[g] = SAMPLED ? 0.0f : p.tau[hd[g]];
     }
 #pragma unroll
     for (int i = 0; i < KEPT; ++i) {
-        my_tau[i] = p.tau[my_h[i]];
+        my_tau[i] = SAMPLED ? 0.0f : p.tau[my_h[i]];
         my_sc[i] = p.scaling[my_h[i]];
     }
 
@@ -450,7 +467,7 @@ void search_kernel(const SearchParams p) {
         const uint64_t B = __ballot(owner && sel != 0u);  // lanes that hold a selected score
         if constexpr (ONE) {
             // (every row of the workgroup's nodes is in some wave's block: fill value or score)
-            if (p.dense != nullptr && p.dense_fill && !is_queue && owner && my_row) {
+            if (dense && p.dense_fill && !is_queue && owner && my_row) {
 #pragma unroll
                 for (int i = 0; i < KEPT; ++i)
                     if (my_g + i < G)
@@ -471,15 +488,15 @@ void search_kernel(const SearchParams p) {
             }
             if (owner && sel) count(HIRA_MAX_LEVELS + 1, (unsigned)__popc(sel));
         }
-        if (!is_queue && (p.dense != nullptr || p.sel_count != nullptr)) {
+        if (!is_queue && (dense || lists)) {
             int idx = my_slot;
             if (owner && sel && p.dense_by_position) idx = p.perm[krow0 + my_slot];
-            if (p.dense != nullptr && owner && !(ONE && p.dense_fill)) {
+            if (dense && owner && !(ONE && p.dense_fill)) {
 #pragma unroll
                 for (int i = 0; i < KEPT; ++i)
                     if ((sel >> i) & 1u) p.dense[(int64_t)my_h[i] * p.dense_stride + idx] = s[i] * my_sc[i];
             }
-            if (p.sel_count != nullptr) {
+            if (lists) {
 #pragma unroll
                 for (int i = 0; i < KEPT; ++i) {
                     const uint64_t Bi = __ballot(owner && ((sel >> i) & 1u));
@@ -680,6 +697,19 @@ void search_kernel(const SearchParams p) {
         for (int u = 0; u < KU; ++u) kraw[u] = row_at(kbase, klayout, krow0, min(slot0 + u * RPW, n_rows - 1));
         __builtin_amdgcn_sched_barrier(0);  // (nothing that uses a load moves above this line)
         queries();
+        if constexpr (SAMPLED) {
+            if (real_nodes) {  // uniform
+                if (wave == 0)
+                    threshold_join<LPR, (GMAX < 4 ? 4 : GMAX)>(p.sample, p.sample_rows, p.q, tree, hoff, G, p.sample_k, p.sample_best,
+                                                               p.sample_wait, s_tau, s_scores);
+                __syncthreads();
+                if (wg == 0 && wave == 0 && lane < G) const_cast<float*>(p.tau)[hoff + lane] = s_tau[lane];
+#pragma unroll
+                for (int g = 0; g < GMAX; ++g) tau[g] = s_tau[min(g, G - 1)];
+#pragma unroll
+                for (int i = 0; i < KEPT; ++i) my_tau[i] = s_tau[min(my_g + i % GMAX, G - 1)];
+            }
+        }
         unsigned alive = gmask;
         if (real_nodes) {  // uniform
             if (wave * RPW < rows2) judge(2, rows2, r0, chunk_ok ? raw2 : none, rad2);  // (uniform in the wave)
@@ -932,7 +962,7 @@ void search_kernel(const SearchParams p) {
                 lsum += lw[w] * f;
             }
         }
-        const size_t slot = (size_t)head_of(g) * p.num_parts + blockIdx.x;
+        const size_t slot = (size_t)head_of(g) * p.num_parts + wg;
         // device-scope stores: written through, so that the workgroup that folds the partials
         // (maybe behind another L2) reads them without cache-wide flushes
         if (mall > -INFINITY)
@@ -948,7 +978,12 @@ void search_kernel(const SearchParams p) {
     __shared__ int s_last;
     hand_off_release();
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if constexpr (SAMPLED) {
+        if (wave == 0) {
+            const bool last = sampled_ticket(p, tree, wgs, hoff, G);
+            if (lane == 0) s_last = last;
+        }
+    } else if (threadIdx.x == 0) {
         int* ctr = p.done + (size_t)tree * gridDim.z + blockIdx.z;
         const int ticket = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s_last = ticket == (int)gridDim.x - 1;
@@ -964,6 +999,13 @@ inline void launch_search(const SearchPlan& plan, const SearchParams& p, dim3 gr
     const size_t smem = p.part_acc ? plan.smem : 0;
     const dim3 block(plan.threads);
     // (a block of the larger kind holds more scores a lane than eight heads leave registers for)
+    if constexpr (sizeof(T) == 2 && (LPR == 8 || LPR == 16)) {
+        if (p.sample_wgs > 0) {
+            if (plan.ahead == kOneSmall) hipLaunchKernelGGL((search_kernel<T, LPR, GMAX, kOneSmall, true>), grid, block, smem, s, p);
+            else hipLaunchKernelGGL((search_kernel<T, LPR, GMAX, (GMAX <= 4 ? kOneLarge : kOneSmall), true>), grid, block, smem, s, p);
+            return;
+        }
+    }
     if (plan.ahead == kOneSmall) hipLaunchKernelGGL((search_kernel<T, LPR, GMAX, kOneSmall>), grid, block, smem, s, p);
     else if (plan.ahead) hipLaunchKernelGGL((search_kernel<T, LPR, GMAX, (GMAX <= 4 ? kOneLarge : kOneSmall)>), grid, block, smem, s, p);
     else hipLaunchKernelGGL((search_kernel<T, LPR, GMAX, 0>), grid, block, smem, s, p);

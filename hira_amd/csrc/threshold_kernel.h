@@ -4,7 +4,7 @@
 #pragma once
 #include <type_traits>
 
-#include "common.hip.h"
+#include "search.h"
 
 namespace hira {
 
@@ -240,7 +240,8 @@ __device__ __forceinline__ float tau_wave_sort(float x, int ln, bool rot4) {
 // arithmetic is threshold_block's, the same bits.
 // us, two launches / this, 8 trees x 4 heads, 1000 samples: 4001 rows of 128 columns 15.0 / 12.3 (waiting for a
 // counter and then asking for the scores 15.3), 8000 16.6 / 13.6, 1000 14.0 / 11.0, 4001 x 64 13.0 / 10.8;
-// 8 heads a tree 16.9 / 14.4; 300 rows, as many samples 12.0 / 9.4.  What bounds it is the chain: arguments, one trip and
+// 8 heads a tree 16.9 / 14.4; 300 rows, as many samples 12.0 / 9.4; on the vector units 2 trees x 4 heads,
+// 1111 rows of 64 columns in five levels 15.4 / 12.5.  What bounds it is the chain: arguments, one trip and
 // half the sample through a compute unit's L1, the sorts (some 6 us from the start), two trips of the hand-over,
 // then the search from its gates on.
 //   best    (H_q, 2, 16) scores, largest first; 0 between launches, which says: not there yet (a score of 0 is
@@ -381,6 +382,16 @@ __device__ __forceinline__ void threshold_join(const void* samples, int S, const
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+}
+
+// The ticket of one of a tree's `wgs` searching workgroups, by its first wave: is it the last of them?  Behind the
+// last of all, stretches too, the tree's counter and scores go back to zero.
+__device__ __forceinline__ bool sampled_ticket(const SearchParams& p, int tree, int wgs, int head0, int G) {
+    int before = 0;
+    if ((threadIdx.x & 63) == 0) before = __hip_atomic_fetch_add(p.done + tree, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    before = __builtin_amdgcn_readfirstlane(before);
+    if (before + 1 == wgs + p.sample_wgs * kTauMade) threshold_reset(p.sample_best + (size_t)head0 * 32, G * 32, p.done + tree);
+    return (before & (kTauMade - 1)) == wgs - 1;
 }
 
 // E = registers per thread of the sort: the padded array has 1024 * E entries

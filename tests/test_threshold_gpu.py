@@ -187,7 +187,13 @@ def test_decode_step_in_a_hip_graph(gpu_device):
      (1, 300, 128, 32, 2, 16, 1, 1, 0),         # a workgroup a tree, one sample row, a full pass of heads
      (4, 900, 64, 32, 2, 3, 513, 2, 0),         # the second round holds one row
      (2, 2000, 128, 16, 4, 8, 1024, 7, 64),     # the largest sample
-     (3, 700, 64, 32, 3, 5, 31, 16, 1)])        # less than a wave of rows
+     (3, 700, 64, 32, 3, 5, 31, 16, 1),         # less than a wave of rows
+     # on the vector units (other fan-outs): both blocks, one to eight heads a pass
+     (2, 1111, 64, 10, 5, 4, 1000, 10, 0),
+     (4, 3000, 128, 10, 4, 3, 513, 16, 23),
+     (8, 300, 64, 4, 2, 1, 300, 3, 5),
+     (2, 2500, 128, 7, 3, 8, 1024, 1, 0),
+     (2, 5003, 64, 24, 3, 1, 100, 10, 40)])
 def test_thresholds_in_the_launch_that_searches(t, n, d, bf, levels, group, s, k, q_rows, wait, gpu_device):
     """The call that makes its thresholds in the search's launch against the two calls, bit for bit; with
     workgroups that do not wait (-1) or hardly (1) and make the thresholds themselves as well."""
