@@ -889,6 +889,7 @@ class HIPIndexer(BaseIndexer):
             size = most[: self.num_levels]
             size[0] = size[1] * self.branching_factor
         self._pending, self._exact_size = 0, None
+        self._append = None  # (it counted from the sizes before)
         if size != self.size:
             self.size = size
             self._sizes_changed()

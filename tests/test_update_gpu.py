@@ -593,3 +593,23 @@ def test_appends_that_describe_the_last_one_again(bf, levels, m, gpu_device):
     for a, b in zip([kept.perm, kept.keys_buf, kept.values_buf] + kept.centers[1:] + kept.radii[1:] + kept.counts[1:],
                     [anew.perm, anew.keys_buf, anew.values_buf] + anew.centers[1:] + anew.radii[1:] + anew.counts[1:]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("bf,levels,m", [(16, 2, 8), (10, 3, 13)])
+def test_an_append_with_a_read_back_between_appends_without(bf, levels, m, gpu_device):
+    """What an append without a read-back found out is void after one with: every key is under a node that
+    the bounds of the level sizes know."""
+    from hira_amd.indexer import HIPIndexer
+
+    n = 10 * bf  # (every level-1 node may be full)
+    k, v = torch.randn(2, 1, 2, n + 1 + m + 3 * bf, 64, device="cuda").to(torch.bfloat16)
+    idx = HIPIndexer(levels, 1, bf).build(k[:, :, :n], v[:, :, :n])
+    part = lambda x, a, b: x[:, :, a:b].contiguous()
+    idx.update(part(k, n, n + 1), part(v, n, n + 1), sync=False)
+    idx.update(part(k, n + 1, n + 1 + m), part(v, n + 1, n + 1 + m))
+    for at in range(n + 1 + m, n + 1 + m + 3 * bf):
+        idx.update(part(k, at, at + 1), part(v, at, at + 1), sync=False)
+        used = idx._state.cpu()[:, 1:levels].max(dim=0).values.tolist()
+        assert all(u <= b for u, b in zip(used, idx.size[1:])), (at, used, idx.size)
+    idx.sync_sizes()
+    assert idx.num_keys == k.shape[2] and (idx.perm >= 0).sum() == 2 * idx.num_keys
