@@ -203,7 +203,7 @@ struct AssignJob {
 // Grids of `blocks` workgroups to each of `trees` trees, trees in the fast index: workgroups go to the eight XCDs in
 // turn by their number, so a tree's run behind the same L2s in one launch after the other, and what a launch
 // wrote is there for the next.  (Trees in the slow index: every tile and bucket came from another XCD's L2 or
-// from memory; 8 x 32768 keys NEW us a build.)
+// from memory; builds of 8 x 32768 keys 729 -> 703 us, of 8 x 131072 3440 -> 3410.)
 static inline dim3 tree_grid(long long blocks, int trees) {
     const long long y = blocks < 32768 ? (blocks > 0 ? blocks : 1) : 32768;
     return dim3((unsigned)trees, (unsigned)y, (unsigned)((blocks + y - 1) / y > 0 ? (blocks + y - 1) / y : 1));

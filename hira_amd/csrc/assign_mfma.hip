@@ -668,7 +668,7 @@ __device__ __forceinline__ void approx_items(const AssignJob& job, int Kt, int t
     for (int ri = 0; ri < RI; ++ri) acc[1][ri] = af32x4_t{-3e38f, -3e38f, -3e38f, -3e38f};
     uint32_t keep_v;  // (in a vector register: with `tag` in a scalar one the bits are one instruction)
     asm volatile("v_mov_b32 %0, %1" : "=v"(keep_v) : "s"(keep));
-    // The four results of an item tile in nine steps: tagged, then two at a time into best and second.  With
+    // The four results of an item tile in LOOKS steps: tagged, then two at a time into best and second.  With
     // best >= second the two largest of {best, second, u, v} are max3(best, u, v) and
     // max(med3(best, u, v), second), and the maxima of `second` of both pairs are one instruction.
     // (Asm: fmaxf quiets its operands first, an instruction each.)

@@ -914,10 +914,11 @@ static void cluster_counts(int n, int bf, int L, int* K) {
 // round what its items take one compute unit, the launches what launches take.  Trees x items x centroids (128
 // columns), launches / one workgroup a tree, of a build of that level alone: 8 x 1024 x 32 164 / 126 us,
 // 64 x 1024 x 32 203 / 141, 8 x 512 x 16 139 / 69, 8 x 1024 x 16 183 / 105.  With more centroids a wave
-// takes them in turns (8 x 512 x 64: 134 / 147); rows of 256 columns: no gain left at 1024 x 32 (174 / 175).
+// takes them in turns (8 x 512 x 64: 134 / 147); rows of 256 columns, whose
+// operands are twice as many: up to 512 x 16.
 static bool level_is_small(const HiraTree* t, int n_c, int K) {
     return assign_exact_on_mfma(t->dtype, t->dim) && n_c <= kSmallItems && K <= kSmallCentroids &&
-           n_c * K <= (t->dim <= 128 ? small_pairs(t->dim) : 8192);
+           n_c * K <= small_pairs(t->dim);
 }
 
 static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {

@@ -8,7 +8,7 @@ namespace hira {
 
 constexpr int kSmallItems = 1024;      // what its LDS has room for
 constexpr int kSmallCentroids = 32;
-constexpr int small_pairs(int D) { return D <= 128 ? 32768 : 16384; }  // items times centroids
+constexpr int small_pairs(int D) { return D <= 128 ? 32768 : 8192; }  // items times centroids
 
 struct SmallLevels {
     const void* x;                     // (T, K[first - 1], D) bf16 items of level `first`

@@ -9,7 +9,7 @@
 // centroids are made once and stay in LDS (128 KiB for 1024 items and 32 centroids), and so do the centroids'
 // operand tiles, the lists and the slots: a round of packing touches no memory.  What bounds it is the chain of
 // barriers and, for the first assignment, the means, the scores and the block centres, trips to the level-2 cache.
-// A level of 8 trees: 1024 items and 32 centroids 115 us (rounds 3-14), 128 and 4 20 us (rounds 1.5; with tiles and
+// A level of 8 trees: 1024 items and 32 centroids 94 us (rounds 3-14), 128 and 4 20 us (rounds 1.5; with tiles and
 // scores in memory, made anew every round, 32).  Builds, launches / with that / this: 2 x 1111 keys of 64 columns, five
 // levels, fan-out 10: 426 / 207 / 181 us; 8 x 500, three levels, fan-out 32: 228 / 116 / 81; 8 x 8192, three levels,
 // fan-out 32, the second level here: - / 395 / 365.

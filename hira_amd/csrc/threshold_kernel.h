@@ -56,20 +56,6 @@ __device__ __forceinline__ void tau_wave_stage(float& x, int ln, bool rot4_first
     if constexpr (J > 1) tau_wave_stage<LEN, J / 2>(x, ln, rot4_first);
 }
 
-// maximum over the wave: inside the rows of 16 by data-path moves, the four rows by reading
-// one lane of each
-__device__ __forceinline__ float tau_wave_max(float v, bool rot4_first) {
-    v = fmaxf(v, tau_partner<1>(v, rot4_first));
-    v = fmaxf(v, tau_partner<2>(v, rot4_first));
-    v = fmaxf(v, tau_partner<4>(v, rot4_first));
-    v = fmaxf(v, tau_partner<8>(v, rot4_first));
-    const float r0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
-    const float r1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
-    const float r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
-    const float r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
-    return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
-}
-
 // One step of the bitonic sort (largest first) of 256 * EE entries, entry e*256 + tid in v[e]
 // of thread tid < 256: entry i meets entry i ^ J; in a stretch that ends up descending
 // ((i & LEN) == 0) the lower index keeps the larger value.  Every thread of the workgroup

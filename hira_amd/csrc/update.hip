@@ -97,8 +97,8 @@ __device__ __forceinline__ void replace_sample(const UpdateParams& p, const Samp
 __device__ __forceinline__ float pad_up(float r) { return r > 0.0f ? r * (1.0f + 4.0f * 1.1920929e-7f) + 1e-30f : r; }
 
 // Nearest node of level l (among nodes first .. used - 1; the ones before `first` are known to
-// be full) with a free child slot; -1 if none.  Wave w scans nodes w, w+4, ...; a full node
-// costs one count read.  Ties go to the lowest id.  *not_full (if given) receives the lowest
+// be full) with a free child slot; -1 if none.  Waves take stretches of 64 nodes in turn; a full
+// node costs one count read.  Ties go to the lowest id.  *not_full (if given) receives the lowest
 // index from `first` on whose node is not full (`used` if there is none).
 constexpr int kCountsInFlight = 16;  // reads of child counts a lane has in flight
 template <typename T, int NT>
@@ -116,7 +116,7 @@ __device__ __forceinline__ int nearest_with_room(const UpdateParams& p, int tree
     int low = used;  // lowest index of a node that is not full, among those I have seen
     for (int nb = (first & ~63) + wave * 64; nb < used; nb += kCountsInFlight * NT) {
         // the reads of the child counts in flight together (a wave's nodes still come in
-        // increasing order): one trip to memory for 4096 nodes
+        // increasing order): one trip to memory for 16 NT nodes
         int c4[kCountsInFlight];
 #pragma unroll
         for (int u = 0; u < kCountsInFlight; ++u) {
@@ -412,8 +412,6 @@ __global__ __launch_bounds__(kTauThreads) void k_update_threshold(
                           tau, (int)blockIdx.x - trees);
 }
 
-// The general way as a call (the kernel below needs it now and then: its loop stays small, and the
-// compiler keeps the loop's values in registers instead of asking for them again every key).
 // ---- windows of several keys ---------------------------------------------------------------
 // Placing a key the general way costs a handful of dependent trips to memory (child counts,
 // the centres of the nodes with room, the ancestors' centres and radii): 4-5 us a key, one key
