@@ -17,7 +17,7 @@ HIRA_MAX_LEVELS = 8
 HIRA_STATS_COLS = HIRA_MAX_LEVELS + 3  # counters per tree a search can fill in
 HIRA_F32, HIRA_BF16 = 0, 1
 HIRA_ROW_MAJOR, HIRA_TILE16, HIRA_TILE16_Q8 = 0, 1, 2
-HIRA_ABI_VERSION = 11
+HIRA_ABI_VERSION = 12
 HIRA_UNIT_SCALE_HEADS = 4096
 
 _vp = C.c_void_p
@@ -164,6 +164,9 @@ SYMBOLS = {
         C.c_int,
         [C.POINTER(HiraTree), _vp, _vp, C.c_int32, _vp, _vp, C.c_int32, C.POINTER(C.c_int32),
          C.POINTER(C.c_int32), C.c_int32, _vp],
+    ),
+    "hira_read_state": (
+        C.c_int, [C.POINTER(HiraTree), _vp, _vp, C.c_uint32, C.POINTER(C.c_int32), _vp],
     ),
     "hira_update_state": (C.c_int, [C.POINTER(HiraTree), C.c_int32, _vp, _vp]),
     "hira_sparse_attention": (

@@ -24,6 +24,9 @@
 // [0] (trees of two or more levels): every level-1 node with a lower index is full -- a lower
 // bound that the search for a node with room starts from and raises as it learns more (0 is
 // always valid; whoever lowers a count of a level-1 node from outside must lower it too).
+#include <algorithm>
+#include <chrono>
+
 #include "rows.h"
 #include "threshold_kernel.h"
 
@@ -1446,6 +1449,59 @@ extern "C" int hira_update_sample(const HiraTree* tree, const void* new_keys, co
     if (n > 0 && !along)
         return hira_replace_rows(sample, tree->dtype, tree->dim, tree->num_trees, rows_per_tree, new_keys, m, m, slot_host,
                                  from_host, n, stream);
+    return HIRA_OK;
+}
+
+namespace hira {
+// The state rows to the host that waits for them.  Value and ticket are one store of eight bytes, so nothing has to be
+// ordered before it (a fence of the system's scope writes the L2 back, some 10 us).
+__global__ __launch_bounds__(256) void k_tell_host(const int32_t* state, uint64_t* rows, uint32_t ticket, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n)
+        __hip_atomic_store(rows + i, ((uint64_t)ticket << 32) | (uint32_t)state[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+}  // namespace hira
+
+// A launch behind the append's writes the rows into host memory, which the host watches: what ran before on the stream
+// is over when they are there, as behind a copy that is waited for.  8 trees, windows of 64 keys, a call: 25 us; with
+// the runtime's wait for the stream instead of the watching 28, a copy to the host and its wait 31; with rows that the
+// append's launch writes itself 21, but then the caller goes on while that launch still runs.
+// The host watches for as long as an append takes behind little else on its stream, then it leaves the waiting to the
+// runtime.
+constexpr std::chrono::microseconds kWatch(500);
+
+/* see include/hira_hip.h */
+extern "C" int hira_read_state(const HiraTree* tree, const int32_t* state, uint64_t* host_rows, uint32_t ticket, int32_t* most,
+                               void* stream) {
+    HIRA_CHECK_ARG(tree && state && host_rows && most && tree->num_trees >= 1, "hira_read_state: null argument");
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)
+        return fail(HIRA_ELAUNCH, "hira_read_state: a stream under capture cannot be waited for");
+    void* rows = nullptr;
+    if (hipHostGetDevicePointer(&rows, host_rows, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(HIRA_EINVAL, "hira_read_state: the rows do not lie in pinned host memory");
+    }
+    const int n = tree->num_trees * (HIRA_MAX_LEVELS + 2);
+    hipLaunchKernelGGL(k_tell_host, dim3((n + 255) / 256), dim3(256), 0, s, state, static_cast<uint64_t*>(rows), ticket, n);
+    HIRA_CHECK_LAUNCH("hira_read_state");
+    for (int i = 0; i < HIRA_MAX_LEVELS + 2; ++i) most[i] = INT32_MIN;
+    const auto begin = std::chrono::steady_clock::now();
+    bool waited = false;
+    for (int i = 0; i < n; ++i) {
+        uint64_t v;
+        for (int spins = 1; (uint32_t)((v = __atomic_load_n(host_rows + i, __ATOMIC_RELAXED)) >> 32) != ticket; ++spins) {
+            if (waited) return fail(HIRA_ELAUNCH, "hira_read_state: the stream has ended without the rows");
+            if (spins % 64 == 0 && std::chrono::steady_clock::now() - begin > kWatch) {
+                if (hipStreamSynchronize(s) != hipSuccess) return fail(HIRA_ELAUNCH, "hira_read_state: the stream failed");
+                waited = true;
+            }
+        }
+        int32_t& to = most[i % (HIRA_MAX_LEVELS + 2)];
+        to = std::max(to, (int32_t)(uint32_t)v);
+    }
+    __atomic_thread_fence(__ATOMIC_ACQUIRE);
     return HIRA_OK;
 }
 

@@ -218,6 +218,8 @@ class HIPIndexer(BaseIndexer):
         self._tree_struct = None
         self._state: Optional[torch.Tensor] = None  # device-side bookkeeping of update()
         self._append: Optional[_Append] = None
+        self._host_rows: Optional[torch.Tensor] = None  # pinned: where the state's rows are read back to
+        self._ticket = 0
 
     # ------------------------------------------------------------------ reference views
     @property
@@ -871,16 +873,35 @@ class HIPIndexer(BaseIndexer):
                                                 _lib.stream_of(self._state.get_device())))
 
     def sync_sizes(self) -> "HIPIndexer":
-        """Read the level sizes back after updates with ``sync=False`` (one small copy that
+        """Read the level sizes back after updates with ``sync=False`` (which
         waits for the stream) and check that no key was dropped."""
         if self._state is None or (self._pending == 0 and self._exact_size is None):
             return self
-        self._adopt_state(self._state.cpu())
+        self._adopt_state()
         self._unsynced_room = 0
         return self
 
-    def _adopt_state(self, st: torch.Tensor) -> None:
-        most = st.numpy().max(axis=0).tolist()
+    def _largest_state(self) -> List[int]:
+        """The largest entry over the trees of every column of the state, behind all that was enqueued."""
+        st = self._state
+        if not st.is_cuda:
+            return st.numpy().max(axis=0).tolist()
+        rows = self._host_rows
+        if rows is None or rows.numel() != st.numel():
+            # (zero once: a row is there when it holds the call's ticket)
+            rows = self._host_rows = torch.zeros(st.numel(), dtype=torch.int64, pin_memory=True)
+            self._ticket = 0
+        self._ticket = self._ticket % 0x7fffffff + 1
+        most = (C.c_int32 * (_lib.HIRA_MAX_LEVELS + 2))()
+        rc = _lib.lib().hira_read_state(C.byref(self.tree_struct()), st.data_ptr(), rows.data_ptr(), self._ticket,
+                                        most, _lib.stream_of(st.get_device()))
+        if rc:
+            self._host_rows = None  # (whatever went wrong: these are not used again)
+            _lib.check(rc)
+        return list(most)
+
+    def _adopt_state(self) -> None:
+        most = self._largest_state()
         if most[_lib.HIRA_MAX_LEVELS + 1] != 0:
             raise RuntimeError("index update ran out of capacity")
         if self.num_levels == 1:
@@ -898,7 +919,7 @@ class HIPIndexer(BaseIndexer):
                sync: bool = True, sample=None):
         """Append new_keys (1, H, m, D) (and new_values (1, H, m, Dv)) in order
         (indexer/cuda.py:544-701).  One launch; afterwards the level sizes are read back
-        (one small device-to-host copy), as the next search needs them.
+        (the call waits for the stream), as the next search needs them.
 
         ``sync=False`` skips the read-back: the host then carries upper bounds of the level
         sizes (slots past a tree's real size hold nodes without children, which every search
@@ -979,7 +1000,7 @@ class HIPIndexer(BaseIndexer):
             _lib.check(rc)
         self.num_keys += m
         if sync:
-            self._adopt_state(self._state.cpu())
+            self._adopt_state()
             self._unsynced_room = 0
             return self
         if self._exact_size is None:  # (inside a stretch self.size already holds bounds)

@@ -31,7 +31,7 @@
 extern "C" {
 #endif
 
-#define HIRA_ABI_VERSION 11
+#define HIRA_ABI_VERSION 12
 #define HIRA_MAX_LEVELS 8
 #define HIRA_STATS_COLS (HIRA_MAX_LEVELS + 3) /* counters per tree a search can fill in */
 
@@ -319,6 +319,17 @@ int hira_update(const HiraTree* tree, const void* new_keys, const void* new_valu
 int hira_update_sample(const HiraTree* tree, const void* new_keys, const void* new_values, int32_t m,
                        int32_t* state, void* sample, int32_t rows_per_tree, const int32_t* slot_host,
                        const int32_t* from_host, int32_t n, void* stream);
+
+/*
+ * The state rows' largest entries over the trees, column by column, into most (HIRA_MAX_LEVELS + 2 numbers of the
+ * caller's): what a caller of hira_update sets size[l] from.  Waits until all that was enqueued on the stream before is
+ * over.
+ *   host_rows  (T, HIRA_MAX_LEVELS + 2) words of pinned host memory (hipHostMalloc) that nothing else uses meanwhile
+ *   ticket     differs from that of every call before on these rows, and from what they held at first (zeros: not 0)
+ * A stream under capture is refused.
+ */
+int hira_read_state(const HiraTree* tree, const int32_t* state, uint64_t* host_rows, uint32_t ticket, int32_t* most,
+                    void* stream);
 
 /* The initial state of every tree, as described above, from tree->size and the number of keys
  * inserted so far: on the stream, without a copy from the host that would wait for it. */

@@ -613,3 +613,28 @@ def test_an_append_with_a_read_back_between_appends_without(bf, levels, m, gpu_d
         assert all(u <= b for u, b in zip(used, idx.size[1:])), (at, used, idx.size)
     idx.sync_sizes()
     assert idx.num_keys == k.shape[2] and (idx.perm >= 0).sum() == 2 * idx.num_keys
+
+
+@pytest.mark.parametrize("heads,levels,busy", [(1, 1, False), (1, 2, False), (8, 3, True), (26, 3, False)])
+def test_sizes_read_back_are_the_states(heads, levels, busy):
+    """update() reads every column's largest entry back (26 trees: more words than a workgroup of the launch that
+    writes them has threads), behind whatever the stream was busy with (longer than the host watches for itself)."""
+    from hira_amd.indexer.hip import HIPIndexer
+
+    g = torch.Generator().manual_seed(heads)
+    keys = torch.randn((1, heads, 70 * levels, 64), generator=g).to(torch.bfloat16).cuda()
+    idx = HIPIndexer(levels, 1, 16).build(keys, keys)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for m in (1, 5, 40, 3):
+            if busy:
+                a = torch.randn((4096, 4096), device="cuda")
+                for _ in range(20):
+                    a = torch.nn.functional.normalize(a @ a, dim=0)
+            new = torch.randn((1, heads, m, 64), generator=g).to(torch.bfloat16).cuda()
+            idx.update(new, new)
+            used = idx._state.cpu().max(dim=0).values.tolist()
+            want = [idx.num_keys] if levels == 1 else [used[1] * 16] + used[1:levels]
+            assert idx.size == want and used[-2] == idx.num_keys
+    side.synchronize()
