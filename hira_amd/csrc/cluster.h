@@ -163,53 +163,73 @@ __device__ __forceinline__ void wave_mean(const void* x, size_t row0, Ids ids, i
 // storage type.  One wave: `lpr` lanes (a power of two) hold a row in 16-byte chunks,
 // the 64 / lpr lane groups take every (64 / lpr)-th slot, and their sums are added pairwise in a
 // fixed order.  An empty block keeps its value.
-// (slot: what lies in slot `lane` of the block, -1 from bf on; U rows a lane group in flight: bf <= 64)
-template <typename T, int U>
-__device__ __forceinline__ void wave_block_mean(const void* x, size_t row0, int D, int slot, int bf,
-                                                int lpr, size_t out, float* cent, void* out_t) {
+// (slot: what lies in slot `lane` of the block, -1 from bf on; U rows a lane group in flight: bf <= 64; B blocks at a
+// time, of which there are `have`)
+template <typename T, int U, int B>
+__device__ __forceinline__ void wave_block_means(const void* x, size_t row0, int D, const int (&slot)[B], int have, int bf,
+                                                 int lpr, const size_t (&out)[B], float* cent, void* out_t) {
     constexpr int EPL = Elem<T>::kPerChunk;
     const int lane = threadIdx.x & 63;
     const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
     const bool chunk_ok = ch * EPL < D;
-    float acc[EPL];
+    float acc[B][EPL];
+    int cnt[B];
 #pragma unroll
-    for (int q = 0; q < EPL; ++q) acc[q] = 0.0f;
-    int cnt = 0;
+    for (int b = 0; b < B; ++b) {
+        cnt[b] = 0;
+#pragma unroll
+        for (int q = 0; q < EPL; ++q) acc[b][q] = 0.0f;
+    }
     for (int e0 = 0; e0 < bf; e0 += U * groups) {  // uniform: the slots come by shuffles
-        int it[U];
-        uint4 raw[U];
+        int it[B][U];
+        uint4 raw[B][U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int e = e0 + u * groups + rg;
-            it[u] = __shfl(slot, e & 63, 64);
-            if (e >= bf) it[u] = -1;
-            raw[u] = load_chunk<T>(x, (row0 + max(it[u], 0)) * D, chunk_ok ? ch : 0);
-        }
+        for (int b = 0; b < B; ++b)
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (it[u] >= 0) {
-                ++cnt;
-                float f[EPL];
-                unpack<T>(raw[u], f);
-#pragma unroll
-                for (int q = 0; q < EPL; ++q) acc[q] += f[q];
+            for (int u = 0; u < U; ++u) {
+                const int e = e0 + u * groups + rg;
+                it[b][u] = __shfl(slot[b], e & 63, 64);
+                if (e >= bf) it[b][u] = -1;
+                raw[b][u] = load_chunk<T>(x, (row0 + max(it[b][u], 0)) * D, chunk_ok ? ch : 0);
             }
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (it[b][u] >= 0) {
+                    ++cnt[b];
+                    float f[EPL];
+                    unpack<T>(raw[b][u], f);
+#pragma unroll
+                    for (int q = 0; q < EPL; ++q) acc[b][q] += f[q];
+                }
     }
-    cnt = cross_group(cnt, lpr, OpSum{});
 #pragma unroll
-    for (int q = 0; q < EPL; ++q) acc[q] = cross_group(acc[q], lpr, OpSum{});
-    if (rg == 0 && chunk_ok) {
+    for (int b = 0; b < B; ++b) {
+        if (b >= have) break;  // uniform
+        cnt[b] = cross_group(cnt[b], lpr, OpSum{});
 #pragma unroll
-        for (int q = 0; q < EPL; ++q) {
-            const size_t o = out + ch * EPL + q;
-            float v = cent[o];
-            if (cnt > 0) {
-                v = acc[q] / (float)cnt;
-                cent[o] = v;
+        for (int q = 0; q < EPL; ++q) acc[b][q] = cross_group(acc[b][q], lpr, OpSum{});
+        if (rg == 0 && chunk_ok) {
+#pragma unroll
+            for (int q = 0; q < EPL; ++q) {
+                const size_t o = out[b] + ch * EPL + q;
+                float v = cent[o];
+                if (cnt[b] > 0) {
+                    v = acc[b][q] / (float)cnt[b];
+                    cent[o] = v;
+                }
+                store_elem<T>(out_t, o, v);
             }
-            store_elem<T>(out_t, o, v);
         }
     }
+}
+template <typename T, int U>
+__device__ __forceinline__ void wave_block_mean(const void* x, size_t row0, int D, int slot, int bf, int lpr, size_t out,
+                                                float* cent, void* out_t) {
+    const int slots[1] = {slot};
+    const size_t outs[1] = {out};
+    wave_block_means<T, U, 1>(x, row0, D, slots, 1, bf, lpr, outs, cent, out_t);
 }
 
 }  // namespace hira

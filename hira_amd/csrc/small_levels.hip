@@ -7,12 +7,12 @@
 // waves has a tree to itself and takes it through such a level, and through the levels above, from one
 // barrier to the next.  The centroids do not move while blocks are packed, so the scores of all items and
 // centroids are made once and stay in LDS (128 KiB for 1024 items and 32 centroids), and so do the centroids'
-// operand tiles, the lists and the slots: a round of packing touches no memory.  What bounds it is the chain of
-// barriers and, for the first assignment, the means, the scores and the block centres, trips to the level-2 cache.
-// A level of 8 trees: 1024 items and 32 centroids 94 us (rounds 3-14), 128 and 4 20 us (rounds 1.5; with tiles and
-// scores in memory, made anew every round, 32).  Builds, launches / with that / this: 2 x 1111 keys of 64 columns, five
-// levels, fan-out 10: 426 / 207 / 181 us; 8 x 500, three levels, fan-out 32: 228 / 116 / 81; 8 x 8192, three levels,
-// fan-out 32, the second level here: - / 395 / 365.
+// operand tiles, the lists and the slots: a round of packing touches no memory.  Sixteen waves on one compute unit are bound
+// by their instructions, and by trips to the level-2 cache for the rows, which are gathered four times (first
+// assignment, means, scores, block centres; the first and the third are asked for ahead, under the first centroids and the means).
+// A launch, 8 trees of 128 columns: 1024 items and 32 centroids 74 us, 256 and 8 26.6, 128 and 4 21.5; 2 x 112 x 12 of 64 columns
+// and the two levels above 40 (95, 33, 27.5 and 49 with the items asked for where they were used, buckets looked for among
+// all items, a wave a centroid at the start and a block at a time at the end).
 //
 // The numbers are those of the launches, bit for bit: the same products in the same order, means and
 // block centres by the same functions (cluster.h), and rules that do not depend on the order of
@@ -30,9 +30,11 @@ static_assert(kSmallThreads >= kSmallItems, "the packing gives every item a thre
 constexpr int kPlaced = -2;
 constexpr int kSmallBig = kSmallItems / 65 + 1;
 
-// items of a wave's stretch: the registers of a wave (128 with sixteen waves a workgroup) hold their
-// operands and those of a centroid tile
-constexpr int small_ri(int KS) { return KS <= 4 ? 2 : 1; }
+// RI, below: item tiles a wave holds at a time, every sixteenth of the tree's: all of its own at the launch's first level, up
+// to four; one of rows of 256 columns, which take twice the registers (a wave has 128).  (Chosen inside the launch, the two sets
+// of registers met in spills: 8 x 1024 x 32 74 -> 112 us; four whatever the items: 128 x 4 31 -> 38.)
+constexpr int kSmallMean = 2;     // steps of a bucket's rows on their way
+constexpr int kSmallPlaces = 64;  // of a bucket, for items in order of arrival: what a wave ranks in registers
 
 // (whole item tiles, and the four rows that a tile's four lane groups write at a time in different banks)
 constexpr int small_stride(int n_c) { return (n_c + 15) / 16 * 16 + 4; }
@@ -41,10 +43,9 @@ template <int KS>
 struct SmallLds {
     static constexpr int kTileChunks = 2 * KS * 64;
     int16_t near[kSmallItems];     // of every item the centroid; -1: none, kPlaced: the item has its slot
-    uint16_t members[kSmallItems]; // Lloyd: of the buckets, end to end, by id; packing: 64 a wave
-    int32_t fill[kSmallCentroids], count[kSmallCentroids], first[kSmallCentroids];
+    int32_t fill[kSmallCentroids], count[kSmallCentroids];
     float n2[kSmallCentroids];     // squared norms of the centroids
-    int32_t big[kSmallBig], big_at[kSmallBig];  // buckets of more than 64 items: the whole workgroup's
+    int32_t big[kSmallBig], big_at[kSmallBig];  // packing: buckets of more than kSmallPlaces items, the whole workgroup's
     int32_t n_big, n_keys, n_left;
     float x2[kSmallItems];         // squared norm of every item
     float dist[kSmallItems];       // of every item to its nearest centroid
@@ -52,30 +53,35 @@ struct SmallLds {
         uint4 tiles[kSmallCentroids / 16 * kTileChunks];  // the centroids' operand tiles, until the scores are there
         struct {
             uint64_t keys[kSmallItems];  // proposers of the large buckets: (distance, id)
-            uint16_t list[kSmallItems];  // what is left, by id
+            union {
+                uint16_t pack_places[kSmallCentroids * kSmallPlaces];
+                uint16_t list[kSmallItems];  // what is left, by id
+            };
             int16_t slots[kSmallCentroids * 64];  // (K, bf)
         };
     };
     union {
-        float piece[kSmallWaves][kWaveMeanPiece<bf16_t>];   // Lloyd
+        struct {  // Lloyd
+            float piece[kSmallWaves][kWaveMeanPiece<bf16_t>];
+            uint16_t places[kSmallCentroids * kSmallPlaces];
+            uint16_t members[kSmallItems];  // of the large buckets, end to end, each by id
+        };
         // packing: the score ||c||^2 - 2 x.c of item i and centroid k at k * small_stride + i
         float score[small_pairs(32 * KS) + 20 * kSmallCentroids];
     };
 };
 static_assert(sizeof(SmallLds<2>) <= 160 * 1024 && sizeof(SmallLds<4>) <= 160 * 1024 && sizeof(SmallLds<8>) <= 160 * 1024, "LDS");
 
-// emit_centroid into the tiles here: centroid k, D fp32 numbers at c (one wave)
+// emit_columns into the tiles here: columns 8 j .. 8 j + 7 of centroid k; `lanes` consecutive lanes hold a centroid
 template <int KS>
-__device__ __forceinline__ void small_emit(SmallLds<KS>& s, const float* c, int k) {
-    const int j = threadIdx.x & 63;
+__device__ __forceinline__ void small_emit(SmallLds<KS>& s, const float (&v)[8], int j, int lanes, bool have, int k, bool usable) {
     float ss = 0.0f;
-    if (j < KS * 4) {
+    if (have && j < KS * 4) {
         float hi[8], lo[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float v = c[j * 8 + e];
-            hi[e] = bf16_bits_to_f32(f32_to_bf16_bits(v));
-            lo[e] = bf16_bits_to_f32(f32_to_bf16_bits(v - hi[e]));
+            hi[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e]));
+            lo[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e] - hi[e]));
             const float w = hi[e] + lo[e];
             ss += w * w;
         }
@@ -83,26 +89,47 @@ __device__ __forceinline__ void small_emit(SmallLds<KS>& s, const float* c, int 
         out[0] = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]), pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
         out[KS * 64] = make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]), pack_bf16(lo[6], lo[7]));
     }
-    ss = group_sum<32>(ss);
-    if (j == 0) s.n2[k] = ss;
+    ss = group_sum_of(ss, lanes);
+    if (have && j == 0) s.n2[k] = usable ? ss : INFINITY;
+}
+// the same with the centroid's D fp32 numbers at c (one wave)
+template <int KS>
+__device__ __forceinline__ void small_emit(SmallLds<KS>& s, const float* c, int k) {
+    const int j = threadIdx.x & 63;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = j < KS * 4 ? c[j * 8 + e] : 0.0f;
+    small_emit<KS>(s, v, j, 32, true, k, true);
 }
 
-// SCORES: the scores of all items and centroids; else the nearest centroid of every item and the buckets' counts
-template <int KS, bool SCORES>
-__device__ __forceinline__ void small_assign(SmallLds<KS>& s, const void* x, size_t row0, int K, int n_items) {
-    constexpr int D = 32 * KS, RI = small_ri(KS), ITEMS = RI * 16, TILE_CHUNKS = 2 * KS * 64;
+// The operands of a wave's next item tiles, from its tile number q0 on (tile q of wave w: items (16 q + w) * 16 ..): asked
+// for well ahead of small_assign, which takes them.
+template <int KS, int RI>
+__device__ __forceinline__ void small_items(const void* x, size_t row0, int n_items, int q0, uint4 (&x_op)[RI][KS]) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n = lane & 15, kb = lane >> 4;
+#pragma unroll
+    for (int ri = 0; ri < RI; ++ri) {
+        const int p0 = ((q0 + ri) * kSmallWaves + wave) * 16;
+#pragma unroll
+        for (int c = 0; c < KS; ++c)  // (whatever the tile: a load under a condition is waited for where that ends)
+            x_op[ri][c] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(x) +
+                                                          (row0 + max(min(p0 + n, n_items - 1), 0)) * (32 * KS) + c * 32 + kb * 8);
+    }
+}
+
+// SCORES: the scores of all items and centroids; else the nearest centroid of every item, the buckets' counts and the
+// first kSmallPlaces items of each.  x_op: small_items of the first tiles.
+template <int KS, int RI, bool SCORES>
+__device__ __forceinline__ void small_assign(SmallLds<KS>& s, const void* x, size_t row0, int K, int n_items, uint4 (&x_op)[RI][KS]) {
+    constexpr int TILE_CHUNKS = 2 * KS * 64;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, kb = lane >> 4, tiles = (K + 15) / 16, stride = small_stride(n_items);
-    for (int p0 = wave * ITEMS; p0 < n_items; p0 += kSmallWaves * ITEMS) {  // uniform in the wave
-        uint4 x_op[RI][KS];
-        float x2[RI], best[RI];
+    for (int q0 = 0; (q0 * kSmallWaves + wave) * 16 < n_items; q0 += RI) {  // uniform in the wave
+        if (q0 > 0) small_items<KS, RI>(x, row0, n_items, q0, x_op);
+        auto first = [&](int ri) { return ((q0 + ri) * kSmallWaves + wave) * 16; };
+        float best[RI];
         int arg[RI];
-#pragma unroll
-        for (int ri = 0; ri < RI; ++ri)
-#pragma unroll
-            for (int c = 0; c < KS; ++c)
-                x_op[ri][c] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(x) +
-                                                              (row0 + min(p0 + ri * 16 + n, n_items - 1)) * D + c * 32 + kb * 8);
         if constexpr (SCORES) {
 #pragma unroll
             for (int ri = 0; ri < RI; ++ri) {
@@ -115,31 +142,32 @@ __device__ __forceinline__ void small_assign(SmallLds<KS>& s, const void* x, siz
                     for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
                 }
                 ss = cross_group_sum<16>(ss);
-                x2[ri] = ss;
+                if (kb == 0 && first(ri) + n < n_items) s.x2[first(ri) + n] = ss;
             }
-        }
+        } else {
 #pragma unroll
-        for (int ri = 0; ri < RI; ++ri) {
-            best[ri] = INFINITY;
-            arg[ri] = -1;
+            for (int ri = 0; ri < RI; ++ri) {
+                best[ri] = INFINITY;
+                arg[ri] = -1;
+            }
         }
         for (int tile = 0; tile < tiles; ++tile) {
             const uint4* src = s.tiles + tile * TILE_CHUNKS + lane;
-            uint4 c_op[2 * KS];
-#pragma unroll
-            for (int c = 0; c < 2 * KS; ++c) c_op[c] = src[c * 64];
             const float4 n2 = *reinterpret_cast<const float4*>(s.n2 + tile * 16 + 4 * kb);
             sf32x4_t acc[RI];
 #pragma unroll
             for (int ri = 0; ri < RI; ++ri) acc[ri] = sf32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int c = 0; c < KS; ++c)
+            for (int c = 0; c < KS; ++c) {
 #pragma unroll
-                for (int half = 0; half < 2; ++half)
+                for (int half = 0; half < 2; ++half) {
+                    const sbf16x8_t c_op = __builtin_bit_cast(sbf16x8_t, src[(half * KS + c) * 64]);
 #pragma unroll
                     for (int ri = 0; ri < RI; ++ri)
-                        acc[ri] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sbf16x8_t, c_op[half * KS + c]),
-                                                                          __builtin_bit_cast(sbf16x8_t, x_op[ri][c]), acc[ri], 0, 0, 0);
+                        acc[ri] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c_op, __builtin_bit_cast(sbf16x8_t, x_op[ri][c]), acc[ri], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);  // (a tile's operands all at once are more than there are registers for)
+            }
             const float nn[4] = {n2.x, n2.y, n2.z, n2.w};
 #pragma unroll
             for (int j = 0; j < 4; ++j) {  // (increasing: ties keep the lower one)
@@ -148,7 +176,7 @@ __device__ __forceinline__ void small_assign(SmallLds<KS>& s, const void* x, siz
                 for (int ri = 0; ri < RI; ++ri) {
                     const float v = nn[j] - 2.0f * acc[ri][j];
                     if constexpr (SCORES) {
-                        if (k < K && p0 + ri * 16 < n_items) s.score[k * stride + p0 + ri * 16 + n] = v;
+                        if (k < K && first(ri) < n_items) s.score[k * stride + first(ri) + n] = v;
                     } else if (k < K && v < best[ri]) {  // (behind the last one a tile holds anything)
                         best[ri] = v;
                         arg[ri] = k;
@@ -156,45 +184,34 @@ __device__ __forceinline__ void small_assign(SmallLds<KS>& s, const void* x, siz
                 }
             }
         }
+        if constexpr (!SCORES) {
+            int mine = -1, item = n_items;  // lane (kb, n): item n of tile kb (RI = 1: every lane group has it)
 #pragma unroll
-        for (int ri = 0; ri < RI; ++ri) {
-            const int item = p0 + ri * 16 + n;
-            if constexpr (SCORES) {
-                if (kb == 0 && item < n_items) s.x2[item] = x2[ri];
-            } else {
-#pragma unroll
-                for (int off = 16; off < 64; off <<= 1) {
-                    const float ob = __shfl_xor(best[ri], off, 64);
-                    const int og = __shfl_xor(arg[ri], off, 64);
-                    if (og >= 0 && (arg[ri] < 0 || ob < best[ri] || (ob == best[ri] && og < arg[ri]))) {
-                        best[ri] = ob;
-                        arg[ri] = og;
-                    }
+            for (int ri = 0; ri < RI; ++ri) {
+                auto nearer = [&](auto v, auto k) {  // of the two lanes that a swap has paired, in both of them
+                    const float v0 = __uint_as_float((uint32_t)v[0]), v1 = __uint_as_float((uint32_t)v[1]);
+                    const int k0 = (int)k[0], k1 = (int)k[1];
+                    const bool second = k1 >= 0 && (k0 < 0 || v1 < v0 || (v1 == v0 && k1 < k0));
+                    best[ri] = second ? v1 : v0;
+                    arg[ri] = second ? k1 : k0;
+                };
+                nearer(__builtin_amdgcn_permlane16_swap(__float_as_uint(best[ri]), __float_as_uint(best[ri]), false, false),
+                       __builtin_amdgcn_permlane16_swap((uint32_t)arg[ri], (uint32_t)arg[ri], false, false));
+                nearer(__builtin_amdgcn_permlane32_swap(__float_as_uint(best[ri]), __float_as_uint(best[ri]), false, false),
+                       __builtin_amdgcn_permlane32_swap((uint32_t)arg[ri], (uint32_t)arg[ri], false, false));
+                if (kb == ri) {
+                    mine = arg[ri];
+                    item = first(ri) + n;
                 }
-                if (kb == 0 && item < n_items) {
-                    s.near[item] = (int16_t)arg[ri];
-                    if (arg[ri] >= 0) atomicAdd(&s.count[arg[ri]], 1);
+            }
+            if (item < n_items) {
+                s.near[item] = (int16_t)mine;
+                if (mine >= 0) {
+                    const int at = atomicAdd(&s.count[mine], 1);
+                    if (at < kSmallPlaces) s.places[mine * kSmallPlaces + at] = (uint16_t)item;
                 }
             }
         }
-    }
-}
-
-// where the bucket of every centroid begins (K <= kSmallCentroids; one wave)
-template <int KS>
-__device__ __forceinline__ void small_offsets(SmallLds<KS>& s, int K) {
-    const int lane = threadIdx.x & 63;
-    int before = 0;
-    for (int k0 = 0; k0 < K; k0 += 64) {
-        const int mine = k0 + lane < K ? s.count[k0 + lane] : 0;
-        int inc = mine;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int o = __shfl_up(inc, off, 64);
-            if (lane >= off) inc += o;
-        }
-        if (k0 + lane < K) s.first[k0 + lane] = before + inc - mine;
-        before += __shfl(inc, 63, 64);
     }
 }
 
@@ -236,47 +253,7 @@ __device__ __forceinline__ int small_left(SmallLds<KS>& s, int n) {
     return at;
 }
 
-// wave_mean over 256 threads: their sums over the m rows members[at ..), R rows of D numbers, to part
-template <int KS>
-__device__ __forceinline__ void small_big_sums(const SmallLds<KS>& s, const void* x, size_t row0, int at, int m, float* part) {
-    constexpr int D = 32 * KS, EPL = 8, CPR = D / EPL, R = 256 / CPR, U = 4;  // (U rows on their way)
-    const int i = threadIdx.x & 255, r = i / CPR, c = i % CPR;
-    float acc[EPL];
-#pragma unroll
-    for (int q = 0; q < EPL; ++q) acc[q] = 0.0f;
-    for (int e = r; e < m; e += U * R) {
-        uint4 raw[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            raw[u] = make_uint4(0, 0, 0, 0);  // (a row that is none adds zeros)
-            if (e + u * R < m) raw[u] = load_chunk<bf16_t>(x, (row0 + s.members[at + e + u * R]) * D, c);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            float f[EPL];
-            unpack<bf16_t>(raw[u], f);
-#pragma unroll
-            for (int q = 0; q < EPL; ++q) acc[q] += f[q];
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < EPL; ++q) part[r * D + c * EPL + q] = acc[q];
-}
-// the sums added in order; the mean's D numbers to cent_row and to part[0 .. D) (a thread's column is
-// nobody else's)
-template <int KS>
-__device__ __forceinline__ void small_big_mean(float* part, int m, float* cent_row) {
-    constexpr int D = 32 * KS, R = 256 / (D / 8);
-    const int j = threadIdx.x & 255, rows = min(R, m);
-    if (j >= D) return;
-    float sum = 0.0f;
-    for (int q = 0; q < rows; ++q) sum += part[q * D + j];
-    const float v = sum / (float)m;
-    cent_row[j] = v;
-    part[j] = v;
-}
-
-template <int KS>
+template <int KS, int RI>
 __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevels p) {
     constexpr int D = 32 * KS;
     extern __shared__ uint64_t s_raw[];
@@ -295,86 +272,70 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
         float* cent = p.cent + (size_t)t * K * D;
         float* piece = s.piece[wave];
 
-        // ---- empty blocks, first centroids -------------------------------------------------------
+        // ---- empty blocks, first centroids (all of them at once, KS * 4 lanes each), the items' operands --------
         for (int i = tid; i < K; i += kSmallThreads) {
             s.fill[i] = i >= K_t ? bf : 0;
             s.count[i] = 0;
         }
-        if (tid == 0) s.n_big = 0;
-        constexpr int kMine = (kSmallCentroids + kSmallWaves - 1) / kSmallWaves, NJ = D / 64;
-        float first[kMine][NJ];  // (a wave's centroids, asked for together)
-#pragma unroll
-        for (int i = 0; i < kMine; ++i) {
-            const int k = min(wave + i * kSmallWaves, K - 1);
-            const size_t src = (row0 + (size_t)first_centroid(p.seed + 7919ull * (uint64_t)l, t, k, max(n_c, 1), K_t)) * D;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) first[i][j] = load_elem<bf16_t>(x, src + j * 64 + lane);
-        }
-#pragma unroll
-        for (int i = 0; i < kMine; ++i) {
-            const int k = wave + i * kSmallWaves;
-            if (k >= K) break;  // uniform
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) cent[(size_t)k * D + j * 64 + lane] = piece[j * 64 + lane] = first[i][j];
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            small_emit<KS>(s, piece, k);
-            if (lane == 0 && k >= K_t) s.n2[k] = INFINITY;
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (tid == 0) s.n_big = s.n_keys = 0;
+        uint4 x_op[RI][KS];
+        {
+            constexpr int LANES = KS * 4;
+            static_assert(kSmallThreads / LANES >= kSmallCentroids, "a pass for all centroids");
+            const int k = tid / LANES, j = lane % LANES, own = min(k, K - 1);
+            const size_t src = (row0 + (size_t)first_centroid(p.seed + 7919ull * (uint64_t)l, t, own, max(n_c, 1), K_t)) * D;
+            const uint4 raw = load_chunk<bf16_t>(x, src, j);
+            small_items<KS, RI>(x, row0, n_c, 0, x_op);
+            float v[8];
+            unpack<bf16_t>(raw, v);
+            if (k < K) {
+                float4* dst = reinterpret_cast<float4*>(cent + (size_t)k * D + j * 8);
+                dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+                dst[1] = make_float4(v[4], v[5], v[6], v[7]);
+            }
+            small_emit<KS>(s, v, j, LANES, k < K, own, own < K_t);
         }
         __syncthreads();
 
         // ---- Lloyd rounds ------------------------------------------------------------------------
         for (int r = 0; r < p.niter; ++r) {
-            small_assign<KS, false>(s, x, row0, K, n_c);
-            __syncthreads();
-            if (wave == 0) small_offsets(s, K);
+            small_assign<KS, RI, false>(s, x, row0, K, n_c, x_op);
             __syncthreads();
             for (int k = wave; k < K; k += kSmallWaves) {
-                const int m = __builtin_amdgcn_readfirstlane(s.count[k]), at = __builtin_amdgcn_readfirstlane(s.first[k]);
+                const int m = __builtin_amdgcn_readfirstlane(s.count[k]);
                 if (m == 0) continue;
-                small_members(s, k, m, n_c, [&](int e, int it) { s.members[at + e] = (uint16_t)it; });
-                if (m > 64) {
-                    if (lane == 0) s.big[atomicAdd(&s.n_big, 1)] = k;
-                    continue;
+                uint16_t* ids = s.places + k * kSmallPlaces;
+                if (m <= kSmallPlaces) {  // by id
+                    const uint32_t id = lane < m ? ids[lane] : 0xffffffffu;
+                    const int rank = wave_rank(id, m);
+                    if (lane < m) ids[rank] = (uint16_t)id;
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                } else {
+                    int at = 0;
+                    if (lane == 0) at = atomicAdd(&s.n_keys, m);
+                    ids = s.members + __builtin_amdgcn_readfirstlane(at);
+                    small_members(s, k, m, n_c, [&](int e, int it) { ids[e] = (uint16_t)it; });
                 }
-                wave_mean<bf16_t, 1>(x, row0, [&](int e) { return (uint32_t)s.members[at + e]; }, m, D, piece,
-                                     cent + (size_t)k * D);
+                wave_mean<bf16_t, kSmallMean>(x, row0, [&](int e) { return (uint32_t)ids[e]; }, m, D, piece, cent + (size_t)k * D);
                 small_emit<KS>(s, piece, k);
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 if (lane == 0) s.count[k] = 0;
             }
+            small_items<KS, RI>(x, row0, n_c, 0, x_op);  // (for what comes next)
             __syncthreads();
-            // the large ones, four at a time: 256 threads each, with the sums of wave_mean
-            const int n_big = __builtin_amdgcn_readfirstlane(s.n_big);
-            float* part = s.piece[wave & ~3];
-            for (int b0 = 0; b0 < n_big; b0 += kSmallWaves / 4) {  // uniform
-                const int b = b0 + (wave >> 2), k = b < n_big ? s.big[b] : 0;
-                const int m = b < n_big ? s.count[k] : 0, at = s.first[k];
-                small_big_sums<KS>(s, x, row0, at, m, part);
-                __syncthreads();
-                if (b < n_big) small_big_mean<KS>(part, m, cent + (size_t)k * D);
-                __syncthreads();
-                if (b < n_big && (wave & 3) == 0) {
-                    small_emit<KS>(s, part, k);
-                    if (lane == 0) s.count[k] = 0;
-                }
-                __syncthreads();
-            }
-            if (tid == 0) s.n_big = 0;  // (read by everybody ahead of a barrier: none was passed if there were none)
+            if (tid == 0) s.n_keys = 0;
         }
 
         // ---- capacity packing: the closest proposers of a bucket (by distance, then id) take the free
         // slots of the block in that order, the others try again.  The centroids stay what they are, so
         // the scores are made once, and a round is a look at those of the centroids with room, a thread an item.
-        __syncthreads();  // (the last centroids' tiles are written)
-        small_assign<KS, true>(s, x, row0, K, n_c);
+        small_assign<KS, RI, true>(s, x, row0, K, n_c, x_op);
         if (tid < n_c) s.near[tid] = -1;
         if (tid == 0) s.n_left = n_c;
         __syncthreads();
         for (int i = tid; i < K * bf; i += kSmallThreads) s.slots[i] = -1;  // (where the tiles were)
         const int stride = small_stride(n_c);
         const float x2 = tid < n_c ? s.x2[tid] : 0.0f;
-        uint16_t* const mem = s.members + wave * 64;
         auto key_of = [&](uint32_t it) { return ((uint64_t)__float_as_uint(s.dist[it]) << 32) | it; };
         for (int r = 0; r < p.pack_rounds; ++r) {
             if (tid == 0) s.n_keys = 0;
@@ -392,7 +353,10 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
                 }
                 s.near[tid] = (int16_t)arg;
                 s.dist[tid] = fmaxf(best + x2, 0.0f);
-                if (arg >= 0) atomicAdd(&s.count[arg], 1);
+                if (arg >= 0) {
+                    const int at = atomicAdd(&s.count[arg], 1);
+                    if (at < kSmallPlaces) s.pack_places[arg * kSmallPlaces + at] = (uint16_t)tid;
+                }
             }
             __syncthreads();
             auto filled = [&](int k, int f, int take) {  // (one thread)
@@ -404,7 +368,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
                 const int m = __builtin_amdgcn_readfirstlane(s.count[k]);
                 if (m == 0) continue;
                 const int f = __builtin_amdgcn_readfirstlane(s.fill[k]), take = max(min(m, bf - f), 0);
-                if (m > 64) {
+                if (m > kSmallPlaces) {
                     int at = 0;
                     if (lane == 0) at = atomicAdd(&s.n_keys, m);
                     at = __builtin_amdgcn_readfirstlane(at);
@@ -416,8 +380,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
                     }
                     continue;
                 }
-                small_members(s, k, m, n_c, [&](int e, int it) { mem[e] = (uint16_t)it; });
-                const uint64_t mine = lane < m ? key_of(mem[lane]) : ~0ull;
+                const uint64_t mine = lane < m ? key_of(s.pack_places[k * kSmallPlaces + lane]) : ~0ull;
                 const int rank = wave_rank(mine, m);
                 if (lane < m && rank < take) {
                     s.slots[k * bf + f + rank] = (int16_t)(uint32_t)mine;
@@ -458,7 +421,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
         __syncthreads();
 
         // ---- what is left, and items that are no numbers, to the free slots in order ------------------
-        if (wave == 0) {
+        if (wave == 0 && s.n_left != 0) {
             const int total = small_left(s, n_c);
             int before = 0;
             for (int k0 = 0; k0 < K && before < total; k0 += 64) {  // uniform
@@ -477,27 +440,45 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
         __syncthreads();
         // ---- block centres ----------------------------------------------------------------------------
         for (int i = tid; i < K * bf; i += kSmallThreads) slots[i] = s.slots[i];
-        for (int k = wave; k < K; k += kSmallWaves)
-            wave_block_mean<bf16_t, 4>(x, row0, D, lane < bf ? s.slots[k * bf + lane] : -1, bf, p.lpr, ((size_t)t * K + k) * D, p.cent,
-                                       p.cent_t[l]);
+        for (int k = wave; k < K; k += 2 * kSmallWaves) {  // uniform; two at a time
+            int slot[2];
+            size_t out[2];
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const int own = min(k + b * kSmallWaves, K - 1);
+                slot[b] = lane < bf && k + b * kSmallWaves < K ? s.slots[own * bf + lane] : -1;
+                out[b] = ((size_t)t * K + own) * D;
+            }
+            wave_block_means<bf16_t, 4, 2>(x, row0, D, slot, k + kSmallWaves < K ? 2 : 1, bf, p.lpr, out, p.cent, p.cent_t[l]);
+        }
         __syncthreads();  // (the next level reads them)
     }
 }
 
-template <int KS>
+template <int KS, int RI>
 static int launch_small(const SmallLevels& p, int num_trees, hipStream_t s) {
     static int asked[kMaxDevices];
-    if (const int rc = ask_for_lds(reinterpret_cast<const void*>(&k_small_levels<KS>), sizeof(SmallLds<KS>), asked, current_device()))
+    if (const int rc = ask_for_lds(reinterpret_cast<const void*>(&k_small_levels<KS, RI>), sizeof(SmallLds<KS>), asked, current_device()))
         return rc;
-    hipLaunchKernelGGL((k_small_levels<KS>), dim3(num_trees), dim3(kSmallThreads), sizeof(SmallLds<KS>), s, p);
+    hipLaunchKernelGGL((k_small_levels<KS, RI>), dim3(num_trees), dim3(kSmallThreads), sizeof(SmallLds<KS>), s, p);
     return HIRA_OK;
+}
+
+template <int KS>
+static int launch_small_of(const SmallLevels& p, int num_trees, hipStream_t s) {
+    const int tiles = (p.K[p.first - 1] + 16 * kSmallWaves - 1) / (16 * kSmallWaves);  // of a wave
+    if constexpr (KS <= 4) {
+        if (tiles > 2) return launch_small<KS, 4>(p, num_trees, s);
+        if (tiles > 1) return launch_small<KS, 2>(p, num_trees, s);
+    }
+    return launch_small<KS, 1>(p, num_trees, s);
 }
 
 int launch_small_levels(const SmallLevels& p, int D, int num_trees, hipStream_t s) {
     switch (D) {
-        case 64: return launch_small<2>(p, num_trees, s);
-        case 128: return launch_small<4>(p, num_trees, s);
-        case 256: return launch_small<8>(p, num_trees, s);
+        case 64: return launch_small_of<2>(p, num_trees, s);
+        case 128: return launch_small_of<4>(p, num_trees, s);
+        case 256: return launch_small_of<8>(p, num_trees, s);
         default: return fail(HIRA_EINVAL, "small levels: %d columns", D);
     }
 }

@@ -72,3 +72,11 @@ def test_levels_above_cluster_the_centres_below(h, n, d, levels, bf, gpu_device)
                                             (2, 97, 128, 3, 1), (2, 1009, 128, 32, 1)])
 def test_as_many_pairs_as_the_scores_have_room_for(kind, h, n, d, bf, niter, gpu_device):
     test_a_small_level_is_clustered_as_a_large_one(kind, h, n, d, bf, niter, gpu_device)
+
+
+@pytest.mark.parametrize("kind", ["normal", "ties", "hub", "nan"])
+@pytest.mark.parametrize("h,n,d,bf", [(2, 16, 64, 8), (2, 255, 128, 16), (2, 256, 64, 32), (2, 257, 128, 16), (1, 512, 64, 64),
+                                      (2, 513, 64, 32), (1, 769, 128, 64), (2, 264, 256, 33)])
+def test_item_tiles_of_a_wave(kind, h, n, d, bf, gpu_device):
+    """Around 256 and 512 items a wave holds one, two or four of the tiles of sixteen."""
+    test_a_small_level_is_clustered_as_a_large_one(kind, h, n, d, bf, 2, gpu_device)
