@@ -132,8 +132,22 @@ struct CentroidTiles {
     float* lo;
 };
 
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-    return (uint32_t)f32_to_bf16_bits(a) | ((uint32_t)f32_to_bf16_bits(b) << 16);
+// Eight numbers as two bf16 halves each, v = hi + lo; joined to ss: the squares of hi + lo, to ls: those of v - hi.
+__device__ __forceinline__ void split_bf16(const float (&v)[8], uint4& hi, uint4& lo, float& ss, float& ls) {
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        h[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
+        const float d0 = v[2 * e] - bf16_lo(h[e]), d1 = v[2 * e + 1] - bf16_hi(h[e]);
+        l[e] = pack_bf16(d0, d1);
+        const float w0 = bf16_lo(h[e]) + bf16_lo(l[e]), w1 = bf16_hi(h[e]) + bf16_hi(l[e]);
+        ss += w0 * w0;
+        ls += d0 * d0;
+        ss += w1 * w1;
+        ls += d1 * d1;
+    }
+    hi = make_uint4(h[0], h[1], h[2], h[3]);
+    lo = make_uint4(l[0], l[1], l[2], l[3]);
 }
 
 // Columns 8 j .. 8 j + 7 of centroid k of tree t (zeros behind the last one) into its tile; `lanes` (a power of two, at
@@ -144,20 +158,10 @@ __device__ __forceinline__ void emit_columns(const float (&v)[8], int j, int lan
     if (have && j < KS * 4) {
         const int s = j >> 2, kb = j & 3, i = k & 15;
         uint4* out = ct.tiles + ((size_t)t * Kt + (k >> 4)) * (size_t)(2 * KS * 64);
-        float hi[8], lo[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            hi[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e]));
-            lo[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e] - hi[e]));
-            const float w = hi[e] + lo[e];
-            ss += w * w;
-            ls += (v[e] - hi[e]) * (v[e] - hi[e]);
-        }
-        out[s * 64 + kb * 16 + i] = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]),
-                                               pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
-        out[KS * 64 + s * 64 + kb * 16 + i] =
-            make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]),
-                       pack_bf16(lo[6], lo[7]));
+        uint4 hi, lo;
+        split_bf16(v, hi, lo, ss, ls);
+        out[s * 64 + kb * 16 + i] = hi;
+        out[KS * 64 + s * 64 + kb * 16 + i] = lo;
     }
     ss = group_sum_of(ss, lanes);
     ls = group_sum_of(ls, lanes);

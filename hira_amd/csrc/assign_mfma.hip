@@ -56,20 +56,13 @@ __global__ __launch_bounds__(64) void k_cent_prep(const float* cent, int K, cons
     float ss = 0.0f;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-        float c[8], hi[8], lo[8];
+        float c[8], ls = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            c[e] = k < K ? cent[((size_t)t * K + k) * D + s * 32 + kb * 8 + e] : 0.0f;
-            hi[e] = bf16_bits_to_f32(f32_to_bf16_bits(c[e]));
-            lo[e] = bf16_bits_to_f32(f32_to_bf16_bits(c[e] - hi[e]));
-            const float v = hi[e] + lo[e];
-            ss += v * v;
-        }
-        out[s * 64 + kb * 16 + i] = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]),
-                                               pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
-        out[KS * 64 + s * 64 + kb * 16 + i] =
-            make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]),
-                       pack_bf16(lo[6], lo[7]));
+        for (int e = 0; e < 8; ++e) c[e] = k < K ? cent[((size_t)t * K + k) * D + s * 32 + kb * 8 + e] : 0.0f;
+        uint4 hi, lo;
+        split_bf16(c, hi, lo, ss, ls);
+        out[s * 64 + kb * 16 + i] = hi;
+        out[KS * 64 + s * 64 + kb * 16 + i] = lo;
     }
     ss = cross_group_sum<16>(ss);
     if (kb == 0) {

@@ -299,7 +299,7 @@ __device__ __forceinline__ void reset_round(const Buckets& b, int t) {  // (one 
 //    What bounds it is the latency of each bucket's chain (count, members, rows, sums): 6 us a workgroup of four
 //    small ones, 20 to 45 us a large one (up to 1473 rows at 8 x 131072 items, beside a mean of 32), so what
 //    counts is how many are on a compute unit: six workgroups (76 registers, 18 KiB), with fewer rows on their way in
-//    each.  8 x 32768 rows of 256 bytes 28 us, 8 x 131072 72 us (33 and 92 with four workgroups of 108 registers, twice the
+//    each.  8 x 32768 rows of 256 bytes 26 us, 8 x 131072 75 us (33 and 92 with four workgroups of 108 registers, twice the
 //    rows on their way and a quarter of the sums added up one load after the other).
 // ------------------------------------------------------------------------------------
 constexpr int kMeanMap = 2048;  // words of a bit map of item ids, for buckets beyond their places
@@ -451,12 +451,12 @@ __global__ __launch_bounds__(kBucketThreads, 6) void k_bucket_mean(
     }
 }
 
-// A wave per block (wave_block_mean).  Bound by the gather of the rows: 8 x 131072 rows of 256
-// bytes 74 -> 60 us
+// A wave per block (wave_block_mean).  Bound by the gather of the rows: 8 x 131072 rows of 256 bytes 44 us, 6.1 TB/s
+// (60 with the centres rounded by shifts and stored a number at a time)
 template <typename T>
 __global__ __launch_bounds__(kNodeThreads) void k_block_mean(const void* x, size_t x_tree_stride, int K,
                                                              int D, const int32_t* slots, int bf, int lpr,
-                                                             float* cent, void* out_t) {
+                                                             const float* cent, void* out_t) {
     const int k = node_of_wave(), t = blockIdx.x;
     if (k >= K) return;  // (the whole wave)
     wave_block_mean<T, 8>(x, (size_t)t * x_tree_stride, D,
@@ -1035,7 +1035,6 @@ static int cluster_levels(const HiraTree* t, const void* keys_in, int n, const i
             p.niter = niter;
             p.pack_rounds = pack_rounds;
             p.bf = bf;
-            p.lpr = lpr;
             if (const int rc = launch_small_levels(p, D, NT, s)) return rc;
             HIRA_CHECK_LAUNCH("build, small levels");
             break;

@@ -159,15 +159,15 @@ __device__ __forceinline__ void wave_mean(const void* x, size_t row0, Ids ids, i
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// block centre = mean of the items in the bf slots of the block, stored in fp32 and rounded to the
+// block centre = mean of the items in the bf slots of the block, rounded to the
 // storage type.  One wave: `lpr` lanes (a power of two) hold a row in 16-byte chunks,
 // the 64 / lpr lane groups take every (64 / lpr)-th slot, and their sums are added pairwise in a
-// fixed order.  An empty block keeps its value.
+// fixed order.  An empty block's is its centroid.
 // (slot: what lies in slot `lane` of the block, -1 from bf on; U rows a lane group in flight: bf <= 64; B blocks at a
 // time, of which there are `have`)
 template <typename T, int U, int B>
 __device__ __forceinline__ void wave_block_means(const void* x, size_t row0, int D, const int (&slot)[B], int have, int bf,
-                                                 int lpr, const size_t (&out)[B], float* cent, void* out_t) {
+                                                 int lpr, const size_t (&out)[B], const float* cent, void* out_t) {
     constexpr int EPL = Elem<T>::kPerChunk;
     const int lane = threadIdx.x & 63;
     const int rg = lane / lpr, ch = lane % lpr, groups = 64 / lpr;
@@ -211,22 +211,21 @@ __device__ __forceinline__ void wave_block_means(const void* x, size_t row0, int
 #pragma unroll
         for (int q = 0; q < EPL; ++q) acc[b][q] = cross_group(acc[b][q], lpr, OpSum{});
         if (rg == 0 && chunk_ok) {
+            const size_t o = out[b] + ch * EPL;
+            if (cnt[b] == 0) {
 #pragma unroll
-            for (int q = 0; q < EPL; ++q) {
-                const size_t o = out[b] + ch * EPL + q;
-                float v = cent[o];
-                if (cnt[b] > 0) {
-                    v = acc[b][q] / (float)cnt[b];
-                    cent[o] = v;
-                }
-                store_elem<T>(out_t, o, v);
+                for (int q = 0; q < EPL; ++q) acc[b][q] = cent[o + q];
+            } else {
+#pragma unroll
+                for (int q = 0; q < EPL; ++q) acc[b][q] = acc[b][q] / (float)cnt[b];
             }
+            store_chunk<T>(out_t, o, acc[b]);
         }
     }
 }
 template <typename T, int U>
 __device__ __forceinline__ void wave_block_mean(const void* x, size_t row0, int D, int slot, int bf, int lpr, size_t out,
-                                                float* cent, void* out_t) {
+                                                const float* cent, void* out_t) {
     const int slots[1] = {slot};
     const size_t outs[1] = {out};
     wave_block_means<T, U, 1>(x, row0, D, slots, 1, bf, lpr, outs, cent, out_t);

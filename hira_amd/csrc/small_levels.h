@@ -19,7 +19,7 @@ struct SmallLevels {
     void* cent_t[HIRA_MAX_LEVELS];     // (T, K[l], D) block centres in bf16
     float* cent;                       // (T, K[l], D)
     uint64_t seed;
-    int32_t niter, pack_rounds, bf, lpr;
+    int32_t niter, pack_rounds, bf;
 };
 int launch_small_levels(const SmallLevels& p, int D, int num_trees, hipStream_t s);
 

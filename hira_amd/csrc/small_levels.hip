@@ -10,9 +10,10 @@
 // operand tiles, the lists and the slots: a round of packing touches no memory.  Sixteen waves on one compute unit are bound
 // by their instructions, and by trips to the level-2 cache for the rows, which are gathered four times (first
 // assignment, means, scores, block centres; the first and the third are asked for ahead, under the first centroids and the means).
-// A launch, 8 trees of 128 columns: 1024 items and 32 centroids 74 us, 256 and 8 26.6, 128 and 4 21.5; 2 x 112 x 12 of 64 columns
-// and the two levels above 40 (95, 33, 27.5 and 49 with the items asked for where they were used, buckets looked for among
-// all items, a wave a centroid at the start and a block at a time at the end).
+// A launch, 8 trees of 128 columns: 1024 items and 32 centroids 64 us, 256 and 8 21, 126 and 4 16.5; 2 x 112 x 12 of 64 columns
+// and the two levels above 28.7 (95, 33, 27.5 and 49 with the items asked for where they were used, buckets looked for among
+// all items, a wave a centroid at the start and a block at a time at the end; 74, 26.6, 21.5 and 40 with all that and numbers
+// rounded to bf16 by shifts and additions).
 //
 // The numbers are those of the launches, bit for bit: the same products in the same order, means and
 // block centres by the same functions (cluster.h), and rules that do not depend on the order of
@@ -32,7 +33,7 @@ constexpr int kSmallBig = kSmallItems / 65 + 1;
 
 // RI, below: item tiles a wave holds at a time, every sixteenth of the tree's: all of its own at the launch's first level, up
 // to four; one of rows of 256 columns, which take twice the registers (a wave has 128).  (Chosen inside the launch, the two sets
-// of registers met in spills: 8 x 1024 x 32 74 -> 112 us; four whatever the items: 128 x 4 31 -> 38.)
+// of registers met in spills: 8 x 1024 x 32 74 -> 112 us; four whatever the items: 128 x 4 25 -> 37.)
 constexpr int kSmallMean = 2;     // steps of a bucket's rows on their way
 constexpr int kSmallPlaces = 64;  // of a bucket, for items in order of arrival: what a wave ranks in registers
 
@@ -77,17 +78,12 @@ template <int KS>
 __device__ __forceinline__ void small_emit(SmallLds<KS>& s, const float (&v)[8], int j, int lanes, bool have, int k, bool usable) {
     float ss = 0.0f;
     if (have && j < KS * 4) {
-        float hi[8], lo[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            hi[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e]));
-            lo[e] = bf16_bits_to_f32(f32_to_bf16_bits(v[e] - hi[e]));
-            const float w = hi[e] + lo[e];
-            ss += w * w;
-        }
+        uint4 hi, lo;
+        float ls = 0.0f;
+        split_bf16(v, hi, lo, ss, ls);
         uint4* out = s.tiles + (k >> 4) * SmallLds<KS>::kTileChunks + (j >> 2) * 64 + (j & 3) * 16 + (k & 15);
-        out[0] = make_uint4(pack_bf16(hi[0], hi[1]), pack_bf16(hi[2], hi[3]), pack_bf16(hi[4], hi[5]), pack_bf16(hi[6], hi[7]));
-        out[KS * 64] = make_uint4(pack_bf16(lo[0], lo[1]), pack_bf16(lo[2], lo[3]), pack_bf16(lo[4], lo[5]), pack_bf16(lo[6], lo[7]));
+        out[0] = hi;
+        out[KS * 64] = lo;
     }
     ss = group_sum_of(ss, lanes);
     if (have && j == 0) s.n2[k] = usable ? ss : INFINITY;
@@ -449,7 +445,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_levels(const SmallLevel
                 slot[b] = lane < bf && k + b * kSmallWaves < K ? s.slots[own * bf + lane] : -1;
                 out[b] = ((size_t)t * K + own) * D;
             }
-            wave_block_means<bf16_t, 4, 2>(x, row0, D, slot, k + kSmallWaves < K ? 2 : 1, bf, p.lpr, out, p.cent, p.cent_t[l]);
+            wave_block_means<bf16_t, 4, 2>(x, row0, D, slot, k + kSmallWaves < K ? 2 : 1, bf, KS * 4, out, p.cent, p.cent_t[l]);
         }
         __syncthreads();  // (the next level reads them)
     }
