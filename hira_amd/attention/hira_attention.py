@@ -83,7 +83,8 @@ def index_thresholds(indexer, query: torch.Tensor, topk: int) -> torch.Tensor:
 def hira_attention_forward(module, query, key, value, attention_mask=None, dropout: float = 0.0,
                            scaling: Optional[float] = None, hira_threshold=None,
                            hira_topk: Optional[int] = None, **kwargs):
-    d = query.shape[-1]
+    shape = query.shape
+    d = shape[-1]
     if scaling is None:
         scaling = getattr(module, "scaling", None) or d ** -0.5
     if not hasattr(key, "indexer"):  # plain tensors: no cache in use
@@ -94,10 +95,10 @@ def hira_attention_forward(module, query, key, value, attention_mask=None, dropo
             raise ValueError(_PADDING_ERROR)
         return _dense(query, cache.prefill_keys, cache.prefill_values, attention_mask, scaling,
                       True), None
-    if query.shape[2] != 1:
+    if shape[2] != 1:
         raise ValueError("sparse decode expects one query position per step")
     indexer, searcher = cache.indexer, cache.searcher
-    b, h_q = query.shape[0], query.shape[1]
+    b, h_q = shape[0], shape[1]
     # a mask that hides keys cannot be honoured by the decode step: looked at once per index
     # (padding does not move between steps, and the look costs a host synchronisation)
     if attention_mask is not None and not getattr(indexer, "_decode_mask_checked", False):
@@ -110,20 +111,27 @@ def hira_attention_forward(module, query, key, value, attention_mask=None, dropo
         hira_topk = getattr(module, "hira_topk", None)
     # with neither given: the cache layer's configured rule on its key sample, one small launch
     # ahead of the search
-    sampled = hira_threshold is None and hira_topk is None and getattr(cache, "samples", None) is not None
+    samples = getattr(cache, "samples", None) if hira_threshold is None and hira_topk is None else None
+    sampled = samples is not None
     if hira_threshold is None and not sampled:
         hira_threshold = index_thresholds(indexer, query, hira_topk or max(1, indexer.num_keys // 100))
     # one plan per (index, head count, scale): a decode step is then a single library call
     plan = searcher.decode_plan(indexer, b * h_q, scaling)
-    dev = indexer.keys_buf.device
+    buf, dtype = indexer.keys_buf, indexer.dtype
+    dev = buf.get_device()
+    # (the search writes its output in the query's own type where that is one of its two)
+    qtype = query.dtype
+    direct = qtype is torch.bfloat16 or qtype is torch.float32
     q2 = query
-    if q2.dtype is not indexer.dtype or q2.device != dev:
-        q2 = q2.to(device=dev, dtype=indexer.dtype)
+    here = query.get_device() == dev
+    if qtype is not dtype or not here:
+        q2 = q2.to(device=buf.device, dtype=dtype)
     if not q2.is_contiguous():
         q2 = q2.contiguous()
-    # (the search writes its output in the query's own type where that is one of its two)
-    direct = query.dtype is torch.bfloat16 or query.dtype is torch.float32
-    out = torch.empty((b, 1, h_q, indexer.vdim), dtype=query.dtype if direct else torch.float32, device=dev)
+    if direct and here:
+        out = query.new_empty((b, 1, h_q, indexer.vdim))
+    else:
+        out = torch.empty((b, 1, h_q, indexer.vdim), dtype=qtype if direct else torch.float32, device=buf.device)
     # the queue: the cache layer's own buffers as they are when they already hold the index's
     # storage type (rows in use, rows per head), else a converted copy of the rows in use
     qk = qv = None
@@ -132,24 +140,23 @@ def hira_attention_forward(module, query, key, value, attention_mask=None, dropo
         qlen = int(cache.queued_keys.shape[-2]) if cache.queued_keys is not None else 0
     if qlen > 0:
         store = getattr(cache, "queue_store", None)
-        if store is not None and store[0].dtype is indexer.dtype and store[0].device == dev \
+        if store is not None and store[0].dtype is dtype and store[0].get_device() == dev \
                 and store[0].is_contiguous() and store[1].is_contiguous():
             qk, qv = store
         else:
-            qk = cache.queued_keys.to(device=dev, dtype=indexer.dtype).reshape(
+            qk = cache.queued_keys.to(device=buf.device, dtype=dtype).reshape(
                 indexer.num_trees, qlen, d).contiguous()
-            qv = cache.queued_values.to(device=dev, dtype=indexer.dtype).reshape(
+            qv = cache.queued_values.to(device=buf.device, dtype=dtype).reshape(
                 indexer.num_trees, qlen, -1).contiguous()
     if sampled:
-        plan.run_sampled(q2, cache.samples, cache.threshold_method, cache.threshold_topk, out,
-                         queue_keys=qk, queue_values=qv, queue_len=qlen)
+        plan.run_sampled(q2, samples, cache.threshold_method, cache.threshold_topk, out, None, qk, qv, qlen)
     else:
-        th = torch.as_tensor(hira_threshold, dtype=torch.float32, device=dev)
+        th = torch.as_tensor(hira_threshold, dtype=torch.float32, device=buf.device)
         if th.ndim == 0:
             th = th.expand(b * h_q)
         th = th.reshape(b * h_q).contiguous()
         plan.run(q2, th, out, queue_keys=qk, queue_values=qv, queue_len=qlen)
-    return (out if direct else out.to(query.dtype)), None
+    return (out if direct else out.to(qtype)), None
 
 
 def register_hira_attention(name: str = "hira") -> str:

@@ -116,9 +116,14 @@ class HiraCacheLayer(CacheLayerMixin):
         if dt not in (torch.float32, torch.bfloat16) or self.dim * esize % 16 or self.vdim * esize % 16:
             self._queue_type = None
         # what a launch is told of the buffers: they are the layer's own, and stay until the next allocation
-        self._queue_at = (self._queue_k.data_ptr(), self._queue_v.data_ptr(), self._queue_type,
-                          self.batch * self.H_kv, rows)
+        self._queue_at = (C.c_void_p(self._queue_k.data_ptr()), C.c_void_p(self._queue_v.data_ptr()),
+                          C.c_int32(self._queue_type or 0), C.c_int32(self.batch * self.H_kv), C.c_int32(rows))
+        self._queue_widths = C.c_int32(self.dim), C.c_int32(self.vdim)
+        self._queue_rows = rows
         self._queue_dev = self._queue_k.get_device()
+        # the shapes of a token's rows (a launch takes them as they are)
+        head = (self.batch, self.H_kv, 1)
+        self._token = torch.Size(head + (self.dim,)), torch.Size(head + (self.vdim,))
 
     @property
     def queued_keys(self):
@@ -137,6 +142,21 @@ class HiraCacheLayer(CacheLayerMixin):
             x.get_device() == like.get_device() and x.is_contiguous() and x.data_ptr() % 16 == 0
 
     def _enqueue(self, key_states, value_states):
+        k, n = self._queue_k, self.queued_len
+        dev, token = self._queue_dev, self._token
+        if n < self._queue_rows and self._queue_type is not None and dev >= 0 and \
+                key_states.shape == token[0] and value_states.shape == token[1] and \
+                key_states.dtype is k.dtype and value_states.dtype is k.dtype and \
+                key_states.get_device() == dev and value_states.get_device() == dev and \
+                key_states.is_contiguous() and value_states.is_contiguous():
+            # a token's rows: what follows, without the questions about shapes
+            kp, vp = key_states.data_ptr(), value_states.data_ptr()
+            if (kp | vp) % 16 == 0:
+                rc = _lib.lib().hira_enqueue(*self._queue_at, n, 1, *self._queue_widths, kp, vp, _lib.stream_of(dev))
+                if rc:
+                    _lib.check(rc)
+                self.queued_len = n + 1
+                return
         m = key_states.shape[-2]
         if self.queued_len + m > self._queue_k.shape[-2]:  # (a step of many tokens)
             old_k, old_v, n = self._queue_k, self._queue_v, self.queued_len
@@ -300,11 +320,11 @@ class HiraCacheLayer(CacheLayerMixin):
     def _output(self, prefill_keys=None, prefill_values=None):
         # (filled in directly: the views of the queue are taken when looked at)
         out = CacheOutput.__new__(CacheOutput)
-        out.__dict__.update(
-            prefill_keys=prefill_keys, prefill_values=prefill_values, indexer=self.indexer,
-            searcher=self.searcher, samples=self.samples, threshold_method=self._rule[0],
-            threshold_topk=self._rule[1], queue_store=(self._queue_k, self._queue_v),
-            queue_rows=self.queued_len)
+        out.__dict__ = {
+            "prefill_keys": prefill_keys, "prefill_values": prefill_values, "indexer": self.indexer,
+            "searcher": self.searcher, "samples": self.samples, "threshold_method": self._rule[0],
+            "threshold_topk": self._rule[1], "queue_store": (self._queue_k, self._queue_v),
+            "queue_rows": self.queued_len}
         return out
 
     def update_index(self):

@@ -424,7 +424,7 @@ class HIPSearcher(BaseSearcher):
         first use and kept: callers that come once per decode step and layer (the attention
         function) then pay one library call per step."""
         plans = self._decode_plans
-        key = (id(indexer), int(num_q_heads), float(scaling))
+        key = (id(indexer), num_q_heads, scaling if type(scaling) is float else float(scaling))
         plan = plans.get(key)
         if plan is None or plan.indexer is not indexer:  # (ids are reused once an index is gone)
             scale = torch.full((num_q_heads,), float(scaling), dtype=torch.float32,
@@ -451,6 +451,7 @@ class DecodePlan:
         self.indexer = indexer
         self.searcher = searcher
         self.lib = _lib.lib()
+        self._search_sampled = self.lib.hira_search_sampled
         dev = indexer.device
         self._dev = indexer.keys_buf.get_device()
         self.scaling = searcher._coerce_scaling(scaling, num_q_heads, dev)
@@ -510,15 +511,16 @@ class DecodePlan:
 
     def _step(self, query, out, queue_keys, queue_values, queue_len):
         """Query, output and queue of a step into the call's structs; the queue's reference, or None."""
-        if self.indexer.tree_struct() is not self.tree:
+        if self.indexer._tree_struct is not self.tree:  # (moved, or not made since the index moved)
             self._follow_index()
         q = self.query
         q.q = query.data_ptr()
         self.out.attn_out = out.data_ptr()
-        q.out_dtype = _OUT_TYPES[out.dtype] if out.dtype in _OUT_TYPES else _refuse_out(out)
+        kind = _OUT_TYPES.get(out.dtype)
+        q.out_dtype = _refuse_out(out) if kind is None else kind
         if queue_keys is None or queue_len == 0:
             return None
-        cap = int(queue_keys.shape[-2])
+        cap = queue_keys.shape[-2]
         if cap == 0:
             return None
         m = cap if queue_len is None else int(queue_len)
@@ -528,7 +530,7 @@ class DecodePlan:
         qs = self.queue
         qs.keys, qs.values, qs.len, qs.cap = queue_keys.data_ptr(), queue_values.data_ptr(), m, cap
         if m > self._ws_rows:
-            self._ws_rows = m
+            self._ws_rows = cap  # (a queue fills up row by row: once for all of them)
             self._follow_index()
         return self._refs[4]
 
@@ -547,11 +549,11 @@ class DecodePlan:
         if tau is None:
             tau = self.tau_buf = torch.empty((self.query.num_q_heads,), dtype=torch.float32,
                                              device=self.indexer.device)
-        tree, shape = self.tree, samples.shape
-        if len(shape) != 3 or shape[0] != tree.num_trees or shape[2] != tree.dim or \
-                samples.dtype != self.indexer.dtype or not samples.is_contiguous():
+        ix, shape = self.indexer, samples.shape
+        if len(shape) != 3 or shape[0] != ix.num_trees or shape[2] != ix.dim or \
+                samples.dtype is not ix.dtype or not samples.is_contiguous():
             raise ValueError(f"samples {tuple(shape)} {samples.dtype}: expected contiguous "
-                             f"({tree.num_trees}, S, {tree.dim}) {self.indexer.dtype}")
+                             f"({ix.num_trees}, S, {ix.dim}) {ix.dtype}")
         if stream is None:
             stream = _lib.stream_of(self._dev)
         rule = 0 if method == "sample_max" else 1
@@ -571,9 +573,9 @@ class DecodePlan:
             return tau
         qu = self._step(query, out, queue_keys, queue_values, queue_len)
         sm = self.sample
-        sm.rows, sm.num_rows, sm.method, sm.k, sm.tau = samples.data_ptr(), shape[1], rule, int(k), tau.data_ptr()
+        sm.rows, sm.num_rows, sm.method, sm.k, sm.tau = samples.data_ptr(), shape[1], rule, k, tau.data_ptr()
         t, q, o, l, _ = self._refs
-        rc = self.lib.hira_search_sampled(t, q, self._sample_ref, qu, o, l, self.ws.data_ptr(), self.ws_bytes, stream)
+        rc = self._search_sampled(t, q, self._sample_ref, qu, o, l, self.ws.data_ptr(), self.ws_bytes, stream)
         if rc:
             _lib.check(rc)
         return tau
