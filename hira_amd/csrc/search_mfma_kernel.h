@@ -200,17 +200,21 @@ struct MfmaShape {
     static constexpr int KA = Q8 ? KS / 2 : KS;  // 16-byte chunks a lane holds of a scanned tile
     // nodes whose key tiles one wave keeps in flight: what the budget of 256 registers leaves
     // after twice the accumulators (GS x D/64) and some seventy registers of everything else
-    // (with the 8-bit shadow: also its B operands, one batch of key rows of the exact test and
-    // the value rows asked for ahead of it), and what keeps the round's list under 48 KiB of LDS
-    static constexpr int KEY_REGS =
-        256 - 72 - 2 * GS * (KS / 2) - (Q8 ? 4 * KS + (KS <= 4 ? 8 : 4) * KS + 32 : 0);
+    // (8-bit shadow: 64 registers, beside which a batch of rows fits without spills), and what keeps the round's
+    // list under 48 KiB of LDS
+    static constexpr int KEY_REGS = Q8 ? 64 : 256 - 72 - 2 * GS * (KS / 2);
     static constexpr int NB_REGS = KEY_REGS / (MT * KA * 4);
     static constexpr int NB_LDS = (12000 / (GS + 1)) / (kMfmaWaves * ROWS);
-    static constexpr int NB_MIN = NB_REGS < NB_LDS ? NB_REGS : NB_LDS;
+    static constexpr int NB_MIN = Q8 || NB_REGS < NB_LDS ? NB_REGS : NB_LDS;
     static constexpr int NB_MAX = Q8 ? 8 : 4;
     static constexpr int NB = NB_MIN < 1 ? 1 : (NB_MIN > NB_MAX ? NB_MAX : NB_MIN);
     static constexpr int LIST = kMfmaWaves * NB * ROWS;  // rows of the list of one round
-    static constexpr int SCAN_WORDS = LIST * (GS + 1) + LIST / 16;  // row list, tile slots, GS scores per row
+    // 8-bit shadow: rows that a wave lists before the workgroup looks at them, and the rounds that never list more;
+    // a batch of rows: its scores, key slots and list entries
+    static constexpr int CAP = 512, CHUNK = CAP / (NB * ROWS);
+    static_assert(!Q8 || CHUNK >= 1, "a round has to fit");
+    static constexpr int SCAN_WORDS = Q8 ? kMfmaWaves * (CAP + kVBatch * (GS + 2))
+                                         : LIST * (GS + 1) + LIST / 16;  // row list, tile slots, GS scores per row
     static constexpr int MERGE_WORDS = kMfmaWaves * 4 * D;  // four heads of every wave
     static constexpr int WORDS = SCAN_WORDS > MERGE_WORDS ? SCAN_WORDS : MERGE_WORDS;
 };
@@ -305,6 +309,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     __shared__ uint4 s_bq8[Q8 ? 2 * KS8 * 64 : 1];
     __shared__ float s_qc[Q8 ? 2 * kHeadsPerPass : 1];
     __shared__ float s_keps[Q8 ? kMfmaMaxTilesPerWg * 16 : 1];
+    __shared__ int s_rows[Q8 ? kMfmaWaves : 1];  // rows that the waves have listed
 
     touch_kernel_arguments();
     const int lane = lane_id();
@@ -377,7 +382,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     // instructions and half the instructions per row of the gather below, which holds a row in
     // 4 bytes a lane.  A launch of several rounds keeps the next round's tiles in flight during
     // the gather: its registers take the eight columns of up to four heads, 233 in all.)
-    constexpr bool WIDE = (ONE ? GS <= 8 : GS <= 4) && !Q8 && KS == 4;
+    constexpr bool WIDE = (ONE || Q8 ? GS <= 8 : GS <= 4) && KS == 4;
     constexpr int LR = D / 8;     // lanes per value row
     constexpr int RPI = 64 / LR;  // rows per load instruction
     const int rg = lane / LR, cc = lane % LR;
@@ -791,412 +796,471 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                 nx_cnt[u] = nx_mask[u] != 0u ? (int)(info >> 16) : 0;
             }
         } else {
-            if (rounds > 0) fetch(0, -1);
+            if (!Q8 && rounds > 0) fetch(0, -1);
         }
         tline.stamp(kTlFetched);
 
-        constexpr int KB0 = KS <= 4 ? 2 : 1;      // batches of 16 key rows asked for ahead
-        constexpr int RP = 64 / GS;               // rows whose weights one pass over the lanes computes
-        constexpr int NPASS = kVBatch / RP;       // GS = 4: 2, GS = 8: 4, GS = 16: 8
-        // one round of a wave
-        auto do_round = [&](const int r) {
-            constexpr bool SINGLE = ONE;
-            // the round's score table and row list; every wave has a stretch of ROWS * NB rows of
-            // its own and nobody else looks at it: no barrier inside the rounds
-            uint32_t* lst_row = s_words;                                        // (LIST) listed row -> table row
-            uint32_t* lst_tslot = lst_row + S::LIST;                            // (LIST/16) table tile -> key slot
-            float* lst_z = reinterpret_cast<float*>(lst_tslot + S::LIST / 16);  // (LIST, GS) the table
-
-            // ---- scan: the key tiles of this round's nodes were asked for a round ago; node by
-            // node: the products, at once the request for the node that takes its place in the
-            // next round, then the node's bookkeeping while the other tiles arrive -------------------
-            // The bookkeeping below derives everything per-lane from this copy, which the compiler
-            // cannot see through: otherwise it computes those values once, ahead of the loop, and
-            // they crowd out the registers that the loads above need.
-            int lane_o = lane;
-            asm volatile("" : "+v"(lane_o));
-            const int col = lane_o & 15, kb = lane_o >> 4;
-
-            int nsel = 0;  // rows of my stretch of the list
-            float zmax = -INFINITY;
-            const int zrow0 = wave * (NB * S::ROWS);  // my stretch of the round's rows
-            int node[NB], cnt[NB];
-            uint32_t nmask[NB];
-            // dense scores / compact lists of the selected rows among 16 scored ones: lane
-            // (kb, head) holds rows 4*kb + j, whose key slots are slot4[j]
-            auto emit = [&](unsigned sel4, const f32x4_t& sco, const unsigned (&slot4)[4]) {
-                unsigned long long sb[4];
+        // dense scores / compact lists of the selected rows among 16 scored ones: lane
+        // (kb, head) holds rows 4*kb + j, whose key slots are slot4[j]
+        auto emit = [&](int col, int kb, unsigned sel4, const f32x4_t& sco, const unsigned (&slot4)[4]) {
+            unsigned long long sb[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) sb[j] = __ballot((sel4 >> j) & 1u);
-                int base = 0;
-                if (p.sel_count != nullptr) {  // one atomic per head of the tile (kb = 0)
-                    int mine = 0;
+            for (int j = 0; j < 4; ++j) sb[j] = __ballot((sel4 >> j) & 1u);
+            int base = 0;
+            if (p.sel_count != nullptr) {  // one atomic per head of the tile (kb = 0)
+                int mine = 0;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        mine += __popcll(sb[j] & (0x0001000100010001ull << col));
-                    int b0 = 0;
-                    if (kb == 0 && mine > 0) b0 = atomicAdd(&p.sel_count[qh], mine);
-                    base = __shfl(b0, col, 64);
-                }
+                for (int j = 0; j < 4; ++j)
+                    mine += __popcll(sb[j] & (0x0001000100010001ull << col));
+                int b0 = 0;
+                if (kb == 0 && mine > 0) b0 = atomicAdd(&p.sel_count[qh], mine);
+                base = __shfl(b0, col, 64);
+            }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if ((sel4 >> j) & 1u) {
-                        const unsigned slot = slot4[j];
-                        int idx = (int)slot;
-                        if (p.dense_by_position) idx = p.perm[row0 + slot];
-                        if (p.dense != nullptr)
-                            p.dense[(int64_t)qh * p.dense_stride + idx] = sco[j] * sc;
-                        if (p.sel_count != nullptr) {
-                            // hits of my head ordered before (kb, j): rows j' < j of any
-                            // kb, then row j of lower kb
-                            int before = 0;
+            for (int j = 0; j < 4; ++j) {
+                if ((sel4 >> j) & 1u) {
+                    const unsigned slot = slot4[j];
+                    int idx = (int)slot;
+                    if (p.dense_by_position) idx = p.perm[row0 + slot];
+                    if (p.dense != nullptr)
+                        p.dense[(int64_t)qh * p.dense_stride + idx] = sco[j] * sc;
+                    if (p.sel_count != nullptr) {
+                        // hits of my head ordered before (kb, j): rows j' < j of any
+                        // kb, then row j of lower kb
+                        int before = 0;
 #pragma unroll
-                            for (int j2 = 0; j2 < 4; ++j2) {
-                                unsigned long long bits = sb[j2] & (0x0001000100010001ull << col);
-                                if (j2 == j) bits &= (1ull << (16 * kb)) - 1ull;
-                                if (j2 <= j) before += __popcll(bits);
-                            }
-                            const int pos = base + before;
-                            if (pos < p.sel_cap) {
-                                p.sel_index[(int64_t)qh * p.sel_cap + pos] = idx;
-                                p.sel_score[(int64_t)qh * p.sel_cap + pos] = sco[j];
-                            }
+                        for (int j2 = 0; j2 < 4; ++j2) {
+                            unsigned long long bits = sb[j2] & (0x0001000100010001ull << col);
+                            if (j2 == j) bits &= (1ull << (16 * kb)) - 1ull;
+                            if (j2 <= j) before += __popcll(bits);
+                        }
+                        const int pos = base + before;
+                        if (pos < p.sel_cap) {
+                            p.sel_index[(int64_t)qh * p.sel_cap + pos] = idx;
+                            p.sel_score[(int64_t)qh * p.sel_cap + pos] = sco[j];
                         }
                     }
                 }
-            };
-            // rows (of 16) for which some head's bit is set: OR over the 16 lanes (heads) of my
-            // row group by rotating inside the group, then the four groups side by side
-            auto rows_of = [&](unsigned sel4) {
-                unsigned any4 = sel4;
-                any4 |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)any4, 0x121, 0xF, 0xF, false);
-                any4 |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)any4, 0x122, 0xF, 0xF, false);
-                any4 |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)any4, 0x124, 0xF, 0xF, false);
-                any4 |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)any4, 0x128, 0xF, 0xF, false);
-                return (unsigned)__builtin_amdgcn_readlane((int)any4, 0) |
-                       ((unsigned)__builtin_amdgcn_readlane((int)any4, 16) << 4) |
-                       ((unsigned)__builtin_amdgcn_readlane((int)any4, 32) << 8) |
-                       ((unsigned)__builtin_amdgcn_readlane((int)any4, 48) << 12);
-            };
-            auto count_selected = [&](unsigned sel4, unsigned rowmask) {
-                const unsigned pairs = (unsigned)__popcll(__ballot(sel4 & 1u)) +
-                                       (unsigned)__popcll(__ballot(sel4 & 2u)) +
-                                       (unsigned)__popcll(__ballot(sel4 & 4u)) +
-                                       (unsigned)__popcll(__ballot(sel4 & 8u));
-                if (lane == 0) {
-                    stat_add(stats, HIRA_MAX_LEVELS, (unsigned)__popc(rowmask));
-                    stat_add(stats, HIRA_MAX_LEVELS + 1, pairs);
+            }
+        };
+        // rows (of 16) for which some head's bit is set: OR over the 16 lanes (heads) of my
+        // row group by rotating inside the group, then the four groups side by side
+        auto rows_of = [&](unsigned sel4) {
+            unsigned any4 = sel4;
+            any4 |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)any4, 0x121, 0xF, 0xF, false);
+            any4 |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)any4, 0x122, 0xF, 0xF, false);
+            any4 |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)any4, 0x124, 0xF, 0xF, false);
+            any4 |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)any4, 0x128, 0xF, 0xF, false);
+            return (unsigned)__builtin_amdgcn_readlane((int)any4, 0) |
+                   ((unsigned)__builtin_amdgcn_readlane((int)any4, 16) << 4) |
+                   ((unsigned)__builtin_amdgcn_readlane((int)any4, 32) << 8) |
+                   ((unsigned)__builtin_amdgcn_readlane((int)any4, 48) << 12);
+        };
+        auto count_selected = [&](unsigned sel4, unsigned rowmask) {
+            const unsigned pairs = (unsigned)__popcll(__ballot(sel4 & 1u)) +
+                                   (unsigned)__popcll(__ballot(sel4 & 2u)) +
+                                   (unsigned)__popcll(__ballot(sel4 & 4u)) +
+                                   (unsigned)__popcll(__ballot(sel4 & 8u));
+            if (lane == 0) {
+                stat_add(stats, HIRA_MAX_LEVELS, (unsigned)__popc(rowmask));
+                stat_add(stats, HIRA_MAX_LEVELS + 1, pairs);
+            }
+        };
+        // ---- the best selected score of every head among rows just scored (zmax), the new
+        // running maximum, and what it does to the sums so far; head g lives in lane g; the
+        // weights are computed with lane = (row, head), head = lane % GS.  Returns the running maximum of head
+        // lane % GS (a finite stand-in for -inf) -----------------------
+        auto raise_max = [&](float zmax) {
+            zmax = cross_group_max<16>(zmax);
+            const float mnew = fmaxf(m_run, zmax);
+            const float f = (m_run == mnew) ? 1.0f : exp2f(m_run - mnew);
+            m_run = mnew;
+            if (__ballot(f != 1.0f) != 0ull) {  // uniform
+                l_mine *= of_head<GS>(f);
+#pragma unroll
+                for (int g = 0; g < GS; ++g) {
+                    const float fg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), g));
+                    if constexpr (WIDE) {
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) acc8[g][j] *= fg;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < VPL; ++e) acc[g][e] *= fg;
+                    }
                 }
-            };
+            }
+            // a head without a selected key has m = -inf and only z = -inf: any finite stand-in
+            return of_head<GS>(mnew == -INFINITY ? 0.0f : mnew);
+        };
+        constexpr int RP = 64 / GS;               // rows whose weights one pass over the lanes computes
+        constexpr int NPASS = kVBatch / RP;       // GS = 4: 2, GS = 8: 4, GS = 16: 8
+        if constexpr (Q8) {
+            // ---- 8-bit shadow: first all tiles, then all rows.  A wave goes through its nodes and lists the rows that
+            // the shadow cannot rule out, with the heads they passed for: a word a row.  Behind a barrier the rows of all
+            // waves are dealt out evenly, kVBatch of a wave at a time: their values and keys asked for together, the exact
+            // test, the running maximum raised to the batch's best scores, the values into the sums.  (Rows looked at
+            // round by round, a batch of 32 places for the twelve that a round of four nodes lists on average, cost every
+            // round a trip to memory, and a wave with many rows kept its workgroup: a step of 8 trees x 131072 keys x 8 heads
+            // 62 us, of which the scan's bytes need 25.)
+            constexpr int CAP = S::CAP;
+            uint32_t* const lists = s_words;                                                   // (waves, CAP)
+            float* const ztab = reinterpret_cast<float*>(s_words + kMfmaWaves * CAP) + wave * (kVBatch * GS);
+            uint32_t* const b_slot = s_words + kMfmaWaves * (CAP + kVBatch * GS) + wave * (2 * kVBatch);
+            uint32_t* const b_word = b_slot + kVBatch;
+            const float slack = su * (kQ8QuerySlack * 127.0f * (float)D), inv_su = 1.0f / su;
+            for (int c0 = 0; c0 < rounds; c0 += S::CHUNK) {  // uniform in the workgroup
+                if (c0 > 0) __syncthreads();  // (the rows listed before have been dealt with)
+                const int c1 = min(c0 + S::CHUNK, rounds);
+                int nl = 0;  // rows on my list
+                fetch(c0, -1);
+                for (int r = c0; r < c1; ++r) {  // uniform
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                node[u] = nx_node[u];
-                cnt[u] = nx_cnt[u];
-                nmask[u] = nx_mask[u];
-                const unsigned slot0 = (unsigned)(node_of(max(node[u], 0)) * bf) + (unsigned)(nx_half[u] * MT * 16);
-                if constexpr (Q8) {
-                    // ---- the shadow's tiles: which rows can it not rule out, for which heads? ----
-                    const float eps_u = nx_eps[u];
-                    i32x4_t est_u[MT];
+                    for (int u = 0; u < NB; ++u) {
+                        const int node = nx_node[u], cnt = nx_cnt[u];
+                        const uint32_t heads = nx_mask[u];
+                        // the score q.k lies within `marg` of su * (the integer): the keys' rounding
+                        // (nx_eps steps a component at most) and the query's (kQ8QuerySlack steps of su)
+                        const float marg = (nx_eps[u] + kQ8KeySlack) * asum + slack;
+                        i32x4_t est[MT];
 #pragma unroll
-                    for (int tt = 0; tt < MT; ++tt)  // (every tile: one that is not there came as zeros)
-                        est_u[tt] = tile_scores_i8<KS8>(a[u][tt], bq8h, bq8l);
-                    // the score q.k lies within `marg` of su * (the integer): the keys' rounding
-                    // (eps_u steps a component at most) and the query's (kQ8QuerySlack steps of su)
-                    const float marg = (eps_u + kQ8KeySlack) * asum + su * (kQ8QuerySlack * 127.0f * (float)D);
-                    const bool head_on = head_ok && ((nmask[u] >> col) & 1u);
-                    const float thr_u = head_on ? tau - marg - 1e-6f * (fabsf(tau) + marg) : INFINITY;
+                        for (int tt = 0; tt < MT; ++tt)  // (every tile: one that is not there came as zeros)
+                            est[tt] = tile_scores_i8<KS8>(a[u][tt], bq8h, bq8l);
+                        fetch(r + 1 < c1 ? r + 1 : 1 << 20, u);  // (past the last round: no node, nothing read)
+                        if (cnt == 0) continue;  // uniform
+                        if (stats && lane == 0) stat_add(stats, 0, (unsigned)cnt);
+                        // (in whole steps, one below: the comparison is one of integers)
+                        const float thr = (tau - marg - 1e-6f * (fabsf(tau) + marg)) * inv_su;
+                        const int least = head_ok && ((heads >> col) & 1u) ? (int)fminf(fmaxf(thr - 1.0f, -2e9f), 2e9f) - 1 : INT32_MAX;
+#pragma unroll
+                        for (int tt = 0; tt < MT; ++tt) {
+                            if (tt * 16 >= cnt) continue;  // uniform
+                            unsigned long long pass[4];
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) pass[j] = __ballot(est[tt][j] >= least);
+                            if ((pass[0] | pass[1] | pass[2] | pass[3]) == 0ull) continue;  // uniform
+                            // row 4 k + j of the tile: its heads are field k of pass[j]; lane i < 16 takes row i
+                            const int j = lane & 3;
+                            const unsigned long long mine = j == 0 ? pass[0] : j == 1 ? pass[1] : j == 2 ? pass[2] : pass[3];
+                            const uint32_t who = (uint32_t)(mine >> (16 * ((lane >> 2) & 3))) & 0xffffu;
+                            const bool in = lane < 16 && who != 0u && tt * 16 + lane < cnt;
+                            const unsigned long long rows = __ballot(in);
+                            if (in)
+                                lists[wave * CAP + nl + __popcll(rows & ((1ull << lane) - 1ull))] =
+                                    (uint32_t)node | ((uint32_t)(tt * 16 + lane) << 8) | (who << 16);
+                            nl += __popcll(rows);
+                        }
+                    }
+                }
+                if (lane == 0) s_rows[wave] = nl;
+                if (c0 == 0) {
+                    tline.stamp_wave(kTlWaveScanned);
+                    tline.stamp(kTlListed);
+                    tline.set(kTlRows, (unsigned long long)nl);
+                    tline.set(kTlRounds, (unsigned long long)rounds);
+                }
+                tline.add_rows(nl);
+                __syncthreads();
+                int ahead[kMfmaWaves + 1];  // rows on the lists of the waves ahead
+                ahead[0] = 0;
+#pragma unroll
+                for (int w = 0; w < kMfmaWaves; ++w) ahead[w + 1] = ahead[w] + (w < nw ? s_rows[w] : 0);
+                const int total = __builtin_amdgcn_readfirstlane(ahead[kMfmaWaves]);
+                const int q0 = total * wave / nw, q1 = total * (wave + 1) / nw;  // my rows
+                if (stats && lane == 0 && wave == 0) stat_add(stats, HIRA_MAX_LEVELS + 2, (unsigned)total);
+                for (int e0 = q0; e0 < q1; e0 += kVBatch) {  // uniform in the wave
+                    // my rows of the batch: list entries and key slots (past the end: no heads, slot 0)
+                    if (lane < kVBatch) {
+                        const int q = min(e0 + lane, q1 - 1);
+                        int at = q;  // (of wave w's list, behind those ahead)
+#pragma unroll
+                        for (int w = 1; w < kMfmaWaves; ++w) at = q >= ahead[w] ? w * CAP + q - ahead[w] : at;
+                        const uint32_t word = lists[at];
+                        const bool there = e0 + lane < q1;
+                        b_word[lane] = there ? word : 0u;
+                        b_slot[lane] = there ? (uint32_t)(node_of((int)(word & 0xffu)) * bf) + ((word >> 8) & 0x3fu) : 0u;
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    constexpr int NLD = WIDE ? kVBatch / RPI : 1;
+                    uint4 vr[NLD];
+                    uint32_t vraw[WIDE ? 1 : kVBatch][VW];
+                    if (want_attn) {
+                        if constexpr (WIDE) {
+#pragma unroll
+                            for (int i = 0; i < NLD; ++i)
+                                vr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                      vrsrc, b_slot[i * RPI + rg] * (unsigned)(D * 2) + (unsigned)cc * 16u, 0, 0));
+                        } else {
+                            const int slots = (int)b_slot[lane & (kVBatch - 1)];
+#pragma unroll
+                            for (int i = 0; i < kVBatch; ++i) {
+                                const unsigned voff = (unsigned)lane * (unsigned)(VPL * 2);
+                                const unsigned soff = (unsigned)__builtin_amdgcn_readlane(slots, i) * (unsigned)(D * 2);
+                                if (VPL == 1) vraw[i][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(vrsrc, voff, soff, 0);
+                                else vraw[i][0] = __builtin_amdgcn_raw_buffer_load_b32(vrsrc, voff, soff, 0);
+                            }
+                        }
+                    }
+                    // the exact test, 16 rows at a time as one A operand (lane (kb, i): columns [32 s + 8 kb, +8) of the i-th)
+                    constexpr int KBV = kVBatch / 16;
+                    uint4 kr[KBV][KS];
+#pragma unroll
+                    for (int b = 0; b < KBV; ++b)
+#pragma unroll
+                        for (int s = 0; s < KS; ++s)
+                            kr[b][s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                     krsrc, b_slot[b * 16 + col] * (unsigned)(D * 2) + (unsigned)(kb * 16 + s * 64), 0, 0));
+                    __builtin_amdgcn_sched_barrier(0);
+                    float zmax = -INFINITY;
+#pragma unroll
+                    for (int b = 0; b < KBV; ++b) {
+                        if (e0 + b * 16 >= q1) continue;  // uniform (no break: the loop has to unroll)
+                        const f32x4_t sco = tile_scores_lds<KS>(kr[b], s_bq, lane);
+                        const uint4 w4 = *reinterpret_cast<const uint4*>(b_word + b * 16 + 4 * kb);
+                        const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
+                        unsigned sel4 = 0u;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            // (its head must be one the shadow let the row pass for)
+                            const bool sel = ((words[j] >> 16 >> col) & 1u) != 0u && sco[j] >= tau;
+                            if (sel) sel4 |= 1u << j;
+                            const float z = sel ? sco[j] * sc2 : -INFINITY;
+                            zmax = fmaxf(zmax, z);
+                            if (col < GS) ztab[(b * 16 + 4 * kb + j) * GS + col] = z;
+                        }
+                        if (stats) count_selected(sel4, rows_of(sel4));
+                        if (OUT && (p.dense != nullptr || p.sel_count != nullptr)) {
+                            const uint4 s4 = *reinterpret_cast<const uint4*>(b_slot + b * 16 + 4 * kb);
+                            const unsigned slot4[4] = {s4.x, s4.y, s4.z, s4.w};
+                            emit(col, kb, sel4, sco, slot4);
+                        }
+                    }
+                    if (c0 == 0 && e0 == q0) tline.stamp_wave(kTlWaveIssued);
+                    if (want_attn) {
+                        const float m_lane = raise_max(zmax);
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        // scores -> weights, in place, 64 (row, head) pairs at a time
+#pragma unroll
+                        for (int ps = 0; ps < NPASS; ++ps) {
+                            if (e0 + ps * RP + lane / GS < q1) {
+                                float* zp = ztab + ps * 64 + lane;
+                                const float w = __builtin_amdgcn_exp2f(*zp - m_lane);
+                                l_mine += w;
+                                *zp = w;
+                            }
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        if constexpr (WIDE) {
+#pragma unroll
+                            for (int i = 0; i < NLD; ++i) {
+                                if (e0 + i * RPI >= q1) break;  // uniform
+                                const bool there = e0 + i * RPI + rg < q1;
+                                float wv[GS];
+#pragma unroll
+                                for (int g4 = 0; g4 < GS / 4; ++g4) {
+                                    float4 w4 = make_float4(0.f, 0.f, 0.f, 0.f);
+                                    if (there) w4 = *reinterpret_cast<const float4*>(ztab + (i * RPI + rg) * GS + 4 * g4);
+                                    wv[4 * g4 + 0] = w4.x;
+                                    wv[4 * g4 + 1] = w4.y;
+                                    wv[4 * g4 + 2] = w4.z;
+                                    wv[4 * g4 + 3] = w4.w;
+                                }
+                                const uint4 raw = there ? vr[i] : make_uint4(0, 0, 0, 0);
+                                float vf[8];
+                                unpack<bf16_t>(raw, vf);
+#pragma unroll
+                                for (int g = 0; g < GS; ++g)
+#pragma unroll
+                                    for (int j = 0; j < 8; ++j) acc8[g][j] += wv[g] * vf[j];
+                            }
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < kVBatch; ++i) {
+                                if ((i & 7) == 0 && e0 + i >= q1) break;  // uniform
+                                const bool there = e0 + i < q1;            // uniform
+                                float vf[VPL];
+                                vf[0] = there ? bf16_lo(vraw[i][0]) : 0.0f;
+                                if (VPL > 1) vf[VPL - 1] = there ? bf16_hi(vraw[i][0]) : 0.0f;
+                                const float* wr = ztab + (there ? i : 0) * GS;  // (a broadcast read)
+#pragma unroll
+                                for (int g = 0; g < GS; ++g)
+#pragma unroll
+                                    for (int e = 0; e < VPL; ++e) acc[g][e] += wr[g] * vf[e];
+                            }
+                        }
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the next batch writes where this one read)
+                    if (c0 == 0 && e0 == q0) tline.stamp_wave(kTlWaveConsumed);
+                }
+                if (c0 == 0) tline.stamp(kTlGathered);
+            }
+        } else {
+            // one round of a wave
+            auto do_round = [&](const int r) {
+                constexpr bool SINGLE = ONE;
+                // the round's score table and row list; every wave has a stretch of ROWS * NB rows of
+                // its own and nobody else looks at it: no barrier inside the rounds
+                uint32_t* lst_row = s_words;                                        // (LIST) listed row -> table row
+                uint32_t* lst_tslot = lst_row + S::LIST;                            // (LIST/16) table tile -> key slot
+                float* lst_z = reinterpret_cast<float*>(lst_tslot + S::LIST / 16);  // (LIST, GS) the table
+
+                // ---- scan: the key tiles of this round's nodes were asked for a round ago; node by
+                // node: the products, at once the request for the node that takes its place in the
+                // next round, then the node's bookkeeping while the other tiles arrive -------------------
+                // The bookkeeping below derives everything per-lane from this copy, which the compiler
+                // cannot see through: otherwise it computes those values once, ahead of the loop, and
+                // they crowd out the registers that the loads above need.
+                int lane_o = lane;
+                asm volatile("" : "+v"(lane_o));
+                const int col = lane_o & 15, kb = lane_o >> 4;
+
+                int nsel = 0;  // rows of my stretch of the list
+                float zmax = -INFINITY;
+                const int zrow0 = wave * (NB * S::ROWS);  // my stretch of the round's rows
+                int node[NB], cnt[NB];
+                uint32_t nmask[NB];
+#pragma unroll
+                for (int u = 0; u < NB; ++u) {
+                    node[u] = nx_node[u];
+                    cnt[u] = nx_cnt[u];
+                    nmask[u] = nx_mask[u];
+                    const unsigned slot0 = (unsigned)(node_of(max(node[u], 0)) * bf) + (unsigned)(nx_half[u] * MT * 16);
+                    if (AHEAD && cnt[u] == 0) continue;  // uniform
+                    f32x4_t sco_u[MT];
+#pragma unroll
+                    for (int tt = 0; tt < MT; ++tt)  // (a tile that is not there came as zeros)
+                        sco_u[tt] = tile_scores_lds<KS>(a[u][tt], s_bq, lane);
+                    if (r == 0 && u == 0) tline.stamp(kTlTiles);
+                    if constexpr (!SINGLE) fetch(r + 1, u);  // (past the last round: no node, nothing read)
+                    // a head for which the node did not survive selects nothing
+                    const float tau_u = ((nmask[u] >> col) & 1u) ? tau : INFINITY;
                     if (stats && lane == 0) stat_add(stats, 0, (unsigned)cnt[u]);
 #pragma unroll
                     for (int tt = 0; tt < MT; ++tt) {
                         if (tt * 16 >= cnt[u]) continue;  // uniform
+                        const f32x4_t sco = sco_u[tt];
                         const int lim = cnt[u] - tt * 16 - 4 * kb;  // my rows j < lim hold keys
-                        unsigned pass4 = 0u;
+                        unsigned sel4 = 0u;
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
-                            if (su * (float)est_u[tt][j] >= thr_u && j < lim) pass4 |= 1u << j;
-                        if (__ballot(pass4 != 0u) == 0ull) continue;  // uniform
-                        const unsigned rowmask = rows_of(pass4);
-                        if (stats && lane == 0) stat_add(stats, HIRA_MAX_LEVELS + 2, (unsigned)__popc(rowmask));
+                            if (sco[j] >= tau_u && j < lim) sel4 |= 1u << j;
+                        if (__ballot(sel4 != 0u) == 0ull) continue;  // uniform
+                        const unsigned rowmask = rows_of(sel4);  // rows selected by some head
+                        if (stats) count_selected(sel4, rowmask);
                         const unsigned tslot = slot0 + tt * 16;
-                        // the tile's rows in the table say, for now, which heads a row passed for
-                        // (0 / -inf); the rows that passed for some head join my list
-                        const int trow = zrow0 + (u * MT + tt) * 16;
-                        if (col < GS) {
-                            float* zp = lst_z + (trow + 4 * kb) * GS + col;
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) zp[j * GS] = ((pass4 >> j) & 1u) ? 0.0f : -INFINITY;
+
+                        // ---- dense scores / compact lists ------------------------------------------
+                        if (OUT && (p.dense != nullptr || p.sel_count != nullptr)) {
+                            const unsigned slot4[4] = {tslot + 4 * kb, tslot + 4 * kb + 1, tslot + 4 * kb + 2,
+                                                       tslot + 4 * kb + 3};
+                            emit(col, kb, sel4, sco, slot4);
                         }
-                        if (lane_o < 16 && ((rowmask >> lane_o) & 1u))
-                            lst_row[zrow0 + nsel + __popc(rowmask & ((1u << lane_o) - 1u))] = (uint32_t)(trow + lane_o);
-                        if (lane_o == 0) lst_tslot[trow >> 4] = tslot;
+
+                        // ---- the tile's scores go to the table, its selected rows join my list -----------
+                        if (want_attn) {
+                            const int trow = zrow0 + (u * MT + tt) * 16;  // the tile's rows in the table
+                            float zs[4];
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                zs[j] = ((sel4 >> j) & 1u) ? sco[j] * sc2 : -INFINITY;
+                                zmax = fmaxf(zmax, zs[j]);
+                            }
+                            if (col < GS) {
+                                float* zp = lst_z + (trow + 4 * kb) * GS + col;
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) zp[j * GS] = zs[j];
+                            }
+                            if (lane_o < 16 && ((rowmask >> lane_o) & 1u))
+                                lst_row[zrow0 + nsel + __popc(rowmask & ((1u << lane_o) - 1u))] = (uint32_t)(trow + lane_o);
+                            if (lane_o == 0) lst_tslot[trow >> 4] = tslot;
+                        }
                         nsel += __popc(rowmask);
                     }
-                } else {
-                if (AHEAD && cnt[u] == 0) continue;  // uniform
-                f32x4_t sco_u[MT];
-#pragma unroll
-                for (int tt = 0; tt < MT; ++tt)  // (a tile that is not there came as zeros)
-                    sco_u[tt] = tile_scores_lds<KS>(a[u][tt], s_bq, lane);
-                if (r == 0 && u == 0) tline.stamp(kTlTiles);
-                if constexpr (!SINGLE) fetch(r + 1, u);  // (past the last round: no node, nothing read)
-                // a head for which the node did not survive selects nothing
-                const float tau_u = ((nmask[u] >> col) & 1u) ? tau : INFINITY;
-                if (stats && lane == 0) stat_add(stats, 0, (unsigned)cnt[u]);
-#pragma unroll
-                for (int tt = 0; tt < MT; ++tt) {
-                    if (tt * 16 >= cnt[u]) continue;  // uniform
-                    const f32x4_t sco = sco_u[tt];
-                    const int lim = cnt[u] - tt * 16 - 4 * kb;  // my rows j < lim hold keys
-                    unsigned sel4 = 0u;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (sco[j] >= tau_u && j < lim) sel4 |= 1u << j;
-                    if (__ballot(sel4 != 0u) == 0ull) continue;  // uniform
-                    const unsigned rowmask = rows_of(sel4);  // rows selected by some head
-                    if (stats) count_selected(sel4, rowmask);
-                    const unsigned tslot = slot0 + tt * 16;
-
-                    // ---- dense scores / compact lists ------------------------------------------
-                    if (OUT && (p.dense != nullptr || p.sel_count != nullptr)) {
-                        const unsigned slot4[4] = {tslot + 4 * kb, tslot + 4 * kb + 1, tslot + 4 * kb + 2,
-                                                   tslot + 4 * kb + 3};
-                        emit(sel4, sco, slot4);
-                    }
-
-                    // ---- the tile's scores go to the table, its selected rows join my list -----------
-                    if (want_attn) {
-                        const int trow = zrow0 + (u * MT + tt) * 16;  // the tile's rows in the table
-                        float zs[4];
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            zs[j] = ((sel4 >> j) & 1u) ? sco[j] * sc2 : -INFINITY;
-                            zmax = fmaxf(zmax, zs[j]);
-                        }
-                        if (col < GS) {
-                            float* zp = lst_z + (trow + 4 * kb) * GS + col;
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) zp[j * GS] = zs[j];
-                        }
-                        if (lane_o < 16 && ((rowmask >> lane_o) & 1u))
-                            lst_row[zrow0 + nsel + __popc(rowmask & ((1u << lane_o) - 1u))] = (uint32_t)(trow + lane_o);
-                        if (lane_o == 0) lst_tslot[trow >> 4] = tslot;
-                    }
-                    nsel += __popc(rowmask);
                 }
-                }  // shadow or bf16 tiles
-            }
-            const int tot = nsel;  // rows on my list
-            if (r == 0) {
-                tline.stamp_wave(kTlWaveScanned);
-                tline.stamp(kTlListed);
-                tline.set(kTlRows, (unsigned long long)tot);
-                tline.set(kTlRounds, (unsigned long long)rounds);
-            }
-            tline.add_rows(tot);
-
-            // ---- value rows: kVBatch in flight; the rows of a batch in the score table (lane =
-            // (row of the pass, head)), their key slots, and the loads ---------------------------------
-            auto issue = [&](int e0, int (&at_v)[NPASS], uint32_t (&vraw)[kVBatch][VW]) {
-#pragma unroll
-                for (int ps = 0; ps < NPASS; ++ps) {
-                    const int le = e0 + ps * RP + lane_o / GS;
-                    at_v[ps] = le < tot ? (int)lst_row[zrow0 + le] : -1;  // (-1: past the end)
+                const int tot = nsel;  // rows on my list
+                if (r == 0) {
+                    tline.stamp_wave(kTlWaveScanned);
+                    tline.stamp(kTlListed);
+                    tline.set(kTlRows, (unsigned long long)tot);
+                    tline.set(kTlRounds, (unsigned long long)rounds);
                 }
-                int slot_v[NPASS];  // the key slots of all the rows of a pass
+                tline.add_rows(tot);
+
+                // ---- value rows: kVBatch in flight; the rows of a batch in the score table (lane =
+                // (row of the pass, head)), their key slots, and the loads ---------------------------------
+                auto issue = [&](int e0, int (&at_v)[NPASS], uint32_t (&vraw)[kVBatch][VW]) {
 #pragma unroll
-                for (int ps = 0; ps < NPASS; ++ps)
-                    slot_v[ps] = at_v[ps] >= 0 ? (int)(lst_tslot[at_v[ps] >> 4] + (unsigned)(at_v[ps] & 15)) : 0;
-                // (a batch is always loaded whole, rows past the end as slot 0: straight-line code;
-                // loads under conditions of their own cost more than they save)
+                    for (int ps = 0; ps < NPASS; ++ps) {
+                        const int le = e0 + ps * RP + lane_o / GS;
+                        at_v[ps] = le < tot ? (int)lst_row[zrow0 + le] : -1;  // (-1: past the end)
+                    }
+                    int slot_v[NPASS];  // the key slots of all the rows of a pass
 #pragma unroll
-                for (int i = 0; i < kVBatch; ++i) {
-                    {
-                        const unsigned slot = (unsigned)__builtin_amdgcn_readlane(slot_v[i / RP], (i % RP) * GS);
-                        const unsigned voff = (unsigned)lane_o * (unsigned)(VPL * 2);
-                        const unsigned soff = slot * (unsigned)(D * 2);
+                    for (int ps = 0; ps < NPASS; ++ps)
+                        slot_v[ps] = at_v[ps] >= 0 ? (int)(lst_tslot[at_v[ps] >> 4] + (unsigned)(at_v[ps] & 15)) : 0;
+                    // (a batch is always loaded whole, rows past the end as slot 0: straight-line code;
+                    // loads under conditions of their own cost more than they save)
+#pragma unroll
+                    for (int i = 0; i < kVBatch; ++i) {
+                        {
+                            const unsigned slot = (unsigned)__builtin_amdgcn_readlane(slot_v[i / RP], (i % RP) * GS);
+                            const unsigned voff = (unsigned)lane_o * (unsigned)(VPL * 2);
+                            const unsigned soff = slot * (unsigned)(D * 2);
+                            if (VPL == 1) {
+                                vraw[i][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(vrsrc, voff, soff, POL == 2 ? kReadOnce : 0);
+                            } else if (VPL == 2) {
+                                vraw[i][0] = __builtin_amdgcn_raw_buffer_load_b32(vrsrc, voff, soff, POL == 2 ? kReadOnce : 0);
+                            } else {
+                                const u32x2_t v2 = __builtin_amdgcn_raw_buffer_load_b64(vrsrc, voff, soff, POL == 2 ? kReadOnce : 0);
+                                vraw[i][0] = v2.x;
+                                vraw[i][VW - 1] = v2.y;
+                            }
+                        }
+                    }
+                };
+                float m_lane = 0.0f;  // (see raise_max)
+                // ---- a batch of value rows into the sums -----------------------------------------------
+                auto consume = [&](int e0, const int (&at_v)[NPASS], const uint32_t (&vraw)[kVBatch][VW]) {
+                    // (nothing of what follows may be scheduled ahead of loads issued before this point)
+                    __builtin_amdgcn_sched_barrier(0);
+                    // scores -> weights, in place, 64 (row, head) pairs at a time
+#pragma unroll
+                    for (int ps = 0; ps < NPASS; ++ps) {
+                        if (at_v[ps] >= 0) {
+                            float* zp = lst_z + at_v[ps] * GS + (lane_o & (GS - 1));
+                            const float w = __builtin_amdgcn_exp2f(*zp - m_lane);
+                            l_mine += w;
+                            *zp = w;
+                        }
+                    }
+                    // eight rows at a time: one test whether the list goes that far, no branch between
+                    // the rows of an eight (their weights and products can then be in flight together);
+                    // a row past the end reads the weights of the batch's first row and counts for nothing
+                    const int at_first = __builtin_amdgcn_readlane(at_v[0], 0);
+#pragma unroll
+                    for (int i = 0; i < kVBatch; ++i) {
+                        if ((i & 7) == 0 && e0 + i >= tot) break;  // uniform
+                        const bool there = e0 + i < tot;           // uniform
+                        const int at_i = __builtin_amdgcn_readlane(at_v[i / RP], (i % RP) * GS);
+                        const int at = there ? at_i : at_first;
+                        float vf[VPL];
                         if (VPL == 1) {
-                            vraw[i][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(vrsrc, voff, soff, POL == 2 ? kReadOnce : 0);
-                        } else if (VPL == 2) {
-                            vraw[i][0] = __builtin_amdgcn_raw_buffer_load_b32(vrsrc, voff, soff, POL == 2 ? kReadOnce : 0);
-                        } else {
-                            const u32x2_t v2 = __builtin_amdgcn_raw_buffer_load_b64(vrsrc, voff, soff, POL == 2 ? kReadOnce : 0);
-                            vraw[i][0] = v2.x;
-                            vraw[i][VW - 1] = v2.y;
-                        }
-                    }
-                }
-            };
-            // ---- the exact test (8-bit shadow): the listed rows' bf16 keys, 16 at a time as one A
-            // operand (lane (kb, i): columns [32 s + 8 kb, +8) of the i-th of them) ---------------------
-            auto rows16 = [&](int e0, int& at, unsigned& slot, uint4 (&kr)[KS]) {
-                const int le = e0 + (lane_o & 15);
-                at = le < tot ? (int)lst_row[zrow0 + le] : -1;  // (-1: past the end)
-                slot = at >= 0 ? lst_tslot[at >> 4] + (unsigned)(at & 15) : 0u;
-#pragma unroll
-                for (int s = 0; s < KS; ++s)
-                    kr[s] = __builtin_bit_cast(
-                        uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                   krsrc, slot * (unsigned)(D * 2) + (unsigned)(kb * 16 + s * 64), 0, 0));
-            };
-            auto exact16 = [&](int at, unsigned slot, const uint4 (&kr)[KS]) {
-                const f32x4_t sco = tile_scores_lds<KS>(kr, s_bq, lane_o);
-                unsigned sel4 = 0u;
-                int at4[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    at4[j] = __shfl(at, 4 * kb + j, 64);
-                    const bool mine = col < GS && at4[j] >= 0;
-                    // (the table holds 0 where the shadow let the row pass for my head)
-                    const float pz = mine ? lst_z[at4[j] * GS + col] : -INFINITY;
-                    const bool sel = pz == 0.0f && sco[j] >= tau;
-                    if (sel) sel4 |= 1u << j;
-                    const float z = sel ? sco[j] * sc2 : -INFINITY;
-                    zmax = fmaxf(zmax, z);
-                    if (mine) lst_z[at4[j] * GS + col] = z;
-                }
-                if (stats) count_selected(sel4, rows_of(sel4));
-                if (OUT && (p.dense != nullptr || p.sel_count != nullptr)) {
-                    unsigned slot4[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) slot4[j] = (unsigned)__shfl((int)slot, 4 * kb + j, 64);
-                    emit(sel4, sco, slot4);
-                }
-            };
-            // ---- what is left to do with the rows of a round (`pr`; the lists and `tot` are its):
-            // the best selected score of every head, the sums rescaled to it, the value rows ----------
-            // ---- the best selected score of every head among rows just scored (zmax), the new
-            // running maximum, and what it does to the sums so far; head g lives in lane g; the
-            // weights are computed with lane = (row, head), head = lane % GS -----------------------
-            float m_lane = 0.0f;  // the running maximum of head lane % GS (a finite stand-in for -inf)
-            auto raise_max = [&]() {
-                zmax = cross_group_max<16>(zmax);
-                const float mnew = fmaxf(m_run, zmax);
-                const float f = (m_run == mnew) ? 1.0f : exp2f(m_run - mnew);
-                m_run = mnew;
-                // a head without a selected key has m = -inf and only z = -inf: any finite stand-in
-                m_lane = of_head<GS>(mnew == -INFINITY ? 0.0f : mnew);
-                if (__ballot(f != 1.0f) != 0ull) {  // uniform
-                    l_mine *= of_head<GS>(f);
-#pragma unroll
-                    for (int g = 0; g < GS; ++g) {
-                        const float fg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), g));
-                        if constexpr (WIDE) {
-#pragma unroll
-                            for (int j = 0; j < 8; ++j) acc8[g][j] *= fg;
+                            vf[0] = there ? bf16_lo(vraw[i][0]) : 0.0f;
                         } else {
 #pragma unroll
-                            for (int e = 0; e < VPL; ++e) acc[g][e] *= fg;
+                            for (int e = 0; e < VPL / 2; ++e) {
+                                vf[2 * e] = there ? bf16_lo(vraw[i][e]) : 0.0f;
+                                vf[2 * e + 1] = there ? bf16_hi(vraw[i][e]) : 0.0f;
+                            }
+                        }
+                        const float* wr = lst_z + at * GS;  // weights of this row, one per head
+#pragma unroll
+                        for (int g = 0; g < GS; ++g) {
+                            const float w = wr[g];  // same address in every lane: a broadcast read
+#pragma unroll
+                            for (int e = 0; e < VPL; ++e) acc[g][e] += w * vf[e];
                         }
                     }
-                }
-            };
-            // ---- a batch of value rows into the sums -----------------------------------------------
-            auto consume = [&](int e0, const int (&at_v)[NPASS], const uint32_t (&vraw)[kVBatch][VW]) {
-                // (nothing of what follows may be scheduled ahead of loads issued before this point)
-                __builtin_amdgcn_sched_barrier(0);
-                // scores -> weights, in place, 64 (row, head) pairs at a time
-#pragma unroll
-                for (int ps = 0; ps < NPASS; ++ps) {
-                    if (at_v[ps] >= 0) {
-                        float* zp = lst_z + at_v[ps] * GS + (lane_o & (GS - 1));
-                        const float w = __builtin_amdgcn_exp2f(*zp - m_lane);
-                        l_mine += w;
-                        *zp = w;
-                    }
-                }
-                // eight rows at a time: one test whether the list goes that far, no branch between
-                // the rows of an eight (their weights and products can then be in flight together);
-                // a row past the end reads the weights of the batch's first row and counts for nothing
-                const int at_first = __builtin_amdgcn_readlane(at_v[0], 0);
-#pragma unroll
-                for (int i = 0; i < kVBatch; ++i) {
-                    if ((i & 7) == 0 && e0 + i >= tot) break;  // uniform
-                    const bool there = e0 + i < tot;           // uniform
-                    const int at_i = __builtin_amdgcn_readlane(at_v[i / RP], (i % RP) * GS);
-                    const int at = there ? at_i : at_first;
-                    float vf[VPL];
-                    if (VPL == 1) {
-                        vf[0] = there ? bf16_lo(vraw[i][0]) : 0.0f;
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < VPL / 2; ++e) {
-                            vf[2 * e] = there ? bf16_lo(vraw[i][e]) : 0.0f;
-                            vf[2 * e + 1] = there ? bf16_hi(vraw[i][e]) : 0.0f;
-                        }
-                    }
-                    const float* wr = lst_z + at * GS;  // weights of this row, one per head
-#pragma unroll
-                    for (int g = 0; g < GS; ++g) {
-                        const float w = wr[g];  // same address in every lane: a broadcast read
-#pragma unroll
-                        for (int e = 0; e < VPL; ++e) acc[g][e] += w * vf[e];
-                    }
-                }
-            };
-            if constexpr (Q8) {
-                // The listed rows go kVBatch at a time: the value rows of the batch (most rows that
-                // the shadow lets through are selected) and their key rows are asked for together,
-                // so a batch costs one trip to memory: exact test, the running maximum raised to the
-                // batch's best scores, the batch's values into the sums.  The first batch is asked
-                // for ahead of the next round's tiles -- loads come back in the order they were asked
-                // for, so its rows are waited for alone, and its work runs while the tiles are on
-                // their way.
-                constexpr int KBV = kVBatch / 16;  // batches of 16 key rows per batch of value rows
-                {
-                    int at_v0[NPASS], at_k[KB0];
-                    uint32_t vraw0[kVBatch][VW];
-                    unsigned slot_k[KB0];
-                    uint4 kr0[KB0][KS];
-                    // (these loads go out whatever the list holds, rows past its end as slot 0: under
-                    // a condition -- even one for all of them -- the waits below can no longer count
-                    // the loads behind them and wait for the next round's tiles as well)
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (want_attn) issue(0, at_v0, vraw0);
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int b = 0; b < KB0; ++b) rows16(16 * b, at_k[b], slot_k[b], kr0[b]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    fetch(r + 1, -1);  // (past the last round: no node, nothing read)
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int b = 0; b < KB0; ++b)
-                        if (16 * b < tot) exact16(at_k[b], slot_k[b], kr0[b]);  // uniform
-                    for (int e0 = 16 * KB0; e0 < min(tot, kVBatch); e0 += 16) {  // (wide rows only)
-                        int at;
-                        unsigned slot;
-                        uint4 kr[KS];
-                        rows16(e0, at, slot, kr);
-                        exact16(at, slot, kr);
-                    }
-                    if (r == 0) tline.stamp_wave(kTlWaveIssued);
-                    if (want_attn && tot > 0) {  // uniform
-                        raise_max();
-                        consume(0, at_v0, vraw0);
-                    }
-                    if (r == 0) tline.stamp_wave(kTlWaveConsumed);
-                }
-                for (int e0 = kVBatch; e0 < tot; e0 += kVBatch) {  // uniform in the wave; a hot wave
-                    int at_v[NPASS], at_k[KB0];
-                    uint32_t vraw[kVBatch][VW];
-                    unsigned slot_k[KB0];
-                    uint4 kr[KB0][KS];
-                    zmax = -INFINITY;
-                    if (want_attn) issue(e0, at_v, vraw);
-#pragma unroll
-                    for (int b0 = 0; b0 < KBV; b0 += KB0) {
-#pragma unroll
-                        for (int b = 0; b < KB0; ++b) rows16(e0 + 16 * (b0 + b), at_k[b], slot_k[b], kr[b]);
-#pragma unroll
-                        for (int b = 0; b < KB0; ++b)
-                            if (e0 + 16 * (b0 + b) < tot) exact16(at_k[b], slot_k[b], kr[b]);  // uniform
-                    }
-                    if (want_attn) {
-                        raise_max();
-                        consume(e0, at_v, vraw);
-                    }
-                }
-            } else {
+                };
                 if constexpr (WIDE) {
                     if (want_attn && tot > 0) {  // uniform in the launch / in the wave
                         constexpr int NLD = kVBatch / RPI;  // load instructions of a batch
@@ -1226,7 +1290,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                             }
                             if (r == 0 && e0 == 0) tline.stamp_wave(kTlWaveIssued);
                             __builtin_amdgcn_sched_barrier(0);
-                            if (e0 == 0) raise_max();  // (while the first values are on their way)
+                            if (e0 == 0) m_lane = raise_max(zmax);  // (while the first values are on their way)
                             // scores -> weights, in place, 64 (row, head) pairs at a time
 #pragma unroll
                             for (int ps = 0; ps < NPASS; ++ps) {
@@ -1264,7 +1328,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     }
                 } else
                 if (want_attn && tot > 0) {  // uniform in the launch / in the wave
-                    raise_max();
+                    m_lane = raise_max(zmax);
                     for (int e0 = 0; e0 < tot; e0 += kVBatch) {  // uniform in the wave
                         int at_v[NPASS];
                         uint32_t vraw[kVBatch][VW];
@@ -1274,14 +1338,14 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                         if (r == 0 && e0 == 0) tline.stamp_wave(kTlWaveConsumed);
                     }
                 }
+                if (r == 0) tline.stamp(kTlGathered);
+            };
+            if constexpr (ONE) {
+                if (rounds > 0) do_round(0);
+            } else {
+                for (int r = 0; r < rounds; ++r) do_round(r);  // uniform in the workgroup
             }
-            if (r == 0) tline.stamp(kTlGathered);
-        };
-        if constexpr (ONE) {
-            if (rounds > 0) do_round(0);
-        } else {
-            for (int r = 0; r < rounds; ++r) do_round(r);  // uniform in the workgroup
-        }
+        }  // shadow or bf16 tiles
     }  // tree or queue
     if (!want_attn) return;  // uniform
     tline.stamp_wave(kTlWaveEnd);
