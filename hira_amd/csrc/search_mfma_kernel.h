@@ -59,6 +59,7 @@ constexpr int kMfmaWaves = kMfmaThreads / 64;  // waves per workgroup, at most: 
 #define HIRA_VBATCH 32
 #endif
 constexpr int kVBatch = HIRA_VBATCH;         // value rows in flight per wave
+constexpr int kQ8Batch = 16;                 // rows that pass the 8-bit shadow, looked at together
 
 __device__ __forceinline__ bf16x8_t as_bf16x8(const uint4& v) {
     return __builtin_bit_cast(bf16x8_t, v);
@@ -213,7 +214,7 @@ struct MfmaShape {
     // a batch of rows: its scores, key slots and list entries
     static constexpr int CAP = 512, CHUNK = CAP / (NB * ROWS);
     static_assert(!Q8 || CHUNK >= 1, "a round has to fit");
-    static constexpr int SCAN_WORDS = Q8 ? kMfmaWaves * (CAP + kVBatch * (GS + 2))
+    static constexpr int SCAN_WORDS = Q8 ? kMfmaWaves * (CAP + kQ8Batch * (GS + 4))
                                          : LIST * (GS + 1) + LIST / 16;  // row list, tile slots, GS scores per row
     static constexpr int MERGE_WORDS = kMfmaWaves * 4 * D;  // four heads of every wave
     static constexpr int WORDS = SCAN_WORDS > MERGE_WORDS ? SCAN_WORDS : MERGE_WORDS;
@@ -904,9 +905,9 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             // 62 us, of which the scan's bytes need 25.)
             constexpr int CAP = S::CAP;
             uint32_t* const lists = s_words;                                                   // (waves, CAP)
-            float* const ztab = reinterpret_cast<float*>(s_words + kMfmaWaves * CAP) + wave * (kVBatch * GS);
-            uint32_t* const b_slot = s_words + kMfmaWaves * (CAP + kVBatch * GS) + wave * (2 * kVBatch);
-            uint32_t* const b_word = b_slot + kVBatch;
+            float* const ztab = reinterpret_cast<float*>(s_words + kMfmaWaves * CAP) + wave * (kQ8Batch * GS);
+            uint32_t* const b_row = s_words + kMfmaWaves * (CAP + kQ8Batch * GS) + wave * (4 * kQ8Batch);
+            uint32_t* const b_word = b_row + 2 * kQ8Batch;
             const float slack = su * (kQ8QuerySlack * 127.0f * (float)D), inv_su = 1.0f / su;
             for (int c0 = 0; c0 < rounds; c0 += S::CHUNK) {  // uniform in the workgroup
                 if (c0 > 0) __syncthreads();  // (the rows listed before have been dealt with)
@@ -967,128 +968,127 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                 const int total = __builtin_amdgcn_readfirstlane(ahead[kMfmaWaves]);
                 const int q0 = total * wave / nw, q1 = total * (wave + 1) / nw;  // my rows
                 if (stats && lane == 0 && wave == 0) stat_add(stats, HIRA_MAX_LEVELS + 2, (unsigned)total);
-                for (int e0 = q0; e0 < q1; e0 += kVBatch) {  // uniform in the wave
-                    // my rows of the batch: list entries and key slots (past the end: no heads, slot 0)
-                    if (lane < kVBatch) {
-                        const int q = min(e0 + lane, q1 - 1);
+                // sixteen rows at a time, the next sixteen on their way meanwhile: what LDS says about them and their loads
+                constexpr int NLD = WIDE ? kQ8Batch / RPI : 1;
+                struct Batch {
+                    uint4 kr[KS];   // the exact test's A operand: lane (kb, i) holds columns [32 s + 8 kb, +8) of the i-th row
+                    uint4 vr[NLD];  // WIDE: values, lane (row group, chunk)
+                    uint32_t vraw[WIDE ? 1 : kQ8Batch][VW];
+                };
+                auto ask = [&](int e0, int half, Batch& o) {
+                    uint32_t* const row_at = b_row + half * kQ8Batch;
+                    if (lane < kQ8Batch) {
+                        const int q = max(min(e0 + lane, q1 - 1), 0);
                         int at = q;  // (of wave w's list, behind those ahead)
 #pragma unroll
                         for (int w = 1; w < kMfmaWaves; ++w) at = q >= ahead[w] ? w * CAP + q - ahead[w] : at;
                         const uint32_t word = lists[at];
                         const bool there = e0 + lane < q1;
-                        b_word[lane] = there ? word : 0u;
-                        b_slot[lane] = there ? (uint32_t)(node_of((int)(word & 0xffu)) * bf) + ((word >> 8) & 0x3fu) : 0u;
+                        b_word[half * kQ8Batch + lane] = there ? word : 0u;
+                        // (past the end: beyond the buffer, zeros and no memory access)
+                        row_at[lane] = there ? ((uint32_t)(node_of((int)(word & 0xffu)) * bf) + ((word >> 8) & 0x3fu)) * (uint32_t)(D * 2) : 0xfffff000u;
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    constexpr int NLD = WIDE ? kVBatch / RPI : 1;
-                    uint4 vr[NLD];
-                    uint32_t vraw[WIDE ? 1 : kVBatch][VW];
                     if (want_attn) {
                         if constexpr (WIDE) {
 #pragma unroll
                             for (int i = 0; i < NLD; ++i)
-                                vr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                                      vrsrc, b_slot[i * RPI + rg] * (unsigned)(D * 2) + (unsigned)cc * 16u, 0, 0));
+                                o.vr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                        vrsrc, row_at[i * RPI + rg] + (unsigned)cc * 16u, 0, 0));
                         } else {
-                            const int slots = (int)b_slot[lane & (kVBatch - 1)];
+                            const int rows = (int)row_at[lane & (kQ8Batch - 1)];
 #pragma unroll
-                            for (int i = 0; i < kVBatch; ++i) {
-                                const unsigned voff = (unsigned)lane * (unsigned)(VPL * 2);
-                                const unsigned soff = (unsigned)__builtin_amdgcn_readlane(slots, i) * (unsigned)(D * 2);
-                                if (VPL == 1) vraw[i][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(vrsrc, voff, soff, 0);
-                                else vraw[i][0] = __builtin_amdgcn_raw_buffer_load_b32(vrsrc, voff, soff, 0);
+                            for (int i = 0; i < kQ8Batch; ++i) {
+                                const unsigned at = (unsigned)__builtin_amdgcn_readlane(rows, i) + (unsigned)lane * (unsigned)(VPL * 2);
+                                if (VPL == 1) o.vraw[i][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(vrsrc, at, 0, 0);
+                                else o.vraw[i][0] = __builtin_amdgcn_raw_buffer_load_b32(vrsrc, at, 0, 0);
                             }
                         }
                     }
-                    // the exact test, 16 rows at a time as one A operand (lane (kb, i): columns [32 s + 8 kb, +8) of the i-th)
-                    constexpr int KBV = kVBatch / 16;
-                    uint4 kr[KBV][KS];
 #pragma unroll
-                    for (int b = 0; b < KBV; ++b)
-#pragma unroll
-                        for (int s = 0; s < KS; ++s)
-                            kr[b][s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                                     krsrc, b_slot[b * 16 + col] * (unsigned)(D * 2) + (unsigned)(kb * 16 + s * 64), 0, 0));
+                    for (int s = 0; s < KS; ++s)
+                        o.kr[s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                                krsrc, row_at[col] + (unsigned)(kb * 16 + s * 64), 0, 0));
                     __builtin_amdgcn_sched_barrier(0);
+                };
+                auto use = [&](int e0, int half, const Batch& o) {
+                    if (e0 >= q1) return;  // uniform
+                    const f32x4_t sco = tile_scores_lds<KS>(o.kr, s_bq, lane);
+                    const uint4 w4 = *reinterpret_cast<const uint4*>(b_word + half * kQ8Batch + 4 * kb);
+                    const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
+                    unsigned sel4 = 0u;
                     float zmax = -INFINITY;
 #pragma unroll
-                    for (int b = 0; b < KBV; ++b) {
-                        if (e0 + b * 16 >= q1) continue;  // uniform (no break: the loop has to unroll)
-                        const f32x4_t sco = tile_scores_lds<KS>(kr[b], s_bq, lane);
-                        const uint4 w4 = *reinterpret_cast<const uint4*>(b_word + b * 16 + 4 * kb);
-                        const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
-                        unsigned sel4 = 0u;
+                    for (int j = 0; j < 4; ++j) {
+                        // (its head must be one the shadow let the row pass for)
+                        const bool sel = ((words[j] >> 16 >> col) & 1u) != 0u && sco[j] >= tau;
+                        if (sel) sel4 |= 1u << j;
+                        const float z = sel ? sco[j] * sc2 : -INFINITY;
+                        zmax = fmaxf(zmax, z);
+                        if (col < GS) ztab[(4 * kb + j) * GS + col] = z;
+                    }
+                    if (stats) count_selected(sel4, rows_of(sel4));
+                    if (OUT && (p.dense != nullptr || p.sel_count != nullptr)) {
+                        const uint4 r4 = *reinterpret_cast<const uint4*>(b_row + half * kQ8Batch + 4 * kb);
+                        const unsigned slot4[4] = {r4.x / (D * 2), r4.y / (D * 2), r4.z / (D * 2), r4.w / (D * 2)};
+                        emit(col, kb, sel4, sco, slot4);
+                    }
+                    if (!want_attn) return;  // uniform
+                    const float m_lane = raise_max(zmax);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    // scores -> weights, in place, 64 (row, head) pairs at a time (past the end: -inf, nothing)
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            // (its head must be one the shadow let the row pass for)
-                            const bool sel = ((words[j] >> 16 >> col) & 1u) != 0u && sco[j] >= tau;
-                            if (sel) sel4 |= 1u << j;
-                            const float z = sel ? sco[j] * sc2 : -INFINITY;
-                            zmax = fmaxf(zmax, z);
-                            if (col < GS) ztab[(b * 16 + 4 * kb + j) * GS + col] = z;
+                    for (int ps = 0; ps < kQ8Batch / RP; ++ps) {
+                        float* zp = ztab + ps * 64 + lane;
+                        const float w = __builtin_amdgcn_exp2f(*zp - m_lane);
+                        l_mine += w;
+                        *zp = w;
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    if constexpr (WIDE) {
+#pragma unroll
+                        for (int i = 0; i < NLD; ++i) {
+                            if (e0 + i * RPI >= q1) break;  // uniform
+                            float wv[GS];
+#pragma unroll
+                            for (int g4 = 0; g4 < GS / 4; ++g4) {
+                                const float4 w = *reinterpret_cast<const float4*>(ztab + (i * RPI + rg) * GS + 4 * g4);
+                                wv[4 * g4 + 0] = w.x;
+                                wv[4 * g4 + 1] = w.y;
+                                wv[4 * g4 + 2] = w.z;
+                                wv[4 * g4 + 3] = w.w;
+                            }
+                            float vf[8];
+                            unpack<bf16_t>(o.vr[i], vf);
+#pragma unroll
+                            for (int g = 0; g < GS; ++g)
+#pragma unroll
+                                for (int j = 0; j < 8; ++j) acc8[g][j] += wv[g] * vf[j];
                         }
-                        if (stats) count_selected(sel4, rows_of(sel4));
-                        if (OUT && (p.dense != nullptr || p.sel_count != nullptr)) {
-                            const uint4 s4 = *reinterpret_cast<const uint4*>(b_slot + b * 16 + 4 * kb);
-                            const unsigned slot4[4] = {s4.x, s4.y, s4.z, s4.w};
-                            emit(col, kb, sel4, sco, slot4);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < kQ8Batch; ++i) {
+                            if ((i & 7) == 0 && e0 + i >= q1) break;  // uniform
+                            float vf[VPL];
+                            vf[0] = bf16_lo(o.vraw[i][0]);
+                            if (VPL > 1) vf[VPL - 1] = bf16_hi(o.vraw[i][0]);
+                            const float* wr = ztab + i * GS;  // (a broadcast read)
+#pragma unroll
+                            for (int g = 0; g < GS; ++g)
+#pragma unroll
+                                for (int e = 0; e < VPL; ++e) acc[g][e] += wr[g] * vf[e];
                         }
                     }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the next sixteen write where these read)
+                };
+                Batch even, odd;
+                ask(q0, 0, even);
+                for (int e0 = q0; e0 < q1; e0 += 2 * kQ8Batch) {  // uniform in the wave
+                    ask(e0 + kQ8Batch, 1, odd);
+                    use(e0, 0, even);
                     if (c0 == 0 && e0 == q0) tline.stamp_wave(kTlWaveIssued);
-                    if (want_attn) {
-                        const float m_lane = raise_max(zmax);
-                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                        // scores -> weights, in place, 64 (row, head) pairs at a time
-#pragma unroll
-                        for (int ps = 0; ps < NPASS; ++ps) {
-                            if (e0 + ps * RP + lane / GS < q1) {
-                                float* zp = ztab + ps * 64 + lane;
-                                const float w = __builtin_amdgcn_exp2f(*zp - m_lane);
-                                l_mine += w;
-                                *zp = w;
-                            }
-                        }
-                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                        if constexpr (WIDE) {
-#pragma unroll
-                            for (int i = 0; i < NLD; ++i) {
-                                if (e0 + i * RPI >= q1) break;  // uniform
-                                const bool there = e0 + i * RPI + rg < q1;
-                                float wv[GS];
-#pragma unroll
-                                for (int g4 = 0; g4 < GS / 4; ++g4) {
-                                    float4 w4 = make_float4(0.f, 0.f, 0.f, 0.f);
-                                    if (there) w4 = *reinterpret_cast<const float4*>(ztab + (i * RPI + rg) * GS + 4 * g4);
-                                    wv[4 * g4 + 0] = w4.x;
-                                    wv[4 * g4 + 1] = w4.y;
-                                    wv[4 * g4 + 2] = w4.z;
-                                    wv[4 * g4 + 3] = w4.w;
-                                }
-                                const uint4 raw = there ? vr[i] : make_uint4(0, 0, 0, 0);
-                                float vf[8];
-                                unpack<bf16_t>(raw, vf);
-#pragma unroll
-                                for (int g = 0; g < GS; ++g)
-#pragma unroll
-                                    for (int j = 0; j < 8; ++j) acc8[g][j] += wv[g] * vf[j];
-                            }
-                        } else {
-#pragma unroll
-                            for (int i = 0; i < kVBatch; ++i) {
-                                if ((i & 7) == 0 && e0 + i >= q1) break;  // uniform
-                                const bool there = e0 + i < q1;            // uniform
-                                float vf[VPL];
-                                vf[0] = there ? bf16_lo(vraw[i][0]) : 0.0f;
-                                if (VPL > 1) vf[VPL - 1] = there ? bf16_hi(vraw[i][0]) : 0.0f;
-                                const float* wr = ztab + (there ? i : 0) * GS;  // (a broadcast read)
-#pragma unroll
-                                for (int g = 0; g < GS; ++g)
-#pragma unroll
-                                    for (int e = 0; e < VPL; ++e) acc[g][e] += wr[g] * vf[e];
-                            }
-                        }
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the next batch writes where this one read)
+                    ask(e0 + 2 * kQ8Batch, 0, even);
+                    use(e0 + kQ8Batch, 1, odd);
                     if (c0 == 0 && e0 == q0) tline.stamp_wave(kTlWaveConsumed);
                 }
                 if (c0 == 0) tline.stamp(kTlGathered);
