@@ -81,6 +81,10 @@ struct SearchParams {
     int32_t out_bf16;   // attn_out's type: bf16, else fp32
     uint32_t bf_magic;  // ceil(2^32 / bf): n / bf = the high word of n * bf_magic (bf > 1, n < 2^26)
     unsigned long long* stats;
+    // MFMA kernel: levels min(L - 1, 3) and the one below, as far as they lie above level 1
+    const void* anc_centers[2];
+    const float* anc_radii[2];
+    int32_t anc_cap[2];
 };
 
 // element i of the attention output, in the type the caller asked for
@@ -133,30 +137,38 @@ __device__ __forceinline__ void hand_off_release() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
 }
 
-// The kernel's arguments lie in nine 64-byte lines of memory, and compiled code asks for each
+// The kernel's arguments lie in ten 64-byte lines of memory, and compiled code asks for each
 // argument where it is first needed: line after line, each a trip to memory that the next one
 // waits for (measured: the gates began 1.5 us after the workgroup).  Asking for a word of every
 // line here, at once, makes them one trip; the reads of the arguments that follow are served from
 // the scalar cache.  (The wait is inside the statement: its destination registers are free again
 // when it ends.)
 __device__ __forceinline__ void touch_kernel_arguments() {
-    static_assert(sizeof(SearchParams) <= 9 * 64, "one load per 64-byte line of the arguments");
+    static_assert(sizeof(SearchParams) > 9 * 64 + 4 && sizeof(SearchParams) <= 10 * 64, "one load per 64-byte line of the arguments");
     auto ka = __builtin_amdgcn_kernarg_segment_ptr();
-    uint32_t d0, d1, d2, d3, d4, d5, d6, d7, d8;
+    uint32_t d0, d1, d2, d3, d4, d5, d6, d7, d8, d9;
     asm volatile(
-        "s_load_dword %0, %9, 0x0\n\t"
-        "s_load_dword %1, %9, 0x40\n\t"
-        "s_load_dword %2, %9, 0x80\n\t"
-        "s_load_dword %3, %9, 0xc0\n\t"
-        "s_load_dword %4, %9, 0x100\n\t"
-        "s_load_dword %5, %9, 0x140\n\t"
-        "s_load_dword %6, %9, 0x180\n\t"
-        "s_load_dword %7, %9, 0x1c0\n\t"
-        "s_load_dword %8, %9, 0x200\n\t"
+        "s_load_dword %0, %10, 0x0\n\t"
+        "s_load_dword %1, %10, 0x40\n\t"
+        "s_load_dword %2, %10, 0x80\n\t"
+        "s_load_dword %3, %10, 0xc0\n\t"
+        "s_load_dword %4, %10, 0x100\n\t"
+        "s_load_dword %5, %10, 0x140\n\t"
+        "s_load_dword %6, %10, 0x180\n\t"
+        "s_load_dword %7, %10, 0x1c0\n\t"
+        "s_load_dword %8, %10, 0x200\n\t"
+        "s_load_dword %9, %10, 0x240\n\t"
         "s_waitcnt lgkmcnt(0)"
-        : "=&s"(d0), "=&s"(d1), "=&s"(d2), "=&s"(d3), "=&s"(d4), "=&s"(d5), "=&s"(d6), "=&s"(d7), "=&s"(d8)
+        : "=&s"(d0), "=&s"(d1), "=&s"(d2), "=&s"(d3), "=&s"(d4), "=&s"(d5), "=&s"(d6), "=&s"(d7), "=&s"(d8), "=&s"(d9)
         : "s"(ka)
         : "memory");
+}
+
+// The address `a` of global memory.  (A pointer that has been through a statement of the assembler's is one the
+// compiler loads through without knowing where it points: such arguments are kept as numbers.)
+template <typename T>
+__device__ __forceinline__ const T* global_at(uintptr_t a) {
+    return (const T*)reinterpret_cast<const __attribute__((address_space(1))) T*>(a);
 }
 
 // Where the keys / the centers of a tree layout sit (HIRA_TILE16_Q8: tiled centers, row-major

@@ -321,6 +321,13 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
         p.size[l] = tree->size[l];
         p.cap[l] = tree->cap[l];
     }
+    for (int i = 0; i < 2; ++i) {
+        const int l = (tree->num_levels - 1 < 3 ? tree->num_levels - 1 : 3) - i;
+        if (l < 2) break;
+        p.anc_centers[i] = tree->centers[l];
+        p.anc_radii[i] = tree->radii[l];
+        p.anc_cap[i] = tree->cap[l];
+    }
     p.num_levels = tree->num_levels;
     p.bf = tree->bf;
     p.bf_magic = tree->bf > 1 ? (uint32_t)((((uint64_t)1 << 32) + tree->bf - 1) / tree->bf) : 0;

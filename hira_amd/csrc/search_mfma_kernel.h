@@ -232,21 +232,44 @@ struct GateLoads {
     unsigned aid[2];
 };
 
+// The arguments that the kernel needs up to the gates, in registers from its first instructions on.  Asked for where they
+// are used they came one after the other, each behind its branch and its wait, a dozen hits of the scalar cache ahead of
+// the last gate's operands (8 trees x 2000 keys 9.48 -> 9.21 us; x 32768, which waits for its fullest workgroup, 17.7 either way).
+// (Addresses as numbers: global_at.)
+struct GateArgs {
+    uintptr_t q, centers, anc_centers[2], tau, scaling, radii, anc_radii[2], keps, counts, keys, part_acc, stats;
+    int32_t num_levels, cap, anc_cap[2], size, group_size, tree_blocks, tiles, bf, cap0, wgs, threads;
+    uint32_t bf_magic;
+};
+__device__ __forceinline__ GateArgs gate_arguments(const SearchParams& p) {
+    auto at = [](const void* a) { return reinterpret_cast<uintptr_t>(a); };
+    GateArgs g{at(p.q), at(p.centers[1]), {at(p.anc_centers[0]), at(p.anc_centers[1])}, at(p.tau), at(p.scaling), at(p.radii[1]),
+               {at(p.anc_radii[0]), at(p.anc_radii[1])}, at(p.keps), at(p.counts[1]), at(p.keys), at(p.part_acc), at(p.stats),
+               p.num_levels, p.cap[1], {p.anc_cap[0], p.anc_cap[1]}, p.size[1], p.group_size,
+               p.tree_blocks, p.nodes_per_wave, p.bf, p.cap[0], (int)gridDim.y, (int)blockDim.x, p.bf_magic};
+    asm volatile("" : "+s"(g.q), "+s"(g.centers), "+s"(g.anc_centers[0]), "+s"(g.anc_centers[1]), "+s"(g.tau), "+s"(g.scaling),
+                      "+s"(g.radii), "+s"(g.anc_radii[0]), "+s"(g.anc_radii[1]), "+s"(g.keps), "+s"(g.counts),
+                      "+s"(g.keys), "+s"(g.part_acc), "+s"(g.stats));
+    asm volatile("" : "+s"(g.num_levels), "+s"(g.cap), "+s"(g.anc_cap[0]), "+s"(g.anc_cap[1]), "+s"(g.size), "+s"(g.group_size),
+                      "+s"(g.tree_blocks), "+s"(g.tiles), "+s"(g.bf), "+s"(g.cap0), "+s"(g.wgs), "+s"(g.threads), "+s"(g.bf_magic));
+    return g;
+}
+
 // Parent of node n.  By a multiplication: the quotients of 64-bit numbers that stood here, one after the
 // other ahead of the ancestors' loads, were 0.3 us of every step (8 trees x 2000 keys 12.7 -> 12.4 us, x 32768 19.6 -> 19.2).
-__device__ __forceinline__ unsigned node_over_bf(const SearchParams& p, unsigned n) {
+__device__ __forceinline__ unsigned node_over_bf(const GateArgs& p, unsigned n) {
     return __umulhi(n, p.bf_magic);  // (fan-outs of 16 and more: never 1)
 }
 
 template <int KS, bool Q8>
-__device__ __forceinline__ void gate_issue(const SearchParams& p, int tree, int t1, int lane,
+__device__ __forceinline__ void gate_issue(const GateArgs& p, int tree, int t1, int lane,
                                            int kb, GateLoads<KS>& g) {
     const int L = p.num_levels;
-    const size_t row1 = (size_t)tree * p.cap[1];
-    load_tile<KS>(tile_ptr<KS>(p.centers[1], row1, (size_t)t1, lane), g.a1);
-    g.r4 = *reinterpret_cast<const float4*>(p.radii[1] + row1 + (size_t)t1 * 16 + 4 * kb);
-    g.cn = p.counts[1][row1 + (size_t)t1 * 16 + (lane & 15)];
-    if (Q8) g.en = p.keps[row1 + (size_t)t1 * 16 + (lane & 15)];
+    const size_t row1 = (size_t)tree * p.cap;
+    load_tile<KS>(tile_ptr<KS>(global_at<char>(p.centers), row1, (size_t)t1, lane), g.a1);
+    g.r4 = *reinterpret_cast<const float4*>(global_at<float>(p.radii) + row1 + (size_t)t1 * 16 + 4 * kb);
+    g.cn = global_at<int32_t>(p.counts)[row1 + (size_t)t1 * 16 + (lane & 15)];
+    if (Q8) g.en = global_at<float>(p.keps)[row1 + (size_t)t1 * 16 + (lane & 15)];
     const int n_par = min(max(L - 2, 0), 2);
     const unsigned id2 = node_over_bf(p, (unsigned)t1 * 16u);
 #pragma unroll
@@ -256,9 +279,8 @@ __device__ __forceinline__ void gate_issue(const SearchParams& p, int tree, int 
         if (i < n_par) {
             const int l = min(L - 1, 3) - i;
             g.aid[i] = l == 3 ? node_over_bf(p, id2) : id2;
-            load_tile<KS>(tile_ptr<KS>(p.centers[l], (size_t)tree * p.cap[l], g.aid[i] / 16, lane),
-                          g.anc[i]);
-            g.arad[i] = p.radii[l][(size_t)tree * p.cap[l] + g.aid[i]];
+            load_tile<KS>(tile_ptr<KS>(global_at<char>(p.anc_centers[i]), (size_t)tree * p.anc_cap[i], g.aid[i] / 16, lane), g.anc[i]);
+            g.arad[i] = global_at<float>(p.anc_radii[i])[(size_t)tree * p.anc_cap[i] + g.aid[i]];
         }
     }
 }
@@ -313,17 +335,18 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     __shared__ int s_rows[Q8 ? kMfmaWaves : 1];  // rows that the waves have listed
 
     touch_kernel_arguments();
+    const GateArgs ga = gate_arguments(p);
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int nw = blockDim.x >> 6;
+    const int nw = ga.threads >> 6;
     const int col = lane & 15;  // head within the pass
     const int kb = lane >> 4;   // column block of 8 inside each 32-column step
     const int tree = blockIdx.x;
-    const int L = p.num_levels, bf = p.bf;
-    const bool want_attn = p.part_acc != nullptr;
+    const int L = ga.num_levels, bf = ga.bf;
+    const bool want_attn = ga.part_acc != 0;
     static_assert(!SAMPLED || (AHEAD && S::WORDS >= kTauFewRows), "");
     __shared__ float s_tau[SAMPLED ? kHeadsPerPass : 1];
-    int wgs = gridDim.y, wg = blockIdx.y;  // searching workgroups of the tree, my number among them
+    int wgs = ga.wgs, wg = blockIdx.y;  // searching workgroups of the tree, my number among them
     if constexpr (SAMPLED) {
         wgs -= p.sample_wgs;
         wg -= p.sample_wgs;
@@ -336,26 +359,26 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     // Workgroup y of a tree owns the tree's tiles y, y + (workgroups of the tree), ...: a stride
     // apart, since neighbouring tiles hold sibling nodes, which tend to survive (and be selected
     // from) together.
-    const int wg_tiles = (p.size[1] + 15) >> 4;
-    const int n_groups = p.tree_blocks;
+    const int wg_tiles = (ga.size + 15) >> 4;
+    const int n_groups = ga.tree_blocks;
     const int grp = wg;
-    const int ntile = wg < p.tree_blocks
-                          ? min(p.nodes_per_wave, (wg_tiles - grp + n_groups - 1) / n_groups)
+    const int ntile = wg < ga.tree_blocks
+                          ? min(ga.tiles, (wg_tiles - grp + n_groups - 1) / n_groups)
                           : 0;
     auto tile_of = [&](int tl) { return grp + tl * n_groups; };
     // level-1 node behind entry n (tile n / 16 of mine, node n % 16 of the tile)
     auto node_of = [&](int n) { return tile_of(n >> 4) * 16 + (n & 15); };
-    const bool is_queue = wg >= p.tree_blocks;  // the workgroup after the tree's
+    const bool is_queue = wg >= ga.tree_blocks;  // the workgroup after the tree's
     Timeline tline(p);  // (empty unless the library is built with time stamps)
     unsigned long long* stats =
-        (p.stats && !Timeline::kOn) ? p.stats + (size_t)tree * HIRA_STATS_COLS : nullptr;
+        (ga.stats != 0 && !Timeline::kOn) ? p.stats + (size_t)tree * HIRA_STATS_COLS : nullptr;
     tline.stamp(kTlStart);
 
     // ---- heads of this pass ----------------------------------------------------------
     int hoff, G;
-    if (p.group_size > 0) {  // head h of the launch belongs to tree h / group_size
-        hoff = tree * p.group_size + blockIdx.z * kHeadsPerPass;
-        G = min(kHeadsPerPass, p.group_size - (int)blockIdx.z * kHeadsPerPass);
+    if (ga.group_size > 0) {  // head h of the launch belongs to tree h / group_size
+        hoff = tree * ga.group_size + blockIdx.z * kHeadsPerPass;
+        G = min(kHeadsPerPass, ga.group_size - (int)blockIdx.z * kHeadsPerPass);
     } else {
         hoff = p.tree_q_off[tree] + blockIdx.z * kHeadsPerPass;
         G = min(kHeadsPerPass, p.tree_q_off[tree + 1] - hoff);
@@ -365,7 +388,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     tline.stamp(kTlArgs);
     const bool head_ok = col < G;
     int qh = 0;
-    if (head_ok) qh = p.group_size > 0 ? hoff + col : p.tree_q_heads[hoff + col];
+    if (head_ok) qh = ga.group_size > 0 ? hoff + col : p.tree_q_heads[hoff + col];
 
     // ---- softmax state: running maximum m of the lane's head (the same in every wave);
     // per wave: l over the rows it gathered, acc[g][e] = column lane*VPL + e of head g -------
@@ -467,23 +490,23 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         uint4 qraw[KS];
 #pragma unroll
         for (int s = 0; s < KS; ++s) qraw[s] = make_uint4(0, 0, 0, 0);
-        float tau = SAMPLED ? 0.0f : p.tau[qh];
-        float sc = p.scaling[qh];
+        float tau = SAMPLED ? 0.0f : global_at<float>(ga.tau)[qh];
+        float sc = global_at<float>(ga.scaling)[qh];
         GateLoads<KS> gl;
         uint4 a[NB][MT][KA];  // key tiles of the nodes that a wave takes in a round
         if (tl_mine < ntile) {
 #pragma unroll
             for (int s = 0; s < KS; ++s)
-                qraw[s] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.q) +
+                qraw[s] = *reinterpret_cast<const uint4*>(global_at<uint16_t>(ga.q) +
                                                           (size_t)qh * D + s * 32 + kb * 8);
-            gate_issue<KS, Q8>(p, tree, tile_of(tl_mine), lane, kb, gl);
+            gate_issue<KS, Q8>(ga, tree, tile_of(tl_mine), lane, kb, gl);
         }
         if constexpr (AHEAD) {
             // (slots beyond the capacity, under nodes that pad the tile or a last node of 48: zeros, no memory
             // access)
-            const size_t r0 = (size_t)tree * p.cap[0];
+            const size_t r0 = (size_t)tree * ga.cap0;
             const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(
-                reinterpret_cast<const uint16_t*>(p.keys) + r0 * (size_t)D, (size_t)p.cap[0] * D * 2);
+                global_at<uint16_t>(ga.keys) + r0 * (size_t)D, (size_t)ga.cap0 * D * 2);
 #pragma unroll
             for (int u = 0; u < NB; ++u)
 #pragma unroll
@@ -622,7 +645,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             // the tile's ancestor at level l; is the tile's first node its first descendant?
             auto ancestor = [&](int l) {
                 unsigned id = (unsigned)t1 * 16u;
-                for (int i = 1; i < l; ++i) id = node_over_bf(p, id);
+                for (int i = 1; i < l; ++i) id = node_over_bf(ga, id);
                 return id;
             };
             auto leads = [&](int l) {
@@ -682,7 +705,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                 if (lane < 16) s_keps[tl_mine * 16 + lane] = gl.en;
             }
             tl_mine += nw;
-            if (tl_mine < ntile) gate_issue<KS, Q8>(p, tree, tile_of(tl_mine), lane, kb, gl);
+            if (tl_mine < ntile) gate_issue<KS, Q8>(ga, tree, tile_of(tl_mine), lane, kb, gl);
         }
         tline.stamp(kTlGated);
         __syncthreads();
@@ -722,14 +745,14 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         asm volatile("" : "+v"(sc2));  // (computed here, where its load has long arrived, and not
                                        // behind the key tiles' requests, where it would be waited
                                        // for with all of them)
-        const size_t row0 = (size_t)tree * p.cap[0];
+        const size_t row0 = (size_t)tree * ga.cap0;
 
         // (8-bit shadow: krsrc = the bf16 rows of the exact test, row-major; k8rsrc = the tiles
         // of the shadow, which the scan reads)
         const __amdgpu_buffer_rsrc_t krsrc = make_rsrc(
-            reinterpret_cast<const uint16_t*>(p.keys) + row0 * (size_t)D, (size_t)p.cap[0] * D * 2);
+            global_at<uint16_t>(ga.keys) + row0 * (size_t)D, (size_t)ga.cap0 * D * 2);
         const __amdgpu_buffer_rsrc_t k8rsrc =
-            Q8 ? make_rsrc(p.keys8 + row0 * (size_t)D, (size_t)p.cap[0] * D) : krsrc;
+            Q8 ? make_rsrc(p.keys8 + row0 * (size_t)D, (size_t)ga.cap0 * D) : krsrc;
         uint4 bq8h[KS8], bq8l[KS8];
         float su = 0.0f, asum = 0.0f;
         if constexpr (Q8) {
@@ -742,7 +765,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             asum = s_qc[kHeadsPerPass + col];
         }
         const __amdgpu_buffer_rsrc_t vrsrc = make_rsrc(
-            reinterpret_cast<const uint16_t*>(p.values) + row0 * (size_t)D, (size_t)p.cap[0] * D * 2);
+            reinterpret_cast<const uint16_t*>(p.values) + row0 * (size_t)D, (size_t)ga.cap0 * D * 2);
         // The nodes a wave takes in a round (up to NB of its share), what LDS says about them,
         // and the loads of their key tiles.
         int nx_node[NB], nx_cnt[NB], nx_half[NB];
