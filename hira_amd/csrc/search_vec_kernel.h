@@ -297,6 +297,45 @@ __device__ __forceinline__ void fold_heads(const SearchParams& p, int hoff, int 
     }
 }
 
+// The arguments that the kernel needs up to the keys, in registers from its first instructions on (asked for where they
+// are used they came one after the other, each behind its branch and its wait).  Levels 1, 2 and the one above
+// that the wave has for itself, whether they are there or not.  (4 trees x 5003 rows of 80 fp32, three
+// heads each: 11.5 -> 11.15 us.)
+struct VecArgs {
+    const void *q, *keys, *queue_keys, *centers[3];
+    const float *tau, *scaling, *radii[3];
+    const int32_t* counts;
+    int32_t level_cap[3], dim, num_levels, group_size, tree_blocks, num_queue_blocks, num_nodes, queue_nodes, nodes_per_wg;
+    int32_t queue_cap, cap[1], queue_len, size[1], bf, layout, key_layout, wgs;
+    uint32_t bf_magic;
+};
+__device__ __forceinline__ VecArgs vec_arguments(const SearchParams& p, int upper) {
+    VecArgs v{p.q, p.keys, p.queue_keys, {p.centers[1], p.centers[2], p.centers[upper]}, p.tau, p.scaling,
+              {p.radii[1], p.radii[2], p.radii[upper]}, p.counts[1], {p.cap[1], p.cap[2], p.cap[upper]}, p.dim, p.num_levels,
+              p.group_size, p.tree_blocks, p.num_queue_blocks, p.num_nodes, p.queue_nodes, p.nodes_per_wg, p.queue_cap, {p.cap[0]},
+              p.queue_len, {p.size[0]}, p.bf, p.layout, p.key_layout, (int)gridDim.x, p.bf_magic};
+    auto at = [](const void* a) { return reinterpret_cast<uintptr_t>(a); };
+    uintptr_t q = at(v.q), keys = at(v.keys), queue = at(v.queue_keys), tau = at(v.tau), scaling = at(v.scaling),
+              c0 = at(v.centers[0]), c1 = at(v.centers[1]), c2 = at(v.centers[2]), r0 = at(v.radii[0]), r1 = at(v.radii[1]),
+              r2 = at(v.radii[2]), counts = at(v.counts);
+    asm volatile("" : "+s"(v.queue_cap), "+s"(v.cap[0]), "+s"(v.queue_len), "+s"(v.size[0]), "+s"(v.bf), "+s"(v.layout),
+                      "+s"(v.key_layout), "+s"(v.wgs), "+s"(v.bf_magic));
+    asm volatile("" : "+s"(v.level_cap[0]), "+s"(v.level_cap[1]), "+s"(v.level_cap[2]), "+s"(v.dim), "+s"(v.num_levels),
+                      "+s"(v.group_size), "+s"(v.tree_blocks), "+s"(v.num_queue_blocks), "+s"(v.num_nodes), "+s"(v.queue_nodes),
+                      "+s"(v.nodes_per_wg));
+    asm volatile("" : "+s"(q), "+s"(keys), "+s"(queue), "+s"(tau), "+s"(scaling), "+s"(c0), "+s"(c1), "+s"(c2), "+s"(r0),
+                      "+s"(r1), "+s"(r2), "+s"(counts));
+    v.q = global_at<char>(q), v.keys = global_at<char>(keys), v.queue_keys = global_at<char>(queue);
+    v.tau = global_at<float>(tau), v.scaling = global_at<float>(scaling), v.counts = global_at<int32_t>(counts);
+    v.centers[0] = global_at<char>(c0), v.centers[1] = global_at<char>(c1), v.centers[2] = global_at<char>(c2);
+    v.radii[0] = global_at<float>(r0), v.radii[1] = global_at<float>(r1), v.radii[2] = global_at<float>(r2);
+    return v;
+}
+
+// Argument x of the kernel: with ONE as vec_arguments has it, else where it lies.  (The general way, which asks for keys
+// once it has its list of nodes, was slower with all of them in registers from the start: 90000 rows of 128 fp32 8.6 -> 8.8 us.)
+#define VEC_ARG(x) (ONE ? va.x : p.x)
+
 // ONE > 0: every workgroup of the launch has one batch of nodes whose key slots are one block of rows for
 // each of its eight waves (of ONE elements a lane).  A wave then asks for its block together with the gates'
 // operands of all levels, whether the nodes survive or not: no list, two trips to memory and a barrier less,
@@ -332,24 +371,27 @@ void search_kernel(const SearchParams p) {
     // (uniform, as the compiler would not know: a level picked by it has its arguments read by vector loads otherwise,
     // a trip to memory ahead of the rows')
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int nwaves = blockDim.x >> 6;
+    // (the level above the second that a wave has for itself: ONE's workgroups are full ones, whose first wave has none)
+    [[maybe_unused]] VecArgs va;
+    if constexpr (ONE) va = vec_arguments(p, min(2 + wave, HIRA_MAX_LEVELS - 1));
+    const int nwaves = ONE ? WAVES : (int)(blockDim.x >> 6);
     const int rg = lane / LPR;
     const int ch = lane % LPR;
     const int tree = blockIdx.y;
-    const int D = p.dim;
+    const int D = VEC_ARG(dim);
     const int Dv = p.vdim;
-    const int L = p.num_levels;
+    const int L = VEC_ARG(num_levels);
     const bool chunk_ok = ch * EPL < D;
     const bool vchunk_ok = ch * EPL < Dv;
     const bool want_attn = p.part_acc != nullptr;
 
     // (group_size > 0: head h of the launch belongs to tree h / group_size; the head map is not
     // read, which saves every wave two dependent trips to memory)
-    const bool by_group = p.group_size > 0;
-    const int hoff = (by_group ? tree * p.group_size : p.tree_q_off[tree]) + blockIdx.z * GMAX;
-    const int G = min(GMAX, (by_group ? (tree + 1) * p.group_size : p.tree_q_off[tree + 1]) - hoff);
+    const bool by_group = VEC_ARG(group_size) > 0;
+    const int hoff = (by_group ? tree * VEC_ARG(group_size) : p.tree_q_off[tree]) + blockIdx.z * GMAX;
+    const int G = min(GMAX, (by_group ? (tree + 1) * VEC_ARG(group_size) : p.tree_q_off[tree + 1]) - hoff);
     if (G <= 0) return;  // uniform for the workgroup
-    int wgs = gridDim.x, wg = blockIdx.x;  // searching workgroups of the tree, my number among them
+    int wgs = ONE ? va.wgs : (int)gridDim.x, wg = blockIdx.x;  // searching workgroups of the tree, my number among them
     if constexpr (SAMPLED) {
         wgs -= p.sample_wgs;
         wg -= p.sample_wgs;
@@ -364,11 +406,11 @@ void search_kernel(const SearchParams p) {
     const unsigned gmask = (1u << G) - 1u;
     auto head_of = [&](int g) { return by_group ? hoff + g : p.tree_q_heads[hoff + g]; };
 
-    const bool is_queue = wg >= p.tree_blocks;
-    const int blk = is_queue ? wg - p.tree_blocks : wg;
-    const int n_nodes = is_queue ? p.num_queue_blocks : p.num_nodes;
+    const bool is_queue = wg >= VEC_ARG(tree_blocks);
+    const int blk = is_queue ? wg - VEC_ARG(tree_blocks) : wg;
+    const int n_nodes = is_queue ? VEC_ARG(num_queue_blocks) : VEC_ARG(num_nodes);
     const bool real_nodes = !is_queue && L >= 2;
-    const int wg_nodes = is_queue ? p.queue_nodes : p.nodes_per_wg;
+    const int wg_nodes = is_queue ? VEC_ARG(queue_nodes) : VEC_ARG(nodes_per_wg);
     const int node_first = blk * wg_nodes;
     const int node_last = min(node_first + wg_nodes, n_nodes);
 
@@ -404,23 +446,23 @@ void search_kernel(const SearchParams p) {
     float tau[GMAX], my_tau[KEPT], my_sc[KEPT];
 #pragma unroll
     for (int g = 0; g < GMAX; ++g) {
-        qraw[g] = load_chunk<T>(p.q, (size_t)hd[g] * D, chunk_ok ? ch : 0);
-        tau[g] = SAMPLED ? 0.0f : p.tau[hd[g]];
+        qraw[g] = load_chunk<T>(VEC_ARG(q), (size_t)hd[g] * D, chunk_ok ? ch : 0);
+        tau[g] = SAMPLED ? 0.0f : VEC_ARG(tau)[hd[g]];
     }
 #pragma unroll
     for (int i = 0; i < KEPT; ++i) {
-        my_tau[i] = SAMPLED ? 0.0f : p.tau[my_h[i]];
-        my_sc[i] = p.scaling[my_h[i]];
+        my_tau[i] = SAMPLED ? 0.0f : VEC_ARG(tau)[my_h[i]];
+        my_sc[i] = VEC_ARG(scaling)[my_h[i]];
     }
 
-    const void* kbase = is_queue ? p.queue_keys : p.keys;
+    const void* kbase = is_queue ? VEC_ARG(queue_keys) : VEC_ARG(keys);
     const void* vbase = is_queue ? p.queue_values : p.values;
-    const size_t krow0 = (size_t)tree * (is_queue ? p.queue_cap : p.cap[0]);
-    const int n_rows = is_queue ? p.queue_len : p.size[0];
-    const int block_rows = real_nodes ? p.bf : kPseudoBlock;
+    const size_t krow0 = (size_t)tree * (is_queue ? VEC_ARG(queue_cap) : VEC_ARG(cap[0]));
+    const int n_rows = is_queue ? VEC_ARG(queue_len) : VEC_ARG(size[0]);
+    const int block_rows = real_nodes ? VEC_ARG(bf) : kPseudoBlock;
     const float inv_rows = 1.0f / (float)block_rows;
-    const int klayout = is_queue ? HIRA_ROW_MAJOR : p.key_layout;
-    auto over_bf = [&](unsigned n) { return p.bf == 1 ? n : __umulhi(n, p.bf_magic); };  // n / bf
+    const int klayout = is_queue ? HIRA_ROW_MAJOR : VEC_ARG(key_layout);
+    auto over_bf = [&](unsigned n) { return VEC_ARG(bf) == 1 ? n : __umulhi(n, VEC_ARG(bf_magic)); };  // n / bf
 
     // counters, straight to memory (registers are worth more here than the few calls that count)
     auto count = [&](int i, unsigned n) {
@@ -661,7 +703,8 @@ void search_kernel(const SearchParams p) {
         // is not there is the last one again, a level that is not there level 1
         constexpr int KA = kOneGateRows;
         const int r0 = wave * RPW + rg, rstep = nwaves * RPW;
-        const int l2 = L > 2 ? 2 : 1, l3w = 2 + (wave == 0 ? nwaves : wave), l3 = l3w < L ? l3w : 1;
+        const int l3w = 2 + (wave == 0 ? nwaves : wave), l3 = l3w < L ? l3w : 1;
+        const int at2 = L > 2 ? 1 : 0, at3 = l3w < L ? 2 : 0;  // theirs of va
         int first2 = 0, rows2 = 0, first3 = 0, rows3 = 0, cnt = 0;
         uint4 raw1[KA], raw2 = none, raw3 = none, kraw[KU];
         float rad1[KA], rad2 = 0.0f, rad3 = 0.0f;
@@ -678,20 +721,22 @@ void search_kernel(const SearchParams p) {
                 last3 = (int)over_bf((unsigned)last3);
             }
             rows3 = l3w < L ? last3 - first3 + 1 : 0;
-            const size_t t1 = (size_t)tree * p.cap[1], t2 = (size_t)tree * p.cap[l2], t3 = (size_t)tree * p.cap[l3];
+            const size_t t1 = (size_t)tree * va.level_cap[0], t2 = (size_t)tree * va.level_cap[at2], t3 = (size_t)tree * va.level_cap[at3];
+            const float *radii1 = va.radii[0], *radii2 = va.radii[at2],
+                        *radii3 = va.radii[at3];
 #pragma unroll
             for (int k = 0; k < KA; ++k) {
                 const int row = n0 + min(r0 + k * rstep, nb - 1);
-                raw1[k] = row_at(p.centers[1], p.layout, t1, row);
-                rad1[k] = p.radii[1][t1 + row];
+                raw1[k] = row_at(va.centers[0], va.layout, t1, row);
+                rad1[k] = radii1[t1 + row];
             }
             const int row2 = rows2 > 0 ? first2 + min(r0, rows2 - 1) : 0;
-            raw2 = row_at(p.centers[l2], p.layout, t2, row2);
-            rad2 = p.radii[l2][t2 + row2];
+            raw2 = row_at(va.centers[at2], va.layout, t2, row2);
+            rad2 = radii2[t2 + row2];
             const int row3 = rows3 > 0 ? first3 + min(rg, rows3 - 1) : 0;
-            raw3 = row_at(p.centers[l3], p.layout, t3, row3);
-            rad3 = p.radii[l3][t3 + row3];
-            cnt = p.counts[1][t1 + n0 + min(lane, nb - 1)];
+            raw3 = row_at(va.centers[at3], va.layout, t3, row3);
+            rad3 = radii3[t3 + row3];
+            cnt = va.counts[t1 + n0 + min(lane, nb - 1)];
         }
 #pragma unroll
         for (int u = 0; u < KU; ++u) kraw[u] = row_at(kbase, klayout, krow0, min(slot0 + u * RPW, n_rows - 1));
@@ -1035,5 +1080,7 @@ inline int dispatch_lpr(const SearchPlan& plan, const SearchParams& p, dim3 grid
     }
     return HIRA_OK;
 }
+
+#undef VEC_ARG
 
 }  // namespace hira
