@@ -29,6 +29,8 @@
 //          in flight, each row once however many heads selected it:
 //          acc[head][:] += weight(row, head) * v[:] with the accumulators in registers
 //          (lane owns Dv/64 columns of every head).
+//          (Over an 8-bit shadow, scan and gather are two phases of the workgroup: first all tiles, the rows that
+//          the shadow cannot rule out listed; then those rows, dealt out evenly over the waves.)
 //   merge  the waves agree on one maximum per head, rescale their sums to it and add them up
 //          through LDS.
 // Keys queued since the tree was last updated (row-major, attended by every head) get one
@@ -921,11 +923,11 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         if constexpr (Q8) {
             // ---- 8-bit shadow: first all tiles, then all rows.  A wave goes through its nodes and lists the rows that
             // the shadow cannot rule out, with the heads they passed for: a word a row.  Behind a barrier the rows of all
-            // waves are dealt out evenly, kVBatch of a wave at a time: their values and keys asked for together, the exact
+            // waves are dealt out evenly, kQ8Batch of a wave at a time: their values and keys asked for together, the exact
             // test, the running maximum raised to the batch's best scores, the values into the sums.  (Rows looked at
             // round by round, a batch of 32 places for the twelve that a round of four nodes lists on average, cost every
             // round a trip to memory, and a wave with many rows kept its workgroup: a step of 8 trees x 131072 keys x 8 heads
-            // 62 us, of which the scan's bytes need 25.)
+            // 63.6 us instead of 56.3.  What bounds it now is the rows phase, a burst of 51 MB of scattered rows.)
             constexpr int CAP = S::CAP;
             uint32_t* const lists = s_words;                                                   // (waves, CAP)
             float* const ztab = reinterpret_cast<float*>(s_words + kMfmaWaves * CAP) + wave * (kQ8Batch * GS);

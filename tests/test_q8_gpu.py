@@ -118,6 +118,33 @@ def test_shadow_scan_selects_what_the_bf16_scan_selects(case, gpu_device):
     assert rel_err(full, ref_full) <= 2e-3
 
 
+@pytest.mark.parametrize("group,n,d,bf", [(1, 4500, 128, 32), (4, 4400, 128, 48), (8, 4200, 128, 64), (16, 2100, 64, 16)])
+def test_rows_of_the_shadow_scan_are_dealt_out_whole(group, n, d, bf, gpu_device):
+    """Lists of the rows that the shadow lets pass at the edges of their batches of sixteen and of a wave's list, in
+    workgroups of one to eight waves and of one to sixteen tiles: the same rows, scores and attention as over the bf16 keys."""
+    from hira_amd.searcher.hip import HIPSearcher
+
+    kw = dict(seed=900 + n, keep=16, niter=1)
+    c = _setup(1, group, n, d, bf, 2, torch.bfloat16, layout="q8", **kw)
+    t = _setup(1, group, n, d, bf, 2, torch.bfloat16, layout="tiled", **kw)
+    q = torch.from_numpy(c["q"])
+    sc = torch.full((group,), d ** -0.5)
+    s = np.where(c["valid"], c["s"], np.float32(-1e30)).astype(np.float32)
+    # sums of at most n weighted values in another order, the weights some units of the last place off
+    tol = (n + 64) * 2.0 ** -23 * float(np.abs(c["vslot"]).max())
+    for keep in (1, 15, 16, 17, 33, n):
+        th = torch.full((group,), -3e38) if keep == n else torch.from_numpy(midpoint_threshold(s, keep))
+        for threads, tiles in ((512, 1), (512, 16), (192, 16), (64, 16)):
+            print(f"keep {keep} threads {threads} tiles {tiles}", flush=True)
+            se = HIPSearcher(kernel=2, block_threads=threads, nodes_per_wave=tiles)
+            out, out_t = (se.search(q, th, x["idx"], scaling=sc).cpu().numpy() for x in (c, t))
+            np.testing.assert_array_equal(out, out_t)
+            if keep < n:
+                assert ((out != 0).sum(axis=1) == keep).all()
+            att, att_t = (se.search_attention(q, th, x["idx"], scaling=sc).cpu().numpy() for x in (c, t))
+            assert np.abs(att - att_t).max() <= tol
+
+
 def _massive(h_kv, n, d, seed):
     """Keys with per-channel scales, an offset and 8 channels blown up twentyfold (the
     benchmark's headline keys), and queries that are noisy copies of keys."""
