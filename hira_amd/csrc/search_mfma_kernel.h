@@ -927,7 +927,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
             // test, the running maximum raised to the batch's best scores, the values into the sums.  (Rows looked at
             // round by round, a batch of 32 places for the twelve that a round of four nodes lists on average, cost every
             // round a trip to memory, and a wave with many rows kept its workgroup: a step of 8 trees x 131072 keys x 8 heads
-            // 63.6 us instead of 56.3.  What bounds it now is the rows phase, a burst of 51 MB of scattered rows.)
+            // 63.6 us instead of 56.7.  What bounds it now is the rows phase, a burst of 51 MB of scattered rows.)
             constexpr int CAP = S::CAP;
             uint32_t* const lists = s_words;                                                   // (waves, CAP)
             float* const ztab = reinterpret_cast<float*>(s_words + kMfmaWaves * CAP) + wave * (kQ8Batch * GS);
@@ -1062,13 +1062,22 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     const float m_lane = raise_max(zmax);
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     // scores -> weights, in place, 64 (row, head) pairs at a time (past the end: -inf, nothing)
+                    uint64_t taken[kQ8Batch / RP];  // pairs of a row and a head that selects it
 #pragma unroll
                     for (int ps = 0; ps < kQ8Batch / RP; ++ps) {
                         float* zp = ztab + ps * 64 + lane;
-                        const float w = __builtin_amdgcn_exp2f(*zp - m_lane);
+                        const float z = *zp, w = __builtin_amdgcn_exp2f(z - m_lane);
+                        taken[ps] = __ballot(z != -INFINITY);
                         l_mine += w;
                         *zp = w;
                     }
+                    // The values of a row that no head selects may be anything: zeros in their place.  (They came with the
+                    // rest: the shadow lets few rows pass in vain.)  Is row i0 + more one that some head selects?  (The
+                    // pairs of both lie in the same 32.)
+                    auto some = [&](int i0, int more) {
+                        const uint32_t w = (uint32_t)(taken[i0 / RP] >> (i0 % RP * GS / 32 * 32));
+                        return ((w >> (i0 % RP * GS % 32 + more * GS)) & ((1u << GS) - 1u)) != 0u;
+                    };
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     if constexpr (WIDE) {
 #pragma unroll
@@ -1084,7 +1093,8 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                                 wv[4 * g4 + 3] = w.w;
                             }
                             float vf[8];
-                            unpack<bf16_t>(o.vr[i], vf);
+                            static_assert(RPI * GS <= 32, "");
+                            unpack<bf16_t>(some(i * RPI, rg) ? o.vr[i] : make_uint4(0, 0, 0, 0), vf);
 #pragma unroll
                             for (int g = 0; g < GS; ++g)
 #pragma unroll
@@ -1095,8 +1105,9 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                         for (int i = 0; i < kQ8Batch; ++i) {
                             if ((i & 7) == 0 && e0 + i >= q1) break;  // uniform
                             float vf[VPL];
-                            vf[0] = bf16_lo(o.vraw[i][0]);
-                            if (VPL > 1) vf[VPL - 1] = bf16_hi(o.vraw[i][0]);
+                            const uint32_t v = some(i, 0) ? o.vraw[i][0] : 0u;
+                            vf[0] = bf16_lo(v);
+                            if (VPL > 1) vf[VPL - 1] = bf16_hi(v);
                             const float* wr = ztab + i * GS;  // (a broadcast read)
 #pragma unroll
                             for (int g = 0; g < GS; ++g)

@@ -145,6 +145,22 @@ def test_rows_of_the_shadow_scan_are_dealt_out_whole(group, n, d, bf, gpu_device
             assert np.abs(att - att_t).max() <= tol
 
 
+@pytest.mark.parametrize("group,d", [(1, 128), (8, 128), (16, 64)])
+def test_values_that_no_head_selected_count_for_nothing(group, d, gpu_device):
+    """Rows that the shadow lets pass and no head selects: their values may be anything."""
+    from hira_amd.searcher.hip import HIPSearcher
+
+    n, bf = 3000, 32
+    c = _setup(1, group, n, d, bf, 2, torch.bfloat16, layout="q8", seed=77, keep=40, niter=1)
+    q, th = torch.from_numpy(c["q"]), torch.from_numpy(c["th"])
+    sc = torch.full((group,), d ** -0.5)
+    se = HIPSearcher(kernel=2)
+    att = se.search_attention(q, th, c["idx"], scaling=sc)
+    taken = torch.from_numpy(((c["s"] >= c["th"][:, None]) & c["valid"]).any(axis=0))
+    c["idx"].values_buf[0, : len(taken)][~taken.cuda()] = float("inf")
+    assert torch.equal(se.search_attention(q, th, c["idx"], scaling=sc), att)
+
+
 def _massive(h_kv, n, d, seed):
     """Keys with per-channel scales, an offset and 8 channels blown up twentyfold (the
     benchmark's headline keys), and queries that are noisy copies of keys."""
