@@ -923,11 +923,11 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         if constexpr (Q8) {
             // ---- 8-bit shadow: first all tiles, then all rows.  A wave goes through its nodes and lists the rows that
             // the shadow cannot rule out, with the heads they passed for: a word a row.  Behind a barrier the rows of all
-            // waves are dealt out evenly, kQ8Batch of a wave at a time: their values and keys asked for together, the exact
+            // waves (but the first few of each) are dealt out evenly, kQ8Batch of a wave at a time: their values and keys asked for together, the exact
             // test, the running maximum raised to the batch's best scores, the values into the sums.  (Rows looked at
             // round by round, a batch of 32 places for the twelve that a round of four nodes lists on average, cost every
             // round a trip to memory, and a wave with many rows kept its workgroup: a step of 8 trees x 131072 keys x 8 heads
-            // 63.6 us instead of 56.7.  What bounds it now is the rows phase, a burst of 51 MB of scattered rows.)
+            // 63.6 us instead of 56.  What bounds it now is the rows phase, a burst of 51 MB of scattered rows.)
             constexpr int CAP = S::CAP;
             uint32_t* const lists = s_words;                                                   // (waves, CAP)
             float* const ztab = reinterpret_cast<float*>(s_words + kMfmaWaves * CAP) + wave * (kQ8Batch * GS);
@@ -977,22 +977,6 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                         }
                     }
                 }
-                if (lane == 0) s_rows[wave] = nl;
-                if (c0 == 0) {
-                    tline.stamp_wave(kTlWaveScanned);
-                    tline.stamp(kTlListed);
-                    tline.set(kTlRows, (unsigned long long)nl);
-                    tline.set(kTlRounds, (unsigned long long)rounds);
-                }
-                tline.add_rows(nl);
-                __syncthreads();
-                int ahead[kMfmaWaves + 1];  // rows on the lists of the waves ahead
-                ahead[0] = 0;
-#pragma unroll
-                for (int w = 0; w < kMfmaWaves; ++w) ahead[w + 1] = ahead[w] + (w < nw ? s_rows[w] : 0);
-                const int total = __builtin_amdgcn_readfirstlane(ahead[kMfmaWaves]);
-                const int q0 = total * wave / nw, q1 = total * (wave + 1) / nw;  // my rows
-                if (stats && lane == 0 && wave == 0) stat_add(stats, HIRA_MAX_LEVELS + 2, (unsigned)total);
                 // sixteen rows at a time, the next sixteen on their way meanwhile: what LDS says about them and their loads
                 constexpr int NLD = WIDE ? kQ8Batch / RPI : 1;
                 struct Batch {
@@ -1000,18 +984,13 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     uint4 vr[NLD];  // WIDE: values, lane (row group, chunk)
                     uint32_t vraw[WIDE ? 1 : kQ8Batch][VW];
                 };
-                auto ask = [&](int e0, int half, Batch& o) {
+                // row `lane` of a batch: what its list says (0: it is not there)
+                auto ask = [&](uint32_t word, int half, Batch& o) {
                     uint32_t* const row_at = b_row + half * kQ8Batch;
                     if (lane < kQ8Batch) {
-                        const int q = max(min(e0 + lane, q1 - 1), 0);
-                        int at = q;  // (of wave w's list, behind those ahead)
-#pragma unroll
-                        for (int w = 1; w < kMfmaWaves; ++w) at = q >= ahead[w] ? w * CAP + q - ahead[w] : at;
-                        const uint32_t word = lists[at];
-                        const bool there = e0 + lane < q1;
-                        b_word[half * kQ8Batch + lane] = there ? word : 0u;
+                        b_word[half * kQ8Batch + lane] = word;
                         // (past the end: beyond the buffer, zeros and no memory access)
-                        row_at[lane] = there ? ((uint32_t)(node_of((int)(word & 0xffu)) * bf) + ((word >> 8) & 0x3fu)) * (uint32_t)(D * 2) : 0xfffff000u;
+                        row_at[lane] = word != 0u ? ((uint32_t)(node_of((int)(word & 0xffu)) * bf) + ((word >> 8) & 0x3fu)) * (uint32_t)(D * 2) : 0xfffff000u;
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     if (want_attn) {
@@ -1036,8 +1015,42 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                                                                 krsrc, row_at[col] + (unsigned)(kb * 16 + s * 64), 0, 0));
                     __builtin_amdgcn_sched_barrier(0);
                 };
-                auto use = [&](int e0, int half, const Batch& o) {
-                    if (e0 >= q1) return;  // uniform
+                // The first sixteen of a list are its wave's, asked for ahead of the barrier; what is left of the lists
+                // is dealt out behind it.  (8 trees x 131072 keys x 8 heads 57.2 -> 56.0 us; 32 of them: 56.2.)
+                Batch even, odd;
+                const int own = min(nl, kQ8Batch);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                ask(lane < own ? lists[wave * CAP + lane] : 0u, 0, even);
+                if (lane == 0) s_rows[wave] = nl;
+                if (c0 == 0) {
+                    tline.stamp_wave(kTlWaveScanned);
+                    tline.stamp(kTlListed);
+                    tline.set(kTlRows, (unsigned long long)nl);
+                    tline.set(kTlRounds, (unsigned long long)rounds);
+                }
+                tline.add_rows(nl);
+                __syncthreads();
+                int ahead[kMfmaWaves + 1];  // rows left on the lists of the waves ahead
+                ahead[0] = 0;
+                int total = 0;
+#pragma unroll
+                for (int w = 0; w < kMfmaWaves; ++w) {
+                    const int listed = w < nw ? s_rows[w] : 0;
+                    ahead[w + 1] = ahead[w] + max(listed - kQ8Batch, 0);
+                    total += listed;
+                }
+                const int left = __builtin_amdgcn_readfirstlane(ahead[kMfmaWaves]);
+                const int q0 = left * wave / nw, q1 = left * (wave + 1) / nw;  // my rows of them
+                if (stats && lane == 0 && wave == 0) stat_add(stats, HIRA_MAX_LEVELS + 2, (unsigned)total);
+                auto dealt = [&](int e0) {  // word of row e0 + lane of mine
+                    const int q = max(min(e0 + lane, q1 - 1), 0);
+                    int at = q + kQ8Batch;  // (of wave w's list, behind those ahead)
+#pragma unroll
+                    for (int w = 1; w < kMfmaWaves; ++w) at = q >= ahead[w] ? w * CAP + kQ8Batch + q - ahead[w] : at;
+                    return lane < kQ8Batch && e0 + lane < q1 ? lists[at] : 0u;
+                };
+                auto use = [&](int there, int half, const Batch& o) {  // so many rows of it
+                    if (there <= 0) return;  // uniform
                     const f32x4_t sco = tile_scores_lds<KS>(o.kr, s_bq, lane);
                     const uint4 w4 = *reinterpret_cast<const uint4*>(b_word + half * kQ8Batch + 4 * kb);
                     const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
@@ -1082,7 +1095,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     if constexpr (WIDE) {
 #pragma unroll
                         for (int i = 0; i < NLD; ++i) {
-                            if (e0 + i * RPI >= q1) break;  // uniform
+                            if (i * RPI >= there) break;  // uniform
                             float wv[GS];
 #pragma unroll
                             for (int g4 = 0; g4 < GS / 4; ++g4) {
@@ -1103,7 +1116,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     } else {
 #pragma unroll
                         for (int i = 0; i < kQ8Batch; ++i) {
-                            if ((i & 7) == 0 && e0 + i >= q1) break;  // uniform
+                            if ((i & 7) == 0 && i >= there) break;  // uniform
                             float vf[VPL];
                             const uint32_t v = some(i, 0) ? o.vraw[i][0] : 0u;
                             vf[0] = bf16_lo(v);
@@ -1117,15 +1130,13 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the next sixteen write where these read)
                 };
-                Batch even, odd;
-                ask(q0, 0, even);
-                for (int e0 = q0; e0 < q1; e0 += 2 * kQ8Batch) {  // uniform in the wave
-                    ask(e0 + kQ8Batch, 1, odd);
-                    use(e0, 0, even);
-                    if (c0 == 0 && e0 == q0) tline.stamp_wave(kTlWaveIssued);
-                    ask(e0 + 2 * kQ8Batch, 0, even);
-                    use(e0 + kQ8Batch, 1, odd);
-                    if (c0 == 0 && e0 == q0) tline.stamp_wave(kTlWaveConsumed);
+                for (int e0 = q0 - kQ8Batch; e0 < q1; e0 += 2 * kQ8Batch) {  // uniform in the wave
+                    ask(dealt(e0 + kQ8Batch), 1, odd);
+                    use(e0 < q0 ? own : q1 - e0, 0, even);
+                    if (c0 == 0 && e0 < q0) tline.stamp_wave(kTlWaveIssued);
+                    ask(dealt(e0 + 2 * kQ8Batch), 0, even);
+                    use(q1 - e0 - kQ8Batch, 1, odd);
+                    if (c0 == 0 && e0 < q0) tline.stamp_wave(kTlWaveConsumed);
                 }
                 if (c0 == 0) tline.stamp(kTlGathered);
             }
