@@ -18,13 +18,13 @@ bool mfma_search_supported(const HiraTree* t, const HiraQueue* queue) {
 // grid: x = tree, y = tile of 16 level-1 nodes, z = pass of 16 heads
 int launch_search_mfma(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s) {
     const bool q8 = p.keys8 != nullptr;  // the scan reads the keys' 8-bit shadow
-    const int pol = q8 ? 0 : plan.key_policy;  // cache policy of the bf16 tiles and the value rows
+    const int pol = plan.key_policy;  // cache policy of the scanned tiles and the value rows
     typedef void (*Launch)(const SearchPlan&, const SearchParams&, dim3, hipStream_t);
-    static const Launch table[3][4] = {
-        {launch_mfma_d64, launch_mfma_nt1_d64, launch_mfma_nt2_d64, launch_mfma_q8_d64},
-        {launch_mfma_d128, launch_mfma_nt1_d128, launch_mfma_nt2_d128, launch_mfma_q8_d128},
-        {launch_mfma_d256, launch_mfma_nt1_d256, launch_mfma_nt2_d256, nullptr}};
-    const int col = q8 ? 3 : pol;
+    static const Launch table[3][5] = {
+        {launch_mfma_d64, launch_mfma_nt1_d64, launch_mfma_nt2_d64, launch_mfma_q8_d64, launch_mfma_q8_nt1_d64},
+        {launch_mfma_d128, launch_mfma_nt1_d128, launch_mfma_nt2_d128, launch_mfma_q8_d128, launch_mfma_q8_nt1_d128},
+        {launch_mfma_d256, launch_mfma_nt1_d256, launch_mfma_nt2_d256, nullptr, nullptr}};
+    const int col = q8 ? 3 + pol : pol;
     // (no shadow scan for rows of 256 columns: its kernels did not fit the register file)
     if (q8 && p.dim == 256) return fail(HIRA_EINVAL, "MFMA kernel: 8-bit shadow with dim 256");
     switch (p.dim) {

@@ -117,8 +117,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, si
 // 22.2 / 22.2 us; and 15 % MORE than POL 0 where a caller searches the same 23 MB of keys again
 // and again, which the L2s would have kept.  The host picks by the size of the launch's keys; a
 // branch around the loads instead of instantiations costs the small launches a microsecond.  The
-// coherence bits of the policy (sc0, sc1) change nothing.  The tiles of the 8-bit shadow keep the
-// default policy: non-temporal they lose more than they gain.
+// coherence bits of the policy (sc0, sc1) change nothing.
+// 8-bit shadow: POL 0 or 1 (its tiles).  Decode steps over 1 / 2 / 6 indexes in turn, POL 0 and POL 1: 128 MiB of shadow in the
+// launch (8 heads a tree) 44.7 / 54.8 / 56.3 us and 48.9 / 49.1 / 52.8, 256 MiB 66.7 / 71.5 / - and 62.0 / 62.2 / -, 64 MiB 29.2 / 29.4 /
+// 36.4 and 31.0 / 31.5 / 32.6, 32 MiB 19.8 / 19.8 / 20.2 and 18.8 / 19.8 / 20.4: what the cache behind the L2s could hold of
+// one index or two is lost, what it holds of several gained -- the rows, which are read behind their tiles.  Those rows
+// non-temporal too gain nothing (128 MiB 49.5 / 50.9 / 52.4).
 constexpr int kReadOnce = 2;   // the `nt` bit of a buffer load's cache policy
 
 template <int KS, bool ONCE>
@@ -799,7 +803,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                         // every load is issued, whatever the node (straight-line code, so that the
                         // waits further down can count the loads behind them); a tile that is not
                         // there is asked for beyond the end of the buffer: zeros, no memory access
-                        load_tile_buf<KA, false>(k8rsrc, (unsigned)lane * 16u + (tt * 16 < nx_cnt[u] ? 0u : 0x80000000u),
+                        load_tile_buf<KA, POL != 0>(k8rsrc, (unsigned)lane * 16u + (tt * 16 < nx_cnt[u] ? 0u : 0x80000000u),
                                           (tile_first + tt) * (unsigned)(KA * 1024), a[u][tt]);
                     } else {
                         // (every load is issued, a tile that is not there beyond the end of the
@@ -1759,8 +1763,8 @@ void launch_mfma_mt(const SearchPlan& plan, const SearchParams& p, dim3 grid, hi
         launch_mfma_gs<KS, 4, Q8, POL>(plan, p, grid, s);
 }
 
-// one translation unit per key width and per kind of scan (bf16 tiles under each cache policy,
-// 8-bit shadow) keeps the build parallel
+// one translation unit per key width and per kind of scan (bf16 tiles and 8-bit shadow, under each
+// cache policy) keeps the build parallel
 void launch_mfma_d64(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
 void launch_mfma_d128(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
 void launch_mfma_d256(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
@@ -1772,5 +1776,7 @@ void launch_mfma_nt1_d256(const SearchPlan& plan, const SearchParams& p, dim3 gr
 void launch_mfma_nt2_d256(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
 void launch_mfma_q8_d64(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
 void launch_mfma_q8_d128(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
+void launch_mfma_q8_nt1_d64(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
+void launch_mfma_q8_nt1_d128(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
 
 }  // namespace hira

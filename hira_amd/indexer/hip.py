@@ -101,7 +101,7 @@ def level_sizes(n: int, bf: int, num_levels: int) -> List[int]:
 
 # layout="auto" adds the 8-bit shadow of the keys where the search gains most from it: long scans
 # shared by many heads (131072 keys a tree and 8 query heads per KV head: a decode step of 64
-# heads takes 47.0 us against 64.5); shorter trees or fewer heads a tree gain little (32768 keys
+# heads takes 51.3 us against 64.5); shorter trees or fewer heads a tree gain little (32768 keys
 # and 4 heads 16.3 against 17.2) or lose (8192 keys 14.0 against 10.9), and the shadow makes
 # builds and appends longer
 Q8_AUTO_MIN_KEYS = 131072

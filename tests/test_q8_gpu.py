@@ -161,6 +161,32 @@ def test_values_that_no_head_selected_count_for_nothing(group, d, gpu_device):
     assert torch.equal(se.search_attention(q, th, c["idx"], scaling=sc), att)
 
 
+@pytest.mark.parametrize("h_kv,n,d", [(8, 65536, 128), (8, 65568, 128), (16, 65568, 64)])
+def test_shadow_scan_on_both_sides_of_its_cache_policy(h_kv, n, d, gpu_device):
+    """64 MiB of shadow in the launch, and more: the scan of the tiles under either policy selects what the bf16 scan does."""
+    from hira_amd.indexer.hip import HIPIndexer
+    from hira_amd.searcher.hip import HIPSearcher
+
+    group = 4
+    g = torch.Generator(device="cuda").manual_seed(n + d)
+    keys, vals = (torch.randn((1, h_kv, n, d), generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    q = torch.randn((h_kv * group, d), generator=g, device="cuda").to(torch.bfloat16).float()
+    th = torch.full((h_kv * group,), 2.5 * d ** 0.5)  # some hundred keys a head
+    sc = torch.full((h_kv * group,), d ** -0.5)
+    se = HIPSearcher(kernel=2)
+    got = []
+    for layout in ("q8", "tiled"):
+        idx = HIPIndexer(3, 1, 32, layout=layout).build(keys, vals)
+        index, _, count = se.search_compact(q, th, idx, scaling=sc, capacity=4096)
+        live = torch.arange(4096, device="cuda")[None] < count[:, None]
+        got.append((se.search_attention(q, th, idx, scaling=sc), count.clone(), torch.where(live, index, -1).sort(dim=1)[0]))
+    assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][2], got[1][2])
+    assert 0 < int(got[0][1].min()) and int(got[0][1].max()) < 4096
+    # sums of a few thousand weighted values at most, in another order
+    tol = float(got[0][1].max() + 64) * 2.0 ** -23 * float(vals.float().abs().max())
+    assert float((got[0][0] - got[1][0]).abs().max()) <= tol
+
+
 def _massive(h_kv, n, d, seed):
     """Keys with per-channel scales, an offset and 8 channels blown up twentyfold (the
     benchmark's headline keys), and queries that are noisy copies of keys."""
