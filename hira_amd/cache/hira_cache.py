@@ -115,10 +115,9 @@ class HiraCacheLayer(CacheLayerMixin):
         esize = self._queue_k.element_size()
         if dt not in (torch.float32, torch.bfloat16) or self.dim * esize % 16 or self.vdim * esize % 16:
             self._queue_type = None
-        # what a launch is told of the buffers: they are the layer's own, and stay until the next allocation
-        self._queue_at = (C.c_void_p(self._queue_k.data_ptr()), C.c_void_p(self._queue_v.data_ptr()),
-                          C.c_int32(self._queue_type or 0), C.c_int32(self.batch * self.H_kv), C.c_int32(rows))
-        self._queue_widths = C.c_int32(self.dim), C.c_int32(self.vdim)
+        # what a launch is told of the buffers beside where they lie, which is asked of the tensors each time: a
+        # layer may be copied or pickled, and its copy's rows go into the copy's buffers
+        self._queue_form = self._queue_type, self.batch * self.H_kv, rows
         self._queue_rows = rows
         self._queue_dev = self._queue_k.get_device()
         # the shapes of a token's rows (a launch takes them as they are)
@@ -142,7 +141,7 @@ class HiraCacheLayer(CacheLayerMixin):
             x.get_device() == like.get_device() and x.is_contiguous() and x.data_ptr() % 16 == 0
 
     def _enqueue(self, key_states, value_states):
-        k, n = self._queue_k, self.queued_len
+        k, v, n = self._queue_k, self._queue_v, self.queued_len
         dev, token = self._queue_dev, self._token
         if n < self._queue_rows and self._queue_type is not None and dev >= 0 and \
                 key_states.shape == token[0] and value_states.shape == token[1] and \
@@ -152,7 +151,8 @@ class HiraCacheLayer(CacheLayerMixin):
             # a token's rows: what follows, without the questions about shapes
             kp, vp = key_states.data_ptr(), value_states.data_ptr()
             if (kp | vp) % 16 == 0:
-                rc = _lib.lib().hira_enqueue(*self._queue_at, n, 1, *self._queue_widths, kp, vp, _lib.stream_of(dev))
+                rc = _lib.lib().hira_enqueue(k.data_ptr(), v.data_ptr(), *self._queue_form, n, 1, self.dim, self.vdim,
+                                             kp, vp, _lib.stream_of(dev))
                 if rc:
                     _lib.check(rc)
                 self.queued_len = n + 1
@@ -170,8 +170,8 @@ class HiraCacheLayer(CacheLayerMixin):
                 self._whole_rows(value_states, m, self.vdim, v):
             # one launch for both
             rc = _lib.lib().hira_enqueue(
-                *self._queue_at, self.queued_len, m, self.dim, self.vdim, key_states.data_ptr(),
-                value_states.data_ptr(), _lib.stream_of(self._queue_dev))
+                k.data_ptr(), v.data_ptr(), *self._queue_form, self.queued_len, m, self.dim, self.vdim,
+                key_states.data_ptr(), value_states.data_ptr(), _lib.stream_of(self._queue_dev))
             if rc:
                 _lib.check(rc)
             self.queued_len += m

@@ -1,6 +1,9 @@
 """Cache glue with recording stand-ins for indexer and searcher (the approach of the
 reference's tests/test_hira_cache.py:29-299): backend selection, prefill, queueing and
 flush at update_every, lengths, reset, layer-count derivation."""
+import copy
+import pickle
+
 import pytest
 import torch
 
@@ -100,6 +103,21 @@ def test_the_queue_is_one_buffer_allocated_once(patched):
     assert torch.equal(fk, torch.cat([t[0] for t in toks] + [many[0]], dim=-2))
     assert torch.equal(fv, torch.cat([t[1] for t in toks] + [many[1]], dim=-2))
     assert l._queue_k.shape[-2] >= 10
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("how", ["copy", "pickle"])
+def test_a_copied_layer_queues_into_buffers_of_its_own(patched, how, device):
+    l = _layer(update_every=4)
+    rows = [[torch.full((1, 2, 1, 16), float(i), device=device) for _ in range(2)] for i in range(3)]
+    l.update(torch.randn(1, 2, 10, 16, device=device), torch.randn(1, 2, 10, 16, device=device))
+    l.update(*rows[0])
+    m = copy.deepcopy(l) if how == "copy" else pickle.loads(pickle.dumps(l))
+    l.update(*rows[1])
+    m.update(*rows[2])
+    for layer, want in ((l, [0.0, 1.0]), (m, [0.0, 2.0])):
+        for q in (layer.queued_keys, layer.queued_values):
+            assert q[0, 1, :, 3].tolist() == want
 
 
 def test_mask_sizes_lengths_and_reset(patched):
