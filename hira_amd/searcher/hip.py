@@ -573,7 +573,7 @@ class DecodePlan:
             return tau
         qu = self._step(query, out, queue_keys, queue_values, queue_len)
         sm = self.sample
-        sm.rows, sm.num_rows, sm.method, sm.k, sm.tau = samples.data_ptr(), shape[1], rule, k, tau.data_ptr()
+        sm.rows, sm.num_rows, sm.method, sm.k, sm.tau = samples.data_ptr(), shape[1], rule, int(k), tau.data_ptr()
         t, q, o, l, _ = self._refs
         rc = self._search_sampled(t, q, self._sample_ref, qu, o, l, self.ws.data_ptr(), self.ws_bytes, stream)
         if rc:

@@ -316,6 +316,24 @@ def test_unsynced_stretch_guards_the_pointers():
     idx._grow([64, 16, 4])                      # nothing to do: fine
 
 
+@pytest.mark.parametrize("k", [10, 10.0, "10", np.int64(10), torch.tensor(10)])
+def test_a_plan_takes_any_number_of_best_scores(k):
+    """What int() takes, DecodePlan.run_sampled takes, as its form with an append does."""
+    from types import SimpleNamespace
+
+    from hira_amd import _lib
+    from hira_amd.searcher.hip import DecodePlan
+
+    plan, seen = DecodePlan.__new__(DecodePlan), []
+    plan.indexer = SimpleNamespace(num_trees=2, dim=16, dtype=torch.float32)
+    plan.tau_buf, plan.ws, plan.ws_bytes, plan.sample = torch.zeros(4), torch.zeros(1), 4, _lib.HiraSample()
+    plan._refs, plan._sample_ref, plan._step = (None,) * 5, None, lambda *a: None
+    plan._search_sampled = lambda *a: seen.append(plan.sample.k) or 0
+    rows, out = torch.zeros(2, 8, 16), torch.zeros(4, 16)
+    assert plan.run_sampled(torch.zeros(4, 16), rows, "sample_mean_topk", k, out, stream=0) is plan.tau_buf
+    assert seen == [10]
+
+
 def test_storage_dtype_policy():
     assert HIPIndexer.storage_dtype(torch.bfloat16) == torch.bfloat16
     assert HIPIndexer.storage_dtype(torch.float32) == torch.float32
