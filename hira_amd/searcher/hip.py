@@ -424,7 +424,7 @@ class HIPSearcher(BaseSearcher):
         first use and kept: callers that come once per decode step and layer (the attention
         function) then pay one library call per step."""
         plans = self._decode_plans
-        key = (id(indexer), num_q_heads, scaling if type(scaling) is float else float(scaling))
+        key = (id(indexer), int(num_q_heads), scaling if type(scaling) is float else float(scaling))
         plan = plans.get(key)
         if plan is None or plan.indexer is not indexer:  # (ids are reused once an index is gone)
             scale = torch.full((num_q_heads,), float(scaling), dtype=torch.float32,

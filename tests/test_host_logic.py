@@ -334,6 +334,16 @@ def test_a_plan_takes_any_number_of_best_scores(k):
     assert seen == [10]
 
 
+def test_one_plan_however_the_number_of_heads_comes():
+    from types import SimpleNamespace
+
+    se, made = HIPSearcher(), []
+    idx = _FakeIndexer(1, 2)
+    se.plan_attention = lambda *a, **k: made.append(a) or SimpleNamespace(indexer=idx)
+    plans = [se.decode_plan(idx, h, s) for h in (4, np.int64(4), torch.tensor(4), torch.tensor(4)) for s in (0.5, np.float32(0.5))]
+    assert len(made) == 1 and all(p is plans[0] for p in plans)
+
+
 def test_storage_dtype_policy():
     assert HIPIndexer.storage_dtype(torch.bfloat16) == torch.bfloat16
     assert HIPIndexer.storage_dtype(torch.float32) == torch.float32
