@@ -530,7 +530,9 @@ class DecodePlan:
         qs = self.queue
         qs.keys, qs.values, qs.len, qs.cap = queue_keys.data_ptr(), queue_values.data_ptr(), m, cap
         if m > self._ws_rows:
-            self._ws_rows = cap  # (a queue fills up row by row: once for all of them)
+            # (a queue fills up row by row: not made anew for each of them, and no more than twice what the rows
+            # in use take where they are few of the buffer's)
+            self._ws_rows = min(cap, max(2 * m, 256))
             self._follow_index()
         return self._refs[4]
 

@@ -81,3 +81,28 @@ def test_no_search_is_launched_over_host_memory():
         for scaling in (None, torch.ones(4)):
             with pytest.raises(ValueError, match="GPU"):
                 call(q, tau, a, scaling=scaling)
+
+
+def test_a_plans_workspace_goes_by_the_queued_rows_in_use():
+    """Few rows in a large buffer take no workspace for all of it; a queue that fills up has a new one made
+    a few times only."""
+    from hira_amd.searcher.hip import HIPSearcher
+
+    a = HIPIndexer.from_layout(device="cpu", layout="row_major", **_parts(torch.float32))
+
+    def plan():
+        return HIPSearcher().plan_attention(a, 8, scaling=torch.ones(8))
+
+    q, out = torch.zeros((8, 64)), torch.zeros((8, 64))
+    large, small = (torch.empty((2, 1, 64)).expand(2, cap, 64) for cap in (1 << 20, 1024))
+    few, whole, filled = plan(), plan(), plan()
+    few._step(q, out, large, large, 3)
+    whole._step(q, out, small, small, 1024)
+    assert few.ws_bytes <= whole.ws_bytes
+    made = 0
+    for m in range(1, 1025):
+        before = filled.ws_bytes
+        filled._step(q, out, small, small, m)
+        made += filled.ws_bytes != before
+        assert filled._ws_rows >= m
+    assert made <= 4 and filled.ws_bytes == whole.ws_bytes
