@@ -887,15 +887,18 @@ class HIPIndexer(BaseIndexer):
         st = self._state
         if not st.is_cuda:
             return st.numpy().max(axis=0).tolist()
-        rows = self._host_rows
-        if rows is None or rows.numel() != st.numel():
-            # (zero once: a row is there when it holds the call's ticket)
-            rows = self._host_rows = torch.zeros(st.numel(), dtype=torch.int64, pin_memory=True)
-            self._ticket = 0
-        self._ticket = self._ticket % 0x7fffffff + 1
-        most = (C.c_int32 * (_lib.HIRA_MAX_LEVELS + 2))()
-        rc = _lib.lib().hira_read_state(C.byref(self.tree_struct()), st.data_ptr(), rows.data_ptr(), self._ticket,
-                                        most, _lib.stream_of(st.get_device()))
+        # (the handle of a default stream is the same on every device and means the current one's: the rows of an
+        # index elsewhere are read with its device current, whatever the caller's is)
+        with torch.cuda.device(st.get_device()):
+            rows = self._host_rows
+            if rows is None or rows.numel() != st.numel():
+                # (zero once: a row is there when it holds the call's ticket)
+                rows = self._host_rows = torch.zeros(st.numel(), dtype=torch.int64, pin_memory=True)
+                self._ticket = 0
+            self._ticket = self._ticket % 0x7fffffff + 1
+            most = (C.c_int32 * (_lib.HIRA_MAX_LEVELS + 2))()
+            rc = _lib.lib().hira_read_state(C.byref(self.tree_struct()), st.data_ptr(), rows.data_ptr(), self._ticket,
+                                            most, _lib.stream_of(st.get_device()))
         if rc:
             self._host_rows = None  # (whatever went wrong: these are not used again)
             _lib.check(rc)

@@ -326,7 +326,8 @@ int hira_update_sample(const HiraTree* tree, const void* new_keys, const void* n
  * over.
  *   host_rows  (T, HIRA_MAX_LEVELS + 2) words of pinned host memory (hipHostMalloc) that nothing else uses meanwhile
  *   ticket     differs from that of every call before on these rows, and from what they held at first (zeros: not 0)
- * A stream under capture is refused.
+ * The device that the state lies on must be the current one, as for every call that launches.  A stream under capture is
+ * refused.
  */
 int hira_read_state(const HiraTree* tree, const int32_t* state, uint64_t* host_rows, uint32_t ticket, int32_t* most,
                     void* stream);

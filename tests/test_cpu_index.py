@@ -106,3 +106,32 @@ def test_a_plans_workspace_goes_by_the_queued_rows_in_use():
         made += filled.ws_bytes != before
         assert filled._ws_rows >= m
     assert made <= 4 and filled.ws_bytes == whole.ws_bytes
+
+
+def test_sizes_are_read_back_with_the_indexs_device_current(monkeypatch):
+    """sync_sizes() and save() take an index on any device, whichever is current."""
+    import contextlib
+    from types import SimpleNamespace
+
+    a = HIPIndexer.from_layout(device="cpu", layout="row_major", **_parts(torch.float32))
+    n = 2 * (_lib.HIRA_MAX_LEVELS + 2)
+    a._state = SimpleNamespace(is_cuda=True, get_device=lambda: 1, data_ptr=lambda: 0, numel=lambda: n)
+    a._host_rows, a._pending = torch.zeros(n, dtype=torch.int64), 1
+    current = [0]
+
+    @contextlib.contextmanager
+    def device(index):
+        current.append(index)
+        yield
+        current.pop()
+
+    def read(tree, state, rows, ticket, most, stream):
+        assert current[-1] == 1 and stream == 7
+        most[1], most[2] = a.size[1], a.size[2]
+        return 0
+
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(_lib, "stream_of", lambda index: 7)
+    monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(hira_read_state=read))
+    a.sync_sizes()
+    assert a._pending == 0 and current == [0]
