@@ -222,6 +222,13 @@ class HIPIndexer(BaseIndexer):
         self._host_rows: Optional[torch.Tensor] = None  # pinned: where the state's rows are read back to
         self._ticket = 0
 
+    def __getstate__(self):
+        """What a copy or a pickle takes along: not what holds addresses of this one's arrays, nor the pinned rows,
+        whose copy would not be pinned.  All of it is made anew when it is asked for."""
+        state = dict(self.__dict__)
+        state["_tree_struct"] = state["_append"] = state["_host_rows"] = None
+        return state
+
     # ------------------------------------------------------------------ reference views
     @property
     def depth(self):

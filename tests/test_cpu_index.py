@@ -1,5 +1,8 @@
 """An index in host memory: restored, adopted, grown and saved without a GPU; what would launch a kernel
 on it is refused."""
+import copy
+import pickle
+
 import numpy as np
 import pytest
 import torch
@@ -135,3 +138,13 @@ def test_sizes_are_read_back_with_the_indexs_device_current(monkeypatch):
     monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(hira_read_state=read))
     a.sync_sizes()
     assert a._pending == 0 and current == [0]
+
+
+def test_a_copied_index_has_pointers_and_pinned_rows_of_its_own():
+    a = HIPIndexer.from_layout(device="cpu", layout="row_major", **_parts(torch.float32))
+    a._host_rows, at = torch.zeros(20, dtype=torch.int64), a.tree_struct().keys
+    for b in (copy.deepcopy(a), pickle.loads(pickle.dumps(a))):
+        assert b._host_rows is None and b._append is None
+        assert b.tree_struct().keys == b.keys_buf.data_ptr() != at
+        assert torch.equal(b.keys_rowmajor(), a.keys_rowmajor()) and b.size == a.size
+    assert a.tree_struct().keys == at and a._host_rows is not None

@@ -638,3 +638,21 @@ def test_sizes_read_back_are_the_states(heads, levels, busy):
             want = [idx.num_keys] if levels == 1 else [used[1] * 16] + used[1:levels]
             assert idx.size == want and used[-2] == idx.num_keys
     side.synchronize()
+
+
+def test_a_copied_index_grows_by_itself(gpu_device):
+    import copy
+
+    from hira_amd.indexer.hip import HIPIndexer
+
+    g = torch.Generator().manual_seed(3)
+    keys = torch.randn((1, 2, 700, 64), generator=g).to(torch.bfloat16).cuda()
+    a = HIPIndexer(3, 1, 16).build(keys[:, :, :600], keys[:, :, :600])
+    a.update(keys[:, :, 600:650], keys[:, :, 600:650])
+    b = copy.deepcopy(a)
+    for x in (b, a):  # (the copy first: it has no rows of the first one's to read back through)
+        x.update(keys[:, :, 650:], keys[:, :, 650:])
+    assert a.size == b.size and a.num_keys == b.num_keys == 700
+    n = a.size[0]
+    assert torch.equal(a.perm[:, :n], b.perm[:, :n]) and torch.equal(a.keys_buf[:, :n], b.keys_buf[:, :n])
+    assert a.keys_buf.data_ptr() != b.keys_buf.data_ptr() and (b.perm >= 0).sum() == 2 * 700
