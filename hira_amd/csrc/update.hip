@@ -1476,8 +1476,10 @@ extern "C" int hira_read_state(const HiraTree* tree, const int32_t* state, uint6
     HIRA_CHECK_ARG(tree && state && host_rows && most && tree->num_trees >= 1, "hira_read_state: null argument");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)
+    if (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();  // (refused here: not an error of the next call's)
         return fail(HIRA_ELAUNCH, "hira_read_state: a stream under capture cannot be waited for");
+    }
     void* rows = nullptr;
     if (hipHostGetDevicePointer(&rows, host_rows, 0) != hipSuccess) {
         (void)hipGetLastError();

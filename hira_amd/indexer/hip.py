@@ -889,6 +889,19 @@ class HIPIndexer(BaseIndexer):
         self._unsynced_room = 0
         return self
 
+    def _rows_to_read_into(self, n: int) -> torch.Tensor:
+        """The pinned rows of a read-back, on the current device.  What can refuse one does so here, ahead of the
+        launches that are to be read back."""
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("the level sizes of an index cannot be read back from a stream under capture: "
+                               "append with sync=False there")
+        rows = self._host_rows
+        if rows is None or rows.numel() != n:
+            # (zero once: a row is there when it holds the call's ticket)
+            rows = self._host_rows = torch.zeros(n, dtype=torch.int64, pin_memory=True)
+            self._ticket = 0
+        return rows
+
     def _largest_state(self) -> List[int]:
         """The largest entry over the trees of every column of the state, behind all that was enqueued."""
         st = self._state
@@ -897,11 +910,7 @@ class HIPIndexer(BaseIndexer):
         # (the handle of a default stream is the same on every device and means the current one's: the rows of an
         # index elsewhere are read with its device current, whatever the caller's is)
         with torch.cuda.device(st.get_device()):
-            rows = self._host_rows
-            if rows is None or rows.numel() != st.numel():
-                # (zero once: a row is there when it holds the call's ticket)
-                rows = self._host_rows = torch.zeros(st.numel(), dtype=torch.int64, pin_memory=True)
-                self._ticket = 0
+            rows = self._rows_to_read_into(st.numel())
             self._ticket = self._ticket % 0x7fffffff + 1
             most = (C.c_int32 * (_lib.HIRA_MAX_LEVELS + 2))()
             rc = _lib.lib().hira_read_state(C.byref(self.tree_struct()), st.data_ptr(), rows.data_ptr(), self._ticket,
@@ -992,6 +1001,9 @@ class HIPIndexer(BaseIndexer):
                 return self._replace_sample(sample, new_keys, m)
         if not sync and 0 < self._unsynced_room < m:  # (checked before anything is launched)
             raise RuntimeError("more appends than begin_unsynced made room for")
+        if sync and self.keys_buf.is_cuda:  # (what it cannot read back it does not launch)
+            with torch.cuda.device(self.keys_buf.get_device()):
+                self._rows_to_read_into(self.num_trees * (_lib.HIRA_MAX_LEVELS + 2))
         need = self._needed_caps(m)
         self._grow(need)
         t = self.num_trees

@@ -134,6 +134,7 @@ def test_sizes_are_read_back_with_the_indexs_device_current(monkeypatch):
         return 0
 
     monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(_lib, "stream_of", lambda index: 7)
     monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(hira_read_state=read))
     a.sync_sizes()

@@ -656,3 +656,48 @@ def test_a_copied_index_grows_by_itself(gpu_device):
     n = a.size[0]
     assert torch.equal(a.perm[:, :n], b.perm[:, :n]) and torch.equal(a.keys_buf[:, :n], b.keys_buf[:, :n])
     assert a.keys_buf.data_ptr() != b.keys_buf.data_ptr() and (b.perm >= 0).sum() == 2 * 700
+
+
+def test_what_cannot_be_read_back_changes_nothing(gpu_device):
+    """The library refuses rows that are not pinned, missing arrays and a stream under capture, and a call after
+    that is none the worse for it; an append with a read-back is refused under capture before it launches."""
+    import ctypes
+
+    from hira_amd import _lib
+    from hira_amd.indexer.hip import HIPIndexer
+
+    g = torch.Generator().manual_seed(4)
+    keys = torch.randn((1, 2, 400, 64), generator=g).to(torch.bfloat16).cuda()
+    idx = HIPIndexer(3, 1, 16).build(keys[:, :, :300], keys[:, :, :300])
+    idx.update(keys[:, :, 300:310], keys[:, :, 300:310])
+    st, n = idx._state, idx._state.numel()
+    most = (ctypes.c_int32 * (_lib.HIRA_MAX_LEVELS + 2))()
+    pinned = torch.zeros(n, dtype=torch.int64, pin_memory=True)
+    plain = (ctypes.c_uint64 * n)()
+
+    def read(state, rows, ticket, stream):
+        return _lib.lib().hira_read_state(ctypes.byref(idx.tree_struct()), state, rows, ticket, most, stream)
+
+    stream = torch.cuda.current_stream().cuda_stream
+    assert read(st.data_ptr(), ctypes.addressof(plain), 1, stream) == -1
+    assert read(None, pinned.data_ptr(), 1, stream) == -1 and read(st.data_ptr(), None, 1, stream) == -1
+    graph, new = torch.cuda.CUDAGraph(), keys[:, :, 310:320].contiguous()
+    before = (idx.num_keys, list(idx.size), list(idx.cap), idx.keys_buf.data_ptr(), st.clone())
+    torch.cuda.synchronize()
+    out = torch.zeros(4, device="cuda")
+    with torch.cuda.graph(graph):
+        out.add_(1.0)
+        assert read(st.data_ptr(), pinned.data_ptr(), 1, torch.cuda.current_stream().cuda_stream) not in (0, -1)
+        with pytest.raises(RuntimeError, match="capture"):
+            idx.update(new, new)
+    for i in (1, 2):  # (the capture is whole, and holds what was launched beside those calls)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert out.tolist() == [float(i)] * 4
+    assert before[:4] == (idx.num_keys, list(idx.size), list(idx.cap), idx.keys_buf.data_ptr())
+    assert torch.equal(before[4], idx._state)
+    assert not pinned.any()
+    assert read(st.data_ptr(), pinned.data_ptr(), 1, stream) == 0
+    assert list(most) == st.cpu().max(dim=0).values.tolist()
+    idx.update(new, new)
+    assert idx.num_keys == 320 and (idx.perm >= 0).sum() == 2 * 320
