@@ -339,6 +339,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     __shared__ float s_qc[Q8 ? 2 * kHeadsPerPass : 1];
     __shared__ float s_keps[Q8 ? kMfmaMaxTilesPerWg * 16 : 1];
     __shared__ int s_rows[Q8 ? kMfmaWaves : 1];  // rows that the waves have listed
+    __shared__ int s_places[Q8 && OUT ? kMfmaWaves * 16 : 1], s_place0[Q8 && OUT ? 16 : 1];  // of a batch on the heads' lists
 
     touch_kernel_arguments();
     const GateArgs ga = gate_arguments(p);
@@ -831,20 +832,18 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         tline.stamp(kTlFetched);
 
         // dense scores / compact lists of the selected rows among 16 scored ones: lane
-        // (kb, head) holds rows 4*kb + j, whose key slots are slot4[j]
-        auto emit = [&](int col, int kb, unsigned sel4, const f32x4_t& sco, const unsigned (&slot4)[4]) {
+        // (kb, head) holds rows 4*kb + j, whose key slots are slot4[j]; reserve: so many places on the lane's head's list
+        auto emit = [&](int col, int kb, unsigned sel4, const f32x4_t& sco, const unsigned (&slot4)[4], auto reserve) {
             unsigned long long sb[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) sb[j] = __ballot((sel4 >> j) & 1u);
             int base = 0;
-            if (p.sel_count != nullptr) {  // one atomic per head of the tile (kb = 0)
+            if (p.sel_count != nullptr) {
                 int mine = 0;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     mine += __popcll(sb[j] & (0x0001000100010001ull << col));
-                int b0 = 0;
-                if (kb == 0 && mine > 0) b0 = atomicAdd(&p.sel_count[qh], mine);
-                base = __shfl(b0, col, 64);
+                base = reserve(mine);
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -1053,8 +1052,10 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     for (int w = 1; w < kMfmaWaves; ++w) at = q >= ahead[w] ? w * CAP + kQ8Batch + q - ahead[w] : at;
                     return lane < kQ8Batch && e0 + lane < q1 ? lists[at] : 0u;
                 };
+                // (selection lists: every wave is here as often as any other)
                 auto use = [&](int there, int half, const Batch& o) {  // so many rows of it
-                    if (there <= 0) return;  // uniform
+                    const bool lists_out = OUT && p.sel_count != nullptr;  // uniform in the launch
+                    if (there <= 0 && !lists_out) return;  // uniform
                     const f32x4_t sco = tile_scores_lds<KS>(o.kr, s_bq, lane);
                     const uint4 w4 = *reinterpret_cast<const uint4*>(b_word + half * kQ8Batch + 4 * kb);
                     const uint32_t words[4] = {w4.x, w4.y, w4.z, w4.w};
@@ -1073,9 +1074,26 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     if (OUT && (p.dense != nullptr || p.sel_count != nullptr)) {
                         const uint4 r4 = *reinterpret_cast<const uint4*>(b_row + half * kQ8Batch + 4 * kb);
                         const unsigned slot4[4] = {r4.x / (D * 2), r4.y / (D * 2), r4.z / (D * 2), r4.w / (D * 2)};
-                        emit(col, kb, sel4, sco, slot4);
+                        // One atomic per head of the workgroup's batches: all waves have their rows at once, and with
+                        // one each they stood in line for the few cache lines that all heads' counters are.  (Lists,
+                        // 8 heads a tree: 8 x 32768 keys of fan-out 64, 1 % selected, 33.6 -> 21.0 us, 8 x 131072, 10 %,
+                        // 256 -> 93; round by round, before there were two phases, 26.3 and 256.)
+                        emit(col, kb, sel4, sco, slot4, [&](int mine) {
+                            if (kb == 0) s_places[wave * 16 + col] = mine;
+                            __syncthreads();
+                            int before = 0, all = 0;
+#pragma unroll
+                            for (int w = 0; w < kMfmaWaves; ++w) {
+                                const int n = w < nw ? s_places[w * 16 + col] : 0;
+                                if (w < wave) before += n;
+                                all += n;
+                            }
+                            if (wave == 0 && kb == 0) s_place0[col] = all > 0 ? atomicAdd(&p.sel_count[qh], all) : 0;
+                            __syncthreads();
+                            return s_place0[col] + before;
+                        });
                     }
-                    if (!want_attn) return;  // uniform
+                    if (!want_attn || there <= 0) return;  // uniform
                     const float m_lane = raise_max(zmax);
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                     // scores -> weights, in place, 64 (row, head) pairs at a time (past the end: -inf, nothing)
@@ -1134,7 +1152,8 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     }
                     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the next sixteen write where these read)
                 };
-                for (int e0 = q0 - kQ8Batch; e0 < q1; e0 += 2 * kQ8Batch) {  // uniform in the wave
+                const int end = q0 + (left + nw - 1) / nw;  // (as many steps in every wave)
+                for (int e0 = q0 - kQ8Batch; e0 < end; e0 += 2 * kQ8Batch) {  // uniform in the wave
                     ask(dealt(e0 + kQ8Batch), 1, odd);
                     use(e0 < q0 ? own : q1 - e0, 0, even);
                     if (c0 == 0 && e0 < q0) tline.stamp_wave(kTlWaveIssued);
@@ -1203,7 +1222,11 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                         if (OUT && (p.dense != nullptr || p.sel_count != nullptr)) {
                             const unsigned slot4[4] = {tslot + 4 * kb, tslot + 4 * kb + 1, tslot + 4 * kb + 2,
                                                        tslot + 4 * kb + 3};
-                            emit(col, kb, sel4, sco, slot4);
+                            emit(col, kb, sel4, sco, slot4, [&](int mine) {  // one atomic per head of the tile
+                                int b0 = 0;
+                                if (kb == 0 && mine > 0) b0 = atomicAdd(&p.sel_count[qh], mine);
+                                return __shfl(b0, col, 64);
+                            });
                         }
 
                         // ---- the tile's scores go to the table, its selected rows join my list -----------

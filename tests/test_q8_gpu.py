@@ -145,6 +145,51 @@ def test_rows_of_the_shadow_scan_are_dealt_out_whole(group, n, d, bf, gpu_device
             assert np.abs(att - att_t).max() <= tol
 
 
+@pytest.mark.parametrize("group,n,d,bf", [(1, 4500, 128, 32), (4, 4400, 128, 48), (8, 4200, 128, 64), (16, 2100, 64, 16),
+                                          (16, 2300, 128, 32), (9, 2200, 128, 64)])
+def test_lists_of_the_shadow_scan_are_whole(group, n, d, bf, gpu_device):
+    """Places on the heads' lists are given out once a batch of all waves: every selected key once, with its score, also
+    where waves have fewer batches than others or none, where a list is too short, and beside attention."""
+    from hira_amd.searcher.hip import HIPSearcher
+
+    c = _setup(1, group, n, d, bf, 2, torch.bfloat16, layout="q8", seed=1300 + n, keep=16, niter=1)
+    q = torch.from_numpy(c["q"])
+    qd = q.to(torch.bfloat16).cuda().reshape(group, d).contiguous()
+    sc = torch.full((group,), d ** -0.5, device="cuda")
+    ones = torch.ones(group)
+    s = np.where(c["valid"], c["s"], np.float32(-1e30)).astype(np.float32)
+    for keep in (1, 15, 17, 33, 700, n):
+        th = torch.full((group,), -3e38) if keep == n else torch.from_numpy(midpoint_threshold(s, keep))
+        for threads, tiles in ((512, 1), (512, 16), (192, 16), (64, 16)):
+            print(f"keep {keep} threads {threads} tiles {tiles}", flush=True)
+            se = HIPSearcher(kernel=2, block_threads=threads, nodes_per_wave=tiles)
+            dense = se.search(q, th, c["idx"], scaling=ones).clone()
+            want = torch.full_like(dense, float("nan"))
+            want[dense != 0] = dense[dense != 0]
+            for cap in (n, 16):
+                index, score, count = se.search_compact(q, th, c["idx"], capacity=cap)
+                assert count.tolist() == (dense != 0).sum(dim=1).tolist()
+                for h in range(group):
+                    m = min(cap, int(count[h]))
+                    at = index[h, :m].long()
+                    assert at.unique().numel() == m and torch.equal(score[h, :m], want[h, at])
+            # both in one launch
+            plan = se.plan_attention(c["idx"], group, scaling=sc)
+            out, alone = (torch.empty((group, d), device="cuda") for _ in range(2))
+            plan.run(qd, th.cuda(), alone)
+            index, score = torch.empty((group, n), dtype=torch.int32, device="cuda"), torch.empty((group, n), device="cuda")
+            count = torch.zeros((group,), dtype=torch.int32, device="cuda")
+            o = plan.out
+            o.sel_index, o.sel_score, o.sel_count, o.sel_cap = index.data_ptr(), score.data_ptr(), count.data_ptr(), n
+            plan.run(qd, th.cuda(), out)
+            # (the rows may come in another order: sums of at most n weighted values)
+            tol = (n + 64) * 2.0 ** -23 * float(np.abs(c["vslot"]).max())
+            assert float((out - alone).abs().max()) <= tol and count.tolist() == (dense != 0).sum(dim=1).tolist()
+            for h in range(group):
+                at = index[h, : int(count[h])].long()
+                assert at.unique().numel() == at.numel() and torch.equal(score[h, : at.numel()], want[h, at])
+
+
 @pytest.mark.parametrize("group,d", [(1, 128), (8, 128), (16, 64)])
 def test_values_that_no_head_selected_count_for_nothing(group, d, gpu_device):
     """Rows that the shadow lets pass and no head selects: their values may be anything."""
