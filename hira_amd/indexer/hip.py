@@ -20,6 +20,7 @@ views of the level arrays.  Differences, all deliberate:
 from __future__ import annotations
 
 import ctypes as C
+import itertools
 from enum import Enum
 from typing import List, Optional, Tuple
 
@@ -31,6 +32,8 @@ from .base import BaseIndexer
 DEFAULT_PAD_VALUE = 0.0
 
 _DTYPES = {torch.float32: _lib.HIRA_F32, torch.bfloat16: _lib.HIRA_BF16}
+
+_TICKETS = itertools.count(1)  # of read-backs (next() hands each number to one thread)
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -219,8 +222,9 @@ class HIPIndexer(BaseIndexer):
         self._tree_struct = None
         self._state: Optional[torch.Tensor] = None  # device-side bookkeeping of update()
         self._append: Optional[_Append] = None
-        self._host_rows: Optional[torch.Tensor] = None  # pinned: where the state's rows are read back to
-        self._ticket = 0
+        # pinned: where the state's rows are read back to.  A read-back takes them while it lasts, so that another
+        # thread's has rows of its own
+        self._host_rows: Optional[torch.Tensor] = None
 
     def __getstate__(self):
         """What a copy or a pickle takes along: not what holds addresses of this one's arrays, nor the pinned rows,
@@ -895,11 +899,11 @@ class HIPIndexer(BaseIndexer):
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("the level sizes of an index cannot be read back from a stream under capture: "
                                "append with sync=False there")
-        rows = self._host_rows
+        rows = self.__dict__.pop("_host_rows", None)  # (looked at and taken in one step)
+        self.__dict__.setdefault("_host_rows", None)
         if rows is None or rows.numel() != n:
             # (zero once: a row is there when it holds the call's ticket)
-            rows = self._host_rows = torch.zeros(n, dtype=torch.int64, pin_memory=True)
-            self._ticket = 0
+            rows = torch.zeros(n, dtype=torch.int64, pin_memory=True)
         return rows
 
     def _largest_state(self) -> List[int]:
@@ -911,13 +915,12 @@ class HIPIndexer(BaseIndexer):
         # index elsewhere are read with its device current, whatever the caller's is)
         with torch.cuda.device(st.get_device()):
             rows = self._rows_to_read_into(st.numel())
-            self._ticket = self._ticket % 0x7fffffff + 1
             most = (C.c_int32 * (_lib.HIRA_MAX_LEVELS + 2))()
-            rc = _lib.lib().hira_read_state(C.byref(self.tree_struct()), st.data_ptr(), rows.data_ptr(), self._ticket,
-                                            most, _lib.stream_of(st.get_device()))
+            rc = _lib.lib().hira_read_state(C.byref(self.tree_struct()), st.data_ptr(), rows.data_ptr(),
+                                            next(_TICKETS) % 0x7fffffff + 1, most, _lib.stream_of(st.get_device()))
         if rc:
-            self._host_rows = None  # (whatever went wrong: these are not used again)
-            _lib.check(rc)
+            _lib.check(rc)  # (whatever went wrong: these rows are not used again)
+        self._host_rows = rows
         return list(most)
 
     def _adopt_state(self) -> None:
@@ -1003,7 +1006,7 @@ class HIPIndexer(BaseIndexer):
             raise RuntimeError("more appends than begin_unsynced made room for")
         if sync and self.keys_buf.is_cuda:  # (what it cannot read back it does not launch)
             with torch.cuda.device(self.keys_buf.get_device()):
-                self._rows_to_read_into(self.num_trees * (_lib.HIRA_MAX_LEVELS + 2))
+                self._host_rows = self._rows_to_read_into(self.num_trees * (_lib.HIRA_MAX_LEVELS + 2))
         need = self._needed_caps(m)
         self._grow(need)
         t = self.num_trees

@@ -149,3 +149,32 @@ def test_a_copied_index_has_pointers_and_pinned_rows_of_its_own():
         assert b.tree_struct().keys == b.keys_buf.data_ptr() != at
         assert torch.equal(b.keys_rowmajor(), a.keys_rowmajor()) and b.size == a.size
     assert a.tree_struct().keys == at and a._host_rows is not None
+
+
+def test_a_read_back_has_rows_of_its_own_while_it_lasts(monkeypatch):
+    """Two threads may ask for an index's sizes at once: neither call's rows or ticket are the other's, and one set of
+    rows is kept."""
+    import contextlib
+    from types import SimpleNamespace
+
+    a = HIPIndexer.from_layout(device="cpu", layout="row_major", **_parts(torch.float32))
+    n = 2 * (_lib.HIRA_MAX_LEVELS + 2)
+    a._state = SimpleNamespace(is_cuda=True, get_device=lambda: 0, data_ptr=lambda: 0, numel=lambda: n)
+    a._host_rows, zeros, seen = torch.zeros(n, dtype=torch.int64), torch.zeros, []
+
+    def read(tree, state, rows, ticket, most, stream):
+        seen.append((rows, ticket))
+        if len(seen) == 1:  # (while the first call waits)
+            a._largest_state()
+        most[:] = range(len(most))
+        return 0
+
+    monkeypatch.setattr(torch, "zeros", lambda *args, pin_memory=False, **kw: zeros(*args, **kw))
+    monkeypatch.setattr(torch.cuda, "device", lambda index: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(_lib, "stream_of", lambda index: 0)
+    monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(hira_read_state=read))
+    assert a._largest_state() == list(range(n // 2))
+    a._largest_state()
+    assert len(seen) == 3 and len({t for _, t in seen}) == 3 and seen[0][0] != seen[1][0]
+    assert seen[2][0] == seen[0][0] == a._host_rows.data_ptr()
