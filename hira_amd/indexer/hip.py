@@ -34,6 +34,7 @@ DEFAULT_PAD_VALUE = 0.0
 _DTYPES = {torch.float32: _lib.HIRA_F32, torch.bfloat16: _lib.HIRA_BF16}
 
 _TICKETS = itertools.count(1)  # of read-backs (next() hands each number to one thread)
+_Row = C.c_int32 * (_lib.HIRA_MAX_LEVELS + 2)
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -222,9 +223,10 @@ class HIPIndexer(BaseIndexer):
         self._tree_struct = None
         self._state: Optional[torch.Tensor] = None  # device-side bookkeeping of update()
         self._append: Optional[_Append] = None
-        # pinned: where the state's rows are read back to.  A read-back takes them while it lasts, so that another
-        # thread's has rows of its own
-        self._host_rows: Optional[torch.Tensor] = None
+
+    # pinned: where the state's rows are read back to.  A read-back takes them while it lasts, so that another thread's
+    # has rows of its own
+    _host_rows: Optional[torch.Tensor] = None
 
     def __getstate__(self):
         """What a copy or a pickle takes along: not what holds addresses of this one's arrays, nor the pinned rows,
@@ -893,15 +895,17 @@ class HIPIndexer(BaseIndexer):
         self._unsynced_room = 0
         return self
 
-    def _rows_to_read_into(self, n: int) -> torch.Tensor:
-        """The pinned rows of a read-back, on the current device.  What can refuse one does so here, ahead of the
-        launches that are to be read back."""
+    @staticmethod
+    def _refuse_capture() -> None:
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("the level sizes of an index cannot be read back from a stream under capture: "
                                "append with sync=False there")
+
+    def _rows_to_read_into(self, n: int) -> torch.Tensor:
+        """The pinned rows of a read-back, on the current device."""
         rows = self.__dict__.pop("_host_rows", None)  # (looked at and taken in one step)
-        self.__dict__.setdefault("_host_rows", None)
         if rows is None or rows.numel() != n:
+            self._refuse_capture()
             # (zero once: a row is there when it holds the call's ticket)
             rows = torch.zeros(n, dtype=torch.int64, pin_memory=True)
         return rows
@@ -913,11 +917,13 @@ class HIPIndexer(BaseIndexer):
             return st.numpy().max(axis=0).tolist()
         # (the handle of a default stream is the same on every device and means the current one's: the rows of an
         # index elsewhere are read with its device current, whatever the caller's is)
-        with torch.cuda.device(st.get_device()):
-            rows = self._rows_to_read_into(st.numel())
-            most = (C.c_int32 * (_lib.HIRA_MAX_LEVELS + 2))()
-            rc = _lib.lib().hira_read_state(C.byref(self.tree_struct()), st.data_ptr(), rows.data_ptr(),
-                                            next(_TICKETS) % 0x7fffffff + 1, most, _lib.stream_of(st.get_device()))
+        dev = st.get_device()
+        if torch.cuda.current_device() != dev:
+            with torch.cuda.device(dev):
+                return self._largest_state()
+        rows, most = self._rows_to_read_into(st.numel()), _Row()
+        rc = _lib.lib().hira_read_state(C.byref(self.tree_struct()), st.data_ptr(), rows.data_ptr(),
+                                        next(_TICKETS) % 0x7fffffff + 1, most, _lib.stream_of(dev))
         if rc:
             _lib.check(rc)  # (whatever went wrong: these rows are not used again)
         self._host_rows = rows
@@ -1005,8 +1011,10 @@ class HIPIndexer(BaseIndexer):
         if not sync and 0 < self._unsynced_room < m:  # (checked before anything is launched)
             raise RuntimeError("more appends than begin_unsynced made room for")
         if sync and self.keys_buf.is_cuda:  # (what it cannot read back it does not launch)
-            with torch.cuda.device(self.keys_buf.get_device()):
-                self._host_rows = self._rows_to_read_into(self.num_trees * (_lib.HIRA_MAX_LEVELS + 2))
+            self._refuse_capture()
+            rows, n = self._host_rows, self.num_trees * (_lib.HIRA_MAX_LEVELS + 2)
+            if rows is None or rows.numel() != n:
+                self._host_rows = self._rows_to_read_into(n)
         need = self._needed_caps(m)
         self._grow(need)
         t = self.num_trees

@@ -134,6 +134,7 @@ def test_sizes_are_read_back_with_the_indexs_device_current(monkeypatch):
         return 0
 
     monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[-1])
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(_lib, "stream_of", lambda index: 7)
     monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(hira_read_state=read))
@@ -154,7 +155,6 @@ def test_a_copied_index_has_pointers_and_pinned_rows_of_its_own():
 def test_a_read_back_has_rows_of_its_own_while_it_lasts(monkeypatch):
     """Two threads may ask for an index's sizes at once: neither call's rows or ticket are the other's, and one set of
     rows is kept."""
-    import contextlib
     from types import SimpleNamespace
 
     a = HIPIndexer.from_layout(device="cpu", layout="row_major", **_parts(torch.float32))
@@ -170,7 +170,7 @@ def test_a_read_back_has_rows_of_its_own_while_it_lasts(monkeypatch):
         return 0
 
     monkeypatch.setattr(torch, "zeros", lambda *args, pin_memory=False, **kw: zeros(*args, **kw))
-    monkeypatch.setattr(torch.cuda, "device", lambda index: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(_lib, "stream_of", lambda index: 0)
     monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(hira_read_state=read))
