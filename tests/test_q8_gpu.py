@@ -50,6 +50,8 @@ Q8_CASES = [
     (2, 8, 40000, 128, 32, 4, 400),     # four levels
     (1, 8, 3000, 128, 64, 2, 40),       # fan-out 64, 8 heads
     (1, 16, 2600, 64, 64, 3, 30),       # d = 64, fan-out 64, 16 heads
+    (1, 16, 2700, 128, 32, 3, 30),      # 9 to 16 heads over rows of 128: values a word a lane
+    (1, 9, 2400, 128, 64, 2, 25),
 ]
 
 
@@ -118,7 +120,8 @@ def test_shadow_scan_selects_what_the_bf16_scan_selects(case, gpu_device):
     assert rel_err(full, ref_full) <= 2e-3
 
 
-@pytest.mark.parametrize("group,n,d,bf", [(1, 4500, 128, 32), (4, 4400, 128, 48), (8, 4200, 128, 64), (16, 2100, 64, 16)])
+@pytest.mark.parametrize("group,n,d,bf", [(1, 4500, 128, 32), (4, 4400, 128, 48), (8, 4200, 128, 64), (16, 2100, 64, 16),
+                                          (16, 4300, 128, 32), (9, 4200, 128, 64)])
 def test_rows_of_the_shadow_scan_are_dealt_out_whole(group, n, d, bf, gpu_device):
     """Lists of the rows that the shadow lets pass at the edges of their batches of sixteen and of a wave's list, in
     workgroups of one to eight waves and of one to sixteen tiles: the same rows, scores and attention as over the bf16 keys."""
@@ -190,9 +193,10 @@ def test_lists_of_the_shadow_scan_are_whole(group, n, d, bf, gpu_device):
                 assert at.unique().numel() == at.numel() and torch.equal(score[h, : at.numel()], want[h, at])
 
 
-@pytest.mark.parametrize("group,d", [(1, 128), (8, 128), (16, 64)])
+@pytest.mark.parametrize("group,d", [(1, 128), (8, 128), (16, 64), (16, 128)])
 def test_values_that_no_head_selected_count_for_nothing(group, d, gpu_device):
     """Rows that the shadow lets pass and no head selects: their values may be anything."""
+    from hira_amd import _lib
     from hira_amd.searcher.hip import HIPSearcher
 
     n, bf = 3000, 32
@@ -200,19 +204,23 @@ def test_values_that_no_head_selected_count_for_nothing(group, d, gpu_device):
     q, th = torch.from_numpy(c["q"]), torch.from_numpy(c["th"])
     sc = torch.full((group,), d ** -0.5)
     se = HIPSearcher(kernel=2)
+    st = torch.zeros((1, _lib.HIRA_STATS_COLS), dtype=torch.int64, device="cuda")
+    se.search(q, th, c["idx"], scaling=sc, stats=st)
+    looked_at, selected = int(st[0, _lib.HIRA_MAX_LEVELS + 2]), int(st[0, _lib.HIRA_MAX_LEVELS])
+    assert looked_at > selected  # rows that passed in vain: theirs are the values in question
     att = se.search_attention(q, th, c["idx"], scaling=sc)
     taken = torch.from_numpy(((c["s"] >= c["th"][:, None]) & c["valid"]).any(axis=0))
     c["idx"].values_buf[0, : len(taken)][~taken.cuda()] = float("inf")
     assert torch.equal(se.search_attention(q, th, c["idx"], scaling=sc), att)
 
 
-@pytest.mark.parametrize("h_kv,n,d", [(8, 65536, 128), (8, 65568, 128), (16, 65568, 64)])
-def test_shadow_scan_on_both_sides_of_its_cache_policy(h_kv, n, d, gpu_device):
+@pytest.mark.parametrize("h_kv,group,n,d", [(8, 4, 65536, 128), (8, 4, 65568, 128), (16, 4, 65568, 64), (8, 16, 65536, 128),
+                                            (8, 16, 65568, 128)])
+def test_shadow_scan_on_both_sides_of_its_cache_policy(h_kv, group, n, d, gpu_device):
     """64 MiB of shadow in the launch, and more: the scan of the tiles under either policy selects what the bf16 scan does."""
     from hira_amd.indexer.hip import HIPIndexer
     from hira_amd.searcher.hip import HIPSearcher
 
-    group = 4
     g = torch.Generator(device="cuda").manual_seed(n + d)
     keys, vals = (torch.randn((1, h_kv, n, d), generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
     q = torch.randn((h_kv * group, d), generator=g, device="cuda").to(torch.bfloat16).float()
