@@ -358,7 +358,7 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
     p.tree_blocks = plan.tree_blocks;
     {   // up to what the eight L2s hold together (32 MiB) the default policy; up to 512 MiB the
         // key tiles and the value rows non-temporal; beyond, the key tiles only.  Tiles of the 8-bit shadow are
-        // non-temporal above 64 MiB of them
+        // non-temporal above 64 MiB of them (measured with two indexes in turn)
         const size_t key_bytes = (size_t)tree->num_trees * (size_t)tree->size[0] * (size_t)tree->dim * 2;
         if (p.keys8 != nullptr) plan.key_policy = key_bytes <= ((size_t)128 << 20) ? 0 : 1;
         else plan.key_policy = key_bytes <= ((size_t)32 << 20) ? 0 : (key_bytes <= ((size_t)512 << 20) ? 2 : 1);

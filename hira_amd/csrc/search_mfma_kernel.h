@@ -121,8 +121,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, si
 // 8-bit shadow: POL 0 or 1 (its tiles).  Decode steps over 1 / 2 / 6 indexes in turn, POL 0 and POL 1: 128 MiB of shadow in the
 // launch (8 heads a tree) 44.7 / 54.8 / 56.3 us and 48.9 / 49.1 / 52.8, 256 MiB 66.7 / 71.5 / - and 62.0 / 62.2 / -, 64 MiB 29.2 / 29.4 /
 // 36.4 and 31.0 / 31.5 / 32.6, 32 MiB 19.8 / 19.8 / 20.2 and 18.8 / 19.8 / 20.4: what the cache behind the L2s could hold of
-// one index or two is lost, what it holds of several gained -- the rows, which are read behind their tiles.  Those rows
-// non-temporal too gain nothing (128 MiB 49.5 / 50.9 / 52.4).
+// one index or two is lost, what it holds of several gained -- the rows, which are read behind their tiles.  The line goes by
+// two indexes in turn: at 64 MiB they lose with POL 1, as one does, where six gain a tenth; at 128 MiB they gain, as six do,
+// where one loses a tenth.  The rows non-temporal too gain nothing (128 MiB 49.5 / 50.9 / 52.4).
 constexpr int kReadOnce = 2;   // the `nt` bit of a buffer load's cache policy
 
 template <int KS, bool ONCE>
@@ -207,8 +208,9 @@ struct MfmaShape {
     static constexpr int KA = Q8 ? KS / 2 : KS;  // 16-byte chunks a lane holds of a scanned tile
     // nodes whose key tiles one wave keeps in flight: what the budget of 256 registers leaves
     // after twice the accumulators (GS x D/64) and some seventy registers of everything else
-    // (8-bit shadow: 64 registers, beside which a batch of rows fits without spills), and what keeps the round's
-    // list under 48 KiB of LDS
+    // (8-bit shadow: 64 registers, beside which a batch of rows fits without spills; ten of them with outputs at fan-out 64
+    // and eight heads, where lists take 21 us for 26 before the scan had two phases), and what keeps the round's list under
+    // 48 KiB of LDS
     static constexpr int KEY_REGS = Q8 ? 64 : 256 - 72 - 2 * GS * (KS / 2);
     static constexpr int NB_REGS = KEY_REGS / (MT * KA * 4);
     static constexpr int NB_LDS = (12000 / (GS + 1)) / (kMfmaWaves * ROWS);

@@ -33,8 +33,14 @@ constexpr int kSmallBig = kSmallItems / 65 + 1;
 
 // RI, below: item tiles a wave holds at a time, every sixteenth of the tree's: all of its own at the launch's first level, up
 // to four; one of rows of 256 columns, which take twice the registers (a wave has 128).  (Chosen inside the launch, the two sets
-// of registers met in spills: 8 x 1024 x 32 74 -> 112 us; four whatever the items: 128 x 4 25 -> 37.)
-constexpr int kSmallMean = 2;     // steps of a bucket's rows on their way
+// of registers met in spills: 8 x 1024 x 32 74 -> 112 us; four whatever the items: 128 x 4 25 -> 37.  Four tiles of 128 columns
+// spill too, 41 registers a lane, the others three to five.)
+// Steps of a bucket's rows on their way.  (One wave has a bucket, however many items it has.  Four waves for each of more than
+// 128 items, or four steps of it: what both take from the registers costs every other level more than they gain.  Launches of
+// 8 x 1024 x 32 keys of 128 columns as a build by itself, one wave / four waves / four steps: drawn from a normal distribution 90 / 94 / 90 us, six
+// of seven close to one another 117 / 120 / 117, seven of eight the same row 276 / 274 / 274; 8 x 256 25 / 27 / 30.  Before one wave had
+// them and items were asked for ahead 113, 130, 268 and 37; 8 x 512 x 16 of 256 columns, seven of eight the same row, 133 -> 144.)
+constexpr int kSmallMean = 2;
 constexpr int kSmallPlaces = 64;  // of a bucket, for items in order of arrival: what a wave ranks in registers
 
 // (whole item tiles, and the four rows that a tile's four lane groups write at a time in different banks)
@@ -181,7 +187,7 @@ __device__ __forceinline__ void small_assign(SmallLds<KS>& s, const void* x, siz
             }
         }
         if constexpr (!SCORES) {
-            int mine = -1, item = n_items;  // lane (kb, n): item n of tile kb (RI = 1: every lane group has it)
+            int mine = -1, item = n_items;  // lane (kb, n): item n of tile kb (lane groups from RI on: none)
 #pragma unroll
             for (int ri = 0; ri < RI; ++ri) {
                 auto nearer = [&](auto v, auto k) {  // of the two lanes that a swap has paired, in both of them
