@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import ctypes as C
 import itertools
+import threading
 from enum import Enum
 from typing import List, Optional, Tuple
 
@@ -34,6 +35,7 @@ DEFAULT_PAD_VALUE = 0.0
 _DTYPES = {torch.float32: _lib.HIRA_F32, torch.bfloat16: _lib.HIRA_BF16}
 
 _TICKETS = itertools.count(1)  # of read-backs (next() hands each number to one thread)
+_TAKING = threading.Lock()  # while one takes an index's rows
 _Row = C.c_int32 * (_lib.HIRA_MAX_LEVELS + 2)
 
 
@@ -903,7 +905,8 @@ class HIPIndexer(BaseIndexer):
 
     def _rows_to_read_into(self, n: int) -> torch.Tensor:
         """The pinned rows of a read-back, on the current device."""
-        rows = self.__dict__.pop("_host_rows", None)  # (looked at and taken in one step)
+        with _TAKING:
+            rows, self._host_rows = self._host_rows, None
         if rows is None or rows.numel() != n:
             self._refuse_capture()
             # (zero once: a row is there when it holds the call's ticket)
@@ -1011,7 +1014,8 @@ class HIPIndexer(BaseIndexer):
         if not sync and 0 < self._unsynced_room < m:  # (checked before anything is launched)
             raise RuntimeError("more appends than begin_unsynced made room for")
         if sync and self.keys_buf.is_cuda:  # (what it cannot read back it does not launch)
-            self._refuse_capture()
+            if _lib.stream_of(self.keys_buf.get_device()):  # (the default stream, 0, is never captured)
+                self._refuse_capture()
             rows, n = self._host_rows, self.num_trees * (_lib.HIRA_MAX_LEVELS + 2)
             if rows is None or rows.numel() != n:
                 self._host_rows = self._rows_to_read_into(n)
