@@ -123,85 +123,133 @@ __global__ __launch_bounds__(kNodeThreads) void k_init_centroids(const void* x, 
 
 // ------------------------------------------------------------------------------------
 // 2. nearest centroid (vector-ALU kernel): argmin_k ||x_i - c_k||^2, lowest k on ties.
-//    LPR lanes hold one item row; each lane group keeps PPG items in registers and walks
-//    all centroids.  fill != NULL: centroids with fill[k] >= bf are skipped.
+//    LPR lanes hold one item row; each lane group keeps PPG items in registers and walks the centroids, kAhead of
+//    them asked for at a time.  `share` waves of a workgroup hold the same items and walk every share-th centroid, as
+//    many as the chip has waves for; the best of theirs meet in LDS.  fill != NULL: centroids with fill[k] >= bf are
+//    skipped.
+//    Long lists are bound by the vector ALUs and the L2s that the centroids come from, short ones (what the approximate
+//    pass leaves: a few hundred items a tree) by the walk's trips to memory, which is why they are shared out and
+//    asked for several at a time: a wave to its items and a trip a centroid took such a list 317 us for 4 x 8000 fp32 items of 128
+//    columns and 500 centroids, now 31; builds of 4 x 8000 keys at a fan-out of 16 1787 -> 501 us, of 8 x 20000 at 32
+//    2335 -> 897, of 1 x 90000 at 8 32.8 -> 4.1 ms.
 // ------------------------------------------------------------------------------------
 constexpr int kPPG = 4;
+constexpr int kSimpleThreads = 512;
+constexpr int kSimpleWaves = kSimpleThreads / 64;
+static_assert(kSimpleWaves == 1 << 3, "simple_share_log2");
+constexpr int kSimpleBlocks = 1024;  // workgroups of all trees, at most: they go through a list in strides
+
+// Waves that share a set of items, of which each of `trees` trees has `sets` (as a power of two): the number whose
+// rounds of waves take least, a wave's items and its end as long as a dozen centroids.
+__device__ __forceinline__ int simple_share_log2(int sets, int trees, int K) {
+    constexpr int kFixed = 12, kOnChipLog2 = 12;
+    int best = 0;
+    long long least = 0;
+#pragma unroll
+    for (int s = 0; s <= 3; ++s) {
+        const long long rounds = (((long long)sets * trees << s) + (1 << kOnChipLog2) - 1) >> kOnChipLog2;
+        const long long cost = rounds * (kFixed + ((K + (1 << s) - 1) >> s));
+        if (s == 0 || cost < least) {
+            best = s;
+            least = cost;
+        }
+    }
+    return best;
+}
 
 template <typename T, int LPR>
-__global__ __launch_bounds__(256) void k_assign_simple(
-    const int32_t* fill, int bf, const AssignJob job) {
-    constexpr int EPL = Elem<T>::kPerChunk;
-    constexpr int RPW = kWave / LPR;
-    const int lane = lane_id();
+__global__ __launch_bounds__(kSimpleThreads, 4) void k_assign_simple(const int32_t* fill, int bf, const AssignJob job) {
+    constexpr int EPL = Elem<T>::kPerChunk, RPW = kWave / LPR, SET = RPW * kPPG;
+    constexpr int kAhead = EPL == 8 ? 2 : 4;
+    __shared__ float s_b[kSimpleWaves][SET];
+    __shared__ int s_g[kSimpleWaves][SET];
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rg = lane / LPR, ch = lane % LPR;
-    const int t = blockIdx.y;
+    const int t = blockIdx.x;
     const int n_items = items_of(job, t), n_c = job.n_c, D = job.D, K = job.K;
-    const int wave_global = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int first = wave_global * (RPW * kPPG);
-    if (job.counting.zero != nullptr && blockIdx.x == 0 && threadIdx.x == 0) job.counting.zero[t * kCounterStride] = 0;
+    if (job.counting.zero != nullptr && blockIdx.y == 0 && threadIdx.x == 0) job.counting.zero[t * kCounterStride] = 0;
+    const int sets = (n_items + SET - 1) / SET, share_log2 = simple_share_log2(sets, gridDim.x, K), share = 1 << share_log2;
+    const int part = wave & (share - 1), per_block = kSimpleWaves >> share_log2;
     const bool chunk_ok = ch * EPL < D;
+    const float* ct = job.cent + (size_t)t * K * D + (chunk_ok ? ch * EPL : 0);
+    const int32_t* ft = fill ? fill + (size_t)t * K : nullptr;
 
-    if (first < n_items) {  // (wave-uniform; no barrier inside)
-        int item[kPPG];
-        float xf[kPPG][EPL];
-        float best[kPPG];
+    for (int b = blockIdx.y; b * per_block < sets; b += gridDim.y) {  // uniform
+        const int first = (b * per_block + (wave >> share_log2)) * SET;
+        float xf[kPPG][EPL], best[kPPG];
         int arg[kPPG];
 #pragma unroll
         for (int p = 0; p < kPPG; ++p) {
             const int pos = first + p * RPW + rg;
-            item[p] = -1;
-            if (pos < n_items) item[p] = job.list ? job.list[(size_t)t * n_c + pos] : pos;
+            int item = -1;
+            if (pos < n_items) item = job.list ? job.list[(size_t)t * n_c + pos] : pos;
             uint4 raw = make_uint4(0, 0, 0, 0);
-            if (item[p] >= 0 && chunk_ok)
-                raw = load_chunk<T>(job.x, ((size_t)t * job.x_tree_stride + item[p]) * D, ch);
+            if (item >= 0 && chunk_ok) raw = load_chunk<T>(job.x, ((size_t)t * job.x_tree_stride + item) * D, ch);
             unpack<T>(raw, xf[p]);
             best[p] = INFINITY;
             arg[p] = -1;
         }
-        const float* ct = job.cent + (size_t)t * K * D;
-        const int32_t* ft = fill ? fill + (size_t)t * K : nullptr;
-        for (int k = 0; k < K; ++k) {
-            if (ft && ft[k] >= bf) continue;  // wave-uniform
-            float cf[4] = {0.f, 0.f, 0.f, 0.f};
-            float cf2[4] = {0.f, 0.f, 0.f, 0.f};
-            if (chunk_ok) {
-                const float4 a = *reinterpret_cast<const float4*>(ct + (size_t)k * D + ch * EPL);
-                cf[0] = a.x, cf[1] = a.y, cf[2] = a.z, cf[3] = a.w;
-                if (EPL == 8) {
-                    const float4 b =
-                        *reinterpret_cast<const float4*>(ct + (size_t)k * D + ch * EPL + 4);
-                    cf2[0] = b.x, cf2[1] = b.y, cf2[2] = b.z, cf2[3] = b.w;
+        // my centroids: part, part + share, ..., 64 of them looked up at a time
+        for (int k0 = part; k0 < K && first < n_items; k0 += share * 64) {  // uniform in the wave
+            const int kl = k0 + lane * share;
+            unsigned long long left = __ballot(kl < K && !(ft && ft[min(kl, K - 1)] >= bf));
+            while (left) {
+                int k[kAhead];
+                float4 c[kAhead][EPL / 4];
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) {  // (behind the last one: that one again)
+                    k[u] = left ? k0 + (__ffsll((long long)left) - 1) * share : k[u > 0 ? u - 1 : 0];
+                    left &= left - (left ? 1ull : 0ull);
+#pragma unroll
+                    for (int e = 0; e < EPL / 4; ++e)
+                        c[u][e] = reinterpret_cast<const float4*>(ct + (size_t)k[u] * D)[e];
                 }
-            }
 #pragma unroll
-            for (int p = 0; p < kPPG; ++p) {
-                float ss = 0.0f;
+                for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float df = xf[p][e] - cf[e];
-                    ss += df * df;
-                }
-                if (EPL == 8) {
+                    for (int p = 0; p < kPPG; ++p) {
+                        float ss = 0.0f;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float df = xf[p][4 + e] - cf2[e];
-                        ss += df * df;
+                        for (int e = 0; e < EPL / 4; ++e) {
+                            const float cf[4] = {c[u][e].x, c[u][e].y, c[u][e].z, c[u][e].w};
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const float df = xf[p][e * 4 + i] - cf[i];
+                                ss += df * df;
+                            }
+                        }
+                        ss = group_sum<LPR>(chunk_ok ? ss : 0.0f);
+                        if (ss < best[p]) {  // (centroids come in increasing order: ties keep the lower one)
+                            best[p] = ss;
+                            arg[p] = k[u];
+                        }
                     }
-                }
-                ss = group_sum<LPR>(ss);
-                if (ss < best[p]) {
-                    best[p] = ss;
-                    arg[p] = k;
-                }
             }
         }
         if (ch == 0) {
 #pragma unroll
             for (int p = 0; p < kPPG; ++p) {
-                if (item[p] >= 0) put_result(job, t, item[p], arg[p], best[p]);
+                s_b[wave][p * RPW + rg] = best[p];
+                s_g[wave][p * RPW + rg] = arg[p];
             }
         }
+        __syncthreads();
+        if (part == 0) {
+            for (int i = lane; i < SET && first + i < n_items; i += 64) {
+                float d = s_b[wave][i];
+                int g = s_g[wave][i];
+                for (int w = wave + 1; w < wave + share; ++w) {  // uniform
+                    const float od = s_b[w][i];
+                    const int og = s_g[w][i];
+                    if (og >= 0 && (g < 0 || od < d || (od == d && og < g))) {
+                        d = od;
+                        g = og;
+                    }
+                }
+                put_result(job, t, job.list ? job.list[(size_t)t * n_c + first + i] : first + i, g, d);
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -970,10 +1018,11 @@ template <typename T>
 static int launch_assign_simple(const AssignJob& job, const int32_t* fill, int bf, hipStream_t s) {
     int lpr = 2;
     while (lpr * Elem<T>::kPerChunk < job.D) lpr <<= 1;
-    const dim3 grid(ceil_div(job.n_c, 4 * (64 / lpr) * kPPG), job.num_trees);
+    // (as many workgroups as a list of all items has sets, if all waves share them)
+    const dim3 grid(job.num_trees, min(ceil_div(job.n_c, 64 / lpr * kPPG), max(kSimpleBlocks / job.num_trees, 16)));
 #define HIRA_ASSIGN_CASE(N)                                                                            \
     case N:                                                                                            \
-        hipLaunchKernelGGL((k_assign_simple<T, N>), grid, dim3(256), 0, s, fill, bf, job);             \
+        hipLaunchKernelGGL((k_assign_simple<T, N>), grid, dim3(kSimpleThreads), 0, s, fill, bf, job);  \
         break;
     switch (lpr) {
         HIRA_ASSIGN_CASE(2)
