@@ -45,21 +45,40 @@ __device__ __forceinline__ int node_of_wave() {
 }
 
 // ------------------------------------------------------------------------------------
-// 0. what a level starts from, in one launch: empty blocks, zero counters; the centroid columns that
-//    pad the last stage of operand tiles are zeros that take no items.
-//    n_live != NULL: tree t holds n_live[t] <= n_c items, the first ones of its rows, and uses its
-//    first ceil(n_t / bf) centroids only: the others count as full.
+// 1. what a level starts from, in one launch: empty blocks, zero counters, the initial centroids: centroid k is item
+//    floor((k + u_k) * n_c / K), u_k in [0,1) from the seed.
+//    n_live != NULL: tree t holds n_live[t] <= n_c items, the first ones of its rows, and uses its first
+//    K_t = ceil(n_t / bf) centroids only: the others count as full.
+//    ct.tiles != NULL: the centroids also go into their operand tiles (those that count as full take no items); the
+//    columns that pad the last stage of tiles are zeros that take no items.
+//    `lanes` (a power of two) hold a centroid, eight columns each, so that a wave takes several: bound by its
+//    instructions (the random number, the split into halves), 8 x 4096 centroids of 128 columns 13.5 us, 27 with a
+//    centroid a wave, most of whose lanes had no columns.  With the filling as a launch of its own ahead a build took 1 to 5 us more
+//    (8 x 8192 keys 253.5 -> 251.7, 4 x 5003 x 80 fp32 644 -> 640).
 // ------------------------------------------------------------------------------------
-__global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_t* n_live, int32_t* fill, int32_t* slots, int32_t* counts,
-                             int32_t* counters /* (kBuildCounters, T) */, float* absmax /* (T, kAbsCopies, D) or NULL */, CentroidTiles ct, int KS) {
-    const int t = blockIdx.x, T = gridDim.x;
+template <typename T>
+__global__ __launch_bounds__(kNodeThreads) void k_level_init(
+    const void* x, int n_c, size_t x_tree_stride, int K, int bf, int D, uint64_t seed, float* cent, const int32_t* n_live, int32_t* fill,
+    int32_t* slots, int32_t* counts, int32_t* counters /* (kBuildCounters, T) */,
+    float* absmax /* (T, kAbsCopies, D) or NULL */, int Kt, CentroidTiles ct, int KS, int lanes) {
+    constexpr int EPL = Elem<T>::kPerChunk, CH = 8 / EPL;
+    const int t = blockIdx.x, lane = threadIdx.x & 63, j = lane % lanes;
+    const int k = node_of_wave() * (64 / lanes) + lane / lanes, own = min(k, K - 1);
     const int n_t = n_live ? min(max(n_live[t], 0), n_c) : n_c;
-    const int K_t = n_live ? max((n_t + bf - 1) / bf, 1) : K;
-    const int stride = tree_blocks() * blockDim.x;
-    const int i0 = tree_block() * blockDim.x + threadIdx.x;
-    if (i0 == 0) {
-        for (int c = 0; c < kBuildCounters; ++c) counters[(c * T + t) * kCounterStride] = 0;
+    const int K_t = n_live ? min(max((n_t + bf - 1) / bf, 1), K) : K;
+    // ---- the centroid's item: on its way while the arrays are filled ---------------------------------
+    const long long idx = first_centroid(seed, t, own, max(n_t, 1), K_t);
+    const size_t src = ((size_t)t * x_tree_stride + (size_t)idx) * D;
+    uint4 raw[CH];
+#pragma unroll
+    for (int h = 0; h < CH; ++h) {
+        raw[h] = make_uint4(0, 0, 0, 0);
+        if ((j * CH + h) * EPL < D) raw[h] = load_chunk<T>(x, src, j * CH + h);
     }
+
+    const int stride = tree_blocks() * blockDim.x, T_ = gridDim.x;
+    const int i0 = tree_block() * blockDim.x + threadIdx.x;
+    if (i0 < kBuildCounters) counters[(i0 * T_ + t) * kCounterStride] = 0;
     if (absmax != nullptr)
         for (int i = i0; i < kAbsCopies * D; i += stride) absmax[(size_t)t * kAbsCopies * D + i] = 0.0f;
     for (int i = i0; i < K; i += stride) {
@@ -70,47 +89,22 @@ __global__ void k_level_init(int n_c, int K, int bf, int D, int Kt, const int32_
     if (ct.tiles != nullptr) {
         const int pad = Kt * 16 - K, cpc = KS * 8;  // chunks of a column: hi and lo halves
         for (int i = i0; i < pad * cpc; i += stride) {
-            const int k = K + i / cpc, c = i % cpc;
-            const int half = c / (KS * 4), j = c % (KS * 4);
-            ct.tiles[((size_t)t * Kt + (k >> 4)) * (size_t)(2 * KS * 64) + half * KS * 64 + (j >> 2) * 64 +
-                     (j & 3) * 16 + (k & 15)] = make_uint4(0, 0, 0, 0);
+            const int kp = K + i / cpc, c = i % cpc;
+            const int half = c / (KS * 4), jc = c % (KS * 4);
+            ct.tiles[((size_t)t * Kt + (kp >> 4)) * (size_t)(2 * KS * 64) + half * KS * 64 + (jc >> 2) * 64 +
+                     (jc & 3) * 16 + (kp & 15)] = make_uint4(0, 0, 0, 0);
         }
         for (int i = i0; i < pad; i += stride) {
             ct.n2[(size_t)t * Kt * 16 + K + i] = INFINITY;
             ct.lo[(size_t)t * Kt * 16 + K + i] = 0.0f;
         }
     }
-}
 
-// ------------------------------------------------------------------------------------
-// 1. initial centroids: item floor((k + u_k) * n_c / K), u_k in [0,1) from the seed
-// ------------------------------------------------------------------------------------
-//    (n_live != NULL: tree t holds n_live[t] <= n_c items, the first ones of its rows)
-//    ct.tiles != NULL: the centroid also goes into its operand tile (fill: the centroids that
-//    count as full from the start take no items)
-//    `lanes` (a power of two) hold a centroid, eight columns each, so that a wave takes several: bound by its
-//    instructions (the random number, the split into halves), 8 x 4096 centroids of 128 columns 13.5 us, 27 with a
-//    centroid a wave, most of whose lanes had no columns.
-template <typename T>
-__global__ __launch_bounds__(kNodeThreads) void k_init_centroids(const void* x, int n_c, size_t x_tree_stride,
-                                                       int K, int D, uint64_t seed, float* cent,
-                                                       const int32_t* n_live, int bf, int Kt,
-                                                       const int32_t* fill, CentroidTiles ct, int KS, int lanes) {
-    constexpr int EPL = Elem<T>::kPerChunk, CH = 8 / EPL;
-    const int t = blockIdx.x, lane = threadIdx.x & 63, j = lane % lanes;
-    const int k = node_of_wave() * (64 / lanes) + lane / lanes, own = min(k, K - 1);
-    const int n_t = n_live ? max(min(n_live[t], n_c), 1) : n_c;
-    // (a tree with fewer items uses the first K_t = ceil(n_t / bf) centroids only)
-    const int K_t = n_live ? min(max((n_t + bf - 1) / bf, 1), K) : K;
-    const long long idx = first_centroid(seed, t, own, n_t, K_t);
-    const size_t src = ((size_t)t * x_tree_stride + (size_t)idx) * D;
     float v[8];
 #pragma unroll
     for (int h = 0; h < CH; ++h) {
-        uint4 raw = make_uint4(0, 0, 0, 0);
-        if ((j * CH + h) * EPL < D) raw = load_chunk<T>(x, src, j * CH + h);
         float f[EPL];
-        unpack<T>(raw, f);
+        unpack<T>(raw[h], f);
 #pragma unroll
         for (int e = 0; e < EPL; ++e) v[h * EPL + e] = f[e];
     }
@@ -118,7 +112,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_init_centroids(const void* x, 
 #pragma unroll
     for (int h = 0; h < 2; ++h)  // (rows are whole fours)
         if (k < K && j * 8 + h * 4 < D) *reinterpret_cast<float4*>(dst + h * 4) = make_float4(v[h * 4], v[h * 4 + 1], v[h * 4 + 2], v[h * 4 + 3]);
-    if (ct.tiles != nullptr) emit_columns(v, j, lanes, k < K, KS, Kt, t, own, fill[(size_t)t * K + own] < bf, ct);
+    if (ct.tiles != nullptr) emit_columns(v, j, lanes, k < K, KS, Kt, t, own, own < K_t, ct);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1103,13 +1097,11 @@ static int cluster_levels(const HiraTree* t, const void* keys_in, int n, const i
         // Trees with fewer items than rows (n_live): the rounds over all items are over the first
         // ones of every tree.
         const bool ragged = n_live != nullptr && l == 1;
-        hipLaunchKernelGGL(k_level_init, tree_grid(min(ceil_div(Kl * bf, 256), 2048), NT), dim3(256), 0, s, n_c, Kl, bf,
-                           D, Kt, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters, l == 1 ? w.absmax : nullptr, tiles, KS);
         int lanes = 1;
         while (lanes * 8 < D || (on_mfma && lanes < KS * 4)) lanes <<= 1;
-        hipLaunchKernelGGL((k_init_centroids<T>), node_grid(ceil_div(Kl, 64 / lanes), NT), dim3(kNodeThreads), 0, s, x, n_c, xs, Kl, D,
-                           seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, bf,
-                           Kt, w.fill, tiles, KS, lanes);
+        hipLaunchKernelGGL((k_level_init<T>), node_grid(ceil_div(Kl, 64 / lanes), NT), dim3(kNodeThreads), 0, s, x, n_c, xs, Kl, bf, D,
+                           seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters,
+                           l == 1 ? w.absmax : nullptr, Kt, tiles, KS, lanes);
         // a round: the assignment (which also puts the items into buckets), then what the round does
         // with every bucket.  A Lloyd round asks for no distances.
         auto buckets = [&]() {
