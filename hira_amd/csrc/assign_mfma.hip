@@ -246,7 +246,12 @@ __global__ __launch_bounds__(kAssignThreads, 2) void k_assign_mfma(const AssignJ
 // centroids few (8 x 7200 items, 330 centroids: 40 us, now 24; 8 x 8300, 330: 58, now 48); one wave to
 // 64 items whatever their number: 8 x ~1000 items, 1024 centroids 52 us, now 9.
 constexpr int kSplitThreads = 512;
-constexpr int kSplitBlocks = 128;        // workgroups of a tree, at most: they go through a list in strides
+// Workgroups of a tree, at most (they go through a list in strides): those of all trees fill the chip twice.  (128
+// whatever the trees: 1 x 100000 rows of 64 columns 805 us a build, now 747.)
+constexpr int split_blocks(int KS, int trees) {
+    const int all = KS <= 2 ? 1024 : 512;
+    return all / 16 < trees ? 16 : all / trees;
+}
 constexpr int kSplitWavesLog2 = 11;      // of the waves on the chip at a time: 256 compute units, 8 each
 static_assert(kSplitThreads == 64 << 3, "split_share_log2");
 
@@ -1122,7 +1127,7 @@ static int launch_exact(const AssignJob& job, hipStream_t s) {
     // length only the device knows, and few items, which would leave the chip idle, 64 a workgroup.
     if (job.list != nullptr || job.after_approx || (long long)job.n_c * job.num_trees <= kApproxListItems) {
         const int per_block = split_ri(KS) * 16, blocks = (job.n_c + per_block - 1) / per_block;
-        hipLaunchKernelGGL((k_assign_split<KS>), dim3(job.num_trees, blocks < kSplitBlocks ? blocks : kSplitBlocks),
+        hipLaunchKernelGGL((k_assign_split<KS>), dim3(job.num_trees, min(blocks, split_blocks(KS, job.num_trees))),
                            dim3(kSplitThreads), 0, s, job, Kt);
         return HIRA_OK;
     }
