@@ -200,7 +200,7 @@ _lib = None
 
 
 def build_library(verbose: bool = False) -> None:
-    """Compile libhira_hip.so for gfx950 (hipcc cross-compiles without a GPU)."""
+    """Compile libhira_hip.so for gfx950 (hipcc cross-compiles without a GPU) and the native host side, _host.so."""
     r = subprocess.run(["make", "-C", str(CSRC), "-B", "-j8"], capture_output=True, text=True)
     if verbose or r.returncode != 0:
         print(r.stdout[-4000:], r.stderr[-4000:])
@@ -236,6 +236,27 @@ def lib() -> C.CDLL:
             raise RuntimeError(f"libhira_hip.so ABI {got}, expected {HIRA_ABI_VERSION}")
         _lib = l
     return _lib
+
+
+_host_module = None
+
+
+def host():
+    """The native host side of the calls a decode step makes (csrc/host.cpp), on the loaded library's functions; raises when
+    it has not been built."""
+    global _host_module
+    if _host_module is None:
+        l = lib()
+        try:
+            import torch  # noqa: F401  (its libraries, which the module needs)
+
+            from hira_amd import _host
+        except ImportError as ex:
+            raise RuntimeError(f"hira_amd/_host.so is missing or was built for another torch ({ex}): build it with "
+                               f"`make -C {CSRC}` (or __graft_entry__.build())") from ex
+        _host.bind({name: C.cast(getattr(l, name), _vp).value for name in SYMBOLS})
+        _host_module = _host
+    return _host_module
 
 
 def check(rc: int) -> None:

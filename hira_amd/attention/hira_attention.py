@@ -117,6 +117,13 @@ def hira_attention_forward(module, query, key, value, attention_mask=None, dropo
         hira_threshold = index_thresholds(indexer, query, hira_topk or max(1, indexer.num_keys // 100))
     # one plan per (index, head count, scale): a decode step is then a single library call
     plan = searcher.decode_plan(indexer, b * h_q, scaling)
+    if sampled:
+        rows, store = getattr(cache, "queue_rows", None), getattr(cache, "queue_store", None)
+        if rows is not None and store is not None:
+            # (the form that a running decode has; what has another goes on below)
+            out = plan.attend(query, samples, cache.threshold_method, cache.threshold_topk, store[0], store[1], rows)
+            if out is not None:
+                return out, None
     buf, dtype = indexer.keys_buf, indexer.dtype
     dev = buf.get_device()
     # (the search writes its output in the query's own type where that is one of its two)

@@ -120,9 +120,6 @@ class HiraCacheLayer(CacheLayerMixin):
         self._queue_form = self._queue_type, self.batch * self.H_kv, rows
         self._queue_rows = rows
         self._queue_dev = self._queue_k.get_device()
-        # the shapes of a token's rows (a launch takes them as they are)
-        head = (self.batch, self.H_kv, 1)
-        self._token = torch.Size(head + (self.dim,)), torch.Size(head + (self.vdim,))
 
     @property
     def queued_keys(self):
@@ -141,18 +138,11 @@ class HiraCacheLayer(CacheLayerMixin):
             x.get_device() == like.get_device() and x.is_contiguous() and x.data_ptr() % 16 == 0
 
     def _enqueue(self, key_states, value_states):
-        k, v, n = self._queue_k, self._queue_v, self.queued_len
-        dev, token = self._queue_dev, self._token
-        if n < self._queue_rows and self._queue_type is not None and dev >= 0 and \
-                key_states.shape == token[0] and value_states.shape == token[1] and \
-                key_states.dtype is k.dtype and value_states.dtype is k.dtype and \
-                key_states.get_device() == dev and value_states.get_device() == dev and \
-                key_states.is_contiguous() and value_states.is_contiguous():
-            # a token's rows: what follows, without the questions about shapes
-            kp, vp = key_states.data_ptr(), value_states.data_ptr()
-            if (kp | vp) % 16 == 0:
-                rc = _lib.lib().hira_enqueue(k.data_ptr(), v.data_ptr(), *self._queue_form, n, 1, self.dim, self.vdim,
-                                             kp, vp, _lib.stream_of(dev))
+        n, dev = self.queued_len, self._queue_dev
+        if dev >= 0 and n < self._queue_rows:
+            # a token's rows, if they come as the queue holds them
+            rc = _lib.host().enqueue(self._queue_k, self._queue_v, key_states, value_states, n, dev, _lib.stream_of(dev))
+            if rc is not None:
                 if rc:
                     _lib.check(rc)
                 self.queued_len = n + 1
@@ -277,15 +267,7 @@ class HiraCacheLayer(CacheLayerMixin):
             self._sample_facts()
             if first == m:
                 return (), ()
-        s, seen = self.samples.shape[1], seen + first
-        draws = torch.rand(m - first, generator=self._sample_gen).tolist()
-        who = [first + i for i, u in enumerate(draws) if u < s / (seen + i + 1)]
-        if not who:
-            return (), ()
-        slots = torch.randint(0, s, (len(who),), generator=self._sample_gen).tolist()
-        # a slot drawn twice keeps its last arrival
-        last = dict(zip(slots, who))
-        return tuple(last.keys()), tuple(last.values())
+        return _lib.host().draw(self._sample_gen, m - first, first, self.samples.shape[1], seen + first)
 
     def _replace_sampled(self, new_keys, slots, which):
         """The members `slots` of the sample replaced by rows `which` of the new keys."""

@@ -60,6 +60,7 @@ def from_tiled(x: torch.Tensor) -> torch.Tensor:
 
 
 _NO_SAMPLE = (None, 0, None, None, 0)
+_NOTHING = None, (), ()
 _MINUS_INF = 0xFF800000  # the bits of an fp32 -inf
 
 
@@ -139,7 +140,7 @@ class _Append:
     tree's struct is the same (its arrays, capacities and size bounds) and `left` calls are not used
     up, the bounds of the level sizes do not move and the capacities suffice."""
 
-    __slots__ = ("tree", "ref", "state", "dev", "m", "kshape", "vshape", "left")
+    __slots__ = ("tree", "at", "state", "dev", "m", "kshape", "vshape", "left")
 
 
 class HIPIndexer(BaseIndexer):
@@ -225,6 +226,8 @@ class HIPIndexer(BaseIndexer):
         self._tree_struct = None
         self._state: Optional[torch.Tensor] = None  # device-side bookkeeping of update()
         self._append: Optional[_Append] = None
+        # shapes of the last rows that update placed one by one, and the graft_min it went by
+        self._placed: Optional[tuple] = None
 
     # pinned: where the state's rows are read back to.  A read-back takes them while it lasts, so that another thread's
     # has rows of its own
@@ -379,7 +382,7 @@ class HIPIndexer(BaseIndexer):
         if specs:
             _fill_arrays(specs, t)
         self._tree_struct = None
-        self._state = self._append = None
+        self._state = self._append = self._placed = None
 
     def tree_struct(self) -> _lib.HiraTree:
         """The C view of the tree; valid while this indexer's tensors are alive."""
@@ -932,8 +935,9 @@ class HIPIndexer(BaseIndexer):
         self._host_rows = rows
         return list(most)
 
-    def _adopt_state(self) -> None:
-        most = self._largest_state()
+    def _adopt_state(self, most: Optional[List[int]] = None) -> None:
+        if most is None:
+            most = self._largest_state()
         if most[_lib.HIRA_MAX_LEVELS + 1] != 0:
             raise RuntimeError("index update ran out of capacity")
         if self.num_levels == 1:
@@ -964,81 +968,100 @@ class HIPIndexer(BaseIndexer):
         slot twice)."""
         a = self._append
         if a is not None and not sync and a.tree is self._tree_struct and a.left > 0 and \
-                new_keys.shape == a.kshape and new_values is not None and new_values.shape == a.vshape and \
-                new_keys.dtype is self.dtype and new_values.dtype is self.dtype and \
-                new_keys.get_device() == a.dev and new_values.get_device() == a.dev and \
-                new_keys.is_contiguous() and new_values.is_contiguous() and \
-                (sample is None or new_keys.data_ptr() % 16 == 0):
-            rc = _lib.lib().hira_update_sample(
-                a.ref, new_keys.data_ptr(), new_values.data_ptr(), a.m, a.state, *self._sample_args(sample),
-                _lib.stream_of(a.dev))
-            if rc:
-                _lib.check(rc)
-            a.left -= 1
-            self.num_keys += a.m
-            self._pending += a.m
-            return self
+                new_keys.shape == a.kshape and new_values is not None and new_values.shape == a.vshape:
+            rows, slots, which = sample or _NOTHING
+            rc = _lib.host().append(a.at, new_keys, new_values, a.m, a.state, rows, slots, which, a.dev, _lib.stream_of(a.dev),
+                                    None, 0)
+            if rc is not None:
+                if rc:
+                    _lib.check(rc)
+                a.left -= 1
+                self.num_keys += a.m
+                self._pending += a.m
+                return self
         if self.keys_buf is None:
             raise ValueError("Indexer is not built: call build() first.")
-        if new_keys.ndim != 4 or new_keys.shape[0] != self.batch or \
-                new_keys.shape[1] != self.num_heads or new_keys.shape[3] != self.dim:
-            raise ValueError(
-                f"new_keys must be ({self.batch},{self.num_heads},m,{self.dim}), got "
-                f"{tuple(new_keys.shape)}")
-        if (new_values is None) != (self.values_buf is None):
-            raise ValueError("values must be given exactly when the index was built with values")
-        m = int(new_keys.shape[2])
-        if new_values is not None and tuple(new_values.shape[:3]) != tuple(new_keys.shape[:3]):
-            raise ValueError("new_values must be aligned with new_keys")
-        if m == 0:
-            return self
-        if not sync and self.num_levels < 2:
-            raise ValueError("sync=False needs a tree of at least two levels (a one-level index "
-                             "has no node counts to tell empty key slots by)")
-        if self.num_levels >= 2 and (not self.tiled or self.branching_factor % 16 == 0):
-            bf, nl = self.branching_factor, self.num_levels
-            full = self.graft_min if self.graft_min is not None else max(256, bf ** (nl - 1) // 2)
-            part = self.graft_min if self.graft_min is not None else max(256, bf ** (nl - 2) // 2)
-            if m >= full:
-                self._graft(new_keys, new_values, m, nl, None)
-                return self._replace_sample(sample, new_keys, m)
-            if nl >= 3 and m >= part:
-                # a mid-size window: further children of an existing root where every tree has
-                # one with room, else a new root (whose free child slots take the next ones)
-                where = self._room_under_a_root(new_keys, m)
-                if where is not None:
-                    self._graft(new_keys, new_values, m, nl - 1, where)
-                else:
+        form = self._placed
+        if form is not None and new_keys.shape == form[0] and new_values is not None and new_values.shape == form[1] and \
+                self.graft_min == form[2] and (sync or self.num_levels >= 2):
+            m = form[0][2]  # (as many rows, of the same shapes, as a call before it that placed them one by one)
+        else:
+            if new_keys.ndim != 4 or new_keys.shape[0] != self.batch or \
+                    new_keys.shape[1] != self.num_heads or new_keys.shape[3] != self.dim:
+                raise ValueError(
+                    f"new_keys must be ({self.batch},{self.num_heads},m,{self.dim}), got "
+                    f"{tuple(new_keys.shape)}")
+            if (new_values is None) != (self.values_buf is None):
+                raise ValueError("values must be given exactly when the index was built with values")
+            m = int(new_keys.shape[2])
+            if new_values is not None and tuple(new_values.shape[:3]) != tuple(new_keys.shape[:3]):
+                raise ValueError("new_values must be aligned with new_keys")
+            if m == 0:
+                return self
+            if not sync and self.num_levels < 2:
+                raise ValueError("sync=False needs a tree of at least two levels (a one-level index "
+                                 "has no node counts to tell empty key slots by)")
+            if self.num_levels >= 2 and (not self.tiled or self.branching_factor % 16 == 0):
+                bf, nl = self.branching_factor, self.num_levels
+                full = self.graft_min if self.graft_min is not None else max(256, bf ** (nl - 1) // 2)
+                part = self.graft_min if self.graft_min is not None else max(256, bf ** (nl - 2) // 2)
+                if m >= full:
                     self._graft(new_keys, new_values, m, nl, None)
-                return self._replace_sample(sample, new_keys, m)
+                    return self._replace_sample(sample, new_keys, m)
+                if nl >= 3 and m >= part:
+                    # a mid-size window: further children of an existing root where every tree has
+                    # one with room, else a new root (whose free child slots take the next ones)
+                    where = self._room_under_a_root(new_keys, m)
+                    if where is not None:
+                        self._graft(new_keys, new_values, m, nl - 1, where)
+                    else:
+                        self._graft(new_keys, new_values, m, nl, None)
+                    return self._replace_sample(sample, new_keys, m)
+            if new_values is not None:
+                self._placed = (new_keys.shape, new_values.shape, self.graft_min)
         if not sync and 0 < self._unsynced_room < m:  # (checked before anything is launched)
             raise RuntimeError("more appends than begin_unsynced made room for")
-        if sync and self.keys_buf.is_cuda:  # (what it cannot read back it does not launch)
-            if _lib.stream_of(self.keys_buf.get_device()):  # (the default stream, 0, is never captured)
+        dev, stream, t = self.keys_buf.get_device(), None, self.num_trees
+        if sync and dev >= 0:  # (what it cannot read back it does not launch)
+            stream = _lib.stream_of(dev)
+            if stream:  # (the default stream, 0, is never captured)
                 self._refuse_capture()
-            rows, n = self._host_rows, self.num_trees * (_lib.HIRA_MAX_LEVELS + 2)
+            rows, n = self._host_rows, t * (_lib.HIRA_MAX_LEVELS + 2)
             if rows is None or rows.numel() != n:
                 self._host_rows = self._rows_to_read_into(n)
         need = self._needed_caps(m)
         self._grow(need)
-        t = self.num_trees
         if self._state is None:
             self._init_state()
-        kin = self._rows(new_keys, t, m, self.dim)
-        vin = None if new_values is None else self._rows(new_values, t, m, self.vdim)
-        tree = self.tree_struct()
-        rows, per_tree, slots, which, n = self._sample_args(sample)
-        if n and kin.data_ptr() % 16:  # (whole chunks of rows move there)
-            kin = kin.clone()
-        rc = _lib.lib().hira_update_sample(C.byref(tree), kin.data_ptr(),
-                                           None if vin is None else vin.data_ptr(), m,
-                                           self._state.data_ptr(), rows, per_tree, slots, which, n,
-                                           _lib.stream_of(self.keys_buf.get_device()))
-        if rc:
+        tree, rc, most = self.tree_struct(), None, None
+        if dev >= 0:  # in one step, the read-back with it, if the tensors are ready
+            back = None
+            if sync and torch.cuda.current_device() == dev:
+                back = self._rows_to_read_into(t * (_lib.HIRA_MAX_LEVELS + 2))
+            rc = _lib.host().append(C.addressof(tree), new_keys, new_values, m, self._state.data_ptr(), *(sample or _NOTHING), dev,
+                                    _lib.stream_of(dev) if stream is None else stream, back,
+                                    next(_TICKETS) % 0x7fffffff + 1)
+            if rc.__class__ is list:
+                most, rc = rc, 0
+            if back is not None and not rc:  # (whatever went wrong: these rows are not used again)
+                self._host_rows = back
+        if rc is None:
+            kin = self._rows(new_keys, t, m, self.dim)
+            vin = None if new_values is None else self._rows(new_values, t, m, self.vdim)
+            rows, per_tree, slots, which, n = self._sample_args(sample)
+            if n and kin.data_ptr() % 16:  # (whole chunks of rows move there)
+                kin = kin.clone()
+            rc = _lib.lib().hira_update_sample(C.byref(tree), kin.data_ptr(),
+                                               None if vin is None else vin.data_ptr(), m,
+                                               self._state.data_ptr(), rows, per_tree, slots, which, n,
+                                               _lib.stream_of(dev))
+        if rc and rc > -100:
             _lib.check(rc)
         self.num_keys += m
+        if rc:  # (the rows are in, their sizes could not be read back)
+            _lib.check(rc + 100)
         if sync:
-            self._adopt_state()
+            self._adopt_state(most)
             self._unsynced_room = 0
             return self
         if self._exact_size is None:  # (inside a stretch self.size already holds bounds)
@@ -1055,7 +1078,7 @@ class HIPIndexer(BaseIndexer):
         if self._unsynced_room == 0 and new_values is not None:
             a = self._append = _Append()
             a.tree, a.state, a.dev, a.m = self.tree_struct(), self._state.data_ptr(), self.keys_buf.get_device(), m
-            a.ref, a.kshape, a.vshape = C.byref(a.tree), new_keys.shape, new_values.shape
+            a.at, a.kshape, a.vshape = C.addressof(a.tree), new_keys.shape, new_values.shape
             # (a new level-1 node at most every `bf` keys: the bounds move when the next one may be)
             a.left = -self._pending % self.branching_factor // m
         return self

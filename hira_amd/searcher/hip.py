@@ -64,12 +64,12 @@ class _Call:
     per head (the library's own; None: not asked for yet), the workspace's size.  Made on first use and
     kept by the searcher: a call that comes with ready tensors (the storage type, on the index's device,
     contiguous) then allocates and copies nothing and its host side is a handful of attribute reads
-    around one library call (21 -> 8 us for ``search``, 25 -> 11 us for ``search_attention``, which the
-    kernels of small indexes are shorter than).  That holds from the second call on a tree whose level
+    around one library call (25 -> 11 us for ``search_attention``, which the kernels of small indexes are shorter
+    than), and for ``search`` one call of the native host side (21 -> 8 -> 4.6 us, the launch's own time).  That holds from the second call on a tree whose level
     sizes stay: the first on an index, and the first after an append that moved them, makes it anew."""
 
     __slots__ = ("tree", "query", "out", "queue", "dev", "keep", "ones", "ws_bytes", "ws_at", "ws_for",
-                 "launch", "tree_ref", "query_ref", "out_ref", "queue_ref", "launch_ref")
+                 "launch", "tree_ref", "query_ref", "out_ref", "queue_ref", "launch_ref", "launch_at", "at")
 
     def __init__(self, tree, query, dev, keep):
         self.tree, self.query, self.dev, self.keep, self.ones = tree, query, dev, keep, None
@@ -79,7 +79,19 @@ class _Call:
         self.ws_bytes, self.ws_at, self.ws_for = 0, 0, (-1, b"")
         self.tree_ref, self.query_ref = C.byref(tree), C.byref(query)
         self.out_ref, self.queue_ref = C.byref(self.out), C.byref(self.queue)
-        self.launch = self.launch_ref = None
+        self.launch = self.launch_ref = self.launch_at = None
+        self.at: Optional[tuple] = None  # what the native search takes of it
+
+    def follow_launch(self, launch) -> None:
+        """The searcher's launch options as they are now (callers may replace them, or change their fields)."""
+        self.launch, self.launch_ref, self.launch_at = launch, C.byref(launch), C.addressof(launch)
+
+    def addresses(self) -> tuple:
+        """(not kept before the scale of ones is known: it is asked for once)"""
+        at = (C.addressof(self.tree), C.addressof(self.query), C.addressof(self.out), self.query.num_q_heads, self.dev, self.ones)
+        if self.ones:
+            self.at = at
+        return at
 
 
 class HIPSearcher(BaseSearcher):
@@ -274,7 +286,7 @@ class HIPSearcher(BaseSearcher):
         queue_ref = c.queue_ref if queue_rows else None
         launch = self.launch  # (as it is now: callers may replace it, or change its fields)
         if c.launch is not launch:
-            c.launch, c.launch_ref = launch, C.byref(launch)
+            c.follow_launch(launch)
         if attn:
             rows, options = c.ws_for
             now = bytes(launch)
@@ -302,8 +314,21 @@ class HIPSearcher(BaseSearcher):
         if indexer.keys_buf is None:
             raise ValueError("Indexer is not built: missing children tensor.")
         space = index_space or self.index_space
-        c, h_q, keep = self._call(query, threshold, indexer, q_head_to_kv, scaling)
         slots = space == "slot"
+        tree, dense = indexer._tree_struct, self._tmp_out
+        if slots and tree is not None and dense is not None and q_head_to_kv is None and stats is None:
+            # a call like one before it on this tree: in one step, if its tensors are ready
+            c = self._calls.get((get_ident(), id(tree), dense.shape[0]))
+            if c is not None:
+                if c.launch is not self.launch:
+                    c.follow_launch(self.launch)
+                rc = _lib.host().search(c.at or c.addresses(), c.launch_at, query, threshold, scaling, dense, self.output_fill_value,
+                                        _lib.stream_of(c.dev))
+                if rc is not None:
+                    if rc:
+                        _lib.check(rc)
+                    return dense
+        c, h_q, keep = self._call(query, threshold, indexer, q_head_to_kv, scaling)
         n = indexer.size[0] if slots else indexer.num_keys
         # in slot space the search fills what it does not select itself: one launch per call
         dense = self._tmp_out
@@ -475,6 +500,7 @@ class DecodePlan:
         self.sample.scratch = self.tau_scratch.data_ptr()
         self._refs = (C.byref(self.tree), C.byref(self.query), C.byref(self.out),
                       C.byref(self.launch), C.byref(self.queue))
+        self._at: Optional[tuple] = None  # where the call's structs lie, for ``attend``
 
     def _workspace_need(self) -> int:
         fake_q = _lib.HiraQuery(self.query.num_q_heads, 1, 1, 1, 1, 1, self.query.max_group,
@@ -492,6 +518,25 @@ class DecodePlan:
         self.ws_bytes = need
         self._refs = (C.byref(self.tree), C.byref(self.query), C.byref(self.out),
                       C.byref(self.launch), C.byref(self.queue))
+        self._at = None
+
+    def attend(self, query: torch.Tensor, samples: torch.Tensor, method: str, k: int, queue_keys: torch.Tensor,
+               queue_values: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
+        """``run_sampled`` for the form that a running decode has, in one step: query (B, H_q, 1, D) of the tree's type, the
+        first `rows` rows of a decode queue (B, H_kv, cap, D / Dv); makes the output (B, 1, H_q, Dv) in the query's type.
+        None, and nothing done, for any other form."""
+        if self.indexer._tree_struct is not self.tree:
+            self._follow_index()
+        at = self._at
+        if at is None:
+            at = self._at = tuple(C.addressof(x) for x in (self.tree, self.query, self.sample, self.queue, self.out, self.launch))
+        if self.tau_buf is None:
+            self.tau_buf = torch.empty((self.query.num_q_heads,), dtype=torch.float32, device=self.indexer.device)
+        out = _lib.host().attend(at, self._dev, self.ws, self.ws_bytes, self._ws_rows, self.tau_buf, query, samples, queue_keys,
+                                 queue_values, rows, 0 if method == "sample_max" else 1, k, _lib.stream_of(self._dev))
+        if out.__class__ is int:
+            _lib.check(out)
+        return out
 
     def run(self, query: torch.Tensor, threshold: torch.Tensor, out: torch.Tensor,
             stream: Optional[int] = None, queue_keys: Optional[torch.Tensor] = None,

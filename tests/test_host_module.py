@@ -1,0 +1,51 @@
+"""The native host side (csrc/host.cpp) without a GPU: the random numbers it draws, and that what is not the form of a running
+program's call is left to the Python body."""
+import ctypes as C
+
+import pytest
+import torch
+
+from hira_amd import _lib
+
+
+def _draw(gen, m, first, members, seen):
+    """Reservoir sampling in torch: the slots of the sample that are replaced, and by which keys."""
+    who = [first + i for i, u in enumerate(torch.rand(m, generator=gen).tolist()) if u < members / (seen + i + 1)]
+    slots = torch.randint(0, members, (len(who),), generator=gen).tolist() if who else []
+    last = dict(zip(slots, who))
+    return tuple(last.keys()), tuple(last.values())
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_the_numbers_of_torch(wide):
+    torch.set_default_dtype(torch.float64 if wide else torch.float32)
+    try:
+        a, b = torch.Generator().manual_seed(3), torch.Generator().manual_seed(3)
+        for m, first, members, extra in [(1, 0, 1000, 0), (1, 0, 1, 5000), (15, 1, 7, 3), (16, 0, 4096, 10), (700, 2, 33, 100),
+                                         (3000, 0, 4096, 1)] * 20:
+            assert _lib.host().draw(a, m, first, members, members + extra) == _draw(b, m, first, members, members + extra)
+        assert torch.equal(a.get_state(), b.get_state())
+    finally:
+        torch.set_default_dtype(torch.float32)
+
+
+def test_what_is_not_the_form_is_left_alone():
+    host = _lib.host()
+    q, k, v = torch.zeros(1, 2, 4, 16), torch.zeros(1, 2, 1, 16), torch.zeros(1, 2, 1, 16)
+    assert host.enqueue(q, q.clone(), k, v, 0, 0, 0) is None  # (host memory)
+    assert host.enqueue(None, q, k, [1], 0, 0, 0) is None
+    tree, query, out, launch = _lib.HiraTree(num_trees=2, dim=16, vdim=16), _lib.HiraQuery(4), _lib.HiraSearchOut(), _lib.HiraLaunch()
+    at = tuple(C.addressof(x) for x in (tree, query, _lib.HiraSample(), _lib.HiraQueue(), out, launch))
+    ws, tau = torch.zeros(64, dtype=torch.uint8), torch.zeros(4)
+    assert host.attend(at, 0, ws, 64, 1, tau, torch.zeros(1, 4, 1, 16), torch.zeros(2, 8, 16), q, q, 1, 0, 1, 0) is None
+    at = C.addressof(tree), C.addressof(query), C.addressof(out), 4, 0, 1
+    assert host.search(at, C.addressof(launch), torch.zeros(4, 16), tau, None, torch.zeros(4, 8), 0.0, 0) is None
+    assert host.append(C.addressof(tree), k, v, 1, 0, None, (), (), 0, 0, None, 0) is None
+    assert query.q is None and out.attn_out is None and out.dense is None
+    for name in ("enqueue", "attend", "search", "append", "draw"):
+        with pytest.raises(TypeError):
+            getattr(host, name)(1)
+    with pytest.raises(TypeError):
+        host.draw(3, 1, 0, 1, 1)
+    with pytest.raises(ValueError):
+        host.draw(torch.Generator(), 1, 0, 0, 1)

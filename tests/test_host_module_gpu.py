@@ -1,0 +1,105 @@
+"""Calls in the form that the native host side takes against the same calls in other forms (strides, types, storage that is not
+aligned), which go through the Python bodies: same results."""
+import pytest
+import torch
+
+from hira_amd.attention.hira_attention import hira_attention_forward
+from hira_amd.cache.hira_cache import HiraCacheLayer
+from hira_amd.indexer import HIPIndexer
+from hira_amd.searcher import HIPSearcher
+
+pytestmark = pytest.mark.gpu
+
+
+def _gen(seed):
+    g = torch.Generator().manual_seed(seed)
+    return lambda *shape, dtype=torch.bfloat16: torch.randn(shape, generator=g).to(dtype).cuda()
+
+
+def _strided(x):
+    """The same numbers a column of gaps apart."""
+    wide = torch.zeros(x.shape[:-1] + (2 * x.shape[-1],), dtype=x.dtype, device=x.device)
+    wide[..., ::2] = x
+    return wide[..., ::2]
+
+
+def _misaligned(x):
+    flat = torch.zeros(x.numel() + 1, dtype=x.dtype, device=x.device)
+    flat[1:] = x.reshape(-1)
+    return flat[1:].view(x.shape)
+
+
+FORMS = {"ready": lambda x: x, "strided": _strided, "misaligned": _misaligned, "fp32": lambda x: x.float(),
+         "parameter": lambda x: torch.nn.Parameter(x, requires_grad=False)}
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("every,n", [(4, 300), (1, 300), (3, 900)])
+def test_a_decode_through_the_cache_layer(form, every, n, gpu_device):
+    if form == "misaligned" and every == 1:
+        pytest.skip("rows that go into the index at once")
+    as_query = FORMS[form] if form in ("strided", "parameter") else FORMS["ready"]
+
+    def run(form):
+        print(f"case form={form} every={every} n={n}", flush=True)
+        x = _gen(n + every)
+        layer = HiraCacheLayer("cuda_only", every, dict(num_levels=3, max_iterations=1, branching_factor=16), {},
+                               dict(method="sample_mean_topk", sample_size=500, topk=7))
+        layer.update(x(1, 2, n, 64), x(1, 2, n, 64))
+        outs, module = [], type("M", (), {"scaling": 0.125})()
+        for _ in range(9):
+            k, v, q = FORMS[form](x(1, 2, 1, 64)), FORMS[form](x(1, 2, 1, 64)), x(1, 8, 1, 64)
+            held, _ = layer.update(k, v)
+            outs.append(hira_attention_forward(module, as_query(q), held, None)[0].clone())
+        return torch.cat(outs), layer
+
+    want, a = run("ready")
+    got, b = run(form)
+    assert torch.equal(want, got) and torch.equal(a.samples, b.samples)
+    assert torch.equal(a.queued_keys, b.queued_keys) and torch.equal(a.queued_values, b.queued_values)
+    assert torch.equal(a.indexer.keys_buf, b.indexer.keys_buf) and torch.equal(a.indexer.perm, b.indexer.perm)
+    assert a.queued_len == b.queued_len and a.indexer.num_keys == b.indexer.num_keys
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_search_like_one_before_it(dtype, gpu_device):
+    x = _gen(5)
+    index = HIPIndexer(3, 1, 16).build(x(1, 2, 900, 64, dtype=dtype))
+    tau, sc = torch.tensor([3.0, 5.0, 8.0, 2.0]).cuda(), torch.tensor([1.0, 0.5, 2.0, 4.0]).cuda()
+    kept = HIPSearcher(output_fill_value=-7.0)
+
+    def fresh():
+        return HIPSearcher(output_fill_value=kept.output_fill_value, kernel=kept.launch.kernel)
+
+    for step in range(3):
+        q = x(4, 64, dtype=dtype)
+        for query in (q, q[None, :, None], _strided(q), q.double()):
+            for t, s in ((tau, None), (tau, sc), (4.0, None), (tau.double(), _strided(sc)), (_strided(tau), sc)):
+                assert torch.equal(kept.search(query, t, index, scaling=s), fresh().search(query, t, index, scaling=s))
+        assert torch.equal(kept.search(q[:2], tau[:2], index), fresh().search(q[:2], tau[:2], index))  # (other heads)
+        kept.output_fill_value += 1.5
+        if step == 0:
+            index.update(x(1, 2, 40, 64, dtype=dtype))  # (level sizes that moved)
+        else:
+            kept.launch = HIPSearcher(kernel=1).launch
+
+
+@pytest.mark.parametrize("form", ["strided", "fp32", "parameter"])
+@pytest.mark.parametrize("m", [1, 40])
+def test_an_append_and_its_read_back(form, m, gpu_device):
+    def run(form):
+        x = _gen(m)
+        index = HIPIndexer(3, 1, 16).build(x(1, 2, 700, 64), x(1, 2, 700, 64))
+        sizes = []
+        for _ in range(4):
+            index.update(FORMS[form](x(1, 2, m, 64)), FORMS[form](x(1, 2, m, 64)))
+            sizes.append(list(index.size))
+        index.update(FORMS[form](x(1, 2, 3, 64)), FORMS[form](x(1, 2, 3, 64)))
+        return index, sizes
+
+    (a, want), (b, got) = run("ready"), run(form)
+    assert want == got and a.size == b.size and a.num_keys == b.num_keys == 700 + 4 * m + 3
+    for l in range(1, 3):
+        assert torch.equal(a.radii[l], b.radii[l]) and torch.equal(a.counts[l], b.counts[l])
+    assert torch.equal(a.perm[:, :a.size[0]], b.perm[:, :b.size[0]]) and torch.equal(a.values_buf[:, :700], b.values_buf[:, :700])
+    assert a._host_rows is not None and b._host_rows is not None
