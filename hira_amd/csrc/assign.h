@@ -8,11 +8,11 @@
 namespace hira {
 
 // Bucketing fused into an assignment launch (counts NULL: the launch only assigns).
-//   counts  (T, K)       zero when the round starts; counts[a] += 1 for every item assigned to a.  The
+//   counts  (T, K), 1 << count_log2 apart  zero when the round starts; counts[a] += 1 for every item assigned to a.  The
 //                        value the item's increment returned is its place in the bucket:
 //   members (T, K, places)  the first `places` items of every bucket, in order of arrival, and
 //   dists   (T, K, places)  their distances (NULL: a Lloyd round, which asks for none)
-//   places_log2             bucket_places_log2 of the fan-out
+//   places_log2, count_log2 bucket_places_log2, bucket_count_log2 of the fan-out
 //   big     (T, K)       the buckets with more than kWaveBucket members, big_count (T) of them
 //   more    (T, n_c)     (centroid, item) of the items behind those, more_count (T) of them, their
 //   more_dist (T, n_c)   distances by item.  Such buckets are rare (a few seeds of a Lloyd round);
@@ -32,6 +32,10 @@ constexpr int kBucketCap = 256;
 constexpr int kWaveBucket = 64;
 static_assert(kWaveBucket == 1 << 6 && kBucketCap == 1 << 8, "bucket_places_log2");
 static inline int bucket_places_log2(int bf) { return bf <= 4 ? 6 : bf <= 8 ? 7 : 8; }
+// Counters of neighbouring buckets lie half a fan-out apart (its power of two): additions to one line of memory wait for each
+// other (9 ns each, and a round makes a fan-out of them for each of the counters in it).  Side by side, 32 a line: builds of 8 x 8192 keys 238.5
+// us, now 222.5, 8 x 4001 194 / 186, 8 x 20000 at a fan-out of 64 410 / 385, 8 x 32768 564 / 558.
+static inline int bucket_count_log2(int bf) { return bf <= 2 ? 0 : bf <= 4 ? 1 : bf <= 8 ? 2 : bf <= 16 ? 3 : bf <= 32 ? 4 : 5; }
 constexpr int kCounterStride = 32;
 struct AssignCounting {
     int32_t* counts;
@@ -45,7 +49,7 @@ struct AssignCounting {
     int32_t* lost;
     int32_t* lost_count;
     int32_t* zero;
-    int places_log2;
+    int places_log2, count_log2;
 };
 
 // item `it` of tree t was assigned to centroid k, at distance d (k < 0: to none)
@@ -55,7 +59,7 @@ __device__ __forceinline__ void count_item(const AssignCounting& ac, int t, int 
         return;
     }
     const size_t b = (size_t)t * K + k;
-    const int pos = atomicAdd(&ac.counts[b], 1);
+    const int pos = atomicAdd(&ac.counts[b << ac.count_log2], 1);
     if (pos == kWaveBucket) ac.big[(size_t)t * K + atomicAdd(&ac.big_count[t * kCounterStride], 1)] = k;
     if (pos < 1 << ac.places_log2) {
         ac.members[(b << ac.places_log2) + pos] = it;

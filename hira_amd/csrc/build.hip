@@ -60,7 +60,7 @@ template <typename T>
 __global__ __launch_bounds__(kNodeThreads) void k_level_init(
     const void* x, int n_c, size_t x_tree_stride, int K, int bf, int D, uint64_t seed, float* cent, const int32_t* n_live, int32_t* fill,
     int32_t* slots, int32_t* counts, int32_t* counters /* (kBuildCounters, T) */,
-    float* absmax /* (T, kAbsCopies, D) or NULL */, int Kt, CentroidTiles ct, int KS, int lanes) {
+    float* absmax /* (T, kAbsCopies, D) or NULL */, int Kt, CentroidTiles ct, int KS, int lanes, int count_log2) {
     constexpr int EPL = Elem<T>::kPerChunk, CH = 8 / EPL;
     const int t = blockIdx.x, lane = threadIdx.x & 63, j = lane % lanes;
     const int k = node_of_wave() * (64 / lanes) + lane / lanes, own = min(k, K - 1);
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(kNodeThreads) void k_level_init(
         for (int i = i0; i < kAbsCopies * D; i += stride) absmax[(size_t)t * kAbsCopies * D + i] = 0.0f;
     for (int i = i0; i < K; i += stride) {
         fill[(size_t)t * K + i] = i >= K_t ? bf : 0;
-        counts[(size_t)t * K + i] = 0;
+        counts[((size_t)t * K + i) << count_log2] = 0;
     }
     for (size_t i = i0; i < (size_t)K * bf; i += stride) slots[(size_t)t * K * bf + i] = -1;
     if (ct.tiles != nullptr) {
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(kSimpleThreads, 4) void k_assign_simple(const int32
 // 3. the buckets of a round: what the assignment left of it (assign.h)
 // ------------------------------------------------------------------------------------
 struct Buckets {
-    int32_t* counts;          // (T, K); every kernel here leaves it zero for the round after it
+    int32_t* counts;          // (T, K), 1 << count_log2 apart; every kernel here leaves it zero for the round after it
     const int32_t* members;   // (T, K, places)
     const float* dists;       // (T, K, places)
     const int32_t* big;       // (T, K)
@@ -262,7 +262,8 @@ struct Buckets {
     int32_t* next_big_count;    // (T): the round after this one counts here; cleared by these kernels
     int32_t* next_more_count;   // (T): the same
     int32_t* unsure_count;      // (T): cleared by these kernels
-    int places_log2;
+    int places_log2, count_log2;
+    __device__ int32_t& count(size_t b) const { return counts[b << count_log2]; }
     __device__ int places() const { return 1 << places_log2; }
     __device__ size_t first(size_t b) const { return b << places_log2; }  // place of bucket b (of all trees)
 };
@@ -326,7 +327,7 @@ __device__ __forceinline__ int pow2_at_least(int n) {
 // (behind a barrier: the count is read through the scalar cache, and only the wait there keeps this
 // store from overtaking it; a bucket's other reader finds a large count, or none, and leaves it)
 __device__ __forceinline__ void reset_count(const Buckets& b, int t, int k, int K) {
-    b.counts[(size_t)t * K + k] = 0;
+    b.count((size_t)t * K + k) = 0;
 }
 __device__ __forceinline__ void reset_round(const Buckets& b, int t) {  // (one thread of the tree)
     b.next_big_count[t * kCounterStride] = 0;
@@ -370,7 +371,7 @@ __global__ __launch_bounds__(kBucketThreads, 6) void k_bucket_mean(
         const int k = (block - large) * kWaves + wave;
         if (k >= K) return;
         uint32_t id = (uint32_t)bk.members[bk.first((size_t)t * K + k) + lane];  // (garbage from m on)
-        const int m = __builtin_amdgcn_readfirstlane(bk.counts[(size_t)t * K + k]);
+        const int m = __builtin_amdgcn_readfirstlane(bk.count((size_t)t * K + k));
         if (m <= 0 || m > kWaveBucket) return;
         if (lane >= m) id = 0xffffffffu;
         const int rank = wave_rank(id, m);
@@ -390,7 +391,7 @@ __global__ __launch_bounds__(kBucketThreads, 6) void k_bucket_mean(
     const int nbig = bk.big_count[t * kCounterStride];
     for (int i = block; i < nbig; i += large) {  // uniform
         const int k = bk.big[(size_t)t * K + i];
-        const int m = bk.counts[(size_t)t * K + k];
+        const int m = bk.count((size_t)t * K + k);
         const int32_t* mem = bk.members + bk.first((size_t)t * K + k);
         __syncthreads();
         if (tid == 0) reset_count(bk, t, k, K);
@@ -541,7 +542,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
         if (k < K) {
             const size_t b = (size_t)t * K + k;
             mine = key_of(bk.dists[bk.first(b) + lane], bk.members[bk.first(b) + lane]);  // (garbage from m on)
-            m = __builtin_amdgcn_readfirstlane(bk.counts[b]);
+            m = __builtin_amdgcn_readfirstlane(bk.count(b));
             f = __builtin_amdgcn_readfirstlane(fill[b]);
             if (m > kWaveBucket) m = 0;
             take = max(min(m, bf - f), 0);
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(kBucketThreads) void k_bucket_accept(
     for (int i = block; i < nbig; i += large) {  // uniform
         const int k = bk.big[(size_t)t * K + i];
         const size_t b = (size_t)t * K + k;
-        const int m = bk.counts[b], f = fill[b];
+        const int m = bk.count(b), f = fill[b];
         const int32_t* mem = bk.members + bk.first(b);
         const float* md = bk.dists + bk.first(b);
         const float* more_d = bk.more_dist + (size_t)t * n_c;
@@ -996,7 +997,7 @@ static void carve(const HiraTree* t, int n, void* ws, BuildWs* b) {
     b->list[0] = c.take<int32_t>((size_t)T * n);
     b->list[1] = c.take<int32_t>((size_t)T * n);
     b->counters = c.take<int32_t>((size_t)T * kBuildCounters * kCounterStride);
-    b->counts = c.take<int32_t>((size_t)T * k1);
+    b->counts = c.take<int32_t>((size_t)T * k1 << bucket_count_log2(bf));
     b->fill = c.take<int32_t>((size_t)T * k1);
     for (int l = 0; l < HIRA_MAX_LEVELS; ++l) {
         b->slots[l] = nullptr;
@@ -1103,13 +1104,13 @@ static int cluster_levels(const HiraTree* t, const void* keys_in, int n, const i
         while (lanes * 8 < D || (on_mfma && lanes < KS * 4)) lanes <<= 1;
         hipLaunchKernelGGL((k_level_init<T>), node_grid(ceil_div(Kl, 64 / lanes), NT), dim3(kNodeThreads), 0, s, x, n_c, xs, Kl, bf, D,
                            seed + 7919ull * (uint64_t)l, w.cent_f32, ragged ? n_live : nullptr, w.fill, w.slots[l], w.counts, w.counters,
-                           l == 1 ? w.absmax : nullptr, Kt, tiles, KS, lanes);
+                           l == 1 ? w.absmax : nullptr, Kt, tiles, KS, lanes, bucket_count_log2(bf));
         // a round: the assignment (which also puts the items into buckets), then what the round does
         // with every bucket.  A Lloyd round asks for no distances.
         auto buckets = [&]() {
             const int now = round & 1, next = now ^ 1;
             return Buckets{w.counts, w.members, w.dists, w.big, big_count + now * ct, w.more, more_count + now * ct,
-                           w.more_dist, big_count + next * ct, more_count + next * ct, unsure_count, bucket_places_log2(bf)};
+                           w.more_dist, big_count + next * ct, more_count + next * ct, unsure_count, bucket_places_log2(bf), bucket_count_log2(bf)};
         };
         auto assign_round = [&](const int32_t* list, const int32_t* lcnt, const int32_t* fill, bool packing,
                                 int32_t* zero, bool only_open, long long expected) -> int {
@@ -1128,7 +1129,7 @@ static int cluster_levels(const HiraTree* t, const void* keys_in, int n, const i
             job.list_count = lcnt;
             job.counting = AssignCounting{w.counts, w.members, packing ? w.dists : nullptr, w.big,
                                           big_count + (round & 1) * ct, w.more, more_count + (round & 1) * ct, w.more_dist, w.lost, lost_count, zero,
-                                          bucket_places_log2(bf)};
+                                          bucket_places_log2(bf), bucket_count_log2(bf)};
             job.unsure = w.unsure;
             job.unsure_count = unsure_count;
             int rc = HIRA_OK;
