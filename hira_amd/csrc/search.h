@@ -105,6 +105,7 @@ struct SearchPlan {
     int num_nodes, num_queue_blocks;
     int tree_blocks, queue_blocks, head_chunks;
     int ahead;        // > 0: keys are asked for together with the gates' operands (vector-ALU kernel: as many elements a lane)
+    int slices;       // MFMA kernel, attention alone: workgroups that may share a tile where keys are asked for ahead
     size_t smem;
 };
 
@@ -119,6 +120,20 @@ bool mfma_search_supported(const HiraTree* t, const HiraQueue* queue);
 constexpr int kMfmaThreads = 512;       // workgroup size of the MFMA kernel (8 waves), at most
 constexpr int kMfmaMaxTilesPerWg = 16;  // tiles of 16 level-1 nodes one workgroup walks, at most
 int launch_search_mfma(const SearchPlan& plan, const SearchParams& p, dim3 grid, hipStream_t s);
+
+// MFMA kernel, rows of 32 KS columns, nodes of MT key tiles, GS heads a pass: nodes whose key tiles one wave keeps in
+// flight: what the budget of 256 registers leaves after twice the accumulators (GS x D/64) and some seventy registers of
+// everything else (8-bit shadow: 64 registers, beside which a batch of rows fits without spills; ten of them with outputs at fan-out 64
+// and eight heads, where lists take 21 us for 26 before the scan had two phases), and what keeps the round's list under
+// 48 KiB of LDS
+constexpr int mfma_round_nodes(int KS, int MT, int GS, bool q8) {
+    const int by_registers = (q8 ? 64 : 256 - 72 - 2 * GS * (KS / 2)) / (MT * (q8 ? KS / 2 : KS) * 4);
+    const int by_lds = (12000 / (GS + 1)) / (kMfmaThreads / 64 * MT * 16);
+    const int fit = q8 || by_registers < by_lds ? by_registers : by_lds;
+    return fit < 1 ? 1 : fit > (q8 ? 8 : 4) ? (q8 ? 8 : 4) : fit;
+}
+// nodes of a wave where key tiles are asked for ahead of the gates: a tile's 16 over 8 waves
+constexpr int kAheadNodes = 16 / (kMfmaThreads / 64);
 
 // Hand-off of the attention partials from the workgroups of a tree to the one that folds them
 // (maybe behind another L2).  The partials are written with device-scope atomic stores: they

@@ -89,7 +89,8 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
             HIRA_CHECK_ARG(t->cap[l] % 16 == 0, "tiled layout: cap[%d]=%d not a multiple of 16",
                            l, t->cap[l]);
     }
-    plan->ahead = false;
+    plan->ahead = 0;
+    plan->slices = 1;
     plan->nodes_per_wg = plan->queue_nodes = 0;
     plan->num_queue_blocks = 0;
     if (queue && queue->keys && queue->len > 0) {
@@ -162,8 +163,21 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
         // rows / of boosted channels, whose balls prune half: 4 MiB of keys 11.3 -> 9.9 / 12.2 -> 10.9 us
         // (indexes taking turns), 16 MiB 12.9 -> 11.4 / 13.0 -> 11.7, 24 MiB 14.5 -> 12.9 / 14.0 -> 12.5;
         // 32 MiB in 32 trees 13.8 -> 12.7 / 12.8 -> 13.1
-        plan->ahead = plan->threads == kMfmaThreads && plan->nodes_per_wave == 1 &&
-                      (size_t)t->num_trees * (size_t)t->size[0] * (size_t)t->dim * 2 <= ((size_t)28 << 20);
+        if (plan->threads == kMfmaThreads && plan->nodes_per_wave == 1 &&
+            (size_t)t->num_trees * (size_t)t->size[0] * (size_t)t->dim * 2 <= ((size_t)28 << 20))
+            plan->ahead = kAheadNodes;
+        // Two to four tiles a tree leave most of the chip idle, and where a tile's keys are 128 KiB or more a compute unit's
+        // L1 takes longer for them (0.9 us) than the trip to memory: two workgroups then share a tile, a node of it a wave.  8 trees x
+        // 4 heads, 128 columns, a fan-out of 32: 2000 keys 9.23 -> 8.73 us, 1000 9.10 -> 8.44; a fan-out of 64: 3000 keys 12.0 -> 10.5.
+        // With more tiles the fold of twice the partials takes what that gives (4001 keys 9.40 -> 9.74), a tile alone
+        // would have a fold at all (500 keys 7.7 -> 8.5), smaller tiles are there soon enough (64 columns, a fan-out of 16: 8.0 -> 8.55),
+        // more workgroups that wait for thresholds are no help (2000 keys 11.5 -> 11.9), nor are they where they would take
+        // more than half of the chip (16 trees, 2000 keys: 9.41 -> 9.56).
+        const int mt = (t->bf + 15) / 16, gs = plan->gmax <= 4 ? 4 : plan->gmax <= 8 ? 8 : 16;
+        if (plan->ahead && tiles >= 2 && tiles <= 4 && t->bf * t->dim >= 4096 && t->layout == HIRA_TILE16 && t->dim <= 128 &&
+            mfma_round_nodes(t->dim / 32, mt <= 2 ? mt : 4, gs, false) >= kAheadNodes && !(launch && launch->nodes_per_wave) &&
+            (int64_t)(tiles * kAheadNodes + 1) * t->num_trees * plan->head_chunks * 2 <= compute_units())
+            plan->slices = kAheadNodes;
         plan->queue_blocks = plan->num_queue_blocks > 0 ? 1 : 0;  // one workgroup takes the whole queue
         plan->smem = 0;
         // every workgroup that walks the tree must own at least one tile: one without a tile
@@ -251,7 +265,7 @@ extern "C" size_t hira_search_workspace_bytes(const HiraTree* tree, const HiraQu
                                               const HiraLaunch* launch) {
     SearchPlan plan;
     if (make_plan(tree, query, queue, launch, true, &plan) != HIRA_OK) return 0;
-    const size_t P = (size_t)plan.tree_blocks + plan.queue_blocks;
+    const size_t P = (size_t)plan.tree_blocks * plan.slices + plan.queue_blocks;
     return counter_bytes(tree->num_trees, plan.head_chunks) + partial_bytes(query->num_q_heads, P, tree->vdim);
 }
 
@@ -289,6 +303,11 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
     const bool attn = out->attn_out != nullptr;
     int rc = make_plan(tree, query, queue, launch, attn, &plan);
     if (rc != HIRA_OK) return rc;
+    // (with outputs of another kind the keys are not asked for ahead)
+    if (plan.slices > 1 && attn && out->dense == nullptr && out->sel_count == nullptr && !(sample && sample->scratch)) {
+        plan.ahead = kAheadNodes / plan.slices;
+        plan.tree_blocks *= plan.slices;
+    }
     if (attn) {
         HIRA_CHECK_ARG(tree->values != nullptr && tree->vdim > 0,
                        "attention needs values in the tree");

@@ -206,17 +206,7 @@ struct MfmaShape {
     static constexpr int D = 32 * KS;
     static constexpr int ROWS = MT * 16;  // key slots of one node
     static constexpr int KA = Q8 ? KS / 2 : KS;  // 16-byte chunks a lane holds of a scanned tile
-    // nodes whose key tiles one wave keeps in flight: what the budget of 256 registers leaves
-    // after twice the accumulators (GS x D/64) and some seventy registers of everything else
-    // (8-bit shadow: 64 registers, beside which a batch of rows fits without spills; ten of them with outputs at fan-out 64
-    // and eight heads, where lists take 21 us for 26 before the scan had two phases), and what keeps the round's list under
-    // 48 KiB of LDS
-    static constexpr int KEY_REGS = Q8 ? 64 : 256 - 72 - 2 * GS * (KS / 2);
-    static constexpr int NB_REGS = KEY_REGS / (MT * KA * 4);
-    static constexpr int NB_LDS = (12000 / (GS + 1)) / (kMfmaWaves * ROWS);
-    static constexpr int NB_MIN = Q8 || NB_REGS < NB_LDS ? NB_REGS : NB_LDS;
-    static constexpr int NB_MAX = Q8 ? 8 : 4;
-    static constexpr int NB = NB_MIN < 1 ? 1 : (NB_MIN > NB_MAX ? NB_MAX : NB_MIN);
+    static constexpr int NB = mfma_round_nodes(KS, MT, GS, Q8);
     static constexpr int LIST = kMfmaWaves * NB * ROWS;  // rows of the list of one round
     // 8-bit shadow: rows that a wave lists before the workgroup looks at them, and the rounds that never list more;
     // a batch of rows: its scores, key slots and list entries
@@ -293,9 +283,6 @@ __device__ __forceinline__ void gate_issue(const GateArgs& p, int tree, int t1, 
     }
 }
 
-// nodes of a wave of the instantiations that ask for key tiles ahead of the gates: a tile's 16 over 8 waves
-constexpr int kAheadNodes = 16 / kMfmaWaves;
-
 // OUT: the launch also wants dense scores or selection lists (kept out of the attention-only
 // instantiation, whose registers are all spoken for).
 // Q8: the index keeps an 8-bit shadow of its keys (HIRA_TILE16_Q8).  The scan then reads the
@@ -310,13 +297,14 @@ constexpr int kAheadNodes = 16 / kMfmaWaves;
 // everything asked for so far.
 // AHEAD: (small launches) a workgroup owns one tile, and its waves ask for the key tiles of their two
 // nodes each together with the gates' operands, whether the nodes survive or not: a trip to memory less,
-// and no list of survivors.
+// and no list of survivors.  As a number: the nodes of a wave; with one, two workgroups share a tile (SearchPlan.slices).
 // SAMPLED: (with AHEAD) the launch makes its thresholds itself, in workgroups ahead of the searching ones.
-template <int KS, int MT, int GS, bool OUT, bool Q8, int POL, int HV, bool ONE, bool AHEAD = false, bool SAMPLED = false>
+template <int KS, int MT, int GS, bool OUT, bool Q8, int POL, int HV, bool ONE, int AHEAD = 0, bool SAMPLED = false>
 __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const SearchParams p) {
     using S = MfmaShape<KS, MT, GS, Q8>;
     constexpr int D = S::D;
-    constexpr int NB = AHEAD ? kAheadNodes : S::NB;
+    constexpr int NB = AHEAD ? AHEAD : S::NB;
+    constexpr int SLICES = AHEAD ? kAheadNodes / AHEAD : 1;  // workgroups that share a tile
     static_assert(!AHEAD || (ONE && !OUT && !Q8 && HV == 1 && NB <= S::NB), "");
     constexpr int KA = S::KA;          // 16-byte chunks per lane of a scanned tile
     constexpr int KS8 = Q8 ? KS / 2 : 1;
@@ -369,8 +357,8 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
     // apart, since neighbouring tiles hold sibling nodes, which tend to survive (and be selected
     // from) together.
     const int wg_tiles = (ga.size + 15) >> 4;
-    const int n_groups = ga.tree_blocks;
-    const int grp = wg;
+    const int n_groups = ga.tree_blocks / SLICES;
+    const int grp = wg / SLICES, slice = wg % SLICES;
     const int ntile = wg < ga.tree_blocks
                           ? min(ga.tiles, (wg_tiles - grp + n_groups - 1) / n_groups)
                           : 0;
@@ -522,7 +510,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                 for (int tt = 0; tt < MT; ++tt)
                     load_tile_buf<KA, POL != 0>(
                         rsrc, (unsigned)lane * 16u,
-                        ((unsigned)(node_of(u * kMfmaWaves + wave) * bf) / 16u + tt) * (unsigned)(KA * 1024), a[u][tt]);
+                        ((unsigned)(node_of((slice * NB + u) * kMfmaWaves + wave) * bf) / 16u + tt) * (unsigned)(KA * 1024), a[u][tt]);
         }
         __builtin_amdgcn_sched_barrier(0);  // (nothing that uses a load moves above this line)
         tline.stamp(kTlGateIssued);
@@ -648,7 +636,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
                     }
                 }
             }
-            const bool count_nodes = stats != nullptr && lane == 0;
+            const bool count_nodes = stats != nullptr && lane == 0 && slice == 0;
             int lcur = L - 1;
             bool chain = head_ok;  // this head is still alive above the current level
             // the tile's ancestor at level l; is the tile's first node its first descendant?
@@ -821,7 +809,7 @@ __global__ __launch_bounds__(64 * kMfmaWaves, 2) void search_mfma_kernel(const S
         if constexpr (AHEAD) {
 #pragma unroll
             for (int u = 0; u < NB; ++u) {
-                const int n = u * kMfmaWaves + wave;
+                const int n = (slice * NB + u) * kMfmaWaves + wave;
                 const uint32_t info = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_ninfo[n]);
                 nx_node[u] = n;
                 nx_half[u] = 0;
@@ -1751,12 +1739,18 @@ void launch_mfma_one(const SearchPlan& plan, const SearchParams& p, dim3 grid, h
     if constexpr (!Q8 && POL == 0 && HV == 1 && KS <= 4 && MfmaShape<KS, MT, GS>::NB >= kAheadNodes) {
         if constexpr (MT <= kSampledTiles) {
             if (plan.ahead && p.sample_wgs > 0) {
-                hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, false, 0, 1, true, true, true>), grid, block, 0, s, p);
+                hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, false, 0, 1, true, kAheadNodes, true>), grid, block, 0, s, p);
+                return;
+            }
+        }
+        if constexpr (KS * MT >= 8) {  // (tiles of 128 KiB)
+            if (plan.ahead == kAheadNodes / 2) {
+                hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, false, 0, 1, true, kAheadNodes / 2>), grid, block, 0, s, p);
                 return;
             }
         }
         if (plan.ahead) {
-            hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, false, 0, 1, true, true>), grid, block, 0, s, p);
+            hipLaunchKernelGGL((search_mfma_kernel<KS, MT, GS, false, false, 0, 1, true, kAheadNodes>), grid, block, 0, s, p);
             return;
         }
     }

@@ -566,3 +566,51 @@ def test_small_trees_on_the_matrix_cores(t, g, n, d, bf, nl, m, gpu_device):
     stats = torch.zeros((t, 11), dtype=torch.int64, device="cuda")
     fused.search_attention(*args, **kw, stats=stats)
     assert int(stats[:, 8].sum()) == int(sel[..., :n].any(dim=1).sum())
+
+
+@pytest.mark.parametrize("t,g,n,d,bf,nl,m", [
+    (2, 4, 600, 128, 32, 3, 0),      # two tiles, the second with three nodes in use
+    (2, 4, 1030, 128, 32, 2, 5),     # three, one node in the last, and the queue's
+    (1, 7, 2048, 128, 32, 3, 0),     # four, all nodes full, eight heads' registers
+    (8, 3, 2000, 128, 32, 3, 16),
+    (2, 16, 1100, 128, 32, 3, 0),    # sixteen heads
+    (14, 4, 2000, 128, 32, 2, 0),    # most of the trees that still leave half of the chip
+    (15, 4, 2000, 128, 32, 2, 0),    # too many: a workgroup a tile
+    (2, 4, 1100, 64, 64, 2, 3),      # nodes of four key tiles
+    (2, 8, 4000, 128, 64, 3, 0),
+    (2, 4, 2100, 128, 48, 2, 0),     # three
+    (1, 20, 2000, 128, 32, 3, 0),    # two passes of heads
+])
+def test_workgroups_that_share_a_tile(t, g, n, d, bf, nl, m, gpu_device):
+    """Launches of two to four tiles a tree against launches that give every tile one workgroup: the counters are
+    the same, the outputs differ by the order of their sums."""
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    print(f"case {t} {g} {n} {d} {bf} {nl} {m}", flush=True)
+    gen = torch.Generator().manual_seed(n + g)
+    K = torch.randn(1, t, n, d, generator=gen).bfloat16().cuda()
+    V = torch.randn(1, t, n, d, generator=gen).bfloat16().cuda()
+    q = torch.randn(t * g, d, generator=gen).bfloat16().cuda()
+    s = torch.matmul(q.float().reshape(t, g, d), K[0].float().transpose(1, 2).contiguous())
+    tau = s.topk(max(2, n // 60), dim=-1).values[..., -1]
+    tau[0, 0] = 1e9            # a head that selects nothing,
+    tau[-1, -1] = -1e9         # one that selects every key,
+    tau[0, -1] = float("nan")  # and one that compares with nothing
+    idx = HIPIndexer(nl, 1, bf).build(K, V)
+    kw = dict(scaling=torch.full((t * g,), d ** -0.5, device="cuda"))
+    if m:
+        kw.update(queue_keys=torch.randn(t, m, d, generator=gen).bfloat16().cuda(),
+                  queue_values=torch.randn(t, m, d, generator=gen).bfloat16().cuda())
+    out, stats = [], []
+    for se in (HIPSearcher(kernel=2), HIPSearcher(kernel=2, separate_merge=True), HIPSearcher(kernel=2, nodes_per_wave=1)):
+        for _ in range(2):  # (the counters of arrivals are back at zero)
+            stats.append(torch.zeros((t, 11), dtype=torch.int64, device="cuda"))
+            out.append(se.search_attention(q, tau.reshape(-1), idx, stats=stats[-1], **kw))
+    ref, counts = out[-1].double(), stats[-1]
+    # (fp32 sums of at most a few thousand terms of a convex combination, in two orders)
+    den = ref.abs().amax(1, keepdim=True).clamp_min(1e-30)
+    for a, c in zip(out, stats):
+        assert torch.equal(c, counts)
+        assert torch.equal(a.isnan(), ref.isnan())
+        assert float(((a.double() - ref).abs() / den).nan_to_num(0.0).max()) <= 4e-6
