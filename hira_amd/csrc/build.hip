@@ -1166,8 +1166,14 @@ static int cluster_levels(const HiraTree* t, const void* keys_in, int n, const i
             const int32_t* lcnt = r == 0 ? nullptr : list_count + (r & 1) * ct;
             int32_t* next_cnt = list_count + ((r + 1) & 1) * ct;
             // (from the second round on most blocks are full: the assignment then sees only the
-            // centroids with room, side by side; worth its launch from 32 tiles on)
-            const int rc = assign_round(list, lcnt, w.fill, true, next_cnt, r >= 1 && Kl >= 512, all_items >> r);
+            // centroids with room, side by side; worth its launch from 32 tiles on, and where rows are of 64 columns, whose products
+            // with the full ones take half as long and leave the registers to twice the waves, only where the list may be long:
+            // builds of 64 columns with the launch in all rounds / by this rule: 2 x 9600 keys at a fan-out of 16 247 / 229 us,
+            // 2 x 16001 274 / 258, 1 x 24000 304 / 296, 8 x 16001 365 / 358, 8 x 30000 at 32 412 / 404; without it in all rounds
+            // 8 x 30000 412, 8 x 60000 762 -> 816, 2 x 60011 at 16 575 -> 585 without it in the last four; of 128 columns
+            // 8 x 32768 without it from the fifth round on 572 -> 575)
+            const bool side_by_side = r >= 1 && Kl >= 512 && (KS > 2 || Kl > 2048 || (all_items >> r) * Kl > 25ll * 1000 * 1000);
+            const int rc = assign_round(list, lcnt, w.fill, true, next_cnt, side_by_side, all_items >> r);
             if (rc != HIRA_OK) return rc;
             hipLaunchKernelGGL(k_bucket_accept, g_bucket, dim3(kBucketThreads), 0, s, buckets(), n_c, Kl, bf,
                                w.fill, w.slots[l], w.list[(r + 1) & 1], next_cnt, Kt, tiles.n2, large);

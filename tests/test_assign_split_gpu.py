@@ -17,6 +17,8 @@ pytestmark = pytest.mark.gpu
     (60, 1985, 64, 8),     # 249: more sets than waves fit
     (130, 1025, 128, 16),  # 65: one wave to 64 items, from the first round on
     (70, 545, 256, 8),     # 69, sets of 32
+    (2, 4161, 64, 8),      # 521: later rounds of the packing walk the full ones too
+    (3, 12001, 64, 8),     # 1501: only from the third on
 ])
 def test_waves_that_share_items(trees, n, d, bf, gpu_device):
     from hira_amd.indexer.hip import HIPIndexer
