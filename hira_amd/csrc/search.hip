@@ -207,11 +207,20 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
         // one block each
         const int rows = t->num_levels >= 2 ? t->bf : kPseudoBlock;
         const int64_t all = (int64_t)plan->num_nodes * t->num_trees * plan->head_chunks;
-        const int64_t wgs = (attn ? 1 : 2) * compute_units();
-        int64_t per = (all + wgs - 1) / wgs;
         const int64_t least = (128 + rows - 1) / rows;
-        if (per < least) per = least;
-        npw = (int)((per + waves - 1) / waves);
+        auto waves_nodes = [&](int64_t wgs) {
+            int64_t per = (all + wgs - 1) / wgs;
+            if (per < least) per = least;
+            return (int)((per + waves - 1) / waves);
+        };
+        npw = waves_nodes((attn ? 1 : 2) * compute_units());
+        // (a compute unit for every tree's queue too: with one workgroup more than there are places, one of those that search
+        // began when the others were done.  us, the tree alone / with a queue / with its place kept: 16 trees x 19889 rows of 96
+        // bf16, seven heads 75 / 126 / 80, four 35 / 59 / 38, one 26 / 41 / 28; 8 trees x 5003, three heads 14.6 / 18.9 / 17.0)
+        const int64_t queues = (int64_t)t->num_trees * plan->head_chunks;
+        const int64_t wgs = ((plan->num_nodes + waves * npw - 1) / (waves * npw) + 1) * queues;
+        if (attn && plan->num_queue_blocks > 0 && wgs > compute_units() && 2 * queues <= compute_units())
+            npw = waves_nodes(compute_units() - queues);
     }
     plan->nodes_per_wg = plan->queue_nodes = waves * npw;
     if (t->num_levels >= 2 && threads == kVecThreads && !(launch && launch->nodes_per_wave)) {
@@ -263,9 +272,10 @@ static size_t partial_bytes(int h_q, size_t P, int vdim) { return (size_t)h_q * 
 extern "C" size_t hira_search_workspace_bytes(const HiraTree* tree, const HiraQuery* query,
                                               const HiraQueue* queue,
                                               const HiraLaunch* launch) {
-    SearchPlan plan;
-    if (make_plan(tree, query, queue, launch, true, &plan) != HIRA_OK) return 0;
-    const size_t P = (size_t)plan.tree_blocks * plan.slices + plan.queue_blocks;
+    SearchPlan plan, alone;  // (a queue may take room from the tree's workgroups: the workspace holds the partials with it and without)
+    if (make_plan(tree, query, queue, launch, true, &plan) != HIRA_OK || make_plan(tree, query, nullptr, launch, true, &alone) != HIRA_OK) return 0;
+    const size_t with = (size_t)plan.tree_blocks * plan.slices + plan.queue_blocks, without = (size_t)alone.tree_blocks * alone.slices;
+    const size_t P = with > without ? with : without;
     return counter_bytes(tree->num_trees, plan.head_chunks) + partial_bytes(query->num_q_heads, P, tree->vdim);
 }
 

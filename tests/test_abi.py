@@ -141,6 +141,21 @@ def test_launch_plan_fills_the_compute_units():
     assert _partials_per_head(128, 32768, 4) == 4           # several rounds: 16 tiles a workgroup
 
 
+@pytest.mark.parametrize("trees,nodes", [(50, 300), (16, 1280), (8, 352), (130, 75), (1, 5000)])
+def test_a_workspace_for_a_queue_serves_calls_without_one(trees, nodes):
+    """A queue may take room from the workgroups that search, and leave fewer partials than there are without it."""
+    lib, dummy = _lib.lib(), ctypes.c_void_p(4096)
+    t = _lib.HiraTree()
+    t.num_trees, t.num_levels, t.bf, t.dim, t.vdim, t.dtype = trees, 2, 4, 32, 32, _lib.HIRA_F32
+    t.size[0], t.size[1], t.cap[0], t.cap[1] = nodes * 4, nodes, nodes * 4, nodes
+    t.keys = t.values = t.perm = t.centers[1] = t.radii[1] = t.counts[1] = dummy
+    q = _lib.HiraQuery(trees * 2, dummy, dummy, dummy, dummy, dummy, 2, 2)
+    alone = lib.hira_search_workspace_bytes(ctypes.byref(t), ctypes.byref(q), None, None)
+    sizes = [lib.hira_search_workspace_bytes(ctypes.byref(t), ctypes.byref(q), ctypes.byref(_lib.HiraQueue(4096, 4096, rows, 1024)), None)
+             for rows in (1, 64, 65, 1024)]
+    assert 0 < alone <= sizes[0] and sizes == sorted(sizes), (alone, sizes)
+
+
 @pytest.mark.parametrize("bf", [1, 2, 4, 8, 10, 16, 32, 64])
 @pytest.mark.parametrize("dtype,dim", [(_lib.HIRA_F32, 36), (_lib.HIRA_BF16, 128)])
 def test_build_workspace_follows_the_number_of_keys(bf, dtype, dim):

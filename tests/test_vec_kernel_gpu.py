@@ -62,6 +62,17 @@ def test_workgroup_shapes(threads, npw, gpu_device):
     _check(2500, 80, torch.float32, 3, 7, 4, seed=threads + npw, queue=33, block_threads=threads, nodes_per_wave=npw)
 
 
+@pytest.mark.parametrize("trees,n,d,levels,bf,group,queue", [
+    (50, 1200, 32, 2, 4, 2, 1),     # 250 workgroups for the trees, or 200 and 50 for the queues
+    (50, 1200, 32, 2, 4, 2, 130),   # three blocks of queued rows, one workgroup
+    (8, 5003, 96, 4, 16, 3, 33),
+    (130, 300, 16, 2, 4, 1, 64),    # no place to keep: more queues than half of the compute units
+])
+def test_a_place_for_every_queue(trees, n, d, levels, bf, group, queue, gpu_device):
+    print(f"case trees={trees} n={n} d={d} queue={queue}", flush=True)
+    _check(n, d, torch.bfloat16 if d == 96 else torch.float32, levels, bf, group, seed=n + queue, queue=queue, trees=trees)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_first_call_on_an_index_may_be_captured(dtype, gpu_device):
     """No scale given, another index than the call before (same heads): nothing comes from the host."""
