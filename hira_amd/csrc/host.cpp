@@ -293,17 +293,22 @@ PyObject* draw(PyObject*, PyObject* const* a, Py_ssize_t n) {
         PyErr_Format(PyExc_ValueError, "draw: a sample of %lld members", (long long)members);
         return nullptr;
     }
-    const bool wide = c10::get_default_dtype_as_scalartype() == at::kDouble;
+    const at::ScalarType type = c10::get_default_dtype_as_scalartype();
     std::vector<int64_t> who;
     std::vector<std::pair<int64_t, int64_t>> pairs;
     {
         std::lock_guard<std::mutex> lock(g->mutex_);
-        at::uniform_real_distribution<float> narrow_share(0, 1);
-        at::uniform_real_distribution<double> wide_share(0, 1);
-        for (int64_t i = 0; i < m; ++i) {
-            const double u = wide ? wide_share(g) : (double)narrow_share(g);
-            if (u < (double)members / (double)(seen + i + 1)) who.push_back(first + i);
-        }
+        auto shares = [&](auto zero) {
+            using Share = decltype(zero);
+            at::uniform_real_distribution<Share> share(0, 1);
+            for (int64_t i = 0; i < m; ++i)
+                if ((double)static_cast<Share>(share(g)) < (double)members / (double)(seen + i + 1)) who.push_back(first + i);
+        };
+        // (torch.rand's type is the default type, which a program that loads a model in 16 bits may have set to that)
+        if (type == at::kDouble) shares(double());
+        else if (type == at::kBFloat16) shares(at::BFloat16());
+        else if (type == at::kHalf) shares(at::Half());
+        else shares(float());
         at::uniform_int_from_to_distribution<int64_t> member(members, 0);
         std::unordered_map<int64_t, size_t> place;
         for (const int64_t key : who) {

@@ -16,9 +16,9 @@ def _draw(gen, m, first, members, seen):
     return tuple(last.keys()), tuple(last.values())
 
 
-@pytest.mark.parametrize("wide", [False, True])
-def test_the_numbers_of_torch(wide):
-    torch.set_default_dtype(torch.float64 if wide else torch.float32)
+@pytest.mark.parametrize("default", [torch.float32, torch.float64, torch.bfloat16, torch.float16])
+def test_the_numbers_of_torch(default):
+    torch.set_default_dtype(default)
     try:
         a, b = torch.Generator().manual_seed(3), torch.Generator().manual_seed(3)
         for m, first, members, extra in [(1, 0, 1000, 0), (1, 0, 1, 5000), (15, 1, 7, 3), (16, 0, 4096, 10), (700, 2, 33, 100),
