@@ -828,23 +828,34 @@ void search_kernel(const SearchParams p) {
         // ---- gates: rows of levels 1 and 2 over all waves, every level above on a wave of its own ----
         if (real_nodes) {
             constexpr int KA = 4;  // level-1 rows a lane group has in flight
-            const int r0 = wave * RPW + rg, rstep = nwaves * RPW;
-            auto ask = [&](int l, int first, int rows, int r, uint4& raw, float& rad) {
-                raw = make_uint4(0, 0, 0, 0);
-                rad = -INFINITY;
-                if (r < rows) {
+            const int rb0 = wave * RPW, rstep = nwaves * RPW;
+            // A lane group's row of those that the wave asks for, from number rb on, the last one again where there is none.  (Under a
+            // condition of the lanes' own every row held registers of zeros, and level 2 was asked for when level 1 had arrived.
+            // Searches of 8 x 60000 rows of 128 fp32 27.1 -> 26.6 us, 8 x 20000 15.1 -> 14.75, 8 x 90000 bf16 at a fan-out of 8 25.0 ->
+            // 24.55; attention over 16 trees x 19889 x 96 bf16, seven heads 64.4 -> 61.6, 4 x 30000 x 32 at a fan-out of 4, eight
+            // heads 27.8 -> 25.4: these were short of registers.)
+            auto ask = [&](int l, int first, int rows, int rb, uint4& raw, float& rad) {
+                if (rb < rows) {  // uniform in the wave
                     const size_t t0 = (size_t)tree * p.cap[l];
-                    if (chunk_ok) raw = load_row_chunk<T>(p.centers[l], p.layout, D, t0, first + r, ch);
-                    rad = p.radii[l][t0 + first + r];
+                    const int row = first + min(rb + rg, rows - 1);
+                    raw = load_row_chunk<T>(p.centers[l], p.layout, D, t0, row, chunk_ok ? ch : 0);
+                    rad = p.radii[l][t0 + row];
                 }
             };
-            uint4 raw1[KA], raw2;
-            float rad1[KA], rad2;
+            uint4 raw1[KA], raw2 = make_uint4(0, 0, 0, 0);
+            float rad1[KA], rad2 = 0.0f;
 #pragma unroll
-            for (int k = 0; k < KA; ++k) ask(1, n0, nb, r0 + k * rstep, raw1[k], rad1[k]);
+            for (int k = 0; k < KA; ++k) {
+                raw1[k] = raw2, rad1[k] = rad2;
+                ask(1, n0, nb, rb0 + k * rstep, raw1[k], rad1[k]);
+            }
             const int first2 = (int)over_bf((unsigned)n0);
             const int rows2 = L > 2 ? (int)over_bf((unsigned)(n0 + nb - 1)) - first2 + 1 : 0;
-            ask(2, first2, rows2, r0, raw2, rad2);
+            ask(2, first2, rows2, rb0, raw2, rad2);
+            __builtin_amdgcn_sched_barrier(0);  // (nothing that uses a load moves above this line)
+            // (nor do the queries' norms leave the loop, to be waited for ahead of it)
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) asm volatile("" : "+v"(qraw[g].x), "+v"(qraw[g].y), "+v"(qraw[g].z), "+v"(qraw[g].w));
             float qn[GMAX];
 #pragma unroll
             for (int g = 0; g < GMAX; ++g) {
@@ -855,28 +866,30 @@ void search_kernel(const SearchParams p) {
                 for (int e = 0; e < EPL; ++e) ss += qf[e] * qf[e];
                 qn[g] = sqrtf(group_sum<LPR>(ss));
             }
-            auto judge = [&](int l, int rows, int r, const uint4& raw, float rad) {
+            auto judge = [&](int l, int rows, int rb, const uint4& raw, float rad) {
+                const int r = rb + rg;
+                const uint4 x = chunk_ok ? raw : make_uint4(0, 0, 0, 0);
                 unsigned pass = 0;
 #pragma unroll
                 for (int g = 0; g < GMAX; ++g) {
-                    const float d = group_sum<LPR>(vec_dot<T>(raw, qraw[g]));
+                    const float d = group_sum<LPR>(vec_dot<T>(x, qraw[g]));
                     if (d + qn[g] * rad >= tau[g]) pass |= 1u << g;
                 }
                 if (ch == 0 && r < rows) s_pass[l][r] = pass | (rad > -INFINITY ? 0x80000000u : 0u);
             };
-            if (wave * RPW < rows2) judge(2, rows2, r0, raw2, rad2);  // (conditions: uniform in the wave)
+            if (rb0 < rows2) judge(2, rows2, rb0, raw2, rad2);  // (conditions: uniform in the wave)
 #pragma unroll
             for (int k = 0; k < KA; ++k)
-                if (wave * RPW + k * rstep < nb) judge(1, nb, r0 + k * rstep, raw1[k], rad1[k]);
+                if (rb0 + k * rstep < nb) judge(1, nb, rb0 + k * rstep, raw1[k], rad1[k]);
 #pragma unroll 1
-            for (int r = r0 + rstep; r - rg < rows2; r += rstep) {  // (fan-outs of one or two)
-                ask(2, first2, rows2, r, raw2, rad2);
-                judge(2, rows2, r, raw2, rad2);
+            for (int rb = rb0 + rstep; rb < rows2; rb += rstep) {  // (fan-outs of one or two)
+                ask(2, first2, rows2, rb, raw2, rad2);
+                judge(2, rows2, rb, raw2, rad2);
             }
 #pragma unroll 1
-            for (int r = r0 + KA * rstep; r - rg < nb; r += rstep) {  // (small workgroups)
-                ask(1, n0, nb, r, raw2, rad2);
-                judge(1, nb, r, raw2, rad2);
+            for (int rb = rb0 + KA * rstep; rb < nb; rb += rstep) {  // (small workgroups)
+                ask(1, n0, nb, rb, raw2, rad2);
+                judge(1, nb, rb, raw2, rad2);
             }
             int fl = first2, ll = first2 + rows2 - 1;  // first and last row of level l - 1
 #pragma unroll 1
@@ -886,9 +899,9 @@ void search_kernel(const SearchParams p) {
                 if ((l - 2) % nwaves != wave) continue;
                 const int rows = ll - fl + 1;
 #pragma unroll 1
-                for (int r = rg; r - rg < rows; r += RPW) {
-                    ask(l, fl, rows, r, raw2, rad2);
-                    judge(l, rows, r, raw2, rad2);
+                for (int rb = 0; rb < rows; rb += RPW) {
+                    ask(l, fl, rows, rb, raw2, rad2);
+                    judge(l, rows, rb, raw2, rad2);
                 }
             }
         } else {
