@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes as C
 import subprocess
+import sys
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
@@ -200,8 +201,8 @@ _lib = None
 
 
 def build_library(verbose: bool = False) -> None:
-    """Compile libhira_hip.so for gfx950 (hipcc cross-compiles without a GPU) and the native host side, _host.so."""
-    r = subprocess.run(["make", "-C", str(CSRC), "-B", "-j8"], capture_output=True, text=True)
+    """Compile libhira_hip.so for gfx950 (hipcc cross-compiles without a GPU) and the native host side, for this interpreter."""
+    r = subprocess.run(["make", "-C", str(CSRC), "-B", "-j8", f"PYTHON={sys.executable}"], capture_output=True, text=True)
     if verbose or r.returncode != 0:
         print(r.stdout[-4000:], r.stderr[-4000:])
     if r.returncode != 0:
@@ -243,17 +244,22 @@ _host_module = None
 
 def host():
     """The native host side of the calls a decode step makes (csrc/host.cpp), on the loaded library's functions; raises when
-    it has not been built."""
+    it has not been built, or was built for another torch, interpreter or library."""
     global _host_module
     if _host_module is None:
         l = lib()
+        build = f"build it with `make -C {CSRC} PYTHON={sys.executable}` (or __graft_entry__.build())"
         try:
-            import torch  # noqa: F401  (its libraries, which the module needs)
+            import torch  # (its libraries, which the module needs)
 
             from hira_amd import _host
         except ImportError as ex:
-            raise RuntimeError(f"hira_amd/_host.so is missing or was built for another torch ({ex}): build it with "
-                               f"`make -C {CSRC}` (or __graft_entry__.build())") from ex
+            raise RuntimeError(f"the native host side, hira_amd/_host, is missing or was built for another torch ({ex}): {build}") from ex
+        here = (f"{torch.__version__} {torch.version.git_version}", sys.version_info[0] << 8 | sys.version_info[1], l.hira_abi_version())
+        built = getattr(_host, "BUILT_FOR", None)
+        if built != here:
+            raise RuntimeError(f"the native host side, {_host.__file__}, was built for {built} (torch, Python, ABI of the library), "
+                               f"here are {here}: {build}")
         _host.bind({name: C.cast(getattr(l, name), _vp).value for name in SYMBOLS})
         _host_module = _host
     return _host_module

@@ -341,4 +341,15 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
-extern "C" __attribute__((visibility("default"))) PyObject* PyInit__host() { return PyModule_Create(&module); }
+// BUILT_FOR: torch's version and commit, the interpreter's version (major and minor, a byte each), the library's ABI.  The layouts of
+// all three are compiled in, and nothing else would notice that they are others now.
+extern "C" __attribute__((visibility("default"))) PyObject* PyInit__host() {
+    PyObject* m = PyModule_Create(&module);
+    PyObject* built = m ? Py_BuildValue("(sii)", HIRA_HOST_TORCH, PY_VERSION_HEX >> 16, HIRA_ABI_VERSION) : nullptr;
+    if (built == nullptr || PyModule_AddObject(m, "BUILT_FOR", built) < 0) {
+        Py_XDECREF(built);
+        Py_XDECREF(m);
+        return nullptr;
+    }
+    return m;
+}

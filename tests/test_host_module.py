@@ -1,6 +1,10 @@
 """The native host side (csrc/host.cpp) without a GPU: the random numbers it draws, and that what is not the form of a running
 program's call is left to the Python body."""
 import ctypes as C
+import shutil
+import subprocess
+import sys
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -27,6 +31,57 @@ def test_the_numbers_of_torch(default):
         assert torch.equal(a.get_state(), b.get_state())
     finally:
         torch.set_default_dtype(torch.float32)
+
+
+@pytest.mark.parametrize("other", ["torch", "commit", "interpreter", "library"])
+def test_a_module_built_for_another_is_refused(other, monkeypatch):
+    assert _lib.host() is _lib._host_module
+    monkeypatch.setattr(_lib, "_host_module", None)
+    if other == "torch":
+        monkeypatch.setattr(torch, "__version__", "2.10.1")
+    elif other == "commit":
+        monkeypatch.setattr(torch.version, "git_version", "0" * 40)
+    elif other == "interpreter":
+        monkeypatch.setattr(_lib, "sys", SimpleNamespace(executable=sys.executable, version_info=(3, 99, 0)))
+    else:
+        monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(hira_abi_version=lambda: _lib.HIRA_ABI_VERSION + 1))
+    with pytest.raises(RuntimeError, match="was built for"):
+        _lib.host()
+    assert _lib._host_module is None
+
+
+def _tree_with_stand_ins(tmp_path):
+    """The Makefile beside empty sources, under an interpreter whose torch is what a file says and a compiler that writes empty files.
+    make(*targets) returns how often that has compiled so far."""
+    csrc = tmp_path / "hira_amd" / "csrc"
+    csrc.mkdir(parents=True)
+    shutil.copy(_lib.CSRC / "Makefile", csrc)
+    (tmp_path / "include").mkdir()
+    for f in (csrc / "host.cpp", tmp_path / "include" / "hira_hip.h", csrc / "libhira_hip.so"):
+        f.touch()
+    python, cxx = tmp_path / "python", tmp_path / "c++"
+    python.write_text(f'#!/bin/sh\ncase "$2" in *EXT_SUFFIX*) echo .tag.so;; *git_version*) cat {tmp_path}/torch;; esac\n')
+    cxx.write_text(f'#!/bin/sh\necho "$*" >> {tmp_path}/compiled\nwhile [ "$1" != -o ]; do shift; done\ntouch "$2"\n')
+    for f in (python, cxx):
+        f.chmod(0o755)
+
+    def make(*targets):
+        subprocess.run(["make", "-C", str(csrc), f"PYTHON={python}", f"CXX={cxx}", "-o", "libhira_hip.so", *targets], check=True,
+                       capture_output=True)
+        log = tmp_path / "compiled"
+        return len(log.read_text().splitlines()) if log.exists() else 0
+
+    return make
+
+
+def test_another_torch_is_another_build(tmp_path):
+    make = _tree_with_stand_ins(tmp_path)
+    (tmp_path / "torch").write_text("2.10.0 abc\n")
+    assert make() == 1 and make() == 1 and make("host") == 1
+    assert (tmp_path / "hira_amd" / "_host.tag.so").exists()
+    (tmp_path / "torch").write_text("2.10.1 abc\n")
+    assert make() == 2 and make() == 2
+    assert [line.split("HIRA_HOST_TORCH=")[1][:12] for line in (tmp_path / "compiled").read_text().splitlines()] == ['"2.10.0 abc"', '"2.10.1 abc"']
 
 
 def test_what_is_not_the_form_is_left_alone():
