@@ -60,7 +60,7 @@ def _tree_with_stand_ins(tmp_path):
     for f in (csrc / "host.cpp", tmp_path / "include" / "hira_hip.h", csrc / "libhira_hip.so"):
         f.touch()
     python, cxx = tmp_path / "python", tmp_path / "c++"
-    python.write_text(f'#!/bin/sh\ncase "$2" in *EXT_SUFFIX*) echo .tag.so;; *git_version*) cat {tmp_path}/torch;; esac\n')
+    python.write_text(f'#!/bin/sh\ncase "$2" in *EXT_SUFFIX*) echo .tag.so;; *torch*) cat {tmp_path}/torch;; esac\n')
     cxx.write_text(f'#!/bin/sh\necho "$*" >> {tmp_path}/compiled\nwhile [ "$1" != -o ]; do shift; done\ntouch "$2"\n')
     for f in (python, cxx):
         f.chmod(0o755)
@@ -82,6 +82,15 @@ def test_another_torch_is_another_build(tmp_path):
     (tmp_path / "torch").write_text("2.10.1 abc\n")
     assert make() == 2 and make() == 2
     assert [line.split("HIRA_HOST_TORCH=")[1][:12] for line in (tmp_path / "compiled").read_text().splitlines()] == ['"2.10.0 abc"', '"2.10.1 abc"']
+
+
+def test_the_library_is_built_without_torch(tmp_path):
+    make = _tree_with_stand_ins(tmp_path)
+    assert make() == 0
+    with pytest.raises(subprocess.CalledProcessError):
+        make("host")
+    (tmp_path / "torch").write_text("2.10.0 abc\n")
+    assert make() == 1
 
 
 def test_what_is_not_the_form_is_left_alone():
