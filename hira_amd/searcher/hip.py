@@ -500,7 +500,7 @@ class DecodePlan:
         self.sample.scratch = self.tau_scratch.data_ptr()
         self._refs = (C.byref(self.tree), C.byref(self.query), C.byref(self.out),
                       C.byref(self.launch), C.byref(self.queue))
-        self._at: Optional[tuple] = None  # where the call's structs lie, for ``attend``
+        self._at: Optional[tuple] = None  # for ``attend``: the call's structs, and where they lie
 
     def _workspace_need(self) -> int:
         fake_q = _lib.HiraQuery(self.query.num_q_heads, 1, 1, 1, 1, 1, self.query.max_group,
@@ -527,12 +527,14 @@ class DecodePlan:
         None, and nothing done, for any other form."""
         if self.indexer._tree_struct is not self.tree:
             self._follow_index()
-        at = self._at
-        if at is None:
-            at = self._at = tuple(C.addressof(x) for x in (self.tree, self.query, self.sample, self.queue, self.out, self.launch))
+        at, tree = self._at, self.tree
+        if at is None or at[0][0] is not tree:
+            structs = tree, self.query, self.sample, self.queue, self.out, self.launch
+            at = self._at = structs, tuple(C.addressof(x) for x in structs)
+        # (the structs stay alive with `at` while the call reads them, whoever replaces the plan's meanwhile)
         if self.tau_buf is None:
             self.tau_buf = torch.empty((self.query.num_q_heads,), dtype=torch.float32, device=self.indexer.device)
-        out = _lib.host().attend(at, self._dev, self.ws, self.ws_bytes, self._ws_rows, self.tau_buf, query, samples, queue_keys,
+        out = _lib.host().attend(at[1], self._dev, self.ws, self.ws_bytes, self._ws_rows, self.tau_buf, query, samples, queue_keys,
                                  queue_values, rows, 0 if method == "sample_max" else 1, k, _lib.stream_of(self._dev))
         if out.__class__ is int:
             _lib.check(out)

@@ -1,15 +1,18 @@
 """The native host side (csrc/host.cpp) without a GPU: the random numbers it draws, and that what is not the form of a running
 program's call is left to the Python body."""
 import ctypes as C
+import gc
 import shutil
 import subprocess
 import sys
+import weakref
 from types import SimpleNamespace
 
 import pytest
 import torch
 
 from hira_amd import _lib
+from hira_amd.searcher.hip import DecodePlan
 
 
 def _draw(gen, m, first, members, seen):
@@ -113,3 +116,59 @@ def test_what_is_not_the_form_is_left_alone():
         host.draw(3, 1, 0, 1, 1)
     with pytest.raises(ValueError):
         host.draw(torch.Generator(), 1, 0, 0, 1)
+
+
+class _Structs:
+    """An index as far as a plan looks at it when its level sizes may have moved."""
+
+    device = torch.device("cpu")
+
+    def __init__(self):
+        self._tree_struct = _lib.HiraTree()
+
+    def tree_struct(self):
+        return self._tree_struct
+
+
+def _plan(monkeypatch, attend, kind=DecodePlan):
+    """A plan whose native call is `attend`."""
+    monkeypatch.setattr(_lib, "host", lambda: SimpleNamespace(attend=attend))
+    monkeypatch.setattr(_lib, "stream_of", lambda dev: 0)
+    plan = kind.__new__(kind)
+    plan.indexer = _Structs()
+    plan.tree, plan.query, plan.sample, plan.queue = plan.indexer._tree_struct, _lib.HiraQuery(4), _lib.HiraSample(), _lib.HiraQueue()
+    plan.out, plan.launch, plan._at, plan._dev = _lib.HiraSearchOut(), _lib.HiraLaunch(), None, 0
+    plan.tau_buf, plan.ws, plan.ws_bytes, plan._ws_rows = torch.zeros(4), torch.zeros(64, dtype=torch.uint8), 64, 1
+    plan._workspace_need = lambda: 64
+    return plan
+
+
+def test_a_plan_holds_its_structs_while_the_call_reads_them(monkeypatch):
+    """The call lets other threads run: one of them may be the first to see that the index moved."""
+    trees = []
+
+    def attend(at, *rest):
+        trees.append(weakref.ref(plan.tree))
+        assert at[0] == C.addressof(plan.tree) and at[1] == C.addressof(plan.query)
+        plan.indexer._tree_struct = _lib.HiraTree()
+        plan._follow_index()
+        gc.collect()
+        assert trees[-1]() is not None and C.addressof(trees[-1]()) == at[0]
+        return rest[5]
+
+    plan = _plan(monkeypatch, attend)
+    for _ in range(3):
+        assert plan.attend("query", None, "sample_mean_topk", 3, None, None, 0) == "query"
+        plan._at = None
+        gc.collect()
+        assert trees[-1]() is None
+
+
+def test_a_plan_whose_tree_is_replaced_while_it_looks_up_the_addresses(monkeypatch):
+    plan = _plan(monkeypatch, lambda at, *rest: at)
+    plan.attend(None, None, "sample_mean_topk", 3, None, None, 0)
+    stale = plan._at
+    plan.indexer._tree_struct = _lib.HiraTree()
+    plan._follow_index()
+    plan._at = stale  # (what a thread that had looked before leaves behind)
+    assert plan.attend(None, None, "sample_mean_topk", 3, None, None, 0)[0] == C.addressof(plan.tree)
