@@ -119,9 +119,10 @@ def hira_attention_forward(module, query, key, value, attention_mask=None, dropo
     plan = searcher.decode_plan(indexer, b * h_q, scaling)
     if sampled:
         rows, store = getattr(cache, "queue_rows", None), getattr(cache, "queue_store", None)
-        if rows is not None and store is not None:
+        attend = getattr(plan, "attend", None)  # (a searcher's own plans may have run_sampled alone)
+        if rows is not None and store is not None and attend is not None:
             # (the form that a running decode has; what has another goes on below)
-            out = plan.attend(query, samples, cache.threshold_method, cache.threshold_topk, store[0], store[1], rows)
+            out = attend(query, samples, cache.threshold_method, cache.threshold_topk, store[0], store[1], rows)
             if out is not None:
                 return out, None
     buf, dtype = indexer.keys_buf, indexer.dtype

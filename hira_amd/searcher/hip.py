@@ -524,7 +524,9 @@ class DecodePlan:
                queue_values: torch.Tensor, rows: int) -> Optional[torch.Tensor]:
         """``run_sampled`` for the form that a running decode has, in one step: query (B, H_q, 1, D) of the tree's type, the
         first `rows` rows of a decode queue (B, H_kv, cap, D / Dv); makes the output (B, 1, H_q, Dv) in the query's type.
-        None, and nothing done, for any other form."""
+        None, and nothing done, for any other form, and where ``run_sampled`` is no longer this class's."""
+        if getattr(self.run_sampled, "__func__", None) is not _RUN_SAMPLED:
+            return None
         if self.indexer._tree_struct is not self.tree:
             self._follow_index()
         at, tree = self._at, self.tree
@@ -628,6 +630,9 @@ class DecodePlan:
         if rc:
             _lib.check(rc)
         return tau
+
+
+_RUN_SAMPLED = DecodePlan.run_sampled  # the one that ``attend`` stands for
 
 
 class StreamingStep:

@@ -12,6 +12,7 @@ import pytest
 import torch
 
 from hira_amd import _lib
+from hira_amd.attention.hira_attention import hira_attention_forward
 from hira_amd.searcher.hip import DecodePlan
 
 
@@ -172,3 +173,32 @@ def test_a_plan_whose_tree_is_replaced_while_it_looks_up_the_addresses(monkeypat
     plan._follow_index()
     plan._at = stale  # (what a thread that had looked before leaves behind)
     assert plan.attend(None, None, "sample_mean_topk", 3, None, None, 0)[0] == C.addressof(plan.tree)
+
+
+def _ones(self, query, samples, method, k, out, *rest):
+    out.fill_(1.0)
+
+
+class _OwnStep(DecodePlan):
+    run_sampled = _ones
+
+
+@pytest.mark.parametrize("how", ["a subclass's", "the plan's", "the class's", "no attend"])
+def test_a_plan_that_takes_its_step_another_way(how, monkeypatch):
+    """The attention function calls run_sampled where it is not the one that the native call stands for."""
+    plan = _plan(monkeypatch, lambda *a: torch.zeros(1, 1, 4, 16), _OwnStep if how == "a subclass's" else DecodePlan)
+    ix = plan.indexer
+    ix.keys_buf, ix.dtype, ix.vdim, ix.num_trees = torch.zeros(2, 32, 16), torch.float32, 16, 2
+    q = torch.zeros(1, 4, 1, 16)
+    rows = torch.zeros(1, 2, 8, 16)
+    cache = SimpleNamespace(prefill_keys=None, indexer=ix, searcher=SimpleNamespace(decode_plan=lambda *a: plan), samples=torch.zeros(2, 8, 16),
+                            threshold_method="sample_mean_topk", threshold_topk=3, queue_rows=2, queue_store=(rows, rows))
+    if how != "a subclass's":
+        assert torch.equal(hira_attention_forward(None, q, cache, None, scaling=1.0)[0], torch.zeros(1, 1, 4, 16))
+    if how == "the plan's":
+        plan.run_sampled = _ones.__get__(plan)
+    elif how == "the class's":
+        monkeypatch.setattr(DecodePlan, "run_sampled", _ones)
+    elif how == "no attend":
+        plan = SimpleNamespace(run_sampled=lambda *a: _ones(None, *a))
+    assert torch.equal(hira_attention_forward(None, q, cache, None, scaling=1.0)[0], torch.ones(1, 1, 4, 16))
