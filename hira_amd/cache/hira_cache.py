@@ -267,7 +267,17 @@ class HiraCacheLayer(CacheLayerMixin):
             self._sample_facts()
             if first == m:
                 return (), ()
-        return _lib.host().draw(self._sample_gen, m - first, first, self.samples.shape[1], seen + first)
+        s, seen = self.samples.shape[1], seen + first
+        if self.samples.is_cuda:
+            return _lib.host().draw(self._sample_gen, m - first, first, s, seen)
+        # a layer in host memory (another indexer's) asks nothing of the library: the same numbers from torch
+        draws = torch.rand(m - first, generator=self._sample_gen).tolist()
+        who = [first + i for i, u in enumerate(draws) if u < s / (seen + i + 1)]
+        if not who:
+            return (), ()
+        slots = torch.randint(0, s, (len(who),), generator=self._sample_gen).tolist()
+        last = dict(zip(slots, who))  # (a slot drawn twice keeps its last arrival)
+        return tuple(last.keys()), tuple(last.values())
 
     def _replace_sampled(self, new_keys, slots, which):
         """The members `slots` of the sample replaced by rows `which` of the new keys."""

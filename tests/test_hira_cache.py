@@ -172,3 +172,32 @@ def test_key_sample_follows_the_index(patched):
         assert torch.equal(out.samples[1, :, 0].long() - 400, ids)  # same positions per head
     assert int((ids >= 200).sum()) >= 3 and int((ids < 200).sum()) >= 3  # old and new keys
     assert hc.HiraCacheLayer(DeviceMode.CUDA_ONLY, 4, {}, {}).update(allk, allk)[0].samples is None
+
+
+def test_a_sample_in_host_memory_needs_no_library(patched, monkeypatch):
+    """A layer over another indexer, its rows in host memory, keeps its key sample with torch alone; the members
+    are the ones that the native side draws."""
+    from hira_amd import _lib
+
+    def run(host):
+        monkeypatch.setattr(_lib, "lib", host)
+        monkeypatch.setattr(_lib, "host", host)
+        g = torch.Generator().manual_seed(1)
+        l = hc.HiraCacheLayer(DeviceMode.CUDA_ONLY, 5, {}, {}, dict(method="sample_mean_topk", sample_size=12, topk=3))
+        l.update(torch.randn(1, 2, 9, 16, generator=g), torch.randn(1, 2, 9, 16, generator=g))
+        pairs, drawn = [], l._sample_pairs
+        l._sample_pairs = lambda *a: pairs.append(drawn(*a)) or pairs[-1]
+        for m in (1, 1, 1, 1, 1, 40, 7):
+            l.update(torch.randn(1, 2, m, 16, generator=g), torch.randn(1, 2, m, 16, generator=g))
+        return l, pairs
+
+    draw = _lib.host().draw
+
+    def missing():
+        raise RuntimeError("no library")
+
+    layer, pairs = run(missing)
+    assert layer.samples.shape == (2, 12, 16) and sum(len(slots) for slots, _ in pairs) > 12
+    gen = torch.Generator().manual_seed(12345)
+    torch.randperm(9, generator=gen)
+    assert pairs == [draw(gen, 2, 3, 12, 12), draw(gen, 40, 0, 12, 14), draw(gen, 7, 0, 12, 54)]
