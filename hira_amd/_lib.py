@@ -265,6 +265,12 @@ def host():
     return _host_module
 
 
+def in_chunks(x):
+    """x, or its copy where it does not start at a multiple of 16 bytes: the kernels read rows in chunks of that, and
+    ``contiguous`` hands a view that starts between two of them back as it is."""
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 def check(rc: int) -> None:
     """Map a return code to the exception the reference's wrappers raise
     (kernels/triton_search_wrappers.py:9-110: ValueError for bad shapes)."""

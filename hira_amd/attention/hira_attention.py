@@ -25,6 +25,7 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 
+from hira_amd import _lib
 
 
 def _repeat_kv(x: torch.Tensor, n_rep: int) -> torch.Tensor:
@@ -136,6 +137,7 @@ def hira_attention_forward(module, query, key, value, attention_mask=None, dropo
         q2 = q2.to(device=buf.device, dtype=dtype)
     if not q2.is_contiguous():
         q2 = q2.contiguous()
+    q2 = _lib.in_chunks(q2)
     if direct and here:
         out = query.new_empty((b, 1, h_q, indexer.vdim))
     else:
@@ -149,13 +151,14 @@ def hira_attention_forward(module, query, key, value, attention_mask=None, dropo
     if qlen > 0:
         store = getattr(cache, "queue_store", None)
         if store is not None and store[0].dtype is dtype and store[0].get_device() == dev \
-                and store[0].is_contiguous() and store[1].is_contiguous():
+                and store[0].is_contiguous() and store[1].is_contiguous() \
+                and (store[0].data_ptr() | store[1].data_ptr()) % 16 == 0:
             qk, qv = store
         else:
-            qk = cache.queued_keys.to(device=buf.device, dtype=dtype).reshape(
-                indexer.num_trees, qlen, d).contiguous()
-            qv = cache.queued_values.to(device=buf.device, dtype=dtype).reshape(
-                indexer.num_trees, qlen, -1).contiguous()
+            qk = _lib.in_chunks(cache.queued_keys.to(device=buf.device, dtype=dtype).reshape(
+                indexer.num_trees, qlen, d).contiguous())
+            qv = _lib.in_chunks(cache.queued_values.to(device=buf.device, dtype=dtype).reshape(
+                indexer.num_trees, qlen, -1).contiguous())
     if sampled:
         plan.run_sampled(q2, samples, cache.threshold_method, cache.threshold_topk, out, None, qk, qv, qlen)
     else:

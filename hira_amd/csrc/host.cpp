@@ -48,7 +48,11 @@ int type_of(const at::Tensor& t) {
     return t.scalar_type() == at::kFloat ? (int)HIRA_F32 : t.scalar_type() == at::kBFloat16 ? (int)HIRA_BF16 : -1;
 }
 
-bool aligned(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+// One whose rows the kernels read in 16-byte chunks: a contiguous view may start between two of them.
+const at::Tensor* in_chunks(PyObject* o, int64_t dev) {
+    const at::Tensor* t = plain(o, dev);
+    return t != nullptr && reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0 ? t : nullptr;
+}
 
 int64_t number(PyObject* o) {
     const long long v = PyLong_AsLongLong(o);
@@ -100,7 +104,7 @@ PyObject* enqueue(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     if (!arguments("enqueue", n, 7)) return nullptr;
     const int64_t at = number(a[4]), dev = number(a[5]);
-    const at::Tensor *qk = plain(a[0], dev), *qv = plain(a[1], dev), *k = plain(a[2], dev), *v = plain(a[3], dev);
+    const at::Tensor *qk = in_chunks(a[0], dev), *qv = in_chunks(a[1], dev), *k = in_chunks(a[2], dev), *v = in_chunks(a[3], dev);
     if (!qk || !qv || !k || !v || qk->dim() != 4 || qv->dim() != 4 || k->dim() != 4 || v->dim() != 4) Py_RETURN_NONE;
     const int type = type_of(*qk);
     if (type < 0 || type_of(*qv) != type || type_of(*k) != type || type_of(*v) != type) Py_RETURN_NONE;
@@ -110,7 +114,7 @@ PyObject* enqueue(PyObject*, PyObject* const* a, Py_ssize_t n) {
         Py_RETURN_NONE;
     const int64_t e = type == HIRA_F32 ? 4 : 2;
     void *qkp = qk->data_ptr(), *qvp = qv->data_ptr(), *kp = k->data_ptr(), *vp = v->data_ptr();
-    if (d * e % 16 || dv * e % 16 || !aligned(kp) || !aligned(vp) || b * h > INT32_MAX) Py_RETURN_NONE;
+    if (d * e % 16 || dv * e % 16 || b * h > INT32_MAX) Py_RETURN_NONE;
     void* stream = address(a[6]);
     return PyLong_FromLong(without_gil([&] {
         return lib.enqueue(qkp, qvp, type, (int32_t)(b * h), (int32_t)cap, (int32_t)at, 1, (int32_t)d, (int32_t)dv, kp, vp, stream);
@@ -134,7 +138,7 @@ PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HiraSearchOut* out = static_cast<HiraSearchOut*>(address(part(4)));
     const HiraLaunch* launch = static_cast<const HiraLaunch*>(address(part(5)));
     const int64_t dev = number(a[1]), bytes = number(a[3]), rows = number(a[10]), rule = number(a[11]), k = number(a[12]);
-    const at::Tensor *ws = plain(a[2], dev), *tau = plain(a[5], dev), *q = plain(a[6], dev), *s = plain(a[7], dev);
+    const at::Tensor *ws = plain(a[2], dev), *tau = plain(a[5], dev), *q = in_chunks(a[6], dev), *s = in_chunks(a[7], dev);
     if (!ws || !tau || !q || !s || q->dim() != 4 || s->dim() != 3 || type_of(*q) != tree->dtype || type_of(*s) != tree->dtype ||
         ws->scalar_type() != at::kByte || ws->numel() < bytes || tau->scalar_type() != at::kFloat)
         Py_RETURN_NONE;
@@ -145,7 +149,7 @@ PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor *qk = nullptr, *qv = nullptr;
     int64_t cap = 0;
     if (rows != 0) {
-        qk = plain(a[8], dev), qv = plain(a[9], dev);
+        qk = in_chunks(a[8], dev), qv = in_chunks(a[9], dev);
         if (!qk || !qv || qk->dim() < 2 || qv->dim() < 2 || type_of(*qk) != tree->dtype || type_of(*qv) != tree->dtype) Py_RETURN_NONE;
         cap = qk->size(-2);
         if (rows < 0 || rows > cap || rows > number(a[4]) || cap > INT32_MAX || qv->size(-2) != cap || qk->size(-1) != tree->dim ||
@@ -183,7 +187,7 @@ PyObject* search(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HiraSearchOut* out = static_cast<HiraSearchOut*>(address(part(2)));
     const int64_t heads = number(part(3)), dev = number(part(4));
     const float* scale = static_cast<const float*>(address(part(5)));
-    const at::Tensor *q = plain(a[2], dev), *tau = plain(a[3], dev), *dense = plain(a[5], dev);
+    const at::Tensor *q = in_chunks(a[2], dev), *tau = plain(a[3], dev), *dense = plain(a[5], dev);
     if (!q || !tau || !dense || type_of(*q) != tree->dtype || !(q->dim() == 2 || (q->dim() == 4 && q->size(2) == 1)) ||
         q->size(-1) != tree->dim || q->numel() != heads * tree->dim || tau->scalar_type() != at::kFloat || tau->numel() != heads ||
         dense->scalar_type() != at::kFloat || dense->dim() != 2 || dense->size(0) != heads || dense->size(1) != tree->size[0])
@@ -220,18 +224,18 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!arguments("append", n, 12)) return nullptr;
     const HiraTree* tree = static_cast<const HiraTree*>(address(a[0]));
     const int64_t m = number(a[3]), dev = number(a[8]);
-    const at::Tensor *k = plain(a[1], dev), *v = nullptr, *s = nullptr;
+    const at::Tensor *k = in_chunks(a[1], dev), *v = nullptr, *s = nullptr;
     if (!k || type_of(*k) != tree->dtype || m < 0 || m > INT32_MAX || k->numel() != tree->num_trees * m * tree->dim) Py_RETURN_NONE;
     if (a[2] != Py_None) {
-        v = plain(a[2], dev);
+        v = in_chunks(a[2], dev);
         if (!v || type_of(*v) != tree->dtype || v->numel() != tree->num_trees * m * tree->vdim) Py_RETURN_NONE;
     }
     std::vector<int32_t> pairs;
     int64_t count = 0;
     if (a[5] != Py_None) {
-        s = plain(a[5], dev);
+        s = in_chunks(a[5], dev);
         if (!s || s->dim() != 3 || type_of(*s) != tree->dtype || s->size(0) != tree->num_trees || s->size(2) != tree->dim ||
-            s->size(1) > INT32_MAX || !aligned(k->data_ptr()) || !PyTuple_CheckExact(a[6]) || !PyTuple_CheckExact(a[7]) ||
+            s->size(1) > INT32_MAX || !PyTuple_CheckExact(a[6]) || !PyTuple_CheckExact(a[7]) ||
             PyTuple_GET_SIZE(a[6]) != PyTuple_GET_SIZE(a[7]))
             Py_RETURN_NONE;
         count = PyTuple_GET_SIZE(a[6]);

@@ -607,10 +607,10 @@ class HIPIndexer(BaseIndexer):
         dtype = self.storage_dtype(keys.dtype)
         vdim = 0 if values is None else int(values.shape[-1])
         self._allocate(b, h, n, d, vdim, dtype, used=True)
-        kin = keys.to(device=self.device, dtype=dtype).reshape(b * h, n, d).contiguous()
+        kin = _lib.in_chunks(keys.to(device=self.device, dtype=dtype).reshape(b * h, n, d).contiguous())
         vin = None
         if values is not None:
-            vin = values.to(device=self.device, dtype=dtype).reshape(b * h, n, vdim).contiguous()
+            vin = _lib.in_chunks(values.to(device=self.device, dtype=dtype).reshape(b * h, n, vdim).contiguous())
         lib = _lib.lib()
         tree = self.tree_struct()
         need = lib.hira_build_workspace_bytes(C.byref(tree), n)
@@ -810,11 +810,11 @@ class HIPIndexer(BaseIndexer):
         return self
 
     def _rows(self, x: torch.Tensor, t: int, m: int, width: int) -> torch.Tensor:
-        """(T, m, width) rows, contiguous, in the storage type and on the index's device."""
-        if x.dtype is self.dtype and x.get_device() == self.keys_buf.get_device() and \
-                x.is_contiguous() and x.numel() == t * m * width:
-            return x
-        return x.to(device=self.device, dtype=self.dtype).reshape(t, m, width).contiguous()
+        """(T, m, width) rows, contiguous, in the storage type and on the index's device, as the kernels read them."""
+        if x.dtype is not self.dtype or x.get_device() != self.keys_buf.get_device() or \
+                not x.is_contiguous() or x.numel() != t * m * width:
+            x = x.to(device=self.device, dtype=self.dtype).reshape(t, m, width).contiguous()
+        return _lib.in_chunks(x)
 
     def _sample_args(self, sample):
         """(address, rows a tree, slots, which, their number) of ``update``'s sample for the library."""
@@ -834,8 +834,6 @@ class HIPIndexer(BaseIndexer):
         rows, per_tree, slots, which, n = self._sample_args(sample)
         if n:
             kin = self._rows(new_keys, self.num_trees, m, self.dim)
-            if kin.data_ptr() % 16:
-                kin = kin.clone()
             _lib.check(_lib.lib().hira_replace_rows(
                 rows, _DTYPES[self.dtype], self.dim, self.num_trees, per_tree, kin.data_ptr(), m, m, slots,
                 which, n, _lib.stream_of(self.keys_buf.get_device())))
@@ -1049,8 +1047,6 @@ class HIPIndexer(BaseIndexer):
             kin = self._rows(new_keys, t, m, self.dim)
             vin = None if new_values is None else self._rows(new_values, t, m, self.vdim)
             rows, per_tree, slots, which, n = self._sample_args(sample)
-            if n and kin.data_ptr() % 16:  # (whole chunks of rows move there)
-                kin = kin.clone()
             rc = _lib.lib().hira_update_sample(C.byref(tree), kin.data_ptr(),
                                                None if vin is None else vin.data_ptr(), m,
                                                self._state.data_ptr(), rows, per_tree, slots, which, n,

@@ -202,7 +202,7 @@ class HIPSearcher(BaseSearcher):
 
     def _query_struct(self, query, threshold, indexer, q_head_to_kv, scaling):
         dev = indexer.device
-        q = self._coerce_query(query, indexer.dim).to(device=dev, dtype=indexer.dtype).contiguous()
+        q = _lib.in_chunks(self._coerce_query(query, indexer.dim).to(device=dev, dtype=indexer.dtype).contiguous())
         h_q = q.shape[0]
         tau = self._coerce_threshold(threshold, h_q, dev)
         sc = self._coerce_scaling(scaling, h_q, dev)
@@ -216,7 +216,7 @@ class HIPSearcher(BaseSearcher):
         tree = indexer.tree_struct()
         dim = indexer.dim
         if q_head_to_kv is None and isinstance(query, torch.Tensor) and \
-                query.dtype is indexer.dtype and query.is_contiguous():
+                query.dtype is indexer.dtype and query.is_contiguous() and query.data_ptr() % 16 == 0:
             shape = query.shape
             nd = len(shape)
             if shape[-1] == dim and (nd == 2 or (nd == 4 and shape[2] == 1)):
@@ -437,12 +437,11 @@ class HIPSearcher(BaseSearcher):
 
     @staticmethod
     def _queue_rows(x: torch.Tensor, indexer, dev: int, width: int) -> torch.Tensor:
-        """Queued rows of all trees, contiguous, in the index's storage type and on its device."""
-        if x.dtype is indexer.dtype and x.get_device() == dev and x.is_contiguous() and \
-                x.numel() % (indexer.num_trees * width) == 0:
-            return x
-        x = x.reshape(indexer.num_trees, -1, width)
-        return x.to(device=indexer.device, dtype=indexer.dtype).contiguous()
+        """Queued rows of all trees, contiguous, in the index's storage type and on its device, as the kernels read them."""
+        if x.dtype is not indexer.dtype or x.get_device() != dev or not x.is_contiguous() or \
+                x.numel() % (indexer.num_trees * width) != 0:
+            x = x.reshape(indexer.num_trees, -1, width).to(device=indexer.device, dtype=indexer.dtype).contiguous()
+        return _lib.in_chunks(x)
 
     def decode_plan(self, indexer, num_q_heads: int, scaling: float) -> "DecodePlan":
         """The plan for (this index, head count, one softmax scale for all heads), made on
@@ -467,7 +466,7 @@ class HIPSearcher(BaseSearcher):
 class DecodePlan:
     """One fused search + attention call per ``run``: ``query`` (H_q, D) in the tree dtype,
     ``threshold`` (H_q,) fp32 and ``out`` (H_q, Dv) fp32 (or bf16: the fp32 sums are then rounded
-    where they are written) must be contiguous device tensors."""
+    where they are written) must be contiguous device tensors that start at a multiple of 16 bytes, as torch allocates them."""
 
     def __init__(self, searcher: HIPSearcher, indexer, num_q_heads: int, scaling, q_head_to_kv,
                  stats):

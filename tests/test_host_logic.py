@@ -344,6 +344,47 @@ def test_one_plan_however_the_number_of_heads_comes():
     assert len(made) == 1 and all(p is plans[0] for p in plans)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_start_where_the_kernels_read_them(dtype):
+    """A contiguous view that starts between two 16-byte chunks is copied, wherever rows come in."""
+    from types import SimpleNamespace
+
+    from hira_amd import _lib
+    from hira_amd.attention.hira_attention import hira_attention_forward
+
+    x = torch.arange(2 * 3 * 16 + 1).to(dtype)[1:]
+    assert x.is_contiguous() and x.data_ptr() % 16
+    copies = []
+
+    def check(y):
+        assert y.data_ptr() % 16 == 0 and torch.equal(y.reshape(-1), x)
+        copies.append(y)
+
+    idx = HIPIndexer(2, 0, 4, device="cpu")
+    idx.batch, idx.num_heads, idx.num_trees, idx.dim, idx.vdim, idx.dtype = 1, 2, 2, 16, 16, dtype
+    idx.keys_buf = idx.values_buf = torch.zeros(2, 4, 16, dtype=dtype)
+    idx._tree_struct = _lib.HiraTree(num_trees=2)
+    check(idx._rows(x.view(1, 2, 3, 16), 2, 3, 16))
+    check(HIPSearcher._queue_rows(x.view(2, 3, 16), idx, -1, 16))
+    se = HIPSearcher()
+    check(se._query_struct(x.view(6, 16), 0.0, idx, None, None)[1][0])
+    for query in (x.view(6, 16), x.view(1, 6, 1, 16)):
+        call, heads, keep = se._call(query, 0.0, idx, None, None)
+        assert heads == 6 and call.query.q == keep[0].data_ptr()
+        check(keep[0])
+    aligned = x.clone().view(6, 16)
+    assert se._call(aligned, 0.0, idx, None, torch.ones(6))[2][0] is aligned
+    plan = SimpleNamespace(run_sampled=lambda q, s, m, k, out, st, qk, qv, n: [check(t) for t in (q, qk, qv)])
+    rows = x.view(1, 2, 3, 16)
+    for store in ((rows, rows), None):
+        cache = SimpleNamespace(prefill_keys=None, indexer=idx, searcher=SimpleNamespace(decode_plan=lambda *a: plan), samples=rows[0],
+                                threshold_method="sample_max", threshold_topk=1, queued_keys=rows, queued_values=rows)
+        if store:
+            cache.queue_store = store
+        hira_attention_forward(None, x.view(1, 6, 1, 16), cache, None, scaling=1.0)
+    assert len(copies) == 11
+
+
 def test_storage_dtype_policy():
     assert HIPIndexer.storage_dtype(torch.bfloat16) == torch.bfloat16
     assert HIPIndexer.storage_dtype(torch.float32) == torch.float32

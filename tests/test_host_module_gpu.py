@@ -1,8 +1,11 @@
 """Calls in the form that the native host side takes against the same calls in other forms (strides, types, storage that is not
 aligned), which go through the Python bodies: same results."""
+import ctypes as C
+
 import pytest
 import torch
 
+from hira_amd import _lib
 from hira_amd.attention.hira_attention import hira_attention_forward
 from hira_amd.cache.hira_cache import HiraCacheLayer
 from hira_amd.indexer import HIPIndexer
@@ -36,9 +39,7 @@ FORMS = {"ready": lambda x: x, "strided": _strided, "misaligned": _misaligned, "
 @pytest.mark.parametrize("form", list(FORMS))
 @pytest.mark.parametrize("every,n", [(4, 300), (1, 300), (3, 900)])
 def test_a_decode_through_the_cache_layer(form, every, n, gpu_device):
-    if form == "misaligned" and every == 1:
-        pytest.skip("rows that go into the index at once")
-    as_query = FORMS[form] if form in ("strided", "parameter") else FORMS["ready"]
+    as_query = FORMS[form] if form in ("strided", "misaligned", "parameter") else FORMS["ready"]
 
     def run(form):
         print(f"case form={form} every={every} n={n}", flush=True)
@@ -73,7 +74,7 @@ def test_a_search_like_one_before_it(dtype, gpu_device):
 
     for step in range(3):
         q = x(4, 64, dtype=dtype)
-        for query in (q, q[None, :, None], _strided(q), q.double()):
+        for query in (q, q[None, :, None], _strided(q), _misaligned(q), q.double()):
             for t, s in ((tau, None), (tau, sc), (4.0, None), (tau.double(), _strided(sc)), (_strided(tau), sc)):
                 assert torch.equal(kept.search(query, t, index, scaling=s), fresh().search(query, t, index, scaling=s))
         assert torch.equal(kept.search(q[:2], tau[:2], index), fresh().search(q[:2], tau[:2], index))  # (other heads)
@@ -84,7 +85,7 @@ def test_a_search_like_one_before_it(dtype, gpu_device):
             kept.launch = HIPSearcher(kernel=1).launch
 
 
-@pytest.mark.parametrize("form", ["strided", "fp32", "parameter"])
+@pytest.mark.parametrize("form", ["strided", "misaligned", "fp32", "parameter"])
 @pytest.mark.parametrize("m", [1, 40])
 def test_an_append_and_its_read_back(form, m, gpu_device):
     def run(form):
@@ -103,3 +104,70 @@ def test_an_append_and_its_read_back(form, m, gpu_device):
         assert torch.equal(a.radii[l], b.radii[l]) and torch.equal(a.counts[l], b.counts[l])
     assert torch.equal(a.perm[:, :a.size[0]], b.perm[:, :b.size[0]]) and torch.equal(a.values_buf[:, :700], b.values_buf[:, :700])
     assert a._host_rows is not None and b._host_rows is not None
+
+
+class _Calls:
+    """The native functions' calls with every argument in the form that they take, over stand-ins for the library's functions:
+    what they would launch is noted and not done.  `args[name]` may be changed before `call(name)`."""
+
+    def __init__(self):
+        self.host, self.launched, self.codes = _lib.host(), [], {}
+        x, t, dev = _gen(1), 2, torch.cuda.current_device()
+        self.tree = _lib.HiraTree(num_trees=t, num_levels=2, bf=16, dim=64, vdim=32, dtype=_lib.HIRA_BF16)
+        self.tree.size[0] = 96
+        self.query, self.out, self.queue = _lib.HiraQuery(4), _lib.HiraSearchOut(), _lib.HiraQueue()
+        self.sample, self.launch = _lib.HiraSample(), _lib.HiraLaunch()
+        at = {n: C.addressof(getattr(self, n)) for n in ("tree", "query", "sample", "queue", "out", "launch")}
+        self.state, one = torch.zeros(t, 10, dtype=torch.int32, device="cuda"), torch.ones(4, device="cuda")
+        self.keep = one
+        k, v, samples = x(1, t, 1, 64), x(1, t, 1, 32), x(t, 40, 64)
+        qk, qv = x(1, t, 8, 64), x(1, t, 8, 32)
+        back = torch.zeros(t * (_lib.HIRA_MAX_LEVELS + 2), dtype=torch.int64, pin_memory=True)
+        self.args = {
+            "enqueue": [qk, qv, k, v, 3, dev, 0],
+            "attend": [tuple(at.values()), dev, torch.zeros(512, dtype=torch.uint8, device="cuda"), 512, 8, one.clone(), x(1, 4, 1, 64),
+                       samples, qk, qv, 5, 1, 3, 0],
+            "search": [(at["tree"], at["query"], at["out"], 4, dev, one.data_ptr()), at["launch"], x(4, 64), one.clone(), one.clone(),
+                       torch.zeros(4, 96, device="cuda"), -7.0, 0],
+            "append": [at["tree"], x(1, t, 3, 64), x(1, t, 3, 32), 3, self.state.data_ptr(), samples, (4, 0), (1, 2), dev, 0, back, 1],
+        }
+
+    def __enter__(self):
+        def stand_in(name):
+            res, args = _lib.SYMBOLS[name]
+            return C.CFUNCTYPE(res, *args)(lambda *a: self.launched.append(name) or self.codes.get(name, 0))
+
+        self.functions = {name: stand_in(name) for name in ("hira_enqueue", "hira_search", "hira_search_sampled", "hira_update_sample",
+                                                            "hira_read_state")}
+        self.host.bind({name: C.cast(f, C.c_void_p).value for name, f in self.functions.items()})
+        return self
+
+    def __exit__(self, *exc):
+        lib = _lib.lib()
+        self.host.bind({name: C.cast(getattr(lib, name), C.c_void_p).value for name in _lib.SYMBOLS})
+
+    def call(self, name):
+        """(what came back, what was launched, were the structs changed)"""
+        structs = self.query, self.out, self.queue, self.sample
+        before, n = [bytes(s) for s in structs], len(self.launched)
+        result = getattr(self.host, name)(*self.args[name])
+        return result, self.launched[n:], [bytes(s) for s in structs] != before
+
+    def refused(self, name):
+        result, launched, changed = self.call(name)
+        return result is None and not launched and not changed
+
+
+CHUNKS = [("enqueue", 0), ("enqueue", 1), ("enqueue", 2), ("enqueue", 3), ("attend", 6), ("attend", 7), ("attend", 8), ("attend", 9),
+          ("search", 2), ("append", 1), ("append", 2), ("append", 5)]
+
+
+@pytest.mark.parametrize("name,i", CHUNKS)
+def test_rows_that_start_between_two_chunks_are_left_alone(name, i, gpu_device):
+    with _Calls() as calls:
+        assert calls.call(name)[1]
+        calls.args[name][i] = _misaligned(calls.args[name][i])
+        assert calls.refused(name)
+        if name == "append" and i < 3:  # (without a sample too)
+            calls.args[name][5:8] = None, (), ()
+            assert calls.refused(name)
