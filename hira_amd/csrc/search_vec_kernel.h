@@ -86,31 +86,6 @@ struct VecLanes {
     }
 };
 
-// The products of a 16-byte chunk of a row and of a query.  bf16: two an instruction, added up in fp32, of the chunks as they
-// lie: five instructions and not sixteen, half the registers for the queries.  16 trees x 19889 rows of 96 columns, seven
-// heads 80 -> 69 us, one 28 -> 26.  In two halves: the scores' error against 64 bits is 0.97 to 1.02 of that of a chain of fmas
-// (32 to 256 columns, normal ones and with eight of them twenty times as large; as one chain of four 0.96 to 1.03, 66 us).
-template <typename T>
-__device__ __forceinline__ float vec_dot(const uint4& x, const uint4& q) {
-    float d = 0.0f;
-    if constexpr (sizeof(T) == 2) {
-        typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-        const uint32_t a[4] = {x.x, x.y, x.z, x.w}, b[4] = {q.x, q.y, q.z, q.w};
-        float half[2] = {0.0f, 0.0f};
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            half[e / 2] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a[e]), __builtin_bit_cast(bf16x2, b[e]), half[e / 2], false);
-        d = half[0] + half[1];
-    } else {
-        float a[4], b[4];
-        unpack<T>(x, a);
-        unpack<T>(q, b);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) d += a[e] * b[e];
-    }
-    return d;
-}
-
 template <int N, int BIT>
 __device__ __forceinline__ void reduce_step(float* v, int lane) {
     // partner: a lane that differs in BIT (and maybe in lower bits)
@@ -512,7 +487,7 @@ void search_kernel(const SearchParams p) {
 #pragma unroll
         for (int u = 0; u < KU; ++u) {
 #pragma unroll
-            for (int g = 0; g < GMAX; ++g) s[u * GMAX + g] = vec_dot<T>(raw[u], qraw[g]);
+            for (int g = 0; g < GMAX; ++g) s[u * GMAX + g] = chunk_dot<T>(raw[u], qraw[g]);
         }
         reduce_scatter<NV, LPR / 2>(s, lane);
         int my_slot;
@@ -671,7 +646,7 @@ void search_kernel(const SearchParams p) {
             unsigned pass = 0;
     #pragma unroll
             for (int g = 0; g < GMAX; ++g) {
-                const float d = group_sum<LPR>(vec_dot<T>(raw, qraw[g]));
+                const float d = group_sum<LPR>(chunk_dot<T>(raw, qraw[g]));
                 if (d + qn[g] * rad >= tau[g]) pass |= 1u << g;
             }
             if (ch == 0 && r < rows) s_pass[l][r] = pass | (rad > -INFINITY ? 0x80000000u : 0u);
@@ -872,7 +847,7 @@ void search_kernel(const SearchParams p) {
                 unsigned pass = 0;
 #pragma unroll
                 for (int g = 0; g < GMAX; ++g) {
-                    const float d = group_sum<LPR>(vec_dot<T>(x, qraw[g]));
+                    const float d = group_sum<LPR>(chunk_dot<T>(x, qraw[g]));
                     if (d + qn[g] * rad >= tau[g]) pass |= 1u << g;
                 }
                 if (ch == 0 && r < rows) s_pass[l][r] = pass | (rad > -INFINITY ? 0x80000000u : 0u);

@@ -472,15 +472,9 @@ __device__ __forceinline__ void threshold_block(
                     raw[u] = make_uint4(v.x, v.y, v.z, v.w);
                 }
             }
-            float b[EPL];
-            unpack<T>(load_chunk<T>(qh, 0, c), b);
+            const uint4 b = load_chunk<T>(qh, 0, c);
 #pragma unroll
-            for (int u = 0; u < kTauRows; ++u) {
-                float a[EPL];
-                unpack<T>(raw[u], a);
-#pragma unroll
-                for (int e = 0; e < EPL; ++e) dot[u] += a[e] * b[e];
-            }
+            for (int u = 0; u < kTauRows; ++u) dot[u] = chunk_dot<T>(raw[u], b, dot[u]);
         }
 #pragma unroll
         for (int u = 0; u < kTauRows; ++u) {

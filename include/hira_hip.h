@@ -358,7 +358,10 @@ int hira_quantize(const HiraTree* tree, int32_t slot_first, int32_t slot_count,
  *   HIRA_TAU_SAMPLE_MEAN_TOPK  tau[h] = mean of the k largest q_h.x  (1 <= k <= num_samples)
  *   samples    (num_trees, num_samples, dim) row-major in `dtype`, num_samples <= 4096
  *   query      q, num_q_heads and the head map are read (tau and scaling are not)
- *   tau_out    (H_q) fp32; scores are accumulated in fp32
+ *   tau_out    (H_q) fp32; scores are accumulated in fp32.  Rows of one or two 16-byte chunks score the same here and
+ *              in hira_search; wider rows' sums are taken in another order there, so that a key whose score is the
+ *              threshold (the best member of a sample under HIRA_TAU_SAMPLE_MAX or k = 1) may come out an ulp below
+ *              it and not be selected
  */
 enum { HIRA_TAU_SAMPLE_MAX = 0, HIRA_TAU_SAMPLE_MEAN_TOPK = 1 };
 int hira_threshold(const void* samples, int32_t dtype, int32_t num_trees, int32_t num_samples,

@@ -43,3 +43,21 @@ def test_equal_scores(gpu_device):
         got = tf.sample_mean_topk(x.cuda(), q.cuda(), k).cpu()
         want = 128.0 * (2.0 * min(k, 78) + max(k - 78, 0)) / k
         assert torch.allclose(got, torch.full((2,), want), rtol=1e-6)
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 8), (torch.bfloat16, 16), (torch.float32, 4), (torch.float32, 8)])
+def test_the_best_member_of_a_sample_is_selected(dtype, d, gpu_device):
+    """Rows of one or two chunks score the same in the threshold and in the search: under a sample's maximum the
+    key that makes the threshold is selected."""
+    from hira_amd.cache import threshold_finder as tf
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    g = torch.Generator().manual_seed(d)
+    keys = torch.randn(1, 8, 900, d, generator=g).to(dtype).cuda()
+    index, searcher = HIPIndexer(2, 1, 16).build(keys), HIPSearcher(output_fill_value=float("-inf"))
+    for _ in range(8):
+        q = torch.randn(64, d, generator=g).to(dtype).cuda()
+        tau = tf.sample_max(keys[0], q)
+        assert torch.equal(tau, tf.sample_mean_topk(keys[0], q, 1))
+        assert torch.equal(searcher.search(q, tau, index).amax(dim=1), tau)
