@@ -158,3 +158,64 @@ def test_one_block_a_wave_equals_the_general_way(t, g, n, d, dv, bf, nl, dtype, 
         idx.keys_buf[0, slot + (idx.perm[0, slot + 1] >= 0).int().item()] = float("nan")
     a, b = (se.search_attention(q, tau, idx, scaling=sc, queue_keys=qk, queue_values=qv) for se in (one, gen_way))
     assert torch.equal(a.isfinite(), b.isfinite()) and torch.equal(a.isnan(), b.isnan())
+
+
+def _chain_of_fmas(x, q):
+    """Scores (T, G, N) of bf16 rows x (T, N, D) and q (T, G, D) as a lane's chain of fmas over its chunk gives them (the
+    products are exact in 32 bits) and the lanes' sums in the kernel's order."""
+    t, n, d = x.shape
+    lanes = 1
+    while lanes * 8 < d:
+        lanes *= 2
+    c = torch.zeros(t, q.shape[1], n, lanes)
+    for e in range(8):
+        p = q[:, :, None, e::8].float() * x[:, None, :, e::8].float()
+        c[..., :p.shape[-1]] += p
+    while lanes > 1:
+        lanes //= 2
+        high = c[..., lanes:]
+        c = c[..., :lanes] + (high if lanes >= 16 else high.flip(-1))
+    return c[..., 0]
+
+
+@pytest.mark.parametrize("large", [0, 8])
+@pytest.mark.parametrize("d", [16, 32, 96, 128, 256])
+def test_bf16_scores_are_no_further_from_64_bits(d, large, gpu_device):
+    """Products two an instruction: the error against 64 bits is that of a chain of fmas."""
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    t, g, n = 2, 8, 3000
+    gen = torch.Generator().manual_seed(d + large)
+    x, q = torch.randn(t, n, d, generator=gen), torch.randn(t, g, d, generator=gen)
+    x[..., :large] *= 20.0
+    x, q = x.bfloat16(), q.bfloat16()
+    index = HIPIndexer(2, 0, 16, layout="row_major").build(x[None].cuda())
+    got = HIPSearcher(kernel=1, index_space="position").search(q.reshape(t * g, d).cuda(), float("-inf"), index)
+    want = torch.matmul(q.double(), x.double().transpose(1, 2).contiguous())
+    err = got.cpu().double().reshape(t, g, n) - want
+    # (two roundings in each of two instructions, the halves, the lanes, each at most 2^-23 of the sum of magnitudes)
+    most = torch.matmul(q.double().abs(), x.double().abs().transpose(1, 2).contiguous())
+    assert float((err.abs() / most).max()) <= (5 + max(0, d // 8 - 1).bit_length()) * 2.0 ** -23
+    chain = _chain_of_fmas(x, q).double() - want
+    # 48000 scores: the two root mean squares vary by a hundredth
+    assert float(err.square().mean().sqrt()) <= 1.05 * float(chain.square().mean().sqrt())
+
+
+@pytest.mark.parametrize("exponent", [0, 100])
+@pytest.mark.parametrize("d", [16, 96, 256])
+def test_bf16_rows_of_subnormal_numbers(d, exponent, gpu_device):
+    """Rows below the normal range count in full: whole multiples of 2^-133, whose sums are exact."""
+    from hira_amd.indexer import HIPIndexer
+    from hira_amd.searcher import HIPSearcher
+
+    gen = torch.Generator().manual_seed(d)
+    k = torch.randint(-127, 128, (2, 500, d), generator=gen)
+    x = torch.where(k < 0, -k - 2 ** 15, k).to(torch.int16).view(torch.bfloat16)  # (the bits: a sign and a multiple)
+    assert torch.equal(x.double(), k.double() * 2.0 ** -133)
+    whole = torch.randint(-9, 10, (2, 3, d), generator=gen)
+    q = (whole.double() * 2.0 ** exponent).bfloat16()
+    index = HIPIndexer(1, 0, 16, layout="row_major").build(x[None].cuda())
+    got = HIPSearcher(kernel=1, index_space="position").search(q.reshape(6, d).cuda(), float("-inf"), index)
+    want = torch.matmul(whole.double(), k.double().transpose(1, 2).contiguous()) * 2.0 ** (exponent - 133)
+    assert torch.equal(got.cpu().double().reshape(2, 3, 500), want)
