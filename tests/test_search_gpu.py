@@ -568,20 +568,34 @@ def test_small_trees_on_the_matrix_cores(t, g, n, d, bf, nl, m, gpu_device):
     assert int(stats[:, 8].sum()) == int(sel[..., :n].any(dim=1).sum())
 
 
-@pytest.mark.parametrize("t,g,n,d,bf,nl,m", [
-    (2, 4, 600, 128, 32, 3, 0),      # two tiles, the second with three nodes in use
-    (2, 4, 1030, 128, 32, 2, 5),     # three, one node in the last, and the queue's
-    (1, 7, 2048, 128, 32, 3, 0),     # four, all nodes full, eight heads' registers
-    (8, 3, 2000, 128, 32, 3, 16),
-    (2, 16, 1100, 128, 32, 3, 0),    # sixteen heads
-    (14, 4, 2000, 128, 32, 2, 0),    # most of the trees that still leave half of the chip
-    (15, 4, 2000, 128, 32, 2, 0),    # too many: a workgroup a tile
-    (2, 4, 1100, 64, 64, 2, 3),      # nodes of four key tiles
-    (2, 8, 4000, 128, 64, 3, 0),
-    (2, 4, 2100, 128, 48, 2, 0),     # three
-    (1, 20, 2000, 128, 32, 3, 0),    # two passes of heads
+def _partials(index, heads, nodes_per_wave):
+    """Partials a head that a launch over the index leaves."""
+    import ctypes as C
+
+    from hira_amd import _lib
+
+    lib, tree, launch = _lib.lib(), C.byref(index.tree_struct()), C.byref(_lib.HiraLaunch(0, nodes_per_wave, 2))
+    query = C.byref(_lib.HiraQuery(heads, 1, 1, 1, 1, 1, heads // index.num_trees, heads // index.num_trees))  # sizes only
+    room = lib.hira_search_workspace_bytes(tree, query, None, launch) - lib.hira_search_counter_bytes(tree, query, launch)
+    a_partial = heads * (index.vdim + 2) * 4
+    assert room > 0 and room % a_partial == 0
+    return room // a_partial
+
+
+@pytest.mark.parametrize("t,g,n,d,bf,nl,m,slices", [
+    (2, 4, 600, 128, 32, 3, 0, 2),      # two tiles, the second with three nodes in use
+    (2, 4, 1030, 128, 32, 2, 5, 2),     # three, one node in the last, and the queue's
+    (1, 7, 2048, 128, 32, 3, 0, 2),     # four, all nodes full, eight heads' registers
+    (8, 3, 2000, 128, 32, 3, 16, 2),
+    (2, 16, 1100, 128, 32, 3, 0, 2),    # sixteen heads
+    (14, 4, 2000, 128, 32, 2, 0, 2),    # most of the trees that still leave half of the chip
+    (15, 4, 2000, 128, 32, 2, 0, 1),    # too many: a workgroup a tile
+    (2, 4, 1100, 64, 64, 2, 3, 2),      # nodes of four key tiles
+    (2, 8, 4000, 128, 64, 3, 0, 2),
+    (2, 4, 2100, 128, 48, 2, 0, 2),     # three
+    (1, 20, 2000, 128, 32, 3, 0, 2),    # two passes of heads
 ])
-def test_workgroups_that_share_a_tile(t, g, n, d, bf, nl, m, gpu_device):
+def test_workgroups_that_share_a_tile(t, g, n, d, bf, nl, m, slices, gpu_device):
     """Launches of two to four tiles a tree against launches that give every tile one workgroup: the counters are
     the same, the outputs differ by the order of their sums."""
     from hira_amd.indexer import HIPIndexer
@@ -602,6 +616,7 @@ def test_workgroups_that_share_a_tile(t, g, n, d, bf, nl, m, gpu_device):
     if m:
         kw.update(queue_keys=torch.randn(t, m, d, generator=gen).bfloat16().cuda(),
                   queue_values=torch.randn(t, m, d, generator=gen).bfloat16().cuda())
+    assert _partials(idx, t * g, 0) == slices * _partials(idx, t * g, 1)
     out, stats = [], []
     for se in (HIPSearcher(kernel=2), HIPSearcher(kernel=2, separate_merge=True), HIPSearcher(kernel=2, nodes_per_wave=1)):
         for _ in range(2):  # (the counters of arrivals are back at zero)
