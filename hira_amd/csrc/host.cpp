@@ -349,6 +349,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 // all three are compiled in, and nothing else would notice that they are others now.
 extern "C" __attribute__((visibility("default"))) PyObject* PyInit__host() {
     PyObject* m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddIntConstant(m, "APPENDED", kAppended) < 0) Py_CLEAR(m);
     PyObject* built = m ? Py_BuildValue("(sii)", HIRA_HOST_TORCH, PY_VERSION_HEX >> 16, HIRA_ABI_VERSION) : nullptr;
     if (built == nullptr || PyModule_AddObject(m, "BUILT_FOR", built) < 0) {
         Py_XDECREF(built);

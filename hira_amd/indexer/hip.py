@@ -1031,18 +1031,19 @@ class HIPIndexer(BaseIndexer):
         self._grow(need)
         if self._state is None:
             self._init_state()
-        tree, rc, most = self.tree_struct(), None, None
+        tree, rc, late, most = self.tree_struct(), None, 0, None
         if dev >= 0:  # in one step, the read-back with it, if the tensors are ready
-            back = None
+            back, host = None, _lib.host()
             if sync and torch.cuda.current_device() == dev:
                 back = self._rows_to_read_into(t * (_lib.HIRA_MAX_LEVELS + 2))
-            rc = _lib.host().append(C.addressof(tree), new_keys, new_values, m, self._state.data_ptr(), *(sample or _NOTHING), dev,
-                                    _lib.stream_of(dev) if stream is None else stream, back,
-                                    next(_TICKETS) % 0x7fffffff + 1)
+            rc = host.append(C.addressof(tree), new_keys, new_values, m, self._state.data_ptr(), *(sample or _NOTHING), dev,
+                             _lib.stream_of(dev) if stream is None else stream, back, next(_TICKETS) % 0x7fffffff + 1)
+            if back is not None and (rc is None or rc.__class__ is list):  # (whatever went wrong: these rows are not used again)
+                self._host_rows = back
             if rc.__class__ is list:
                 most, rc = rc, 0
-            if back is not None and not rc:  # (whatever went wrong: these rows are not used again)
-                self._host_rows = back
+            elif rc is not None and rc <= -host.APPENDED:  # (the rows are in, their sizes could not be read back)
+                late, rc = rc + host.APPENDED, 0
         if rc is None:
             kin = self._rows(new_keys, t, m, self.dim)
             vin = None if new_values is None else self._rows(new_values, t, m, self.vdim)
@@ -1051,11 +1052,11 @@ class HIPIndexer(BaseIndexer):
                                                None if vin is None else vin.data_ptr(), m,
                                                self._state.data_ptr(), rows, per_tree, slots, which, n,
                                                _lib.stream_of(dev))
-        if rc and rc > -100:
+        if rc:
             _lib.check(rc)
         self.num_keys += m
-        if rc:  # (the rows are in, their sizes could not be read back)
-            _lib.check(rc + 100)
+        if late:
+            _lib.check(late)
         if sync:
             self._adopt_state(most)
             self._unsynced_room = 0

@@ -13,6 +13,7 @@ import torch
 
 from hira_amd import _lib
 from hira_amd.attention.hira_attention import hira_attention_forward
+from hira_amd.indexer import HIPIndexer
 from hira_amd.searcher.hip import DecodePlan
 
 
@@ -202,3 +203,23 @@ def test_a_plan_that_takes_its_step_another_way(how, monkeypatch):
     elif how == "no attend":
         plan = SimpleNamespace(run_sampled=lambda *a: _ones(None, *a))
     assert torch.equal(hira_attention_forward(None, q, cache, None, scaling=1.0)[0], torch.ones(1, 1, 4, 16))
+
+
+@pytest.mark.parametrize("code,added", [(-2, 0), (-2 - _lib.host().APPENDED, 3), (-1 - _lib.host().APPENDED, 3)])
+def test_an_append_whose_sizes_could_not_be_read_back(code, added, monkeypatch):
+    """The keys count as soon as their rows are in, and the error is the read-back's; rows that something may yet write into are
+    not used again."""
+    monkeypatch.setattr(_lib, "host", lambda: SimpleNamespace(append=lambda *a: code, APPENDED=_lib._host_module.APPENDED))
+    monkeypatch.setattr(_lib, "stream_of", lambda dev: 0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    ix = HIPIndexer(2, 0, 16, device="cpu")
+    ix.batch, ix.num_heads, ix.num_trees, ix.dim, ix.vdim, ix.num_keys, ix.tiled = 1, 2, 2, 16, 16, 40, False
+    ix.keys_buf = ix.values_buf = SimpleNamespace(get_device=lambda: 0)
+    ix._state = torch.zeros(2, 10, dtype=torch.int32)
+    ix._needed_caps, ix._grow, ix.tree_struct = lambda m: None, lambda need: None, _lib.HiraTree
+    ix._rows_to_read_into = lambda n: torch.zeros(n, dtype=torch.int64)
+    ix._host_rows = kept = torch.zeros(20, dtype=torch.int64)
+    rows = torch.zeros(1, 2, 3, 16)
+    with pytest.raises(ValueError if code == -1 - _lib._host_module.APPENDED else RuntimeError):
+        ix.update(rows, rows)
+    assert ix.num_keys == 40 + added and ix._host_rows is kept

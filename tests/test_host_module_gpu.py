@@ -171,3 +171,70 @@ def test_rows_that_start_between_two_chunks_are_left_alone(name, i, gpu_device):
         if name == "append" and i < 3:  # (without a sample too)
             calls.args[name][5:8] = None, (), ()
             assert calls.refused(name)
+
+
+def _to(i, value):
+    return lambda args: args.__setitem__(i, value(args[i]) if callable(value) else value)
+
+
+def _rows(*shape, dtype=torch.bfloat16):
+    return lambda old: torch.zeros(shape, dtype=dtype, device="cuda")
+
+
+BIG = 2 ** 31
+WRONG = {
+    "enqueue": {
+        "a full queue": _to(4, 8), "before the queue": _to(4, -1), "two rows": _to(2, _rows(1, 2, 2, 64)), "more heads": _to(2, _rows(1, 3, 1, 64)),
+        "more sequences": _to(3, _rows(2, 2, 1, 32)), "narrow keys": _to(2, _rows(1, 2, 1, 32)), "wide values": _to(3, _rows(1, 2, 1, 64)),
+        "another type": _to(3, _rows(1, 2, 1, 32, dtype=torch.float32)), "a shorter queue of values": _to(1, _rows(1, 2, 7, 32)),
+        "a queue of fewer heads": _to(1, _rows(1, 1, 8, 32)), "three dimensions": _to(2, _rows(2, 1, 64)), "half precision": _to(0, _rows(1, 2, 8, 64, dtype=torch.float16)),
+        "strided": _to(2, _strided), "host memory": _to(2, lambda x: x.cpu()), "another device": _to(5, lambda d: d + 1), "no tensor": _to(3, None)},
+    "attend": {
+        "more rows than the queue holds": _to(10, 9), "more rows than the workspace is for": _to(4, 4), "rows below none": _to(10, -1),
+        "rows that are no number": _to(10, 5.0), "a workspace that is too small": _to(3, 513), "a workspace of numbers": _to(2, _rows(512, dtype=torch.float32)),
+        "few thresholds": _to(5, _rows(3, dtype=torch.float32)), "thresholds in 16 bits": _to(5, _rows(4)), "more heads": _to(6, _rows(1, 5, 1, 64)),
+        "two positions": _to(6, _rows(1, 2, 2, 64)), "a wide query": _to(6, _rows(1, 4, 1, 128)), "a query in fp32": _to(6, lambda x: x.float()),
+        "samples of three trees": _to(7, _rows(3, 40, 64)), "narrow samples": _to(7, _rows(2, 40, 32)), "samples in fp32": _to(7, lambda x: x.float()),
+        "a queue of three trees": _to(8, _rows(1, 3, 8, 64)), "a queue of wide keys": _to(8, _rows(1, 2, 8, 128)), "a longer queue of values": _to(9, _rows(1, 2, 9, 32)),
+        "a queue of wide values": _to(9, _rows(1, 2, 8, 64)), "values of one tree": _to(9, _rows(1, 1, 8, 32)), "no queue": _to(8, None),
+        "a large k": _to(12, BIG), "a k that is no number": _to(12, 3.0), "five structs": _to(0, lambda at: at[:5]), "strided": _to(6, _strided)},
+    "search": {
+        "more heads": _to(2, _rows(5, 64)), "a wide query": _to(2, _rows(4, 128)), "as many numbers in wider rows": _to(2, _rows(2, 128)),
+        "a query in fp32": _to(2, lambda x: x.float()), "two positions": _to(2, _rows(1, 2, 2, 64)), "few thresholds": _to(3, _rows(3, dtype=torch.float32)),
+        "thresholds in 16 bits": _to(3, _rows(4)), "a number": _to(3, 4.0), "few scales": _to(4, _rows(2, dtype=torch.float32)), "scales in 64 bits": _to(4, lambda x: x.double()),
+        "fewer slots": _to(5, _rows(4, 95, dtype=torch.float32)), "more slots": _to(5, _rows(4, 97, dtype=torch.float32)), "fewer rows": _to(5, _rows(3, 96, dtype=torch.float32)),
+        "an output in 16 bits": _to(5, _rows(4, 96)), "five structs": _to(0, lambda at: at[:5]), "strided": _to(2, _strided)},
+    "append": {
+        "fewer rows": _to(3, 2), "more rows": _to(3, 4), "rows below none": _to(3, -3), "values of more rows": _to(2, _rows(1, 2, 4, 32)), "wide values": _to(2, _rows(1, 2, 3, 64)),
+        "keys in fp32": _to(1, lambda x: x.float()), "values in fp32": _to(2, lambda x: x.float()), "a sample of three trees": _to(5, _rows(3, 40, 64)),
+        "a narrow sample": _to(5, _rows(2, 40, 32)), "a sample in fp32": _to(5, lambda x: x.float()), "a flat sample": _to(5, _rows(80, 64)),
+        "more slots than keys": _to(6, (1, 2, 3)), "slots in a list": _to(6, [4, 0]), "a large slot": _to(6, (BIG, 0)), "a slot that is no number": _to(6, (4.0, 0)),
+        "a very large key": _to(7, (1, 2 ** 70)), "few rows to read into": _to(10, lambda r: r[:-1]), "rows of half the size": _to(10, lambda r: r.int()),
+        "rows on the device": _to(10, lambda r: r.cuda()), "strided": _to(1, _strided), "another device": _to(8, lambda d: d + 1)},
+}
+
+
+@pytest.mark.parametrize("name,wrong", [(name, wrong) for name in WRONG for wrong in WRONG[name]])
+def test_what_is_not_the_form_is_left_alone(name, wrong, gpu_device):
+    """One property off: None, nothing launched, nothing changed."""
+    with _Calls() as calls:
+        result, launched, changed = calls.call(name)
+        assert launched and result is not None
+        WRONG[name][wrong](calls.args[name])
+        assert calls.refused(name)
+
+
+def test_what_the_library_answers_comes_back(gpu_device):
+    with _Calls() as calls:
+        assert calls.call("enqueue")[:2] == (0, ["hira_enqueue"]) and calls.call("search")[:2] == (0, ["hira_search"])
+        out, launched, changed = calls.call("attend")
+        assert launched == ["hira_search_sampled"] and changed and out.shape == (1, 1, 4, 32) and calls.out.attn_out == out.data_ptr()
+        assert (calls.queue.len, calls.queue.cap, calls.sample.num_rows, calls.sample.k) == (5, 8, 40, 3)
+        back, launched, _ = calls.call("append")
+        assert launched == ["hira_update_sample", "hira_read_state"] and len(back) == _lib.HIRA_MAX_LEVELS + 2
+        for function in ("hira_enqueue", "hira_search", "hira_search_sampled", "hira_read_state"):
+            calls.codes[function] = -2
+        assert calls.call("enqueue")[0] == calls.call("search")[0] == calls.call("attend")[0] == -2
+        assert calls.call("append")[0] == -2 - calls.host.APPENDED
+        calls.codes["hira_update_sample"] = -1
+        assert calls.call("append")[:2] == (-1, ["hira_update_sample"])
