@@ -216,7 +216,7 @@ class HIPSearcher(BaseSearcher):
         tree = indexer.tree_struct()
         dim = indexer.dim
         if q_head_to_kv is None and isinstance(query, torch.Tensor) and \
-                query.dtype is indexer.dtype and query.is_contiguous() and query.data_ptr() % 16 == 0:
+                query.dtype is indexer.dtype and query.is_contiguous():
             shape = query.shape
             nd = len(shape)
             if shape[-1] == dim and (nd == 2 or (nd == 4 and shape[2] == 1)):
@@ -247,7 +247,11 @@ class HIPSearcher(BaseSearcher):
                         sc = scaling
                     else:
                         sc = self._coerce_scaling(scaling, h_q, indexer.device)
-                    qs.q, qs.tau, qs.scaling = query.data_ptr(), tau.data_ptr(), one or sc.data_ptr()
+                    at = query.data_ptr()
+                    if at % 16:
+                        query = _lib.in_chunks(query)
+                        at = query.data_ptr()
+                    qs.q, qs.tau, qs.scaling = at, tau.data_ptr(), one or sc.data_ptr()
                     return c, h_q, (query, tau, sc)
         qs, keep = self._query_struct(query, threshold, indexer, q_head_to_kv, scaling)
         return (_Call(tree, qs, indexer.keys_buf.get_device(), keep), qs.num_q_heads, keep)
@@ -428,8 +432,12 @@ class HIPSearcher(BaseSearcher):
             if qv.numel() != rows * indexer.num_trees * indexer.vdim:
                 raise ValueError(f"queue: keys {tuple(queue_keys.shape)} and values "
                                  f"{tuple(queue_values.shape)} hold different numbers of rows")
+            kp, vp = qk.data_ptr(), qv.data_ptr()
+            if (kp | vp) % 16:
+                qk, qv = _lib.in_chunks(qk), _lib.in_chunks(qv)
+                kp, vp = qk.data_ptr(), qv.data_ptr()
             qu = c.queue
-            qu.keys, qu.values, qu.len, qu.cap = qk.data_ptr(), qv.data_ptr(), rows, rows
+            qu.keys, qu.values, qu.len, qu.cap = kp, vp, rows, rows
             keep = keep + (qk, qv)
         self._run(indexer, c, True, rows)
         del keep
@@ -437,11 +445,12 @@ class HIPSearcher(BaseSearcher):
 
     @staticmethod
     def _queue_rows(x: torch.Tensor, indexer, dev: int, width: int) -> torch.Tensor:
-        """Queued rows of all trees, contiguous, in the index's storage type and on its device, as the kernels read them."""
-        if x.dtype is not indexer.dtype or x.get_device() != dev or not x.is_contiguous() or \
-                x.numel() % (indexer.num_trees * width) != 0:
-            x = x.reshape(indexer.num_trees, -1, width).to(device=indexer.device, dtype=indexer.dtype).contiguous()
-        return _lib.in_chunks(x)
+        """Queued rows of all trees, contiguous, in the index's storage type and on its device."""
+        if x.dtype is indexer.dtype and x.get_device() == dev and x.is_contiguous() and \
+                x.numel() % (indexer.num_trees * width) == 0:
+            return x
+        x = x.reshape(indexer.num_trees, -1, width)
+        return x.to(device=indexer.device, dtype=indexer.dtype).contiguous()
 
     def decode_plan(self, indexer, num_q_heads: int, scaling: float) -> "DecodePlan":
         """The plan for (this index, head count, one softmax scale for all heads), made on
@@ -526,16 +535,16 @@ class DecodePlan:
         None, and nothing done, for any other form, and where ``run_sampled`` is no longer this class's."""
         if getattr(self.run_sampled, "__func__", None) is not _RUN_SAMPLED:
             return None
-        if self.indexer._tree_struct is not self.tree:
-            self._follow_index()
-        at, tree = self._at, self.tree
-        if at is None or at[0][0] is not tree:
-            structs = tree, self.query, self.sample, self.queue, self.out, self.launch
-            at = self._at = structs, tuple(C.addressof(x) for x in structs)
+        at = self._at
+        if at is None or at[0] is not self.indexer._tree_struct:  # (moved, or not made since the index moved)
+            if self.indexer._tree_struct is not self.tree:
+                self._follow_index()
+            structs = self.tree, self.query, self.sample, self.queue, self.out, self.launch
+            at = self._at = *structs, tuple(C.addressof(x) for x in structs)
+            if self.tau_buf is None:
+                self.tau_buf = torch.empty((self.query.num_q_heads,), dtype=torch.float32, device=self.indexer.device)
         # (the structs stay alive with `at` while the call reads them, whoever replaces the plan's meanwhile)
-        if self.tau_buf is None:
-            self.tau_buf = torch.empty((self.query.num_q_heads,), dtype=torch.float32, device=self.indexer.device)
-        out = _lib.host().attend(at[1], self._dev, self.ws, self.ws_bytes, self._ws_rows, self.tau_buf, query, samples, queue_keys,
+        out = _lib.host().attend(at[6], self._dev, self.ws, self.ws_bytes, self._ws_rows, self.tau_buf, query, samples, queue_keys,
                                  queue_values, rows, 0 if method == "sample_max" else 1, k, _lib.stream_of(self._dev))
         if out.__class__ is int:
             _lib.check(out)

@@ -365,8 +365,11 @@ def test_rows_start_where_the_kernels_read_them(dtype):
     idx.keys_buf = idx.values_buf = torch.zeros(2, 4, 16, dtype=dtype)
     idx._tree_struct = _lib.HiraTree(num_trees=2)
     check(idx._rows(x.view(1, 2, 3, 16), 2, 3, 16))
-    check(HIPSearcher._queue_rows(x.view(2, 3, 16), idx, -1, 16))
     se = HIPSearcher()
+    se._run = lambda index, call, attn, rows: queues.append((call.queue.keys, call.queue.values, call.queue.len))
+    queues = []
+    se.search_attention(torch.zeros(2, 16, dtype=dtype), 0.0, idx, scaling=torch.ones(2), queue_keys=x.view(2, 3, 16), queue_values=x.view(2, 3, 16))
+    assert queues[0][0] % 16 == queues[0][1] % 16 == 0 and queues[0][2] == 3
     check(se._query_struct(x.view(6, 16), 0.0, idx, None, None)[1][0])
     for query in (x.view(6, 16), x.view(1, 6, 1, 16)):
         call, heads, keep = se._call(query, 0.0, idx, None, None)
@@ -382,7 +385,7 @@ def test_rows_start_where_the_kernels_read_them(dtype):
         if store:
             cache.queue_store = store
         hira_attention_forward(None, x.view(1, 6, 1, 16), cache, None, scaling=1.0)
-    assert len(copies) == 11
+    assert len(copies) == 10
 
 
 def test_storage_dtype_policy():
