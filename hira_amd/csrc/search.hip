@@ -169,8 +169,8 @@ static int make_plan(const HiraTree* t, const HiraQuery* q, const HiraQueue* que
         // Two to four tiles a tree leave most of the chip idle, and where a tile's keys are 128 KiB or more a compute unit's
         // L1 takes longer for them (0.9 us) than the trip to memory: two workgroups then share a tile, a node of it a wave.  8 trees x
         // 4 heads, 128 columns, a fan-out of 32: 2000 keys 9.23 -> 8.73 us, 1000 9.10 -> 8.44; a fan-out of 64: 3000 keys 12.0 -> 10.5.
-        // With more tiles the fold of twice the partials takes what that gives (4001 keys 9.40 -> 9.74), a tile alone
-        // would have a fold at all (500 keys 7.7 -> 8.5), smaller tiles are there soon enough (64 columns, a fan-out of 16: 8.0 -> 8.55),
+        // With more tiles the fold of twice the partials takes what that gives (4001 keys, eight tiles, 9.40 -> 9.74; five to seven
+        // not measured), a tile alone would have a fold at all (500 keys 7.7 -> 8.5), smaller tiles are there soon enough (64 columns, a fan-out of 16: 8.0 -> 8.55),
         // more workgroups that wait for thresholds are no help (2000 keys 11.5 -> 11.9), nor are they where they would take
         // more than half of the chip (16 trees, 2000 keys: 9.41 -> 9.56).
         const int mt = (t->bf + 15) / 16, gs = plan->gmax <= 4 ? 4 : plan->gmax <= 8 ? 8 : 16;
@@ -313,7 +313,8 @@ static int search_impl(const HiraTree* tree, const HiraQuery* query, const HiraQ
     const bool attn = out->attn_out != nullptr;
     int rc = make_plan(tree, query, queue, launch, attn, &plan);
     if (rc != HIRA_OK) return rc;
-    // (with outputs of another kind the keys are not asked for ahead)
+    // (with outputs of another kind the keys are not asked for ahead.  A step that may make its thresholds itself keeps a workgroup a tile, also
+    // where it then makes them in a launch of their own, which was not measured)
     if (plan.slices > 1 && attn && out->dense == nullptr && out->sel_count == nullptr && !(sample && sample->scratch)) {
         plan.ahead = kAheadNodes / plan.slices;
         plan.tree_blocks *= plan.slices;

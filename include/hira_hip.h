@@ -11,6 +11,8 @@
  *   - Return value: 0 on success, a negative HIRA_E* code otherwise.
  *   - dtype: HIRA_F32 or HIRA_BF16; it is the storage type of keys, values, centers and
  *     queries.  All arithmetic accumulates in fp32.
+ *   - Arrays of rows (keys, values, centers, queries, samples, queues) start at a multiple of
+ *     16 bytes: rows are read in chunks of that.
  *
  * Tree layout (depth-generic, fixed fan-out; the layout of the reference's GPU indexer,
  * indexer/cuda.py:338-357, 439-446, generalised to any depth and to many trees):
