@@ -61,8 +61,10 @@ def device_thresholds(samples: torch.Tensor, query: torch.Tensor, method: str, k
     h_q = query.shape[0]
     if n_s > MAX_DEVICE_SAMPLES:
         raise ValueError(f"{n_s} samples per tree: at most {MAX_DEVICE_SAMPLES}")
-    samples = _lib.in_chunks(samples.contiguous())
-    query = _lib.in_chunks(query.to(device=samples.device, dtype=samples.dtype).contiguous())
+    samples = samples.contiguous()
+    query = query.to(device=samples.device, dtype=samples.dtype).contiguous()
+    if stream is None:  # (a copy is made on the current stream, which a caller's own need not wait for)
+        samples, query = _lib.in_chunks(samples), _lib.in_chunks(query)
     keep = None
     if q_head_to_kv is None:
         if h_q % t:

@@ -388,6 +388,23 @@ def test_rows_start_where_the_kernels_read_them(dtype):
     assert len(copies) == 10
 
 
+def test_thresholds_on_a_stream_of_the_callers_copy_nothing(monkeypatch):
+    """A copy of rows that start between two chunks would be made on the current stream."""
+    from types import SimpleNamespace
+
+    from hira_amd import _lib
+
+    seen = []
+    monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(hira_threshold=lambda rows, *a: seen.append((rows, a[4]._obj.q)) or 0))
+    monkeypatch.setattr(_lib, "current_stream", lambda dev: 0)
+    x = torch.zeros(2 * 8 * 16 + 1)[1:].view(2, 8, 16)
+    q = torch.zeros(4 * 16 + 1)[1:].view(4, 16)
+    threshold_finder.device_thresholds(x, q, "sample_max", stream=5)
+    assert seen == [(x.data_ptr(), q.data_ptr())]
+    threshold_finder.device_thresholds(x, q, "sample_max")
+    assert all(at % 16 == 0 for at in seen[1])
+
+
 def test_storage_dtype_policy():
     assert HIPIndexer.storage_dtype(torch.bfloat16) == torch.bfloat16
     assert HIPIndexer.storage_dtype(torch.float32) == torch.float32
