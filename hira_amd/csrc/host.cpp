@@ -122,14 +122,14 @@ PyObject* enqueue(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// attend((tree, query, sample, queue, out, launch), dev, workspace, bytes of it, queue rows it is for, thresholds (H_q), query
+// attend((tree, query, sample, queue, out, launch, dev, workspace, bytes of it, queue rows it is for), thresholds (H_q), query
 // (B, H_q, 1, D), samples (T, S, D), queue_keys, queue_values (..., cap, D / Dv), rows in use, rule, k, stream): a decode step whose
 // thresholds come from a key sample (DecodePlan.run_sampled).  The output (B, 1, H_q, Dv) in the query's type, or the
 // library's return code where that is an error.
 PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (!arguments("attend", n, 14)) return nullptr;
-    if (!PyTuple_CheckExact(a[0]) || PyTuple_GET_SIZE(a[0]) != 6 || !PyLong_CheckExact(a[10]) || !PyLong_CheckExact(a[12])) Py_RETURN_NONE;
+    if (!arguments("attend", n, 10)) return nullptr;
+    if (!PyTuple_CheckExact(a[0]) || PyTuple_GET_SIZE(a[0]) != 10 || !PyLong_CheckExact(a[6]) || !PyLong_CheckExact(a[8])) Py_RETURN_NONE;
     auto part = [&](int i) { return PyTuple_GET_ITEM(a[0], i); };
     const HiraTree* tree = static_cast<const HiraTree*>(address(part(0)));
     HiraQuery* query = static_cast<HiraQuery*>(address(part(1)));
@@ -137,8 +137,8 @@ PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HiraQueue* queue = static_cast<HiraQueue*>(address(part(3)));
     HiraSearchOut* out = static_cast<HiraSearchOut*>(address(part(4)));
     const HiraLaunch* launch = static_cast<const HiraLaunch*>(address(part(5)));
-    const int64_t dev = number(a[1]), bytes = number(a[3]), rows = number(a[10]), rule = number(a[11]), k = number(a[12]);
-    const at::Tensor *ws = plain(a[2], dev), *tau = plain(a[5], dev), *q = in_chunks(a[6], dev), *s = in_chunks(a[7], dev);
+    const int64_t dev = number(part(6)), bytes = number(part(8)), rows = number(a[6]), rule = number(a[7]), k = number(a[8]);
+    const at::Tensor *ws = plain(part(7), dev), *tau = plain(a[1], dev), *q = in_chunks(a[2], dev), *s = in_chunks(a[3], dev);
     if (!ws || !tau || !q || !s || q->dim() != 4 || s->dim() != 3 || type_of(*q) != tree->dtype || type_of(*s) != tree->dtype ||
         ws->scalar_type() != at::kByte || ws->numel() < bytes || tau->scalar_type() != at::kFloat)
         Py_RETURN_NONE;
@@ -149,10 +149,10 @@ PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor *qk = nullptr, *qv = nullptr;
     int64_t cap = 0;
     if (rows != 0) {
-        qk = in_chunks(a[8], dev), qv = in_chunks(a[9], dev);
+        qk = in_chunks(a[4], dev), qv = in_chunks(a[5], dev);
         if (!qk || !qv || qk->dim() < 2 || qv->dim() < 2 || type_of(*qk) != tree->dtype || type_of(*qv) != tree->dtype) Py_RETURN_NONE;
         cap = qk->size(-2);
-        if (rows < 0 || rows > cap || rows > number(a[4]) || cap > INT32_MAX || qv->size(-2) != cap || qk->size(-1) != tree->dim ||
+        if (rows < 0 || rows > cap || rows > number(part(9)) || cap > INT32_MAX || qv->size(-2) != cap || qk->size(-1) != tree->dim ||
             qv->size(-1) != tree->vdim || qk->numel() != tree->num_trees * cap * tree->dim || qv->numel() != tree->num_trees * cap * tree->vdim)
             Py_RETURN_NONE;
     }
@@ -166,7 +166,7 @@ PyObject* attend(PyObject*, PyObject* const* a, Py_ssize_t n) {
     sample->method = (int32_t)rule;
     sample->k = (int32_t)k;
     sample->tau = tau->mutable_data_ptr<float>();
-    void *workspace = ws->data_ptr(), *stream = address(a[13]);
+    void *workspace = ws->data_ptr(), *stream = address(a[9]);
     const int rc = without_gil([&] {
         return lib.search_sampled(tree, query, sample, rows != 0 ? queue : nullptr, out, launch, workspace, (size_t)bytes, stream);
     });

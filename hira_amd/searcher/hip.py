@@ -508,7 +508,7 @@ class DecodePlan:
         self.sample.scratch = self.tau_scratch.data_ptr()
         self._refs = (C.byref(self.tree), C.byref(self.query), C.byref(self.out),
                       C.byref(self.launch), C.byref(self.queue))
-        self._at: Optional[tuple] = None  # for ``attend``: the call's structs, and where they lie
+        self._at: Optional[tuple] = None  # for ``attend``: the call's structs; where they lie, and the workspace
 
     def _workspace_need(self) -> int:
         fake_q = _lib.HiraQuery(self.query.num_q_heads, 1, 1, 1, 1, 1, self.query.max_group,
@@ -540,12 +540,12 @@ class DecodePlan:
             if self.indexer._tree_struct is not self.tree:
                 self._follow_index()
             structs = self.tree, self.query, self.sample, self.queue, self.out, self.launch
-            at = self._at = *structs, tuple(C.addressof(x) for x in structs)
+            at = self._at = *structs, (*map(C.addressof, structs), self._dev, self.ws, self.ws_bytes, self._ws_rows)
             if self.tau_buf is None:
                 self.tau_buf = torch.empty((self.query.num_q_heads,), dtype=torch.float32, device=self.indexer.device)
         # (the structs stay alive with `at` while the call reads them, whoever replaces the plan's meanwhile)
-        out = _lib.host().attend(at[6], self._dev, self.ws, self.ws_bytes, self._ws_rows, self.tau_buf, query, samples, queue_keys,
-                                 queue_values, rows, 0 if method == "sample_max" else 1, k, _lib.stream_of(self._dev))
+        out = _lib.host().attend(at[6], self.tau_buf, query, samples, queue_keys, queue_values, rows,
+                                 0 if method == "sample_max" else 1, k, _lib.stream_of(self._dev))
         if out.__class__ is int:
             _lib.check(out)
         return out

@@ -104,9 +104,9 @@ def test_what_is_not_the_form_is_left_alone():
     assert host.enqueue(q, q.clone(), k, v, 0, 0, 0) is None  # (host memory)
     assert host.enqueue(None, q, k, [1], 0, 0, 0) is None
     tree, query, out, launch = _lib.HiraTree(num_trees=2, dim=16, vdim=16), _lib.HiraQuery(4), _lib.HiraSearchOut(), _lib.HiraLaunch()
-    at = tuple(C.addressof(x) for x in (tree, query, _lib.HiraSample(), _lib.HiraQueue(), out, launch))
-    ws, tau = torch.zeros(64, dtype=torch.uint8), torch.zeros(4)
-    assert host.attend(at, 0, ws, 64, 1, tau, torch.zeros(1, 4, 1, 16), torch.zeros(2, 8, 16), q, q, 1, 0, 1, 0) is None
+    sample, queue, ws, tau = _lib.HiraSample(), _lib.HiraQueue(), torch.zeros(64, dtype=torch.uint8), torch.zeros(4)
+    at = *(C.addressof(x) for x in (tree, query, sample, queue, out, launch)), 0, ws, 64, 1
+    assert host.attend(at, tau, torch.zeros(1, 4, 1, 16), torch.zeros(2, 8, 16), q, q, 1, 0, 1, 0) is None
     at = C.addressof(tree), C.addressof(query), C.addressof(out), 4, 0, 1
     assert host.search(at, C.addressof(launch), torch.zeros(4, 16), tau, None, torch.zeros(4, 8), 0.0, 0) is None
     assert host.append(C.addressof(tree), k, v, 1, 0, None, (), (), 0, 0, None, 0) is None
@@ -156,7 +156,7 @@ def test_a_plan_holds_its_structs_while_the_call_reads_them(monkeypatch):
         plan._follow_index()
         gc.collect()
         assert trees[-1]() is not None and C.addressof(trees[-1]()) == at[0]
-        return rest[5]
+        return rest[1]
 
     plan = _plan(monkeypatch, attend)
     for _ in range(3):

@@ -125,8 +125,8 @@ class _Calls:
         back = torch.zeros(t * (_lib.HIRA_MAX_LEVELS + 2), dtype=torch.int64, pin_memory=True)
         self.args = {
             "enqueue": [qk, qv, k, v, 3, dev, 0],
-            "attend": [tuple(at.values()), dev, torch.zeros(512, dtype=torch.uint8, device="cuda"), 512, 8, one.clone(), x(1, 4, 1, 64),
-                       samples, qk, qv, 5, 1, 3, 0],
+            "attend": [(*at.values(), dev, torch.zeros(512, dtype=torch.uint8, device="cuda"), 512, 8), one.clone(), x(1, 4, 1, 64), samples,
+                       qk, qv, 5, 1, 3, 0],
             "search": [(at["tree"], at["query"], at["out"], 4, dev, one.data_ptr()), at["launch"], x(4, 64), one.clone(), one.clone(),
                        torch.zeros(4, 96, device="cuda"), -7.0, 0],
             "append": [at["tree"], x(1, t, 3, 64), x(1, t, 3, 32), 3, self.state.data_ptr(), samples, (4, 0), (1, 2), dev, 0, back, 1],
@@ -158,7 +158,7 @@ class _Calls:
         return result is None and not launched and not changed
 
 
-CHUNKS = [("enqueue", 0), ("enqueue", 1), ("enqueue", 2), ("enqueue", 3), ("attend", 6), ("attend", 7), ("attend", 8), ("attend", 9),
+CHUNKS = [("enqueue", 0), ("enqueue", 1), ("enqueue", 2), ("enqueue", 3), ("attend", 2), ("attend", 3), ("attend", 4), ("attend", 5),
           ("search", 2), ("append", 1), ("append", 2), ("append", 5)]
 
 
@@ -177,6 +177,11 @@ def _to(i, value):
     return lambda args: args.__setitem__(i, value(args[i]) if callable(value) else value)
 
 
+def _part(i, value):
+    """A part of the first argument."""
+    return _to(0, lambda at: (*at[:i], value(at[i]) if callable(value) else value, *at[i + 1:]))
+
+
 def _rows(*shape, dtype=torch.bfloat16):
     return lambda old: torch.zeros(shape, dtype=dtype, device="cuda")
 
@@ -190,14 +195,14 @@ WRONG = {
         "a queue of fewer heads": _to(1, _rows(1, 1, 8, 32)), "three dimensions": _to(2, _rows(2, 1, 64)), "half precision": _to(0, _rows(1, 2, 8, 64, dtype=torch.float16)),
         "strided": _to(2, _strided), "host memory": _to(2, lambda x: x.cpu()), "another device": _to(5, lambda d: d + 1), "no tensor": _to(3, None)},
     "attend": {
-        "more rows than the queue holds": _to(10, 9), "more rows than the workspace is for": _to(4, 4), "rows below none": _to(10, -1),
-        "rows that are no number": _to(10, 5.0), "a workspace that is too small": _to(3, 513), "a workspace of numbers": _to(2, _rows(512, dtype=torch.float32)),
-        "few thresholds": _to(5, _rows(3, dtype=torch.float32)), "thresholds in 16 bits": _to(5, _rows(4)), "more heads": _to(6, _rows(1, 5, 1, 64)),
-        "two positions": _to(6, _rows(1, 2, 2, 64)), "a wide query": _to(6, _rows(1, 4, 1, 128)), "a query in fp32": _to(6, lambda x: x.float()),
-        "samples of three trees": _to(7, _rows(3, 40, 64)), "narrow samples": _to(7, _rows(2, 40, 32)), "samples in fp32": _to(7, lambda x: x.float()),
-        "a queue of three trees": _to(8, _rows(1, 3, 8, 64)), "a queue of wide keys": _to(8, _rows(1, 2, 8, 128)), "a longer queue of values": _to(9, _rows(1, 2, 9, 32)),
-        "a queue of wide values": _to(9, _rows(1, 2, 8, 64)), "values of one tree": _to(9, _rows(1, 1, 8, 32)), "no queue": _to(8, None),
-        "a large k": _to(12, BIG), "a k that is no number": _to(12, 3.0), "five structs": _to(0, lambda at: at[:5]), "strided": _to(6, _strided)},
+        "more rows than the queue holds": _to(6, 9), "more rows than the workspace is for": _part(9, 4), "rows below none": _to(6, -1),
+        "rows that are no number": _to(6, 5.0), "a workspace that is too small": _part(8, 513), "a workspace of numbers": _part(7, _rows(512, dtype=torch.float32)),
+        "few thresholds": _to(1, _rows(3, dtype=torch.float32)), "thresholds in 16 bits": _to(1, _rows(4)), "more heads": _to(2, _rows(1, 5, 1, 64)),
+        "two positions": _to(2, _rows(1, 2, 2, 64)), "a wide query": _to(2, _rows(1, 4, 1, 128)), "a query in fp32": _to(2, lambda x: x.float()),
+        "samples of three trees": _to(3, _rows(3, 40, 64)), "narrow samples": _to(3, _rows(2, 40, 32)), "samples in fp32": _to(3, lambda x: x.float()),
+        "a queue of three trees": _to(4, _rows(1, 3, 8, 64)), "a queue of wide keys": _to(4, _rows(1, 2, 8, 128)), "a longer queue of values": _to(5, _rows(1, 2, 9, 32)),
+        "a queue of wide values": _to(5, _rows(1, 2, 8, 64)), "values of one tree": _to(5, _rows(1, 1, 8, 32)), "no queue": _to(4, None),
+        "a large k": _to(8, BIG), "a k that is no number": _to(8, 3.0), "five structs": _to(0, lambda at: at[1:]), "strided": _to(2, _strided)},
     "search": {
         "more heads": _to(2, _rows(5, 64)), "a wide query": _to(2, _rows(4, 128)), "as many numbers in wider rows": _to(2, _rows(2, 128)),
         "a query in fp32": _to(2, lambda x: x.float()), "two positions": _to(2, _rows(1, 2, 2, 64)), "few thresholds": _to(3, _rows(3, dtype=torch.float32)),
